@@ -394,6 +394,7 @@ value_chunk_kernel(const void* __restrict__ v, Source src, int d, int gs, Sink s
   } else {
     ta = src.tile_addr(tile);
   }
+  if (ta.hi <= 0) return;                          // (uniform) a page behind the end of a ragged run
   const bool ok = t >= ta.lo && t < ta.hi;
   const int64_t off = ta.base + (int64_t)t * src.slot_stride();
   const bool page_ok = page >= 0;                    // uniform over the workgroup; false: nothing is stored
@@ -975,6 +976,7 @@ extern "C" int tq_append_kv_ragged(const void* k, const void* v, int dtype, int 
   PagedSource src{B, T_max, H, tiles_per_seq, 0, stride_t, stride_h, start_pos};
   src.run_len = run_len;
   src.row0 = row0;
+  src.compact = B > 1 && B <= PagedSource::MAX_COMPACT;
   return append_runs(k, v, dtype, src, block_table, max_pages, layer, layout, pool, num_pages, stream);
 }
 
@@ -997,6 +999,7 @@ extern "C" int tq_append_kv_from_blocks(const void* k_cache, const void* v_cache
   src.src_stride = src_stride;
   src.stride_blk = stride_blk;
   src.run_len = run_len;
+  src.compact = run_len && B > 1 && B <= PagedSource::MAX_COMPACT;
   return append_runs(k_cache, v_cache, dtype, src, block_table, max_pages, layer, layout, pool, num_pages, stream);
 }
 
