@@ -245,7 +245,10 @@ int tq_pool_export(const uint8_t *pool, int64_t num_pages, int H, const int32_t 
  * kernel of the head sizes 320 .. 704 (a block of 32 tokens per workgroup).  Negative: an error code.           */
 int tq_decode_page_kernel(const tq_layer *layer /*host*/, const tq_page_layout *layout /*host*/);
 
-/* Bytes of workspace tq_decode_attn_paged needs for these sizes.                   */
+/* Bytes of workspace tq_decode_attn_paged needs for these sizes.  n_split > 0: that many equal shares of every
+ * sequence.  n_split < 0: -n_split workgroups per sequence and KV head on average, dealt out by the lengths of the
+ * sequences in device memory (a long one gets more of them); needs more workspace.  The decode entries take the same
+ * two forms (tq_decode_attn_paged_noalloc the first only).                          */
 size_t tq_decode_workspace_bytes(int B, int Hq, int d, int n_split);
 
 /* Fused decode attention over the paged compressed history plus an optional

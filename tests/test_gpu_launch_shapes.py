@@ -46,3 +46,52 @@ def test_ragged_append_numbers_only_the_pages_that_exist(gpu, d, B, H):
     torch.cuda.synchronize()
     assert torch.equal(pa.data, pb.data)
     assert int((pa.data != 0).sum()) > 0
+
+
+def _ragged_pool(gpu, d, key_bits, vb, H, lens, dtype, seed):
+    g = torch.Generator(device=gpu).manual_seed(seed)
+    tq = TurboQuantProd(d, bits=key_bits, device=gpu)
+    B, width = len(lens), max(1, max(-(-n // 16) for n in lens))
+    table = torch.rand(B * width, generator=g, device=gpu).argsort().to(torch.int32).view(B, width).contiguous()
+    pool = PagedKVPool(tq, H, B * width, value_bits=vb, dtype=dtype, device=gpu)
+    rows = sum(lens)
+    k = torch.randn(rows, H, d, generator=g, device=gpu).to(dtype)
+    v = torch.randn(rows, H, d, generator=g, device=gpu).to(dtype)
+    run = _i32(lens, gpu)
+    row0 = (torch.cumsum(run, 0) - run).to(torch.int32)
+    pool.append_ragged(k, v, row0, run, torch.zeros_like(run), table, max_run=max(lens))
+    return pool, table, run, g
+
+
+# (head_dim, key bits, heads per KV head, KV heads, sequences): workgroups of 4 and of 8 wavefronts, a share per wavefront (more
+# pairs than workgroups fit), the merge in the launch and by a kernel of its own, more shares than one pass of the merge
+@pytest.mark.parametrize("d,kb,G,H,B", [(128, 3, 4, 2, 3), (128, 3, 5, 8, 16), (128, 4, 5, 8, 97), (128, 3, 12, 8, 97),
+                                        (64, 3, 4, 4, 200), (256, 3, 8, 2, 5), (256, 2, 4, 4, 90), (128, 2, 1, 1, 1024)])
+@pytest.mark.parametrize("ring", [0, 40])
+def test_shares_by_length_give_what_equal_shares_give(gpu, d, kb, G, H, B, ring):
+    """A step whose workgroups are dealt out by length against the same step with two equal shares per sequence: the same
+    sums in another order.  The weights are rounded to bf16 relative to another reference, so values differ by a few
+    bf16 half-steps of the largest weight: |difference| <= 2^-8 of the largest |value| of a row, and far less on average."""
+    g = torch.Generator().manual_seed(B + d)
+    longest = 9000 if B < 300 else 1500
+    lens = [int(longest * 2.0 ** (-11.0 * float(x))) for x in torch.rand(B, generator=g)]
+    lens[0] = longest
+    if B > 4:
+        lens[1], lens[2], lens[B // 2], lens[-1] = 0, 1, 64, 63
+    dtype = torch.float16 if kb == 4 else torch.bfloat16
+    pool, table, seq, dg = _ragged_pool(gpu, d, kb, 4, H, lens, dtype, 31 * B + d)
+    q = torch.randn(B, H * G, d, generator=dg, device=gpu).to(dtype)
+    _say(f"by length d={d} kb={kb} G={G} H={H} B={B} ring={ring}")
+    if ring:
+        exact = torch.randn(2, pool.num_pages, 16, H, d, generator=dg, device=gpu).to(dtype)
+        outs = [pool.decode_attention_ring(q, table, seq, exact[0], exact[1], ring, max_len=longest, n_split=n).float()
+                for n in (None, 2, None)]
+    else:
+        outs = [pool.decode_attention(q, table, seq, max_len=longest, n_split=n).float() for n in (None, 2, None)]
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[2])
+    a, b = outs[0], outs[1]
+    scale = b.abs().amax(-1, keepdim=True).clamp_min(1e-6)
+    assert float(((a - b).abs() / scale).max()) <= 2.0 ** -5 and float((a - b).norm() / b.norm()) <= 6e-3
+    if B > 4:
+        assert ring or not a[1].any()                    # an empty sequence

@@ -833,9 +833,13 @@ template <int PER, int DT, bool PAGED, bool PACKED>
 __global__ void __launch_bounds__(TAIL_THREADS, 4)
 prep_tail_kernel(TailArgs A, int n_tail, int B, int Gq, tq_layer ly, float* __restrict__ q_rot, float* __restrict__ q_sk,
                  float* __restrict__ q_stat, uint32_t* __restrict__ qa_pack, unsigned long long* __restrict__ arrivals,
-                 int prep_gpw, int n_front, PagePrefetch pf, int g_tot, int head_rows) {
+                 int prep_gpw, int n_front, PagePrefetch pf, int g_tot, int head_rows, SplitPlan sp) {
   extern __shared__ __align__(16) float sm[];
-  const int id = blockIdx.x;
+  if (sp.items && blockIdx.x < SCHED_FRONT) {  // the page kernel's schedule
+    if (blockIdx.x == 0) schedule_splits_body<TAIL_THREADS>(sp, threadIdx.x, (int*)sm);
+    return;
+  }
+  const int id = blockIdx.x - (sp.items ? SCHED_FRONT : 0);
   if (id < n_tail) {
     const int per_z = A.Hkv * B;
     exact_tail_words_body<DT, 1, PAGED, true>(A, id % A.Hkv, (id / A.Hkv) % B, id / per_z, sm);
@@ -890,7 +894,18 @@ static size_t merge_smem(int n_parts, int d, int ny) {
 
 __global__ void __launch_bounds__(256)
 merge_kernel(const float* __restrict__ parts, int n_parts, int part_stride, int d, int dtype, void* __restrict__ out,
-             int row_groups) {
+             int row_groups, const SplitItem* __restrict__ sched, const int32_t* __restrict__ n_of, int n_static,
+             int rows_per_seq, int tail_part) {
+  // (n_of: parts of a scheduled step - n_of[sequence] of them, or n_static if the schedule says equal shares, and those of the exact tail from tail_part on, n_parts -
+  // tail_part in number)
+  int n_first = n_parts, skip = 0;               // part j >= n_first lies skip parts further on
+  if (n_of) {
+    const int equal = sched->n, own = n_of[blockIdx.x / rows_per_seq];
+    n_first = equal ? n_static : own;
+    skip = tail_part - n_first;
+    n_parts = n_first + n_parts - tail_part;
+  }
+  auto at = [&](int j) { return (int64_t)(j < n_first ? j : j + skip); };
   extern __shared__ float s_w[];                 // [n_parts] weights, [n_parts] m, [n_parts] l, [8] scratch, [S][dw] sums
   const int64_t row = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -912,11 +927,11 @@ merge_kernel(const float* __restrict__ parts, int n_parts, int part_stride, int 
 #pragma unroll
   for (int k = 0; k < MERGE_CHUNK; ++k) {
     const int sp = min(sub + k * S, n_parts - 1);
-    v[k] = *(const f2*)(p + (int64_t)sp * (d + 2) + 2 + c0 + 2 * min(pr, np - 1));
+    v[k] = *(const f2*)(p + at(sp) * (d + 2) + 2 + c0 + 2 * min(pr, np - 1));
   }
   float mm = NEG_BIG;
   for (int sp = tid; sp < n_parts; sp += blockDim.x) {
-    const f2 ml = *(const f2*)(p + (int64_t)sp * (d + 2));
+    const f2 ml = *(const f2*)(p + at(sp) * (d + 2));
     s_m[sp] = ml[0];
     s_l[sp] = ml[1];
     if (ml[1] > 0.0f) mm = fmaxf(mm, ml[0]);
@@ -944,7 +959,7 @@ merge_kernel(const float* __restrict__ parts, int n_parts, int part_stride, int 
 #pragma unroll
         for (int k = 0; k < MERGE_CHUNK; ++k) {
           const int sp = min(sub + (k0 + k) * S, n_parts - 1);
-          v[k] = *(const f2*)(p + (int64_t)sp * (d + 2) + 2 + c0 + 2 * p0);
+          v[k] = *(const f2*)(p + at(sp) * (d + 2) + 2 + c0 + 2 * p0);
         }
       }
 #pragma unroll
@@ -973,7 +988,8 @@ using namespace tq;
 namespace tq {
 int launch_rotate_query(const void* q, int dtype, int64_t rows, const tq_layer* layer, float* q_rot, float* q_sk,
                         float* q_stat, uint32_t* qa_pack, int G, float sm_scale, hipStream_t st, bool q_rot_unused,
-                        unsigned long long* arrivals, const PagePrefetch* prefetch, int g_tot, const WidePack* wide);
+                        unsigned long long* arrivals, const PagePrefetch* prefetch, int g_tot, const WidePack* wide,
+                        const SplitPlan& plan);
 bool prep_on_matrix_cores(const void* q, int dtype, int64_t rows, const tq_layer* layer, int G, int g_tot);
 bool rotate_on_matrix_cores(const void* q, int dtype, int64_t rows, const tq_layer* layer, const WidePack* wide);
 }  // namespace tq
@@ -1061,7 +1077,20 @@ extern "C" int tq_decode_page_kernel(const tq_layer* layer, const tq_page_layout
   return decode_wide_has_kernel(*layer, *layout) ? 2 : 0;
 }
 
+// Most shares of one sequence in a step whose n_split B workgroups per KV head are dealt out by length
+static int sched_max_shares(int B, int n_split) {
+  const int64_t most = std::min<int64_t>((int64_t)n_split * B, std::min<int64_t>((int64_t)8 * n_split, 256));
+  return (int)std::max<int64_t>(most, 16);
+}
+// bytes of the schedule in the workspace: items and share counts (at most 8 wavefronts on each of 512 compute units, see
+// decode_sched_items)
+static size_t sched_bytes(int B, int n_split) {
+  return ((size_t)n_split * B + B + 8 * 512 + 1) * sizeof(SplitItem) + (size_t)B * sizeof(int32_t);
+}
+
 extern "C" size_t tq_decode_workspace_bytes(int B, int Hq, int d, int n_split) {
+  if (n_split < 0 && n_split > -(1 << 20) && B > 0)
+    return tq_decode_workspace_bytes(B, Hq, d, sched_max_shares(B, -n_split)) + sched_bytes(B, -n_split);
   if (B <= 0 || Hq <= 0 || d <= 0 || n_split <= 0) return 0;
   // partials for n_split history splits + up to TAIL_MAX_CHUNKS of the exact tail, then q_rot, q_sk, 4 statistics per query row and
   // the packed query operands of the matrix-core kernel (sized for the largest kernel: 9 term planes, 8 heads)
@@ -1076,7 +1105,7 @@ extern "C" int tq_decode_merge(const float* parts, int64_t rows, int n_parts, in
   if (rows == 0) return TQ_OK;
   const int ny = merge_row_groups(rows, n_parts, d);
   merge_kernel<<<dim3((unsigned)rows, ny), dim3(256), merge_smem(n_parts, d, ny), (hipStream_t)stream>>>(
-      parts, n_parts, n_parts, d, dtype, out, ny);
+      parts, n_parts, n_parts, d, dtype, out, ny, nullptr, nullptr, 0, 1, 0);
   TQ_CHECK_LAUNCH();
   return TQ_OK;
 }
@@ -1105,7 +1134,11 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
   const int64_t rs_b = ts.s_b, rs_r = ts.s_r, rs_h = ts.s_h;
   const int32_t* recent_len = ts.len;
   if (!q || !pool || !block_table || !seq_lens || !layer || !layout || !out || !workspace) return TQ_ENULL;
-  if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || n_split <= 0 || num_pages <= 0) return TQ_EINVAL;
+  // n_split < 0: -n_split workgroups per sequence and KV head on average, dealt out by the lengths of the sequences
+  const bool by_length = n_split < 0;
+  const int n_asked = n_split < 0 ? -n_split : n_split;
+  n_split = n_asked;
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || n_split <= 0 || n_split >= (1 << 20) || num_pages <= 0) return TQ_EINVAL;
   if (B > 65535 || Hkv > 65535) return TQ_EUNSUPPORTED;
   // bt_stride > 0: a table row per sequence, that many entries; 0: one row shared by all sequences, length
   // unknown; < 0: one shared row of -bt_stride entries.  Lengths beyond the row are cut to it in the kernels.
@@ -1136,6 +1169,10 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
   // uses the halved count, for every stage of the step alike.
   const bool wide_wg = mfma_shape && layout->key_lane_major && decode_mfma_wide_workgroups(d, Gq, n_split, max_pages);
   if (wide_wg) n_split /= 2;
+  // by length: only on the matrix-core kernel, and with more than one sequence (one is shared out equally anyway)
+  const bool sched = by_length && mfma_shape && stages == 7 && B > 1 && B <= SCHED_MAX_SEQS &&
+                     opt_sequence_walkers.load(std::memory_order_relaxed) < 0;
+  const int n_max = sched ? sched_max_shares(B, n_split) : n_split;
   if (dtype < TQ_F32 || dtype > TQ_BF16) return TQ_EINVAL;
   // the exact tail as 32-bit words: always for fp32, for 16-bit rows when they are word-aligned
   const int epw = dtype == TQ_F32 ? 1 : 2;
@@ -1151,13 +1188,30 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
     const int64_t groups = (int64_t)Hkv * B * ((G + TAIL_GC - 1) / TAIL_GC);
     while (t_chunks < TAIL_MAX_CHUNKS && groups * t_chunks * 2 <= 128 && recent_rows / (t_chunks * 2) >= 16) t_chunks *= 2;
   }
-  const int n_parts = n_split + t_chunks;
+  const int n_parts = n_max + t_chunks;
   float* parts = (float*)workspace;
   float* q_rot = parts + parts_floats(B, Hq, d, n_parts);
   float* q_sk = q_rot + (size_t)B * Hq * d;
   float* q_stat = q_sk + (size_t)B * Hq * d;
   unsigned long long* arrivals = (unsigned long long*)(q_stat + (size_t)4 * B * Hq);    // 8-byte aligned: every term above is even
   uint32_t* qa_pack = (uint32_t*)(arrivals + counter_words(B, Hq));
+  SplitPlan plan;
+  if (sched) {
+    // (behind everything a step with n_max equal shares keeps in the workspace)
+    const uintptr_t end = (uintptr_t)workspace + tq_decode_workspace_bytes(B, Hq, d, sched_max_shares(B, n_asked));
+    plan.items = (SplitItem*)((end + 31) & ~(uintptr_t)31);
+    plan.cap = decode_sched_items(d, layer->mse_bits, B, Hkv * kv_div, n_split, wide_wg);
+    plan.n_of = (int32_t*)(plan.items + 1 + plan.cap);
+    plan.seq_lens = seq_lens;
+    plan.B = B; plan.n_max = n_max; plan.n_static = n_split;
+    PagePrefetch shape;
+    decode_mfma_plan(shape, d, B, Hkv * kv_div, kv_div, n_split, wide_wg);
+    plan.gx = shape.gx; plan.skew16 = shape.skew16; plan.ngrp = shape.ngrp;
+    const bool by_wave = decode_sched_by_wave(d, layer->mse_bits, B, Hkv * kv_div, n_split, wide_wg);
+    plan.step = by_wave ? 1 : shape.ngrp;
+    plan.floor_blocks = by_wave ? 4 : 4 * shape.ngrp;
+    plan.max_tok = max_pages * TQ_PAGE_TOKENS; plan.len_sub = len_sub;
+  }
   // Head sizes of the wide-head page kernel: the rotation launch also packs the kernel's query operands (one copy per
   // group of heads, instead of one per page-kernel workgroup) and writes the row statistics.  All stages of a step
   // decide alike, from the layer, the layout and the options.
@@ -1182,7 +1236,7 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
             !((ta.ws_b | ta.ws_r | ta.ws_h | ta.ws_blk) & 3) && (d / epw) / 4 <= TAIL_THREADS;
   ta.tile_words = tail_tile_words(d / epw, recent_rows, ta.wide != 0);
   ta.max_pages = max_pages; ta.num_blocks = pool_pages;       // the exact cache shares the pool's block numbers
-  ta.sm_scale = sm_scale; ta.parts = parts; ta.n_parts = n_parts; ta.part_index = n_split;
+  ta.sm_scale = sm_scale; ta.parts = parts; ta.n_parts = n_parts; ta.part_index = n_max;
   ta.t_chunks = t_chunks;
   const int n_tail = Hkv * B * ((G + TAIL_GC - 1) / TAIL_GC) * t_chunks;
   bool tail_done = false;
@@ -1198,6 +1252,9 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
     fm.counters = arrivals;
     fm.n_extra = tail ? 1 : 0;          // the exact tail's partial, written by an earlier launch of this step
   }
+  fm.sched = plan.items;
+  fm.sched_cap = plan.cap;
+  fm.extra_part = n_max;
   if (stages & 1) {
     if (!layer->Pi || !layer->PiT || !layer->S || !layer->ST || !layer->centroids) return TQ_ENULL;
     // Workgroups added to the preparation launch read the first pages of every page-kernel workgroup's range
@@ -1232,6 +1289,8 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
     // (16 x 8192: 48.9 -> 45.2 us per step, 32 x 32768: 223.6 -> 221.5 us).
     size_t fsm = tail_words_smem(d, recent_rows, ta.tile_words);
     if (prep_smem_bytes(prep_rows, d) > fsm) fsm = prep_smem_bytes(prep_rows, d);
+    const int n_sched = plan.items ? SCHED_FRONT : 0;
+    if (n_sched && fsm < SCHED_SMEM_INTS * sizeof(int)) fsm = SCHED_SMEM_INTS * sizeof(int);
     // ... unless the tail's tiles leave room for one workgroup per compute unit only (head_dim 256 with 128 exact
     // tokens: 139 KB) and the grid is larger than the card: the preparation workgroups would queue behind that
     // LDS size too (128 x 2048, 16 q / 2 KV heads: 109.7 us per step fused, 88.1 as two launches)
@@ -1249,11 +1308,11 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
       hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)fsm);   \
       if (e != hipSuccess) return (int)e;                                                                            \
     }                                                                                                                \
-    pf.front = n_tail + n_prep;                                                                                      \
+    pf.front = n_tail + n_prep + n_sched;                                                                            \
     if (pf.front > 2 * device_compute_units()) pf.blocks = 0;                                                        \
-    kern<<<dim3((unsigned)(n_tail + n_prep + (pf.blocks > 0 ? pf.n_wg : 0))), dim3(TAIL_THREADS), fsm, st>>>(        \
+    kern<<<dim3((unsigned)(n_sched + n_tail + n_prep + (pf.blocks > 0 ? pf.n_wg : 0))), dim3(TAIL_THREADS), fsm, st>>>( \
         ta, n_tail, B, Gq, *layer, q_rot, q_sk, q_stat, qa_pack, fm.counters, prep_gpw, n_tail + n_prep, pf, g_tot, \
-        decode_mfma_head_rows(d, Gq));                                                                               \
+        decode_mfma_head_rows(d, Gq), plan);                                                                         \
   }
 #define TQ_LAUNCH_PT_DT(PER, PAGED)                                \
   {                                                                \
@@ -1305,7 +1364,7 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
     } else {
       int rc = launch_rotate_query(q, dtype, (int64_t)B * Hq, layer, q_rot, q_sk, q_stat,
                                    mfma_shape ? qa_pack : nullptr, mfma_shape ? Gq : G, sm_scale, st, mfma_shape,
-                                   fm.counters, &pf, mfma_shape ? g_tot : 0, wide_pre.qa ? &wide_pre : nullptr);
+                                   fm.counters, &pf, mfma_shape ? g_tot : 0, wide_pre.qa ? &wide_pre : nullptr, plan);
       if (rc) return rc;
     }
   }
@@ -1325,7 +1384,7 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
     }                                                                                                                \
     kern<<<tgrid, dim3(TAIL_THREADS), tsm, st>>>(__VA_ARGS__);                                                       \
   }
-#define TQ_TAIL_ROWS_ARGS q, Hq, Hkv, d, recent_k, recent_v, recent_rows, rs_b, rs_r, rs_h, recent_len, sm_scale, parts, n_parts, n_split
+#define TQ_TAIL_ROWS_ARGS q, Hq, Hkv, d, recent_k, recent_v, recent_rows, rs_b, rs_r, rs_h, recent_len, sm_scale, parts, n_parts, n_max
 #define TQ_TAIL_WORD_ARGS ta
 #define TQ_TAIL_WORDS(PAGED, WIDE)                                                                                   \
   {                                                                                                                  \
@@ -1411,9 +1470,9 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
 
   if (!(stages & 4)) return TQ_OK;
   // without a tail the merge simply reads one part fewer
-  const int merged = tail ? n_parts : n_split, ny = merge_row_groups((int64_t)B * Hq, merged, d);
+  const int merged = tail ? n_parts : n_max, ny = merge_row_groups((int64_t)B * Hq, merged, d);
   merge_kernel<<<dim3((unsigned)(B * Hq), ny), dim3(256), merge_smem(n_parts, d, ny), st>>>(
-      parts, merged, n_parts, d, dtype, out, ny);
+      parts, merged, n_parts, d, dtype, out, ny, plan.items, plan.n_of, n_split, Hq, n_max);
   TQ_CHECK_LAUNCH();
   return TQ_OK;
 }

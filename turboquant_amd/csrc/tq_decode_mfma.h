@@ -16,8 +16,38 @@ struct FusedMerge {
   int out_dtype = 0;
   unsigned long long* counters = nullptr;
   int n_extra = 0;                   // parts after the n_split splits that an earlier launch has written (the exact tail)
+  const struct SplitItem* sched = nullptr;   // shares of the workgroups by length (see SplitPlan); nullptr: n_split equal shares
+  int sched_cap = 0;                 // items of the schedule (per KV head)
+  int extra_part = 0;                // with a schedule: where the exact tail's part lies (behind the parts of the most splits)
 };
 constexpr int MERGE_IN_KERNEL_MAX_SPLITS = 8;
+
+// Sequences of different lengths: with n_split equal shares each, a step takes as long as its longest sequence needs on
+// n_split workgroups, while those of the short ones idle.  The preparation launch therefore deals the same number of
+// workgroups out by length (schedule_splits_body, tq_prep.h): item i is what the i-th page-kernel workgroup of every
+// KV head does, in the order of dispatch, the largest shares first.  When all lengths are equal (header: n = 1) there are no items and the shares are
+// equal.  96 sequences of 61 .. 8190 tokens, 40 q / 8 KV heads of 128,
+// 4-bit keys: page kernel 129 -> 66 us.
+struct SplitItem {
+  int32_t b, begin, end;             // sequence (-1: nothing to do), blocks [begin, end)
+  int32_t len;                       // its compressed tokens
+  int32_t split, n;                  // this share's number among the n of its sequence
+  int32_t pad[2];
+};
+struct SplitPlan {
+  SplitItem* items = nullptr;        // a header (its n: equal shares), then the items
+  int32_t* n_of = nullptr;           // shares per sequence, for the merge kernel
+  const int32_t* seq_lens = nullptr;
+  int B = 0, cap = 0;                // sequences; items behind the header
+  int n_max = 0;                     // most shares of a sequence (parts in the workspace)
+  int n_static = 0, gx = 0, skew16 = 0, ngrp = 1;     // the launch with equal shares (decode_block_range)
+  int step = 1;                      // walkers of a share: its blocks are a multiple of this many
+  int floor_blocks = 1;              // a smaller share is not worth a workgroup
+  int max_tok = 0, len_sub = 0;
+};
+constexpr int SCHED_FRONT = 8;        // workgroups in front of the preparation's (one of them works: the others keep their dies)
+constexpr int SCHED_MAX_SEQS = 1024;
+constexpr int SCHED_SMEM_INTS = SCHED_MAX_SEQS + 64 + 48;
 
 // Operand rows (query heads) of a group that the page kernel reads from the packed query operands: with at most four
 // heads per group the kernels that take them (two pages per score instruction at head_dim 64, one operand per plane
@@ -69,6 +99,12 @@ struct PagePrefetch {
 // Shape of the page kernel's launch for a step (what launch_one will decide), for the prefetch: fills n_split,
 // groups, kv_div, n_seq, skew16, ngrp, gx, n_wg.
 void decode_mfma_plan(PagePrefetch& pf, int d, int B, int groups, int kv_div, int n_split, bool wide_wg);
+
+// Whether a step that is scheduled by length and has one share per sequence runs a share per wavefront (IW = 1 of the page
+// kernel), and the number of items of a schedule: the workgroups of n_split equal shares, or with one share
+// per sequence what the card holds at once, and room for half as many again when the sequences alone fill it.
+bool decode_sched_by_wave(int d, int mb, int B, int groups, int n_split, bool wide_wg);
+int decode_sched_items(int d, int mb, int B, int groups, int n_split, bool wide_wg);
 
 // Events armed by tq_time_next_page_kernel (which = 0) / tq_time_next_key_kernel (which = 1) on this thread:
 // returns them and disarms; false when none is armed.

@@ -67,6 +67,18 @@ int decode_mfma_split_skew(int n_split, int rows) {
   return units > 0 && groups <= 2 * (int64_t)units && groups * 16 >= 30 * (int64_t)units ? skew : 0;
 }
 
+bool decode_sched_by_wave(int d, int mb, int B, int groups, int n_split, bool wide_wg) {
+  return n_split == 1 && !wide_wg && d != 256 && mb < 4 && (int64_t)groups * B > 2 * (int64_t)device_compute_units();
+}
+
+int decode_sched_items(int d, int mb, int B, int groups, int n_split, bool wide_wg) {
+  if (n_split > 1) return n_split * B;
+  const int units = device_compute_units() > 0 ? device_compute_units() : 256;
+  const int slots = (decode_sched_by_wave(d, mb, B, groups, n_split, wide_wg) ? 8 : (wide_wg ? 1 : 2)) * units;
+  const int fill = slots / groups, over = B + slots / (2 * groups);
+  return fill > over ? fill : over;
+}
+
 void decode_mfma_plan(PagePrefetch& pf, int d, int B, int groups, int kv_div, int n_split, bool wide_wg) {
   const int ds = d == 256 ? 2 : 1, nw = wide_wg ? 2 * MF_WAVES : MF_WAVES;
   pf.n_split = n_split; pf.groups = groups; pf.kv_div = kv_div; pf.n_seq = B;

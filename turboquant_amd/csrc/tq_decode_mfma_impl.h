@@ -234,11 +234,13 @@ __device__ __forceinline__ constexpr int v_bitpos(int t) {
 // The grid is (1, ceil(items IW / 4), 1).
 template <int D, int MB, int NX, int VB, int GS, int DS, int WPS, bool F16P, bool PP, bool NR, bool SG, int NW, int IW>
 __global__ void __launch_bounds__(NW * 64, WPS)
-decode_mfma_kernel(uint32_t* qa_pack, float* q_stat, int Hq, int Hkv, int kv_div,
-                   const uint8_t* __restrict__ pool, const int32_t* __restrict__ block_table,
-                   int bt_stride, const int32_t* __restrict__ seq_lens, float sm_scale, tq_layer ly, tq_page_layout L,
-                   float* __restrict__ parts, int n_parts, int n_split, int len_sub, int max_pages, int num_pages,
-                   int skew16, int n_seq, FusedMerge fm) {
+decode_mfma_kernel(const int32_t* __restrict__ seq_lens, const SplitItem* __restrict__ sched,
+                   const int32_t* __restrict__ block_table, const uint8_t* __restrict__ pool, int n_split, int skew16, int n_seq,
+                   int bt_stride, int len_sub, int max_pages, int num_pages, int Hq, int Hkv, int kv_div,
+                   uint32_t* qa_pack, float* q_stat, float* __restrict__ parts, int n_parts, float sm_scale,
+                   tq_page_layout L, FusedMerge fm, tq_layer ly) {
+  // (the first arguments arrive in registers - the build asks for it -: those that the chain schedule / sequence length ->
+  // page numbers -> pages starts from come first)
   constexpr int DW = D / DS;                  // coordinates / channels of one wavefront
   constexpr int WPLT = (D + 127) / 128;       // plane words per lane per plane per page, all wavefronts
   constexpr int WPL = (DW + 127) / 128;       // ... of one wavefront (head_dim 64: one, with half of the lanes idle)
@@ -277,6 +279,8 @@ decode_mfma_kernel(uint32_t* qa_pack, float* q_stat, int Hq, int Hkv, int kv_div
   // to a compute unit, and a SIMD serves its older wavefronts first: with equal shares the first half of the grid
   // finishes early and the second half runs on alone.
   int split = blockIdx.x, b = blockIdx.z;
+  // (sched: the share of this workgroup - of this wavefront when IW > 0 - is item `slot` of the step's schedule)
+  int n_mine = n_split, slot = blockIdx.x + (skew16 > 0 ? n_split / 2 : n_split) * blockIdx.z;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wgrp = wave / DS, hf = wave % DS; // block walker this wavefront belongs to; its share of the head
@@ -288,11 +292,11 @@ decode_mfma_kernel(uint32_t* qa_pack, float* q_stat, int Hq, int Hkv, int kv_div
   constexpr int IWC = IW > 0 ? IW : 1;
   const int wsub = IW > 0 ? wgrp % IWC : wgrp;  // this walker's number among those of its (sequence, head group)
   if constexpr (IW > 0) {
-    const int item = blockIdx.y * (NW / DS / IWC) + wgrp / IWC, items = Hkv * n_seq;
+    const int item = blockIdx.y * (NW / DS / IWC) + wgrp / IWC, items = Hkv * (sched ? fm.sched_cap : n_seq);
     item_live = item < items;
     const int item_c = item_live ? item : items - 1;          // (a wavefront without an item repeats the last one and stores nothing)
     h = item_c % Hkv;
-    b = item_c / Hkv;
+    b = slot = item_c / Hkv;
   }
   if (kv_div > 1) {
     const int kv_heads = Hkv / kv_div, grp = h / kv_heads, kvh = h - grp * kv_heads;
@@ -303,7 +307,21 @@ decode_mfma_kernel(uint32_t* qa_pack, float* q_stat, int Hq, int Hkv, int kv_div
   } else {
     qbase = h * G;
   }
-  if (DS == 2 && skew16 > 0) {                                  // (only the launcher of DS == 2 kernels passes a skew)
+  SplitItem share;
+  bool by_length = false;
+  if (sched) {
+    share = sched[1 + slot];
+    int equal = sched->n;
+    asm volatile("" : "+s"(equal));                           // (one wait for both)
+    by_length = !equal;
+  }
+  if (by_length) {
+    if (IW == 0 && share.b < 0) return;                       // (the whole workgroup: the items' order is that of dispatch)
+    item_live = item_live && share.b >= 0;
+    b = max(share.b, 0);
+    split = share.split;
+    n_mine = share.n;
+  } else if (DS == 2 && skew16 > 0) {                                  // (only the launcher of DS == 2 kernels passes a skew)
     // (n_seq arrives with the other kernel arguments; the grid's size would be one more scalar load of the
     // launch's implicit data in front of everything that depends on the sequence)
     const int late = b >= n_seq;
@@ -438,10 +456,14 @@ decode_mfma_kernel(uint32_t* qa_pack, float* q_stat, int Hq, int Hkv, int kv_div
   TQ_STAMP(1);
   // ---------------------------------------------------------------- work range (all scalar)
   // len_sub: newest tokens that are attended to exactly.  A length beyond the block table is cut to the table.
-  const int seq_len = item_live ? max(min(seq_lens[b], max_pages * TQ_PAGE_TOKENS) - len_sub, 0) : 0;
+  int seq_len = 0, blk_begin = 0, blk_end = 0;
+  if (by_length) {
+    if (item_live) { seq_len = share.len; blk_begin = share.begin; blk_end = share.end; }
+  } else {
+    seq_len = item_live ? max(min(seq_lens[b], max_pages * TQ_PAGE_TOKENS) - len_sub, 0) : 0;
+    decode_block_range(seq_len, n_split, split, DS == 2 ? skew16 : 0, NGRP, blk_begin, blk_end);
+  }
   const int n_pages = (seq_len + TQ_PAGE_TOKENS - 1) / TQ_PAGE_TOKENS;
-  int blk_begin, blk_end;
-  decode_block_range(seq_len, n_split, split, DS == 2 ? skew16 : 0, NGRP, blk_begin, blk_end);
   const int32_t* bt = block_table + (int64_t)b * bt_stride;
   const uint8_t* pool_h = pool + (int64_t)(h / kv_div) * L.page_bytes;
   const int64_t page_stride = (int64_t)(Hkv / kv_div) * L.page_bytes;
@@ -1084,6 +1106,59 @@ decode_mfma_kernel(uint32_t* qa_pack, float* q_stat, int Hq, int Hkv, int kv_div
   }
   __syncthreads();
   TQ_STAMP(7);
+  // The log-sum-exp merge of this (sequence, head group)'s n_mine parts and the exact tail's, by the nt threads of the
+  // workgroup (or wavefront) that finished last.  All loads of up to NP parts before the first use; more parts (only a
+  // schedule has them) follow NP at a time.
+  auto merge_parts = [&](int t0, auto nt_tag) __attribute__((always_inline)) {
+    constexpr int NT = decltype(nt_tag)::value, NP = MERGE_IN_KERNEL_MAX_SPLITS + 1;
+    const int n_merge = n_mine + fm.n_extra;
+    // (every thread's rounds are independent: unrolled, so that the loads of all of them are in flight together; the
+    // wavefront version has four times as many rounds and takes four at a time)
+    constexpr int ROUNDS = 8 * D / NT, TOGETHER = ROUNDS > 4 ? 4 : ROUNDS;
+    for (int k0 = 0; k0 < ROUNDS; k0 += TOGETHER)
+#pragma unroll
+    for (int kk = 0; kk < TOGETHER; ++kk) {
+      const int k = k0 + kk;
+      const int o = t0 + k * NT;
+      const bool live = o < G * D;
+      const int g = live ? o / D : 0, ch = o % D;
+      const float* row = parts + ((int64_t)b * Hq + qbase + g) * n_parts * (D + 2);
+      float m_s[NP], l_s[NP], a_s[NP];
+      auto request = [&](int s0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+          const int sp = min(s0 + i, n_merge - 1);
+          const float* r = row + (int64_t)(sp < n_mine ? sp : fm.extra_part) * (D + 2);
+          m_s[i] = load_coherent(r); l_s[i] = load_coherent(r + 1); a_s[i] = load_coherent(r + 2 + ch);
+        }
+      };
+      float mm = MF_NEG, ll = 0.0f, aa = 0.0f;
+      auto take = [&](int s0) __attribute__((always_inline)) {
+        float top = mm;
+#pragma unroll
+        for (int i = 0; i < NP; ++i)
+          if (s0 + i < n_merge && l_s[i] > 0.0f) top = fmaxf(top, m_s[i]);
+        const float keep = __expf(mm - top);                 // (nothing so far: anything times zero)
+        mm = top;
+        ll *= keep;
+        aa *= keep;
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+          const float wgt = (s0 + i < n_merge && l_s[i] > 0.0f) ? __expf(m_s[i] - mm) : 0.0f;
+          ll = fmaf(wgt, l_s[i], ll);
+          aa = fmaf(wgt, a_s[i], aa);
+        }
+      };
+      request(0);
+      take(0);
+      for (int s0 = NP; s0 < n_merge; s0 += NP) {
+        request(s0);
+        take(s0);
+      }
+      const float inv = ll > 0.0f ? 1.0f / ll : 0.0f;
+      if (live) store_from_f32(fm.out, ((int64_t)b * Hq + qbase + g) * D + ch, aa * inv, fm.out_dtype);
+    }
+  };
   if constexpr (IW > 0) {
     // The IW wavefronts of a (sequence, head group) finish it among themselves: their rows of s_red hold its walkers.
     constexpr int TP = 64 * IWC;                 // threads of a (sequence, head group)
@@ -1108,7 +1183,7 @@ decode_mfma_kernel(uint32_t* qa_pack, float* q_stat, int Hq, int Hkv, int kv_div
       }
       return aa;
     };
-    if (fm.out != nullptr && fm.n_extra <= 1) {
+    if (fm.out != nullptr && fm.n_extra <= 1 && n_mine == 1) {
       // the attention output, merged with the exact tail's partial if there is one (an earlier launch wrote it)
 #pragma unroll
       for (int k = 0; k < 8 * D / TP; ++k) {
@@ -1122,7 +1197,7 @@ decode_mfma_kernel(uint32_t* qa_pack, float* q_stat, int Hq, int Hkv, int kv_div
           const float inv = ll > 0.0f ? 1.0f / ll : 0.0f;
           store_from_f32(fm.out, ((int64_t)b * Hq + qbase + g) * D + ch, aa * inv, fm.out_dtype);
         } else if (live) {
-          const float* x = parts + (((int64_t)b * Hq + qbase + g) * n_parts + 1) * (D + 2);     // the exact tail's part
+          const float* x = parts + (((int64_t)b * Hq + qbase + g) * n_parts + fm.extra_part) * (D + 2);     // the exact tail's part
           const float m_x = x[0], l_x = x[1], a_x = x[2 + ch];
           float top = MF_NEG;
           if (ll > 0.0f) top = fmaxf(top, mm);
@@ -1143,6 +1218,16 @@ decode_mfma_kernel(uint32_t* qa_pack, float* q_stat, int Hq, int Hkv, int kv_div
           const float a0 = merged(g, 2 * pr, mm, ll), a1 = merged(g, 2 * pr + 1, m2, l2);
           float* out = parts + (((int64_t)b * Hq + qbase + g) * n_parts + split) * (D + 2);
           store_coherent2(out + 2 * pr, pr == 0 ? f32x2{mm, ll} : f32x2{a0, a1});
+        }
+      }
+      // a sequence with several shares: the wavefront that finishes last among them merges (IW = 1; see below)
+      if constexpr (IW == 1) {
+        if (by_length && fm.out != nullptr && item_live) {
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          unsigned long long before = 0;
+          if (lane == 0)
+            before = __hip_atomic_fetch_add(fm.counters + ((int64_t)b * Hkv + h), 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if (__builtin_amdgcn_readfirstlane((int)before) + 1 == n_mine) merge_parts(lane, std::integral_constant<int, 64>{});
         }
       }
     }
@@ -1170,7 +1255,7 @@ decode_mfma_kernel(uint32_t* qa_pack, float* q_stat, int Hq, int Hkv, int kv_div
   // alone; a path of its own, so that the others' epilogue stays what it was): the walkers' sum, merged with the
   // exact tail's partial if there is one (an earlier launch wrote it: plain loads), is the result - what the merge
   // further down would compute from the same parts in the same order, without the trip through memory and the counting.
-  if (DS == 1 && fm.out != nullptr && n_split == 1 && fm.n_extra <= 1) {
+  if (DS == 1 && fm.out != nullptr && n_mine == 1 && fm.n_extra <= 1) {
 #pragma unroll
     for (int k = 0; k < 8 * D / (MF_WAVES * 64); ++k) {
       const int o = tid + k * (MF_WAVES * 64);
@@ -1182,7 +1267,7 @@ decode_mfma_kernel(uint32_t* qa_pack, float* q_stat, int Hq, int Hkv, int kv_div
         const float inv = ll > 0.0f ? 1.0f / ll : 0.0f;
         store_from_f32(fm.out, ((int64_t)b * Hq + qbase + g) * D + ch, aa * inv, fm.out_dtype);
       } else if (live) {
-        const float* x = parts + (((int64_t)b * Hq + qbase + g) * n_parts + 1) * (D + 2);     // the exact tail's part
+        const float* x = parts + (((int64_t)b * Hq + qbase + g) * n_parts + fm.extra_part) * (D + 2);     // the exact tail's part
         const float m_x = x[0], l_x = x[1], a_x = x[2 + ch];
         float top = MF_NEG;
         if (ll > 0.0f) top = fmaxf(top, mm);
@@ -1265,42 +1350,14 @@ decode_mfma_kernel(uint32_t* qa_pack, float* q_stat, int Hq, int Hkv, int kv_div
     if (tid == 0) {
       const unsigned long long before = __hip_atomic_fetch_add(fm.counters + ((int64_t)b * Hkv + h), 1ull, __ATOMIC_RELAXED,
                                                                __HIP_MEMORY_SCOPE_AGENT);
-      s_last = before + 1ull == (unsigned long long)n_split;
+      s_last = before + 1ull == (unsigned long long)n_mine;
     }
     __syncthreads();
     if (s_last) {
       // Acquire: the loads below are device-coherent loads issued after the counter's value has come back
       // (s_last depends on it), and every other workgroup's stores were acknowledged before its increment.
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-#pragma unroll
-      for (int k = 0; k < 8 * D / (MF_WAVES * 64); ++k) {
-        const int o = tid + k * (MF_WAVES * 64);
-        const bool live = o < G * D;
-        const int g = live ? o / D : 0, ch = o % D;
-        const float* row = parts + ((int64_t)b * Hq + qbase + g) * n_parts * (D + 2);
-        // all loads first (clamped to an existing part), then the log-sum-exp merge
-        constexpr int NP = MERGE_IN_KERNEL_MAX_SPLITS + 1;
-        const int n_merge = n_split + fm.n_extra;
-        float m_s[NP], l_s[NP], a_s[NP];
-#pragma unroll
-        for (int sp = 0; sp < NP; ++sp) {
-          const float* r = row + (int64_t)min(sp, n_merge - 1) * (D + 2);
-          m_s[sp] = load_coherent(r); l_s[sp] = load_coherent(r + 1); a_s[sp] = load_coherent(r + 2 + ch);
-        }
-        float mm = MF_NEG;
-#pragma unroll
-        for (int sp = 0; sp < NP; ++sp)
-          if (sp < n_merge && l_s[sp] > 0.0f) mm = fmaxf(mm, m_s[sp]);
-        float ll = 0.0f, aa = 0.0f;
-#pragma unroll
-        for (int sp = 0; sp < NP; ++sp) {
-          const float wgt = (sp < n_merge && l_s[sp] > 0.0f) ? __expf(m_s[sp] - mm) : 0.0f;
-          ll = fmaf(wgt, l_s[sp], ll);
-          aa = fmaf(wgt, a_s[sp], aa);
-        }
-        const float inv = ll > 0.0f ? 1.0f / ll : 0.0f;
-        if (live) store_from_f32(fm.out, ((int64_t)b * Hq + qbase + g) * D + ch, aa * inv, fm.out_dtype);
-      }
+      merge_parts(tid, std::integral_constant<int, MF_WAVES * 64>{});
     }
   }
 }
@@ -1350,6 +1407,7 @@ static int launch_one(uint32_t* qa_pack, float* q_stat, int B, int Hq, int Hkv, 
   if constexpr (can_iw && IW == 0) {
     if (n_split == 1 && !wide_wg) {
       int walkers = opt_sequence_walkers.load(std::memory_order_relaxed);
+      if (fm.sched) walkers = decode_sched_by_wave(D, MB, B, Hkv, n_split, wide_wg) ? 1 : 4;
       if (walkers < 0) {
         const int64_t slots = (int64_t)8 * device_compute_units(), items = (int64_t)Hkv * B;
         walkers = slots <= 0 || 4 * items <= slots ? 4 : (2 * items <= slots ? 2 : 1);
@@ -1375,7 +1433,8 @@ static int launch_one(uint32_t* qa_pack, float* q_stat, int B, int Hq, int Hkv, 
   // what they move (32 x 32768: 203 -> 208 us).
   const int skew16 = NW == MF_WAVES && WPS == 2 && DS == 2 ? decode_mfma_split_skew(n_split, Hkv * B) : 0;
   constexpr int IPW = NW / DS / (IW > 0 ? IW : 1);          // (sequence, head group) pairs of a workgroup with IW > 0
-  const dim3 grid = IW > 0 ? dim3(1, (unsigned)(((int64_t)Hkv * B + IPW - 1) / IPW), 1)
+  const dim3 grid = IW > 0 ? dim3(1, (unsigned)(((int64_t)Hkv * (fm.sched ? fm.sched_cap : B) + IPW - 1) / IPW), 1)
+                    : fm.sched && n_split == 1 ? dim3(1, Hkv, fm.sched_cap)
                        : (skew16 > 0 ? dim3(n_split / 2, Hkv, 2 * B) : dim3(n_split, Hkv, B));
   auto kern = decode_mfma_kernel<D, MB, NX, VB, GS, DS, WPS, F16P, PP, NR, SG, NW, IW>;
   if (smem > 48 * 1024) {
@@ -1385,12 +1444,12 @@ static int launch_one(uint32_t* qa_pack, float* q_stat, int B, int Hq, int Hkv, 
   hipEvent_t t_start_event = nullptr, t_stop_event = nullptr;
   if (take_time_hook(0, t_start_event, t_stop_event)) {
     hipExtLaunchKernelGGL(kern, grid, dim3(NW * 64), smem, st, t_start_event, t_stop_event, 0,
-                          qa_pack, q_stat, Hq, Hkv, kv_div, pool, block_table, bt_stride, seq_lens, sm_scale, ly, L, parts,
-                          n_parts, n_split, len_sub, max_pages, num_pages, skew16, B, fm);
+                          seq_lens, fm.sched, block_table, pool, n_split, skew16, B, bt_stride, len_sub, max_pages, num_pages, Hq, Hkv,
+                          kv_div, qa_pack, q_stat, parts, n_parts, sm_scale, L, fm, ly);
   } else {
-    kern<<<grid, dim3(NW * 64), smem, st>>>(qa_pack, q_stat, Hq, Hkv, kv_div, pool, block_table, bt_stride, seq_lens,
-                                            sm_scale, ly, L, parts, n_parts, n_split, len_sub, max_pages, num_pages, skew16,
-                                            B, fm);
+    kern<<<grid, dim3(NW * 64), smem, st>>>(seq_lens, fm.sched, block_table, pool, n_split, skew16, B, bt_stride, len_sub,
+                                            max_pages, num_pages, Hq, Hkv, kv_div, qa_pack, q_stat, parts, n_parts, sm_scale,
+                                            L, fm, ly);
   }
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? TQ_OK : (int)e;

@@ -326,6 +326,110 @@ __device__ __forceinline__ unsigned long long load_coherent(const unsigned long 
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// The schedule of a step (see SplitPlan), by one workgroup of NT threads of the preparation launch, which has the time
+// that the preparation takes: the smallest share of blocks with which all shares fit the items is found by trying 64
+// sizes at a time, then the shares are written largest first (by sixteenths of the largest).
+__device__ __forceinline__ int sched_pieces(int nb, int tau, float inv, int n_max) {
+  const int n = (int)((float)(nb + tau - 1) * inv);          // (any rounding will do: the share size follows from the count)
+  return n < 1 ? 1 : (n > n_max ? n_max : n);
+}
+template <int NT>
+__device__ __forceinline__ void schedule_splits_body(const SplitPlan& P, int tid, int* sm) {
+  int* nb = sm;                                  // [B] blocks
+  int* cand = sm + SCHED_MAX_SEQS;               // [64] shares with a candidate size
+  int* red = cand + 64;                          // [0] most blocks, [2] largest share; [16..31] bucket sizes, [32..47] next item of a bucket
+  auto blocks_of = [&](int b) { return (max(min(P.seq_lens[b], P.max_tok) - P.len_sub, 0) + 63) / 64; };
+  // Equal lengths (in blocks): equal shares, and the page kernel works them out itself.  The usual case, and one whose
+  // time counts: in a serving loop the caches are full of pages and every instruction comes from memory.
+  if (P.cap == P.n_static * P.B) {
+    const int n0 = blocks_of(0);
+    int same = 1;
+    for (int b = tid; b < P.B; b += NT) same &= blocks_of(b) == n0;
+    same = __syncthreads_and(same);
+    if (tid == 0) P.items->n = same;
+    if (same) return;
+  } else if (tid == 0) {
+    P.items->n = 0;
+  }
+  if (tid < 48) red[tid] = 0;
+  __syncthreads();
+  for (int b = tid; b < P.B; b += NT) {
+    nb[b] = blocks_of(b);
+    atomicMax(red + 0, nb[b]);
+  }
+  __syncthreads();
+  const int most = red[0];
+  SplitItem* items = P.items + 1;
+  int lo = max(P.floor_blocks, 1), hi = max(most, lo);       // hi always fits
+  constexpr int TPC = NT / 64;                               // threads per candidate
+  while (lo < hi) {
+    const int stride = (hi - lo + 63) / 64, tau = min(lo + (tid / TPC) * stride, hi);
+    const float inv = 1.0f / (float)tau;
+    if (tid < 64) cand[tid] = 0;
+    __syncthreads();
+    int n = 0;
+    for (int b = tid % TPC; b < P.B; b += TPC) n += sched_pieces(nb[b], tau, inv, P.n_max);
+    atomicAdd(cand + tid / TPC, n);
+    __syncthreads();
+    // the first candidate that fits (monotone but for the clamp to n_max and the rounding; hi fits in any case)
+    const bool fits = cand[tid & 63] <= P.cap;
+    const unsigned long long m = __builtin_amdgcn_ballot_w64(fits);
+    const int first = m ? __builtin_ctzll(m) : 63;
+    const int tau_f = m ? min(lo + first * stride, hi) : hi;
+    const int lo_n = first > 0 ? min(lo + (first - 1) * stride + 1, tau_f) : lo;
+    __syncthreads();
+    lo = lo_n; hi = tau_f;
+    if (stride == 1) break;
+  }
+  const int tau = hi;
+  const float inv = 1.0f / (float)tau;
+  auto share = [&](int n_blocks, int& n) {                   // blocks of a share, and how many there are
+    n = sched_pieces(n_blocks, tau, inv, P.n_max);
+    int per = (n_blocks + n - 1) / n;
+    per = max((per + P.step - 1) / P.step, 1) * P.step;
+    n = max((n_blocks + per - 1) / per, 1);
+    return per;
+  };
+  for (int b = tid; b < P.B; b += NT) {
+    int n;
+    const int per = share(nb[b], n);
+    atomicMax(red + 2, min(per, nb[b]));
+    P.n_of[b] = n;
+  }
+  __syncthreads();
+  const float to16 = 16.0f / (float)(red[2] + 1);
+  auto bucket = [&](int per, int n_blocks) { return 15 - min((int)((float)min(per, n_blocks) * to16), 15); };
+  for (int b = tid; b < P.B; b += NT) {
+    int n;
+    const int per = share(nb[b], n);
+    atomicAdd(red + 16 + bucket(per, nb[b]), n);
+  }
+  __syncthreads();
+  if (tid < 16) {
+    int at = 0;
+    for (int k = 0; k < tid; ++k) at += red[16 + k];
+    red[32 + tid] = at;
+  }
+  __syncthreads();
+  for (int b = tid; b < P.B; b += NT) {
+    int n;
+    const int per = share(nb[b], n), at = atomicAdd(red + 32 + bucket(per, nb[b]), n);
+    const int len = max(min(P.seq_lens[b], P.max_tok) - P.len_sub, 0);
+    for (int s = 0; s < n; ++s) {
+      SplitItem it;
+      it.b = b; it.split = s; it.n = n; it.len = len;
+      it.begin = s * per; it.end = min(it.begin + per, nb[b]);
+      it.pad[0] = it.pad[1] = 0;
+      items[at + s] = it;
+    }
+  }
+  __syncthreads();
+  SplitItem none;
+  none.b = -1; none.begin = none.end = none.len = none.split = 0; none.n = 1;
+  none.pad[0] = none.pad[1] = 0;
+  for (int i = red[47] + tid; i < P.cap; i += NT) items[i] = none;
+}
+
 // Prefetch workgroup p of a preparation launch (see PagePrefetch): reads, and discards, the pages that one
 // page-kernel workgroup will ask for first.  Workgroups go to the card's dies in turn, so the page-kernel
 // workgroup picked is the one whose position in its grid is congruent to this workgroup's position in this

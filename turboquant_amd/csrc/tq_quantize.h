@@ -82,43 +82,7 @@ struct PagedSource {         // (b, t, h, :) strided, tokens mapped onto 16-toke
   // Optional ragged mode: the rows of all sequences lie one after another in one (rows, H, :) tensor; the
   // run of sequence b begins at row row0[b] (stride_b is unused, run_len gives its length).
   const int32_t* row0 = nullptr;
-  // Runs of different lengths (run_len): the launch is sized for B runs of T tokens, most of which a ragged batch
-  // does not have.  With `compact` the tiles are numbered over the pages that the runs really touch; a workgroup
-  // builds the index of them (first page of every sequence, page_index) in its LDS from start_pos and run_len.
-  static constexpr int MAX_COMPACT = 1024;     // sequences
-  int compact = 0;
-  __device__ int run_pages(int b) const {
-    const int s0 = start_pos ? start_pos[b] : 0, n = min(run_len[b], T);
-    return n > 0 ? (s0 % TILE + n + TILE - 1) / TILE : 0;
-  }
-  // cum[b] = pages of the sequences before b, b = 0 .. B; called by all NT threads of the workgroup (with a barrier)
-  template <int NT>
-  __device__ void page_index(int* cum, int* scratch, int tid) const {
-    constexpr int PER = MAX_COMPACT / NT;
-    int n[PER], sum = 0;
-#pragma unroll
-    for (int k = 0; k < PER; ++k) {
-      n[k] = tid * PER + k < B ? run_pages(tid * PER + k) : 0;
-      sum += n[k];
-    }
-    int incl = sum;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int up = __shfl_up(incl, o, 64);
-      incl += (tid & 63) >= o ? up : 0;
-    }
-    if ((tid & 63) == 63) scratch[tid >> 6] = incl;
-    __syncthreads();
-    int at = incl - sum;
-    for (int w = 0; w < (tid >> 6); ++w) at += scratch[w];
-#pragma unroll
-    for (int k = 0; k < PER; ++k) {
-      if (tid * PER + k <= B) cum[tid * PER + k] = at;
-      at += n[k];
-    }
-    if (tid == NT - 1 && B == MAX_COMPACT) cum[B] = at;
-    __syncthreads();
-  }
+  int compact = 0;                       // (host) the kernels with a RaggedSource take this call
   // (sequence, page slot window, head) of a tile, and of the tile after it (a walk that leaves the last
   // sequence stays on its last tile): the divisions by run-time sizes are done once per group of tiles
   struct Coord { int b, pg, h; };
@@ -128,21 +92,6 @@ struct PagedSource {         // (b, t, h, :) strided, tokens mapped onto 16-toke
     const int r = (int)tile / H;
     c.pg = r % tiles_per_seq;
     c.b = r / tiles_per_seq;
-    return c;
-  }
-  // the same through the index of the pages that exist: the sequence is found with one comparison per 64 sequences
-  __device__ Coord coord(int64_t tile, const int* cum, int lane) const {
-    Coord c;
-    c.h = (int)tile % H;
-    const int page = (int)tile / H;
-    int b = 0;
-    for (int b0 = 0; b0 < B; b0 += 64) {
-      const uint64_t below = __builtin_amdgcn_ballot_w64(b0 + lane < B && cum[b0 + lane + 1] <= page);
-      b += __builtin_popcountll(below);
-      if (below != ~0ull) break;
-    }
-    c.b = min(b, B - 1);
-    c.pg = page - __builtin_amdgcn_readfirstlane(cum[c.b]);
     return c;
   }
   __device__ void next(Coord& c) const {
@@ -210,6 +159,61 @@ struct PagedSource {         // (b, t, h, :) strided, tokens mapped onto 16-toke
   }
   __device__ bool locate(int tile, int slot, int64_t& elem_off) const {
     return slot_off(tile_ref(tile), slot, elem_off);
+  }
+};
+
+// Runs of different lengths (run_len): the launch is sized for B runs of T tokens, most of which a ragged batch
+// does not have.  Here the tiles are numbered over the pages that the runs really touch; a workgroup
+// builds the index of them (first page of every sequence, page_index) in its LDS from start_pos and run_len.  A type of its own, so that the other
+// calls - the page write of a decode step, whose code comes from memory every time - carry none of it.
+struct RaggedSource : PagedSource {
+  static constexpr int MAX_COMPACT = 1024;     // sequences
+  __device__ int run_pages(int b) const {
+    const int s0 = start_pos ? start_pos[b] : 0, n = min(run_len[b], T);
+    return n > 0 ? (s0 % TILE + n + TILE - 1) / TILE : 0;
+  }
+  // cum[b] = pages of the sequences before b, b = 0 .. B; called by all NT threads of the workgroup (with a barrier)
+  template <int NT>
+  __device__ void page_index(int* cum, int* scratch, int tid) const {
+    constexpr int PER = MAX_COMPACT / NT;
+    int n[PER], sum = 0;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      n[k] = tid * PER + k < B ? run_pages(tid * PER + k) : 0;
+      sum += n[k];
+    }
+    int incl = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int up = __shfl_up(incl, o, 64);
+      incl += (tid & 63) >= o ? up : 0;
+    }
+    if ((tid & 63) == 63) scratch[tid >> 6] = incl;
+    __syncthreads();
+    int at = incl - sum;
+    for (int w = 0; w < (tid >> 6); ++w) at += scratch[w];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      if (tid * PER + k <= B) cum[tid * PER + k] = at;
+      at += n[k];
+    }
+    if (tid == NT - 1 && B == MAX_COMPACT) cum[B] = at;
+    __syncthreads();
+  }
+  // coordinates of a tile through the index of the pages that exist: the sequence is found with one comparison per 64 sequences
+  __device__ Coord coord(int64_t tile, const int* cum, int lane) const {
+    Coord c;
+    c.h = (int)tile % H;
+    const int page = (int)tile / H;
+    int b = 0;
+    for (int b0 = 0; b0 < B; b0 += 64) {
+      const uint64_t below = __builtin_amdgcn_ballot_w64(b0 + lane < B && cum[b0 + lane + 1] <= page);
+      b += __builtin_popcountll(below);
+      if (below != ~0ull) break;
+    }
+    c.b = min(b, B - 1);
+    c.pg = page - __builtin_amdgcn_readfirstlane(cum[c.b]);
+    return c;
   }
 };
 

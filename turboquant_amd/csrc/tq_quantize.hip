@@ -382,7 +382,7 @@ value_chunk_kernel(const void* __restrict__ v, Source src, int d, int gs, Sink s
   // single existing slot may lie beyond it, and then nothing is stored anyway)
   int64_t page = 0;
   int head = 0;
-  if constexpr (std::is_same<Source, PagedSource>::value) {
+  if constexpr (std::is_base_of<PagedSource, Source>::value) {
     PagedSource::Coord c[1] = {src.coord(tile)};
     TileAddr ta1[1];
     int lpage[1];
@@ -976,7 +976,7 @@ extern "C" int tq_append_kv_ragged(const void* k, const void* v, int dtype, int 
   PagedSource src{B, T_max, H, tiles_per_seq, 0, stride_t, stride_h, start_pos};
   src.run_len = run_len;
   src.row0 = row0;
-  src.compact = B > 1 && B <= PagedSource::MAX_COMPACT;
+  src.compact = B > 1 && B <= RaggedSource::MAX_COMPACT;
   return append_runs(k, v, dtype, src, block_table, max_pages, layer, layout, pool, num_pages, stream);
 }
 
@@ -999,7 +999,7 @@ extern "C" int tq_append_kv_from_blocks(const void* k_cache, const void* v_cache
   src.src_stride = src_stride;
   src.stride_blk = stride_blk;
   src.run_len = run_len;
-  src.compact = run_len && B > 1 && B <= PagedSource::MAX_COMPACT;
+  src.compact = run_len && B > 1 && B <= RaggedSource::MAX_COMPACT;
   return append_runs(k_cache, v_cache, dtype, src, block_table, max_pages, layer, layout, pool, num_pages, stream);
 }
 

@@ -284,10 +284,10 @@ struct XStage {
     const int64_t first = tile0 < n_tiles ? tile0 : 0;
 #pragma unroll
     for (int m = 0; m < Gm::MT; ++m) live[m] = m < ML && tile0 + m < n_tiles;
-    if constexpr (std::is_same<Source, PagedSource>::value) {
+    if constexpr (std::is_base_of<PagedSource, Source>::value) {
       PagedSource::Coord c[Gm::MT];
       int lpage[Gm::MT];
-      if (src.compact) {
+      if constexpr (std::is_same<Source, RaggedSource>::value) {
 #pragma unroll
         for (int m = 0; m < Gm::MT; ++m) c[m] = src.coord(m < ML && live[m] ? first + m : first, cum, lane);
       } else {
@@ -397,11 +397,9 @@ key_mfma_kernel(const void* __restrict__ x, Source src, tq_layer ly, Sink sink, 
   // the LDS), so that a workgroup computes no empty ones and the live ones are dealt out evenly.  Nine prompts of
   // 17 .. 4099 tokens, 2 KV heads of 256 (a quarter of the 4644 tiles exist): call 154.6 -> 62.5 us.
   int* cum = (int*)(smem + Sm::bytes);
-  if constexpr (std::is_same<Source, PagedSource>::value) {
-    if (src.compact) {
-      src.template page_index<KQ_THREADS>(cum, cum + src.B + 1, tid0);
-      n_tiles = (int64_t)__builtin_amdgcn_readfirstlane(cum[src.B]) * src.H;
-    }
+  if constexpr (std::is_same<Source, RaggedSource>::value) {
+    src.template page_index<KQ_THREADS>(cum, cum + src.B + 1, tid0);
+    n_tiles = (int64_t)__builtin_amdgcn_readfirstlane(cum[src.B]) * src.H;
   }
   const int64_t n_groups = (n_tiles + ML - 1) / ML;             // a group = the TT vectors of one pass
   if (blockIdx.x >= n_groups) return;
@@ -822,9 +820,8 @@ static int launch_dt_d(const void* x, const Source& src, const tq_layer& ly, con
   }
   auto kern = key_mfma_kernel<DT, D, MSE_ONLY, FX, Source, Sink, ML>;
   size_t smem = Sm::bytes;                               // + the index of the existing tiles (first pages, four partial sums)
-  if constexpr (std::is_same<Source, PagedSource>::value)
-    if (src.compact) smem += ((size_t)src.B + 1 + KQ_WAVES) * 4;
-  constexpr size_t smem_max = Sm::bytes + (PagedSource::MAX_COMPACT + 1 + KQ_WAVES) * 4;
+  if constexpr (std::is_same<Source, RaggedSource>::value) smem += ((size_t)src.B + 1 + KQ_WAVES) * 4;
+  constexpr size_t smem_max = Sm::bytes + (RaggedSource::MAX_COMPACT + 1 + KQ_WAVES) * 4;
   static std::atomic<uint64_t> configured{0};           // per instantiation, one bit per device; the attribute is sticky
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return TQ_EINVAL;
@@ -864,6 +861,13 @@ int launch_key_mfma(const void* x, int dtype, const Source& src, const tq_layer&
   if (ly.mse_bits < 1 || ly.mse_bits > 4) return TQ_EUNSUPPORTED;
   if (!aligned_for_chunks(x, dtype, src) || !sink_ok(sink, mse_only)) return TQ_EUNSUPPORTED;
   constexpr bool paged = std::is_same<Sink, KeyPagedSink>::value;     // pages always hold the full code
+  if constexpr (std::is_same<Source, PagedSource>::value) {
+    if (src.compact) {
+      RaggedSource ragged;
+      static_cast<PagedSource&>(ragged) = src;
+      return launch_key_mfma<RaggedSource, Sink>(x, dtype, ragged, ly, sink, mse_only, tiles, st);
+    }
+  }
   if (paged && mse_only) return TQ_EUNSUPPORTED;
   // head_dim 128 with the fp6 digits of Pi^T and a codebook whose Walsh expansion has single-bit terms only:
   // the centroid contraction on the block-scaled MFMA

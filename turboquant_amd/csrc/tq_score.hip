@@ -202,11 +202,16 @@ __global__ void __launch_bounds__(PREP_COLS * PREP_SLICES)
 prep_query_kernel(const void* __restrict__ q, int G, int gpw, int64_t n_rows, int g_tot, tq_layer ly, float sm_scale,
                   float* __restrict__ q_rot, float* __restrict__ q_sk, float* __restrict__ q_stat,
                   uint32_t* __restrict__ qa_pack, unsigned long long* __restrict__ arrivals, int head_rows, int n_units,
-                  int n_prep, PagePrefetch pf) {
+                  int n_prep, PagePrefetch pf, SplitPlan sp) {
   extern __shared__ __align__(16) float sm[];
+  // the schedule of the page kernel's workgroups in front
+  if (sp.items && blockIdx.x < SCHED_FRONT) {
+    if (blockIdx.x == 0) schedule_splits_body<PREP_COLS * PREP_SLICES>(sp, threadIdx.x, (int*)sm);
+    return;
+  }
   // the preparation workgroups first (unit fastest, as a two-dimensional grid would order them), then the
   // workgroups that read the page kernel's first pages ahead of it
-  const int id = blockIdx.x;
+  const int id = blockIdx.x - (sp.items ? SCHED_FRONT : 0);
   if (id < n_prep)
     prep_query_body<PER, DT, PACKED>(q, G, gpw, n_rows, g_tot, ly, sm_scale, q_rot, q_sk, q_stat, qa_pack, arrivals, head_rows,
                                      id % n_units, id / n_units, sm);
@@ -221,9 +226,13 @@ template <int D, bool WW>
 __global__ void __launch_bounds__(PREP_MFMA_THREADS)
 prep_mfma_kernel(const uint16_t* __restrict__ q, int G, int64_t n_rows, tq_layer ly, float sm_scale,
                  float* __restrict__ q_stat, uint32_t* __restrict__ qa_pack, unsigned long long* __restrict__ arrivals,
-                 int head_rows, int n_tiles, int n_prep, PagePrefetch pf) {
+                 int head_rows, int n_tiles, int n_prep, PagePrefetch pf, SplitPlan sp) {
   extern __shared__ __align__(16) float sm[];
-  const int id = blockIdx.x;
+  if (sp.items && blockIdx.x < SCHED_FRONT) {
+    if (blockIdx.x == 0) schedule_splits_body<PREP_MFMA_THREADS>(sp, threadIdx.x, (int*)sm);
+    return;
+  }
+  const int id = blockIdx.x - (sp.items ? SCHED_FRONT : 0);
   if (id < n_prep)
     prep_mfma_body<D, WW>(q, G, n_rows, ly, sm_scale, q_stat, qa_pack, arrivals, head_rows, id % n_tiles, id / n_tiles, sm);
   else
@@ -550,7 +559,8 @@ bool rotate_on_matrix_cores(const void* q, int dtype, int64_t rows, const tq_lay
 // cores), not the fp32 rotated / sketched queries
 int launch_rotate_query(const void* q, int dtype, int64_t rows, const tq_layer* layer, float* q_rot, float* q_sk,
                         float* q_stat, uint32_t* qa_pack, int G, float sm_scale, hipStream_t st, bool q_rot_unused,
-                        unsigned long long* arrivals, const PagePrefetch* prefetch, int g_tot, const WidePack* wide) {
+                        unsigned long long* arrivals, const PagePrefetch* prefetch, int g_tot, const WidePack* wide,
+                        const SplitPlan& plan) {
   const int d = layer->d;
   if (qa_pack) {       // operands of the matrix-core decode kernel wanted
     // g_tot: query heads per KV head when its groups of G are unequal (0: the rows are whole groups of G)
@@ -573,21 +583,23 @@ int launch_rotate_query(const void* q, int dtype, int64_t rows, const tq_layer* 
       const int n_mprep = ww ? n_tiles : n_tiles * (d / 32);
       PagePrefetch pf;
       if (prefetch && prefetch->blocks > 0 && prefetch->n_wg > 0 && n_mprep <= 2 * device_compute_units()) pf = *prefetch;
-      pf.front = n_mprep;
-      const dim3 grid((unsigned)(n_mprep + (pf.blocks > 0 ? pf.n_wg : 0))), block(PREP_MFMA_THREADS);
-      const size_t smem = (size_t)prep_mfma_smem_floats() * sizeof(float) * (ww ? 4 : 1);
+      const int n_sched = plan.items ? SCHED_FRONT : 0;
+      pf.front = n_mprep + n_sched;
+      const dim3 grid((unsigned)(n_sched + n_mprep + (pf.blocks > 0 ? pf.n_wg : 0))), block(PREP_MFMA_THREADS);
+      size_t smem = (size_t)prep_mfma_smem_floats() * sizeof(float) * (ww ? 4 : 1);
+      if (n_sched && smem < SCHED_SMEM_INTS * sizeof(int)) smem = SCHED_SMEM_INTS * sizeof(int);
       if (d == 128 && ww)
         prep_mfma_kernel<128, true><<<grid, block, smem, st>>>((const uint16_t*)q, G, rows, *layer, sm_scale, q_stat, qa_pack,
-                                                               arrivals, head_rows, n_tiles, n_mprep, pf);
+                                                               arrivals, head_rows, n_tiles, n_mprep, pf, plan);
       else if (d == 128)
         prep_mfma_kernel<128, false><<<grid, block, smem, st>>>((const uint16_t*)q, G, rows, *layer, sm_scale, q_stat, qa_pack,
-                                                                arrivals, head_rows, n_tiles, n_mprep, pf);
+                                                                arrivals, head_rows, n_tiles, n_mprep, pf, plan);
       else if (ww)
         prep_mfma_kernel<256, true><<<grid, block, smem, st>>>((const uint16_t*)q, G, rows, *layer, sm_scale, q_stat, qa_pack,
-                                                               arrivals, head_rows, n_tiles, n_mprep, pf);
+                                                               arrivals, head_rows, n_tiles, n_mprep, pf, plan);
       else
         prep_mfma_kernel<256, false><<<grid, block, smem, st>>>((const uint16_t*)q, G, rows, *layer, sm_scale, q_stat, qa_pack,
-                                                                arrivals, head_rows, n_tiles, n_mprep, pf);
+                                                                arrivals, head_rows, n_tiles, n_mprep, pf, plan);
       hipError_t e = hipGetLastError();
       return e == hipSuccess ? TQ_OK : (int)e;
     }
@@ -603,16 +615,18 @@ int launch_rotate_query(const void* q, int dtype, int64_t rows, const tq_layer* 
     // (a preparation that already fills the card - hundreds of sequences - gains nothing from more workgroups:
     // 64 x 2048 tokens at 32 q / 8 KV heads measured 44.6 -> 46.3 us per step with them)
     if (prefetch && prefetch->blocks > 0 && prefetch->n_wg > 0 && n_prep <= 2 * device_compute_units()) pf = *prefetch;
-    pf.front = n_prep;
-    const dim3 grid((unsigned)(n_prep + (pf.blocks > 0 ? pf.n_wg : 0))), block(PREP_COLS * PREP_SLICES);
+    const int n_sched = plan.items ? SCHED_FRONT : 0;
+    if (n_sched && smem < SCHED_SMEM_INTS * sizeof(int)) smem = SCHED_SMEM_INTS * sizeof(int);
+    pf.front = n_prep + n_sched;
+    const dim3 grid((unsigned)(n_sched + n_prep + (pf.blocks > 0 ? pf.n_wg : 0))), block(PREP_COLS * PREP_SLICES);
 #define TQ_PREP(PER, DT)                                                                                               \
   {                                                                                                                    \
     if (gpw > 1)                                                                                                       \
       prep_query_kernel<PER, DT, true><<<grid, block, smem, st>>>(q, G, gpw, rows, g_tot, *layer, sm_scale, q_rot, q_sk, q_stat, \
-                                                                  qa_pack, arrivals, head_rows, n_units, n_prep, pf);              \
+                                                                  qa_pack, arrivals, head_rows, n_units, n_prep, pf, plan);              \
     else                                                                                                               \
       prep_query_kernel<PER, DT, false><<<grid, block, smem, st>>>(q, G, gpw, rows, g_tot, *layer, sm_scale, q_rot, q_sk, q_stat, \
-                                                                   qa_pack, arrivals, head_rows, n_units, n_prep, pf);             \
+                                                                   qa_pack, arrivals, head_rows, n_units, n_prep, pf, plan);             \
   }
 #define TQ_PREP_DT(PER)                              \
   {                                                  \
@@ -703,7 +717,7 @@ extern "C" int tq_rotate_query(const void* q, int dtype, int64_t rows, const tq_
   if (!q || !q_rot || !q_sk) return TQ_ENULL;
   if (rows < 0 || dtype < TQ_F32 || dtype > TQ_BF16) return TQ_EINVAL;
   if (rows == 0) return TQ_OK;
-  return launch_rotate_query(q, dtype, rows, layer, q_rot, q_sk, nullptr, nullptr, 1, 0.0f, (hipStream_t)stream, false, nullptr, nullptr, 0, nullptr);
+  return launch_rotate_query(q, dtype, rows, layer, q_rot, q_sk, nullptr, nullptr, 1, 0.0f, (hipStream_t)stream, false, nullptr, nullptr, 0, nullptr, SplitPlan{});
 }
 
 extern "C" int tq_score(const void* q, int dtype, int64_t batch, int64_t n_q, const uint8_t* idx, const uint8_t* signs,

@@ -251,6 +251,8 @@ class PagedKVPool:
             if max_len is None:
                 max_len = (bt.shape[-1]) * PAGE_TOKENS
             n_split = self.default_splits(B, max_len, Hq)
+            if workspace is None and not static_scratch and stages == 7:
+                n_split = -n_split             # that many workgroups per sequence on average, dealt out by length
         if static_scratch:
             if workspace is not None or stages != 7:
                 raise ValueError("static_scratch takes no workspace and runs all stages")
@@ -331,6 +333,8 @@ class PagedKVPool:
             if max_len is None:
                 max_len = (bt.shape[-1]) * PAGE_TOKENS
             n_split = self.default_splits(B, max_len, Hq)
+            if workspace is None:
+                n_split = -n_split             # that many workgroups per sequence on average, dealt out by length
         if workspace is None:
             workspace = self.workspace(B, Hq, n_split)
         if out is None:
