@@ -70,10 +70,10 @@ typedef struct tq_layer {
    * raw bf16 bit patterns, 3*d*d each, stored in the order the kernel loads its MFMA
    * operands: element (row, col) of term t sits at
    *   ((((t*(d/16) + row/16)*(d/32) + col/32)*4 + (col%32)/8)*16 + row%16)*8 + col%8.
-   * ST_split (the transpose of S) serves the de-quantiser.  NULL selects the vector-ALU
-   * kernels.  At the head sizes of the wide-head decode kernel (320 ... 704 in steps of 64)
-   * Pi_split and S_split alone serve the decode step's query rotation (bf16 / fp16 queries); the
-   * transposes may stay NULL there.                                                    */
+   * ST_split (the transpose of S) serves the de-quantiser of head_dim 128 / 256 and may stay NULL
+   * elsewhere.  NULL selects the vector-ALU kernels.  At the head sizes of the wide-head decode
+   * kernel (320 ... 704 in steps of 64) Pi_split and S_split also serve the decode step's query
+   * rotation (bf16 / fp16 queries).                                                     */
   const uint16_t *Pi_split, *PiT_split, *S_split, *ST_split;
   /* Optional constants of the fused query-preparation kernel of the decode path:
    * Pi_colsum[i] = sum_j Pi[j][i], S_colsum[i] = sum_j S[j][i] (d floats each) and the

@@ -95,3 +95,48 @@ def test_shares_by_length_give_what_equal_shares_give(gpu, d, kb, G, H, B, ring)
     assert float(((a - b).abs() / scale).max()) <= 2.0 ** -5 and float((a - b).norm() / b.norm()) <= 6e-3
     if B > 4:
         assert ring or not a[1].any()                    # an empty sequence
+
+
+# every count of column tiles per wavefront, 1 .. 4 bits, groups of one tile (up to a tile per compute unit) and of several, and
+# one tile more and less than that
+@pytest.mark.parametrize("d,key_bits,vb,dtype", [(64, 3, 2, torch.bfloat16), (192, 2, 4, torch.float16), (320, 5, 2, torch.bfloat16),
+                                                 (448, 3, 4, torch.float32), (576, 4, 4, torch.bfloat16), (640, 4, 2, torch.float16),
+                                                 (704, 5, 4, torch.bfloat16), (768, 3, 4, torch.bfloat16)])
+@pytest.mark.parametrize("tokens", [1, 33, 4096, 4111])
+def test_appends_at_other_head_sizes_on_both_quantisers(gpu, d, key_bits, vb, dtype, tokens):
+    """Rows on a 16-byte boundary go to the matrix-core key quantiser and the chunked value kernel, the same rows one element
+    further into a buffer to the vector-ALU kernels: values and scales byte for byte; an index or a sign may flip where an
+    fp32 sum meets a threshold (and a flipped index changes a tenth of its vector's signs): 1e-4 of the codes; norms are
+    sums of d <= 768 squares in another order, 2^-21."""
+    g = torch.Generator(device=gpu).manual_seed(d + tokens)
+    tq = TurboQuantProd(d, bits=key_bits, device=gpu)
+    pages = -(-tokens // 16) + 1
+    table = torch.arange(pages, dtype=torch.int32, device=gpu)[None]
+    start = _i32([5], gpu)
+    _say(f"append d={d} bits={key_bits}/{vb} {dtype} tokens={tokens}")
+    x = torch.randn(2, 1, tokens, 1, d, generator=g, device=gpu).to(dtype)
+    x[0, 0, tokens // 2] = 0
+    got = []
+    for pad in (0, 1):
+        buf = torch.zeros(2 * tokens * d + 16, dtype=dtype, device=gpu)
+        rows = buf[pad:pad + 2 * tokens * d].view(2, 1, tokens, 1, d)
+        rows.copy_(x)
+        pool = PagedKVPool(tq, 1, pages, value_bits=vb, value_group_size=32, dtype=dtype, device=gpu)
+        pool.append(rows[0], rows[1], table, start_pos=start)
+        got.append((pool, pool.export_flat(table[0], tokens + 5)))
+    torch.cuda.synchronize()
+    (pa, a), (pb, b) = got
+    L = pa.layout
+    assert torch.equal(pa.data[..., L.off_vdata:], pb.data[..., L.off_vdata:])
+    codes = tokens * d
+    assert int((a[0] != b[0]).sum()) <= max(1, 1e-4 * codes)
+    assert int(sum(((a[1] ^ b[1]) >> s & 1).sum() for s in range(8))) <= max(d // 4, 2e-4 * codes)
+    norm_tol = {torch.float32: 2.0 ** -21, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}[dtype]
+    assert torch.allclose(a[2].float(), b[2].float(), rtol=norm_tol, atol=0)
+    # (a 16-bit norm whose 32-bit value meets a rounding tie comes out a step apart, one in a few thousand; the unit vector and
+    # the residual, which is taken from it, move with it)
+    apart = ~torch.isclose(a[2].float(), b[2].float(), rtol=2.0 ** -21, atol=0)
+    flipped = (a[0] != b[0]).any(-1)
+    assert int(apart.sum()) <= max(1, 2e-3 * tokens) and int(flipped.sum()) <= max(1, 3e-3 * tokens)
+    assert torch.allclose(a[3][~flipped & ~apart], b[3][~flipped & ~apart], rtol=1e-5, atol=1e-6)
+    assert int((a[0] != 0).sum()) > 0

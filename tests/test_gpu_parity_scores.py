@@ -138,7 +138,7 @@ def test_config5_layer_at_full_size_against_the_oracle(gpu):
 
 @pytest.mark.parametrize("d,key_bits,dtype", [(576, 4, torch.bfloat16), (576, 3, torch.float32), (192, 4, torch.float16)])
 def test_wide_head_quantiser_against_the_oracle(gpu, d, key_bits, dtype):
-    """Head sizes without a matrix-core quantiser (the fp32 vector-ALU kernel): 576 with 4-bit keys is the shape
+    """Head sizes other than 128 / 256 (the matrix-core quantiser with a run-time size): 576 with 4-bit keys is the shape
     the reference ships a codebook for (codebook_d576_b3.json; integration/vllm.py:378-379 sizes a layer from
     kv_lora_rank).  Bytes against the oracle on the same Pi / S (quantizer.py:231-257): a coordinate that
     sits on a threshold may flip with the fp32 summation order, bounded at 1e-4 per coordinate; norms and

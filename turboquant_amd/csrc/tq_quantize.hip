@@ -354,18 +354,21 @@ __device__ __forceinline__ void round_pairs(const float (&in)[8], float sub, flo
   }
 }
 
-// Faster value kernel for 16-bit inputs, 2/4-bit codes and head_dim 64 / 128 / 256: a thread owns 8
-// consecutive channels of one token (one 16-byte load), a group's minimum / maximum meet through
-// cross-lane exchanges, and the codes pass through LDS only to be transposed into the page's
-// per-channel fields.  Arithmetic and rounding are those of value_tile_kernel.
+// Faster value kernel for 16-bit inputs and 2/4-bit codes: a thread owns 8 consecutive channels of one token (one
+// 16-byte load), a group's minimum / maximum meet through cross-lane exchanges, and the codes pass through LDS only to
+// be transposed into the page's per-channel fields.  Arithmetic and rounding are those of value_tile_kernel.
+// A workgroup takes one tile's `slab` channels (64, 128 or 256: whole tokens in a row of 16 lanes); head sizes that are
+// not one of these are slabs side by side in the grid's second dimension (a group never crosses a slab).
+// Bound by memory: 8192 vectors of 576, 4-bit codes, 9.4 MB in: value_tile_kernel 17.5 us, nine slabs of 64 7.8 us.
 template <int DT, int VB, class Source, class Sink>
 __global__ void __launch_bounds__(512)
-value_chunk_kernel(const void* __restrict__ v, Source src, int d, int gs, Sink sink) {
+value_chunk_kernel(const void* __restrict__ v, Source src, int d, int slab, int gs, Sink sink) {
   using E = Elem<DT>;
   static_assert(DT != TQ_F32, "16-bit inputs");
   const int tid = threadIdx.x, tile = blockIdx.x;
-  const int cpt = d >> 3;                          // chunks (threads) per token
-  const int t = tid >> (31 - __builtin_clz(cpt)), ck = tid & (cpt - 1);     // token slot, chunk (head_dim 64 / 128 / 256)
+  const int cpt = slab >> 3;                       // chunks (threads) per token
+  const int c0 = blockIdx.y * slab;                // first channel
+  const int t = tid >> (31 - __builtin_clz(cpt)), ck = tid & (cpt - 1);     // token slot, chunk
   const int tpg = gs >> 3;                         // threads per group (power of two, <= 16)
   // a thread's 8 codes are one word of 8 * VB bits; the words of a chunk's 16 tokens lie together
   // (rows padded by 16 bytes), so that the thread that assembles half a channel field reads the
@@ -373,7 +376,7 @@ value_chunk_kernel(const void* __restrict__ v, Source src, int d, int gs, Sink s
   using CodeWord = typename std::conditional<VB == 2, uint16_t, uint32_t>::type;
   constexpr int CROW = TILE * (int)sizeof(CodeWord) + 16;      // bytes per chunk row
   extern __shared__ __align__(16) unsigned char smem[];
-  unsigned char* scode = smem;                     // [d / 8] rows of CROW bytes
+  unsigned char* scode = smem;                     // [slab / 8] rows of CROW bytes
   int* svalid = (int*)(smem + (size_t)cpt * CROW); // [TILE]
 
   // where the tile's rows are and which of its slots exist: uniform, looked up through the scalar cache
@@ -399,7 +402,7 @@ value_chunk_kernel(const void* __restrict__ v, Source src, int d, int gs, Sink s
   const int64_t off = ta.base + (int64_t)t * src.slot_stride();
   const bool page_ok = page >= 0;                    // uniform over the workgroup; false: nothing is stored
   // unconditional load (slots that do not exist read the first vector)
-  const uint4 raw = *(const uint4*)((const uint16_t*)v + (ok ? off : 0) + ck * 8);
+  const uint4 raw = *(const uint4*)((const uint16_t*)v + (ok ? off : 0) + c0 + ck * 8);
   if (ck == 0) svalid[t] = ok;
   // a tile none of whose slots exists may lie beyond the block table: leave before looking it up
   const int n_ok = __syncthreads_count(ok);
@@ -487,13 +490,13 @@ value_chunk_kernel(const void* __restrict__ v, Source src, int d, int gs, Sink s
     codes |= (uint32_t)acc << (16 * hw);
   }
   if constexpr (!std::is_same<Sink, ValFlatSink>::value) *(CodeWord*)(scode + ck * CROW + t * sizeof(CodeWord)) = (CodeWord)codes;
-  const int ng = d / gs, g = (ck * 8) / gs;
+  const int ng = d / gs, g = (c0 + ck * 8) / gs;
   const bool leader = (ck & (tpg - 1)) == 0;
 
   if constexpr (std::is_same<Sink, ValFlatSink>::value) {
     if (ok) {
       const int64_t vec = (int64_t)tile * TILE + t;
-      uint8_t* dst = sink.data + vec * (d * VB / 8) + ck * VB;           // 8 codes = VB bytes, little-end first
+      uint8_t* dst = sink.data + vec * (d * VB / 8) + (c0 / 8 + ck) * VB;           // 8 codes = VB bytes, little-end first
       if (VB == 2) *(uint16_t*)dst = (uint16_t)codes;
       else *(uint32_t*)dst = codes;
       if (leader) {
@@ -514,7 +517,7 @@ value_chunk_kernel(const void* __restrict__ v, Source src, int d, int gs, Sink s
     // every thread assembles half a field: 8 tokens of one channel (16 bits of 2-bit codes, 32 of 4-bit)
     {
       const int c = tid >> 1, half = tid & 1;
-      uint8_t* fbytes = pg + vfield_off(L, c) + half * VB;
+      uint8_t* fbytes = pg + vfield_off(L, c0 + c) + half * VB;
       const unsigned char* row = scode + (c >> 3) * CROW + half * 8 * sizeof(CodeWord);
       const int sh = (c & 7) * VB;                   // the channel's code inside a word
       uint32_t neu = 0, mask = VB == 2 ? 0xffffu : 0xffffffffu;
@@ -778,13 +781,17 @@ namespace tq {
 template <class Source, class Sink>
 int launch_key_mfma(const void* x, int dtype, const Source& src, const tq_layer& ly, const Sink& sink, int mse_only,
                     int64_t tiles, hipStream_t st);
+template <class Source, class Sink>
+int launch_key_wide(const void* x, int dtype, const Source& src, const tq_layer& ly, const Sink& sink, int mse_only,
+                    int64_t tiles, hipStream_t st);
 }
 
 template <class Source, class Sink>
 static int launch_key(const void* x, int dtype, const Source& src, const tq_layer& ly, const Sink& sink, int mse_only,
                       int64_t tiles, hipStream_t st) {
-  {  // matrix-core kernel when the layer carries split matrices and head_dim is 128 / 256
+  {  // matrix-core kernels when the layer carries split matrices: head_dim 128 / 256, and the other multiples of 64
     int rc = launch_key_mfma(x, dtype, src, ly, sink, mse_only, tiles, st);
+    if (rc == TQ_EUNSUPPORTED) rc = launch_key_wide(x, dtype, src, ly, sink, mse_only, tiles, st);
     if (rc != TQ_EUNSUPPORTED) return rc;
   }
   size_t smem = key_tile_smem(ly.d);
@@ -820,12 +827,13 @@ static bool value_chunks_aligned(const void* v, const PagedSource& s) {
 template <class Source, class Sink>
 static int launch_value(const void* v, int dtype, const Source& src, int d, int gs, int bits, const Sink& sink,
                         int64_t tiles, hipStream_t st) {
-  // 16-bit inputs with 2/4-bit codes on the usual head sizes take the chunked kernel
-  if (dtype != TQ_F32 && (bits == 2 || bits == 4) && (d == 64 || d == 128 || d == 256) && gs >= 16 && gs <= 128 &&
-      (gs & (gs - 1)) == 0 && value_chunks_aligned(v, src)) {
-    const size_t sm = (size_t)(d / 8) * (TILE * (bits == 2 ? 2 : 4) + 16) + TILE * sizeof(int);
-    const dim3 g2((unsigned)tiles), b2(TILE * d / 8);
-#define TQ_LAUNCH_VC(DT, VB) value_chunk_kernel<DT, VB, Source, Sink><<<g2, b2, sm, st>>>(v, src, d, gs, sink)
+  // 16-bit inputs with 2/4-bit codes take the chunked kernel: the widest slab of channels that divides the head
+  const int slab = d % 256 == 0 ? 256 : (d % 128 == 0 ? 128 : 64);
+  if (dtype != TQ_F32 && (bits == 2 || bits == 4) && gs >= 16 && gs <= 128 && slab % gs == 0 && (gs & (gs - 1)) == 0 &&
+      value_chunks_aligned(v, src)) {
+    const size_t sm = (size_t)(slab / 8) * (TILE * (bits == 2 ? 2 : 4) + 16) + TILE * sizeof(int);
+    const dim3 g2((unsigned)tiles, (unsigned)(d / slab)), b2(TILE * slab / 8);
+#define TQ_LAUNCH_VC(DT, VB) value_chunk_kernel<DT, VB, Source, Sink><<<g2, b2, sm, st>>>(v, src, d, slab, gs, sink)
     if (dtype == TQ_BF16) { if (bits == 2) TQ_LAUNCH_VC(TQ_BF16, 2); else TQ_LAUNCH_VC(TQ_BF16, 4); }
     else { if (bits == 2) TQ_LAUNCH_VC(TQ_F16, 2); else TQ_LAUNCH_VC(TQ_F16, 4); }
 #undef TQ_LAUNCH_VC
