@@ -55,6 +55,14 @@ def test_split_matrices_sum_exactly_and_follow_the_documented_operand_order(d):
         _ffi.split_bf16x3(torch.zeros(48, 48))
 
 
+@pytest.mark.parametrize("B", [1, 2, 3, 64, 1024, 1025])
+@pytest.mark.parametrize("n_split", [1, 2, 31, 256, 257, 512, 2048])
+def test_workspace_of_a_step_by_length_holds_the_equal_shares_it_may_fall_back_to(B, n_split):
+    lib = _ffi.lib()
+    for Hq, d in ((1, 64), (8, 128), (128, 576)):
+        assert lib.tq_decode_workspace_bytes(B, Hq, d, -n_split) >= lib.tq_decode_workspace_bytes(B, Hq, d, n_split)
+
+
 def test_argument_errors_are_reported_before_any_launch():
     lib = _ffi.lib()
     assert lib.tq_bucketize_pack(None, 4, 128, None, 2, None, None) == -3

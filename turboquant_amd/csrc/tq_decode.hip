@@ -1077,10 +1077,11 @@ extern "C" int tq_decode_page_kernel(const tq_layer* layer, const tq_page_layout
   return decode_wide_has_kernel(*layer, *layout) ? 2 : 0;
 }
 
-// Most shares of one sequence in a step whose n_split B workgroups per KV head are dealt out by length
+// Most shares of one sequence in a step whose n_split B workgroups per KV head are dealt out by length; never fewer
+// than the n_split equal shares that the step falls back to (one sequence, equal lengths, the other page kernels)
 static int sched_max_shares(int B, int n_split) {
   const int64_t most = std::min<int64_t>((int64_t)n_split * B, std::min<int64_t>((int64_t)8 * n_split, 256));
-  return (int)std::max<int64_t>(most, 16);
+  return (int)std::max<int64_t>(most, std::max(n_split, 16));
 }
 // bytes of the schedule in the workspace: items and share counts (at most 8 wavefronts on each of 512 compute units, see
 // decode_sched_items)
