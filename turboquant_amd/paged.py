@@ -218,6 +218,12 @@ class PagedKVPool:
         longest = max(1, blocks // 16)          # keep >= 4 blocks per wavefront
         return int(max(1, min(want, longest, 512)))
 
+    def _shares_by_length(self, B: int, Hq: int) -> bool:
+        """Whether the library deals a step's workgroups out by length (matrix-core kernel, several sequences, at most 1024);
+        asked for otherwise it keeps equal shares and the larger workspace goes unused (16 x 8192, 128 heads of 576:
+        482 instead of 411 MB)."""
+        return 1 < B <= 1024 and self._matrix_core_shape(Hq)
+
     def workspace(self, B: int, Hq: int, n_split: int) -> torch.Tensor:
         nbytes = _ffi.lib().tq_decode_workspace_bytes(B, Hq, self.head_dim, n_split)
         return torch.empty(nbytes // 4, dtype=torch.float32, device=self.device)
@@ -251,7 +257,7 @@ class PagedKVPool:
             if max_len is None:
                 max_len = (bt.shape[-1]) * PAGE_TOKENS
             n_split = self.default_splits(B, max_len, Hq)
-            if workspace is None and not static_scratch and stages == 7:
+            if workspace is None and not static_scratch and stages == 7 and self._shares_by_length(B, Hq):
                 n_split = -n_split             # that many workgroups per sequence on average, dealt out by length
         if static_scratch:
             if workspace is not None or stages != 7:
@@ -333,7 +339,7 @@ class PagedKVPool:
             if max_len is None:
                 max_len = (bt.shape[-1]) * PAGE_TOKENS
             n_split = self.default_splits(B, max_len, Hq)
-            if workspace is None:
+            if workspace is None and self._shares_by_length(B, Hq):
                 n_split = -n_split             # that many workgroups per sequence on average, dealt out by length
         if workspace is None:
             workspace = self.workspace(B, Hq, n_split)
