@@ -107,7 +107,7 @@ def test_appends_at_other_head_sizes_on_both_quantisers(gpu, d, key_bits, vb, dt
     """Rows on a 16-byte boundary go to the matrix-core key quantiser and the chunked value kernel, the same rows one element
     further into a buffer to the vector-ALU kernels: values and scales byte for byte; an index or a sign may flip where an
     fp32 sum meets a threshold (and a flipped index changes a tenth of its vector's signs): 1e-4 of the codes; norms are
-    sums of d <= 768 squares in another order, 2^-21."""
+    equal."""
     g = torch.Generator(device=gpu).manual_seed(d + tokens)
     tq = TurboQuantProd(d, bits=key_bits, device=gpu)
     pages = -(-tokens // 16) + 1
@@ -131,12 +131,8 @@ def test_appends_at_other_head_sizes_on_both_quantisers(gpu, d, key_bits, vb, dt
     codes = tokens * d
     assert int((a[0] != b[0]).sum()) <= max(1, 1e-4 * codes)
     assert int(sum(((a[1] ^ b[1]) >> s & 1).sum() for s in range(8))) <= max(d // 4, 2e-4 * codes)
-    norm_tol = {torch.float32: 2.0 ** -21, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}[dtype]
-    assert torch.allclose(a[2].float(), b[2].float(), rtol=norm_tol, atol=0)
-    # (a 16-bit norm whose 32-bit value meets a rounding tie comes out a step apart, one in a few thousand; the unit vector and
-    # the residual, which is taken from it, move with it)
-    apart = ~torch.isclose(a[2].float(), b[2].float(), rtol=2.0 ** -21, atol=0)
+    assert torch.equal(a[2], b[2])                       # both add the squares in one order
     flipped = (a[0] != b[0]).any(-1)
-    assert int(apart.sum()) <= max(1, 2e-3 * tokens) and int(flipped.sum()) <= max(1, 3e-3 * tokens)
-    assert torch.allclose(a[3][~flipped & ~apart], b[3][~flipped & ~apart], rtol=1e-5, atol=1e-6)
+    assert int(flipped.sum()) <= max(1, 3e-3 * tokens)
+    assert torch.allclose(a[3][~flipped], b[3][~flipped], rtol=1e-5, atol=1e-6)
     assert int((a[0] != 0).sum()) > 0

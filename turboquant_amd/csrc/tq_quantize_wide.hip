@@ -187,16 +187,24 @@ key_wide_kernel(const void* __restrict__ x, Source src, tq_layer ly, Sink sink, 
 #pragma unroll
           for (int i = 0; i < 4; ++i) xs[j][i] = ok ? xs[j][i] : 0.0f;
         }
-      // (pairwise over a chunk and over the chunks: the rounding errors of up to 48 squares do not line up)
-      float sq[JX];
+      // The squares are added in the order of the vector-ALU kernel (coordinates 64 apart in turn, then a butterfly over the
+      // 64 sums): a 16-bit norm that meets a rounding tie would else come out a step apart, and the unit vector, a handful of
+      // indices and a quarter of the signs with it.  (Rotations by 8, 4, 2, 1 lanes are the butterfly's exchanges.)
+      float sq[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int j = 0; j < JX; ++j)
-        sq[j] = j < kb_n / 2 ? (xs[j][0] * xs[j][0] + xs[j][1] * xs[j][1]) + (xs[j][2] * xs[j][2] + xs[j][3] * xs[j][3]) : 0.0f;
+        if (j < kb_n / 2) {
 #pragma unroll
-      for (int o = 1; o < JX; o <<= 1)
+          for (int i = 0; i < 4; ++i) sq[i] += xs[j][i] * xs[j][i];
+        }
 #pragma unroll
-        for (int j = 0; j + o < JX; j += 2 * o) sq[j] += sq[j + o];
-      const float ss = sum_lanes<16>(sq[0]);
+      for (int i = 0; i < 4; ++i) {
+        sq[i] += dpp_mov<0x128>(sq[i]);
+        sq[i] += dpp_mov<0x124>(sq[i]);
+        sq[i] += dpp_mov<0x122>(sq[i]);
+        sq[i] += dpp_mov<0x121>(sq[i]);
+      }
+      const float ss = (sq[0] + sq[2]) + (sq[1] + sq[3]);
       const float nrm = E::round(sqrtf(ss));
       const float den = E::round(nrm + 1e-10f);
       if (n == 0) {
