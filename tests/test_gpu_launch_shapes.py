@@ -136,3 +136,60 @@ def test_appends_at_other_head_sizes_on_both_quantisers(gpu, d, key_bits, vb, dt
     assert int(flipped.sum()) <= max(1, 3e-3 * tokens)
     assert torch.allclose(a[3][~flipped], b[3][~flipped], rtol=1e-5, atol=1e-6)
     assert int((a[0] != 0).sum()) > 0
+
+
+def _both_quantisers(gpu, quantizer, x):
+    """Codes of the same rows on a 16-byte boundary (matrix-core kernel) and one element further on (vector-ALU kernel)."""
+    codes = []
+    for pad in (0, 1):
+        buf = torch.empty(x.numel() + 16, dtype=x.dtype, device=gpu)
+        rows = buf[pad:pad + x.numel()].view(x.shape)
+        rows.copy_(x)
+        codes.append(quantizer.quantize(rows))
+    return codes
+
+
+# sizes with one to four column tiles per wavefront, one to four index bits, every input type; vectors as models make them, with a
+# few channels ten times as large, with nearly all of their length in one channel, and far from the origin
+@pytest.mark.parametrize("d,key_bits,dtype", [(64, 3, torch.bfloat16), (192, 4, torch.float16), (320, 3, torch.float32), (384, 2, torch.bfloat16),
+                                              (448, 3, torch.float16), (576, 4, torch.bfloat16), (576, 5, torch.float16), (704, 4, torch.float32),
+                                              (768, 4, torch.bfloat16), (768, 5, torch.bfloat16)])
+@pytest.mark.parametrize("values", ["plain", "outliers", "spike", "offset"])
+def test_codes_do_not_depend_on_the_quantiser_that_a_row_reaches(gpu, d, key_bits, dtype, values):
+    """The two key quantisers add their products in different orders; an index whose coordinate lies on a threshold within
+    rounding, and a sign whose projection is zero within it, must come out alike all the same: indices, signs and norms are
+    equal.  (65536 vectors of 576, 4-bit keys: two dozen indices and some thirty signs lie that near.)  The residual norm is a sum
+    of d squares in two orders, each relative error below d 2^-24."""
+    n = 65536 if d != 64 else 262144
+    g = torch.Generator(device=gpu).manual_seed(d * 7 + key_bits)
+    x = torch.randn(n, d, generator=g, device=gpu)
+    if values == "outliers":
+        x[:, torch.randperm(d, generator=g, device=gpu)[:4]] *= 10
+    elif values == "spike":
+        x *= 0.01
+        x[torch.arange(n, device=gpu), torch.randint(0, d, (n,), generator=g, device=gpu)] = 50.0
+    elif values == "offset":
+        x = torch.rand(n, d, generator=g, device=gpu) + 1
+    x = x.to(dtype)
+    x[7], x[8] = 0, x[9]
+    _say(f"codes of both quantisers d={d} bits={key_bits} {dtype} {values}")
+    a, b = _both_quantisers(gpu, TurboQuantProd(d, bits=key_bits, device=gpu), x)
+    torch.cuda.synchronize()
+    for name in ("mse_indices", "qjl_signs", "norms"):
+        assert int((getattr(a, name) != getattr(b, name)).sum()) == 0, name
+    assert torch.allclose(a.residual_norms, b.residual_norms, rtol=d * 2.0 ** -24, atol=0)
+
+
+def test_a_vector_without_a_residual_keeps_its_signs(gpu):
+    """Keys that are de-quantised and quantised again have a residual of rounding errors, so every projection is zero within
+    rounding and all signs are decided by the sums in order."""
+    d = 576
+    g = torch.Generator(device=gpu).manual_seed(5)
+    tq = TurboQuantProd(d, bits=4, device=gpu)
+    mse = tq.mse_quantizer
+    x = mse.dequantize(mse.quantize(torch.randn(96, d, generator=g, device=gpu)))
+    _say("vectors without a residual")
+    a, b = _both_quantisers(gpu, tq, x)
+    torch.cuda.synchronize()
+    for name in ("mse_indices", "qjl_signs", "norms"):
+        assert int((getattr(a, name) != getattr(b, name)).sum()) == 0, name

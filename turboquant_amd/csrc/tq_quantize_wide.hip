@@ -12,8 +12,10 @@
 // owns NPW column tiles for all vectors, and a ring of two slices per wavefront (2 x NPW x 3 KB) that is refilled while the
 // other slice is multiplied - across the ends of the contractions, so the first slices of the next matrix are
 // there when it begins.
-// 8192 vectors of 576, bf16, 4-bit keys: 411 us on the vector-ALU kernel, 92 us here (6 MB through each compute unit);
-// one token of each of 32 sequences: append 181 -> 70 us; 8192 x 64: 39 -> 24, x 320: 129 -> 49, x 704: 515 -> 155.
+// The codes are those of the vector-ALU kernel, byte for byte: what rounding could decide is summed again in its order (see
+// KW_NEAR_Y).
+// Appends of 8192 vectors of 576, bf16, 4-bit keys: 404 us on the vector-ALU kernel, 119 us here; one token of each of 32
+// sequences 181 -> 74 us; 8192 x 320: 129 -> 49, x 704: 515 -> 177.
 
 #include <atomic>
 
@@ -35,8 +37,9 @@ struct WideSmem {
     off_planes = 3 * tt * rs * 2;                              // term tiles [3][tt][rs]
     off_off = off_planes + (mb + 1) * tt * (d / 32) * 4;       // bit planes [plane][tt][d / 32]
     off_small = off_off + tt * 8;                              // element offset of every vector
-    // norm[tt], residual norm[tt], partial sums[waves][tt], validity[tt], thresholds[16], centroid terms[16] (8 bytes each)
-    bytes = off_small + tt * (3 + waves) * 4 + 16 * 4 + 16 * 8;
+    // norm[tt], residual norm[tt], partial sums[waves][tt], validity[tt], thresholds between -inf and +inf[18], centroid
+    // terms[16] (8 bytes each), vectors with a projection near zero[2]
+    bytes = off_small + tt * (3 + waves) * 4 + 18 * 4 + 16 * 8 + 2 * 4;
   }
 };
 
@@ -57,44 +60,153 @@ __device__ __forceinline__ void load_wide_slice(const uint16_t* m_terms, int ct0
     }
 }
 
-// out[t][n] = sum_k A[t][k] M[n][k] for the wavefront's column tiles; the ring holds slices 0 and 1 of M on entry and
-// of m_next on return.  acc[m][c][i] = out[16 m + (lane & 15)][16 (ct0 + c) + 4 (lane >> 4) + i].
+template <int NPW>
+__device__ __forceinline__ void fill_ring(const uint16_t* m_terms, int ct0, int tiles, int kb_n, int lane, WideRing<NPW>& ring) {
+  load_wide_slice<NPW>(m_terms, ct0, tiles, kb_n, 0, lane * 16, ring.b[0]);
+  load_wide_slice<NPW>(m_terms, ct0, tiles, kb_n, 1, lane * 16, ring.b[1]);
+}
+
+// One slice of a contraction for the wavefront's column tiles
 template <int NPW, int MT, int NA>
+__device__ __forceinline__ void multiply_slice(const uint16_t* a_lane, int rs, int kblk, const u32x4 (&b)[NPW][3], f32x4 (&acc)[MT][NPW]) {
+#pragma unroll
+  for (int a = 0; a < NA; ++a) {
+    u32x4 av[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) av[m] = *(const u32x4*)(a_lane + (a * 16 * MT + 16 * m) * rs + 32 * kblk);
+#pragma unroll
+    for (int t = 0; t < 3; ++t)
+      if (a + t <= 2) {
+#pragma unroll
+        for (int c = 0; c < NPW; ++c)                           // consecutive MFMAs go to different accumulators
+#pragma unroll
+          for (int m = 0; m < MT; ++m) acc[m][c] = mfma_bf16(b[c][t], av[m], acc[m][c]);
+      }
+  }
+}
+
+// out[t][n] = sum_k A[t][k] M[n][k] for the wavefront's column tiles; the ring holds slices 0 and 1 of M on entry and, if
+// NEXT, of m_next on return.  acc[m][c][i] = out[16 m + (lane & 15)][16 (ct0 + c) + 4 (lane >> 4) + i].
+template <int NPW, int MT, int NA, bool NEXT>
 __device__ __forceinline__ void contract_wide(const uint16_t* a_terms, int rs, const uint16_t* m_terms, const uint16_t* m_next,
                                               int ct0, int tiles, int kb_n, int lane, WideRing<NPW>& ring, f32x4 (&acc)[MT][NPW]) {
-  constexpr int TT = 16 * MT;
-  const uint32_t lane_off = lane * 16;
   const uint16_t* a_lane = a_terms + (lane & 15) * rs + 8 * (lane >> 4);
 #pragma unroll
   for (int m = 0; m < MT; ++m)
 #pragma unroll
     for (int c = 0; c < NPW; ++c) acc[m][c] = f32x4{0, 0, 0, 0};
 #pragma unroll 1
-  for (int k2 = 0; k2 < kb_n; k2 += 2) {                        // (d is a multiple of 64: an even number of slices)
+  for (int k2 = 0; k2 < kb_n - (NEXT ? 0 : 2); k2 += 2) {       // (d is a multiple of 64: an even number of slices)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-#pragma unroll
-      for (int a = 0; a < NA; ++a) {
-        u32x4 av[MT];
-#pragma unroll
-        for (int m = 0; m < MT; ++m) av[m] = *(const u32x4*)(a_lane + (a * TT + 16 * m) * rs + 32 * (k2 + h));
-#pragma unroll
-        for (int b = 0; b < 3; ++b)
-          if (a + b <= 2) {
-#pragma unroll
-            for (int c = 0; c < NPW; ++c)                       // consecutive MFMAs go to different accumulators
-#pragma unroll
-              for (int m = 0; m < MT; ++m) acc[m][c] = mfma_bf16(ring.b[h][c][b], av[m], acc[m][c]);
-          }
-      }
+      multiply_slice<NPW, MT, NA>(a_lane, rs, k2 + h, ring.b[h], acc);
       const int next = k2 + h + 2;
-      load_wide_slice<NPW>(next < kb_n ? m_terms : m_next, ct0, tiles, kb_n, next < kb_n ? next : next - kb_n, lane_off, ring.b[h]);
+      const bool over = NEXT && next >= kb_n;
+      load_wide_slice<NPW>(over ? m_next : m_terms, ct0, tiles, kb_n, over ? next - kb_n : next, lane * 16, ring.b[h]);
     }
+  }
+  if constexpr (!NEXT) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) multiply_slice<NPW, MT, NA>(a_lane, rs, kb_n - 2 + h, ring.b[h], acc);
   }
 }
 
+// ---- sums in the order of the vector-ALU kernel ---------------------------------------------------------------------------
+
+// 16 consecutive numbers of a vector in the LDS: NA bf16 terms, term_stride apart (their sum, smallest first, is exact) ...
+template <int NA>
+struct TermRow {
+  const uint16_t* p;
+  int term_stride;
+  __device__ __forceinline__ void get(int j, float (&u)[16]) const {
+#pragma unroll
+    for (int a = NA - 1; a >= 0; --a)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const u32x4 v = *(const u32x4*)(p + a * term_stride + j + 8 * h);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float f = __uint_as_float((e & 1) ? v[e >> 1] & 0xffff0000u : v[e >> 1] << 16);
+          u[8 * h + e] = a == NA - 1 ? f : u[8 * h + e] + f;
+        }
+      }
+  }
+};
+// ... or fp32
+struct FloatRow {
+  const float* p;
+  __device__ __forceinline__ void get(int j, float (&u)[16]) const {
+#pragma unroll
+    for (int e = 0; e < 16; e += 4) {
+      const f32x4 v = *(const f32x4*)(p + j + e);
+      u[e] = v.x; u[e + 1] = v.y; u[e + 2] = v.z; u[e + 3] = v.w;
+    }
+  }
+};
+
+// sum = fma(u[e], m of element 16 Q + e, sum) for e = 0 .. 15 in turn; lane i of a DPP row holds elements 4 i .. 4 i + 3 and its
+// row's lanes read them through the row broadcast.  (A register that a VALU instruction wrote may be read through DPP
+// two instructions later, which the compiler does not see inside assembly: hence the s_nop.)
+template <int Q>
+__device__ __forceinline__ void ordered_steps(const float (&u)[16], const f32x4& m, float& sum) {
+#define TQ_STEP(M, U, L) "\n\tv_fmac_f32_dpp %0, %" #M ", %" #U " row_newbcast:%" #L " row_mask:0xf bank_mask:0xf"
+  asm("s_nop 1"
+      TQ_STEP(1, 5, 21) TQ_STEP(2, 6, 21) TQ_STEP(3, 7, 21) TQ_STEP(4, 8, 21)
+      TQ_STEP(1, 9, 22) TQ_STEP(2, 10, 22) TQ_STEP(3, 11, 22) TQ_STEP(4, 12, 22)
+      TQ_STEP(1, 13, 23) TQ_STEP(2, 14, 23) TQ_STEP(3, 15, 23) TQ_STEP(4, 16, 23)
+      TQ_STEP(1, 17, 24) TQ_STEP(2, 18, 24) TQ_STEP(3, 19, 24) TQ_STEP(4, 20, 24)
+      : "+v"(sum)
+      : "v"(m.x), "v"(m.y), "v"(m.z), "v"(m.w), "v"(u[0]), "v"(u[1]), "v"(u[2]), "v"(u[3]), "v"(u[4]), "v"(u[5]), "v"(u[6]),
+        "v"(u[7]), "v"(u[8]), "v"(u[9]), "v"(u[10]), "v"(u[11]), "v"(u[12]), "v"(u[13]), "v"(u[14]), "v"(u[15]),
+        "n"(4 * Q), "n"(4 * Q + 1), "n"(4 * Q + 2), "n"(4 * Q + 3));
+#undef TQ_STEP
+}
+// sum_j u[j] row[j], the products added one by one in ascending order: the bits of the vector-ALU kernel.  The 16 lanes of a DPP
+// row share one matrix row, requested three times 64 elements ahead (the fp32 matrices are in no cache), and every lane
+// has a vector of its own.  All lanes of the wavefront have to be active.
+template <class U>
+__device__ __forceinline__ float ordered_dot(const U& vec, const float* __restrict__ row, int d, int n) {
+  const f32x4* run = (const f32x4*)row + n;
+  f32x4 ahead[3];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) ahead[q] = run[min(64 * q, d - 64) / 4];
+  float sum = 0.0f;
+#pragma unroll 1
+  for (int j0 = 0; j0 < d; j0 += 64) {
+    const f32x4 cur = ahead[0];
+    ahead[0] = ahead[1];
+    ahead[1] = ahead[2];
+    ahead[2] = run[min(j0 + 192, d - 64) / 4];
+    float u[16];
+    vec.get(j0, u); ordered_steps<0>(u, cur, sum);
+    vec.get(j0 + 16, u); ordered_steps<1>(u, cur, sum);
+    vec.get(j0 + 32, u); ordered_steps<2>(u, cur, sum);
+    vec.get(j0 + 48, u); ordered_steps<3>(u, cur, sum);
+  }
+  return sum;
+}
+
+// `bits` of the first lane of this lane's DPP row that has any (`open`: the lanes that do); 0 if none has.
+__device__ __forceinline__ uint32_t leader_bits(uint32_t bits, uint64_t open, int lane) {
+  const uint32_t row = (uint32_t)(open >> (lane & 48)) & 0xffffu;
+  const uint32_t got = __shfl(bits, (lane & 48) + (row ? __builtin_ctz(row) : 0), 64);
+  return row ? got : 0u;
+}
+
+// How near to a threshold a coordinate of the unit vector, and how near to zero a projection of the residual, is decided by the
+// sums in the order of the vector-ALU kernel, so that a row gets that kernel's codes whatever its alignment and its batch: an
+// index that falls the other way takes a quarter of the vector's signs with it, and what is attended to changes.  The two orders
+// come apart by 2.1e-8 in the root mean square (coordinates; relative to the vector's length) and by 2.4e-8 (projections; relative to
+// sqrt(d) times it); the margins are eleven and five times that.  Over 65536 vectors of each of eight sizes 64 .. 768,
+// three types and four distributions (Gaussian, ten-fold channels, one spike, off-centre) no code differs, where without
+// them one index in about 3000 vectors of 576 did.  Residual norms agree to 1e-6.
+// What it costs, 8192 vectors of 576: 85.8 -> 112 us (nothing near anything 94, indices 95: a pass over fp32 Pi, 16 us, by the
+// workgroups that have a projection near zero - one group of 32 in five).
+constexpr float KW_NEAR_Y = 0x1p-22f, KW_NEAR_P = 0x1p-23f;
+constexpr int KW_REDO = 2;                 // vectors whose residual is computed again at a time (more: bound by the LDS reads)
+
 template <int DT, int NPW, int MT, class Source, class Sink>
-__global__ void __launch_bounds__(KW_MAX_WAVES * 64)
+__global__ void __launch_bounds__(KW_MAX_WAVES * 64, NPW == 1 ? 4 : 3)       // (head_dim 64: four workgroups of four wavefronts)
 key_wide_kernel(const void* __restrict__ x, Source src, tq_layer ly, Sink sink, int64_t n_tiles, int mse_only) {
   using E = Elem<DT>;
   using S = typename E::storage;
@@ -106,8 +218,7 @@ key_wide_kernel(const void* __restrict__ x, Source src, tq_layer ly, Sink sink, 
   const int tid0 = threadIdx.x, wave0 = __builtin_amdgcn_readfirstlane(tid0 >> 6);
   const int waves = blockDim.x >> 6, nthreads = blockDim.x;
   WideRing<NPW> ring;
-  load_wide_slice<NPW>(ly.Pi_split, wave0 * NPW, tiles, kb_n, 0, (tid0 & 63) * 16, ring.b[0]);
-  load_wide_slice<NPW>(ly.Pi_split, wave0 * NPW, tiles, kb_n, 1, (tid0 & 63) * 16, ring.b[1]);
+  fill_ring<NPW>(ly.Pi_split, wave0 * NPW, tiles, kb_n, tid0 & 63, ring);
 
   extern __shared__ __align__(16) unsigned char smem[];
   const WideSmem sm(d, mb, TT, waves);
@@ -120,8 +231,10 @@ key_wide_kernel(const void* __restrict__ x, Source src, tq_layer ly, Sink sink, 
   float* spart = srn + TT;
   int* svalid = (int*)(spart + waves * TT);
   float* sthr = (float*)(svalid + TT);
-  u32x2* slut = (u32x2*)(sthr + 16);                            // bf16 terms of a centroid: {t0 | t1 << 16, t2}
-  if (tid0 < n_thr) sthr[tid0] = ly.thresholds[tid0];
+  u32x2* slut = (u32x2*)(sthr + 18);                            // bf16 terms of a centroid: {t0 | t1 << 16, t2}
+  if (tid0 < n_thr) sthr[tid0 + 1] = ly.thresholds[tid0];       // (index i lies between sthr[i] and sthr[i + 1])
+  if (tid0 < 2) sthr[tid0 * (n_thr + 1)] = tid0 ? INFINITY : -INFINITY;
+  uint32_t* sopen = (uint32_t*)(slut + 16);
   if (tid0 < (1 << mb)) {
     uint32_t t[3];
     split3_pk(ly.centroids[tid0], 0.0f, t);
@@ -168,6 +281,7 @@ key_wide_kernel(const void* __restrict__ x, Source src, tq_layer ly, Sink sink, 
     int tid = tid0, wave = wave0;
     asm volatile("" : "+v"(tid), "+s"(wave));
     const int lane = tid & 63, n = lane & 15, kb = lane >> 4, ct0 = wave * NPW;
+    if (tid < 2) sopen[tid] = 0;
     // (1) norm, unit vector in the input dtype (quantizer.py:136-138) and its bf16 terms: 16 lanes per vector, which
     //     hold all of it, four coordinates per lane and chunk
 #pragma unroll 1
@@ -246,7 +360,56 @@ key_wide_kernel(const void* __restrict__ x, Source src, tq_layer ly, Sink sink, 
 
     f32x4 acc[MT][NPW];
     // (2) y = u Pi^T, bucketise: index bit planes and the centroids' bf16 terms
-    contract_wide<NPW, MT, NA1>(terms, rs, ly.Pi_split, mse_only ? ly.Pi_split : ly.PiT_split, ct0, tiles, kb_n, lane, ring, acc);
+    // (the next matrix is asked for when the indices are settled: what that takes would push its operands out of the registers)
+    contract_wide<NPW, MT, NA1, false>(terms, rs, ly.Pi_split, nullptr, ct0, tiles, kb_n, lane, ring, acc);
+    uint32_t codes[MT][NPW];                                    // four indices, a byte each
+    uint32_t near = 0;                                          // coordinates that lie on a threshold within rounding
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      const float nrm = snorm[16 * m + n];
+      const float margin = svalid[16 * m + n] ? KW_NEAR_Y * (nrm / E::round(nrm + 1e-10f)) : 0.0f;
+#pragma unroll
+      for (int c = 0; c < NPW; ++c) {
+        int idx[4] = {0, 0, 0, 0};
+#pragma unroll 1
+        for (int k = 1; k <= n_thr; ++k) {                      // searchsorted: count thresholds below y (NaN counts all)
+          const float th = sthr[k];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) idx[i] += !(acc[m][c][i] <= th);
+        }
+        codes[m][c] = idx[0] | idx[1] << 8 | idx[2] << 16 | idx[3] << 24;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float y = acc[m][c][i], lo = sthr[idx[i]], hi = sthr[idx[i] + 1];
+          near |= (uint32_t)(fminf(y - lo, hi - y) < margin) << ((m * NPW + c) * 4 + i);
+        }
+      }
+    }
+    // Those coordinates (one vector in a hundred has one): a DPP row of lanes works on one matrix row at a time, for all of
+    // its 16 vectors.
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(near != 0) != 0, 0))
+    while (const uint64_t open = __builtin_amdgcn_ballot_w64(near != 0)) {
+      const uint32_t first = leader_bits(near, open, lane);
+      const int bit = first ? __builtin_ctz(first) : 0, i = bit & 3, mc = bit >> 2, m = mc / NPW, c = mc % NPW;
+      const float y = ordered_dot(TermRow<NA1>{terms + (16 * m + n) * rs, TT * rs},
+                                  ly.Pi + (size_t)(16 * (ct0 + c) + 4 * kb + i) * d, d, n);
+      uint32_t code = 0;
+#pragma unroll 1
+      for (int k = 1; k <= n_thr; ++k) code += !(y <= sthr[k]);
+      const bool mine = near >> bit & 1;
+      near &= ~((uint32_t)mine << bit);
+#pragma unroll
+      for (int o = 0; o < MT * NPW; ++o) {
+        const bool here = mine && o == mc;
+        const uint32_t old = codes[o / NPW][o % NPW];
+        codes[o / NPW][o % NPW] = here ? (old & ~(0xffu << 8 * i)) | code << 8 * i : old;
+        if constexpr (!paged) {
+#pragma unroll
+          for (int i2 = 0; i2 < 4; ++i2) acc[o / NPW][o % NPW][i2] = here && i2 == i ? y : acc[o / NPW][o % NPW][i2];
+        }
+      }
+    }
+    fill_ring<NPW>(mse_only ? ly.Pi_split : ly.PiT_split, ct0, tiles, kb_n, lane, ring);
     __syncthreads();                                            // every wavefront has read the unit-vector terms
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
@@ -257,13 +420,9 @@ key_wide_kernel(const void* __restrict__ x, Source src, tq_layer ly, Sink sink, 
         if constexpr (!paged) {
           if (sink.y_dbg && svalid[t]) *(f32x4*)(sink.y_dbg + (tile0 * TILE + t) * d + col0) = acc[m][c];
         }
-        int idx[4] = {0, 0, 0, 0};
-#pragma unroll 1
-        for (int k = 0; k < n_thr; ++k) {                       // searchsorted: count thresholds below y (NaN counts all)
-          const float th = sthr[k];
+        int idx[4];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) idx[i] += !(acc[m][c][i] <= th);
-        }
+        for (int i = 0; i < 4; ++i) idx[i] = codes[m][c] >> 8 * i & 0xff;
         // a column tile is half a plane word
 #pragma unroll 1
         for (int p = 0; p < mb; ++p) {
@@ -285,7 +444,7 @@ key_wide_kernel(const void* __restrict__ x, Source src, tq_layer ly, Sink sink, 
     __syncthreads();
     if (!mse_only) {
       // (3) x_hat = (c Pi) * norm ; r = x - x_hat ; ||r||^2 ; r as bf16 terms (quantizer.py:241-245)
-      contract_wide<NPW, MT, 3>(terms, rs, ly.PiT_split, ly.S_split, ct0, tiles, kb_n, lane, ring, acc);
+      contract_wide<NPW, MT, 3, true>(terms, rs, ly.PiT_split, ly.S_split, ct0, tiles, kb_n, lane, ring, acc);
       __syncthreads();                                          // every wavefront has read the centroid terms
 #pragma unroll
       for (int m = 0; m < MT; ++m) {
@@ -321,23 +480,103 @@ key_wide_kernel(const void* __restrict__ x, Source src, tq_layer ly, Sink sink, 
         srn[tid] = sqrtf(v);
       }
       // (4) p = r S^T ; sign bits (quantizer.py:248-249)
-      contract_wide<NPW, MT, 3>(terms, rs, ly.S_split, ly.Pi_split, ct0, tiles, kb_n, lane, ring, acc);
+      contract_wide<NPW, MT, 3, false>(terms, rs, ly.S_split, nullptr, ct0, tiles, kb_n, lane, ring, acc);
+      uint32_t near_p = 0;
+      const float near_scale = KW_NEAR_P * sqrtf((float)d);
 #pragma unroll
       for (int m = 0; m < MT; ++m) {
         const int t = 16 * m + n;
+        const float margin = svalid[t] ? near_scale * snorm[t] : 0.0f;
+        const uint32_t before = near_p;
 #pragma unroll
         for (int c = 0; c < NPW; ++c) {
           const int ct = ct0 + c;
           uint32_t v = 0;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) v |= (uint32_t)(acc[m][c][i] > 0.0f) << (4 * kb + i);
+          for (int i = 0; i < 4; ++i) {
+            v |= (uint32_t)(acc[m][c][i] > 0.0f) << (4 * kb + i);
+            near_p |= (uint32_t)(fabsf(acc[m][c][i]) < margin) << ((m * NPW + c) * 4 + i);
+          }
           v = or_over_kb(v);
           if (kb == 0) ((uint16_t*)spl)[(mb * TT + t) * (2 * W) + ct] = (uint16_t)v;
           if constexpr (!paged) {
             if (sink.p_dbg && svalid[t]) *(f32x4*)(sink.p_dbg + (tile0 * TILE + t) * d + 16 * ct + 4 * kb) = acc[m][c];
           }
         }
+        if (near_p != before) atomicOr(sopen + (t >> 5), 1u << (t & 31));
       }
+      __syncthreads();
+      // Projections that are zero within rounding: the vector's residual is computed again in the vector-ALU kernel's order,
+      // a thread per coordinate, KW_REDO vectors over one pass of Pi, then the sums over the rows of S in question.
+      // The terms are no longer needed: the numbers take their place.
+      uint64_t redo = sopen[0] | (MT > 2 ? (uint64_t)sopen[1] << 32 : 0);
+      if (__builtin_expect(redo != 0, 0))
+      do {
+        float* cbuf = (float*)smem;                             // [KW_REDO][d] centroids
+        float* rbuf = cbuf + KW_REDO * d;                       // [KW_REDO][d] residuals
+        const int t0 = __builtin_amdgcn_readfirstlane(__builtin_ctzll(redo));
+        redo &= redo - 1;
+        const int t1 = redo ? __builtin_amdgcn_readfirstlane(__builtin_ctzll(redo)) : t0;
+        redo &= redo - 1;
+        for (int j = tid; j < d; j += nthreads) {
+          int i0 = 0, i1 = 0;
+#pragma unroll 1
+          for (int p = 0; p < mb; ++p) {
+            i0 = 2 * i0 + (int)(spl[(p * TT + t0) * W + (j >> 5)] >> (j & 31) & 1);
+            i1 = 2 * i1 + (int)(spl[(p * TT + t1) * W + (j >> 5)] >> (j & 31) & 1);
+          }
+          const u32x2 e0 = slut[i0], e1 = slut[i1];             // (the terms add up exactly)
+          cbuf[j] = (__uint_as_float(e0.y << 16) + __uint_as_float(e0.x & 0xffff0000u)) + __uint_as_float(e0.x << 16);
+          cbuf[d + j] = (__uint_as_float(e1.y << 16) + __uint_as_float(e1.x & 0xffff0000u)) + __uint_as_float(e1.x << 16);
+        }
+        __syncthreads();
+        for (int j = tid; j < d; j += nthreads) {
+          float xh0 = 0.0f, xh1 = 0.0f;
+          constexpr int U = NPW == 1 ? 32 : 64;                 // rows of Pi in flight: no cache holds it
+#pragma unroll 1
+          for (int i0 = 0; i0 < d; i0 += U) {
+            float m[U];
+#pragma unroll
+            for (int i = 0; i < U; ++i) m[i] = ly.Pi[(size_t)(i0 + i) * d + j];
+#pragma unroll
+            for (int i = 0; i < U; i += 4) {
+              const f32x4 u0 = *(const f32x4*)(cbuf + i0 + i), u1 = *(const f32x4*)(cbuf + d + i0 + i);
+#pragma unroll
+              for (int k = 0; k < 4; ++k) {
+                xh0 = fmaf(u0[k], m[i + k], xh0);
+                xh1 = fmaf(u1[k], m[i + k], xh1);
+              }
+            }
+          }
+          rbuf[j] = E::load(x, soff[t0] + j) - xh0 * snorm[t0];
+          rbuf[d + j] = E::load(x, soff[t1] + j) - xh1 * snorm[t1];
+        }
+        __syncthreads();
+        uint32_t open_now = 0, second = 0;                      // this lane's open signs of these vectors, of t1
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          const uint32_t own = near_p & (((1u << (4 * NPW - 1)) * 2 - 1) << (m * NPW * 4));
+          if (16 * m + n == t0) open_now |= own;
+          else if (16 * m + n == t1) { open_now |= own; second |= own; }
+        }
+        while (const uint64_t open = __builtin_amdgcn_ballot_w64(open_now != 0)) {
+          const uint32_t first = leader_bits(open_now, open, lane);
+          const int bit = first ? __builtin_ctz(first) : 0, i = bit & 3, mc = bit >> 2, m = mc / NPW, c = mc % NPW;
+          const int col = 16 * (ct0 + c) + 4 * kb + i, t = 16 * m + n;
+          const float p = ordered_dot(FloatRow{rbuf + ((second >> bit & 1) ? d : 0)}, ly.S + (size_t)col * d, d, n);
+          if (open_now >> bit & 1) {
+            uint32_t* word = spl + (mb * TT + t) * W + (col >> 5);
+            if (p > 0.0f) atomicOr(word, 1u << (col & 31));
+            else atomicAnd(word, ~(1u << (col & 31)));
+            if constexpr (!paged) {
+              if (sink.p_dbg) sink.p_dbg[(tile0 * TILE + t) * d + col] = p;
+            }
+            open_now &= ~(1u << bit);
+          }
+        }
+        __syncthreads();                                        // the next vectors overwrite the numbers
+      } while (redo);
+      fill_ring<NPW>(ly.Pi_split, ct0, tiles, kb_n, lane, ring);
     }
     __syncthreads();
     // (5) write
