@@ -193,3 +193,43 @@ def test_a_vector_without_a_residual_keeps_its_signs(gpu):
     torch.cuda.synchronize()
     for name in ("mse_indices", "qjl_signs", "norms"):
         assert int((getattr(a, name) != getattr(b, name)).sum()) == 0, name
+
+
+# the matrix-core quantiser with a run-time size numbers ragged tiles with 256 of its 256 .. 768 threads; at head_dim 768 the index
+# of many runs leaves room for one tile per workgroup only
+@pytest.mark.parametrize("d,key_bits,B,H", [(64, 3, 65, 2), (192, 3, 130, 1), (320, 4, 257, 1), (576, 4, 65, 3), (576, 4, 1024, 1),
+                                            (704, 4, 130, 1), (768, 4, 40, 8), (768, 4, 300, 1), (768, 3, 1024, 1)])
+def test_ragged_append_of_other_head_sizes(gpu, d, key_bits, B, H):
+    """Against one append per sequence, byte for byte, and against the vector-ALU kernel (rows one element off the boundary) but for
+    the residual norms - whose last bits also tell that two kernels ran."""
+    g = torch.Generator().manual_seed(d + B)
+    runs = [int(x) for x in torch.randint(0, 40, (B,), generator=g)]
+    runs[B // 2] = 200
+    runs[0], runs[-1] = 0, 17
+    starts = [int(x) for x in torch.randint(0, 17, (B,), generator=g)]
+    rows, width = sum(runs), 15
+    row0 = [sum(runs[:b]) for b in range(B)]
+    buf = torch.randn(2 * rows * H * d + 16, generator=g).bfloat16().to(gpu)
+    k, v = buf[:2 * rows * H * d].view(2, rows, H, d)
+    off = torch.empty_like(buf)
+    ko, vo = off[1:1 + 2 * rows * H * d].view(2, rows, H, d)
+    ko.copy_(k), vo.copy_(v)
+    table = torch.randperm(B * width, generator=g).view(B, width).to(torch.int32).to(gpu)
+    tq = TurboQuantProd(d, bits=key_bits, device=gpu)
+    pa, pb, pc = (PagedKVPool(tq, H, B * width, value_bits=4, dtype=torch.bfloat16, device=gpu) for _ in range(3))
+    _say(f"ragged append d={d} bits={key_bits} B={B} H={H} rows={rows}")
+    args = _i32(row0, gpu), _i32(runs, gpu), _i32(starts, gpu), table
+    pa.append_ragged(k, v, *args, max_run=max(runs))
+    pc.append_ragged(ko, vo, *args, max_run=max(runs))
+    for b in range(B):
+        if runs[b]:
+            s = slice(row0[b], row0[b] + runs[b])
+            pb.append(k[None, s], v[None, s], table[b:b + 1], start_pos=_i32([starts[b]], gpu))
+    torch.cuda.synchronize()
+    assert torch.equal(pa.data, pb.data)
+    meta = slice(pa.layout.off_meta, pa.layout.off_meta + 8 * 16)
+    ma, mc = (p.data[..., meta].contiguous().view(torch.float32) for p in (pa, pc))
+    assert torch.equal(ma[..., 0::2], mc[..., 0::2]) and not torch.equal(ma, mc)
+    assert torch.allclose(ma, mc, rtol=d * 2.0 ** -24, atol=0)
+    pa.data[..., meta] = pc.data[..., meta]
+    assert torch.equal(pa.data, pc.data)

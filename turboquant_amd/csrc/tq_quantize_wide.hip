@@ -713,12 +713,14 @@ int launch_key_wide(const void* x, int dtype, const Source& src, const tq_layer&
   while (npw <= 4 && (ly.d / 16 % npw != 0 || ly.d / 16 / npw > KW_MAX_WAVES)) ++npw;
   if (npw > 4) return TQ_EUNSUPPORTED;
   const int cus = device_compute_units();
-  // one 16-vector tile per workgroup while every tile has a compute unit to itself: half of the MFMAs behind one another
+  // one 16-vector tile per workgroup while every tile has a compute unit to itself: half of the MFMAs behind one another; and
+  // where more do not fit the LDS (head_dim 768: 4-bit keys with the index of more than 35 ragged runs, 5-bit keys)
   const bool small = tiles <= cus;
 #define TQ_KW(DT_, NPW_, MT_)                                                                                             \
   if (dtype == DT_ && npw == NPW_) {                                                                                       \
-    if (small) return launch_wide<DT_, NPW_, 1, Source, Sink>(x, src, ly, sink, mse_only, tiles, cus, st);                 \
-    return launch_wide<DT_, NPW_, MT_, Source, Sink>(x, src, ly, sink, mse_only, tiles, cus, st);                          \
+    const int rc = small ? TQ_EUNSUPPORTED : launch_wide<DT_, NPW_, MT_, Source, Sink>(x, src, ly, sink, mse_only, tiles, cus, st); \
+    if (rc != TQ_EUNSUPPORTED) return rc;                                                                                  \
+    return launch_wide<DT_, NPW_, 1, Source, Sink>(x, src, ly, sink, mse_only, tiles, cus, st);                            \
   }
 #define TQ_KW_ALL(DT_) TQ_KW(DT_, 1, 4) TQ_KW(DT_, 2, 2) TQ_KW(DT_, 3, 2) TQ_KW(DT_, 4, 2)
   TQ_KW_ALL(TQ_BF16) TQ_KW_ALL(TQ_F16) TQ_KW_ALL(TQ_F32)
