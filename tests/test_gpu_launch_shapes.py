@@ -97,6 +97,37 @@ def test_shares_by_length_give_what_equal_shares_give(gpu, d, kb, G, H, B, ring)
         assert ring or not a[1].any()                    # an empty sequence
 
 
+def _step(pool, q, table, seq, longest, n_split, exact, ring):
+    if ring:
+        return pool.decode_attention_ring(q, table, seq, exact[0], exact[1], ring, max_len=longest, n_split=n_split)
+    return pool.decode_attention(q, table, seq, max_len=longest, n_split=n_split)
+
+
+# (head_dim, key bits, heads per KV head, KV heads, sequences, tokens): one share per sequence walked by four, two and one wavefronts
+# and by a workgroup of eight; a few shares, merged in the launch; dozens, merged by a kernel of their own; 5-bit keys
+_EQUAL = [(128, 3, 4, 8, 64, 2048), (128, 3, 4, 8, 96, 700), (128, 4, 5, 8, 128, 512), (64, 3, 4, 8, 100, 700), (128, 3, 4, 8, 192, 333),
+          (128, 3, 4, 8, 300, 200), (128, 3, 4, 8, 32, 8192), (128, 2, 4, 2, 16, 4000), (256, 3, 8, 2, 128, 2048), (256, 3, 8, 2, 4, 33000),
+          (128, 3, 4, 8, 2, 33000), (128, 5, 4, 8, 64, 700)]
+
+
+@pytest.mark.parametrize("d,kb,G,H,B,N", _EQUAL)
+@pytest.mark.parametrize("ring", [0, 40])
+def test_steps_of_equal_length_are_those_of_equal_shares(gpu, d, kb, G, H, B, N, ring):
+    """A step whose sequences are as long as one another, or nearly, gains nothing from shares by length and has to be the step with
+    that many equal shares, bit for bit: it once split sequences between wavefronts and took half as long again."""
+    pool, table, seq, dg = _ragged_pool(gpu, d, kb, 4, H, [N] * B, torch.bfloat16, B + d)
+    q = torch.randn(B, H * G, d, generator=dg, device=gpu).bfloat16()
+    exact = torch.randn(2, pool.num_pages, 16, H, d, generator=dg, device=gpu).bfloat16() if ring else None
+    n = pool.default_splits(B, N, H * G)
+    nearly = seq - torch.randint(0, max(2, N // 25), (B,), generator=dg, device=gpu).to(torch.int32)
+    nearly[0] = N
+    for name, lens in (("equal", seq), ("nearly equal", nearly)):
+        _say(f"{name} lengths d={d} kb={kb} G={G} H={H} B={B} N={N} ring={ring} splits={n}")
+        outs = [_step(pool, q, table, lens, N, k, exact, ring) for k in (None, n)]
+        torch.cuda.synchronize()
+        assert torch.equal(*outs) and bool(outs[0].any())
+
+
 # every count of column tiles per wavefront, 1 .. 4 bits, groups of one tile (up to a tile per compute unit) and of several, and
 # one tile more and less than that
 @pytest.mark.parametrize("d,key_bits,vb,dtype", [(64, 3, 2, torch.bfloat16), (192, 2, 4, torch.float16), (320, 5, 2, torch.bfloat16),

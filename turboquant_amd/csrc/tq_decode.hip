@@ -896,15 +896,11 @@ __global__ void __launch_bounds__(256)
 merge_kernel(const float* __restrict__ parts, int n_parts, int part_stride, int d, int dtype, void* __restrict__ out,
              int row_groups, const SplitItem* __restrict__ sched, const int32_t* __restrict__ n_of, int n_static,
              int rows_per_seq, int tail_part) {
-  // (n_of: parts of a scheduled step - n_of[sequence] of them, or n_static if the schedule says equal shares, and those of the exact tail from tail_part on, n_parts -
-  // tail_part in number)
-  int n_first = n_parts, skip = 0;               // part j >= n_first lies skip parts further on
-  if (n_of) {
-    const int equal = sched->n, own = n_of[blockIdx.x / rows_per_seq];
-    n_first = equal ? n_static : own;
-    skip = tail_part - n_first;
-    n_parts = n_first + n_parts - tail_part;
-  }
+  // (n_of: parts of a scheduled step - n_of[sequence] of them, or n_static if the schedule says equal shares, and those of the exact tail
+  // from tail_part on, n_parts - tail_part in number)
+  const int n_tail = n_of ? n_parts - tail_part : 0;
+  int n_first = n_of ? n_static : n_parts, skip = n_of ? tail_part - n_static : 0;      // part j >= n_first lies skip parts further on
+  n_parts = n_first + n_tail;
   auto at = [&](int j) { return (int64_t)(j < n_first ? j : j + skip); };
   extern __shared__ float s_w[];                 // [n_parts] weights, [n_parts] m, [n_parts] l, [8] scratch, [S][dw] sums
   const int64_t row = blockIdx.x;
@@ -913,25 +909,38 @@ merge_kernel(const float* __restrict__ parts, int n_parts, int part_stride, int 
   // of the launch's implicit data in front of the first accumulator loads)
   const int dw = d / row_groups, c0 = (int)blockIdx.y * dw;       // this workgroup's channels: c0 .. c0 + dw - 1
   const float* p = parts + row * part_stride * (int64_t)(d + 2);
-  float* s_m = s_w + n_parts;
-  float* s_l = s_m + n_parts;
-  float* scratch = s_l + n_parts;
-  float* s_sum = scratch + 8;
   const int np = dw >> 1;                                       // channel pairs of this workgroup
   const int S = np >= 256 ? 1 : 256 / np;                       // subsets of parts (dw is a multiple of 64)
   const int tps = 256 / S;                                      // threads per subset
   const int sub = tid / tps, pr = tid - sub * tps;
   typedef float f2 __attribute__((ext_vector_type(2)));
-  // first chunk of this thread's accumulator loads (pair pr; parts sub, sub + S, ...), clamped in range
-  f2 v[MERGE_CHUNK];
+  // first chunk of this thread's accumulator loads (pair pr; parts sub, sub + S, ...), clamped in range, and its first (m, l)
+  f2 v[MERGE_CHUNK], ml0;
+  auto request = [&]() {
 #pragma unroll
-  for (int k = 0; k < MERGE_CHUNK; ++k) {
-    const int sp = min(sub + k * S, n_parts - 1);
-    v[k] = *(const f2*)(p + at(sp) * (d + 2) + 2 + c0 + 2 * min(pr, np - 1));
+    for (int k = 0; k < MERGE_CHUNK; ++k) {
+      const int sp = min(sub + k * S, n_parts - 1);
+      v[k] = *(const f2*)(p + at(sp) * (d + 2) + 2 + c0 + 2 * min(pr, np - 1));
+    }
+    ml0 = *(const f2*)(p + at(min(tid, n_parts - 1)) * (d + 2));
+  };
+  request();                                     // (as if the shares were equal, so that a step of equal lengths does not wait for the schedule)
+  if (n_of) {
+    const int equal = sched->n, own = n_of[blockIdx.x / rows_per_seq];
+    if (!equal) {
+      n_first = own;
+      skip = tail_part - own;
+      n_parts = own + n_tail;
+      request();
+    }
   }
+  float* s_m = s_w + n_parts;
+  float* s_l = s_m + n_parts;
+  float* scratch = s_l + n_parts;
+  float* s_sum = scratch + 8;
   float mm = NEG_BIG;
   for (int sp = tid; sp < n_parts; sp += blockDim.x) {
-    const f2 ml = *(const f2*)(p + at(sp) * (d + 2));
+    const f2 ml = sp == tid ? ml0 : *(const f2*)(p + at(sp) * (d + 2));
     s_m[sp] = ml[0];
     s_l[sp] = ml[1];
     if (ml[1] > 0.0f) mm = fmaxf(mm, ml[0]);
@@ -1084,7 +1093,7 @@ static int sched_max_shares(int B, int n_split) {
   return (int)std::max<int64_t>(most, std::max(n_split, 16));
 }
 // bytes of the schedule in the workspace: items and share counts (at most 8 wavefronts on each of 512 compute units, see
-// decode_sched_items)
+// decode_sched_plan)
 static size_t sched_bytes(int B, int n_split) {
   return ((size_t)n_split * B + B + 8 * 512 + 1) * sizeof(SplitItem) + (size_t)B * sizeof(int32_t);
 }
@@ -1201,16 +1210,10 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
     // (behind everything a step with n_max equal shares keeps in the workspace)
     const uintptr_t end = (uintptr_t)workspace + tq_decode_workspace_bytes(B, Hq, d, sched_max_shares(B, n_asked));
     plan.items = (SplitItem*)((end + 31) & ~(uintptr_t)31);
-    plan.cap = decode_sched_items(d, layer->mse_bits, B, Hkv * kv_div, n_split, wide_wg);
+    decode_sched_plan(plan, d, layer->mse_bits, B, Hkv * kv_div, n_split, wide_wg);
     plan.n_of = (int32_t*)(plan.items + 1 + plan.cap);
     plan.seq_lens = seq_lens;
-    plan.B = B; plan.n_max = n_max; plan.n_static = n_split;
-    PagePrefetch shape;
-    decode_mfma_plan(shape, d, B, Hkv * kv_div, kv_div, n_split, wide_wg);
-    plan.gx = shape.gx; plan.skew16 = shape.skew16; plan.ngrp = shape.ngrp;
-    const bool by_wave = decode_sched_by_wave(d, layer->mse_bits, B, Hkv * kv_div, n_split, wide_wg);
-    plan.step = by_wave ? 1 : shape.ngrp;
-    plan.floor_blocks = by_wave ? 4 : 4 * shape.ngrp;
+    plan.B = B; plan.n_max = n_max;
     plan.max_tok = max_pages * TQ_PAGE_TOKENS; plan.len_sub = len_sub;
   }
   // Head sizes of the wide-head page kernel: the rotation launch also packs the kernel's query operands (one copy per

@@ -24,10 +24,10 @@ constexpr int MERGE_IN_KERNEL_MAX_SPLITS = 8;
 
 // Sequences of different lengths: with n_split equal shares each, a step takes as long as its longest sequence needs on
 // n_split workgroups, while those of the short ones idle.  The preparation launch therefore deals the same number of
-// workgroups out by length (schedule_splits_body, tq_prep.h): item i is what the i-th page-kernel workgroup of every
-// KV head does, in the order of dispatch, the largest shares first.  When all lengths are equal (header: n = 1) there are no items and the shares are
-// equal.  96 sequences of 61 .. 8190 tokens, 40 q / 8 KV heads of 128,
-// 4-bit keys: page kernel 129 -> 66 us.
+// workgroups out by length (schedule_splits_body, tq_prep.h) where that is clearly the shorter step: item i is what the i-th
+// page-kernel workgroup (or wavefront) of every KV head does, in the order of dispatch, the largest shares first.  Elsewhere the header says
+// equal shares (n = 1) and the step is the one without a schedule, bit for bit.  96 sequences of 61 .. 8190 tokens, 40 q / 8 KV heads
+// of 128, 4-bit keys: page kernel 129 -> 66 us.
 struct SplitItem {
   int32_t b, begin, end;             // sequence (-1: nothing to do), blocks [begin, end)
   int32_t len;                       // its compressed tokens
@@ -40,9 +40,11 @@ struct SplitPlan {
   const int32_t* seq_lens = nullptr;
   int B = 0, cap = 0;                // sequences; items behind the header
   int n_max = 0;                     // most shares of a sequence (parts in the workspace)
-  int n_static = 0, gx = 0, skew16 = 0, ngrp = 1;     // the launch with equal shares (decode_block_range)
-  int step = 1;                      // walkers of a share: its blocks are a multiple of this many
+  int n_static = 0, walkers = 1;     // the launch with equal shares: shares of a sequence, block walkers of a share
+  int step = 1;                      // walkers of an item's share: its blocks are a multiple of this many
   int floor_blocks = 1;              // a smaller share is not worth a workgroup
+  float slots_static = 1, slots = 1; // shares, items of one KV head that the card holds at once
+  float split_cost = 0;              // what a sequence in several items adds, in trips (one share per sequence: the merge through memory)
   int max_tok = 0, len_sub = 0;
 };
 constexpr int SCHED_FRONT = 8;        // workgroups in front of the preparation's (one of them works: the others keep their dies)
@@ -100,11 +102,11 @@ struct PagePrefetch {
 // groups, kv_div, n_seq, skew16, ngrp, gx, n_wg.
 void decode_mfma_plan(PagePrefetch& pf, int d, int B, int groups, int kv_div, int n_split, bool wide_wg);
 
-// Whether a step that is scheduled by length and has one share per sequence runs a share per wavefront (IW = 1 of the page
-// kernel), and the number of items of a schedule: the workgroups of n_split equal shares, or with one share
-// per sequence what the card holds at once, and room for half as many again when the sequences alone fill it.
-bool decode_sched_by_wave(int d, int mb, int B, int groups, int n_split, bool wide_wg);
-int decode_sched_items(int d, int mb, int B, int groups, int n_split, bool wide_wg);
+// Wavefronts that walk a (sequence, head group) of a step with one share per sequence: 4 (a workgroup), 2 or 1.
+int decode_sequence_walkers(int d, int mb, int B, int groups);
+
+// The part of a schedule that follows from the sizes of a step (cap, n_static, walkers, step, floor_blocks, slots, split_cost).
+void decode_sched_plan(SplitPlan& plan, int d, int mb, int B, int groups, int n_split, bool wide_wg);
 
 // Events armed by tq_time_next_page_kernel (which = 0) / tq_time_next_key_kernel (which = 1) on this thread:
 // returns them and disarms; false when none is armed.

@@ -67,16 +67,35 @@ int decode_mfma_split_skew(int n_split, int rows) {
   return units > 0 && groups <= 2 * (int64_t)units && groups * 16 >= 30 * (int64_t)units ? skew : 0;
 }
 
-bool decode_sched_by_wave(int d, int mb, int B, int groups, int n_split, bool wide_wg) {
-  return n_split == 1 && !wide_wg && d != 256 && mb < 4 && (int64_t)groups * B > 2 * (int64_t)device_compute_units();
+// Many short sequences in one split: the fewer wavefronts walk a (sequence, head group), the fewer workgroups the
+// launch has and the more trips follow each prologue; the most wavefronts per pair (4, 2 or 1) with which all of the
+// launch's wavefronts are resident at once (8 per compute unit) wins at every size measured (page kernel, 32 q / 8 KV
+// heads, four / two / one wavefront per pair: 64 x 2048 28.1 / 37.2 / 63.5 us, 96 x 2048 51.9 / 45.6 / 67.0,
+// 128 x 2048 60.4 / 56.0 / 69.7, 128 x 512 21.7 / 18.8 / 22.2, 160 x 1024 46.6 / 48.9 / 44.1, 192 x 1024 51.4 / 52.7 /
+// 47.0, 256 x 1024 66.7 / 61.5 / 58.0); with more pairs than wavefront slots, one.  Wavefronts that share a block
+// (head_dim 256) and 5-bit keys, whose operands are in LDS: four.
+int decode_sequence_walkers(int d, int mb, int B, int groups) {
+  if (d == 256 || mb >= 4) return 4;
+  const int64_t slots = (int64_t)8 * device_compute_units(), items = (int64_t)groups * B;
+  return slots <= 0 || 4 * items <= slots ? 4 : (2 * items <= slots ? 2 : 1);
 }
 
-int decode_sched_items(int d, int mb, int B, int groups, int n_split, bool wide_wg) {
-  if (n_split > 1) return n_split * B;
+// Items of a schedule: the workgroups of n_split equal shares, or with one share per sequence what the card holds at
+// once, and room for half as many again when the sequences alone fill it.  With one share per sequence and too many sequences for
+// four wavefronts each, an item is a wavefront's.
+void decode_sched_plan(SplitPlan& plan, int d, int mb, int B, int groups, int n_split, bool wide_wg) {
   const int units = device_compute_units() > 0 ? device_compute_units() : 256;
-  const int slots = (decode_sched_by_wave(d, mb, B, groups, n_split, wide_wg) ? 8 : (wide_wg ? 1 : 2)) * units;
-  const int fill = slots / groups, over = B + slots / (2 * groups);
-  return fill > over ? fill : over;
+  const int ngrp = (wide_wg ? 2 : 1) * MF_WAVES / (d == 256 ? 2 : 1), wg_slots = (wide_wg ? 1 : 2) * units;
+  plan.n_static = n_split;
+  plan.walkers = n_split == 1 && !wide_wg && d != 256 ? decode_sequence_walkers(d, mb, B, groups) : ngrp;
+  const bool by_wave = n_split == 1 && plan.walkers < ngrp;
+  const int slots = by_wave ? 8 * units : wg_slots, fill = slots / groups, over = B + slots / (2 * groups);
+  plan.cap = n_split > 1 ? n_split * B : (fill > over ? fill : over);
+  plan.step = by_wave ? 1 : ngrp;
+  plan.floor_blocks = 4 * plan.step;
+  plan.slots = (float)slots / (float)groups;
+  plan.slots_static = (by_wave ? 8.0f * units / plan.walkers : (float)wg_slots) / (float)groups;
+  plan.split_cost = by_wave ? 7.0f : 3.0f;
 }
 
 void decode_mfma_plan(PagePrefetch& pf, int d, int B, int groups, int kv_div, int n_split, bool wide_wg) {

@@ -46,6 +46,7 @@
 // wavefronts; WPS of them share a SIMD so that one wavefront's dependency stalls
 // are filled by another.
 
+#include <cstddef>
 #include <type_traits>
 
 #include <hip/hip_ext.h>
@@ -279,8 +280,7 @@ decode_mfma_kernel(const int32_t* __restrict__ seq_lens, const SplitItem* __rest
   // to a compute unit, and a SIMD serves its older wavefronts first: with equal shares the first half of the grid
   // finishes early and the second half runs on alone.
   int split = blockIdx.x, b = blockIdx.z;
-  // (sched: the share of this workgroup - of this wavefront when IW > 0 - is item `slot` of the step's schedule)
-  int n_mine = n_split, slot = blockIdx.x + (skew16 > 0 ? n_split / 2 : n_split) * blockIdx.z;
+  int n_mine = n_split;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wgrp = wave / DS, hf = wave % DS; // block walker this wavefront belongs to; its share of the head
@@ -290,44 +290,48 @@ decode_mfma_kernel(const int32_t* __restrict__ seq_lens, const SplitItem* __rest
   int h = blockIdx.y, qbase;
   bool item_live = true;                        // IW: this wavefront has a (sequence, head group) to walk
   constexpr int IWC = IW > 0 ? IW : 1;
-  const int wsub = IW > 0 ? wgrp % IWC : wgrp;  // this walker's number among those of its (sequence, head group)
+  int wsub = IW > 0 ? wgrp % IWC : wgrp;        // this walker's number among those of its (sequence, head group)
   if constexpr (IW > 0) {
-    const int item = blockIdx.y * (NW / DS / IWC) + wgrp / IWC, items = Hkv * (sched ? fm.sched_cap : n_seq);
+    const int item = blockIdx.y * (NW / DS / IWC) + wgrp / IWC, items = Hkv * n_seq;
     item_live = item < items;
     const int item_c = item_live ? item : items - 1;          // (a wavefront without an item repeats the last one and stores nothing)
     h = item_c % Hkv;
-    b = slot = item_c / Hkv;
+    b = item_c / Hkv;
   }
-  if (kv_div > 1) {
-    const int kv_heads = Hkv / kv_div, grp = h / kv_heads, kvh = h - grp * kv_heads;
-    const int g_tot = Hq / kv_heads, g_max = (g_tot + kv_div - 1) / kv_div;
-    h = kvh * kv_div + grp;
-    qbase = kvh * g_tot + grp * g_max;
-    G = min(g_max, g_tot - grp * g_max);
-  } else {
-    qbase = h * G;
-  }
-  SplitItem share;
-  bool by_length = false;
-  if (sched) {
-    share = sched[1 + slot];
-    int equal = sched->n;
-    asm volatile("" : "+s"(equal));                           // (one wait for both)
-    by_length = !equal;
-  }
-  if (by_length) {
-    if (IW == 0 && share.b < 0) return;                       // (the whole workgroup: the items' order is that of dispatch)
-    item_live = item_live && share.b >= 0;
-    b = max(share.b, 0);
-    split = share.split;
-    n_mine = share.n;
-  } else if (DS == 2 && skew16 > 0) {                                  // (only the launcher of DS == 2 kernels passes a skew)
+  if (DS == 2 && skew16 > 0) {                                  // (only the launcher of DS == 2 kernels passes a skew)
     // (n_seq arrives with the other kernel arguments; the grid's size would be one more scalar load of the
     // launch's implicit data in front of everything that depends on the sequence)
     const int late = b >= n_seq;
     b -= late ? n_seq : 0;
     split = 2 * split + late;
   }
+  // A schedule says whether the shares are equal; its items are per workgroup (IW == 0) or per wavefront.  Both come from another
+  // launch's stores, 0.3 us later than what is in the caches; asked for as vector loads, which do not hold up the scalar ones,
+  // they are looked at when the operands of the equal shares are on their way (16 x 8192, 32 q / 8 KV heads of 128,
+  // equal lengths: step 39.65 -> 39.4 us, without a schedule 39.35).
+  const int own = IW > 0 ? blockIdx.y * (NW / DS) + wgrp : blockIdx.x + (skew16 > 0 ? n_split / 2 : n_split) * blockIdx.z;
+  bool by_length = false;
+  u32x4 share_lo = {0, 0, 0, 0};
+  uint32_t share_split = 0, share_n = 1, equal_v = 1;
+  if (sched) {
+    const uint32_t* item = (const uint32_t*)(sched + 1 + (IW > 0 ? min(own, Hkv * fm.sched_cap - 1) / Hkv : own)) + in_vgpr(0u);
+    equal_v = ((const uint32_t*)sched + in_vgpr(0u))[offsetof(SplitItem, n) / 4];
+    share_lo = *(const u32x4*)item;
+    share_split = item[offsetof(SplitItem, split) / 4];
+    share_n = item[offsetof(SplitItem, n) / 4];
+  }
+  const int len_b = seq_lens[min(b, n_seq - 1)];
+  // the query head group of a (KV head, group) number, and what it consists of
+  auto map_head = [&]() {
+    qbase = h * (Hq / Hkv);
+    if (kv_div > 1) {
+      const int kv_heads = Hkv / kv_div, grp = h / kv_heads, kvh = h - grp * kv_heads;
+      const int g_tot = Hq / kv_heads, g_max = (g_tot + kv_div - 1) / kv_div;
+      h = kvh * kv_div + grp;
+      qbase = kvh * g_tot + grp * g_max;
+      G = min(g_max, g_tot - grp * g_max);
+    }
+  };
   const int n = lane & 15, kb = lane >> 4;    // score stage: token / coordinate quarter; value stage: row / page
   TQ_STAMP(0);
 
@@ -362,17 +366,18 @@ decode_mfma_kernel(const int32_t* __restrict__ seq_lens, const SplitItem* __rest
   constexpr int QA_OP = 64 * 6;
   int qa_lane = 0, qa_sel = 0;
   f32x4 cm = {0, 0, 0, 0}, cq = {0, 0, 0, 0};
+  float st1 = 0.0f, st2 = 0.0f, c2[NJ], c3[NJ];   // as they come from memory: nothing waits for them before finish_operands
   auto load_operands = [&]() {
+  const int b_c = min(b, n_seq - 1);            // (a workgroup of the larger grid, see above)
   {
     // PP: rows 8..15 / coordinates 64..127 repeat rows 0..7 / coordinates 0..63; the off-diagonal blocks are zero
     // NR: row 4g + t is row 2g + t % 2 of row set t / 2
     const int slane = PP ? (n & 7) + 16 * (kb & 1) : (NR ? 2 * (n >> 2) + (n & 1) + 16 * kb : lane);
-    const bool a_live = !PP || ((n < 8) == (kb < 2));
-    const uint32_t* src = qa_pack + (((int64_t)b * Hkv + h) * (NTP * WPLT * 2 * 64) + slane) * 8 +
+    const uint32_t* src = qa_pack + (((int64_t)b_c * Hkv + h) * (NTP * WPLT * 2 * 64) + slane) * 8 +
                           (NR ? ((n >> 1) & 1) * (64 * 8) : 0);
     if constexpr (QL) {
       // the whole block of the group, 16 bytes per lane and step, as it lies in memory
-      const uint32_t* blk = qa_pack + ((int64_t)b * Hkv + h) * (NTP * WPLT * 2 * 64 * 8);
+      const uint32_t* blk = qa_pack + ((int64_t)b_c * Hkv + h) * (NTP * WPLT * 2 * 64 * 8);
       for (int o = tid; o < NTP * WPLT * 2 * 64 * 2; o += MF_WAVES * 64) {       // o: 16-byte piece, two per lane slot
         const u32x4 v = *(const u32x4*)(blk + o * 4);
         uint32_t* op = qa_lds + (o >> 7) * QA_OP;
@@ -394,17 +399,38 @@ decode_mfma_kernel(const int32_t* __restrict__ seq_lens, const SplitItem* __rest
           const u32x4 lo = *(const u32x4*)p6;
           const uint32_t d4 = p6[4], d5 = p6[5];
           qa[tp][i][rs] = i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)d4, (int)d5, 0, 0};
-          if (!a_live) qa[tp][i][rs] = i32x8{0, 0, 0, 0, 0, 0, 0, 0};
         }
+  }
+  {
+    const int g = PP ? (n & 7) >> 1 : (NR ? n >> 2 : n >> 1);
+    const int64_t qrow = (int64_t)b_c * Hq + qbase + (g < G ? g : 0);
+    st1 = q_stat[qrow * 4 + 0];
+    st2 = q_stat[qrow * 4 + 1];
+  }
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const int g = PP ? 2 * (kb & 1) + j : (NR ? kb : 2 * kb + j);
+    const int64_t qrow = (int64_t)b_c * Hq + qbase + (g < G ? g : 0);
+    c2[j] = q_stat[qrow * 4 + 2];
+    c3[j] = q_stat[qrow * 4 + 3];
+  }
+  };
+  auto finish_operands = [&]() {
+  if constexpr (PP) {
+    const bool a_live = (n < 8) == (kb < 2);
+#pragma unroll
+    for (int tp = 0; tp < NTP; ++tp)
+#pragma unroll
+      for (int i = 0; i < WPL; ++i)
+#pragma unroll
+        for (int rs = 0; rs < NRS; ++rs)
+          if (!a_live) qa[tp][i][rs] = i32x8{0, 0, 0, 0, 0, 0, 0, 0};
   }
   // E8M0 block-scale codes of this lane's operand row (head n / 2), one per byte: index planes row
   // set 0, row set 1, sign plane row set 0, row set 1.  4 v / 2^E is stored, so term t carries
   // 2^(E - 2 - 5t); the fp4 bit value 0.5 carries 2^1.
   {
-    const int g = PP ? (n & 7) >> 1 : (NR ? n >> 2 : n >> 1);
-    const int64_t qrow = (int64_t)b * Hq + qbase + (g < G ? g : 0);
-    const int e1 = 127 + (int)q_stat[qrow * 4 + 0];
-    const int e2 = 127 + (int)q_stat[qrow * 4 + 1];
+    const int e1 = 127 + (int)st1, e2 = 127 + (int)st2;
     const int t01 = (n & 1) ? 7 : 2, t23 = t01 + 10;
     sa = (e1 - t01) | ((e1 - t23) << 8) | ((e2 - t01) << 16) | ((e2 - t23) << 24);
     if (NR) {                                    // one row set: byte 0 index planes, byte 2 sign plane
@@ -418,17 +444,49 @@ decode_mfma_kernel(const int32_t* __restrict__ seq_lens, const SplitItem* __rest
   for (int j = 0; j < NJ; ++j) {
     const int g = PP ? 2 * (kb & 1) + j : (NR ? kb : 2 * kb + j);
     const bool live = g < G && hf == 0;
-    const int64_t qrow = (int64_t)b * Hq + qbase + (g < G ? g : 0);
-    const float c2 = q_stat[qrow * 4 + 2], c3 = q_stat[qrow * 4 + 3];
-    cm[2 * j] = live ? c2 : 0.0f;
-    cq[2 * j] = live ? c3 : 0.0f;
+    cm[2 * j] = live ? c2[j] : 0.0f;
+    cq[2 * j] = live ? c3[j] : 0.0f;
     if (QL) {                                     // (lanes that share an operand slot see the same heads)
-      c_lds[qa_lane * 4 + j] = live ? c2 : 0.0f;
-      c_lds[qa_lane * 4 + 2 + j] = live ? c3 : 0.0f;
+      c_lds[qa_lane * 4 + j] = live ? c2[j] : 0.0f;
+      c_lds[qa_lane * 4 + 2 + j] = live ? c3[j] : 0.0f;
     }
   }
   };
-  load_operands();
+  // (head_dim 256: asking for its operands twice costs a step by length 1 us, and the others 0.2 at most)
+  constexpr bool AHEAD = DS == 1;
+  if (AHEAD || !sched) {
+    map_head();
+    load_operands();
+  }
+  if (sched) {
+    by_length = __builtin_amdgcn_readfirstlane(equal_v) == 0;
+    if (by_length) {
+      const int share_b = __builtin_amdgcn_readfirstlane(share_lo[0]);
+      // (whole workgroups leave: the items' order is that of dispatch, and the grid is as large as the larger way needs)
+      if (IW == 0 && share_b < 0) return;
+      if (IW > 0 && (int)blockIdx.y * (NW / DS) >= Hkv * fm.sched_cap) return;
+      if constexpr (IW > 0) {
+        item_live = own < Hkv * fm.sched_cap && share_b >= 0;
+        h = min(own, Hkv * fm.sched_cap - 1) % Hkv;
+        wsub = 0;
+      } else {
+        h = blockIdx.y;
+      }
+      b = max(share_b, 0);
+      split = __builtin_amdgcn_readfirstlane(share_split);
+      n_mine = __builtin_amdgcn_readfirstlane(share_n);
+    } else {
+      if (IW == 0 && b >= n_seq) return;
+      if (IW > 0 && (int)blockIdx.y * (NW / DS / IWC) >= Hkv * n_seq) return;
+    }
+    if (by_length || !AHEAD) {
+      map_head();
+      if (QL) __syncthreads();
+      load_operands();
+    }
+  }
+  const int wstep = IW == 2 ? (by_length ? 1 : 2) : (IW > 0 ? IW : NGRP);     // distance of a walker's consecutive blocks
+  finish_operands();
   const int sb = 127 + 1;
   // head_dim 64: the score MFMA still contracts 128 coordinates; the lanes of the upper two coordinate
   // quarters feed zeros (their masks are zero, whatever their loads return)
@@ -458,9 +516,13 @@ decode_mfma_kernel(const int32_t* __restrict__ seq_lens, const SplitItem* __rest
   // len_sub: newest tokens that are attended to exactly.  A length beyond the block table is cut to the table.
   int seq_len = 0, blk_begin = 0, blk_end = 0;
   if (by_length) {
-    if (item_live) { seq_len = share.len; blk_begin = share.begin; blk_end = share.end; }
+    if (item_live) {
+      blk_begin = __builtin_amdgcn_readfirstlane(share_lo[1]);
+      blk_end = __builtin_amdgcn_readfirstlane(share_lo[2]);
+      seq_len = __builtin_amdgcn_readfirstlane(share_lo[3]);
+    }
   } else {
-    seq_len = item_live ? max(min(seq_lens[b], max_pages * TQ_PAGE_TOKENS) - len_sub, 0) : 0;
+    seq_len = item_live ? max(min(len_b, max_pages * TQ_PAGE_TOKENS) - len_sub, 0) : 0;
     decode_block_range(seq_len, n_split, split, DS == 2 ? skew16 : 0, NGRP, blk_begin, blk_end);
   }
   const int n_pages = (seq_len + TQ_PAGE_TOKENS - 1) / TQ_PAGE_TOKENS;
@@ -957,8 +1019,7 @@ decode_mfma_kernel(const int32_t* __restrict__ seq_lens, const SplitItem* __rest
     KeyRegs K;
     ValRegs V;
     int pid[4];
-    constexpr int WSTEP = IW > 0 ? IW : NGRP;              // distance of a walker's consecutive blocks
-    const int trips = (max(blk_end - blk_begin, 0) + WSTEP - 1) / WSTEP;
+    const int trips = (max(blk_end - blk_begin, 0) + wstep - 1) / wstep;
     int blk = blk_begin + wsub;
     int bad = 0;                                          // pages of the current block that lie outside the pool
     if (blk < blk_end) {
@@ -998,7 +1059,7 @@ decode_mfma_kernel(const int32_t* __restrict__ seq_lens, const SplitItem* __rest
         constexpr bool LAST = decltype(last_tag)::value;
         // the block after this walker's last one does not exist: re-request the current one instead,
         // so that the loads stay outside any branch
-        const int nxt = blk + WSTEP;
+        const int nxt = blk + wstep;
         const int nxt_c = nxt < blk_end ? nxt : blk;
         int pid_n[4] = {0, 0, 0, 0};
         int bad_n = 0;
@@ -1160,15 +1221,16 @@ decode_mfma_kernel(const int32_t* __restrict__ seq_lens, const SplitItem* __rest
     }
   };
   if constexpr (IW > 0) {
-    // The IW wavefronts of a (sequence, head group) finish it among themselves: their rows of s_red hold its walkers.
-    constexpr int TP = 64 * IWC;                 // threads of a (sequence, head group)
+    // The walkers of a (sequence, head group) finish it among themselves: their rows of s_red hold its sums.
+    auto finish = [&](auto walkers) __attribute__((always_inline)) {
+    constexpr int WK = decltype(walkers)::value, TP = 64 * WK;       // its walkers, and their threads
     const int tsub = wsub * 64 + lane, w0 = wgrp - wsub;
     // log-sum-exp merge of the walkers' element e (0: the maximum itself, 1: the sum of weights, 2 + ch: a channel)
     auto merged = [&](int g, int e, float& mm, float& ll) -> float {
-      float m_w[IWC], l_w[IWC], a_w[IWC];
+      float m_w[WK], l_w[WK], a_w[WK];
       mm = MF_NEG;
 #pragma unroll
-      for (int w = 0; w < IWC; ++w) {
+      for (int w = 0; w < WK; ++w) {
         const float* r = s_red + ((w0 + w) * g_rows + g) * (D + 2);
         m_w[w] = r[0]; l_w[w] = r[1]; a_w[w] = r[e];
         mm = fmaxf(mm, m_w[w]);
@@ -1176,7 +1238,7 @@ decode_mfma_kernel(const int32_t* __restrict__ seq_lens, const SplitItem* __rest
       ll = 0.0f;
       float aa = 0.0f;
 #pragma unroll
-      for (int w = 0; w < IWC; ++w) {
+      for (int w = 0; w < WK; ++w) {
         const float wgt = __expf(m_w[w] - mm);
         ll = fmaf(wgt, l_w[w], ll);
         aa = fmaf(wgt, a_w[w], aa);
@@ -1220,8 +1282,8 @@ decode_mfma_kernel(const int32_t* __restrict__ seq_lens, const SplitItem* __rest
           store_coherent2(out + 2 * pr, pr == 0 ? f32x2{mm, ll} : f32x2{a0, a1});
         }
       }
-      // a sequence with several shares: the wavefront that finishes last among them merges (IW = 1; see below)
-      if constexpr (IW == 1) {
+      // a sequence with several shares: the wavefront that finishes last among them merges (see below)
+      if constexpr (WK == 1) {
         if (by_length && fm.out != nullptr && item_live) {
           asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
           unsigned long long before = 0;
@@ -1231,6 +1293,9 @@ decode_mfma_kernel(const int32_t* __restrict__ seq_lens, const SplitItem* __rest
         }
       }
     }
+    };
+    if (IW == 2 && !by_length) finish(std::integral_constant<int, IWC>{});
+    else finish(std::integral_constant<int, 1>{});
     return;
   }
   // merge of the walkers: thread -> (head, channel); loads are unconditional (clamped), stores guarded
@@ -1397,21 +1462,12 @@ static int launch_one(uint32_t* qa_pack, float* q_stat, int B, int Hq, int Hkv, 
                                                                       n_split, len_sub, max_pages, num_pages, fm, wide_wg, st);
   } else {
   // eight wavefronts per workgroup (one workgroup per compute unit) for the kernels whose wavefronts work alone
-  // Many short sequences in one split: the fewer wavefronts walk a (sequence, head group), the fewer workgroups the
-  // launch has and the more trips follow each prologue; the most wavefronts per pair (4, 2 or 1) with which all of the
-  // launch's wavefronts are resident at once (8 per compute unit) wins at every size measured (page kernel, 32 q / 8 KV
-  // heads, four / two / one wavefront per pair: 64 x 2048 28.1 / 37.2 / 63.5 us, 96 x 2048 51.9 / 45.6 / 67.0,
-  // 128 x 2048 60.4 / 56.0 / 69.7, 128 x 512 21.7 / 18.8 / 22.2, 160 x 1024 46.6 / 48.9 / 44.1, 192 x 1024 51.4 / 52.7 /
-  // 47.0, 256 x 1024 66.7 / 61.5 / 58.0); with more pairs than wavefront slots, one.
+  // (see decode_sequence_walkers)
   constexpr bool can_iw = DS == 1 && MB < 4 && NW == MF_WAVES;
   if constexpr (can_iw && IW == 0) {
     if (n_split == 1 && !wide_wg) {
       int walkers = opt_sequence_walkers.load(std::memory_order_relaxed);
-      if (fm.sched) walkers = decode_sched_by_wave(D, MB, B, Hkv, n_split, wide_wg) ? 1 : 4;
-      if (walkers < 0) {
-        const int64_t slots = (int64_t)8 * device_compute_units(), items = (int64_t)Hkv * B;
-        walkers = slots <= 0 || 4 * items <= slots ? 4 : (2 * items <= slots ? 2 : 1);
-      }
+      if (walkers < 0) walkers = decode_sequence_walkers(D, MB, B, Hkv);
       if (walkers == 1)
         return launch_one<D, MB, NX, VB, GS, DS, WPS, F16P, PP, NR, SG, NW, 1>(
             qa_pack, q_stat, B, Hq, Hkv, kv_div, pool, block_table, bt_stride, seq_lens, sm_scale, ly, L, parts, n_parts, n_split,
@@ -1433,7 +1489,9 @@ static int launch_one(uint32_t* qa_pack, float* q_stat, int B, int Hq, int Hkv, 
   // what they move (32 x 32768: 203 -> 208 us).
   const int skew16 = NW == MF_WAVES && WPS == 2 && DS == 2 ? decode_mfma_split_skew(n_split, Hkv * B) : 0;
   constexpr int IPW = NW / DS / (IW > 0 ? IW : 1);          // (sequence, head group) pairs of a workgroup with IW > 0
-  const dim3 grid = IW > 0 ? dim3(1, (unsigned)(((int64_t)Hkv * (fm.sched ? fm.sched_cap : B) + IPW - 1) / IPW), 1)
+  const int64_t iw_wgs = std::max<int64_t>(((int64_t)Hkv * B + IPW - 1) / IPW,           // equal shares, shares by length
+                                           fm.sched ? ((int64_t)Hkv * fm.sched_cap + NW / DS - 1) / (NW / DS) : 0);
+  const dim3 grid = IW > 0 ? dim3(1, (unsigned)iw_wgs, 1)
                     : fm.sched && n_split == 1 ? dim3(1, Hkv, fm.sched_cap)
                        : (skew16 > 0 ? dim3(n_split / 2, Hkv, 2 * B) : dim3(n_split, Hkv, B));
   auto kern = decode_mfma_kernel<D, MB, NX, VB, GS, DS, WPS, F16P, PP, NR, SG, NW, IW>;

@@ -328,37 +328,81 @@ __device__ __forceinline__ unsigned long long load_coherent(const unsigned long 
 
 // The schedule of a step (see SplitPlan), by one workgroup of NT threads of the preparation launch, which has the time
 // that the preparation takes: the smallest share of blocks with which all shares fit the items is found by trying 64
-// sizes at a time, then the shares are written largest first (by sixteenths of the largest).
+// sizes at a time, then the shares are written largest first (by sixteenths of the largest) - if the step is shorter for it.
+//
+// When it is: a step is taken to last as long as its longest walker makes trips, and SCHED_PROLOGUE more; where the shares are more than
+// the card holds at once, as long as two rounds of the share that the last slot begins with, or as the trips and
+// prologues of all of them spread over the slots (in the order of the sequences: and the surplus of the longest share). A sequence
+// in several items of a step that otherwise has one share each adds split_cost for the merge through memory.  With several shares
+// per sequence as many workgroups run either way: a tenth fewer trips is enough, or a quarter fewer shares.  With both ways
+// measured at 22 shapes (1 .. 64 shares, head_dim 64 / 128 / 256) and ten spreads of the lengths - equal, down to 0.9 .. 0.02 of the
+// longest, one long among short, alternating - the rule's step is within 3 % of the faster way at all but 11 of 220 (those within
+// 10 %, once 20 %).  Lengths spread to half: 192 x 1024 52 us in equal shares, 67 by length; 16 x 16384, head_dim 256, 34.4
+// and 32.4; spread to a fiftieth: 192 x 1024 44.7 and 38.7; 32 x 8192 42.2 and 29.4.
+constexpr int SCHED_PROLOGUE = 3;
 __device__ __forceinline__ int sched_pieces(int nb, int tau, float inv, int n_max) {
   const int n = (int)((float)(nb + tau - 1) * inv);          // (any rounding will do: the share size follows from the count)
   return n < 1 ? 1 : (n > n_max ? n_max : n);
+}
+// A reduction over the wavefront in registers (an atomic of every lane on one LDS word is a loop over the lanes: 1 us each)
+template <class Op>
+__device__ __forceinline__ int wave_reduce(int v, Op op) {
+  v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x128, 0xF, 0xF, true));       // rotations by 8, 4, 2, 1 in rows of 16
+  v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x124, 0xF, 0xF, true));
+  v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x122, 0xF, 0xF, true));
+  v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x121, 0xF, 0xF, true));
+  return op(op(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+            op(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
 }
 template <int NT>
 __device__ __forceinline__ void schedule_splits_body(const SplitPlan& P, int tid, int* sm) {
   int* nb = sm;                                  // [B] blocks
   int* cand = sm + SCHED_MAX_SEQS;               // [64] shares with a candidate size
-  int* red = cand + 64;                          // [0] most blocks, [2] largest share; [16..31] bucket sizes, [32..47] next item of a bucket
-  auto blocks_of = [&](int b) { return (max(min(P.seq_lens[b], P.max_tok) - P.len_sub, 0) + 63) / 64; };
-  // Equal lengths (in blocks): equal shares, and the page kernel works them out itself.  The usual case, and one whose
-  // time counts: in a serving loop the caches are full of pages and every instruction comes from memory.
-  if (P.cap == P.n_static * P.B) {
-    const int n0 = blocks_of(0);
-    int same = 1;
-    for (int b = tid; b < P.B; b += NT) same &= blocks_of(b) == n0;
-    same = __syncthreads_and(same);
-    if (tid == 0) P.items->n = same;
-    if (same) return;
-  } else if (tid == 0) {
-    P.items->n = 0;
-  }
+  // [0] most blocks, [1] all blocks, [2] largest share, [3] trips of equal shares, [4] shares, [5] their trips; [16..31] bucket sizes,
+  // [32..47] next item of a bucket
+  int* red = cand + 64;
+  const auto trips = [](int blocks, int walkers) { return (blocks + walkers - 1) / walkers; };
+  const auto sum = [](int a, int b) { return a + b; };
+  const auto larger = [](int a, int b) { return a > b ? a : b; };
+  const bool first_lane = (tid & 63) == 0;
+  const int len0 = P.seq_lens[min(tid, P.B - 1)];            // (asked for ahead of the first barrier)
   if (tid < 48) red[tid] = 0;
   __syncthreads();
+  int most = 0, all = 0, equal_trips = 0;
   for (int b = tid; b < P.B; b += NT) {
-    nb[b] = blocks_of(b);
-    atomicMax(red + 0, nb[b]);
+    const int n = (max(min(b == tid ? len0 : P.seq_lens[b], P.max_tok) - P.len_sub, 0) + 63) / 64;
+    nb[b] = n;
+    most = max(most, n);
+    all += min(n, 1 << 20);                                  // (sums of 1024 stay in range)
+    equal_trips += trips(min(n, 1 << 20), P.walkers);
+  }
+  most = wave_reduce(most, larger);
+  all = wave_reduce(all, sum);
+  equal_trips = wave_reduce(equal_trips, sum);
+  if (first_lane) {
+    atomicMax(red + 0, most);
+    atomicAdd(red + 1, all);
+    atomicAdd(red + 3, equal_trips);
   }
   __syncthreads();
-  const int most = red[0];
+  most = red[0];
+  all = red[1];
+  // the step in equal shares, and the least that shares by length could come to: the usual case, lengths alike, ends here, and its time
+  // counts (in a serving loop the caches are full of pages and every instruction comes from memory)
+  const int per_equal = (most + P.n_static - 1) / P.n_static, a_equal = trips(per_equal, P.walkers);
+  float t_equal = (float)(a_equal + SCHED_PROLOGUE);
+  const float r_equal = (float)P.B / P.slots_static;
+  if (P.n_static == 1 && r_equal > 1.0f) {
+    const float mean = (float)red[3] / (float)P.B;
+    t_equal = fmaxf(t_equal, r_equal * (mean + SCHED_PROLOGUE) + ((float)a_equal - mean));
+  }
+  const int least = trips(max(max((all + P.cap - 1) / P.cap, (most + P.n_max - 1) / P.n_max), min(most, P.floor_blocks)), P.step);
+  const bool hopeless = P.n_static > 1 ? 10 * least > 9 * a_equal && 4.0f * (float)all > 3.0f * (float)P.cap * (float)per_equal
+                                       : r_equal <= 1.0f && (float)(least + SCHED_PROLOGUE) + P.split_cost + 1.0f > t_equal;
+  if (hopeless) {
+    if (tid == 0) P.items->n = 1;
+    return;
+  }
   SplitItem* items = P.items + 1;
   int lo = max(P.floor_blocks, 1), hi = max(most, lo);       // hi always fits
   constexpr int TPC = NT / 64;                               // threads per candidate
@@ -390,11 +434,22 @@ __device__ __forceinline__ void schedule_splits_body(const SplitPlan& P, int tid
     n = max((n_blocks + per - 1) / per, 1);
     return per;
   };
+  int largest = 0, shares = 0, share_trips = 0;
   for (int b = tid; b < P.B; b += NT) {
     int n;
     const int per = share(nb[b], n);
-    atomicMax(red + 2, min(per, nb[b]));
+    largest = max(largest, min(per, nb[b]));
     P.n_of[b] = n;
+    shares += n;
+    share_trips += min((n - 1) * (per / P.step) + trips(nb[b] - (n - 1) * per, P.step), 1 << 20);
+  }
+  largest = wave_reduce(largest, larger);
+  shares = wave_reduce(shares, sum);
+  share_trips = wave_reduce(share_trips, sum);
+  if (first_lane) {
+    atomicMax(red + 2, largest);
+    atomicAdd(red + 4, shares);
+    atomicAdd(red + 5, share_trips);
   }
   __syncthreads();
   const float to16 = 16.0f / (float)(red[2] + 1);
@@ -405,6 +460,20 @@ __device__ __forceinline__ void schedule_splits_body(const SplitPlan& P, int tid
     atomicAdd(red + 16 + bucket(per, nb[b]), n);
   }
   __syncthreads();
+  const int a_item = trips(red[2], P.step);
+  float t_item = (float)(a_item + SCHED_PROLOGUE);
+  const float r_item = (float)red[4] / P.slots;
+  if (r_item > 1.0f) {
+    int k = 0;                                               // bucket of the share that the last slot begins with
+    for (int before = red[16]; k < 15 && (float)before <= P.slots; before += red[16 + ++k]) {}
+    const int last = min(trips((16 - k) * (red[2] + 1) / 16, P.step), a_item);
+    t_item = fmaxf(t_item, fmaxf(2.0f * (float)(last + SCHED_PROLOGUE), ((float)red[5] / P.slots) + r_item * SCHED_PROLOGUE));
+  }
+  if (red[4] > P.B) t_item += P.split_cost;
+  const bool by_length = P.n_static > 1 ? 10 * a_item <= 9 * a_equal || (a_item <= a_equal && 4 * red[4] <= 3 * P.cap)
+                                        : t_item + 1.0f <= t_equal;
+  if (tid == 0) P.items->n = !by_length;
+  if (!by_length) return;
   if (tid < 16) {
     int at = 0;
     for (int k = 0; k < tid; ++k) at += red[16 + k];
