@@ -245,10 +245,8 @@ int tq_pool_export(const uint8_t *pool, int64_t num_pages, int H, const int32_t 
  * kernel of the head sizes 320 .. 704 (a block of 32 tokens per workgroup).  Negative: an error code.           */
 int tq_decode_page_kernel(const tq_layer *layer /*host*/, const tq_page_layout *layout /*host*/);
 
-/* Bytes of workspace tq_decode_attn_paged needs for these sizes.  n_split > 0: that many equal shares of every
- * sequence.  n_split < 0: -n_split workgroups per sequence and KV head on average, dealt out by the lengths of the
- * sequences in device memory (a long one gets more of them); needs more workspace.  The decode entries take the same
- * two forms (tq_decode_attn_paged_noalloc the first only).                          */
+/* Bytes of workspace tq_decode_attn_paged needs for these sizes (n_split > 0), or with -n_split in its place those that
+ * tq_decode_attn_paged_by_length needs.                                            */
 size_t tq_decode_workspace_bytes(int B, int Hq, int d, int n_split);
 
 /* Fused decode attention over the paged compressed history plus an optional
@@ -299,6 +297,23 @@ int tq_decode_attn_paged_ring(const void *q, int dtype, int B, int Hq, int Hkv, 
                               float sm_scale, const tq_layer *layer, const tq_page_layout *layout,
                               const void *k_cache, const void *v_cache, int64_t cs_blk, int64_t cs_t, int64_t cs_h,
                               int ring_rows, void *out, void *workspace, int n_split, void *stream);
+
+/* tq_decode_attn_paged / _ring for sequences of different lengths: n_split workgroups per sequence and KV head on average,
+ * dealt out by the lengths that the device holds (a long sequence gets more of them) where that makes the step
+ * shorter; equal shares, with the same result bit for bit, where it does not, and on the page kernels and batches
+ * (one sequence, more than 1024) that know no other.  The workspace is that of tq_decode_workspace_bytes(.., -n_split).  */
+int tq_decode_attn_paged_by_length(const void *q, int dtype, int B, int Hq, int Hkv, const uint8_t *pool,
+                                   int64_t num_pages, const int32_t *block_table, int bt_stride,
+                                   const int32_t *seq_lens, float sm_scale, const tq_layer *layer,
+                                   const tq_page_layout *layout, const void *recent_k, const void *recent_v,
+                                   int recent_rows, int64_t rs_b, int64_t rs_r, int64_t rs_h,
+                                   const int32_t *recent_len, void *out, void *workspace, int n_split, void *stream);
+int tq_decode_attn_paged_ring_by_length(const void *q, int dtype, int B, int Hq, int Hkv, const uint8_t *pool,
+                                        int64_t num_pages, const int32_t *block_table, int bt_stride,
+                                        const int32_t *seq_lens, float sm_scale, const tq_layer *layer,
+                                        const tq_page_layout *layout, const void *k_cache, const void *v_cache,
+                                        int64_t cs_blk, int64_t cs_t, int64_t cs_h, int ring_rows, void *out,
+                                        void *workspace, int n_split, void *stream);
 
 /* tq_decode_attn_paged for callers that cannot allocate or pass a workspace (code under HIP graph capture
  * that owns no buffers, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the

@@ -63,6 +63,26 @@ def test_workspace_of_a_step_by_length_holds_the_equal_shares_it_may_fall_back_t
         assert lib.tq_decode_workspace_bytes(B, Hq, d, -n_split) >= lib.tq_decode_workspace_bytes(B, Hq, d, n_split)
 
 
+def _decode_args(n_split, rows=(None, None, 0, 0, 0, 0, None), stages=()):
+    """Arguments of a decode entry that end in a refusal before anything is read or launched (a layer of head_dim 100)."""
+    ly, layout = _ffi.TqLayer(), _ffi.TqPageLayout()
+    ly.d = layout.d = 100
+    return (1, 2, 4, 8, 2, 1, 16, 1, 4, 1, 1.0, C.byref(ly), C.byref(layout), *rows, 1, 1, n_split, *stages, None)
+
+
+@pytest.mark.parametrize("n_split", [0, -1, -64, -(1 << 20), -(1 << 31)])
+def test_a_split_count_that_is_not_positive_is_refused(n_split):
+    """By every decode entry, with the code of an invalid argument; positive counts get as far as the head size."""
+    lib, ring = _ffi.lib(), (1, 1, 64, 4, 4, 16)
+    for n, want in ((n_split, -1), (1, -2), (1 << 20, -2)):
+        assert lib.tq_decode_attn_paged(*_decode_args(n)) == want
+        assert lib.tq_decode_attn_paged_stages(*_decode_args(n, stages=(7,))) == want
+        assert lib.tq_decode_attn_paged_ring(*_decode_args(n, rows=ring)) == want
+    for n, want in ((n_split, -1), (1 << 20, -1), (1, -2)):
+        assert lib.tq_decode_attn_paged_by_length(*_decode_args(n)) == want
+        assert lib.tq_decode_attn_paged_ring_by_length(*_decode_args(n, rows=ring)) == want
+
+
 def test_argument_errors_are_reported_before_any_launch():
     lib = _ffi.lib()
     assert lib.tq_bucketize_pack(None, 4, 128, None, 2, None, None) == -3

@@ -79,6 +79,12 @@ _SIGNATURES = {
                                               _i, _vp]),
     "tq_decode_attn_paged_ring": (C.c_int, [_vp, _i, _i, _i, _i, _vp, _i64, _vp, _i, _vp, _f, C.POINTER(TqLayer),
                                             C.POINTER(TqPageLayout), _vp, _vp, _i64, _i64, _i64, _i, _vp, _vp, _i, _vp]),
+    "tq_decode_attn_paged_by_length": (C.c_int, [_vp, _i, _i, _i, _i, _vp, _i64, _vp, _i, _vp, _f, C.POINTER(TqLayer),
+                                                 C.POINTER(TqPageLayout), _vp, _vp, _i, _i64, _i64, _i64, _vp, _vp, _vp, _i,
+                                                 _vp]),
+    "tq_decode_attn_paged_ring_by_length": (C.c_int, [_vp, _i, _i, _i, _i, _vp, _i64, _vp, _i, _vp, _f, C.POINTER(TqLayer),
+                                                      C.POINTER(TqPageLayout), _vp, _vp, _i64, _i64, _i64, _i, _vp, _vp, _i,
+                                                      _vp]),
     "tq_decode_attn_paged_noalloc": (C.c_int, [_vp, _i, _i, _i, _i, _vp, _i64, _vp, _i, _vp, _f, C.POINTER(TqLayer),
                                                C.POINTER(TqPageLayout), _vp, _vp, _i, _i64, _i64, _i64, _vp, _vp, _i, _vp]),
     "tq_decode_noalloc_bytes": (C.c_size_t, [_i, _i, _i, _i, C.POINTER(TqLayer)]),

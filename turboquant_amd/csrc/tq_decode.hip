@@ -1133,22 +1133,28 @@ struct TailSpec {
   const int32_t* len = nullptr;
   bool paged = false;
 };
+int ring_tail(TailSpec& ts, const void* k_cache, const void* v_cache, int64_t cs_blk, int64_t cs_t, int64_t cs_h, int ring_rows) {
+  if (!k_cache || !v_cache) return TQ_ENULL;
+  if (ring_rows <= 0 || cs_blk <= 0 || cs_t <= 0 || cs_h <= 0) return TQ_EINVAL;
+  ts.k = k_cache; ts.v = v_cache; ts.rows = ring_rows;
+  ts.s_blk = cs_blk; ts.s_r = cs_t; ts.s_h = cs_h; ts.paged = true;
+  return TQ_OK;
+}
 }  // namespace
 
 static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const uint8_t* pool, int64_t num_pages,
                          const int32_t* block_table, int bt_stride, const int32_t* seq_lens, float sm_scale,
                          const tq_layer* layer, const tq_page_layout* layout, const TailSpec& ts, void* out,
-                         void* workspace, int n_split, int stages, void* stream) {
+                         void* workspace, int n_split, int stages, void* stream, bool by_length = false) {
   const void *recent_k = ts.k, *recent_v = ts.v;
   const int recent_rows = ts.rows;
   const int64_t rs_b = ts.s_b, rs_r = ts.s_r, rs_h = ts.s_h;
   const int32_t* recent_len = ts.len;
   if (!q || !pool || !block_table || !seq_lens || !layer || !layout || !out || !workspace) return TQ_ENULL;
-  // n_split < 0: -n_split workgroups per sequence and KV head on average, dealt out by the lengths of the sequences
-  const bool by_length = n_split < 0;
-  const int n_asked = n_split < 0 ? -n_split : n_split;
-  n_split = n_asked;
-  if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || n_split <= 0 || n_split >= (1 << 20) || num_pages <= 0) return TQ_EINVAL;
+  // by_length: n_split workgroups per sequence and KV head on average, dealt out by the lengths of the sequences
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || n_split <= 0 || num_pages <= 0) return TQ_EINVAL;
+  if (by_length && n_split >= (1 << 20)) return TQ_EINVAL;
+  const int n_asked = n_split;
   if (B > 65535 || Hkv > 65535) return TQ_EUNSUPPORTED;
   // bt_stride > 0: a table row per sequence, that many entries; 0: one row shared by all sequences, length
   // unknown; < 0: one shared row of -bt_stride entries.  Lengths beyond the row are cut to it in the kernels.
@@ -1501,11 +1507,9 @@ extern "C" int tq_decode_attn_paged_ring(const void* q, int dtype, int B, int Hq
                                          const tq_page_layout* layout, const void* k_cache, const void* v_cache,
                                          int64_t cs_blk, int64_t cs_t, int64_t cs_h, int ring_rows, void* out,
                                          void* workspace, int n_split, void* stream) {
-  if (!k_cache || !v_cache) return TQ_ENULL;
-  if (ring_rows <= 0 || cs_blk <= 0 || cs_t <= 0 || cs_h <= 0) return TQ_EINVAL;
   TailSpec ts;
-  ts.k = k_cache; ts.v = v_cache; ts.rows = ring_rows;
-  ts.s_blk = cs_blk; ts.s_r = cs_t; ts.s_h = cs_h; ts.paged = true;
+  const int rc = ring_tail(ts, k_cache, v_cache, cs_blk, cs_t, cs_h, ring_rows);
+  if (rc) return rc;
   return decode_stages(q, dtype, B, Hq, Hkv, pool, num_pages, block_table, bt_stride, seq_lens, sm_scale, layer, layout,
                        ts, out, workspace, n_split, 7, stream);
 }
@@ -1519,6 +1523,33 @@ extern "C" int tq_decode_attn_paged(const void* q, int dtype, int B, int Hq, int
   return tq_decode_attn_paged_stages(q, dtype, B, Hq, Hkv, pool, num_pages, block_table, bt_stride, seq_lens, sm_scale,
                                      layer, layout, recent_k, recent_v, recent_rows, rs_b, rs_r, rs_h, recent_len, out,
                                      workspace, n_split, 7, stream);
+}
+
+extern "C" int tq_decode_attn_paged_by_length(const void* q, int dtype, int B, int Hq, int Hkv, const uint8_t* pool,
+                                              int64_t num_pages, const int32_t* block_table, int bt_stride,
+                                              const int32_t* seq_lens, float sm_scale, const tq_layer* layer,
+                                              const tq_page_layout* layout, const void* recent_k, const void* recent_v,
+                                              int recent_rows, int64_t rs_b, int64_t rs_r, int64_t rs_h,
+                                              const int32_t* recent_len, void* out, void* workspace, int n_split,
+                                              void* stream) {
+  TailSpec ts;
+  ts.k = recent_k; ts.v = recent_v; ts.rows = recent_rows;
+  ts.s_b = rs_b; ts.s_r = rs_r; ts.s_h = rs_h; ts.len = recent_len;
+  return decode_stages(q, dtype, B, Hq, Hkv, pool, num_pages, block_table, bt_stride, seq_lens, sm_scale, layer, layout,
+                       ts, out, workspace, n_split, 7, stream, true);
+}
+
+extern "C" int tq_decode_attn_paged_ring_by_length(const void* q, int dtype, int B, int Hq, int Hkv, const uint8_t* pool,
+                                                   int64_t num_pages, const int32_t* block_table, int bt_stride,
+                                                   const int32_t* seq_lens, float sm_scale, const tq_layer* layer,
+                                                   const tq_page_layout* layout, const void* k_cache, const void* v_cache,
+                                                   int64_t cs_blk, int64_t cs_t, int64_t cs_h, int ring_rows, void* out,
+                                                   void* workspace, int n_split, void* stream) {
+  TailSpec ts;
+  const int rc = ring_tail(ts, k_cache, v_cache, cs_blk, cs_t, cs_h, ring_rows);
+  if (rc) return rc;
+  return decode_stages(q, dtype, B, Hq, Hkv, pool, num_pages, block_table, bt_stride, seq_lens, sm_scale, layer, layout,
+                       ts, out, workspace, n_split, 7, stream, true);
 }
 
 // ---- the entry point that allocates nothing -----------------------------------------------------------

@@ -253,17 +253,17 @@ class PagedKVPool:
         bt = block_table.contiguous()
         bt_stride = -bt.shape[0] if bt.dim() == 1 else bt.shape[1]      # negative: one shared row of that length
         seq_lens = seq_lens.to(device=self.device, dtype=torch.int32).contiguous()
+        by_length = False
         if n_split is None:
             if max_len is None:
                 max_len = (bt.shape[-1]) * PAGE_TOKENS
             n_split = self.default_splits(B, max_len, Hq)
-            if workspace is None and not static_scratch and stages == 7 and self._shares_by_length(B, Hq):
-                n_split = -n_split             # that many workgroups per sequence on average, dealt out by length
+            by_length = workspace is None and not static_scratch and stages == 7 and self._shares_by_length(B, Hq)
         if static_scratch:
             if workspace is not None or stages != 7:
                 raise ValueError("static_scratch takes no workspace and runs all stages")
         elif workspace is None:
-            workspace = self.workspace(B, Hq, n_split)
+            workspace = self.workspace(B, Hq, -n_split if by_length else n_split)
         if out is None:
             out = torch.empty_like(query)
         rk_ptr = rv_ptr = rl_ptr = None
@@ -290,11 +290,13 @@ class PagedKVPool:
                     n_split, _ffi.stream_ptr(self.device)), "tq_decode_attn_paged_noalloc")
             return out
         with _ffi.on_device(self.device):
-            _ffi.check(_ffi.lib().tq_decode_attn_paged_stages(
+            entry, tail = (_ffi.lib().tq_decode_attn_paged_by_length, ()) if by_length else (
+                _ffi.lib().tq_decode_attn_paged_stages, (stages,))
+            _ffi.check(entry(
                 query.data_ptr(), _ffi.dtype_tag(query.dtype), B, Hq, self.num_kv_heads, self.data.data_ptr(),
                 self.num_pages, bt.data_ptr(), bt_stride, seq_lens.data_ptr(), float(scale), C.byref(ly),
                 C.byref(self.layout), rk_ptr, rv_ptr, rows, rs[0], rs[1], rs[2], rl_ptr, out.data_ptr(),
-                workspace.data_ptr(), n_split, stages, _ffi.stream_ptr(self.device)), "tq_decode_attn_paged")
+                workspace.data_ptr(), n_split, *tail, _ffi.stream_ptr(self.device)), "tq_decode_attn_paged")
         return out
 
     @staticmethod
@@ -335,19 +337,20 @@ class PagedKVPool:
         bt = block_table.contiguous()
         bt_stride = -bt.shape[0] if bt.dim() == 1 else bt.shape[1]      # negative: one shared row of that length
         seq_lens = seq_lens.to(device=self.device, dtype=torch.int32).contiguous()
+        by_length = False
         if n_split is None:
             if max_len is None:
                 max_len = (bt.shape[-1]) * PAGE_TOKENS
             n_split = self.default_splits(B, max_len, Hq)
-            if workspace is None and self._shares_by_length(B, Hq):
-                n_split = -n_split             # that many workgroups per sequence on average, dealt out by length
+            by_length = workspace is None and self._shares_by_length(B, Hq)
         if workspace is None:
-            workspace = self.workspace(B, Hq, n_split)
+            workspace = self.workspace(B, Hq, -n_split if by_length else n_split)
         if out is None:
             out = torch.empty_like(query)
         ly = self.quantizer._layer()
         with _ffi.on_device(self.device):
-            _ffi.check(_ffi.lib().tq_decode_attn_paged_ring(
+            entry = _ffi.lib().tq_decode_attn_paged_ring_by_length if by_length else _ffi.lib().tq_decode_attn_paged_ring
+            _ffi.check(entry(
                 query.data_ptr(), _ffi.dtype_tag(query.dtype), B, Hq, self.num_kv_heads, self.data.data_ptr(),
                 self.num_pages, bt.data_ptr(), bt_stride, seq_lens.data_ptr(), float(scale), C.byref(ly),
                 C.byref(self.layout), key_cache.data_ptr(), value_cache.data_ptr(), key_cache.stride(0),
