@@ -64,14 +64,14 @@ def _ragged_pool(gpu, d, key_bits, vb, H, lens, dtype, seed):
 
 
 # (head_dim, key bits, heads per KV head, KV heads, sequences): workgroups of 4 and of 8 wavefronts, a share per wavefront (more
-# pairs than workgroups fit), the merge in the launch and by a kernel of its own, more shares than one pass of the merge
+# pairs than workgroups fit), the merge in the launch, more shares than one pass of it takes
 @pytest.mark.parametrize("d,kb,G,H,B", [(128, 3, 4, 2, 3), (128, 3, 5, 8, 16), (128, 4, 5, 8, 97), (128, 3, 12, 8, 97),
                                         (64, 3, 4, 4, 200), (256, 3, 8, 2, 5), (256, 2, 4, 4, 90), (128, 2, 1, 1, 1024)])
 @pytest.mark.parametrize("ring", [0, 40])
 def test_shares_by_length_give_what_equal_shares_give(gpu, d, kb, G, H, B, ring):
-    """A step whose workgroups are dealt out by length against the same step with two equal shares per sequence: the same
-    sums in another order.  The weights are rounded to bf16 relative to another reference, so values differ by a few
-    bf16 half-steps of the largest weight: |difference| <= 2^-8 of the largest |value| of a row, and far less on average."""
+    """A step whose workgroups may be dealt out by length against the same step with two equal shares per sequence: the same
+    sums in another order, the weights rounded to bf16 relative to another reference.  Either is within 2^-7 of the largest |value|
+    of a row of the oracle's result (the bound of the decode tests), so they are within twice that of each other."""
     g = torch.Generator().manual_seed(B + d)
     longest = 9000 if B < 300 else 1500
     lens = [int(longest * 2.0 ** (-11.0 * float(x))) for x in torch.rand(B, generator=g)]
@@ -92,9 +92,80 @@ def test_shares_by_length_give_what_equal_shares_give(gpu, d, kb, G, H, B, ring)
     assert torch.equal(outs[0], outs[2])
     a, b = outs[0], outs[1]
     scale = b.abs().amax(-1, keepdim=True).clamp_min(1e-6)
-    assert float(((a - b).abs() / scale).max()) <= 2.0 ** -5 and float((a - b).norm() / b.norm()) <= 6e-3
+    assert float(((a - b).abs() / scale).max()) <= 2.0 ** -6 and float((a - b).norm() / b.norm()) <= 6e-3
     if B > 4:
-        assert ring or not a[1].any()                    # an empty sequence
+        assert not a[1].any()                            # an empty sequence
+
+
+# (head_dim, key bits, heads per KV head, KV heads, lengths of the few sequences): more than eight shares each, merged by a kernel of
+# its own from parts that lie where the most shares would end
+@pytest.mark.parametrize("d,kb,G,H,lens", [(128, 3, 4, 1, [30000, 900, 0]), (128, 3, 4, 2, [24001, 3000, 11, 24000, 7000]), (256, 3, 8, 1, [30011, 64, 2000]),
+                                           (256, 2, 4, 2, [20000, 100, 1, 0, 5000]), (64, 3, 4, 2, [30000, 2000]), (128, 5, 4, 2, [26000, 500, 1700])])
+@pytest.mark.parametrize("recent", [None, 128])
+def test_dozens_of_shares_by_length_against_the_oracle(gpu, d, kb, G, H, lens, recent):
+    from tests.test_gpu_parity import _decode_case
+    B, tail = len(lens), None
+    if recent:                                           # (with few groups of heads the exact tail is several parts)
+        tail = [recent, 3, 0, 77, recent][:B]
+    for seed in (1, 2):
+        _say(f"oracle, by length d={d} kb={kb} G={G} H={H} lens={lens} recent={tail}")
+        _decode_case(gpu, d, kb, 4, B, H * G, H, lens, tail, seed=seed)
+
+
+# one share per sequence, walked by four, two and one wavefronts, and 5-bit keys, whose operands are in LDS
+@pytest.mark.parametrize("d,kb,G,H,B", [(128, 3, 4, 8, 60), (128, 3, 4, 8, 97), (64, 3, 4, 8, 200), (256, 3, 8, 4, 60), (128, 5, 4, 8, 60)])
+@pytest.mark.parametrize("ring", [0, 40])
+@pytest.mark.parametrize("in_launch", [1, 0])
+def test_very_uneven_lengths_split_sequences_and_merge_them_either_way(gpu, d, kb, G, H, B, ring, in_launch):
+    """One long sequence among short ones: the schedule deals the long one out (the result is not that of equal shares bit for
+    bit), merged by the workgroup or wavefront that finishes last, or by a kernel of its own."""
+    from turboquant_amd import _ffi
+    lens = [6000] + [40 + 7 * b % 200 for b in range(B - 1)]
+    lens[5], lens[B // 2] = 0, 1
+    pool, table, seq, dg = _ragged_pool(gpu, d, kb, 4, H, lens, torch.bfloat16, B + d)
+    q = torch.randn(B, H * G, d, generator=dg, device=gpu).bfloat16()
+    exact = torch.randn(2, pool.num_pages, 16, H, d, generator=dg, device=gpu).bfloat16() if ring else None
+    _say(f"one long sequence d={d} kb={kb} G={G} H={H} B={B} ring={ring} in_launch={in_launch}")
+    n = pool.default_splits(B, 6000, H * G)
+    try:
+        _ffi.check(_ffi.lib().tq_set_option(b"merge_in_kernel", in_launch), "tq_set_option")
+        a, again, b = (_step(pool, q, table, seq, 6000, k, exact, ring).float() for k in (None, None, n))
+        torch.cuda.synchronize()
+    finally:
+        _ffi.check(_ffi.lib().tq_set_option(b"merge_in_kernel", 1), "tq_set_option")
+    assert torch.equal(a, again) and not torch.equal(a[0], b[0])
+    scale = b.abs().amax(-1, keepdim=True).clamp_min(1e-6)
+    assert float(((a - b).abs() / scale).max()) <= 2.0 ** -6            # (twice the bound against the oracle)
+    assert not a[5].any() and torch.equal(a[B // 2], b[B // 2])
+
+
+@pytest.mark.parametrize("d,H,G,B", [(128, 8, 4, 16), (128, 8, 4, 97), (256, 2, 8, 4)])
+def test_a_captured_step_reads_the_lengths_of_every_replay(gpu, d, H, G, B):
+    """Captured with one set of lengths and replayed with others - equal, uneven, empty sequences, shorter -, eager steps in between."""
+    N = 8000 if B < 50 else 1500
+    pool, table, seq, dg = _ragged_pool(gpu, d, 3, 4, H, [N] * B, torch.bfloat16, B)
+    q = torch.randn(B, H * G, d, generator=dg, device=gpu).bfloat16()
+    sets = [[N] * B, [max(1, int(N * 0.6 ** b)) for b in range(B)], [N if b == 1 else 0 for b in range(B)], [N // 3] * B,
+            [1 + (97 * b) % N for b in range(B)]]
+    lens, out = seq.clone(), torch.empty_like(q)
+    step = lambda o: pool.decode_attention(q, table, lens, max_len=N, out=o)
+    _say(f"captured step d={d} H={H} B={B}")
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step(out)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step(out)
+    for new in sets + sets[::-1]:
+        lens.copy_(_i32(new, gpu))
+        want = step(torch.empty_like(q))
+        torch.cuda.synchronize()
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), new
 
 
 def _step(pool, q, table, seq, longest, n_split, exact, ring):
@@ -264,3 +335,50 @@ def test_ragged_append_of_other_head_sizes(gpu, d, key_bits, B, H):
     assert torch.allclose(ma, mc, rtol=d * 2.0 ** -24, atol=0)
     pa.data[..., meta] = pc.data[..., meta]
     assert torch.equal(pa.data, pc.data)
+
+
+@pytest.mark.parametrize("d,key_bits,vb,dtype", [(64, 3, 2, torch.bfloat16), (320, 3, 4, torch.float16), (576, 4, 4, torch.bfloat16), (576, 4, 2, torch.float16),
+                                                 (384, 2, 4, torch.bfloat16), (704, 5, 2, torch.float16)])
+@pytest.mark.parametrize("layout", ["tokens first", "heads first", "every other token"])
+def test_odd_values_and_strides_at_other_head_sizes(gpu, d, key_bits, vb, dtype, layout):
+    """Infinities, NaN, zeros, the type's largest and smallest numbers, in rows that lie apart: the matrix-core quantiser and the chunked
+    value kernel (rows on a 16-byte boundary) against the vector-ALU kernels (one element further on), all bytes but those of
+    the residual norms, which agree but for the order of the sum."""
+    B, T, H = 2, 37, 3
+    g = torch.Generator(device=gpu).manual_seed(d + vb)
+    x = torch.randn(2, B, T, H, d, generator=g, device=gpu).to(dtype)
+    big, small = torch.finfo(dtype).max, torch.finfo(dtype).tiny
+    for t, odd in enumerate((float("inf"), -float("inf"), float("nan"), 0.0, big, -big, small)):
+        x[:, :, 2 * t, :, (5 * t + 3) % d] = odd
+    x[:, 0, 20], x[:, 0, 21], x[:, 1, 22], x[:, 1, 23], x[:, 1, 24] = 0, float("nan"), float("inf"), small, 7.0
+    x[:, 0, 25] = torch.finfo(dtype).smallest_normal * x[:, 0, 26].float().sign().to(dtype)
+    tq = TurboQuantProd(d, bits=key_bits, device=gpu)
+    table = torch.randperm(B * 4, generator=torch.Generator().manual_seed(3)).view(B, 4).to(torch.int32).to(gpu)
+    start = _i32([5, 0], gpu)
+    _say(f"odd values d={d} bits={key_bits}/{vb} {dtype} {layout}")
+    pools = []
+    for pad in (0, 1):
+        shape = {"tokens first": (2, B, T, H, d), "heads first": (2, B, H, T, d), "every other token": (2, B, 2 * T, H, d)}[layout]
+        n = 1
+        for k in shape:
+            n *= k
+        buf = torch.zeros(n + 16, dtype=dtype, device=gpu)
+        rows = buf[pad:pad + n].view(shape)
+        if layout == "heads first":
+            rows = rows.transpose(2, 3)
+        elif layout == "every other token":
+            rows = rows[:, :, ::2]
+        rows.copy_(x)
+        pool = PagedKVPool(tq, H, 8, value_bits=vb, dtype=dtype, device=gpu)
+        pool.append(rows[0], rows[1], table, start_pos=start)
+        pools.append(pool)
+    torch.cuda.synchronize()
+    L = pools[0].layout
+    a, b = (p.data.clone() for p in pools)
+    meta = slice(L.off_meta, L.off_meta + 8 * 16)
+    ma, mb = (p[..., meta].contiguous().view(torch.float32) for p in (a, b))
+    assert torch.equal(torch.nan_to_num(ma[..., 0::2], nan=-1.0), torch.nan_to_num(mb[..., 0::2], nan=-1.0))
+    assert torch.allclose(ma, mb, rtol=d * 2.0 ** -24, atol=0, equal_nan=True)
+    a[..., meta] = b[..., meta] = 0
+    assert torch.equal(a[..., L.off_vdata:], b[..., L.off_vdata:]), "values"
+    assert torch.equal(a, b), "keys"
