@@ -55,6 +55,14 @@ def test_split_matrices_sum_exactly_and_follow_the_documented_operand_order(d):
         _ffi.split_bf16x3(torch.zeros(48, 48))
 
 
+@pytest.mark.parametrize("d", [64, 192, 576])
+def test_several_matrices_are_split_as_each_by_itself(d):
+    m = torch.randn(3, d, d, generator=torch.Generator().manual_seed(d))
+    raw = _ffi.split_bf16x3(m)
+    for i in range(3):
+        assert raw[i].is_contiguous() and torch.equal(raw[i], _ffi.split_bf16x3(m[i]))
+
+
 @pytest.mark.parametrize("B", [1, 2, 3, 64, 1024, 1025])
 @pytest.mark.parametrize("n_split", [1, 2, 31, 256, 257, 512, 2048])
 def test_workspace_of_a_step_by_length_holds_the_equal_shares_it_may_fall_back_to(B, n_split):

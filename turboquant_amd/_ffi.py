@@ -220,22 +220,22 @@ def make_layer(d: int, mse_bits: int, Pi: torch.Tensor, PiT: torch.Tensor, centr
 
 
 def split_bf16x3(m: torch.Tensor) -> torch.Tensor:
-    """fp32 (d, d) matrix -> int16 tensor of bf16 bit patterns of three terms that sum
+    """fp32 (d, d) matrix, or (n, d, d) of them -> int16 tensor of bf16 bit patterns of three terms that sum
     to the matrix exactly (each term rounds the running remainder), in the operand order
     of the matrix-core quantise kernel: [term][row // 16][col // 32][(col % 32) // 8]
     [row % 16][col % 8], i.e. the 64 lanes' 16-byte MFMA operands of one (row tile,
     32-column slice) are contiguous.  d must be a multiple of 32."""
     rest = m.float()
-    d = rest.shape[0]
-    if rest.dim() != 2 or rest.shape[1] != d or d % 32:
-        raise ValueError("split_bf16x3 needs a square matrix whose size is a multiple of 32")
+    d = rest.shape[-1]
+    if rest.dim() not in (2, 3) or rest.shape[-2] != d or d % 32:
+        raise ValueError("split_bf16x3 needs square matrices whose size is a multiple of 32")
     parts = []
     for _ in range(3):
         term = rest.to(torch.bfloat16)
         parts.append(term)
         rest = rest - term.float()
-    t = torch.stack(parts).view(3, d // 16, 16, d // 32, 4, 8)      # term, row tile, n, kblk, kb, j
-    return t.permute(0, 1, 3, 4, 2, 5).contiguous().view(torch.int16)
+    t = torch.stack(parts, dim=-3).unflatten(-1, (d // 32, 4, 8)).unflatten(-4, (d // 16, 16))  # term, row tile, n, kblk, kb, j
+    return t.movedim(-4, -2).contiguous().view(torch.int16)
 
 
 FP6_TERMS = 5
