@@ -48,6 +48,33 @@ def test_ragged_append_numbers_only_the_pages_that_exist(gpu, d, B, H):
     assert int((pa.data != 0).sum()) > 0
 
 
+# 256 compute units: up to 1024 tiles at head_dim 128 and 512 at 256 every group of tiles has one to itself, and no index is built
+@pytest.mark.parametrize("d,H,B,max_run", [(128, 8, 2, 1009), (128, 8, 2, 1010), (256, 4, 2, 1009), (256, 4, 2, 1010), (128, 3, 7, 770)])
+def test_ragged_append_of_few_sequences_with_and_without_the_index(gpu, d, H, B, max_run):
+    """The longest run first, last or in the middle, an empty one and one of a single token: against one append per sequence, byte for
+    byte (the kernels and their arithmetic are the same, only the numbering of the tiles differs)."""
+    g = torch.Generator().manual_seed(d + max_run)
+    width = max_run // 16 + 3
+    k, v = (torch.randn(max_run + 64, H, d, generator=g).bfloat16().to(gpu) for _ in range(2))
+    tq = TurboQuantProd(d, bits=3, device=gpu)
+    for long_at in sorted({0, B // 2, B - 1}):
+        runs = [(1, 0, 15, 16, 17, 0, 2)[b % 7] for b in range(B)]
+        runs[long_at] = max_run - 1 if long_at else max_run
+        row0 = [sum(runs[:b]) for b in range(B)]
+        starts = [int(x) for x in torch.randint(0, 17, (B,), generator=g)]
+        table = torch.randperm(B * width, generator=g).view(B, width).to(torch.int32).to(gpu)
+        pa, pb = (PagedKVPool(tq, H, B * width, value_bits=2, dtype=torch.bfloat16, device=gpu) for _ in range(2))
+        _say(f"few ragged runs d={d} H={H} runs={runs}")
+        pa.append_ragged(k, v, _i32(row0, gpu), _i32(runs, gpu), _i32(starts, gpu), table, max_run=max_run)
+        for b in range(B):
+            if runs[b]:
+                rows = slice(row0[b], row0[b] + runs[b])
+                pb.append(k[None, rows], v[None, rows], table[b:b + 1], start_pos=_i32([starts[b]], gpu))
+        torch.cuda.synchronize()
+        assert torch.equal(pa.data, pb.data)
+        assert int((pa.data != 0).sum()) > 0
+
+
 def _ragged_pool(gpu, d, key_bits, vb, H, lens, dtype, seed):
     g = torch.Generator(device=gpu).manual_seed(seed)
     tq = TurboQuantProd(d, bits=key_bits, device=gpu)

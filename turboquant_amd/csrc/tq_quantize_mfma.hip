@@ -709,7 +709,7 @@ static int launch_dt_d(const void* x, const Source& src, const tq_layer& ly, con
   using Sm = KeySmem<DT, D>;
   // Few tiles, written to pages (the page write of a decode step: a token per sequence): a workgroup per tile, which
   // then computes that tile only, while they all fit the card at once
-  if constexpr (ML == Gm::MT && std::is_same<Sink, KeyPagedSink>::value && !MSE_ONLY) {
+  if constexpr (ML == Gm::MT && std::is_same<Sink, KeyPagedSink>::value && !std::is_same<Source, RaggedSource>::value && !MSE_ONLY) {
     const int opt = opt_append_small.load(std::memory_order_relaxed);
     if (opt != 0 && tiles <= (opt < 0 ? 2 * (int64_t)device_compute_units() : (int64_t)opt))
       return launch_dt_d<DT, D, MSE_ONLY, FX, Source, Sink, 1>(x, src, ly, sink, tiles, st);
@@ -758,7 +758,11 @@ int launch_key_mfma(const void* x, int dtype, const Source& src, const tq_layer&
   if (!aligned_for_chunks(x, dtype, src) || !sink_ok(sink, mse_only)) return TQ_EUNSUPPORTED;
   constexpr bool paged = std::is_same<Sink, KeyPagedSink>::value;     // pages always hold the full code
   if constexpr (std::is_same<Source, PagedSource>::value) {
-    if (src.compact) {
+    // where every group of tiles, absent ones too, has a compute unit to itself the index only delays them: head_dim 128, 8 KV heads,
+    // eight prompts of 15 .. 30 tokens 16.0 us with it and 14.8 without, eighteen of 5 .. 57 (720 tiles) 22.9 and 20.2; beyond, forty
+    // of 2 .. 100 (2560 tiles) 26.3 and 36.0, though forty of 100 each 40.5 and 36.8: the lengths are in device memory
+    const int tiles_per_group = ly.d == 128 ? KeyGeom<128>::MT : KeyGeom<256>::MT;
+    if (src.compact && tiles > tiles_per_group * (int64_t)device_compute_units()) {
       RaggedSource ragged;
       static_cast<PagedSource&>(ragged) = src;
       return launch_key_mfma<RaggedSource, Sink>(x, dtype, ragged, ly, sink, mse_only, tiles, st);
