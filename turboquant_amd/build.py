@@ -27,7 +27,7 @@ FLAGS = [
     # the kernels call fmaf() explicitly wherever a fused multiply-add is wanted
     "-ffp-contract=off",
     # the first 14 argument dwords of a kernel arrive in registers: a launch does not begin with a memory latency
-    # (16 x 8192 tokens, 32 q / 8 KV heads of 128: 40.3 -> 39.8 us per decode step)
+    # (14 decode steps of 24 - 72 us: 0.1 - 0.5 us each; 16 x 8192 tokens, 32 q / 8 KV heads of 128: 38.7 -> 38.6)
     "-mllvm", "-amdgpu-kernarg-preload-count=16",
     "-fno-gpu-rdc", "-Wall", "-Wno-unused-function",
     # the LDS-direct loads name m0 in their clobber lists, which the compiler reports as a reserved register

@@ -5,17 +5,19 @@
 // reference (quantizer.py:141,160,248) are assembled from bf16 products with fp32 accumulation, and the pairs of terms
 // (a, b) with a + b > 2, which are below fp32 resolution, are left out.
 //
-// What bounds it: the matrices.  A workgroup reads all three of them - three terms each, 6 MB at d = 576 - for every
-// group of vectors, more than an L2 slice holds beside the pages, at the 64 bytes per clock that a compute unit takes
-// from L2 (about 40 us for 6 MB), against 32 us of MFMA for 32 vectors.  Hence the widest group whose terms fit the LDS
+// What bounds it: nothing alone.  A workgroup reads all three matrices - three terms each, 6.8 MB at d = 576 with what it
+// reads twice - for every group of vectors, at the 64 bytes per clock that a compute unit takes from L2 (44 us), beside 32 us of
+// MFMA and about 26 us of vector instructions for 32 vectors; these overlap within a contraction and not across its ends, where
+// all wavefronts meet, and the contractions are three fifths of the kernel's time.  Hence the widest group whose terms fit the LDS
 // (32 vectors: 3 x 32 x 1168 bytes at d = 576), one workgroup of up to 12 wavefronts per compute unit, each of which
 // owns NPW column tiles for all vectors, and a ring of two slices per wavefront (2 x NPW x 3 KB) that is refilled while the
-// other slice is multiplied - across the ends of the contractions, so the first slices of the next matrix are
-// there when it begins.
+// other slice is multiplied - from the second contraction into the third across its end, so that the first slices of S are
+// there when it begins; behind the first and the third, where single coordinates may be summed again, it is filled anew (kept
+// through those sums it spills: 116 - 130 us where 88 were measured without them).
 // The codes are those of the vector-ALU kernel, byte for byte: what rounding could decide is summed again in its order (see
 // KW_NEAR_Y).
-// Appends of 8192 vectors of 576, bf16, 4-bit keys: 404 us on the vector-ALU kernel, 119 us here; one token of each of 32
-// sequences 181 -> 74 us; 8192 x 320: 129 -> 49, x 704: 515 -> 177.
+// Appends of 8192 vectors of 576, bf16, 4-bit keys: 404 us on the vector-ALU kernel, 118 us here; one token of each of 32
+// sequences 181 -> 74 us; 8192 x 320: 129 -> 48, x 704: 515 -> 172.
 
 #include <atomic>
 
