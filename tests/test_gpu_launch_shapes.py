@@ -5,6 +5,8 @@ import torch
 
 from turboquant_amd.paged import PagedKVPool
 from turboquant_amd.quantizer import TurboQuantProd
+from tests.test_gpu_parity import _decode_case, _make_pool
+from tests.test_gpu_parity_scores import _set_option
 
 pytestmark = pytest.mark.gpu
 
@@ -409,3 +411,87 @@ def test_odd_values_and_strides_at_other_head_sizes(gpu, d, key_bits, vb, dtype,
     a[..., meta] = b[..., meta] = 0
     assert torch.equal(a[..., L.off_vdata:], b[..., L.off_vdata:]), "values"
     assert torch.equal(a, b), "keys"
+
+
+# ------------------------------------------------------------------ sixteen query heads per wavefront (head_dim 512 / 576)
+@pytest.mark.parametrize("d,key_bits,vb,Hq,Hkv,dtype,lens,recent,n_split", [
+    (576, 4, 4, 9, 1, torch.bfloat16, [1, 33, 200], None, 1),                  # one tile, 7 columns without a head; a sequence of one token
+    (576, 4, 4, 16, 1, torch.bfloat16, [700, 96, 97], None, None),             # one full tile: three blocks side by side, a last turn with one
+    (576, 3, 2, 17, 1, torch.float16, [300, 31], [0, 9], 2),                   # two tiles, the second with one head; fp16 pages; exact tail
+    (576, 4, 2, 64, 2, torch.bfloat16, [513, 64], None, 4),                    # two KV heads of two tiles; splits without tokens
+    (576, 3, 4, 40, 1, torch.bfloat16, [2100, 5], None, 1),                    # three tiles: a pair of wavefronts without heads; the table registers move on
+    (576, 4, 4, 65, 1, torch.float16, [130, 32], None, 3),                     # five tiles: two workgroups, the second with three idle pairs
+    (576, 4, 4, 128, 1, torch.bfloat16, [400, 16, 15], [3, 0, 7], 2),          # eight tiles, exact tail
+    (512, 4, 4, 128, 1, torch.float16, [300, 77], None, None),                 # lane-major key words
+    (512, 3, 2, 24, 1, torch.bfloat16, [257, 480], None, 2),
+    (512, 3, 4, 12, 1, torch.bfloat16, [64, 1000], None, 5),
+    (512, 4, 2, 80, 2, torch.bfloat16, [129, 31], [7, 0], None)])
+def test_more_than_eight_heads_per_wide_kv_head(gpu, d, key_bits, vb, Hq, Hkv, dtype, lens, recent, n_split):
+    """Decode at head_dim 512 / 576 with 9 .. 128 query heads per KV head: every sequence against the oracle on the same
+    store, and against the kernel that takes 8 heads per workgroup (operands not packed ahead).  Both round the weighted scales
+    to bf16 (2^-9 each) and agree in everything else to fp32: 2^-7 of the largest output bounds two such sums."""
+    out = {}
+    try:
+        for pre in (1, 0):
+            _set_option("wide_prepack", pre)
+            out[pre] = _decode_case(gpu, d, key_bits, vb, len(lens), Hq, Hkv, lens, recent, seed=40 + Hq + d, n_split=n_split,
+                                    dtype=dtype, return_out=True).float()
+    finally:
+        _set_option("wide_prepack", 1)
+    assert float((out[1] - out[0]).abs().max()) <= 2.0 ** -7 * float(out[0].abs().max())
+
+
+@pytest.mark.parametrize("case", ["page", "all", "scale"])
+def test_sixteen_heads_per_wavefront_and_slots_without_tokens(gpu, case):
+    """Table entries outside the pool give their tokens no weight, and page slots behind a sequence's last token may hold
+    anything (infinite scales and zero points, NaN norms): the results are those of the tokens that exist."""
+    d, Hq, N = 576, 32, 200
+    pool, tq = _make_pool(gpu, d, 4, 4, 1, 16, torch.bfloat16)
+    g = torch.Generator().manual_seed(5)
+    k, v = (torch.randn(1, N, 1, d, generator=g).bfloat16().to(gpu) for _ in range(2))
+    q = torch.randn(1, Hq, d, generator=g).bfloat16().to(gpu)
+    table = torch.arange(13, dtype=torch.int32, device=gpu)[None]
+    pool.append(k, v, table)
+    seq = torch.tensor([N], dtype=torch.int32, device=gpu)
+    want = pool.decode_attention(q, table, seq, n_split=2, max_len=N)
+    if case == "scale":
+        L = pool.layout
+        page = pool.data[12, 0]                                   # tokens 192 .. 207, eight of them written
+        page[L.off_meta + 64:L.off_meta + 128] = 0xff             # (NaN)
+        for off in (L.off_vscale, L.off_vzero):
+            sect = page[off:off + 2 * 18 * 16].view(torch.int16).view(18, 16)
+            sect[:, 8:] = 0x7f80                                  # (infinity)
+        assert torch.equal(pool.decode_attention(q, table, seq, n_split=2, max_len=N), want)
+        return
+    bad = table.clone()
+    if case == "all":
+        bad[:] = 99
+        assert torch.count_nonzero(pool.decode_attention(q, bad, seq, n_split=2, max_len=N)) == 0
+        return
+    bad[0, 12] = -1                                               # the last page: what is left is the sequence of 192 tokens
+    short = torch.tensor([192], dtype=torch.int32, device=gpu)
+    assert torch.equal(pool.decode_attention(q, bad, seq, n_split=1, max_len=N), pool.decode_attention(q, table, short, n_split=1, max_len=N))
+
+
+@pytest.mark.parametrize("d,Hq,B,dtype", [(576, 8, 40, torch.bfloat16), (576, 5, 53, torch.float16), (704, 8, 33, torch.bfloat16),
+                                          (320, 7, 80, torch.bfloat16), (576, 128, 3, torch.bfloat16), (576, 128, 17, torch.float16),
+                                          (512, 100, 21, torch.bfloat16), (640, 3, 200, torch.float16)])
+def test_rotation_of_hundreds_of_rows(gpu, d, Hq, B, dtype):
+    """Steps whose rotation passes over the row tiles with the matrix terms in LDS (265 .. 2176 rows, shares of one to three
+    tiles per wavefront, a last tile that is not full): the operands are those of the vector-ALU rotation to rounding (sums in another order),
+    so the outputs agree within a rounding step of the output type."""
+    pool, tq = _make_pool(gpu, d, 4, 4, 1, 6, dtype)
+    g = torch.Generator().manual_seed(d + Hq)
+    k, v = (torch.randn(1, 90, 1, d, generator=g).to(dtype).to(gpu) for _ in range(2))
+    table = torch.arange(6, dtype=torch.int32, device=gpu)
+    pool.append(k, v, table[None])
+    q = torch.randn(B, Hq, d, generator=g).to(dtype).to(gpu)
+    seq = torch.randint(1, 91, (B,), generator=g).to(torch.int32).to(gpu)
+    outs = []
+    try:
+        for opt in (1, 0):
+            _set_option("prep_mfma", opt)
+            outs.append(pool.decode_attention(q, table, seq, n_split=1, max_len=90).float())
+    finally:
+        _set_option("prep_mfma", 1)
+    assert float((outs[0] - outs[1]).abs().max()) <= 2.0 ** -7 * float(outs[1].abs().max())

@@ -1233,6 +1233,12 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
     wide_pre.q_stat = q_stat;
     wide_pre.Hq = Hq; wide_pre.Hkv = Hkv; wide_pre.kv_div = kv_div; wide_pre.ntp = decode_wide_term_planes(*layer);
     wide_pre.sm_scale = sm_scale;
+    // more than 8 heads per KV head at the sizes of latent attention: tiles of sixteen heads for a kernel of their own
+    if (decode_heads_has_kernel(*layer, *layout, G) && (G + 15) / 16 * heads_qa_words(d) <= kv_div * wide_pre.ntp * 2 * wide_qa_stride(d)) {
+      wide_pre.heads = true;
+      wide_pre.kv_div = (G + 15) / 16;
+      wide_pre.ntp = 2;
+    }
   }
 
   if (tail && ts.paged && !words) return TQ_EUNSUPPORTED;       // a paged exact cache has to be word-aligned
@@ -1431,7 +1437,9 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
   if (mf == TQ_OK && fm.out != nullptr) return TQ_OK;         // merged in the launch
   // head sizes above 256: the matrix-core kernel that works on a block per workgroup
   if ((stages & 2) && mf == TQ_EUNSUPPORTED) {
-    mf = launch_decode_wide(q_rot, q_sk, B, Hq, Hkv, pool, block_table, bt_stride, seq_lens, sm_scale, *layer, *layout,
+    mf = wide_pre.heads ? launch_decode_heads(B, Hq, Hkv, pool, block_table, bt_stride, seq_lens, *layer, *layout, parts, n_parts,
+                                              n_split, len_sub, max_pages, pool_pages, wide_pre, st)
+                        : launch_decode_wide(q_rot, q_sk, B, Hq, Hkv, pool, block_table, bt_stride, seq_lens, sm_scale, *layer, *layout,
                             parts, n_parts, n_split, len_sub, max_pages, pool_pages, wide_pre, st);
     if (mf > 0) return mf;
   }

@@ -164,7 +164,19 @@ struct WidePack {
   float* q_stat = nullptr;
   int Hq = 0, Hkv = 0, kv_div = 1, ntp = 0;
   float sm_scale = 0.0f;
+  // Operands of the kernel for dozens of heads per KV head instead (tq_decode_heads.hip): kv_div tiles of sixteen heads, and per
+  // tile [rotated, sketched][term pair][64 coordinates] operands of HQ_OP dwords ([64 lanes][4] then [64 lanes][2]),
+  // lane = head + 16 (term % 2) + 32 (word % 2); no codebook coefficient in them (ntp = 2 "planes").
+  bool heads = false;
 };
+constexpr int HQ_OP = 64 * 6;
+__host__ __device__ constexpr int heads_qa_words(int d) { return 4 * (d / 64) * HQ_OP; }     // dwords per tile of sixteen heads
+
+// The matrix-core kernel for more than 8 query heads per KV head at head_dim 512 / 576 (tq_decode_heads.hip)
+bool decode_heads_has_kernel(const tq_layer& ly, const tq_page_layout& L, int g_tot);
+int launch_decode_heads(int B, int Hq, int Hkv, const uint8_t* pool, const int32_t* block_table, int bt_stride,
+                        const int32_t* seq_lens, const tq_layer& ly, const tq_page_layout& L, float* parts, int n_parts,
+                        int n_split, int len_sub, int max_pages, int num_pages, const WidePack& pre, hipStream_t st);
 
 // The matrix-core kernel for head sizes above 256 (tq_decode_wide.hip; a workgroup per block of 32 tokens): reads the
 // fp32 rotated / sketched queries the general kernel reads and writes the same partials.  TQ_EUNSUPPORTED when the

@@ -580,8 +580,9 @@ constexpr int ROT_COLS = 32;          // output columns (one plane word) of a ro
 
 // coefficient of term plane tp as the wide-head page kernel orders them: the index planes from the highest bit down,
 // the multi-bit Walsh terms, the sign plane
-__device__ __forceinline__ float wide_term_plane_coef(const tq_layer& ly, int ntp, int tp) {
-  const int mb = ly.mse_bits;
+__device__ __forceinline__ float wide_term_plane_coef(const tq_layer& ly, const WidePack& wp, int tp) {
+  if (wp.heads) return 1.0f;                       // (operands without coefficients)
+  const int mb = ly.mse_bits, ntp = wp.ntp;
   float coef = 1.0f;                               // the sign plane
   if (tp < mb) {
     coef = 0.0f;
@@ -600,33 +601,43 @@ __device__ __forceinline__ float wide_term_plane_coef(const tq_layer& ly, int nt
   return coef;
 }
 
+// the largest coefficient that the rotated query meets in its operands
+__device__ __forceinline__ float wide_coef_bound(const tq_layer& ly, const WidePack& wp) {
+  float cmax = wp.heads ? 1.0f : 0.0f;
+  if (!wp.heads)
+    for (int t = 0; t < ly.n_terms; ++t) cmax = fmaxf(cmax, fabsf(ly.term_coef[t]));
+  return cmax;
+}
+
 // PACK epilogue of the rotation kernels: plane word j (32 coordinates) of nr query rows from row0 on, as the wide-head
-// page kernel's fp6 operands.  s_rot / s_sk: [row][32] rotated / sketched values of the word; s_rs: [row][2] the
+// page kernel's fp6 operands.  s_rot / s_sk: [row][LD] rotated / sketched values of the word; s_rs: [row][2] the
 // rows' multipliers; s_cf: coefficient of each term plane.
+template <int LD = ROT_COLS>
 __device__ __forceinline__ void wide_pack_word(const WidePack& wp, int d, int nr, int row0, int j, const float* s_rot,
                                                const float* s_sk, const float* s_rs, const float* s_cf, int tid,
                                                int n_threads, int tp_begin, int tp_end) {
   // one lane per (term plane, row): the word's 32 values as four fp6 terms (the packing conversion of gfx950 and its
   // inverse for the residual), written where lane (row 2 g + term % 2, quarter word % 4) of operand (plane, row set
-  // term / 2, chunk word / 4) of the row's head group reads them
+  // term / 2, chunk word / 4) of the row's head group reads them - for the kernel of dozens of heads: lane (head + 16 (term % 2) +
+  // 32 (word % 2)) of operand (product, term / 2, word / 2) of the row's tile of sixteen heads
   typedef float f32x16_t __attribute__((ext_vector_type(16)));
   typedef float f32x32_t __attribute__((ext_vector_type(32)));
   typedef uint32_t u32x6_t __attribute__((ext_vector_type(6)));
   const int ntp = wp.ntp;
-  const int qa_stride = wide_qa_stride(d);
-  const bool half_op = (d & 127) != 0 && (j >> 2) == ((d + 127) >> 7) - 1;
+  const int qa_stride = wp.heads ? (d >> 6) * HQ_OP : wide_qa_stride(d);
+  const bool half_op = !wp.heads && (d & 127) != 0 && (j >> 2) == ((d + 127) >> 7) - 1;
   const int hi_at = half_op ? 32 * 4 : 64 * 4;
   for (int it = tp_begin * nr + tid; it < tp_end * nr; it += n_threads) {      // (term planes tp_begin .. tp_end - 1)
     const int tp = it / nr, r = it - tp * nr;
     const bool is_sign = tp == ntp - 1;
-    // the row's place: sequence, head, group of at most 8 heads of its KV head, slot in the group
+    // the row's place: sequence, head, group of at most 8 heads (tile of sixteen) of its KV head, slot in the group
     const int row = row0 + r;                        // (32-bit arithmetic: the launcher checks the row count)
     const int bq = row / wp.Hq, head = row - bq * wp.Hq;
     const int g_tot = wp.Hq / wp.Hkv, kvh = head / g_tot, hh = head - kvh * g_tot;
-    const int g_max = (g_tot + wp.kv_div - 1) / wp.kv_div, grp = hh / g_max, g = hh - grp * g_max;
+    const int g_max = wp.heads ? 16 : (g_tot + wp.kv_div - 1) / wp.kv_div, grp = hh / g_max, g = hh - grp * g_max;
     const int64_t group = ((int64_t)bq * wp.Hkv + kvh) * wp.kv_div + grp;
     const float base = 4.0f * (is_sign ? s_rs[2 * r + 1] : s_cf[tp] * s_rs[2 * r]);
-    const float4* src = (const float4*)((is_sign ? s_sk : s_rot) + r * ROT_COLS);
+    const float4* src = (const float4*)((is_sign ? s_sk : s_rot) + r * LD);
     float x[32];
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
@@ -642,16 +653,17 @@ __device__ __forceinline__ void wide_pack_word(const WidePack& wp, int d, int nr
       if (kloc & 1) vb[kloc >> 1] = v;
       else va[kloc >> 1] = v;
     }
-    uint32_t* op0 = wp.qa + group * (int64_t)(ntp * 2 * qa_stride) + (tp * 2) * qa_stride + (j >> 2) * WD_QA_OP;
-    const int slot0 = 2 * g + 16 * (j & 3);
+    uint32_t* op0 = wp.qa + group * (int64_t)(ntp * 2 * qa_stride) + (tp * 2) * qa_stride + (wp.heads ? j >> 1 : j >> 2) * WD_QA_OP;
+    const int slot0 = wp.heads ? g + 32 * (j & 1) : 2 * g + 16 * (j & 3), step = wp.heads ? 16 : 1;
     const float one = 1.0f;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       u32x6_t code;
       asm volatile("v_cvt_scalef32_2xpk16_fp6_f32 %0, %1, %2, %3" : "=&v"(code) : "v"(va), "v"(vb), "v"(one));
       uint32_t* op = op0 + (t >> 1) * qa_stride;
-      *(uint4*)(op + (slot0 + (t & 1)) * 4) = make_uint4(code[0], code[1], code[2], code[3]);
-      *(uint2*)(op + hi_at + (slot0 + (t & 1)) * 2) = make_uint2(code[4], code[5]);
+      const int slot = slot0 + (t & 1) * step;
+      *(uint4*)(op + slot * 4) = make_uint4(code[0], code[1], code[2], code[3]);
+      *(uint2*)(op + hi_at + slot * 2) = make_uint2(code[4], code[5]);
       if (t < 3) {
         f32x32_t rr;
         asm volatile("v_cvt_scalef32_pk32_f32_fp6 %0, %1, %2" : "=&v"(rr) : "v"(code), "v"(one));
@@ -794,7 +806,7 @@ __device__ __forceinline__ void rotate_mfma_body(const uint16_t* __restrict__ q,
     const int r = o >> 5, c = o & 31;
     const float v = part[r * ROTM_LD + c] + part[(16 + r) * ROTM_LD + c];
     s_val[o] = v;
-    if (r < nr) dst[(row0 + r) * D + word * ROT_COLS + c] = v;
+    if (r < nr && !wp.heads) dst[(row0 + r) * D + word * ROT_COLS + c] = v;
   }
   if (tid < 16) {                                                      // the statistics of row tid
     const int r = tid;
@@ -808,8 +820,7 @@ __device__ __forceinline__ void rotate_mfma_body(const uint16_t* __restrict__ q,
     float* st = wp.q_stat + (row0 + r) * 4;
     // bound < 2^e: e = exponent field - 126, kept within +-100
     if (m == 0) {
-      float cmax = 0.0f;
-      for (int t = 0; t < ly.n_terms; ++t) cmax = fmaxf(cmax, fabsf(ly.term_coef[t]));
+      const float cmax = wide_coef_bound(ly, wp);
       const int e1 = min(max((int)((__float_as_uint(fabsf(k) * nq * cmax) >> 23) & 255u) - 126, -100), 100);
       s_rs[2 * r] = k * __uint_as_float((uint32_t)(127 - e1) << 23);
       if (word == 0 && r < nr) { st[0] = (float)e1; st[2] = k * ly.term_const * s1; }
@@ -819,7 +830,7 @@ __device__ __forceinline__ void rotate_mfma_body(const uint16_t* __restrict__ q,
       if (word == 0 && r < nr) { st[1] = (float)e2; st[3] = -k * ly.qjl_scale * s1; }
     }
   } else if (tid >= 64 && tid < 80) {
-    s_cf[tid - 64] = wide_term_plane_coef(ly, wp.ntp, tid - 64);
+    s_cf[tid - 64] = wide_term_plane_coef(ly, wp, tid - 64);
   }
   __syncthreads();
   // the index and term planes from the rotated values, the sign plane from the sketched ones
@@ -827,142 +838,168 @@ __device__ __forceinline__ void rotate_mfma_body(const uint16_t* __restrict__ q,
                  m ? wp.ntp : wp.ntp - 1);
 }
 
-// The same rotation for thousands of rows (more workgroups than the card holds at once): a workgroup takes `tpw`
-// consecutive row tiles of its (plane word, product) pair against ONE fetch of the matrix terms and column sums
-// (2048 rows at head_dim 576 as a workgroup per tile pulled 560 MB of terms through the L2s: 61 us, now 46).  First every tile's
-// products, sums and statistics - the matrix terms stay in registers, the halves meet in LDS buffers that alternate
-// by tile, the results wait in LDS -, then the packing of all tiles, which needs the registers the terms held.
-constexpr int ROTM_MAX_TPW = 16;
-__host__ __device__ inline int rotate_mfma_tiles_smem_floats(int tpw) {
-  return 2 * (2 * 16 * ROTM_LD + 4 * 16 * 2) + tpw * (16 * ROT_COLS + 2 * 16) + 16;
+// The same rotation for hundreds of rows and more: a workgroup takes one (plane word, product) pair, whose matrix terms it
+// copies to LDS once, and its wavefronts pass over the row tiles of the workgroup's share, NT at a time against one read of a
+// term, whole contractions each: no wavefront waits for another after the copy.  With two tiles LDS reads and MFMAs are level (a term
+// of a kilobyte, eight clocks of the compute unit's LDS, feeds NT products of sixteen clocks of one of its four matrix units).  fp16 queries as two bf16 terms, as above.
+// 2048 rows at head_dim 576: 41 -> 23 us, 512 rows: 16 -> 11 us (before: the terms in registers, a barrier and the statistics
+// in every tile, fp16 queries on the vector ALU).  What is left is the packing and the ends of a launch of one round.
+constexpr int ROTR_WAVES = 8, ROTR_LD = 36;
+__host__ __device__ constexpr int rotate_rows_pack_tiles(int d) { return d <= 576 ? 2 : 1; }      // (what LDS has room for beside the terms)
+__host__ __device__ constexpr int rotate_rows_smem_bytes(int d) {
+  return 3 * 2 * (d / 32) * 1024 + ROTR_WAVES * rotate_rows_pack_tiles(d) * (16 * ROTR_LD + 16 * 2) * 4 + (16 + d) * 4;
 }
 
-template <int KPW>
-__device__ __forceinline__ void rotate_mfma_tiles_body(const uint16_t* __restrict__ q, int64_t rows, int n_tiles, int tpw,
-                                                       const tq_layer& ly, float* __restrict__ q_rot,
-                                                       float* __restrict__ q_sk, const WidePack& wp, int id, float* sm) {
+template <int KPW, bool F16Q, int NT>
+__device__ __forceinline__ void rotate_rows_body(const uint16_t* __restrict__ q, int64_t rows, int n_tiles, int n_groups,
+                                                 const tq_layer& ly, float* __restrict__ q_rot, float* __restrict__ q_sk,
+                                                 const WidePack& wp, int id, unsigned char* smem) {
   constexpr int KS = 2 * KPW, D = 32 * KS;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, kb = lane >> 4;
-  const int jt = wave & 1, kh = wave >> 1;
-  const int n_tg = (n_tiles + tpw - 1) / tpw;
-  const int pair = (id & 7) + 8 * ((id >> 3) / n_tg);              // (pair p on die p % 8, as in rotate_mfma_body)
+  const int pair = (id & 7) + 8 * ((id >> 3) / n_groups);            // (pair p on die p % 8, as in rotate_mfma_body)
   if (pair >= 2 * KS) return;
-  const int word = pair >> 1, m = pair & 1;
-  const int tile0 = ((id >> 3) % n_tg) * tpw, tile1 = min(tile0 + tpw, n_tiles);
-  float* part = sm;                                  // [2 buffers][kh][16 rows][ROTM_LD]
-  float* s_st = part + 2 * 2 * 16 * ROTM_LD;         // [2 buffers][4 wavefronts][16 rows][2]
-  float* s_val = s_st + 2 * 4 * 16 * 2;              // [tpw][16][32]
-  float* s_rs = s_val + tpw * 16 * ROT_COLS;         // [tpw][16][2]
-  float* s_cf = s_rs + tpw * 2 * 16;                 // [16]
-  constexpr int NS = (KPW + 1) / 2;
-  const float* colsum = m ? ly.S_colsum : ly.Pi_colsum;
-  prep_f32x4 cs[NS][2];
-#pragma unroll
-  for (int i = 0; i < NS; ++i) {
-    const int kl = jt + 2 * i < KPW ? jt + 2 * i : 0;
-    const int ks = kh * KPW + kl;
-    cs[i][0] = *(const prep_f32x4*)(colsum + ks * 32 + kb * 8);
-    cs[i][1] = *(const prep_f32x4*)(colsum + ks * 32 + kb * 8 + 4);
-  }
-  prep_u32x4 ma[3][KPW];
+  const int word = pair >> 1, m = pair & 1, grp = (id >> 3) % n_groups;
+  const int tile0 = (int)((int64_t)n_tiles * grp / n_groups), tile1 = (int)((int64_t)n_tiles * (grp + 1) / n_groups);
+  uint16_t* mat = (uint16_t*)smem;                                   // [3 terms][2 halves of the word][KS][64 lanes][8]
+  constexpr int PT = rotate_rows_pack_tiles(D);
+  static_assert(rotate_rows_smem_bytes(D) <= 160 * 1024, "LDS");
+  float* s_val = (float*)(smem + 3 * 2 * KS * 1024) + wave * PT * (16 * ROTR_LD + 16 * 2);      // [PT tiles][16 rows][ROTR_LD]
+  float* s_rs = s_val + PT * 16 * ROTR_LD;                           // [PT tiles][16 rows][2] multipliers of q_rot / q_sk
+  float* s_cf = (float*)(smem + 3 * 2 * KS * 1024) + ROTR_WAVES * PT * (16 * ROTR_LD + 16 * 2);      // [16]
+  float* s_cs = s_cf + 16;                                           // [D] column sums, for the workgroups that write the statistics
   {
-    const uint16_t* mat = m ? ly.S_split : ly.Pi_split;
+    const uint16_t* src = m ? ly.S_split : ly.Pi_split;
+    constexpr int PIECES = 3 * 2 * KS, PER = (PIECES + ROTR_WAVES - 1) / ROTR_WAVES;
+    prep_u32x4 v[PER];
 #pragma unroll
-    for (int t = 0; t < 3; ++t) {
-      const uint16_t* base = mat + (((int64_t)(t * (D / 16) + word * 2 + jt) * KS + kh * KPW) * 64 + lane) * 8;
-#pragma unroll
-      for (int k = 0; k < KPW; ++k) ma[t][k] = *(const prep_u32x4*)(base + k * (64 * 8));
+    for (int k = 0; k < PER; ++k) {
+      const int pc = min(wave + k * ROTR_WAVES, PIECES - 1), t = pc / (2 * KS), r = pc - t * (2 * KS);
+      v[k] = *(const prep_u32x4*)(src + (((int64_t)(t * (D / 16) + word * 2) * KS + r) * 64 + lane) * 8);
     }
+#pragma unroll
+    for (int k = 0; k < PER; ++k)
+      if (wave + k * ROTR_WAVES < PIECES) *(prep_u32x4*)(mat + ((wave + k * ROTR_WAVES) * 64 + lane) * 8) = v[k];
   }
-  if (tid >= 64 && tid < 80) s_cf[tid - 64] = wide_term_plane_coef(ly, wp.ntp, tid - 64);
-  float cmax = 0.0f;
-  for (int t = 0; t < ly.n_terms; ++t) cmax = fmaxf(cmax, fabsf(ly.term_coef[t]));
+  if (tid < 16) s_cf[tid] = wide_term_plane_coef(ly, wp, tid);
+  const float cmax = wide_coef_bound(ly, wp);
+  if (word == 0)
+    for (int c = tid; c < D; c += 64 * ROTR_WAVES) s_cs[c] = (m ? ly.S_colsum : ly.Pi_colsum)[c];
   float* dst = m ? q_sk : q_rot;
-#pragma unroll 1
-  for (int tile = tile0; tile < tile1; ++tile) {
-    const int buf = (tile - tile0) & 1, ti = tile - tile0;
-    const int64_t row0 = (int64_t)tile * 16;
-    const int nr = (int)(rows - row0 < 16 ? rows - row0 : 16);
-    const uint16_t* qrow = q + (row0 + (n < nr ? n : nr - 1)) * D + kb * 8;
-    prep_u32x4 qb[KPW];
-#pragma unroll
-    for (int k = 0; k < KPW; ++k) qb[k] = *(const prep_u32x4*)(qrow + (kh * KPW + k) * 32);
-    if (n >= nr) {
-#pragma unroll
-      for (int k = 0; k < KPW; ++k) qb[k] = prep_u32x4{0u, 0u, 0u, 0u};
-    }
-    {  // this wavefront's share of the statistics: steps jt, jt + 2, ... of its contraction half
-      float ss = 0.0f, s1 = 0.0f;
-#pragma unroll
-      for (int i = 0; i < NS; ++i) {
-        const bool real = jt + 2 * i < KPW;
-        // (step 2 i + jt of the operand registers, picked with masks: an index that depends on the wavefront would
-        // move the registers to scratch memory)
-        const uint32_t odd = jt ? 0xffffffffu : 0u;
-        const int KO = 2 * i + 1 < KPW ? 2 * i + 1 : 2 * i;      // (a constant once the loop is unrolled)
-        prep_u32x4 x4;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) x4[e] = (qb[KO][e] & odd) | (qb[2 * i][e] & ~odd);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float xl = real ? __uint_as_float(x4[e] << 16) : 0.0f;
-          const float xh = real ? __uint_as_float(x4[e] & 0xffff0000u) : 0.0f;
-          ss = fmaf(xl, xl, fmaf(xh, xh, ss));
-          s1 = fmaf(xl, cs[i][e >> 1][2 * (e & 1)], fmaf(xh, cs[i][e >> 1][2 * (e & 1) + 1], s1));
-        }
-      }
-      ss += __shfl_xor(ss, 16, 64); s1 += __shfl_xor(s1, 16, 64);
-      ss += __shfl_xor(ss, 32, 64); s1 += __shfl_xor(s1, 32, 64);
-      if (kb == 0) *(float2*)(s_st + ((buf * 4 + wave) * 16 + n) * 2) = make_float2(ss, s1);
-    }
-    prep_f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int t = 2; t >= 0; --t)
-#pragma unroll
-      for (int k = 0; k < KPW; ++k)
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(prep_bf16x8, ma[t][k]),
-                                                      __builtin_bit_cast(prep_bf16x8, qb[k]), acc, 0, 0, 0);
-    *(prep_f32x4*)(part + ((buf * 2 + kh) * 16 + n) * ROTM_LD + jt * 16 + 4 * kb) = acc;
-    // (one barrier per tile: the buffers alternate, and a thread two tiles ahead has passed the barrier of the tile
-    // between, which every reader of this buffer reaches only after its reads)
-    __syncthreads();
-#pragma unroll
-    for (int o = tid; o < 16 * ROT_COLS; o += ROTM_THREADS) {
-      const int r = o >> 5, c = o & 31;
-      const float v = part[((buf * 2) * 16 + r) * ROTM_LD + c] + part[((buf * 2 + 1) * 16 + r) * ROTM_LD + c];
-      s_val[ti * 16 * ROT_COLS + o] = v;
-      if (r < nr) dst[(row0 + r) * D + word * ROT_COLS + c] = v;
-    }
-    if (tid < 16) {
-      const int r = tid;
-      float ss = 0.0f, s1 = 0.0f;
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        const float2 p = *(const float2*)(s_st + ((buf * 4 + w) * 16 + r) * 2);
-        ss += p.x; s1 += p.y;
-      }
-      const float nq = sqrtf(ss), k = wp.sm_scale * 1.4426950408889634f;
-      float* st = wp.q_stat + (row0 + r) * 4;
-      if (m == 0) {
-        const int e1 = min(max((int)((__float_as_uint(fabsf(k) * nq * cmax) >> 23) & 255u) - 126, -100), 100);
-        s_rs[ti * 32 + 2 * r] = k * __uint_as_float((uint32_t)(127 - e1) << 23);
-        if (word == 0 && r < nr) { st[0] = (float)e1; st[2] = k * ly.term_const * s1; }
-      } else {
-        const int e2 = min(max((int)((__float_as_uint(2.0f * fabsf(k * ly.qjl_scale) * nq * ly.S_rownorm_max) >> 23) & 255u) - 126, -100), 100);
-        s_rs[ti * 32 + 2 * r + 1] = 2.0f * k * ly.qjl_scale * __uint_as_float((uint32_t)(127 - e2) << 23);
-        if (word == 0 && r < nr) { st[1] = (float)e2; st[3] = -k * ly.qjl_scale * s1; }
-      }
-    }
-  }
   __syncthreads();
 #pragma unroll 1
-  for (int tile = tile0; tile < tile1; ++tile) {
-    const int ti = tile - tile0;
+  for (int tile = tile0 + NT * wave; tile < tile1; tile += NT * ROTR_WAVES) {
     const int64_t row0 = (int64_t)tile * 16;
-    const int nr = (int)(rows - row0 < 16 ? rows - row0 : 16);
-    wide_pack_word(wp, D, nr, (int)row0, word, s_val + ti * 16 * ROT_COLS, s_val + ti * 16 * ROT_COLS, s_rs + ti * 32, s_cf, tid,
-                   ROTM_THREADS, m ? wp.ntp - 1 : 0, m ? wp.ntp : wp.ntp - 1);
+    const int nt = min(NT, tile1 - tile);
+    const int nr = (int)(rows - row0 < 16 * nt ? rows - row0 : 16 * nt);         // rows of the tiles (the later ones may be absent)
+    // column operands: lane (row n, block kb) holds q[n][32 ks + 8 kb .. + 7]; rows beyond the last repeat it and are left out
+    const uint16_t* qrow[NT];
+#pragma unroll
+    for (int ti = 0; ti < NT; ++ti) qrow[ti] = q + (row0 + min(16 * ti + n, nr - 1)) * D + kb * 8;
+    constexpr int AHEAD = 2;                                         // contraction steps whose queries are requested ahead
+    prep_u32x4 qn[AHEAD][NT];
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k)
+#pragma unroll
+      for (int ti = 0; ti < NT; ++ti) qn[k][ti] = *(const prep_u32x4*)(qrow[ti] + k * 32);
+    prep_f32x4 acc[3][2][NT];                                        // [term][half of the word][tile]: the terms meet at the end, the small ones first
+    float ss[NT], s1[NT];
+#pragma unroll
+    for (int ti = 0; ti < NT; ++ti) {
+      ss[ti] = s1[ti] = 0.0f;
+#pragma unroll
+      for (int t = 0; t < 3; ++t) acc[t][0][ti] = acc[t][1][ti] = prep_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+#pragma unroll 1
+    for (int ks0 = 0; ks0 < KS; ks0 += AHEAD)
+#pragma unroll
+    for (int kk = 0; kk < AHEAD; ++kk) {
+      const int ks = ks0 + kk;
+      prep_u32x4 qb[NT], ql[NT];
+#pragma unroll
+      for (int ti = 0; ti < NT; ++ti) {
+        qb[ti] = qn[kk][ti];
+        qn[kk][ti] = *(const prep_u32x4*)(qrow[ti] + min(ks + AHEAD, KS - 1) * 32);
+        typedef float rot_f32x2 __attribute__((ext_vector_type(2)));
+        typedef __bf16 rot_bf16x2 __attribute__((ext_vector_type(2)));
+        typedef _Float16 rot_f16x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          // (the sum of squares only bounds the row)
+          if constexpr (F16Q) ss[ti] = __builtin_amdgcn_fdot2(__builtin_bit_cast(rot_f16x2, qb[ti][e]), __builtin_bit_cast(rot_f16x2, qb[ti][e]), ss[ti], false);
+          else ss[ti] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(rot_bf16x2, qb[ti][e]), __builtin_bit_cast(rot_bf16x2, qb[ti][e]), ss[ti], false);
+        }
+        if (word == 0 || F16Q) {
+          float x[8];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            x[2 * e] = F16Q ? f16_bits_to_f32((uint16_t)(qb[ti][e] & 0xffffu)) : __uint_as_float(qb[ti][e] << 16);
+            x[2 * e + 1] = F16Q ? f16_bits_to_f32((uint16_t)(qb[ti][e] >> 16)) : __uint_as_float(qb[ti][e] & 0xffff0000u);
+          }
+          if (word == 0) {                                           // (the column sums: by the workgroups of the first word, which write the statistics)
+            const prep_f32x4 c0 = *(const prep_f32x4*)(s_cs + ks * 32 + kb * 8), c1 = *(const prep_f32x4*)(s_cs + ks * 32 + kb * 8 + 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s1[ti] = fmaf(x[e], c0[e], fmaf(x[4 + e], c1[e], s1[ti]));
+          }
+          if constexpr (F16Q) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const rot_f32x2 xv = {x[2 * e], x[2 * e + 1]};
+              const uint32_t hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(xv, rot_bf16x2));
+              const rot_f32x2 rem = {xv[0] - __uint_as_float(hi << 16), xv[1] - __uint_as_float(hi & 0xffff0000u)};
+              qb[ti][e] = hi;
+              ql[ti][e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(rem, rot_bf16x2));
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int t = 2; t >= 0; --t)
+#pragma unroll
+        for (int jt = 0; jt < 2; ++jt) {
+          const prep_bf16x8 ma = __builtin_bit_cast(prep_bf16x8, *(const prep_u32x4*)(mat + (((t * 2 + jt) * KS + ks) * 64 + lane) * 8));
+#pragma unroll
+          for (int ti = 0; ti < NT; ++ti) {
+            if constexpr (F16Q) acc[t][jt][ti] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ma, __builtin_bit_cast(prep_bf16x8, ql[ti]), acc[t][jt][ti], 0, 0, 0);
+            acc[t][jt][ti] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ma, __builtin_bit_cast(prep_bf16x8, qb[ti]), acc[t][jt][ti], 0, 0, 0);
+          }
+        }
+    }
+    const float k = wp.sm_scale * 1.4426950408889634f;
+#pragma unroll
+    for (int ti = 0; ti < NT; ++ti) {
+      // result register i of lane (row n, quarter kb) is coordinate 16 jt + 4 kb + i of row n
+#pragma unroll
+      for (int jt = 0; jt < 2; ++jt) {
+        const prep_f32x4 v = (acc[2][jt][ti] + acc[1][jt][ti]) + acc[0][jt][ti];
+        *(prep_f32x4*)(s_val + (ti % PT * 16 + n) * ROTR_LD + jt * 16 + 4 * kb) = v;
+        if (!wp.heads && 16 * ti + n < nr) *(prep_f32x4*)(dst + (row0 + 16 * ti + n) * D + word * ROT_COLS + jt * 16 + 4 * kb) = v;
+      }
+      ss[ti] += __shfl_xor(ss[ti], 16, 64); s1[ti] += __shfl_xor(s1[ti], 16, 64);
+      ss[ti] += __shfl_xor(ss[ti], 32, 64); s1[ti] += __shfl_xor(s1[ti], 32, 64);
+      const float nq = sqrtf(ss[ti]);
+      float* st = wp.q_stat + (row0 + 16 * ti + n) * 4;
+      const bool mine = kb == 0, put = mine && word == 0 && 16 * ti + n < nr;
+      // bound < 2^e: e = exponent field - 126, kept within +-100
+      if (m == 0) {
+        const int e1 = min(max((int)((__float_as_uint(fabsf(k) * nq * cmax) >> 23) & 255u) - 126, -100), 100);
+        if (mine) s_rs[(ti % PT * 16 + n) * 2] = k * __uint_as_float((uint32_t)(127 - e1) << 23);
+        if (put) { st[0] = (float)e1; st[2] = k * ly.term_const * s1[ti]; }
+      } else {
+        const int e2 = min(max((int)((__float_as_uint(2.0f * fabsf(k * ly.qjl_scale) * nq * ly.S_rownorm_max) >> 23) & 255u) - 126, -100), 100);
+        if (mine) s_rs[(ti % PT * 16 + n) * 2 + 1] = 2.0f * k * ly.qjl_scale * __uint_as_float((uint32_t)(127 - e2) << 23);
+        if (put) { st[1] = (float)e2; st[3] = -k * ly.qjl_scale * s1[ti]; }
+      }
+      if (ti % PT == PT - 1 || ti == NT - 1) {
+        // (this wavefront's own part of LDS: its writes have to be done, nobody else's)
+        const int first = ti / PT * PT, have = min(nr - 16 * first, 16 * (ti + 1 - first));
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (have > 0)
+          wide_pack_word<ROTR_LD>(wp, D, have, (int)row0 + 16 * first, word, s_val, s_val, s_rs, s_cf, lane, 64, m ? wp.ntp - 1 : 0,
+                                  m ? wp.ntp : wp.ntp - 1);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      }
+    }
   }
 }
 

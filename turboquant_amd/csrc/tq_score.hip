@@ -98,8 +98,7 @@ rotate_query_kernel(const void* __restrict__ q, int dtype, int64_t rows, int R, 
   if constexpr (PACK) {
     // row statistics, a wavefront per row (every workgroup of the rows computes the same ones)
     const int lane = tid & 63, wv = tid >> 6, n_wv = (int)blockDim.x >> 6;
-    float cmax = 0.0f;
-    for (int t = 0; t < ly.n_terms; ++t) cmax = fmaxf(cmax, fabsf(ly.term_coef[t]));
+    const float cmax = wide_coef_bound(ly, wp);
     for (int r = wv; r < nr; r += n_wv) {
       float ss = 0.0f, s1 = 0.0f, s2 = 0.0f;
 #pragma unroll
@@ -124,7 +123,7 @@ rotate_query_kernel(const void* __restrict__ q, int dtype, int64_t rows, int R, 
         }
       }
     }
-    if (tid < 16) s_cf[tid] = wide_term_plane_coef(ly, wp.ntp, tid);
+    if (tid < 16) s_cf[tid] = wide_term_plane_coef(ly, wp, tid);
   }
   const int r0 = half * ROT_MAX_ROWS, RH = min(R - r0, ROT_MAX_ROWS);      // this half's rows: r0 .. r0 + RH - 1
   float a[ROT_MAX_ROWS], b[ROT_MAX_ROWS];
@@ -189,12 +188,12 @@ rotate_mfma_kernel(const uint16_t* __restrict__ q, int64_t rows, int n_tiles, tq
   rotate_mfma_body<KPW, F16Q>(q, rows, n_tiles, ly, q_rot, q_sk, wp, (int)blockIdx.x, sm);
 }
 
-template <int KPW>
-__global__ void __launch_bounds__(ROTM_THREADS)
-rotate_mfma_tiles_kernel(const uint16_t* __restrict__ q, int64_t rows, int n_tiles, int tpw, tq_layer ly,
-                         float* __restrict__ q_rot, float* __restrict__ q_sk, WidePack wp) {
-  extern __shared__ __align__(16) float sm[];
-  rotate_mfma_tiles_body<KPW>(q, rows, n_tiles, tpw, ly, q_rot, q_sk, wp, (int)blockIdx.x, sm);
+template <int KPW, bool F16Q, int NT>
+__global__ void __launch_bounds__(64 * ROTR_WAVES, 2)
+rotate_rows_kernel(const uint16_t* __restrict__ q, int64_t rows, int n_tiles, int n_groups, tq_layer ly,
+                   float* __restrict__ q_rot, float* __restrict__ q_sk, WidePack wp) {
+  extern __shared__ __align__(16) unsigned char rows_smem[];
+  rotate_rows_body<KPW, F16Q, NT>(q, rows, n_tiles, n_groups, ly, q_rot, q_sk, wp, (int)blockIdx.x, rows_smem);
 }
 
 template <int PER, int DT, bool PACKED>
@@ -535,23 +534,18 @@ static bool rotate_packs(int64_t rows, const tq_layer* layer, const WidePack* wi
          wide->ntp >= 2 && wide->ntp <= 9 && rows % wide->Hq == 0 && rows < (1 << 30) && layer->d <= 768;
 }
 // ... and whether it does so on the matrix cores (bf16 queries with the layer's split matrices)
-// row tiles a rotation workgroup takes: one while the card holds all workgroups at once (two per compute unit of the
-// kernel that takes several)
-static int rotate_tiles_per_workgroup(int64_t rows, int d) {
-  const int64_t n_tiles = (rows + 15) / 16, pair_rounds = (2 * (d / ROT_COLS) + 7) / 8;
-  const int64_t slots = 2 * (int64_t)device_compute_units();
-  // (workgroups of a (word, product) pair the card has room for: the tiles are shared out among that many, so that
-  // the launch is one round of workgroups and not one and a bit)
-  const int64_t per_pair = slots / (8 * pair_rounds) > 0 ? slots / (8 * pair_rounds) : 1;
-  const int64_t tpw = (n_tiles + per_pair - 1) / per_pair;
-  return (int)(tpw > ROTM_MAX_TPW ? ROTM_MAX_TPW : (tpw < 1 ? 1 : tpw));
+// Row tiles from which a rotation keeps a (plane word, product) pair's matrix terms in LDS and passes over the tiles
+// (rotate_rows_body) instead of running a workgroup per (tile, word, product): when the latter are more than the card holds
+// at once, two per compute unit.
+static bool rotate_by_rows(int64_t rows, int d) {
+  return ((rows + 15) / 16) * 8 * ((2 * (d / ROT_COLS) + 7) / 8) > 2 * (int64_t)device_compute_units();
 }
-// (bf16 queries; fp16 queries as two bf16 terms while a workgroup takes one row tile)
+// (bf16 queries; fp16 queries as two bf16 terms)
 bool rotate_on_matrix_cores(const void* q, int dtype, int64_t rows, const tq_layer* layer, const WidePack* wide) {
   const int d = layer->d;
   return rotate_packs(rows, layer, wide) && layer->Pi_split && layer->S_split &&
          (((uintptr_t)q) & 15) == 0 && d % 64 == 0 && d >= 320 && d <= 704 &&
-         (dtype == TQ_BF16 || (dtype == TQ_F16 && rotate_tiles_per_workgroup(rows, d) == 1)) &&
+         (dtype == TQ_BF16 || dtype == TQ_F16) &&
          opt_prep_mfma.load(std::memory_order_relaxed) != 0;
 }
 
@@ -653,18 +647,26 @@ int launch_rotate_query(const void* q, int dtype, int64_t rows, const tq_layer* 
   // bf16 queries with the layer's split matrices: rotation and packing on the matrix cores
   if (rotate_on_matrix_cores(q, dtype, rows, layer, wide)) {
     const int n_tiles = (int)((rows + 15) / 16), pair_rounds = (2 * (d / ROT_COLS) + 7) / 8;
-    // more workgroups than the card holds at once (two per compute unit of the kernel below): several row tiles per workgroup
-    const int tpw = rotate_tiles_per_workgroup(rows, d);
-    if (tpw > 1) {
-      const int n_tg = (n_tiles + tpw - 1) / tpw;
-      const dim3 tgrid((unsigned)(8 * pair_rounds * n_tg));
-      const size_t tsm = (size_t)rotate_mfma_tiles_smem_floats(tpw) * sizeof(float);
-#define TQ_ROTT(KPW) \
-  case KPW: rotate_mfma_tiles_kernel<KPW><<<tgrid, dim3(ROTM_THREADS), tsm, st>>>((const uint16_t*)q, rows, n_tiles, tpw, *layer, q_rot, q_sk, wp); break;
+    if (rotate_by_rows(rows, d)) {
+      // shares of the tiles: one workgroup per compute unit (the terms fill its LDS), at least a tile each
+      const int slots = device_compute_units() / (8 * pair_rounds);
+      const int n_groups = slots < 1 ? 1 : (slots > n_tiles ? n_tiles : slots);
+      // row tiles a wavefront takes at a time: a workgroup's share in one pass where three each are enough
+      const int per = (n_tiles + n_groups - 1) / n_groups, nt = per <= ROTR_WAVES ? 1 : (per <= 2 * ROTR_WAVES ? 2 : 3);
+      const dim3 rgrid((unsigned)(8 * pair_rounds * n_groups));
+      const size_t rsm = (size_t)rotate_rows_smem_bytes(d);
+#define TQ_ROTR(KPW)                                                                                                   \
+  case KPW: {                                                                                                          \
+    auto kern = dtype == TQ_F16 ? (nt == 1 ? rotate_rows_kernel<KPW, true, 1> : nt == 2 ? rotate_rows_kernel<KPW, true, 2> : rotate_rows_kernel<KPW, true, 3>) \
+                                : (nt == 1 ? rotate_rows_kernel<KPW, false, 1> : nt == 2 ? rotate_rows_kernel<KPW, false, 2> : rotate_rows_kernel<KPW, false, 3>); \
+    hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)rsm);       \
+    if (e != hipSuccess) return (int)e;                                                                                \
+    kern<<<rgrid, dim3(64 * ROTR_WAVES), rsm, st>>>((const uint16_t*)q, rows, n_tiles, n_groups, *layer, q_rot, q_sk, wp); \
+  } break;
       switch (d / 64) {
-        TQ_ROTT(5) TQ_ROTT(6) TQ_ROTT(7) TQ_ROTT(8) TQ_ROTT(9) TQ_ROTT(10) TQ_ROTT(11)
+        TQ_ROTR(5) TQ_ROTR(6) TQ_ROTR(7) TQ_ROTR(8) TQ_ROTR(9) TQ_ROTR(10) TQ_ROTR(11)
       }
-#undef TQ_ROTT
+#undef TQ_ROTR
       hipError_t e = hipGetLastError();
       return e == hipSuccess ? TQ_OK : (int)e;
     }

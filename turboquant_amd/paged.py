@@ -192,13 +192,27 @@ class PagedKVPool:
             return True
         return max(1, Hq // self.num_kv_heads) <= 128       # (more than 8 heads per KV head: groups of at most 8)
 
-    def default_splits(self, B: int, max_len: int, Hq: Optional[int] = None) -> int:
+    def _head_tiles_shape(self, Hq: int) -> bool:
+        """Whether a step runs the kernel of sixteen heads per wavefront (head_dim 512 / 576 with more than 8 query heads per
+        KV head); only the split heuristic depends on it."""
+        return (self.head_dim in (512, 576) and self.quantizer.bits in (3, 4) and self.value_bits in (2, 4) and
+                8 < Hq // self.num_kv_heads <= 128 and self.page_kernel() == 2)
+
+    def default_splits(self, B: int, max_len: int, Hq: Optional[int] = None, static_scratch: bool = False) -> int:
         """Split count of the page-streaming kernel.  Matrix-core kernel: its workgroups (4 wavefronts,
         one per SIMD, each walking 64-token blocks) should number about two per CU (256 CUs) while every
         wavefront still gets several blocks, because each wavefront first builds its query operands.
         General kernel: it hides its memory latency by occupancy, so about eight workgroups per CU, each
         with at least one 256-token chunk."""
         pairs = max(1, B * self.num_kv_heads)
+        if Hq is not None and self._head_tiles_shape(Hq) and not static_scratch:
+            # sixteen query heads per pair of wavefronts, up to four such tiles on the same pages (with two, two blocks of 32
+            # tokens side by side, with one, three): one workgroup per compute unit, at least four turns of its loop
+            # (128 heads of 576: 1 x 8192 56.9 us with 32 splits, 50.8 with 64; 16 x 8192 182 with 8, 192 with 16, 284 with 4)
+            tiles = (Hq // self.num_kv_heads + 15) // 16
+            groups, side = ((tiles + 3) // 4, 1) if tiles >= 3 else (1, 4 - tiles)
+            turns = max(1, (max_len + 32 * side - 1) // (32 * side))
+            return int(max(1, min(max(1, 256 // (pairs * groups)), max(1, turns // 4), 512)))
         if self.head_dim > 256 and self.page_kernel() == 2:
             # head sizes above 256: one workgroup per compute unit, a block of 32 tokens at a time; each workgroup
             # first packs its query operands, so it should have at least 16 blocks
@@ -257,7 +271,7 @@ class PagedKVPool:
         if n_split is None:
             if max_len is None:
                 max_len = (bt.shape[-1]) * PAGE_TOKENS
-            n_split = self.default_splits(B, max_len, Hq)
+            n_split = self.default_splits(B, max_len, Hq, static_scratch)
             by_length = workspace is None and not static_scratch and stages == 7 and self._shares_by_length(B, Hq)
         if static_scratch:
             if workspace is not None or stages != 7:
