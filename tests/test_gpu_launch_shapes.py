@@ -495,3 +495,67 @@ def test_rotation_of_hundreds_of_rows(gpu, d, Hq, B, dtype):
     finally:
         _set_option("prep_mfma", 1)
     assert float((outs[0] - outs[1]).abs().max()) <= 2.0 ** -7 * float(outs[1].abs().max())
+
+
+# ------------------------------------------------------------------ the exact tail on the matrix cores
+@pytest.mark.parametrize("d,Hq,Hkv,B,dtype,rows,n_split", [
+    (128, 5, 1, 2, torch.bfloat16, [1, 16], 1), (128, 16, 1, 3, torch.float16, [15, 17, 0], 3), (128, 17, 1, 1, torch.bfloat16, [129], 2),
+    (128, 40, 8, 65, torch.float16, [128, 127, 33], 1),               # 520 units: two wavefronts each; matrix-core preparation of fp16 queries
+    (128, 24, 8, 67, torch.bfloat16, [200, 64, 3], 2),                # 536 units of three heads, more tiles than a wavefront's four
+    (256, 16, 2, 4, torch.bfloat16, [128, 100, 1, 31], 16),           # shares of a unit's tokens (a merge kernel behind)
+    (256, 6, 1, 300, torch.float16, [130, 5], 1), (64, 8, 2, 3, torch.bfloat16, [300, 16, 1024], 1), (64, 4, 4, 130, torch.float16, [40, 128], 1),
+    (576, 8, 1, 3, torch.bfloat16, [128, 17, 90], 2), (576, 40, 1, 2, torch.float16, [128, 33], 2), (512, 16, 1, 2, torch.bfloat16, [300, 1], 9),
+    (576, 16, 2, 2, torch.bfloat16, [1024, 500], 1)])
+def test_exact_tail_on_the_matrix_cores(gpu, d, Hq, Hkv, B, dtype, rows, n_split):
+    """Exact tokens that start on 16-byte boundaries run on the matrix cores, others on the vector ALU; both take products and
+    weights in fp32 and sum in different orders, so the outputs agree within a rounding step of the output type.  The slots
+    behind a sequence's last exact token hold NaN and infinity."""
+    pool, tq = _make_pool(gpu, d, 3, 4, Hkv, 8, dtype)
+    g = torch.Generator().manual_seed(d + B + Hq)
+    k, v = (torch.randn(1, 100, Hkv, d, generator=g).to(dtype).to(gpu) for _ in range(2))
+    table = torch.arange(7, dtype=torch.int32, device=gpu)
+    pool.append(k, v, table[None])
+    R = max(rows)
+    n_rows = torch.tensor([rows[b % len(rows)] for b in range(B)], dtype=torch.int32)
+    rk, rv = (torch.randn(B, R, Hkv, d, generator=g).to(dtype) for _ in range(2))
+    for b in range(B):
+        rk[b, n_rows[b]:] = float("nan")
+        rv[b, n_rows[b]:] = float("inf")
+    q = torch.randn(B, Hq, d, generator=g).to(dtype).to(gpu)
+    seq = torch.randint(0, 101, (B,), generator=g).to(torch.int32).to(gpu)
+    outs = []
+    for pad in (0, 1):                                                # (one element in: rows that are not even word-aligned)
+        wide = [torch.zeros(B, R, Hkv, d + 2, dtype=dtype, device=gpu) for _ in range(2)]
+        for w, x in zip(wide, (rk, rv)):
+            w[..., 1:1 + d] = x.to(gpu)
+        ks, vs = (wide[0][..., 1:1 + d], wide[1][..., 1:1 + d]) if pad else (rk.to(gpu), rv.to(gpu))
+        outs.append(pool.decode_attention(q, table, seq, recent_k=ks, recent_v=vs, recent_len=n_rows.to(gpu), n_split=n_split,
+                                          max_len=100).float())
+    assert torch.isfinite(outs[0]).all()
+    assert float((outs[0] - outs[1]).abs().max()) <= 2.0 ** -7 * float(outs[1].abs().max())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_exact_tail_in_place_with_two_wavefronts_per_unit(gpu, dtype):
+    """The newest tokens read in place from a paged cache by 528 units, against the same rows gathered (same kernel, same bits up
+    to the shared launch's preparation): blocks anywhere, sequences shorter than the ring, a block outside the cache behind the end."""
+    d, Hkv, Hq, B, ring = 128, 8, 16, 66, 128
+    pool, tq = _make_pool(gpu, d, 3, 4, Hkv, B * 16, dtype)
+    g = torch.Generator().manual_seed(3)
+    lens = [int(x) for x in torch.randint(1, 250, (B,), generator=g)]
+    table = torch.randperm(B * 16, generator=g).view(B, 16).to(torch.int32).to(gpu)
+    x = torch.randn(B, 250, Hkv, d, generator=g).to(dtype).to(gpu)
+    pool.append(x, x.flip(-1), table)
+    cache = torch.randn(2, B * 16, 16, Hkv, d, generator=g).to(dtype).to(gpu)
+    q = torch.randn(B, Hq, d, generator=g).to(dtype).to(gpu)
+    seq = _i32(lens, gpu)
+    got = pool.decode_attention_ring(q, table, seq, cache[0], cache[1], ring, n_split=1, max_len=250).float()
+    rk, rv = (torch.zeros(B, ring, Hkv, d, dtype=dtype, device=gpu) for _ in range(2))
+    for b, n in enumerate(lens):
+        r = min(n, ring)
+        pos = torch.arange(n - r, n, device=gpu)
+        rk[b, :r], rv[b, :r] = (c[table[b].long()[pos // 16], pos % 16] for c in cache)
+    old = _i32([n - min(n, ring) for n in lens], gpu)
+    want = pool.decode_attention(q, table, old, recent_k=rk, recent_v=rv, recent_len=_i32([min(n, ring) for n in lens], gpu),
+                                 n_split=1, max_len=250).float()
+    assert torch.equal(got, want)

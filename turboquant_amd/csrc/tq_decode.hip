@@ -507,6 +507,7 @@ struct TailArgs {
   float* parts;
   int n_parts, part_index;
   int t_chunks;                    // workgroups that share the exact tokens of a (sequence, head group); chunk c writes part part_index + c
+  int n_units, wpu;                // matrix-core body: (chunk, sixteen heads, sequence, KV head) units, and the wavefronts that share one
 };
 
 // (a device function: the stand-alone kernel and the launch that shares its grid with the query
@@ -823,6 +824,238 @@ exact_tail_words_kernel(TailArgs A) {
   exact_tail_words_body<DT, KC, PAGED, WIDE>(A, blockIdx.x, blockIdx.y, blockIdx.z, sm);
 }
 
+// The same partial on the matrix cores, for 16-bit rows that start on 16-byte boundaries (and such a query) at the head sizes
+// that name a template: a workgroup is sixteen query heads of one KV head of one sequence, eight wavefronts with 16 tokens each at
+// a time, and nothing passes through LDS before the wavefronts' sums meet.  Every key row is read once for all heads of the
+// workgroup, where the body above reads and unpacks the rows for every four heads.
+//   * scores: tokens as rows, heads as columns, v_mfma_f32_16x16x32 on the rows as they lie in memory (16-bit products
+//     are exact in fp32); a lane ends with the scores of its head and tokens 4 kb .. 4 kb + 3, and the weights stay in it.
+//   * values: channels as rows, v_mfma_f32_16x16x4_f32 with fp32 weights and widened values.  A lane reads eight channels of its
+//     four tokens; tile j is channel j of every lane's eight.  The rows are requested with the key rows: one memory latency.
+// Bound: HBM with many units (256 sequences x 8 KV heads x 128 tokens of 128: 33 us for 134 MB), else the latency of length,
+// table and rows.  Hybrid steps, vector-ALU tail and this one: 96 sequences of 61 .. 8190 tokens, 40 q / 8 KV heads of 128, fp16
+// (preparation on the matrix cores too) 127 -> 93 us; 256 x 1024, 32 q heads 117 -> 103; 128 x 2048 at 16 q / 2 KV heads of
+// 256 74 -> 64; 16 x 8192 37.8 -> 37.6; 8 heads on a latent of 576 60.4 -> 57.5.
+typedef float tl_f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t tl_u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 tl_bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 tl_f16x8 __attribute__((ext_vector_type(8)));
+__host__ __device__ constexpr int tail_mfma_slots(int d) { return d <= 256 ? 4 : 2; }       // wavefronts' sums in LDS at once
+static size_t tail_mfma_smem(int d, int wpu) {
+  return (size_t)(TAIL_WAVES * 16 * 2 + (wpu == 2 ? TAIL_WAVES / 2 : tail_mfma_slots(d)) * (d / 16) * 256) * sizeof(float);
+}
+static bool tail_mfma_size(int d) { return d == 64 || d == 128 || d == 256 || d == 512 || d == 576; }
+
+// WPU: wavefronts that share a unit (sixteen heads of one KV head of one sequence): all eight of the workgroup, or two (four
+// units per workgroup: less to meet in LDS, four tiles of 16 tokens behind one another instead of one).
+template <int DT, int D, bool PAGED, int WPU>
+__device__ __forceinline__ void exact_tail_mfma_body(const TailArgs& A, int wg, int B, float* sm) {
+  constexpr int KS = D / 32, NT = D / 16, NF = D / 128, REST = D % 128;      // contraction steps, channel tiles, chunks of 128 channels (+ one of 64)
+  static_assert(REST == 0 || REST == 64, "chunks of 128 channels and at most one of 64");
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15, kb = lane >> 4;
+  const int Hkv = A.Hkv, G = A.Hq / Hkv, tiles = (G + 15) / 16;
+  const int unit = wg * (TAIL_WAVES / WPU) + w / WPU, wi = w % WPU, id = min(unit, A.n_units - 1);
+  const bool on = unit < A.n_units;                                // (a unit that does not exist: its wavefronts keep the barriers)
+  const int h = id % Hkv, b = (id / Hkv) % B, gz = id / (Hkv * B), chunk = gz / tiles, tile = gz - chunk * tiles;
+  const int Gc = min(16, G - 16 * tile), head0 = h * G + 16 * tile;
+  const int seq = PAGED ? min(A.seq_lens[b], A.max_pages * TQ_PAGE_TOKENS) : 0;     // cut to the block table
+  const int R_all = max(PAGED ? min(seq, A.recent_rows) : (A.recent_len ? min(A.recent_len[b], A.recent_rows) : A.recent_rows), 0);
+  // this workgroup's share of the exact tokens (all of them with one chunk); it may be empty
+  const int r_lo = (int)((int64_t)R_all * chunk / A.t_chunks), R = on ? (int)((int64_t)R_all * (chunk + 1) / A.t_chunks) - r_lo : 0;
+  const int first = (PAGED ? seq - R_all : 0) + r_lo;              // position (row, when not paged) of the first exact token of the share
+  const int32_t* bt = A.block_table + (PAGED ? (int64_t)b * A.bt_stride : 0);
+  const int64_t base0 = (PAGED ? 0 : b * A.ws_b) + h * A.ws_h;
+  // word offset of exact row `row` (< R)
+  auto row_base = [&](int row) -> int64_t {
+    const int p = first + row;
+    if (PAGED) {
+      const int raw = bt[p >> 4];                        // an entry outside the cache is read as block 0
+      return base0 + (int64_t)((unsigned)raw < (unsigned)A.num_blocks ? raw : 0) * A.ws_blk + (int64_t)(p & 15) * A.ws_r;
+    }
+    return base0 + (int64_t)p * A.ws_r;
+  };
+  constexpr int NS = WPU == 2 ? TAIL_WAVES / 2 : tail_mfma_slots(D);
+  float* s_ml = sm;                                                // [8 wavefronts][16 heads][2]
+  float* s_acc = s_ml + TAIL_WAVES * 16 * 2;                       // [NS][NT][64 lanes][4]
+  // column operands: lane (head n, block kb); columns beyond the last head repeat it and are not written
+  // (kept in registers up to head_dim 256, read beside the rows beyond)
+  constexpr bool QREG = D <= 256;
+  constexpr int KB = KS > 8 ? (KS % 6 == 0 ? 6 : 8) : KS;            // contraction steps whose rows are requested together
+  const uint16_t* qrow = (const uint16_t*)A.q + ((int64_t)b * A.Hq + head0 + min(n, Gc - 1)) * D + kb * 8;
+  tl_u32x4 qv[QREG ? KS : KB];
+  if constexpr (QREG) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qv[ks] = *(const tl_u32x4*)(qrow + ks * 32);
+  }
+  tl_f32x4 acc[NT];
+#pragma unroll
+  for (int c = 0; c < NT; ++c) acc[c] = tl_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  float m_run = NEG_BIG, l_run = 0.0f;
+#pragma unroll 1
+  for (int t0 = 16 * wi; t0 < R; t0 += 16 * WPU) {
+    const bool partial = t0 + 16 > R;
+    const int64_t kr = row_base(min(t0 + n, R - 1)) + kb * 4;
+    int64_t vr[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) vr[i] = row_base(min(t0 + 4 * kb + i, R - 1));
+    tl_f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+    // value rows, a chunk of channels at a time; up to head_dim 256 all of them with the key rows, beyond two chunks ahead of their use
+    constexpr int NC = NF + (REST != 0 ? 1 : 0), VA = QREG ? NC : 2;
+    tl_u32x4 v[VA][4];
+    auto request_values = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (c < NF) v[c % VA][i] = *(const tl_u32x4*)(A.rv + vr[i] + c * 64 + n * 4);
+        else {
+          const uint2 x = *(const uint2*)(A.rv + vr[i] + NF * 64 + n * 2);
+          v[c % VA][i] = tl_u32x4{x.x, x.y, 0u, 0u};
+        }
+        if (partial && t0 + 4 * kb + i >= R) v[c % VA][i] = tl_u32x4{0u, 0u, 0u, 0u};      // (a row that does not exist: weight zero, and values zero too)
+      }
+    };
+#pragma unroll
+    for (int k0 = 0; k0 < KS; k0 += KB) {
+      tl_u32x4 kv[KB];
+#pragma unroll
+      for (int k = 0; k < KB; ++k) kv[k] = *(const tl_u32x4*)(A.rk + kr + (k0 + k) * 16);
+      if constexpr (!QREG) {
+#pragma unroll
+        for (int k = 0; k < KB; ++k) qv[k] = *(const tl_u32x4*)(qrow + (k0 + k) * 32);
+      }
+      if (k0 + KB >= KS) {                               // (requested before the first of these key rows is waited for)
+#pragma unroll
+        for (int c = 0; c < VA; ++c) request_values(c);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int k = 0; k < KB; ++k) {
+        if constexpr (DT == TQ_BF16)
+          s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(tl_bf16x8, kv[k]), __builtin_bit_cast(tl_bf16x8, qv[QREG ? k0 + k : k]), s, 0, 0, 0);
+        else
+          s = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(tl_f16x8, kv[k]), __builtin_bit_cast(tl_f16x8, qv[QREG ? k0 + k : k]), s, 0, 0, 0);
+      }
+      if constexpr (!QREG) __builtin_amdgcn_sched_barrier(0);          // (one batch of rows in registers, not all of them)
+    }
+    float p[4], mx = NEG_BIG;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      p[i] = s[i] * A.sm_scale;
+      if (partial && t0 + 4 * kb + i >= R) p[i] = -INFINITY;
+      mx = fmaxf(mx, p[i]);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float m_new = fmaxf(m_run, mx), f = __expf(m_run - m_new);
+    m_run = m_new;
+    l_run *= f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      p[i] = __expf(p[i] - m_new);
+      l_run += p[i];
+    }
+    if (t0 >= 16 * WPU) {
+#pragma unroll
+      for (int c = 0; c < NT; ++c) acc[c] *= f;
+    }
+    // a word of a row is two channels
+    auto lo = [](uint32_t x) { return DT == TQ_BF16 ? __uint_as_float(x << 16) : f16_bits_to_f32((uint16_t)(x & 0xffffu)); };
+    auto hi = [](uint32_t x) { return DT == TQ_BF16 ? __uint_as_float(x & 0xffff0000u) : f16_bits_to_f32((uint16_t)(x >> 16)); };
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      if (c > 0 && c - 1 + VA < NC) request_values(c - 1 + VA);
+      if constexpr (!QREG) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < (c < NF ? 8 : 4); ++j) {
+          const uint32_t x = v[c % VA][i][j >> 1];
+          acc[8 * c + j] = __builtin_amdgcn_mfma_f32_16x16x4f32((j & 1) ? hi(x) : lo(x), p[i], acc[8 * c + j], 0, 0, 0);
+        }
+    }
+  }
+  // the wavefronts' sums, against their common maximum
+  l_run += __shfl_xor(l_run, 16, 64);
+  l_run += __shfl_xor(l_run, 32, 64);
+  if (kb == 0) *(float2*)(s_ml + (w * 16 + n) * 2) = make_float2(m_run, l_run);
+  __syncthreads();
+  float mm = NEG_BIG, ll = 0.0f;
+  const float* ml = s_ml + (w - wi) * 32 + n * 2;
+#pragma unroll
+  for (int k = 0; k < WPU; ++k) mm = fmaxf(mm, ml[k * 32]);
+#pragma unroll
+  for (int k = 0; k < WPU; ++k) ll += ml[k * 32 + 1] * __expf(ml[k * 32] - mm);
+  {
+    const float f = __expf(m_run - mm);
+#pragma unroll
+    for (int c = 0; c < NT; ++c) acc[c] *= f;
+  }
+  // register r of tile j of a chunk: channel j of the eight (four, in a chunk of 64) of row 4 kb + r
+  float* out = A.parts + (((int64_t)b * A.Hq + head0 + min(n, Gc - 1)) * A.n_parts + A.part_index + chunk) * (D + 2);
+  auto put = [&](int c, const tl_f32x4& a0, const tl_f32x4& a1) __attribute__((always_inline)) {      // channel tiles c, c + 1
+    const bool rest = c >= 8 * NF;
+    const int ch = rest ? 128 * NF + 16 * kb + (c - 8 * NF) : 128 * (c >> 3) + 32 * kb + (c & 7), st = rest ? 4 : 8;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) *(float2*)(out + 2 + ch + st * r) = make_float2(a0[r], a1[r]);
+  };
+  if constexpr (WPU == 2) {
+    if (wi == 1) {
+#pragma unroll
+      for (int c = 0; c < NT; ++c) *(tl_f32x4*)(s_acc + (((w >> 1) * NT + c) * 64 + lane) * 4) = acc[c];
+    }
+    __syncthreads();
+    if (wi == 0 && on && n < Gc) {
+      if (kb == 0) *(float2*)out = make_float2(mm, ll);
+#pragma unroll
+      for (int c = 0; c < NT; c += 2)
+        put(c, acc[c] + *(const tl_f32x4*)(s_acc + (((w >> 1) * NT + c) * 64 + lane) * 4),
+            acc[c + 1] + *(const tl_f32x4*)(s_acc + (((w >> 1) * NT + c + 1) * 64 + lane) * 4));
+    }
+    return;
+  }
+  const int nw = min((R + 15) / 16, TAIL_WAVES);         // wavefronts that had tokens
+#pragma unroll
+  for (int top = TAIL_WAVES; top > NS; top -= NS) {
+    if (nw <= top - NS) continue;                        // (the same for the whole workgroup)
+    if (w >= top - NS && w < top) {
+#pragma unroll
+      for (int c = 0; c < NT; ++c) *(tl_f32x4*)(s_acc + (((w - (top - NS)) * NT + c) * 64 + lane) * 4) = acc[c];
+    }
+    __syncthreads();
+    if (w >= top - 2 * NS && w < top - NS) {
+#pragma unroll
+      for (int c = 0; c < NT; ++c) acc[c] += *(const tl_f32x4*)(s_acc + (((w - (top - 2 * NS)) * NT + c) * 64 + lane) * 4);
+    }
+    __syncthreads();
+  }
+  if (w < NS) {
+#pragma unroll
+    for (int c = 0; c < NT; ++c) *(tl_f32x4*)(s_acc + ((w * NT + c) * 64 + lane) * 4) = acc[c];
+  }
+  __syncthreads();
+  // a head's sums: every wavefront its share of the channel tiles
+  if (n < Gc) {
+    if (w == 0 && kb == 0) *(float2*)out = make_float2(mm, ll);
+    for (int c = 2 * w; c < NT; c += 2 * TAIL_WAVES) {
+      tl_f32x4 a0 = *(const tl_f32x4*)(s_acc + (c * 64 + lane) * 4), a1 = *(const tl_f32x4*)(s_acc + ((c + 1) * 64 + lane) * 4);
+#pragma unroll
+      for (int k = 1; k < NS; ++k) {
+        a0 += *(const tl_f32x4*)(s_acc + ((k * NT + c) * 64 + lane) * 4);
+        a1 += *(const tl_f32x4*)(s_acc + ((k * NT + c + 1) * 64 + lane) * 4);
+      }
+      put(c, a0, a1);
+    }
+  }
+}
+
+template <int DT, int D, bool PAGED>
+__global__ void __launch_bounds__(TAIL_THREADS, D <= 128 ? 4 : 2)
+exact_tail_mfma_kernel(TailArgs A, int B) {
+  extern __shared__ __align__(16) float sm[];
+  if (A.wpu == 2) exact_tail_mfma_body<DT, D, PAGED, 2>(A, blockIdx.x, B, sm);
+  else exact_tail_mfma_body<DT, D, PAGED, TAIL_WAVES>(A, blockIdx.x, B, sm);
+}
+
 // One launch for the two things a hybrid step does before its page kernel: the exact-tail workgroups
 // (the first n_tail, so that the longer-running ones start first) and the query preparation of the
 // matrix-core kernel.  They are independent of each other, both have 512 lanes, and together they are
@@ -830,7 +1063,7 @@ exact_tail_words_kernel(TailArgs A) {
 // the two instead of their sum plus a dispatch gap.
 static_assert(TAIL_THREADS == PREP_COLS * PREP_SLICES, "the two roles share a workgroup size");
 template <int PER, int DT, bool PAGED, bool PACKED>
-__global__ void __launch_bounds__(TAIL_THREADS, 4)
+__global__ void __launch_bounds__(TAIL_THREADS, DT != TQ_F32 && PER == 16 ? 2 : 4)
 prep_tail_kernel(TailArgs A, int n_tail, int B, int Gq, tq_layer ly, float* __restrict__ q_rot, float* __restrict__ q_sk,
                  float* __restrict__ q_stat, uint32_t* __restrict__ qa_pack, unsigned long long* __restrict__ arrivals,
                  int prep_gpw, int n_front, PagePrefetch pf, int g_tot, int head_rows, SplitPlan sp) {
@@ -841,8 +1074,9 @@ prep_tail_kernel(TailArgs A, int n_tail, int B, int Gq, tq_layer ly, float* __re
   }
   const int id = blockIdx.x - (sp.items ? SCHED_FRONT : 0);
   if (id < n_tail) {
-    const int per_z = A.Hkv * B;
-    exact_tail_words_body<DT, 1, PAGED, true>(A, id % A.Hkv, (id / A.Hkv) % B, id / per_z, sm);
+    if constexpr (DT == TQ_F32) exact_tail_words_body<DT, 1, PAGED, true>(A, id % A.Hkv, (id / A.Hkv) % B, id / (A.Hkv * B), sm);
+    else if (A.wpu == 2) exact_tail_mfma_body<DT, PER * PREP_SLICES, PAGED, 2>(A, id, B, sm);
+    else exact_tail_mfma_body<DT, PER * PREP_SLICES, PAGED, TAIL_WAVES>(A, id, B, sm);
   } else if (id >= n_front) {      // behind the tail and the preparation: the page kernel's first pages, read ahead of it
     prefetch_pages_body<TAIL_THREADS>(pf, id - n_front);
   } else {
@@ -850,6 +1084,30 @@ prep_tail_kernel(TailArgs A, int n_tail, int B, int Gq, tq_layer ly, float* __re
     // (arrivals: the arrival counters of the groups of query heads, zeroed for a page kernel that merges its splits itself)
     prep_query_body<PER, DT, PACKED>(A.q, Gq, prep_gpw, (int64_t)B * A.Hq, g_tot, ly, A.sm_scale, q_rot, q_sk, q_stat, qa_pack,
                                      arrivals, head_rows, p / words, p % words, sm);
+  }
+}
+
+// The same with the preparation on the matrix cores (prep_on_matrix_cores), in the first half of a workgroup.
+template <int D, bool F16Q, bool PAGED, bool WW>
+__global__ void __launch_bounds__(TAIL_THREADS, D <= 128 ? 4 : 2)
+prep_mfma_tail_kernel(TailArgs A, int n_tail, int B, int Gq, tq_layer ly, float* __restrict__ q_stat, uint32_t* __restrict__ qa_pack,
+                      unsigned long long* __restrict__ arrivals, int n_tiles, int n_front, PagePrefetch pf, int head_rows, SplitPlan sp) {
+  extern __shared__ __align__(16) float sm[];
+  constexpr int DT = F16Q ? TQ_F16 : TQ_BF16;
+  if (sp.items && blockIdx.x < SCHED_FRONT) {
+    if (blockIdx.x == 0) schedule_splits_body<TAIL_THREADS>(sp, threadIdx.x, (int*)sm);
+    return;
+  }
+  const int id = blockIdx.x - (sp.items ? SCHED_FRONT : 0);
+  if (id < n_tail) {
+    if (A.wpu == 2) exact_tail_mfma_body<DT, D, PAGED, 2>(A, id, B, sm);
+    else exact_tail_mfma_body<DT, D, PAGED, TAIL_WAVES>(A, id, B, sm);
+  } else if (id >= n_front) {
+    prefetch_pages_body<TAIL_THREADS>(pf, id - n_front);
+  } else if (threadIdx.x < PREP_MFMA_THREADS) {
+    const int p = id - n_tail;
+    prep_mfma_body<D, WW, F16Q>((const uint16_t*)A.q, Gq, (int64_t)B * A.Hq, ly, A.sm_scale, q_stat, qa_pack, arrivals, head_rows,
+                                p % n_tiles, p / n_tiles, sm);
   }
 }
 
@@ -862,8 +1120,7 @@ rotate_tail_kernel(TailArgs A, int n_tail, int B, int n_tiles, tq_layer ly, floa
   extern __shared__ __align__(16) float sm[];
   const int id = blockIdx.x;
   if (id < n_tail) {
-    const int per_z = A.Hkv * B;
-    exact_tail_words_body<TQ_BF16, 1, PAGED, true>(A, id % A.Hkv, (id / A.Hkv) % B, id / per_z, sm);
+    exact_tail_mfma_body<TQ_BF16, 64 * KPW, PAGED, TAIL_WAVES>(A, id, B, sm);
   } else if (threadIdx.x < ROTM_THREADS) {
     rotate_mfma_body<KPW>((const uint16_t*)A.q, (int64_t)B * A.Hq, n_tiles, ly, q_rot, q_sk, wp, id - n_tail, sm);
   }
@@ -1001,6 +1258,8 @@ int launch_rotate_query(const void* q, int dtype, int64_t rows, const tq_layer* 
                         const SplitPlan& plan);
 bool prep_on_matrix_cores(const void* q, int dtype, int64_t rows, const tq_layer* layer, int G, int g_tot);
 bool rotate_on_matrix_cores(const void* q, int dtype, int64_t rows, const tq_layer* layer, const WidePack* wide);
+bool rotate_by_rows(int64_t rows, int d);
+bool prep_tile_per_workgroup(int n_tiles, int d);
 }  // namespace tq
 
 static size_t parts_floats(int B, int Hq, int d, int n_parts) { return (size_t)B * Hq * n_parts * (d + 2); }
@@ -1194,14 +1453,20 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
   const int epw = dtype == TQ_F32 ? 1 : 2;
   const bool words = epw == 1 || (((((uintptr_t)recent_k | (uintptr_t)recent_v) & 3) == 0) &&
                                   !((rs_b | rs_r | rs_h | ts.s_blk) & 1));
+  // 16-byte pieces when every row starts on a 16-byte boundary and a row's pieces fit the workgroup
+  const int64_t tws_b = rs_b / epw, tws_r = rs_r / epw, tws_h = rs_h / epw, tws_blk = ts.s_blk / epw;      // strides in words
+  const bool tail_wide = words && ((((uintptr_t)recent_k | (uintptr_t)recent_v) & 15) == 0) &&
+                         !((tws_b | tws_r | tws_h | tws_blk) & 3) && (d / epw) / 4 <= TAIL_THREADS;
+  // The exact tail on the matrix cores: a workgroup per sixteen heads
+  const bool tail_mfma = tail && tail_wide && epw == 2 && (((uintptr_t)q) & 15) == 0 && tail_mfma_size(d);
   // Workgroups per (sequence, KV head, group of TAIL_GC query heads) of the exact tail, each with a share of the
   // exact tokens and a partial of its own.  One such workgroup pulls 2 x recent_rows rows into one compute unit
   // and is the longest-running part of its launch; with few of them and a merge kernel behind (many splits - the
   // in-launch merge takes exactly one partial of the tail) up to TAIL_MAX_CHUNKS share the rows
   // (4 x 131072, 16 q / 2 KV heads, 128 exact tokens: 16 -> 64 workgroups).
   int t_chunks = 1;
-  if (tail && words && n_split > MERGE_IN_KERNEL_MAX_SPLITS && opt_tail_chunks.load(std::memory_order_relaxed) != 0) {
-    const int64_t groups = (int64_t)Hkv * B * ((G + TAIL_GC - 1) / TAIL_GC);
+  if (tail && words && (n_split > MERGE_IN_KERNEL_MAX_SPLITS || (tail_mfma && !mfma_shape)) && opt_tail_chunks.load(std::memory_order_relaxed) != 0) {
+    const int64_t groups = (int64_t)Hkv * B * (tail_mfma ? (G + 15) / 16 : (G + TAIL_GC - 1) / TAIL_GC);
     while (t_chunks < TAIL_MAX_CHUNKS && groups * t_chunks * 2 <= 128 && recent_rows / (t_chunks * 2) >= 16) t_chunks *= 2;
   }
   const int n_parts = n_max + t_chunks;
@@ -1245,16 +1510,17 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
   TailArgs ta;
   ta.q = q; ta.Hq = Hq; ta.Hkv = Hkv; ta.d = d;
   ta.rk = (const uint32_t*)recent_k; ta.rv = (const uint32_t*)recent_v; ta.recent_rows = recent_rows;
-  ta.ws_b = rs_b / epw; ta.ws_r = rs_r / epw; ta.ws_h = rs_h / epw; ta.recent_len = recent_len;
-  ta.block_table = block_table; ta.bt_stride = bt_stride; ta.seq_lens = seq_lens; ta.ws_blk = ts.s_blk / epw;
-  // 16-byte pieces when every row starts on a 16-byte boundary and a row's pieces fit the workgroup
-  ta.wide = words && ((((uintptr_t)recent_k | (uintptr_t)recent_v) & 15) == 0) &&
-            !((ta.ws_b | ta.ws_r | ta.ws_h | ta.ws_blk) & 3) && (d / epw) / 4 <= TAIL_THREADS;
+  ta.ws_b = tws_b; ta.ws_r = tws_r; ta.ws_h = tws_h; ta.recent_len = recent_len;
+  ta.block_table = block_table; ta.bt_stride = bt_stride; ta.seq_lens = seq_lens; ta.ws_blk = tws_blk;
+  ta.wide = tail_wide;
   ta.tile_words = tail_tile_words(d / epw, recent_rows, ta.wide != 0);
   ta.max_pages = max_pages; ta.num_blocks = pool_pages;       // the exact cache shares the pool's block numbers
   ta.sm_scale = sm_scale; ta.parts = parts; ta.n_parts = n_parts; ta.part_index = n_max;
   ta.t_chunks = t_chunks;
-  const int n_tail = Hkv * B * ((G + TAIL_GC - 1) / TAIL_GC) * t_chunks;
+  ta.n_units = Hkv * B * ((G + 15) / 16) * t_chunks;
+  ta.wpu = ta.n_units >= 2 * device_compute_units() ? 2 : TAIL_WAVES;
+  const int n_tail = tail_mfma ? (ta.n_units * ta.wpu + TAIL_WAVES - 1) / TAIL_WAVES : Hkv * B * ((G + TAIL_GC - 1) / TAIL_GC) * t_chunks;
+  const size_t tail_lds = tail_mfma ? tail_mfma_smem(d, ta.wpu) : tail_words_smem(d, recent_rows, ta.tile_words);
   bool tail_done = false;
 
   // A whole compressed-only step with few context splits: the workgroup that finishes last among the splits of a
@@ -1303,7 +1569,7 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
     // per lane and the tail's LDS is sized by the rows it holds, so two workgroups fit a compute unit; with more
     // workgroups than that the rest follow as slots free up, which still measured faster than a launch each
     // (16 x 8192: 48.9 -> 45.2 us per step, 32 x 32768: 223.6 -> 221.5 us).
-    size_t fsm = tail_words_smem(d, recent_rows, ta.tile_words);
+    size_t fsm = tail_lds;
     if (prep_smem_bytes(prep_rows, d) > fsm) fsm = prep_smem_bytes(prep_rows, d);
     const int n_sched = plan.items ? SCHED_FRONT : 0;
     if (n_sched && fsm < SCHED_SMEM_INTS * sizeof(int)) fsm = SCHED_SMEM_INTS * sizeof(int);
@@ -1311,12 +1577,41 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
     // tokens: 139 KB) and the grid is larger than the card: the preparation workgroups would queue behind that
     // LDS size too (128 x 2048, 16 q / 2 KV heads: 109.7 us per step fused, 88.1 as two launches)
     const bool one_per_unit = fsm > (size_t)80 * 1024;
-    // ... or the preparation alone is more than the card holds at once and can run on the matrix cores, which the
-    // shared launch (vector-ALU preparation body) cannot: then a launch each
-    const bool mfma_prep_ahead = mfma_shape && n_prep > 2 * device_compute_units() &&
-                                 prep_on_matrix_cores(q, dtype, (int64_t)B * Hq, layer, Gq, g_tot);
-    if (tail && ta.wide && mfma_shape && stages == 7 && !mfma_prep_ahead &&
-        !(one_per_unit && n_tail + n_prep > device_compute_units())) {
+    const bool tail_shares = tail && ta.wide && (tail_mfma || dtype == TQ_F32) && mfma_shape && stages == 7;
+    // The preparation on the matrix cores shares the launch too (96 sequences of 61 .. 8190 tokens at 40 q / 8 KV heads of 128: a
+    // launch each 98 us, shared 89), but at head_dim 256 only while the card holds it beside the tail: its
+    // workgroups have the tail's registers and LDS there (128 x 2048 at 16 q / 2 KV heads: shared 73.6 us, a launch each 63.9)
+    const bool mfma_prep = tail_mfma && prep_on_matrix_cores(q, dtype, (int64_t)B * Hq, layer, Gq, g_tot);
+    const int rows_tile = (16 / Gq) * Gq;                         // (whole groups of heads, see prep_mfma_body; Gq <= 8)
+    const int n_tiles = (int)(((int64_t)B * Hq + rows_tile - 1) / rows_tile);
+    const bool ww = prep_tile_per_workgroup(n_tiles, d);
+    const int n_mprep = ww ? n_tiles : n_tiles * (d / 32);
+    if (tail_shares && mfma_prep && (d == 128 || n_mprep <= 2 * device_compute_units())) {
+      size_t fsm = tail_lds, psm = (size_t)prep_mfma_smem_floats() * sizeof(float) * (ww ? 4 : 1);
+      if (psm > fsm) fsm = psm;
+      if (n_sched && fsm < SCHED_SMEM_INTS * sizeof(int)) fsm = SCHED_SMEM_INTS * sizeof(int);
+      pf.front = n_tail + n_mprep + n_sched;
+      if (pf.front > 2 * device_compute_units()) pf.blocks = 0;
+      const dim3 pgrid((unsigned)(pf.front + (pf.blocks > 0 ? pf.n_wg : 0)));
+#define TQ_LAUNCH_PMT(D, WW)                                                                                           \
+  {                                                                                                                    \
+    auto kern = dtype == TQ_F16 ? (ts.paged ? prep_mfma_tail_kernel<128, true, true, WW> : prep_mfma_tail_kernel<128, true, false, WW>) \
+                                : (ts.paged ? prep_mfma_tail_kernel<D, false, true, WW> : prep_mfma_tail_kernel<D, false, false, WW>); \
+    if (fsm > 48 * 1024) {                                                                                             \
+      hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)fsm);     \
+      if (e != hipSuccess) return (int)e;                                                                              \
+    }                                                                                                                  \
+    kern<<<pgrid, dim3(TAIL_THREADS), fsm, st>>>(ta, n_tail, B, Gq, *layer, q_stat, qa_pack, fm.counters, n_tiles,      \
+                                                 n_tail + n_mprep, pf, decode_mfma_head_rows(d, Gq), plan);            \
+  }
+      if (d == 128 && ww) TQ_LAUNCH_PMT(128, true)
+      else if (d == 128) TQ_LAUNCH_PMT(128, false)
+      else if (ww) TQ_LAUNCH_PMT(256, true)
+      else TQ_LAUNCH_PMT(256, false)
+#undef TQ_LAUNCH_PMT
+      TQ_CHECK_LAUNCH();
+      tail_done = true;
+    } else if (tail_shares && !mfma_prep && !(one_per_unit && n_tail + n_prep > device_compute_units())) {
 #define TQ_LAUNCH_PT(PER, DT, PAGED)                                                                                 \
   {                                                                                                                  \
     auto kern = prep_gpw > 1 ? prep_tail_kernel<PER, DT, PAGED, true> : prep_tail_kernel<PER, DT, PAGED, false>;     \
@@ -1350,12 +1645,12 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
 #undef TQ_LAUNCH_PT
       TQ_CHECK_LAUNCH();
       tail_done = true;
-    } else if (tail && ta.wide && stages == 7 && dtype == TQ_BF16 && (d == 512 || d == 576) && static_cast<int64_t>(n_tail) <= 4 * device_compute_units() &&
+    } else if (tail_mfma && stages == 7 && dtype == TQ_BF16 && (d == 512 || d == 576) && ta.wpu == TAIL_WAVES && !rotate_by_rows((int64_t)B * Hq, d) &&
                rotate_on_matrix_cores(q, dtype, (int64_t)B * Hq, layer, wide_pre.qa ? &wide_pre : nullptr)) {
       // Hybrid step at the head sizes of latent attention: the exact tail shares the launch of the rotation
       // (16 x 8192 at head_dim 576: one launch of 13 us instead of 10 + 13)
       const int n_tiles = (B * Hq + 15) / 16, pair_rounds = (2 * (d / ROT_COLS) + 7) / 8;
-      size_t fsm = tail_words_smem(d, recent_rows, ta.tile_words);
+      size_t fsm = tail_lds;
       if ((size_t)rotate_mfma_smem_floats() * sizeof(float) > fsm) fsm = (size_t)rotate_mfma_smem_floats() * sizeof(float);
 #define TQ_LAUNCH_RT(KPW, PAGED)                                                                                     \
   {                                                                                                                  \
@@ -1409,7 +1704,29 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
     else if (d <= TAIL_THREADS) TQ_LAUNCH_TAIL((exact_tail_words_kernel<TQ_F32, 1, PAGED, WIDE>), TQ_TAIL_WORD_ARGS) \
     else TQ_LAUNCH_TAIL((exact_tail_words_kernel<TQ_F32, 2, PAGED, WIDE>), TQ_TAIL_WORD_ARGS)                        \
   }
-    if (words) {
+    if (tail_mfma) {
+#define TQ_TAIL_MFMA(DT, D)                                                                                            \
+  {                                                                                                                    \
+    auto kern = ts.paged ? exact_tail_mfma_kernel<DT, D, true> : exact_tail_mfma_kernel<DT, D, false>;                 \
+    if (tail_lds > 48 * 1024) {                                                                                        \
+      hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)tail_lds); \
+      if (e != hipSuccess) return (int)e;                                                                              \
+    }                                                                                                                  \
+    kern<<<dim3((unsigned)n_tail), dim3(TAIL_THREADS), tail_lds, st>>>(ta, B);                                         \
+  }
+#define TQ_TAIL_MFMA_DT(D)                          \
+  {                                                 \
+    if (dtype == TQ_BF16) TQ_TAIL_MFMA(TQ_BF16, D)  \
+    else TQ_TAIL_MFMA(TQ_F16, D)                    \
+  }
+      if (d == 64) TQ_TAIL_MFMA_DT(64)
+      else if (d == 128) TQ_TAIL_MFMA_DT(128)
+      else if (d == 256) TQ_TAIL_MFMA_DT(256)
+      else if (d == 512) TQ_TAIL_MFMA_DT(512)
+      else TQ_TAIL_MFMA_DT(576)
+#undef TQ_TAIL_MFMA_DT
+#undef TQ_TAIL_MFMA
+    } else if (words) {
       if (ts.paged) {
         if (ta.wide) TQ_TAIL_WORDS(true, true)
         else TQ_TAIL_WORDS(true, false)

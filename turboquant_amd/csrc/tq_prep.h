@@ -1005,7 +1005,8 @@ __device__ __forceinline__ void rotate_rows_body(const uint16_t* __restrict__ q,
 
 __host__ __device__ inline int prep_mfma_smem_floats() { return 2 * 16 * PREP_MFMA_LD + 32; }
 
-template <int D, bool WW>
+// (F16Q: fp16 queries, as two bf16 terms: see rotate_mfma_body)
+template <int D, bool WW, bool F16Q = false>
 __device__ __forceinline__ void prep_mfma_body(const uint16_t* __restrict__ q, int G, int64_t n_rows, const tq_layer& ly,
                                                float sm_scale, float* __restrict__ q_stat, uint32_t* __restrict__ qa_pack,
                                                unsigned long long* __restrict__ arrivals, int head_rows, int64_t tile,
@@ -1032,6 +1033,7 @@ __device__ __forceinline__ void prep_mfma_body(const uint16_t* __restrict__ q, i
       for (int ks = 0; ks < KS; ++ks) qb[ks] = prep_u32x4{0u, 0u, 0u, 0u};
     }
   }
+  prep_u32x4 ql[F16Q ? KS : 1];                                      // fp16 queries: qb becomes the rounded values, ql the remainders
   // one 16 x 16 piece: half jt of plane word `word`, product m (0: q Pi^T, 1: q S^T).  Row operands: the three bf16
   // terms of 16 matrix rows, all requested before anything waits.
   auto piece = [&](int word, int jt, int m) __attribute__((always_inline)) {
@@ -1047,9 +1049,13 @@ __device__ __forceinline__ void prep_mfma_body(const uint16_t* __restrict__ q, i
 #pragma unroll
     for (int t = 2; t >= 0; --t)                                       // the small terms first
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
+      for (int ks = 0; ks < KS; ++ks) {
+        if constexpr (F16Q)
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(prep_bf16x8, ma[t][ks]),
+                                                        __builtin_bit_cast(prep_bf16x8, ql[ks]), acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(prep_bf16x8, ma[t][ks]),
                                                       __builtin_bit_cast(prep_bf16x8, qb[ks]), acc, 0, 0, 0);
+      }
     // result register i of lane (row n, quarter kb) is coordinate 16 jt + 4 kb + i of query row n
     *(prep_f32x4*)((m ? s_sk : s_rot) + n * PREP_MFMA_LD + jt * 16 + 4 * kb) = acc;
   };
@@ -1063,7 +1069,8 @@ __device__ __forceinline__ void prep_mfma_body(const uint16_t* __restrict__ q, i
       const prep_f32x4 a0 = c1[0], a1 = c1[1], b0 = c2[0], b1 = c2[1];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float xl = __uint_as_float(qb[ks][e] << 16), xh = __uint_as_float(qb[ks][e] & 0xffff0000u);
+        const float xl = F16Q ? f16_bits_to_f32((uint16_t)(qb[ks][e] & 0xffffu)) : __uint_as_float(qb[ks][e] << 16);
+        const float xh = F16Q ? f16_bits_to_f32((uint16_t)(qb[ks][e] >> 16)) : __uint_as_float(qb[ks][e] & 0xffff0000u);
         const float cl1 = e < 2 ? a0[2 * e] : a1[2 * e - 4], ch1 = e < 2 ? a0[2 * e + 1] : a1[2 * e - 3];
         const float cl2 = e < 2 ? b0[2 * e] : b1[2 * e - 4], ch2 = e < 2 ? b0[2 * e + 1] : b1[2 * e - 3];
         ss = fmaf(xl, xl, fmaf(xh, xh, ss));
@@ -1085,6 +1092,21 @@ __device__ __forceinline__ void prep_mfma_body(const uint16_t* __restrict__ q, i
         float* st = q_stat + (row0 + n) * 4;
         st[0] = (float)e1; st[1] = (float)e2;
         st[2] = k * ly.term_const * s1; st[3] = -k * ly.qjl_scale * s2;
+      }
+    }
+  }
+  if constexpr (F16Q) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        typedef float rot_f32x2 __attribute__((ext_vector_type(2)));
+        typedef __bf16 rot_bf16x2 __attribute__((ext_vector_type(2)));
+        const rot_f32x2 x = {f16_bits_to_f32((uint16_t)(qb[ks][e] & 0xffffu)), f16_bits_to_f32((uint16_t)(qb[ks][e] >> 16))};
+        const uint32_t hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, rot_bf16x2));
+        const rot_f32x2 rem = {x[0] - __uint_as_float(hi << 16), x[1] - __uint_as_float(hi & 0xffff0000u)};
+        qb[ks][e] = hi;
+        ql[ks][e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(rem, rot_bf16x2));
       }
     }
   }

@@ -7,6 +7,7 @@
 #include "tq_decode_mfma.h"
 
 namespace tq {
+bool prep_tile_per_workgroup(int n_tiles, int d);
 
 // q_rot = q Pi^T, q_sk = q S^T for `rows` query vectors (triton_kernels.py:527-528), fp32.
 // A workgroup handles R consecutive rows (the query heads of one KV head when
@@ -221,7 +222,7 @@ prep_query_kernel(const void* __restrict__ q, int G, int gpw, int64_t n_rows, in
 // The preparation on the matrix cores (bf16 queries, head_dim 128 / 256): a workgroup per (tile of up to 16 query
 // rows, plane word), then the page-prefetch workgroups.
 // WW: a workgroup per tile, its wavefronts each taking a plane word at a time.
-template <int D, bool WW>
+template <int D, bool WW, bool F16Q>
 __global__ void __launch_bounds__(PREP_MFMA_THREADS)
 prep_mfma_kernel(const uint16_t* __restrict__ q, int G, int64_t n_rows, tq_layer ly, float sm_scale,
                  float* __restrict__ q_stat, uint32_t* __restrict__ qa_pack, unsigned long long* __restrict__ arrivals,
@@ -233,7 +234,7 @@ prep_mfma_kernel(const uint16_t* __restrict__ q, int G, int64_t n_rows, tq_layer
   }
   const int id = blockIdx.x - (sp.items ? SCHED_FRONT : 0);
   if (id < n_prep)
-    prep_mfma_body<D, WW>(q, G, n_rows, ly, sm_scale, q_stat, qa_pack, arrivals, head_rows, id % n_tiles, id / n_tiles, sm);
+    prep_mfma_body<D, WW, F16Q>(q, G, n_rows, ly, sm_scale, q_stat, qa_pack, arrivals, head_rows, id % n_tiles, id / n_tiles, sm);
   else
     prefetch_pages_body<PREP_MFMA_THREADS>(pf, id - n_prep);
 }
@@ -523,9 +524,16 @@ bool prep_on_matrix_cores(const void* q, int dtype, int64_t rows, const tq_layer
   const int rows_tile = (16 / G) * G;
   const int64_t n_mprep = ((rows + rows_tile - 1) / rows_tile) * (d / 32);
   const int mfma_opt = opt_prep_mfma.load(std::memory_order_relaxed);
-  return dtype == TQ_BF16 && (d == 128 || d == 256) && layer->Pi_split && layer->S_split && layer->Pi_colsum &&
+  // (fp16 queries, as two bf16 terms, at head_dim 128: 96 sequences of 40 heads 29.4 us on the vector ALU, 16 here)
+  return ((dtype == TQ_BF16 && (d == 128 || d == 256)) || (dtype == TQ_F16 && d == 128)) && layer->Pi_split && layer->S_split && layer->Pi_colsum &&
          layer->S_colsum && g_tot == 0 && G <= ROT_MAX_ROWS && rows % G == 0 && (((uintptr_t)q) & 15) == 0 &&
          mfma_opt != 0 && (d == 128 || n_mprep >= 64 || mfma_opt > 1);
+}
+
+// Matrix-core preparation: a workgroup per tile of query rows (its wavefronts a plane word each) instead of one per (tile, word)
+bool prep_tile_per_workgroup(int n_tiles, int d) {
+  const int opt_ww = opt_prep_words.load(std::memory_order_relaxed);
+  return opt_ww < 0 ? d == 128 && (int64_t)n_tiles * (d / 32) > (int64_t)4 * device_compute_units() : opt_ww != 0;
 }
 
 // Whether the rotation launch of a decode step also packs the wide-head page kernel's query operands ...
@@ -537,7 +545,7 @@ static bool rotate_packs(int64_t rows, const tq_layer* layer, const WidePack* wi
 // Row tiles from which a rotation keeps a (plane word, product) pair's matrix terms in LDS and passes over the tiles
 // (rotate_rows_body) instead of running a workgroup per (tile, word, product): when the latter are more than the card holds
 // at once, two per compute unit.
-static bool rotate_by_rows(int64_t rows, int d) {
+bool rotate_by_rows(int64_t rows, int d) {
   return ((rows + 15) / 16) * 8 * ((2 * (d / ROT_COLS) + 7) / 8) > 2 * (int64_t)device_compute_units();
 }
 // (bf16 queries; fp16 queries as two bf16 terms)
@@ -572,8 +580,7 @@ int launch_rotate_query(const void* q, int dtype, int64_t rows, const tq_layer* 
       // unit): a workgroup per tile, its wavefronts taking a plane word each (256 x 1024 tokens, 32 q / 8 KV heads:
       // preparation 16.5 -> 12.3 us; smaller ones lose 1 - 2 us, and at head_dim 256, where a wavefront takes two words in
       // turn, 128 x 2048 at 16 q / 2 KV heads goes from 44.6 to 54.5 us per step).
-      const int opt_ww = opt_prep_words.load(std::memory_order_relaxed);
-      const bool ww = opt_ww < 0 ? d == 128 && (int64_t)n_tiles * (d / 32) > (int64_t)4 * device_compute_units() : opt_ww != 0;
+      const bool ww = prep_tile_per_workgroup(n_tiles, d);
       const int n_mprep = ww ? n_tiles : n_tiles * (d / 32);
       PagePrefetch pf;
       if (prefetch && prefetch->blocks > 0 && prefetch->n_wg > 0 && n_mprep <= 2 * device_compute_units()) pf = *prefetch;
@@ -582,18 +589,17 @@ int launch_rotate_query(const void* q, int dtype, int64_t rows, const tq_layer* 
       const dim3 grid((unsigned)(n_sched + n_mprep + (pf.blocks > 0 ? pf.n_wg : 0))), block(PREP_MFMA_THREADS);
       size_t smem = (size_t)prep_mfma_smem_floats() * sizeof(float) * (ww ? 4 : 1);
       if (n_sched && smem < SCHED_SMEM_INTS * sizeof(int)) smem = SCHED_SMEM_INTS * sizeof(int);
-      if (d == 128 && ww)
-        prep_mfma_kernel<128, true><<<grid, block, smem, st>>>((const uint16_t*)q, G, rows, *layer, sm_scale, q_stat, qa_pack,
-                                                               arrivals, head_rows, n_tiles, n_mprep, pf, plan);
-      else if (d == 128)
-        prep_mfma_kernel<128, false><<<grid, block, smem, st>>>((const uint16_t*)q, G, rows, *layer, sm_scale, q_stat, qa_pack,
-                                                                arrivals, head_rows, n_tiles, n_mprep, pf, plan);
-      else if (ww)
-        prep_mfma_kernel<256, true><<<grid, block, smem, st>>>((const uint16_t*)q, G, rows, *layer, sm_scale, q_stat, qa_pack,
-                                                               arrivals, head_rows, n_tiles, n_mprep, pf, plan);
-      else
-        prep_mfma_kernel<256, false><<<grid, block, smem, st>>>((const uint16_t*)q, G, rows, *layer, sm_scale, q_stat, qa_pack,
-                                                                arrivals, head_rows, n_tiles, n_mprep, pf, plan);
+#define TQ_PREP_MFMA(D, WW)                                                                                            \
+  {                                                                                                                    \
+    auto kern = dtype == TQ_F16 ? prep_mfma_kernel<128, WW, true> : prep_mfma_kernel<D, WW, false>;                    \
+    kern<<<grid, block, smem, st>>>((const uint16_t*)q, G, rows, *layer, sm_scale, q_stat, qa_pack, arrivals, head_rows, \
+                                    n_tiles, n_mprep, pf, plan);                                                       \
+  }
+      if (d == 128 && ww) TQ_PREP_MFMA(128, true)
+      else if (d == 128) TQ_PREP_MFMA(128, false)
+      else if (ww) TQ_PREP_MFMA(256, true)
+      else TQ_PREP_MFMA(256, false)
+#undef TQ_PREP_MFMA
       hipError_t e = hipGetLastError();
       return e == hipSuccess ? TQ_OK : (int)e;
     }
