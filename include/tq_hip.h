@@ -187,6 +187,37 @@ int tq_score(const void *q, int dtype, int64_t batch, int64_t n_q, const uint8_t
 int tq_rotate_query(const void *q, int dtype, int64_t rows, const tq_layer *layer, float *q_rot, float *q_sk,
                     void *stream);
 
+/* ---- the self-contained cache object (TurboQuantKVCache, kv_cache.py:119-349) -------------------------------------
+ * fp32 throughout, d = 64, 128 or 256; `batch` = batch size x H heads.  Compressed sections are the flat tensors of
+ * tq_quantize_keys / tq_quantize_values, contiguous (batch, n_c, ...); exact rows are (batch / H, H, n_buf, d) with element
+ * strides s_b / s_h / s_r and contiguous channels.
+ *
+ * tq_cache_append (kv_cache.py:203-245): a token (batch rows, key_stride / value_stride elements apart) enters a full buffer,
+ * the buffer's first row leaves it and is quantised: every section is written anew with one more token, and the
+ * buffers with their rows one further (contiguous).  The buffers' rows have to lie one behind another (s_r = d) and, with more
+ * than one batch, s_b = H s_h; else TQ_EUNSUPPORTED.  n_c may be 0 (the sections are not read then).  work:
+ * tq_cache_append_bytes bytes.
+ * tq_cache_scores (kv_cache.py:247-284): scores (batch, n_q, n_c + n_buf) = scale * <q, k> over the compressed keys, then the
+ * exact ones; n_c, n_buf > 0.  work: 2 * batch * n_q * d floats.
+ * tq_cache_attend (kv_cache.py:286-321): out (batch, n_q, d) = weights (batch, n_q, n_c + n_buf) times the values.  work:
+ * tq_cache_attend_bytes bytes.                                                                              */
+size_t tq_cache_append_bytes(int64_t batch, int d, int mse_bits, int value_bits, int group_size);
+int tq_cache_append(const float *key, const float *value, int64_t key_stride, int64_t value_stride, const float *key_buf,
+                    const float *value_buf, int64_t ks_b, int64_t ks_h, int64_t ks_r, int64_t vs_b, int64_t vs_h,
+                    int64_t vs_r, int64_t batch, int H, int n_buf, const tq_layer *layer, int value_bits, int group_size,
+                    int64_t n_c, const uint8_t *idx, const uint8_t *signs, const float *norms, const float *rnorms,
+                    const uint8_t *data, const float *scales, const float *zeros, uint8_t *idx_out, uint8_t *signs_out,
+                    float *norms_out, float *rnorms_out, uint8_t *data_out, float *scales_out, float *zeros_out,
+                    float *key_buf_out, float *value_buf_out, void *work, void *stream);
+int tq_cache_scores(const float *q, int64_t batch, int H, int64_t n_q, const uint8_t *idx, const uint8_t *signs,
+                    const float *norms, const float *rnorms, int64_t n_c, const tq_layer *layer, const float *key_buf,
+                    int64_t s_b, int64_t s_h, int64_t s_r, int n_buf, float scale, float *scores, float *work,
+                    void *stream);
+size_t tq_cache_attend_bytes(int64_t batch, int64_t n_q, int d, int64_t n_c, int n_buf);
+int tq_cache_attend(const float *weights, int64_t batch, int H, int64_t n_q, const uint8_t *data, const float *scales,
+                    const float *zeros, int64_t n_c, int d, int group_size, int value_bits, const float *value_buf,
+                    int64_t s_b, int64_t s_h, int64_t s_r, int n_buf, float *out, float *work, void *stream);
+
 /* ---- paged store ---------------------------------------------------------------- */
 
 /* Quantise T new tokens of each of B sequences and write them into pages

@@ -559,3 +559,64 @@ def test_exact_tail_in_place_with_two_wavefronts_per_unit(gpu, dtype):
     want = pool.decode_attention(q, table, old, recent_k=rk, recent_v=rv, recent_len=_i32([min(n, ring) for n in lens], gpu),
                                  n_split=1, max_len=250).float()
     assert torch.equal(got, want)
+
+
+# ------------------------------------------------------------------ a token of the cache object in fp32
+@pytest.mark.parametrize("d,B,H,prompt,buffer,key_bits,vb,gs,n_q", [
+    (128, 1, 8, 400, 128, 3, 2, 32, 1), (64, 2, 3, 150, 128, 4, 4, 32, 1), (256, 1, 2, 300, 1, 2, 8, 64, 3), (128, 2, 1, 129, 128, 3, 4, 16, 9),
+    (64, 1, 5, 65, 64, 5, 2, 64, 2), (128, 3, 4, 384, 33, 3, 2, 128, 1)])
+def test_cache_token_in_few_launches(gpu, monkeypatch, d, B, H, prompt, buffer, key_bits, vb, gs, n_q):
+    """Tokens, scores and values of the cache object through the entries of their own, against the general paths: codes,
+    norms and buffers bit for bit, inner products with the compressed keys bit for bit, everything else within fp32 sums in another
+    order.  Prompts as views of a (batch, tokens, heads, d) tensor, the buffer's rows then not behind one another: the
+    first token takes the general path, the ones after it do not."""
+    from turboquant_amd import kv_cache as KC
+    g = torch.Generator().manual_seed(d + prompt)
+    for view in (False, True):
+        shape = (B, prompt + 4, H, d) if view else (B, H, prompt + 4, d)
+        k, v = (torch.randn(*shape, generator=g).to(gpu) for _ in range(2))
+        if view:
+            k, v = k.transpose(1, 2), v.transpose(1, 2)
+        qs = torch.randn(4, B, H, n_q, d, generator=g).to(gpu)
+        results = []
+        for fast in (True, False):
+            if not fast:
+                monkeypatch.setattr(KC, "_plain", lambda *t: False)
+            cache = KC.TurboQuantKVCache(d, key_bits=key_bits, value_bits=vb, value_group_size=gs, buffer_size=buffer, device=gpu,
+                                         dtype=torch.float32)
+            cache.prefill(k[..., :prompt, :], v[..., :prompt, :])
+            outs = []
+            for i in range(4):
+                t = prompt + i
+                before = cache.key_quantized
+                cache.append(k[..., t:t + 1, :], v[..., t:t + 1, :])
+                assert before.norms.shape[-1] == t - buffer                # (what a caller kept is as it was)
+                scores = cache.attention_scores(qs[i])
+                outs.append((scores, cache.attend(torch.softmax(scores, dim=-1))))
+            results.append((cache, outs))
+            monkeypatch.undo()
+        (a, oa), (b, ob) = results
+        assert a.get_seq_length() == b.get_seq_length() and a.memory_bytes() == b.memory_bytes()
+        for x, y in zip((*a.key_quantized[:4], *a.value_quantized[:3], a.key_buffer, a.value_buffer),
+                        (*b.key_quantized[:4], *b.value_quantized[:3], b.key_buffer, b.value_buffer)):
+            assert x.dtype == y.dtype and torch.equal(x, y)
+        for (s1, r1), (s2, r2) in zip(oa, ob):
+            n_c = s1.shape[-1] - buffer
+            assert s1.shape == s2.shape and torch.equal(s1[..., :n_c], s2[..., :n_c])
+            assert float((s1 - s2).abs().max()) <= 1e-6 * (d ** 0.5) * float(s2.abs().max())
+            assert r1.shape == r2.shape and float((r1 - r2).norm()) <= 2e-6 * float(r2.norm())
+
+
+def test_cache_token_that_has_to_be_differentiated(gpu):
+    """Weights and queries with a gradient take the general paths, through which torch differentiates."""
+    from turboquant_amd.kv_cache import TurboQuantKVCache
+    g = torch.Generator().manual_seed(1)
+    k = torch.randn(1, 2, 300, 128, generator=g).to(gpu)
+    cache = TurboQuantKVCache(128, buffer_size=128, device=gpu, dtype=torch.float32)
+    cache.prefill(k, k)
+    q = torch.randn(1, 2, 1, 128, generator=g).to(gpu).requires_grad_()
+    scores = cache.attention_scores(q)
+    out = cache.attend(torch.softmax(scores, dim=-1))
+    out.sum().backward()
+    assert q.grad is not None and torch.isfinite(q.grad).all() and float(q.grad.abs().max()) > 0
+    assert torch.allclose(out, cache.attend(torch.softmax(scores, dim=-1).detach()), rtol=1e-4, atol=1e-5)

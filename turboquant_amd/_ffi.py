@@ -63,6 +63,13 @@ _SIGNATURES = {
     "tq_dequant_values": (C.c_int, [_vp, _vp, _vp, _i, _i64, _i, _i, _i, _vp, _vp]),
     "tq_score": (C.c_int, [_vp, _i, _i64, _i64, _vp, _vp, _vp, _i, _vp, _i64, C.POINTER(TqLayer), _vp, _vp, _vp]),
     "tq_rotate_query": (C.c_int, [_vp, _i, _i64, C.POINTER(TqLayer), _vp, _vp, _vp]),
+    "tq_cache_append_bytes": (C.c_size_t, [_i64, _i, _i, _i, _i]),
+    "tq_cache_append": (C.c_int, [_vp, _vp, _i64, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i, _i,
+                                  C.POINTER(TqLayer), _i, _i, _i64] + [_vp] * 18),
+    "tq_cache_scores": (C.c_int, [_vp, _i64, _i, _i64, _vp, _vp, _vp, _vp, _i64, C.POINTER(TqLayer), _vp, _i64, _i64, _i64, _i,
+                                  _f, _vp, _vp, _vp]),
+    "tq_cache_attend_bytes": (C.c_size_t, [_i64, _i64, _i, _i64, _i]),
+    "tq_cache_attend": (C.c_int, [_vp, _i64, _i, _i64, _vp, _vp, _vp, _i64, _i, _i, _i, _vp, _i64, _i64, _i64, _i, _vp, _vp, _vp]),
     "tq_append_kv_paged": (C.c_int, [_vp, _vp, _i, _i, _i, _i, _i64, _i64, _i64, _vp, _vp, _i,
                                      C.POINTER(TqLayer), C.POINTER(TqPageLayout), _vp, _i64, _vp]),
     "tq_append_kv_ragged": (C.c_int, [_vp, _vp, _i, _i, _i, _i, _i64, _i64, _vp, _vp, _vp, _vp, _i,

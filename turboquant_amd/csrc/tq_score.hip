@@ -1,6 +1,7 @@
 // Read-side kernels on the reference's flat tensor layouts: query rotation /
 // sketch, the asymmetric score estimator, and key / value de-quantisation.
 
+#include <algorithm>
 #include "tq_common.h"
 #include "tq_prep.h"
 #include "tq_options.h"
@@ -242,7 +243,7 @@ prep_mfma_kernel(const uint16_t* __restrict__ q, int G, int64_t n_rows, tq_layer
 // scores[b, i, k] for a tile of QT queries and one key per thread.  The rotated and sketched queries sit
 // in LDS as [coordinate][QT] rows, so a 16-byte broadcast read feeds four queries; a thread reads its key's
 // packed codes 32 coordinates (eff index words, one sign word) at a time.  NQ = 4 serves tiles of at most four
-// queries with half the work.  Each (query, key) sum runs over the coordinates in ascending order.
+// queries with half the work, NQ = 1 a single query.  Each (query, key) sum runs over the coordinates in ascending order.
 constexpr int QT = 8;
 
 template <int NQ>
@@ -265,6 +266,10 @@ __device__ __forceinline__ void score_accumulate(const float* s_rot, const float
         const int cl = j * per_w + s, c = c0 + cl;
         const float cv = s_cent[(iw[j] >> (eff * s)) & mask];
         const float sg = ((sb >> cl) & 1u) ? 1.0f : -1.0f;
+        if (NQ == 1) {
+          am[0] = fmaf(s_rot[c * QT], cv, am[0]);
+          aq[0] = fmaf(s_sk[c * QT], sg, aq[0]);
+        }
 #pragma unroll
         for (int i4 = 0; i4 < NQ / 4; ++i4) {
           const float4 r = *reinterpret_cast<const float4*>(s_rot + c * QT + 4 * i4);
@@ -283,12 +288,41 @@ __device__ __forceinline__ void score_accumulate(const float* s_rot, const float
   }
 }
 
+// The exact tokens of a cache object: fp32 rows (batch, H, n, d) with element strides, and the queries they meet.
+struct CacheTail {
+  const float* q;
+  const float* k;
+  int64_t s_b, s_h, s_r;
+  int H, n;
+  float scale;
+};
+
+// CACHE: the workgroups behind those of the compressed keys take the exact ones, a wavefront per row at a time
+template <bool CACHE>
 __global__ void __launch_bounds__(256)
 score_kernel(const float* __restrict__ q_rot, const float* __restrict__ q_sk, int64_t n_q,
              const uint8_t* __restrict__ idx, const uint8_t* __restrict__ signs, const void* __restrict__ norms,
-             int norm_dtype, const float* __restrict__ rnorms, int64_t n_k, tq_layer ly, float* __restrict__ scores) {
+             int norm_dtype, const float* __restrict__ rnorms, int64_t n_k, tq_layer ly, float* __restrict__ scores, CacheTail tail) {
   extern __shared__ __align__(16) float sm[];
   const int d = ly.d, mb = ly.mse_bits;
+  if constexpr (CACHE) {
+    const int64_t nkb = (n_k + 255) / 256;
+    if ((int64_t)blockIdx.x >= nkb) {
+      const int64_t bq = blockIdx.z, i0 = (int64_t)blockIdx.y * QT;
+      const int lane = threadIdx.x & 63, ni = (int)((n_q - i0) < QT ? (n_q - i0) : QT);
+      for (int r = ((int)blockIdx.x - (int)nkb) * 32 + (threadIdx.x >> 6), e = min(r + 32, tail.n); r < e; r += 4) {
+        const float* row = tail.k + bq / tail.H * tail.s_b + bq % tail.H * tail.s_h + r * tail.s_r;
+        for (int i = 0; i < ni; ++i) {
+          const float* qr = tail.q + (bq * n_q + i0 + i) * d;
+          float a = 0.0f;
+          for (int c = lane; c < d; c += 64) a = fmaf(qr[c], row[c], a);
+          a = wave_sum_fast(a);
+          if (lane == 0) scores[(bq * n_q + i0 + i) * (n_k + tail.n) + n_k + r] = __fmul_rn(a, tail.scale);
+        }
+      }
+      return;
+    }
+  }
   float* s_rot = sm;              // [d][QT]
   float* s_sk = sm + QT * d;      // [d][QT]
   float* s_cent = s_sk + QT * d;  // [16]
@@ -311,11 +345,17 @@ score_kernel(const float* __restrict__ q_rot, const float* __restrict__ q_sk, in
   float am[QT], aq[QT];
 #pragma unroll
   for (int i = 0; i < QT; ++i) am[i] = aq[i] = 0.0f;
-  if (nq <= 4) score_accumulate<4>(s_rot, s_sk, s_cent, d, eff, ip, sp, am, aq);
+  if (nq == 1) score_accumulate<1>(s_rot, s_sk, s_cent, d, eff, ip, sp, am, aq);
+  else if (nq <= 4) score_accumulate<4>(s_rot, s_sk, s_cent, d, eff, ip, sp, am, aq);
   else score_accumulate<8>(s_rot, s_sk, s_cent, d, eff, ip, sp, am, aq);
   const float nk = load_as_f32(norms, b * n_k + k, norm_dtype);
   const float rk = __fmul_rn(ly.qjl_scale, rnorms[b * n_k + k]);
-  for (int i = 0; i < nq; ++i) scores[(b * n_q + q0 + i) * n_k + k] = __fadd_rn(__fmul_rn(am[i], nk), __fmul_rn(aq[i], rk));
+  // (CACHE: the rows of scores go on with those of the exact tokens, and all of them are scaled)
+  for (int i = 0; i < nq; ++i) {
+    const float s = __fadd_rn(__fmul_rn(am[i], nk), __fmul_rn(aq[i], rk));
+    if constexpr (CACHE) scores[(b * n_q + q0 + i) * (n_k + tail.n) + k] = __fmul_rn(s, tail.scale);
+    else scores[(b * n_q + q0 + i) * n_k + k] = s;
+  }
 }
 
 // the same sums with byte loads, for index / sign rows that are not 4-byte aligned
@@ -745,8 +785,8 @@ extern "C" int tq_score(const void* q, int dtype, int64_t batch, int64_t n_q, co
   dim3 grid((unsigned)((n_k + 255) / 256), (unsigned)((n_q + QT - 1) / QT), (unsigned)batch);
   size_t smem = (2 * QT * d + 16) * sizeof(float);
   if ((uintptr_t)idx % 4 == 0 && (uintptr_t)signs % 4 == 0)
-    score_kernel<<<grid, dim3(256), smem, (hipStream_t)stream>>>(q_rot, q_sk, n_q, idx, signs, norms, norm_dtype,
-                                                                rnorms, n_k, *layer, scores);
+    score_kernel<false><<<grid, dim3(256), smem, (hipStream_t)stream>>>(q_rot, q_sk, n_q, idx, signs, norms, norm_dtype,
+                                                                       rnorms, n_k, *layer, scores, CacheTail{});
   else
     score_bytes_kernel<<<grid, dim3(256), smem, (hipStream_t)stream>>>(q_rot, q_sk, n_q, idx, signs, norms,
                                                                       norm_dtype, rnorms, n_k, *layer, scores);
@@ -796,6 +836,207 @@ extern "C" int tq_dequant_values(const uint8_t* data, const void* scales, const 
   int64_t total = n_vec * d;
   dequant_values_kernel<<<dim3((unsigned)((total + 255) / 256)), dim3(256), 0, (hipStream_t)stream>>>(
       data, scales, zeros, dtype, n_vec, d, group_size, bits, out);
+  TQ_CHECK_LAUNCH();
+  return TQ_OK;
+}
+
+// ---- a step of the self-contained cache object (kv_cache.py:119-349): fp32 rows, one flat tensor per section --------
+namespace tq {
+
+// Rows of several sections at once: row r of section s becomes its `a` bytes followed by its `b` bytes.  One launch where a
+// concatenation per section (and its host time) stood; bound by the latency of a small copy.
+constexpr int CAT_MAX = 9;
+struct CatSection { const uint8_t *a, *b; uint8_t* dst; int64_t a_stride, b_stride; int a_bytes, b_bytes; };
+struct CatArgs { CatSection s[CAT_MAX]; };
+
+__global__ void __launch_bounds__(256)
+cat_rows_kernel(CatArgs A) {
+  const CatSection c = A.s[blockIdx.z];
+  const int64_t r = blockIdx.y;
+  const uint8_t *a = c.a + r * c.a_stride, *b = c.b + r * c.b_stride;
+  uint8_t* dst = c.dst + r * ((int64_t)c.a_bytes + c.b_bytes);
+  const int total = c.a_bytes + c.b_bytes;
+  // (16-byte pieces where a row of the section and both its parts allow them, else words)
+  if (((((uintptr_t)a | (uintptr_t)b | (uintptr_t)dst) & 15) | ((c.a_bytes | c.b_bytes) & 15)) == 0) {
+    for (int o = (blockIdx.x * 256 + threadIdx.x) * 16; o < total; o += gridDim.x * 256 * 16)
+      *(uint4*)(dst + o) = *(const uint4*)(o < c.a_bytes ? a + o : b + (o - c.a_bytes));
+  } else {
+    for (int o = (blockIdx.x * 256 + threadIdx.x) * 4; o < total; o += gridDim.x * 256 * 4)
+      *(uint32_t*)(dst + o) = *(const uint32_t*)(o < c.a_bytes ? a + o : b + (o - c.a_bytes));
+  }
+}
+
+// Weighted sum of the values: a share of the compressed tokens, or 32 exact rows, per workgroup.  A thread owns one word of
+// codes (32 / VB channels of one group) of every 256 / words-th token of the share; code * scale + zero rounds twice, as
+// dequantize_values does, and meets its weight in fp32.  Bound by latency (32,768 tokens of 128: 2.4 MB): shares of 128 tokens.
+constexpr int ATT_TOKENS = 128, ATT_ROWS = 32;
+template <int VB>
+__global__ void __launch_bounds__(256)
+cache_attend_kernel(const float* __restrict__ w, int64_t n_q, const uint32_t* __restrict__ data, const float* __restrict__ scales,
+                    const float* __restrict__ zeros, int n_c, int d, int gs, const float* __restrict__ v, int64_t s_b, int64_t s_h,
+                    int64_t s_r, int H, int n_buf, int n_shares, float* __restrict__ part) {
+  constexpr int CPW = 32 / VB;
+  __shared__ float s_acc[256 * (CPW + 1)];
+  const int tid = threadIdx.x, share = blockIdx.x;
+  const int64_t bh = blockIdx.z, row = bh * n_q + blockIdx.y;
+  const float* wr = w + row * (n_c + n_buf);
+  float* out = part + (row * gridDim.x + share) * d;
+  if (share < n_shares) {
+    const int WR = d / CPW, ng = d / gs, col = tid % WR, t_in = tid / WR, RP = 256 / WR, g = col * CPW / gs;
+    const int t1 = min((share + 1) * ATT_TOKENS, n_c);
+    float acc[CPW];
+#pragma unroll
+    for (int e = 0; e < CPW; ++e) acc[e] = 0.0f;
+#pragma unroll 4
+    for (int t = share * ATT_TOKENS + t_in; t < t1; t += RP) {
+      const int64_t tok = bh * n_c + t;
+      const uint32_t x = data[tok * WR + col];
+      const float sc = scales[tok * ng + g], z = zeros[tok * ng + g], wt = wr[t];
+#pragma unroll
+      for (int e = 0; e < CPW; ++e)
+        acc[e] = fmaf(wt, __fadd_rn(__fmul_rn((float)((x >> (VB * e)) & ((1u << VB) - 1u)), sc), z), acc[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < CPW; ++e) s_acc[tid * (CPW + 1) + e] = acc[e];
+    __syncthreads();
+    if (tid < d) {
+      float a = 0.0f;
+      for (int r = 0; r < RP; ++r) a += s_acc[(r * WR + tid / CPW) * (CPW + 1) + tid % CPW];
+      out[tid] = a;
+    }
+  } else {
+    const int r0 = (share - n_shares) * ATT_ROWS, r1 = min(r0 + ATT_ROWS, n_buf), c = tid % d, sub = tid / d, RS = 256 / d;
+    const float* vb = v + bh / H * s_b + bh % H * s_h + c;
+    float a = 0.0f;
+#pragma unroll 8
+    for (int r = r0 + sub; r < r1; r += RS) a = fmaf(wr[n_c + r], vb[r * s_r], a);
+    s_acc[tid] = a;
+    __syncthreads();
+    if (tid < d) {
+      for (int k = 1; k < RS; ++k) a += s_acc[k * d + tid];
+      out[tid] = a;
+    }
+  }
+}
+
+__global__ void cache_attend_sum_kernel(const float* __restrict__ part, int n, int d, float* __restrict__ out) {
+  const int64_t row = blockIdx.x;
+  const int c = threadIdx.x;
+  float a = 0.0f;
+#pragma unroll 8
+  for (int s = 0; s < n; ++s) a += part[(row * n + s) * d + c];
+  out[row * d + c] = a;
+}
+
+static bool cache_dims(int64_t batch, int H, int d) { return batch > 0 && batch <= 65535 && H > 0 && batch % H == 0 && (d == 64 || d == 128 || d == 256); }
+
+}  // namespace tq
+
+extern "C" size_t tq_cache_append_bytes(int64_t batch, int d, int mse_bits, int value_bits, int group_size) {
+  if (batch <= 0 || d <= 0 || mse_bits < 1 || mse_bits > 4 || value_bits <= 0 || group_size <= 0) return 0;
+  const size_t per = (size_t)idx_row_bytes(d, mse_bits) + d / 8 + 8 + (size_t)d * value_bits / 8 + 8 * (size_t)(d / group_size);
+  return batch * per + 7 * 16;
+}
+
+extern "C" int tq_cache_append(const float* key, const float* value, int64_t key_stride, int64_t value_stride, const float* key_buf,
+                               const float* value_buf, int64_t ks_b, int64_t ks_h, int64_t ks_r, int64_t vs_b, int64_t vs_h, int64_t vs_r, int64_t batch,
+                               int H, int n_buf, const tq_layer* layer, int value_bits, int group_size, int64_t n_c,
+                               const uint8_t* idx, const uint8_t* signs, const float* norms, const float* rnorms,
+                               const uint8_t* data, const float* scales, const float* zeros, uint8_t* idx_out,
+                               uint8_t* signs_out, float* norms_out, float* rnorms_out, uint8_t* data_out, float* scales_out,
+                               float* zeros_out, float* key_buf_out, float* value_buf_out, void* work, void* stream) {
+  if (!key || !value || !key_buf || !value_buf || !layer || !idx_out || !signs_out || !norms_out || !rnorms_out || !data_out ||
+      !scales_out || !zeros_out || !key_buf_out || !value_buf_out || !work)
+    return TQ_ENULL;
+  const int d = layer->d;
+  if (!cache_dims(batch, H, d) || n_buf < 1 || n_c < 0 || group_size < 16 || d % group_size || key_stride < d || value_stride < d) return TQ_EINVAL;
+  // (lengths in bytes of a section's row are ints)
+  if (n_c > (1 << 20) || n_buf > (1 << 20)) return TQ_EUNSUPPORTED;
+  if (ks_r != d || vs_r != d || ks_h < d || vs_h < d) return TQ_EUNSUPPORTED;      // a buffer's rows lie one behind another
+  if (batch != H && (ks_b != H * ks_h || vs_b != H * vs_h)) return TQ_EUNSUPPORTED;
+  if (n_c > 0 && (!idx || !signs || !norms || !rnorms || !data || !scales || !zeros)) return TQ_ENULL;
+  const int ng = d / group_size, ib = idx_row_bytes(d, layer->mse_bits), sb = d / 8, db = d * value_bits / 8;
+  // the codes of the rows that leave the buffer
+  uintptr_t at = ((uintptr_t)work + 15) & ~(uintptr_t)15;
+  auto take = [&](size_t n) { const uintptr_t p = at; at += (n + 15) & ~(size_t)15; return p; };
+  uint8_t* n_idx = (uint8_t*)take(batch * ib);
+  uint8_t* n_sgn = (uint8_t*)take(batch * sb);
+  float* n_nrm = (float*)take(batch * 4);
+  float* n_rn = (float*)take(batch * 4);
+  uint8_t* n_dat = (uint8_t*)take(batch * db);
+  float* n_sc = (float*)take(batch * ng * 4);
+  float* n_z = (float*)take(batch * ng * 4);
+  int rc = tq_quantize_keys(key_buf, TQ_F32, batch, ks_h, layer, n_idx, n_sgn, n_nrm, n_rn, nullptr, nullptr, 0, stream);
+  if (rc) return rc;
+  rc = tq_quantize_values(value_buf, TQ_F32, batch, vs_h, d, group_size, value_bits, n_dat, n_sc, n_z, stream);
+  if (rc) return rc;
+  CatArgs A;
+  auto section = [&](int i, const void* a, int64_t a_stride, int a_bytes, const void* b, int64_t b_stride, int b_bytes, void* dst) {
+    A.s[i] = CatSection{(const uint8_t*)a, (const uint8_t*)b, (uint8_t*)dst, a_stride, b_stride, a_bytes, b_bytes};
+  };
+  const int n = (int)n_c;
+  section(0, idx, (int64_t)n * ib, n * ib, n_idx, ib, ib, idx_out);
+  section(1, signs, (int64_t)n * sb, n * sb, n_sgn, sb, sb, signs_out);
+  section(2, norms, (int64_t)n * 4, n * 4, n_nrm, 4, 4, norms_out);
+  section(3, rnorms, (int64_t)n * 4, n * 4, n_rn, 4, 4, rnorms_out);
+  section(4, data, (int64_t)n * db, n * db, n_dat, db, db, data_out);
+  section(5, scales, (int64_t)n * ng * 4, n * ng * 4, n_sc, ng * 4, ng * 4, scales_out);
+  section(6, zeros, (int64_t)n * ng * 4, n * ng * 4, n_z, ng * 4, ng * 4, zeros_out);
+  section(7, key_buf + d, ks_h * 4, (n_buf - 1) * d * 4, key, key_stride * 4, d * 4, key_buf_out);
+  section(8, value_buf + d, vs_h * 4, (n_buf - 1) * d * 4, value, value_stride * 4, d * 4, value_buf_out);
+  const int longest = std::max(n * std::max(std::max(ib, db), std::max(sb, ng * 4)), n_buf * d * 4);
+  const int blocks = std::max(1, std::min(32, longest / (256 * 16 * 2)));
+  cat_rows_kernel<<<dim3(blocks, (unsigned)batch, CAT_MAX), dim3(256), 0, (hipStream_t)stream>>>(A);
+  TQ_CHECK_LAUNCH();
+  return TQ_OK;
+}
+
+extern "C" int tq_cache_scores(const float* q, int64_t batch, int H, int64_t n_q, const uint8_t* idx, const uint8_t* signs,
+                               const float* norms, const float* rnorms, int64_t n_c, const tq_layer* layer, const float* key_buf,
+                               int64_t s_b, int64_t s_h, int64_t s_r, int n_buf, float scale, float* scores, float* work,
+                               void* stream) {
+  int rc = check_layer_rd(layer, true);
+  if (rc) return rc;
+  if (!q || !idx || !signs || !norms || !rnorms || !key_buf || !scores || !work) return TQ_ENULL;
+  const int d = layer->d;
+  if (!cache_dims(batch, H, d) || n_q <= 0 || n_c <= 0 || n_buf <= 0) return TQ_EINVAL;
+  if (((uintptr_t)idx | (uintptr_t)signs) & 3 || n_c > (1 << 28) || n_q > (1 << 18)) return TQ_EUNSUPPORTED;
+  float* q_rot = work;
+  float* q_sk = work + batch * n_q * d;
+  rc = tq_rotate_query(q, TQ_F32, batch * n_q, layer, q_rot, q_sk, stream);
+  if (rc) return rc;
+  const CacheTail tail{q, key_buf, s_b, s_h, s_r, H, n_buf, scale};
+  const dim3 grid((unsigned)((n_c + 255) / 256 + (n_buf + 31) / 32), (unsigned)((n_q + QT - 1) / QT), (unsigned)batch);
+  score_kernel<true><<<grid, dim3(256), (2 * QT * d + 16) * sizeof(float), (hipStream_t)stream>>>(
+      q_rot, q_sk, n_q, idx, signs, norms, TQ_F32, rnorms, n_c, *layer, scores, tail);
+  TQ_CHECK_LAUNCH();
+  return TQ_OK;
+}
+
+extern "C" size_t tq_cache_attend_bytes(int64_t batch, int64_t n_q, int d, int64_t n_c, int n_buf) {
+  if (batch <= 0 || n_q <= 0 || d <= 0 || n_c < 0 || n_buf < 0) return 0;
+  return (size_t)batch * n_q * d * sizeof(float) * ((n_c + ATT_TOKENS - 1) / ATT_TOKENS + (n_buf + ATT_ROWS - 1) / ATT_ROWS);
+}
+
+extern "C" int tq_cache_attend(const float* weights, int64_t batch, int H, int64_t n_q, const uint8_t* data, const float* scales,
+                               const float* zeros, int64_t n_c, int d, int group_size, int value_bits, const float* value_buf,
+                               int64_t s_b, int64_t s_h, int64_t s_r, int n_buf, float* out, float* work, void* stream) {
+  if (!weights || !data || !scales || !zeros || !value_buf || !out || !work) return TQ_ENULL;
+  if (!cache_dims(batch, H, d) || n_q <= 0 || n_c <= 0 || n_buf <= 0 || group_size < 16 || d % group_size) return TQ_EINVAL;
+  if (group_size % 16 || ((uintptr_t)data & 3) || n_c > (1 << 28) || n_q > 65535) return TQ_EUNSUPPORTED;
+  const int shares = (int)((n_c + ATT_TOKENS - 1) / ATT_TOKENS), all = shares + (n_buf + ATT_ROWS - 1) / ATT_ROWS;
+  const dim3 grid((unsigned)all, (unsigned)n_q, (unsigned)batch);
+#define TQ_ATTEND(VB)                                                                                                   \
+  cache_attend_kernel<VB><<<grid, dim3(256), 0, (hipStream_t)stream>>>(weights, n_q, (const uint32_t*)data, scales, zeros, \
+                                                                       (int)n_c, d, group_size, value_buf, s_b, s_h, s_r, H, n_buf, \
+                                                                       shares, work)
+  if (value_bits == 2) TQ_ATTEND(2);
+  else if (value_bits == 4) TQ_ATTEND(4);
+  else if (value_bits == 8) TQ_ATTEND(8);
+  else return TQ_EUNSUPPORTED;
+#undef TQ_ATTEND
+  TQ_CHECK_LAUNCH();
+  cache_attend_sum_kernel<<<dim3((unsigned)(batch * n_q)), dim3(d), 0, (hipStream_t)stream>>>(work, all, d, out);
   TQ_CHECK_LAUNCH();
   return TQ_OK;
 }

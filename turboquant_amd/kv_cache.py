@@ -8,6 +8,7 @@ dtypes; the arithmetic runs in libtq_hip.so.
 
 from __future__ import annotations
 
+import ctypes as C
 import math
 from typing import NamedTuple, Optional
 
@@ -75,6 +76,20 @@ def dequantize_values(vq: ValueQuantized, group_size: int = 32) -> torch.Tensor:
     return out
 
 
+def _plain(*tensors) -> bool:
+    """Whether torch would run an operation on these GPU tensors as it stands: ordinary fp32 tensors of four dimensions with
+    contiguous channels, nothing to differentiate, no transform, trace or dispatch mode that has to see the operation."""
+    if (torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack() or torch._C._are_functorch_transforms_active()
+            or torch.autograd.forward_ad._current_level >= 0 or torch.compiler.is_compiling() or torch.jit.is_tracing()):
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if (type(t) is not torch.Tensor or not t.is_cuda or t.dtype != torch.float32 or t.dim() != 4 or t.stride(-1) != 1
+                or (grad and t.requires_grad) or t.device != tensors[0].device):
+            return False
+    return True
+
+
 class TurboQuantKVCache:
     """Self-contained cache: the newest `buffer_size` tokens stay exact, older
     ones are TurboQuant keys + group-quantised values.  Tensors are
@@ -128,10 +143,58 @@ class TurboQuantKVCache:
         self.key_quantized = self.value_quantized = None
         self._compress(keys[..., :cut, :], values[..., :cut, :])
 
+    # ---- a decode token in fp32 (the general paths below take everything else) -----------------------------------------
+    # A step of the general paths is some thirty small launches and seven concatenations of the whole history: 270 us, nearly all of it
+    # host time, at 4096 tokens of 8 heads of 128.  The entries below are three launches for the token, two for the scores and
+    # two for the values: 85 us.
+    def _compressed_plain(self) -> bool:
+        kq, vq = self.key_quantized, self.value_quantized
+        return (kq is not None and vq is not None and self.head_dim in (64, 128, 256) and self.value_group_size % 16 == 0
+                and kq.norms.dtype == torch.float32 and vq.scales.dtype == torch.float32 and kq.norms.dim() == 3
+                and all(type(t) is torch.Tensor and t.is_contiguous() for t in (*kq[:4], *vq[:3])))
+
+    def _append_spill(self, key: torch.Tensor, value: torch.Tensor) -> bool:
+        """One token into a full buffer whose first row leaves for the compressed part, in one library call; False: the case is
+        not that one, nothing was done."""
+        kb, vb = self.key_buffer, self.value_buffer
+        if kb is None or vb is None or not self._compressed_plain() or not _plain(key, value, kb, vb):
+            return False
+        B, H, n_buf, d = kb.shape
+        kq, vq = self.key_quantized, self.value_quantized
+        n_c = kq.norms.shape[-1]
+        if (n_buf != self.buffer_size or n_buf < 1 or d != self.head_dim or vb.shape != kb.shape or key.shape != (B, H, 1, d)
+                or value.shape != key.shape or tuple(kq.norms.shape) != (B, H, n_c) or tuple(vq.scales.shape[:3]) != (B, H, n_c)
+                or B * H > 65535 or n_c >= 1 << 20 or kq.norms.device != kb.device):
+            return False
+        if any(t.stride(2) != d or t.stride(1) < d or (B > 1 and t.stride(0) != H * t.stride(1)) for t in (kb, vb)):
+            return False
+        if B > 1 and any(t.stride(0) != H * t.stride(1) for t in (key, value)) or any(t.stride(1) < d for t in (key, value)):
+            return False
+        lib, dev, ly = _ffi.lib(), kb.device, self.key_quantizer._layer()
+        grown = [torch.empty(B, H, n_c + 1, *t.shape[3:], dtype=t.dtype, device=dev) for t in (*kq[:4], *vq[:3])]
+        nk, nv = torch.empty(B, H, n_buf, d, dtype=torch.float32, device=dev), torch.empty(B, H, n_buf, d, dtype=torch.float32, device=dev)
+        work = torch.empty(lib.tq_cache_append_bytes(B * H, d, self.key_bits - 1, self.value_bits, self.value_group_size),
+                           dtype=torch.uint8, device=dev)
+        idx, signs, rnorms, norms = grown[:4]
+        with _ffi.on_device(dev):
+            _ffi.check(lib.tq_cache_append(
+                key.data_ptr(), value.data_ptr(), key.stride(1), value.stride(1), kb.data_ptr(), vb.data_ptr(), *kb.stride()[:3],
+                *vb.stride()[:3], B * H, H, n_buf, C.byref(ly), self.value_bits, self.value_group_size, n_c,
+                kq.mse_indices.data_ptr(), kq.qjl_signs.data_ptr(), kq.norms.data_ptr(), kq.residual_norms.data_ptr(),
+                vq.data.data_ptr(), vq.scales.data_ptr(), vq.zeros.data_ptr(), idx.data_ptr(), signs.data_ptr(),
+                norms.data_ptr(), rnorms.data_ptr(), *[t.data_ptr() for t in grown[4:]], nk.data_ptr(), nv.data_ptr(),
+                work.data_ptr(), _ffi.stream_ptr(dev)), "tq_cache_append")
+        self.key_quantized = ProdQuantized(idx, signs, rnorms, norms, kq.mse_bits)
+        self.value_quantized = ValueQuantized(*grown[4:], bits=self.value_bits)
+        self.key_buffer, self.value_buffer = nk, nv
+        return True
+
     def append(self, key: torch.Tensor, value: torch.Tensor):
         """One decode token (batch, heads, 1, head_dim); the oldest buffered
         tokens spill into the compressed part once the buffer overflows."""
         self.seq_len += 1
+        if self._append_spill(key, value):
+            return
         if self.key_buffer is None:
             self.key_buffer, self.value_buffer = key, value
         else:
@@ -147,6 +210,22 @@ class TurboQuantKVCache:
         """scale * <q, k> over [compressed ; buffer]: (batch, heads, n_q, seq_len)."""
         if scale is None:
             scale = 1.0 / math.sqrt(self.head_dim)
+        kb = self.key_buffer
+        if kb is not None and isinstance(scale, (int, float)) and self._compressed_plain() and _plain(query, kb):
+            kq = self.key_quantized
+            B, H, n_buf, d = kb.shape
+            n_c, n_q = kq.norms.shape[-1], query.shape[2]
+            if (query.shape == (B, H, n_q, self.head_dim) and d == self.head_dim and tuple(kq.norms.shape) == (B, H, n_c)
+                    and n_c and n_buf and n_q and B * H <= 65535 and kq.norms.device == kb.device):
+                q, ly, dev = query.contiguous(), self.key_quantizer._layer(), kb.device
+                scores = torch.empty(B, H, n_q, n_c + n_buf, dtype=torch.float32, device=dev)
+                work = torch.empty(2 * B * H * n_q * d, dtype=torch.float32, device=dev)
+                with _ffi.on_device(dev):
+                    _ffi.check(_ffi.lib().tq_cache_scores(
+                        q.data_ptr(), B * H, H, n_q, kq.mse_indices.data_ptr(), kq.qjl_signs.data_ptr(), kq.norms.data_ptr(),
+                        kq.residual_norms.data_ptr(), n_c, C.byref(ly), kb.data_ptr(), *kb.stride()[:3], n_buf, float(scale),
+                        scores.data_ptr(), work.data_ptr(), _ffi.stream_ptr(dev)), "tq_cache_scores")
+                return scores
         pieces = []
         if self.key_quantized is not None:
             pieces.append(self.key_quantizer.attention_score(query, self.key_quantized) * scale)
@@ -156,6 +235,22 @@ class TurboQuantKVCache:
 
     def attend(self, attn_weights: torch.Tensor) -> torch.Tensor:
         """softmaxed weights (batch, heads, n_q, seq_len) -> (batch, heads, n_q, head_dim)."""
+        vb = self.value_buffer
+        if vb is not None and self._compressed_plain() and _plain(attn_weights, vb):
+            vq = self.value_quantized
+            B, H, n_buf, d = vb.shape
+            n_c, n_q = vq.data.shape[-2], attn_weights.shape[2]
+            if (attn_weights.shape == (B, H, n_q, n_c + n_buf) and d == self.head_dim and tuple(vq.scales.shape[:3]) == (B, H, n_c)
+                    and n_c and n_buf and 0 < n_q <= 65535 and B * H <= 65535 and vq.scales.device == vb.device):
+                w, dev, lib = attn_weights.contiguous(), vb.device, _ffi.lib()
+                out = torch.empty(B, H, n_q, d, dtype=torch.float32, device=dev)
+                work = torch.empty(lib.tq_cache_attend_bytes(B * H, n_q, d, n_c, n_buf) // 4, dtype=torch.float32, device=dev)
+                with _ffi.on_device(dev):
+                    _ffi.check(lib.tq_cache_attend(
+                        w.data_ptr(), B * H, H, n_q, vq.data.data_ptr(), vq.scales.data_ptr(), vq.zeros.data_ptr(), n_c, d,
+                        self.value_group_size, self.value_bits, vb.data_ptr(), *vb.stride()[:3], n_buf, out.data_ptr(),
+                        work.data_ptr(), _ffi.stream_ptr(dev)), "tq_cache_attend")
+                return out
         result = None
         col = 0
         if self.value_quantized is not None:
