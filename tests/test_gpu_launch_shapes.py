@@ -620,3 +620,49 @@ def test_cache_token_that_has_to_be_differentiated(gpu):
     out.sum().backward()
     assert q.grad is not None and torch.isfinite(q.grad).all() and float(q.grad.abs().max()) > 0
     assert torch.allclose(out, cache.attend(torch.softmax(scores, dim=-1).detach()), rtol=1e-4, atol=1e-5)
+
+
+# ------------------------------------------------------------------ inner products and flat codes of small calls
+@pytest.mark.parametrize("d,bits,lead,n_k,n_q,dtype", [
+    (64, 2, (), 1, 1, torch.float32), (128, 3, (2,), 63, 16, torch.bfloat16), (128, 5, (1, 3), 65, 17, torch.float32),
+    (256, 4, (), 64, 33, torch.float16), (320, 3, (2,), 130, 5, torch.float32), (576, 4, (), 100, 40, torch.float32),
+    (192, 2, (), 17, 15, torch.float32), (128, 3, (8,), 4097, 31, torch.float32)])
+def test_inner_products_on_the_matrix_cores(gpu, d, bits, lead, n_k, n_q, dtype):
+    """tq_score against the same codes in float64.  Bound: two fp32 sums of d products each, of numbers that are themselves fp32
+    sums of d products of the query with a row of Pi (norm 1) or S (at most `big`): d 2^-24 of the magnitudes, twice."""
+    from turboquant_amd.quantizer import TurboQuantProd
+    tq = TurboQuantProd(d, bits=bits, device=gpu)
+    g = torch.Generator().manual_seed(d + n_k)
+    k = torch.randn(*lead, n_k, d, generator=g).to(gpu, dtype)
+    q = torch.randn(*lead, n_q, d, generator=g).to(gpu, dtype)
+    code = tq.quantize(k)
+    got = tq.attention_score(q, code).double().cpu()
+    per = 8 // {1: 1, 2: 2, 3: 4, 4: 4}[bits - 1]
+    packed = code.mse_indices.cpu().long()
+    index = torch.stack([packed >> (8 // per * s) & (1 << 8 // per) - 1 for s in range(per)], -1).flatten(-2)[..., :d]
+    sign = torch.stack([code.qjl_signs.cpu().long() >> s & 1 for s in range(8)], -1).flatten(-2)[..., :d].double() * 2 - 1
+    cent = tq.mse_quantizer.centroids.double().cpu()[index] * code.norms.double().cpu()[..., None]
+    sign = sign * (tq.qjl_scale * code.residual_norms.double().cpu()[..., None])
+    Pi, S, q64 = tq.mse_quantizer.Pi.double().cpu(), tq.S.double().cpu(), q.double().cpu()
+    rot, sk = q64 @ Pi.T, q64 @ S.T
+    want = rot @ cent.transpose(-1, -2) + sk @ sign.transpose(-1, -2)
+    big = max(1.0, float(S.norm(dim=1).max()))
+    length = q64.norm(dim=-1, keepdim=True) * torch.ones(d, dtype=torch.float64)
+    bound = 2 * d * 2 ** -24 * ((rot.abs() + length) @ cent.abs().transpose(-1, -2) + (sk.abs() + big * length) @ sign.abs().transpose(-1, -2))
+    assert got.shape == want.shape and bool(((got - want).abs() <= bound + 4e-7 * want.abs()).all())
+
+
+@pytest.mark.parametrize("d,bits,dtype", [(128, 3, torch.float32), (128, 4, torch.bfloat16), (256, 3, torch.float16)])
+def test_flat_codes_of_few_vectors_are_those_of_many(gpu, d, bits, dtype):
+    """A tile of 16 vectors per workgroup in small calls, groups of tiles in large ones: codes, norms and de-quantised rows bit for bit."""
+    from turboquant_amd.quantizer import ProdQuantized, TurboQuantProd
+    tq = TurboQuantProd(d, bits=bits, device=gpu)
+    g = torch.Generator().manual_seed(d)
+    k = (torch.randn(20000, d, generator=g) * 2).to(gpu, dtype)
+    many = tq.quantize(k)
+    rows = tq.dequantize(many)
+    for n in (1, 15, 16, 17, 33, 8191, 8192, 8193):
+        few = tq.quantize(k[5:5 + n])
+        for x, y in zip(few[:4], many[:4]):
+            assert torch.equal(x, y[5:5 + n])
+        assert torch.equal(tq.dequantize(few), rows[5:5 + n])

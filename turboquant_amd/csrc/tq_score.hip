@@ -240,53 +240,7 @@ prep_mfma_kernel(const uint16_t* __restrict__ q, int G, int64_t n_rows, tq_layer
     prefetch_pages_body<PREP_MFMA_THREADS>(pf, id - n_prep);
 }
 
-// scores[b, i, k] for a tile of QT queries and one key per thread.  The rotated and sketched queries sit
-// in LDS as [coordinate][QT] rows, so a 16-byte broadcast read feeds four queries; a thread reads its key's
-// packed codes 32 coordinates (eff index words, one sign word) at a time.  NQ = 4 serves tiles of at most four
-// queries with half the work, NQ = 1 a single query.  Each (query, key) sum runs over the coordinates in ascending order.
-constexpr int QT = 8;
-
-template <int NQ>
-__device__ __forceinline__ void score_accumulate(const float* s_rot, const float* s_sk, const float* s_cent, int d,
-                                                 int eff, const uint32_t* ip, const uint32_t* sp, float (&am)[QT],
-                                                 float (&aq)[QT]) {
-  const unsigned mask = (1u << eff) - 1u;
-  for (int c0 = 0; c0 < d; c0 += 32) {
-    uint32_t iw[4] = {0, 0, 0, 0};
-    const uint32_t* w = ip + (c0 >> 5) * eff;
-    iw[0] = w[0];
-    if (eff >= 2) iw[1] = w[1];
-    if (eff == 4) { iw[2] = w[2]; iw[3] = w[3]; }
-    const uint32_t sb = sp[c0 >> 5];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {                    // index word j of this run: 32 / eff coordinates
-      const int per_w = 32 / eff;
-      if (j * per_w >= 32) break;
-      for (int s = 0; s < per_w; ++s) {
-        const int cl = j * per_w + s, c = c0 + cl;
-        const float cv = s_cent[(iw[j] >> (eff * s)) & mask];
-        const float sg = ((sb >> cl) & 1u) ? 1.0f : -1.0f;
-        if (NQ == 1) {
-          am[0] = fmaf(s_rot[c * QT], cv, am[0]);
-          aq[0] = fmaf(s_sk[c * QT], sg, aq[0]);
-        }
-#pragma unroll
-        for (int i4 = 0; i4 < NQ / 4; ++i4) {
-          const float4 r = *reinterpret_cast<const float4*>(s_rot + c * QT + 4 * i4);
-          const float4 k = *reinterpret_cast<const float4*>(s_sk + c * QT + 4 * i4);
-          am[4 * i4 + 0] = fmaf(r.x, cv, am[4 * i4 + 0]);
-          am[4 * i4 + 1] = fmaf(r.y, cv, am[4 * i4 + 1]);
-          am[4 * i4 + 2] = fmaf(r.z, cv, am[4 * i4 + 2]);
-          am[4 * i4 + 3] = fmaf(r.w, cv, am[4 * i4 + 3]);
-          aq[4 * i4 + 0] = fmaf(k.x, sg, aq[4 * i4 + 0]);
-          aq[4 * i4 + 1] = fmaf(k.y, sg, aq[4 * i4 + 1]);
-          aq[4 * i4 + 2] = fmaf(k.z, sg, aq[4 * i4 + 2]);
-          aq[4 * i4 + 3] = fmaf(k.w, sg, aq[4 * i4 + 3]);
-        }
-      }
-    }
-  }
-}
+constexpr int QT = 8;              // queries per workgroup of the byte-wise kernel
 
 // The exact tokens of a cache object: fp32 rows (batch, H, n, d) with element strides, and the queries they meet.
 struct CacheTail {
@@ -297,65 +251,124 @@ struct CacheTail {
   float scale;
 };
 
+// scores[b, i, k] on the matrix cores: v_mfma_f32_16x16x4_f32 with sixteen rotated / sketched queries as rows, sixteen keys as columns
+// and fp32 operands on both sides (a centroid or a sign is an fp32 number), so nothing is split or rounded.  Of every sixteen
+// coordinates a lane holds four of its key and the same four of its query, which it reads straight from the rotation's rows: the four lanes
+// of a row take 64 consecutive bytes (a quarter of the coordinates in a row per lane touched 64 lines per load: 8 heads x 16384 keys x 128
+// queries 180 us; now 120).  NT tiles of sixteen queries share one expansion of the codes.
+// Bound by latency in small calls, else by the fp32 matrix rate (two MFMAs of 32 cycles per 4 coordinates of a 16 x 16 tile).  One key per
+// thread with the queries as LDS broadcasts, which this replaces, read 64 bytes of LDS per key and coordinate: 32 queries x 4096 keys of
+// 128 18.0 -> 5.1 us; the call with its rotation at 1000 keys of 576 and 33 queries 79 -> 27.
 // CACHE: the workgroups behind those of the compressed keys take the exact ones, a wavefront per row at a time
-template <bool CACHE>
+constexpr int SCORE_KEYS = 64;     // keys per workgroup: sixteen for each of four wavefronts
+constexpr int SCORE_ROWS = 4;      // exact rows per workgroup: one per wavefront (eight behind one another, 4000 keys and 128 rows of 8 heads: 9.7 us, now 7.8)
+
+template <int EFF, int NT>
+__device__ __forceinline__ void score_tiles(const float* __restrict__ rot, const float* __restrict__ sk, const int64_t (&row)[NT],
+                                            const float* s_cent, int d, int kb, const uint32_t* __restrict__ ip,
+                                            const uint32_t* __restrict__ sp, prep_f32x4 (&am)[NT], prep_f32x4 (&aq)[NT]) {
+  typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));        // (the caller's scratch: any float address)
+  constexpr unsigned mask = (1u << EFF) - 1u;
+  for (int c0 = 0; c0 < d; c0 += 64) {
+    uint32_t sb[2], iw[4];                                      // shifted to this lane's four coordinates of each sixteen
+#pragma unroll
+    for (int j = 0; j < 2; ++j) sb[j] = sp[(c0 >> 5) + j] >> (4 * kb);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (EFF == 1) iw[j] = ip[(c0 >> 5) + (j >> 1)] >> (16 * (j & 1) + 4 * kb);
+      if (EFF == 2) iw[j] = ip[(c0 >> 4) + j] >> (8 * kb);
+      if (EFF == 4) iw[j] = ip[(c0 >> 3) + 2 * j + (kb >> 1)] >> (16 * (kb & 1));
+    }
+    f32x4_u r[NT][4], k[NT][4];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        r[t][j] = *(const f32x4_u*)(rot + row[t] + c0 + 16 * j + 4 * kb);
+        k[t][j] = *(const f32x4_u*)(sk + row[t] + c0 + 16 * j + 4 * kb);
+      }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float cv = s_cent[(iw[j] >> (EFF * e)) & mask];
+        const float sg = __uint_as_float(0xbf800000u ^ (sb[j >> 1] << (31 - 16 * (j & 1) - e) & 0x80000000u));   // bit set: +1
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          am[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(r[t][j][e], cv, am[t], 0, 0, 0);
+          aq[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[t][j][e], sg, aq[t], 0, 0, 0);
+        }
+      }
+  }
+}
+
+template <bool CACHE, int NT>
 __global__ void __launch_bounds__(256)
 score_kernel(const float* __restrict__ q_rot, const float* __restrict__ q_sk, int64_t n_q,
              const uint8_t* __restrict__ idx, const uint8_t* __restrict__ signs, const void* __restrict__ norms,
              int norm_dtype, const float* __restrict__ rnorms, int64_t n_k, tq_layer ly, float* __restrict__ scores, CacheTail tail) {
-  extern __shared__ __align__(16) float sm[];
+  __shared__ float s_cent[16];
   const int d = ly.d, mb = ly.mse_bits;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t b = blockIdx.z, q0 = (int64_t)blockIdx.y * (16 * NT);
   if constexpr (CACHE) {
-    const int64_t nkb = (n_k + 255) / 256;
+    const int64_t nkb = (n_k + SCORE_KEYS - 1) / SCORE_KEYS;
     if ((int64_t)blockIdx.x >= nkb) {
-      const int64_t bq = blockIdx.z, i0 = (int64_t)blockIdx.y * QT;
-      const int lane = threadIdx.x & 63, ni = (int)((n_q - i0) < QT ? (n_q - i0) : QT);
-      for (int r = ((int)blockIdx.x - (int)nkb) * 32 + (threadIdx.x >> 6), e = min(r + 32, tail.n); r < e; r += 4) {
-        const float* row = tail.k + bq / tail.H * tail.s_b + bq % tail.H * tail.s_h + r * tail.s_r;
+      const int ni = (int)((n_q - q0) < 16 * NT ? (n_q - q0) : 16 * NT);
+      for (int r = ((int)blockIdx.x - (int)nkb) * SCORE_ROWS + wave, e = min(r - wave + SCORE_ROWS, tail.n); r < e; r += 4) {
+        const float* row = tail.k + b / tail.H * tail.s_b + b % tail.H * tail.s_h + r * tail.s_r;
         for (int i = 0; i < ni; ++i) {
-          const float* qr = tail.q + (bq * n_q + i0 + i) * d;
+          const float* qr = tail.q + (b * n_q + q0 + i) * d;
           float a = 0.0f;
           for (int c = lane; c < d; c += 64) a = fmaf(qr[c], row[c], a);
           a = wave_sum_fast(a);
-          if (lane == 0) scores[(bq * n_q + i0 + i) * (n_k + tail.n) + n_k + r] = __fmul_rn(a, tail.scale);
+          if (lane == 0) scores[(b * n_q + q0 + i) * (n_k + tail.n) + n_k + r] = __fmul_rn(a, tail.scale);
         }
       }
       return;
     }
   }
-  float* s_rot = sm;              // [d][QT]
-  float* s_sk = sm + QT * d;      // [d][QT]
-  float* s_cent = s_sk + QT * d;  // [16]
-  const int64_t b = blockIdx.z;
-  const int64_t q0 = (int64_t)blockIdx.y * QT;
-  const int nq = (int)((n_q - q0) < QT ? (n_q - q0) : QT);
-  for (int o = threadIdx.x; o < QT * d; o += blockDim.x) {
-    int i = o / d, c = o - i * d;
-    bool ok = i < nq;
-    s_rot[c * QT + i] = ok ? q_rot[(b * n_q + q0) * d + o] : 0.0f;
-    s_sk[c * QT + i] = ok ? q_sk[(b * n_q + q0) * d + o] : 0.0f;
-  }
   if (threadIdx.x < (1 << mb)) s_cent[threadIdx.x] = ly.centroids[threadIdx.x];
   __syncthreads();
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n_k) return;
-  const int eff = eff_bits(mb), row = idx_row_bytes(d, mb), srow = d >> 3;
-  const uint32_t* ip = (const uint32_t*)(idx + (b * n_k + k) * row);
-  const uint32_t* sp = (const uint32_t*)(signs + (b * n_k + k) * srow);
-  float am[QT], aq[QT];
+  const int64_t k0 = (int64_t)blockIdx.x * SCORE_KEYS + wave * 16;
+  if (k0 >= n_k) return;
+  const int n = lane & 15, kb = lane >> 4;
+  const int64_t key = k0 + n < n_k ? k0 + n : n_k - 1;          // (keys and queries that do not exist: the last one, not stored)
+  const int eff = eff_bits(mb);
+  const uint32_t* ip = (const uint32_t*)(idx + (b * n_k + key) * idx_row_bytes(d, mb));
+  const uint32_t* sp = (const uint32_t*)(signs + (b * n_k + key) * (d >> 3));
+  int64_t row[NT];
+  prep_f32x4 am[NT], aq[NT];
 #pragma unroll
-  for (int i = 0; i < QT; ++i) am[i] = aq[i] = 0.0f;
-  if (nq == 1) score_accumulate<1>(s_rot, s_sk, s_cent, d, eff, ip, sp, am, aq);
-  else if (nq <= 4) score_accumulate<4>(s_rot, s_sk, s_cent, d, eff, ip, sp, am, aq);
-  else score_accumulate<8>(s_rot, s_sk, s_cent, d, eff, ip, sp, am, aq);
-  const float nk = load_as_f32(norms, b * n_k + k, norm_dtype);
-  const float rk = __fmul_rn(ly.qjl_scale, rnorms[b * n_k + k]);
-  // (CACHE: the rows of scores go on with those of the exact tokens, and all of them are scaled)
-  for (int i = 0; i < nq; ++i) {
-    const float s = __fadd_rn(__fmul_rn(am[i], nk), __fmul_rn(aq[i], rk));
-    if constexpr (CACHE) scores[(b * n_q + q0 + i) * (n_k + tail.n) + k] = __fmul_rn(s, tail.scale);
-    else scores[(b * n_q + q0 + i) * n_k + k] = s;
+  for (int t = 0; t < NT; ++t) {
+    const int64_t i = q0 + 16 * t + n;
+    row[t] = (b * n_q + (i < n_q ? i : n_q - 1)) * d;
+    am[t] = aq[t] = prep_f32x4{0, 0, 0, 0};
   }
+  const float nk = load_as_f32(norms, b * n_k + key, norm_dtype);
+  const float rk = __fmul_rn(ly.qjl_scale, rnorms[b * n_k + key]);
+  if (eff == 1) score_tiles<1, NT>(q_rot, q_sk, row, s_cent, d, kb, ip, sp, am, aq);
+  else if (eff == 2) score_tiles<2, NT>(q_rot, q_sk, row, s_cent, d, kb, ip, sp, am, aq);
+  else score_tiles<4, NT>(q_rot, q_sk, row, s_cent, d, kb, ip, sp, am, aq);
+  if (k0 + n >= n_k) return;
+  // (CACHE: the rows of scores go on with those of the exact tokens, and all of them are scaled)
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int64_t qi = q0 + 16 * t + 4 * kb + i;
+      if (qi >= n_q) continue;
+      const float s = __fadd_rn(__fmul_rn(am[t][i], nk), __fmul_rn(aq[t][i], rk));
+      if constexpr (CACHE) scores[(b * n_q + qi) * (n_k + tail.n) + key] = __fmul_rn(s, tail.scale);
+      else scores[(b * n_q + qi) * n_k + key] = s;
+    }
+}
+
+// Tiles of sixteen queries per wavefront: two where that still leaves two workgroups per compute unit (the call, 8 heads x 16384 keys x 128
+// queries of 128 / 256: 133 / 254 us with two, 137 / 265 with one; fewer queries or keys: the same)
+__host__ static int score_query_tiles(int64_t batch, int64_t n_q, int64_t n_k) {
+  if (n_q <= 16) return 1;
+  return batch * ((n_q + 31) / 32) * ((n_k + SCORE_KEYS - 1) / SCORE_KEYS) >= 2 * (int64_t)device_compute_units() ? 2 : 1;
 }
 
 // the same sums with byte loads, for index / sign rows that are not 4-byte aligned
@@ -782,14 +795,17 @@ extern "C" int tq_score(const void* q, int dtype, int64_t batch, int64_t n_q, co
   float* q_sk = work + batch * n_q * d;
   rc = tq_rotate_query(q, dtype, batch * n_q, layer, q_rot, q_sk, stream);
   if (rc) return rc;
-  dim3 grid((unsigned)((n_k + 255) / 256), (unsigned)((n_q + QT - 1) / QT), (unsigned)batch);
-  size_t smem = (2 * QT * d + 16) * sizeof(float);
-  if ((uintptr_t)idx % 4 == 0 && (uintptr_t)signs % 4 == 0)
-    score_kernel<false><<<grid, dim3(256), smem, (hipStream_t)stream>>>(q_rot, q_sk, n_q, idx, signs, norms, norm_dtype,
-                                                                       rnorms, n_k, *layer, scores, CacheTail{});
-  else
-    score_bytes_kernel<<<grid, dim3(256), smem, (hipStream_t)stream>>>(q_rot, q_sk, n_q, idx, signs, norms,
-                                                                      norm_dtype, rnorms, n_k, *layer, scores);
+  if ((uintptr_t)idx % 4 == 0 && (uintptr_t)signs % 4 == 0) {
+    const int nt = score_query_tiles(batch, n_q, n_k);
+    const dim3 grid((unsigned)((n_k + SCORE_KEYS - 1) / SCORE_KEYS), (unsigned)((n_q + 16 * nt - 1) / (16 * nt)), (unsigned)batch);
+    auto kern = nt == 2 ? score_kernel<false, 2> : score_kernel<false, 1>;
+    kern<<<grid, dim3(256), 0, (hipStream_t)stream>>>(q_rot, q_sk, n_q, idx, signs, norms, norm_dtype, rnorms, n_k, *layer, scores,
+                                                      CacheTail{});
+  } else {
+    const dim3 grid((unsigned)((n_k + 255) / 256), (unsigned)((n_q + QT - 1) / QT), (unsigned)batch);
+    score_bytes_kernel<<<grid, dim3(256), (2 * QT * d + 16) * sizeof(float), (hipStream_t)stream>>>(
+        q_rot, q_sk, n_q, idx, signs, norms, norm_dtype, rnorms, n_k, *layer, scores);
+  }
   TQ_CHECK_LAUNCH();
   return TQ_OK;
 }
@@ -1006,8 +1022,11 @@ extern "C" int tq_cache_scores(const float* q, int64_t batch, int H, int64_t n_q
   rc = tq_rotate_query(q, TQ_F32, batch * n_q, layer, q_rot, q_sk, stream);
   if (rc) return rc;
   const CacheTail tail{q, key_buf, s_b, s_h, s_r, H, n_buf, scale};
-  const dim3 grid((unsigned)((n_c + 255) / 256 + (n_buf + 31) / 32), (unsigned)((n_q + QT - 1) / QT), (unsigned)batch);
-  score_kernel<true><<<grid, dim3(256), (2 * QT * d + 16) * sizeof(float), (hipStream_t)stream>>>(
+  const int nt = score_query_tiles(batch, n_q, n_c);
+  const dim3 grid((unsigned)((n_c + SCORE_KEYS - 1) / SCORE_KEYS + (n_buf + SCORE_ROWS - 1) / SCORE_ROWS), (unsigned)((n_q + 16 * nt - 1) / (16 * nt)),
+                  (unsigned)batch);
+  auto kern = nt == 2 ? score_kernel<true, 2> : score_kernel<true, 1>;
+  kern<<<grid, dim3(256), 0, (hipStream_t)stream>>>(
       q_rot, q_sk, n_q, idx, signs, norms, TQ_F32, rnorms, n_c, *layer, scores, tail);
   TQ_CHECK_LAUNCH();
   return TQ_OK;
