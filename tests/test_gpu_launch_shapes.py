@@ -666,3 +666,40 @@ def test_flat_codes_of_few_vectors_are_those_of_many(gpu, d, bits, dtype):
         for x, y in zip(few[:4], many[:4]):
             assert torch.equal(x, y[5:5 + n])
         assert torch.equal(tq.dequantize(few), rows[5:5 + n])
+
+
+# ------------------------------------------------------------------ keys and values of a small append in one launch
+@pytest.mark.parametrize("d,B,H,T,kb,vb,gs,dtype,ragged", [
+    (128, 1, 1, 1, 3, 2, 32, torch.bfloat16, False), (128, 33, 3, 1, 4, 4, 16, torch.float16, False),
+    (256, 5, 2, 17, 3, 4, 128, torch.bfloat16, False), (256, 16, 8, 1, 2, 2, 64, torch.float16, False),
+    (128, 128, 4, 1, 2, 4, 32, torch.bfloat16, False), (128, 3, 2, 40, 5, 2, 64, torch.bfloat16, True), (256, 7, 1, 33, 4, 4, 32, torch.float16, True)])
+def test_small_append_in_one_launch(gpu, d, B, H, T, kb, vb, gs, dtype, ragged):
+    """The same pages as two launches write, byte for byte, over pages that hold other tokens already; a sequence whose run
+    leaves the block table and one whose page lies outside the pool write nothing there."""
+    g = torch.Generator().manual_seed(d + B)
+    per_seq = 5
+    tq = TurboQuantProd(d, bits=kb, device=gpu)
+    table = torch.randperm(B * per_seq, generator=g).view(B, per_seq).to(torch.int32)
+    starts = torch.randint(0, 30, (B,), generator=g).to(torch.int32)
+    if B > 4:
+        starts[2] = per_seq * 16 - 1 if T > 1 else per_seq * 16
+        table[3] = B * per_seq + 7
+    lens = [T - (b % 3 if ragged else 0) for b in range(B)]
+    rows = (sum(lens), H, d) if ragged else (B, T, H, d)
+    k, v = (torch.randn(*rows, generator=g).to(gpu, dtype) for _ in range(2))
+    fill = torch.randint(0, 256, (B * per_seq,), generator=g, dtype=torch.uint8).to(gpu)
+    got = []
+    for one in (True, False):
+        pool = PagedKVPool(tq, H, B * per_seq, value_bits=vb, value_group_size=gs, dtype=dtype, device=gpu)
+        pool.data += fill[:, None, None]
+        try:
+            _set_option("append_small", -1 if one else 0)
+            if ragged:
+                row0 = _i32([sum(lens[:b]) for b in range(B)], gpu)
+                pool.append_ragged(k, v, row0, _i32(lens, gpu), starts.to(gpu), table.to(gpu), max_run=T)
+            else:
+                pool.append(k, v, table.to(gpu), start_pos=starts.to(gpu))
+        finally:
+            _set_option("append_small", -1)
+        got.append(pool.data.clone())
+    assert torch.equal(*got) and not torch.equal(got[0], torch.zeros_like(got[0]) + fill[:, None, None])

@@ -28,6 +28,7 @@
 #include <atomic>
 
 #include "tq_key_mfma.h"
+#include "tq_value_chunk.h"
 #include "tq_decode_mfma.h"
 #include "tq_options.h"
 #include <hip/hip_ext.h>
@@ -236,9 +237,10 @@ struct XStage {
 // fp32 product sum).  10 MFMAs per 16 x 16 tile instead of 24, and no centroid terms go through the LDS.
 // ML (1 or the MT tiles of a group): small appends - the page write of a decode step - give every 16-vector tile a
 // workgroup of its own that computes one tile instead of four, a quarter of the instructions behind one another.
-template <int DT, int D, bool MSE_ONLY, bool FX, class Source, class Sink, int ML = KeyGeom<D>::MT>
-__global__ void __launch_bounds__(KQ_THREADS, 2)
-key_mfma_kernel(const void* __restrict__ x, Source src, tq_layer ly, Sink sink, int64_t n_tiles) {
+// Workgroup `id` of the n_wg that share the groups.
+template <int DT, int D, bool MSE_ONLY, bool FX, class Source, class Sink, int ML>
+__device__ __forceinline__ void key_mfma_body(const void* __restrict__ x, const Source& src, const tq_layer& ly, const Sink& sink,
+                                              int64_t n_tiles, int id, int n_wg, unsigned char* smem) {
   static_assert(!FX || (D == 128 && !MSE_ONLY), "the fp6 centroid contraction: head_dim 128, full quantiser");
   constexpr int mse_only = MSE_ONLY;
   using E = Elem<DT>;
@@ -252,7 +254,6 @@ key_mfma_kernel(const void* __restrict__ x, Source src, tq_layer ly, Sink sink, 
   MatRegs<D> mr;
   prefetch_matrix<D>(ly.Pi_split, wave0, tid0 & 63, mr);        // in flight while the vectors are staged
 
-  extern __shared__ __align__(16) unsigned char smem[];
   S* sx = (S*)(smem + Sm::off_x);                               // [TT][XRS] input
   uint16_t* terms = (uint16_t*)(smem + Sm::off_terms);          // [3][TT][RS]: unit vector, then centroids, then residual
   uint32_t* spl = (uint32_t*)(smem + Sm::off_planes);           // [plane][TT][W]
@@ -298,14 +299,14 @@ key_mfma_kernel(const void* __restrict__ x, Source src, tq_layer ly, Sink sink, 
     n_tiles = (int64_t)__builtin_amdgcn_readfirstlane(cum[src.B]) * src.H;
   }
   const int64_t n_groups = (n_tiles + ML - 1) / ML;             // a group = the TT vectors of one pass
-  if (blockIdx.x >= n_groups) return;
+  if (id >= n_groups) return;
   // (1) staging (XStage): the next group's chunks wait in registers while the current group is worked on
   XStage<DT, D, Source> stg;
   stg.init(src, tid0);
-  stg.template lookup<ML>(src, blockIdx.x, n_tiles, wave0 % ML, cum, tid0 & 63);
+  stg.template lookup<ML>(src, id, n_tiles, wave0 % ML, cum, tid0 & 63);
   stg.issue(x);
 
-  for (int64_t g = blockIdx.x; g < n_groups; g += gridDim.x) {
+  for (int64_t g = id; g < n_groups; g += n_wg) {
   // The thread index is re-read through an opaque copy in every pass: otherwise the compiler
   // hoists all per-thread address arithmetic out of this loop and spills it.
   int tid = tid0, wave = wave0;
@@ -315,7 +316,7 @@ key_mfma_kernel(const void* __restrict__ x, Source src, tq_layer ly, Sink sink, 
   // coordinates of the tile this wavefront writes: looked up one pass ago together with this group's loads;
   // then the lookups of the group to fetch next (long before issue() needs them)
   const int wr_b = stg.w_b, wr_lpage = stg.w_lpage, wr_h = stg.w_h;
-  stg.template lookup<ML>(src, g + gridDim.x, n_tiles, wave % ML, cum, lane);
+  stg.template lookup<ML>(src, g + n_wg, n_tiles, wave % ML, cum, lane);
   // page of that tile, read now so that the write phase does not wait for it (a page outside the table or
   // the pool comes back as -1 and is not written)
   int64_t wpage = 0;
@@ -686,6 +687,32 @@ key_mfma_kernel(const void* __restrict__ x, Source src, tq_layer ly, Sink sink, 
   }
 }
 
+template <int DT, int D, bool MSE_ONLY, bool FX, class Source, class Sink, int ML = KeyGeom<D>::MT>
+__global__ void __launch_bounds__(KQ_THREADS, 2)
+key_mfma_kernel(const void* __restrict__ x, Source src, tq_layer ly, Sink sink, int64_t n_tiles) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  key_mfma_body<DT, D, MSE_ONLY, FX, Source, Sink, ML>(x, src, ly, sink, n_tiles, blockIdx.x, gridDim.x, smem);
+}
+
+// The page write of a decode step (a token of each sequence): the workgroups of the keys, a tile each, and behind them those of the
+// values (128 channels of a tile each) in one launch.  Bound by the serial chain of a key tile (three contractions and the latency of
+// their matrices, 10 us); the values, 4 us in a launch of their own behind it, now run beside it: a token of 32 sequences
+// of 8 heads of 128 12.7 -> 9.4 us in a graph, of one 11.5 -> 8.4, of 64 (two key tiles per compute unit, the values behind them)
+// 15.9 -> 14.5; 64 x 2 heads of 256 19.5 -> 16.5
+template <int DT, int D, bool FX>
+__global__ void __launch_bounds__(KQ_THREADS, 2)
+append_small_kernel(const void* __restrict__ k, const void* __restrict__ v, PagedSource src, tq_layer ly, KeyPagedSink ks, ValPagedSink vs,
+                    int n_tiles, int gs) {
+  constexpr int SLAB = KQ_THREADS / 2;
+  extern __shared__ __align__(16) unsigned char smem[];
+  if ((int)blockIdx.x < n_tiles) {
+    key_mfma_body<DT, D, false, FX, PagedSource, KeyPagedSink, 1>(k, src, ly, ks, n_tiles, blockIdx.x, n_tiles, smem);
+    return;
+  }
+  const int id = blockIdx.x - n_tiles, tile = id / (D / SLAB), c0 = id % (D / SLAB) * SLAB;
+  if (vs.L.value_bits == 2) value_chunk_body<DT, 2>(v, src, D, SLAB, gs, vs, tile, c0, smem);
+  else value_chunk_body<DT, 4>(v, src, D, SLAB, gs, vs, tile, c0, smem);
+}
 
 __host__ static bool aligned_for_chunks(const void* x, int dtype, const FlatSource& s) {
   const int64_t ch = 16 / elem_bytes(dtype);
@@ -747,6 +774,61 @@ static int launch_dt_d(const void* x, const Source& src, const tq_layer& ly, con
   return e == hipSuccess ? TQ_OK : (int)e;
 }
 
+// Whether the centroid contraction runs on the block-scaled MFMA: head_dim 128 with the fp6 digits of Pi^T and a codebook whose Walsh
+// expansion has single-bit terms only
+static bool fp6_centroids(const tq_layer& ly) {
+  bool fx = ly.d == 128 && ly.PiT_fp6 && ly.PiT_fp6_scale && ly.Pi_colsum && ly.mse_bits <= 2 && opt_fp6_centroids.load() != 0;
+  for (int t = 0; t < ly.n_terms; ++t) fx = fx && __builtin_popcount((unsigned)ly.term_mask[t]) == 1;
+  return fx;
+}
+
+template <int DT, int D, bool FX>
+static int launch_append_small_d(const void* k, const void* v, const PagedSource& src, const tq_layer& ly, const KeyPagedSink& ks,
+                                 const ValPagedSink& vs, int tiles, hipStream_t st) {
+  constexpr size_t smem = KeySmem<DT, D>::bytes;
+  auto kern = append_small_kernel<DT, D, FX>;
+  static std::atomic<uint64_t> configured{0};           // one bit per device; the attribute is sticky
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return TQ_EINVAL;
+  if (dev >= 64 || !(configured.load() >> dev & 1)) {
+    hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    if (e != hipSuccess) return (int)e;
+    if (dev < 64) configured.fetch_or(1ull << dev);
+  }
+  const dim3 grid((unsigned)(tiles * (1 + D / (KQ_THREADS / 2))));
+  hipEvent_t ev_start = nullptr, ev_stop = nullptr;
+  if (take_time_hook(1, ev_start, ev_stop))
+    hipExtLaunchKernelGGL(kern, grid, dim3(KQ_THREADS), smem, st, ev_start, ev_stop, 0, k, v, src, ly, ks, vs, tiles, ks.L.group_size);
+  else
+    kern<<<grid, dim3(KQ_THREADS), smem, st>>>(k, v, src, ly, ks, vs, tiles, ks.L.group_size);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? TQ_OK : (int)e;
+}
+
+// Keys and values of a small append in one launch: where the keys take a workgroup per tile and the values are 16-bit chunks.
+// TQ_EUNSUPPORTED: the caller launches the two kernels.
+int launch_append_small(const void* k, const void* v, int dtype, const PagedSource& src, const tq_layer& ly, const KeyPagedSink& ks,
+                        const ValPagedSink& vs, int64_t tiles, hipStream_t st) {
+  const int opt = opt_append_small.load(std::memory_order_relaxed);
+  if (opt == 0 || tiles > (opt < 0 ? 2 * (int64_t)device_compute_units() : (int64_t)opt) || tiles > (1 << 20)) return TQ_EUNSUPPORTED;
+  if (!ly.Pi_split || !ly.PiT_split || !ly.S_split || ly.mse_bits < 1 || ly.mse_bits > 4) return TQ_EUNSUPPORTED;
+  if (!aligned_for_chunks(k, dtype, src) || !sink_ok(ks, 0) || !value_chunks_aligned(v, src) ||
+      !value_chunk_takes(dtype, vs.L.value_bits, vs.L.group_size, KQ_THREADS / 2))
+    return TQ_EUNSUPPORTED;
+  if (ly.d == 128) {
+    const bool fx = fp6_centroids(ly);
+    if (dtype == TQ_BF16)
+      return fx ? launch_append_small_d<TQ_BF16, 128, true>(k, v, src, ly, ks, vs, (int)tiles, st)
+                : launch_append_small_d<TQ_BF16, 128, false>(k, v, src, ly, ks, vs, (int)tiles, st);
+    return fx ? launch_append_small_d<TQ_F16, 128, true>(k, v, src, ly, ks, vs, (int)tiles, st)
+              : launch_append_small_d<TQ_F16, 128, false>(k, v, src, ly, ks, vs, (int)tiles, st);
+  }
+  if (ly.d == 256)
+    return dtype == TQ_BF16 ? launch_append_small_d<TQ_BF16, 256, false>(k, v, src, ly, ks, vs, (int)tiles, st)
+                            : launch_append_small_d<TQ_F16, 256, false>(k, v, src, ly, ks, vs, (int)tiles, st);
+  return TQ_EUNSUPPORTED;
+}
+
 // TQ_EUNSUPPORTED when there is no matrix-core kernel for this call (head_dim other than
 // 128 / 256, no split matrices, or operands not aligned for 16-byte loads): the caller
 // falls back to the vector-ALU kernel.
@@ -769,11 +851,7 @@ int launch_key_mfma(const void* x, int dtype, const Source& src, const tq_layer&
     }
   }
   if (paged && mse_only) return TQ_EUNSUPPORTED;
-  // head_dim 128 with the fp6 digits of Pi^T and a codebook whose Walsh expansion has single-bit terms only:
-  // the centroid contraction on the block-scaled MFMA
-  bool fx = ly.d == 128 && !mse_only && ly.PiT_fp6 && ly.PiT_fp6_scale && ly.Pi_colsum && ly.mse_bits <= 2 &&
-            opt_fp6_centroids.load() != 0;
-  for (int t = 0; t < ly.n_terms; ++t) fx = fx && __builtin_popcount((unsigned)ly.term_mask[t]) == 1;
+  const bool fx = !mse_only && fp6_centroids(ly);
 #define TQ_KQ(DT_, D_)                                                                                     \
   if (dtype == DT_ && ly.d == D_) {                                                                        \
     if constexpr (!paged)                                                                                  \
