@@ -261,6 +261,11 @@ int tq_append_kv_from_blocks(const void *k_cache, const void *v_cache, int dtype
                              const int32_t *block_table, int max_pages, const tq_layer *layer,
                              const tq_page_layout *layout, uint8_t *pool, int64_t num_pages, void *stream);
 
+/* n exact tokens (rows of row_bytes, k_stride / v_stride bytes apart) into consecutive rows of a ring's key and value planes
+ * (RingBuffer.write, capture.py:60-95).  Pointers, strides and row_bytes multiples of 16, else TQ_EUNSUPPORTED. */
+int tq_ring_write(const void* k, const void* v, int64_t k_stride, int64_t v_stride, void* k_rows, void* v_rows, int64_t row_bytes,
+                  int64_t n, void* stream);
+
 /* Gather a sequence's pages back into the reference's flat tensors
  * (store.py:92-114 get_flat_cache): idx (H, n_tok, d*eff/8), signs (H, n_tok, d/8),
  * norms (H, n_tok) input dtype, rnorms fp32, v_data (H, n_tok, d*vb/8),

@@ -703,3 +703,38 @@ def test_small_append_in_one_launch(gpu, d, B, H, T, kb, vb, gs, dtype, ragged):
             _set_option("append_small", -1)
         got.append(pool.data.clone())
     assert torch.equal(*got) and not torch.equal(got[0], torch.zeros_like(got[0]) + fill[:, None, None])
+
+
+# ------------------------------------------------------------------ a ring's rows in one launch
+@pytest.mark.parametrize("H,d,dtype,n,capacity", [(8, 128, torch.bfloat16, 1, 4), (1, 64, torch.float16, 5, 3), (3, 64, torch.float32, 257, 300),
+                                                  (5, 66, torch.bfloat16, 2, 4)])
+def test_ring_rows_from_any_layout(gpu, H, d, dtype, n, capacity):
+    """Rows of every layout a caller may hand over - side by side, in a wider tensor, heads transposed, one row repeated, misaligned, of
+    another type, needing a gradient, the ring's own - end in the ring as torch's copies leave them, whoever copies them."""
+    from turboquant_amd.capture import RingBuffer
+    g = torch.Generator().manual_seed(n)
+    wide = torch.randn(n, 3, H, d, generator=g).to(gpu, dtype)
+    flat = torch.randn(n * H * d + 1, generator=g).to(gpu, dtype)
+    forms = [wide[:, 1].contiguous(), wide[:, 1], wide[:, 0].transpose(0, 1).contiguous().transpose(0, 1), wide[:1, 2].expand(n, H, d),
+             flat[1:].view(n, H, d), wide[:, 2].double(), wide[:, 2].clone().requires_grad_()]
+    for x in forms:
+        for y in forms:
+            ring, want = RingBuffer(capacity, H, d, gpu, dtype), RingBuffer(capacity, H, d, gpu, dtype)
+            want._write_rows = lambda *a: False
+            outs = []
+            for r in (ring, want):
+                out = [r.write(x, y, n), r.write(x[:1], y[:1], 1)]
+                outs.append([t.detach() for o in out if o is not None for t in o] + [t.detach() for t in r.peek()])
+            assert len(outs[0]) == len(outs[1]) and all(torch.equal(a, b) for a, b in zip(*outs))
+            assert ring._rows.requires_grad == want._rows.requires_grad
+    ring = RingBuffer(capacity, H, d, gpu, dtype)
+    ring.write(forms[0], forms[0], 1)
+    before = ring._rows._version
+    ring.write(*ring.peek(), 1)
+    assert torch.equal(ring._rows[0, 0], ring._rows[0, 1]) and ring._rows._version > before
+    with torch.inference_mode():
+        r2 = RingBuffer(capacity, H, d, gpu, dtype)
+        r2.write(forms[0], forms[1], 1)
+        assert torch.equal(r2.peek()[0], forms[0][:1]) and torch.equal(r2.peek()[1], forms[1][:1])
+    with pytest.raises(RuntimeError):
+        r2.write(forms[0], forms[1], 1)

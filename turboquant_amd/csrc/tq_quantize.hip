@@ -763,6 +763,35 @@ extern "C" int tq_append_kv_from_blocks(const void* k_cache, const void* v_cache
   return append_runs(k_cache, v_cache, dtype, src, block_table, max_pages, layer, layout, pool, num_pages, stream);
 }
 
+namespace tq {
+// n exact tokens into a ring's key and value planes, a 16-byte chunk per thread (a copy per plane, with its slices, cost 12 us of host
+// time per decode token; this is one launch).  Bound by the latency of one load.
+__global__ void __launch_bounds__(256)
+ring_write_kernel(const uint4* __restrict__ k, const uint4* __restrict__ v, int64_t k_stride, int64_t v_stride, uint4* __restrict__ k_rows,
+                  uint4* __restrict__ v_rows, int row, int64_t chunks) {
+  const int64_t o = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (o >= chunks) return;
+  const int64_t t = o / row, c = o - t * row;
+  if (blockIdx.y == 0) k_rows[o] = k[t * k_stride + c];
+  else v_rows[o] = v[t * v_stride + c];
+}
+}  // namespace tq
+
+extern "C" int tq_ring_write(const void* k, const void* v, int64_t k_stride, int64_t v_stride, void* k_rows, void* v_rows, int64_t row_bytes,
+                             int64_t n, void* stream) {
+  if (!k || !v || !k_rows || !v_rows) return TQ_ENULL;
+  if (n < 0 || row_bytes <= 0 || row_bytes > (1 << 24)) return TQ_EINVAL;
+  if (((uintptr_t)k | (uintptr_t)v | (uintptr_t)k_rows | (uintptr_t)v_rows | (uintptr_t)k_stride | (uintptr_t)v_stride | (uintptr_t)row_bytes) & 15)
+    return TQ_EUNSUPPORTED;
+  if (n == 0) return TQ_OK;
+  const int64_t chunks = n * (row_bytes / 16);
+  if ((chunks + 255) / 256 > 0x7fffffff) return TQ_EUNSUPPORTED;
+  ring_write_kernel<<<dim3((unsigned)((chunks + 255) / 256), 2), dim3(256), 0, (hipStream_t)stream>>>(
+      (const uint4*)k, (const uint4*)v, k_stride / 16, v_stride / 16, (uint4*)k_rows, (uint4*)v_rows, (int)(row_bytes / 16), chunks);
+  TQ_CHECK_LAUNCH();
+  return TQ_OK;
+}
+
 extern "C" int tq_pool_export(const uint8_t* pool, int64_t num_pages, int H, const int32_t* block_table, int n_tok,
                               const tq_page_layout* layout, uint8_t* idx, uint8_t* signs, void* norms, float* rnorms,
                               uint8_t* v_data, void* v_scales, void* v_zeros, void* stream) {

@@ -77,17 +77,8 @@ def dequantize_values(vq: ValueQuantized, group_size: int = 32) -> torch.Tensor:
 
 
 def _plain(*tensors) -> bool:
-    """Whether torch would run an operation on these GPU tensors as it stands: ordinary fp32 tensors of four dimensions with
-    contiguous channels, nothing to differentiate, no transform, trace or dispatch mode that has to see the operation."""
-    if (torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack() or torch._C._are_functorch_transforms_active()
-            or torch.autograd.forward_ad._current_level >= 0 or torch.compiler.is_compiling() or torch.jit.is_tracing()):
-        return False
-    grad = torch.is_grad_enabled()
-    for t in tensors:
-        if (type(t) is not torch.Tensor or not t.is_cuda or t.dtype != torch.float32 or t.dim() != 4 or t.stride(-1) != 1
-                or (grad and t.requires_grad) or t.device != tensors[0].device):
-            return False
-    return True
+    """Ordinary fp32 tensors of four dimensions with contiguous channels, on which torch would run an operation as it stands."""
+    return _ffi.ordinary(*tensors) and all(t.dtype == torch.float32 and t.dim() == 4 and t.stride(-1) == 1 for t in tensors)
 
 
 class TurboQuantKVCache:

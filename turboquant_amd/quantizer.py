@@ -76,6 +76,19 @@ def _unpack_indices(packed: torch.Tensor, bits: int, d: int) -> torch.Tensor:
     return torch.stack(fields, dim=-1).reshape(*packed.shape[:-1], -1)[..., :d].long()
 
 
+def _buffer(module: torch.nn.Module, name: str) -> torch.Tensor:
+    """module.<name>, past nn.Module's attribute look-up (0.4 us apiece, seven of them per call) where it is a registered buffer."""
+    t = module._buffers.get(name)
+    return getattr(module, name) if t is None else t
+
+
+def _codes(x: torch.Tensor, n: int, *tail: int, dtype: torch.dtype = torch.uint8) -> torch.Tensor:
+    """An output row (of `tail`) per vector of x."""
+    if n == 0:                                # (as a reshape of no rows goes: refused where a width is to be inferred)
+        return torch.empty(0, *tail, dtype=dtype, device=x.device).reshape(*x.shape[:-1], *(-1 for _ in tail))
+    return torch.empty((*x.shape[:-1], *tail), dtype=dtype, device=x.device)
+
+
 def _rows(x: torch.Tensor):
     """View (..., d) as (n_vec, d) with a constant row stride, copying only if needed."""
     d = x.shape[-1]
@@ -112,7 +125,7 @@ class TurboQuantMSE(torch.nn.Module):
     def _layer(self, S: Optional[torch.Tensor] = None, ST: Optional[torch.Tensor] = None) -> _ffi.TqLayer:
         # One descriptor per state of the buffers: building it costs more host time than a decode call has to
         # spare (a dozen buffer look-ups and a library call), so it is kept until a buffer moves or is written.
-        Pi, cen, thr = self.Pi, self.centroids, self.decision_boundaries
+        Pi, cen, thr = _buffer(self, "Pi"), _buffer(self, "centroids"), _buffer(self, "decision_boundaries")
         state = (Pi.data_ptr(), Pi._version, cen.data_ptr(), cen._version, thr.data_ptr(), thr._version,
                  None if S is None else (S.data_ptr(), S._version, None if ST is None else ST.data_ptr()))
         cached = self._layer_cache
@@ -160,7 +173,7 @@ class TurboQuantMSE(torch.nn.Module):
         packed = torch.empty(n, (self.dim + per_byte - 1) // per_byte, dtype=torch.uint8, device=x.device)
         norms = torch.empty(n, dtype=x.dtype, device=x.device)
         ly = self._layer()
-        with torch.cuda.device(x.device):
+        with _ffi.on_device(x.device):
             _ffi.check(_ffi.lib().tq_quantize_keys(
                 rows.data_ptr(), _ffi.dtype_tag(x.dtype), n, stride, C.byref(ly), packed.data_ptr(), None,
                 norms.data_ptr(), None, None, None, 1, _ffi.stream_ptr(x.device)), "tq_quantize_keys")
@@ -175,7 +188,7 @@ class TurboQuantMSE(torch.nn.Module):
         n = norms.numel()
         out = torch.empty(n, self.dim, dtype=torch.float32, device=idx.device)
         ly = self._layer()
-        with torch.cuda.device(idx.device):
+        with _ffi.on_device(idx.device):
             _ffi.check(_ffi.lib().tq_dequant_keys(
                 idx.data_ptr(), None, norms.data_ptr(), _ffi.dtype_tag(norms.dtype), None, n, C.byref(ly),
                 out.data_ptr(), _ffi.stream_ptr(idx.device)), "tq_dequant_keys")
@@ -202,10 +215,11 @@ class TurboQuantProd(torch.nn.Module):
         self.qjl_scale = math.sqrt(math.pi / 2.0) / dim
 
     def _layer(self) -> _ffi.TqLayer:
-        if self._ST.device != self.S.device or getattr(self, "_ST_version", None) != self.S._version:
-            self._ST = self.S.T.contiguous()
-            self._ST_version = self.S._version
-        return self.mse_quantizer._layer(self.S, self._ST)
+        S, ST = _buffer(self, "S"), _buffer(self, "_ST")
+        if ST.device != S.device or getattr(self, "_ST_version", None) != S._version:
+            self._ST = ST = S.T.contiguous()
+            self._ST_version = S._version
+        return self.mse_quantizer._layer(S, ST)
 
     def quantize(self, x: torch.Tensor) -> ProdQuantized:
         _ffi.require_gpu(x, "x")
@@ -213,18 +227,14 @@ class TurboQuantProd(torch.nn.Module):
         n, d = rows.shape[0], self.dim
         mb = self.bits - 1
         width, per_byte = _packing(mb)
-        packed = torch.empty(n, (d + per_byte - 1) // per_byte, dtype=torch.uint8, device=x.device)
-        signs = torch.empty(n, (d + 7) // 8, dtype=torch.uint8, device=x.device)
-        norms = torch.empty(n, dtype=x.dtype, device=x.device)
-        rnorms = torch.empty(n, dtype=torch.float32, device=x.device)
+        packed, signs = _codes(x, n, (d + per_byte - 1) // per_byte), _codes(x, n, (d + 7) // 8)
+        norms, rnorms = _codes(x, n, dtype=x.dtype), _codes(x, n, dtype=torch.float32)
         ly = self._layer()
-        with torch.cuda.device(x.device):
+        with _ffi.on_device(x.device):
             _ffi.check(_ffi.lib().tq_quantize_keys(
                 rows.data_ptr(), _ffi.dtype_tag(x.dtype), n, stride, C.byref(ly), packed.data_ptr(), signs.data_ptr(),
                 norms.data_ptr(), rnorms.data_ptr(), None, None, 0, _ffi.stream_ptr(x.device)), "tq_quantize_keys")
-        lead = x.shape[:-1]
-        return ProdQuantized(mse_indices=packed.reshape(*lead, -1), qjl_signs=signs.reshape(*lead, -1),
-                             residual_norms=rnorms.reshape(lead), norms=norms.reshape(lead), mse_bits=mb)
+        return ProdQuantized(mse_indices=packed, qjl_signs=signs, residual_norms=rnorms, norms=norms, mse_bits=mb)
 
     def quantize_traced(self, x: torch.Tensor):
         """quantize() plus the two fp32 intermediates the packing consumes: the
@@ -242,7 +252,7 @@ class TurboQuantProd(torch.nn.Module):
         y = torch.empty(n, d, dtype=torch.float32, device=dev)
         p = torch.empty(n, d, dtype=torch.float32, device=dev)
         ly = self._layer()
-        with torch.cuda.device(dev):
+        with _ffi.on_device(dev):
             _ffi.check(_ffi.lib().tq_quantize_keys(
                 rows.data_ptr(), _ffi.dtype_tag(x.dtype), n, stride, C.byref(ly), packed.data_ptr(), signs.data_ptr(),
                 norms.data_ptr(), rnorms.data_ptr(), y.data_ptr(), p.data_ptr(), 0, _ffi.stream_ptr(dev)),
@@ -261,7 +271,7 @@ class TurboQuantProd(torch.nn.Module):
         n = norms.numel()
         out = torch.empty(n, self.dim, dtype=torch.float32, device=idx.device)
         ly = self._layer()
-        with torch.cuda.device(idx.device):
+        with _ffi.on_device(idx.device):
             _ffi.check(_ffi.lib().tq_dequant_keys(
                 idx.data_ptr(), signs.data_ptr(), norms.data_ptr(), _ffi.dtype_tag(norms.dtype), rnorms.data_ptr(), n,
                 C.byref(ly), out.data_ptr(), _ffi.stream_ptr(idx.device)), "tq_dequant_keys")
@@ -272,18 +282,24 @@ class TurboQuantProd(torch.nn.Module):
         without the 1/sqrt(d) factor."""
         _ffi.require_gpu(query, "query")
         d = self.dim
-        lead = torch.broadcast_shapes(query.shape[:-2], quantized_key.norms.shape[:-1])
+        lead = query.shape[:-2]
+        if lead != quantized_key.norms.shape[:-1]:
+            lead = torch.broadcast_shapes(lead, quantized_key.norms.shape[:-1])
         n_q, n_k = query.shape[-2], quantized_key.norms.shape[-1]
-        q = query.expand(*lead, n_q, d).contiguous()
-        idx = quantized_key.mse_indices.expand(*lead, n_k, quantized_key.mse_indices.shape[-1]).contiguous()
-        signs = quantized_key.qjl_signs.expand(*lead, n_k, quantized_key.qjl_signs.shape[-1]).contiguous()
-        norms = quantized_key.norms.expand(*lead, n_k).contiguous()
-        rnorms = quantized_key.residual_norms.expand(*lead, n_k).contiguous().float()
+
+        def spread(t, *tail):
+            return (t if t.shape == lead + tail else t.expand(*lead, *tail)).contiguous()
+
+        q = spread(query, n_q, d)
+        idx = spread(quantized_key.mse_indices, n_k, quantized_key.mse_indices.shape[-1])
+        signs = spread(quantized_key.qjl_signs, n_k, quantized_key.qjl_signs.shape[-1])
+        norms = spread(quantized_key.norms, n_k)
+        rnorms = spread(quantized_key.residual_norms, n_k).float()
         batch = int(math.prod(lead)) if len(lead) else 1
         scores = torch.empty(*lead, n_q, n_k, dtype=torch.float32, device=q.device)
         work = torch.empty(2 * batch * n_q * d, dtype=torch.float32, device=q.device)
         ly = self._layer()
-        with torch.cuda.device(q.device):
+        with _ffi.on_device(q.device):
             _ffi.check(_ffi.lib().tq_score(
                 q.data_ptr(), _ffi.dtype_tag(q.dtype), batch, n_q, idx.data_ptr(), signs.data_ptr(), norms.data_ptr(),
                 _ffi.dtype_tag(norms.dtype), rnorms.data_ptr(), n_k, C.byref(ly), scores.data_ptr(), work.data_ptr(),

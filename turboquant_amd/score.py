@@ -53,11 +53,12 @@ def compute_hybrid_attention(query: torch.Tensor, store: CompressedKVStore, rece
     q = query.to(work_dtype)
     pool = store.ensure_pool(store.pool.dtype if store.pool is not None else
                              (recent_k.dtype if has_recent else query.dtype))
-    seq_lens = torch.full((T,), n_hist if has_history else 0, dtype=torch.int32, device=pool.device)
+    seq_lens = store.lengths(n_hist if has_history else 0, T)
     rk = rv = None
     if has_recent:
-        rk = recent_k.to(work_dtype).unsqueeze(0).expand(T, *recent_k.shape)
-        rv = recent_v.to(work_dtype).unsqueeze(0).expand(T, *recent_v.shape)
+        rk, rv = recent_k.to(work_dtype).unsqueeze(0), recent_v.to(work_dtype).unsqueeze(0)
+        if T != 1:
+            rk, rv = rk.expand(T, *recent_k.shape), rv.expand(T, *recent_v.shape)
     out = pool.decode_attention(q, store.block_table[0], seq_lens, scale=scale, recent_k=rk, recent_v=rv,
                                 max_len=max(n_hist, 1))
     return out.to(query.dtype)

@@ -44,6 +44,7 @@ class CompressedKVStore:
         self._chunk_lengths: list[int] = []
         self._pool: Optional[PagedKVPool] = None
         self._block_table: Optional[torch.Tensor] = None
+        self._counts: Optional[torch.Tensor] = None
         self._flat: Optional[FlatCache] = None
 
     # ---- bookkeeping ---------------------------------------------------------------
@@ -72,8 +73,16 @@ class CompressedKVStore:
         elif need > self._pool.num_pages:
             self._pool.grow(max(need, 2 * self._pool.num_pages))
         if self._block_table is None or self._block_table.shape[1] != self._pool.num_pages:
-            self._block_table = torch.arange(self._pool.num_pages, dtype=torch.int32, device=self._pool.device)[None, :]
+            # (0, 1, 2, ...: the pages in order, and every length the sequence can have, so that a step need not write its own)
+            self._counts = torch.arange(self._pool.num_pages * PAGE_TOKENS + 1, dtype=torch.int32, device=self._pool.device)
+            self._block_table = self._counts[None, : self._pool.num_pages]
         return self._pool
+
+    def lengths(self, n: int, rows: int) -> torch.Tensor:
+        """n, `rows` times, as the decode kernels read it.  The pool has to exist."""
+        if rows == 1 and n < self._counts.shape[0]:
+            return self._counts[n: n + 1]
+        return torch.full((rows,), n, dtype=torch.int32, device=self._pool.device)
 
     # ---- write -----------------------------------------------------------------------
     def append_chunk(self, key: torch.Tensor, value: torch.Tensor):
@@ -85,8 +94,8 @@ class CompressedKVStore:
         pool = self.ensure_pool(key.dtype, start + chunk_len)
         if key.dtype != pool.dtype:
             raise TypeError(f"store holds {pool.dtype} pages; got a {key.dtype} chunk")
-        start_pos = torch.tensor([start], dtype=torch.int32, device=pool.device)
-        pool.append(key.unsqueeze(0), value.unsqueeze(0), self._block_table, start_pos)
+        # (a number copied from the host would wait for the stream: 40 us of a chat turn's first token)
+        pool.append(key.unsqueeze(0), value.unsqueeze(0), self._block_table, self.lengths(start, 1))
         self._chunk_lengths.append(chunk_len)
         self._flat = None
 
