@@ -738,3 +738,40 @@ def test_ring_rows_from_any_layout(gpu, H, d, dtype, n, capacity):
         assert torch.equal(r2.peek()[0], forms[0][:1]) and torch.equal(r2.peek()[1], forms[1][:1])
     with pytest.raises(RuntimeError):
         r2.write(forms[0], forms[1], 1)
+
+
+# ------------------------------------------------------------------ groups of tiles that are heads of one page, and others
+@pytest.mark.parametrize("d,H,kb,dtype", [(128, 8, 3, torch.bfloat16), (128, 6, 2, torch.float16), (128, 7, 4, torch.bfloat16), (256, 3, 3, torch.bfloat16),
+                                          (256, 4, 4, torch.float16)])
+@pytest.mark.parametrize("form", ["runs", "ragged", "blocks"])
+def test_append_of_many_heads_is_that_of_each(gpu, d, H, kb, dtype, form):
+    """More tiles than a launch of single tiles takes: groups whose tiles are heads of one page share an address, groups that
+    begin in one page and end in the next do not.  Every head's pages are those of a pool that holds it alone."""
+    g = torch.Generator().manual_seed(10 * d + H)
+    B, T = 3, 1500
+    tq = TurboQuantProd(d, bits=kb, device=gpu)
+    per_seq = T // 16 + 4
+    table = torch.randperm(B * per_seq, generator=g).view(B, per_seq).to(torch.int32).to(gpu)
+    lens, starts = [T, T - 33, 700], [0, 5, 31]
+    if form == "blocks":
+        starts = [16, 0, 32]
+    k, v = (torch.randn(B, T, H + 1, d, generator=g).to(gpu, dtype) for _ in range(2))
+    blocks = torch.randn(2, B * per_seq, 16, H + 1, d, generator=g).to(gpu, dtype)
+    src = torch.randperm(B * per_seq, generator=g).view(B, per_seq).to(torch.int32).to(gpu)
+
+    def pages(lo, n):
+        pool = PagedKVPool(tq, n, B * per_seq, value_bits=2, dtype=dtype, device=gpu)
+        kk, vv = k[:, :, lo:lo + n], v[:, :, lo:lo + n]
+        if form == "runs":
+            pool.append(kk, vv, table, start_pos=_i32(starts, gpu))
+        elif form == "ragged":
+            pool.append_ragged(kk.reshape(B * T, n, d), vv.reshape(B * T, n, d), _i32([0, T, 2 * T], gpu), _i32(lens, gpu), _i32(starts, gpu), table,
+                               max_run=T)
+        else:
+            pool.append_from_blocks(blocks[0][:, :, lo:lo + n], blocks[1][:, :, lo:lo + n], src, table, _i32(lens, gpu), start_pos=_i32(starts, gpu),
+                                    max_tokens=T)
+        return pool.data
+
+    whole = pages(0, H)
+    for h in range(H):
+        assert torch.equal(whole[:, h], pages(h, 1)[:, 0])
