@@ -775,3 +775,27 @@ def test_append_of_many_heads_is_that_of_each(gpu, d, H, kb, dtype, form):
     whole = pages(0, H)
     for h in range(H):
         assert torch.equal(whole[:, h], pages(h, 1)[:, 0])
+
+
+# ------------------------------------------------------------------ the last round of a large append
+@pytest.mark.parametrize("d,H,rest", [(128, 8, 8), (128, 8, 512), (128, 8, 520), (128, 3, 301), (256, 2, 2), (256, 2, 256), (256, 2, 258), (256, 1, 511)])
+@pytest.mark.parametrize("ragged", [False, True])
+def test_last_round_of_single_tiles(gpu, d, H, rest, ragged):
+    """`rest` tiles more than whole rounds of 512 workgroups: up to the limit of the rule, one behind it.  The pages are those of
+    appends of a few tokens each."""
+    g = torch.Generator().manual_seed(d + rest)
+    tiles = 512 * (8192 // d // 16)
+    pages = -(-(tiles + rest) // H)
+    N = 16 * pages - 3
+    tq = TurboQuantProd(d, bits=3, device=gpu)
+    k, v = (torch.randn(1, N, H, d, generator=g).bfloat16().to(gpu) for _ in range(2))
+    table = torch.randperm(2 * pages, generator=g).view(2, pages).to(torch.int32).to(gpu)
+    got, want = (PagedKVPool(tq, H, 2 * pages, value_bits=2, device=gpu) for _ in range(2))
+    if ragged:
+        got.append_ragged(k[0], v[0], _i32([N, 0], gpu), _i32([0, N], gpu), _i32([0, 0], gpu), table, max_run=N)
+    else:
+        got.append(k, v, table[1:])
+    step = 4096
+    for t in range(0, N, step):
+        want.append(k[:, t:t + step], v[:, t:t + step], table[1:], start_pos=_i32([t], gpu))
+    assert torch.equal(got.data, want.data)

@@ -173,11 +173,10 @@ struct XStage {
       lane_off[k] = (int64_t)slot[k] * src.slot_stride() + ck * CH;
     }
   }
-  // uniform part for `group`: tile addresses, and (paged sources) the coordinates of tile group * MT + wtile
-  // (ML: tiles of a group that hold vectors - groups are ML tiles apart; the other MT - ML are not loaded)
+  // uniform part for the group that begins with tile0: tile addresses, and (paged sources) the coordinates of tile tile0 + wtile
+  // (ML: tiles of a group that hold vectors; the other MT - ML are not loaded)
   template <int ML = Gm::MT>
-  __device__ __forceinline__ void lookup(const Source& src, int64_t group, int64_t n_tiles, int wtile, const int* cum, int lane) {
-    const int64_t tile0 = group * ML;
+  __device__ __forceinline__ void lookup(const Source& src, int64_t tile0, int64_t n_tiles, int wtile, const int* cum, int lane) {
     const int64_t first = tile0 < n_tiles ? tile0 : 0;
 #pragma unroll
     for (int m = 0; m < Gm::MT; ++m) live[m] = m < ML && tile0 + m < n_tiles;
@@ -263,10 +262,11 @@ __device__ __forceinline__ void plane_bits(uint32_t (&bits)[2][4]) {
 // fp32 product sum).  10 MFMAs per 16 x 16 tile instead of 24, and no centroid terms go through the LDS.
 // ML (1 or the MT tiles of a group): small appends - the page write of a decode step - give every 16-vector tile a
 // workgroup of its own that computes one tile instead of four, a quarter of the instructions behind one another.
-// Workgroup `id` of the n_wg that share the groups.
-template <int DT, int D, bool MSE_ONLY, bool FX, class Source, class Sink, int ML>
-__device__ __forceinline__ void key_mfma_body(const void* __restrict__ x, const Source& src, const tq_layer& ly, const Sink& sink,
-                                              int64_t n_tiles, int id, int n_wg, unsigned char* smem) {
+// Workgroup `id` of the n_wg that share the tiles first .. n_tiles - 1.  SPLIT: what would be a last round with fewer tiles than
+// workgroups is left out; returns the first tile of it (n_tiles: nothing left), and n_tiles as it turned out for runs of different length.
+template <int DT, int D, bool MSE_ONLY, bool FX, class Source, class Sink, int ML, bool SPLIT = false>
+__device__ __forceinline__ int64_t key_mfma_body(const void* __restrict__ x, const Source& src, const tq_layer& ly, const Sink& sink,
+                                                 int64_t first, int64_t& n_tiles, int id, int n_wg, unsigned char* smem) {
   static_assert(!FX || (D == 128 && !MSE_ONLY), "the fp6 centroid contraction: head_dim 128, full quantiser");
   constexpr int mse_only = MSE_ONLY;
   using E = Elem<DT>;
@@ -320,16 +320,21 @@ __device__ __forceinline__ void key_mfma_body(const void* __restrict__ x, const 
   // the LDS), so that a workgroup computes no empty ones and the live ones are dealt out evenly.  Nine prompts of
   // 17 .. 4099 tokens, 2 KV heads of 256 (a quarter of the 4644 tiles exist): call 154.6 -> 62.5 us.
   int* cum = (int*)(smem + Sm::bytes);
-  if constexpr (std::is_same<Source, RaggedSource>::value) {
+  if constexpr (std::is_same<Source, RaggedSource>::value && (SPLIT || ML == MT)) {
     src.template page_index<KQ_THREADS>(cum, cum + src.B + 1, tid0);
     n_tiles = (int64_t)__builtin_amdgcn_readfirstlane(cum[src.B]) * src.H;
   }
-  const int64_t n_groups = (n_tiles + ML - 1) / ML;             // a group = the TT vectors of one pass
-  if (id >= n_groups) return;
+  int64_t end = n_tiles;
+  if constexpr (SPLIT) {
+    const int64_t rounds = n_tiles / ((int64_t)ML * n_wg), whole = rounds * ML * n_wg;
+    if (n_tiles - whole <= (D == 128 ? n_wg : n_wg / 2)) end = whole;
+  }
+  const int64_t n_groups = (end - first + ML - 1) / ML;         // a group = the TT vectors of one pass
+  if (id >= n_groups) return end;
   // (1) staging (XStage): the next group's chunks wait in registers while the current group is worked on
   XStage<DT, D, Source> stg;
   stg.init(src, tid0);
-  stg.template lookup<ML>(src, id, n_tiles, wave0 % ML, cum, tid0 & 63);
+  stg.template lookup<ML>(src, first + (int64_t)id * ML, end, wave0 % ML, cum, tid0 & 63);
   stg.issue(x);
 
   for (int64_t g = id; g < n_groups; g += n_wg) {
@@ -338,16 +343,16 @@ __device__ __forceinline__ void key_mfma_body(const void* __restrict__ x, const 
   int tid = tid0, wave = wave0;
   asm volatile("" : "+v"(tid), "+s"(wave));
   const int lane = tid & 63, n = lane & 15, kb = lane >> 4;
-  const int64_t tile0 = g * ML;
+  const int64_t tile0 = first + g * ML;
   // coordinates of the tile this wavefront writes: looked up one pass ago together with this group's loads;
   // then the lookups of the group to fetch next (long before issue() needs them)
   const int wr_b = stg.w_b, wr_lpage = stg.w_lpage, wr_h = stg.w_h;
-  stg.template lookup<ML>(src, g + n_wg, n_tiles, wave % ML, cum, lane);
+  stg.template lookup<ML>(src, first + (g + n_wg) * ML, end, wave % ML, cum, lane);
   // page of that tile, read now so that the write phase does not wait for it (a page outside the table or
   // the pool comes back as -1 and is not written)
   int64_t wpage = 0;
   if constexpr (!std::is_same<Sink, KeyFlatSink>::value) {
-    if (tile0 + wave % ML < n_tiles) wpage = checked_page(sink.block_table, sink.max_pages, sink.num_pages, wr_b, wr_lpage);
+    if (tile0 + wave % ML < end) wpage = checked_page(sink.block_table, sink.max_pages, sink.num_pages, wr_b, wr_lpage);
   }
   stg.template store<XRS>(sx, svalid, tid);
   __syncthreads();
@@ -695,7 +700,7 @@ __device__ __forceinline__ void key_mfma_body(const void* __restrict__ x, const 
     const int planes = mb + 1;
     for (int m = wave % ML; m < ML; m += KQ_WAVES) {
       const int64_t tile = tile0 + m;
-      if (tile >= n_tiles) break;
+      if (tile >= end) break;
       // a tile none of whose slots exists may lie beyond the block table: do not look it up
       // (and a page outside the table or the pool is not written)
       if (__builtin_amdgcn_ballot_w64(lane < TILE && svalid[16 * m + lane]) == 0 || wpage < 0) continue;
@@ -718,13 +723,24 @@ __device__ __forceinline__ void key_mfma_body(const void* __restrict__ x, const 
   }
   __syncthreads();                                              // the next group overwrites what the writers read
   }
+  return end;
 }
 
 template <int DT, int D, bool MSE_ONLY, bool FX, class Source, class Sink, int ML = KeyGeom<D>::MT>
 __global__ void __launch_bounds__(KQ_THREADS, 2)
 key_mfma_kernel(const void* __restrict__ x, Source src, tq_layer ly, Sink sink, int64_t n_tiles) {
   extern __shared__ __align__(16) unsigned char smem[];
-  key_mfma_body<DT, D, MSE_ONLY, FX, Source, Sink, ML>(x, src, ly, sink, n_tiles, blockIdx.x, gridDim.x, smem);
+  if constexpr (ML == KeyGeom<D>::MT && std::is_same<Sink, KeyPagedSink>::value && !MSE_ONLY) {
+    // A last round of fewer tiles than workgroups is dealt out a tile each instead of a group to a few of them: the round is as long as
+    // a tile then, and not as a group: key kernel, head_dim 128, 8 heads of 4176 tokens (2088 tiles, 512 workgroups of four at a time)
+    // 28.7 -> 23.8 us, of 5120 28.0 -> 27.0, of 8384 39.9 -> 33.7.  At 256, where the matrices of a tile keep its compute unit busy, only up
+    // to a tile per compute unit: 2 heads of 8352 44.6 -> 42.1, of 10240 45.1 -> 43.5 (of 12288, two tiles per compute unit, 47.3 -> 56.2)
+    const int64_t rest = key_mfma_body<DT, D, MSE_ONLY, FX, Source, Sink, ML, true>(x, src, ly, sink, 0, n_tiles, blockIdx.x, gridDim.x, smem);
+    if (rest + blockIdx.x < n_tiles)
+      key_mfma_body<DT, D, MSE_ONLY, FX, Source, Sink, 1>(x, src, ly, sink, rest, n_tiles, blockIdx.x, gridDim.x, smem);
+  } else {
+    key_mfma_body<DT, D, MSE_ONLY, FX, Source, Sink, ML>(x, src, ly, sink, 0, n_tiles, blockIdx.x, gridDim.x, smem);
+  }
 }
 
 // The page write of a decode step (a token of each sequence): the workgroups of the keys, a tile each, and behind them those of the
@@ -739,7 +755,8 @@ append_small_kernel(const void* __restrict__ k, const void* __restrict__ v, Page
   constexpr int SLAB = KQ_THREADS / 2;
   extern __shared__ __align__(16) unsigned char smem[];
   if ((int)blockIdx.x < n_tiles) {
-    key_mfma_body<DT, D, false, FX, PagedSource, KeyPagedSink, 1>(k, src, ly, ks, n_tiles, blockIdx.x, n_tiles, smem);
+    int64_t end = n_tiles;
+    key_mfma_body<DT, D, false, FX, PagedSource, KeyPagedSink, 1>(k, src, ly, ks, 0, end, blockIdx.x, n_tiles, smem);
     return;
   }
   const int id = blockIdx.x - n_tiles, tile = id / (D / SLAB), c0 = id % (D / SLAB) * SLAB;
