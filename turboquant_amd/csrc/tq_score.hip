@@ -240,8 +240,6 @@ prep_mfma_kernel(const uint16_t* __restrict__ q, int G, int64_t n_rows, tq_layer
     prefetch_pages_body<PREP_MFMA_THREADS>(pf, id - n_prep);
 }
 
-constexpr int QT = 8;              // queries per workgroup of the byte-wise kernel
-
 // The exact tokens of a cache object: fp32 rows (batch, H, n, d) with element strides, and the queries they meet.
 struct CacheTail {
   const float* q;
@@ -263,21 +261,29 @@ struct CacheTail {
 constexpr int SCORE_KEYS = 64;     // keys per workgroup: sixteen for each of four wavefronts
 constexpr int SCORE_ROWS = 4;      // exact rows per workgroup: one per wavefront (eight behind one another, 4000 keys and 128 rows of 8 heads: 9.7 us, now 7.8)
 
-template <int EFF, int NT>
+// Word w of a row of codes; BYTES: rows that are not 4-byte aligned
+template <bool BYTES>
+__device__ __forceinline__ uint32_t code_word(const uint8_t* __restrict__ row, int w) {
+  if constexpr (!BYTES) return ((const uint32_t*)row)[w];
+  const uint8_t* p = row + 4 * w;
+  return p[0] | (uint32_t)p[1] << 8 | (uint32_t)p[2] << 16 | (uint32_t)p[3] << 24;
+}
+
+template <int EFF, int NT, bool BYTES>
 __device__ __forceinline__ void score_tiles(const float* __restrict__ rot, const float* __restrict__ sk, const int64_t (&row)[NT],
-                                            const float* s_cent, int d, int kb, const uint32_t* __restrict__ ip,
-                                            const uint32_t* __restrict__ sp, prep_f32x4 (&am)[NT], prep_f32x4 (&aq)[NT]) {
+                                            const float* s_cent, int d, int kb, const uint8_t* __restrict__ ip,
+                                            const uint8_t* __restrict__ sp, prep_f32x4 (&am)[NT], prep_f32x4 (&aq)[NT]) {
   typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));        // (the caller's scratch: any float address)
   constexpr unsigned mask = (1u << EFF) - 1u;
   for (int c0 = 0; c0 < d; c0 += 64) {
     uint32_t sb[2], iw[4];                                      // shifted to this lane's four coordinates of each sixteen
 #pragma unroll
-    for (int j = 0; j < 2; ++j) sb[j] = sp[(c0 >> 5) + j] >> (4 * kb);
+    for (int j = 0; j < 2; ++j) sb[j] = code_word<BYTES>(sp, (c0 >> 5) + j) >> (4 * kb);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      if (EFF == 1) iw[j] = ip[(c0 >> 5) + (j >> 1)] >> (16 * (j & 1) + 4 * kb);
-      if (EFF == 2) iw[j] = ip[(c0 >> 4) + j] >> (8 * kb);
-      if (EFF == 4) iw[j] = ip[(c0 >> 3) + 2 * j + (kb >> 1)] >> (16 * (kb & 1));
+      if (EFF == 1) iw[j] = code_word<BYTES>(ip, (c0 >> 5) + (j >> 1)) >> (16 * (j & 1) + 4 * kb);
+      if (EFF == 2) iw[j] = code_word<BYTES>(ip, (c0 >> 4) + j) >> (8 * kb);
+      if (EFF == 4) iw[j] = code_word<BYTES>(ip, (c0 >> 3) + 2 * j + (kb >> 1)) >> (16 * (kb & 1));
     }
     f32x4_u r[NT][4], k[NT][4];
 #pragma unroll
@@ -302,7 +308,7 @@ __device__ __forceinline__ void score_tiles(const float* __restrict__ rot, const
   }
 }
 
-template <bool CACHE, int NT>
+template <bool CACHE, int NT, bool BYTES = false>
 __global__ void __launch_bounds__(256)
 score_kernel(const float* __restrict__ q_rot, const float* __restrict__ q_sk, int64_t n_q,
              const uint8_t* __restrict__ idx, const uint8_t* __restrict__ signs, const void* __restrict__ norms,
@@ -335,8 +341,8 @@ score_kernel(const float* __restrict__ q_rot, const float* __restrict__ q_sk, in
   const int n = lane & 15, kb = lane >> 4;
   const int64_t key = k0 + n < n_k ? k0 + n : n_k - 1;          // (keys and queries that do not exist: the last one, not stored)
   const int eff = eff_bits(mb);
-  const uint32_t* ip = (const uint32_t*)(idx + (b * n_k + key) * idx_row_bytes(d, mb));
-  const uint32_t* sp = (const uint32_t*)(signs + (b * n_k + key) * (d >> 3));
+  const uint8_t* ip = idx + (b * n_k + key) * idx_row_bytes(d, mb);
+  const uint8_t* sp = signs + (b * n_k + key) * (d >> 3);
   int64_t row[NT];
   prep_f32x4 am[NT], aq[NT];
 #pragma unroll
@@ -347,9 +353,9 @@ score_kernel(const float* __restrict__ q_rot, const float* __restrict__ q_sk, in
   }
   const float nk = load_as_f32(norms, b * n_k + key, norm_dtype);
   const float rk = __fmul_rn(ly.qjl_scale, rnorms[b * n_k + key]);
-  if (eff == 1) score_tiles<1, NT>(q_rot, q_sk, row, s_cent, d, kb, ip, sp, am, aq);
-  else if (eff == 2) score_tiles<2, NT>(q_rot, q_sk, row, s_cent, d, kb, ip, sp, am, aq);
-  else score_tiles<4, NT>(q_rot, q_sk, row, s_cent, d, kb, ip, sp, am, aq);
+  if (eff == 1) score_tiles<1, NT, BYTES>(q_rot, q_sk, row, s_cent, d, kb, ip, sp, am, aq);
+  else if (eff == 2) score_tiles<2, NT, BYTES>(q_rot, q_sk, row, s_cent, d, kb, ip, sp, am, aq);
+  else score_tiles<4, NT, BYTES>(q_rot, q_sk, row, s_cent, d, kb, ip, sp, am, aq);
   if (k0 + n >= n_k) return;
   // (CACHE: the rows of scores go on with those of the exact tokens, and all of them are scaled)
 #pragma unroll
@@ -369,56 +375,6 @@ score_kernel(const float* __restrict__ q_rot, const float* __restrict__ q_sk, in
 __host__ static int score_query_tiles(int64_t batch, int64_t n_q, int64_t n_k) {
   if (n_q <= 16) return 1;
   return batch * ((n_q + 31) / 32) * ((n_k + SCORE_KEYS - 1) / SCORE_KEYS) >= 2 * (int64_t)device_compute_units() ? 2 : 1;
-}
-
-// the same sums with byte loads, for index / sign rows that are not 4-byte aligned
-__global__ void __launch_bounds__(256)
-score_bytes_kernel(const float* __restrict__ q_rot, const float* __restrict__ q_sk, int64_t n_q,
-                   const uint8_t* __restrict__ idx, const uint8_t* __restrict__ signs, const void* __restrict__ norms,
-                   int norm_dtype, const float* __restrict__ rnorms, int64_t n_k, tq_layer ly,
-                   float* __restrict__ scores) {
-  extern __shared__ float sm[];
-  const int d = ly.d, mb = ly.mse_bits;
-  float* s_rot = sm;              // [QT][d]
-  float* s_sk = sm + QT * d;      // [QT][d]
-  float* s_cent = s_sk + QT * d;  // [16]
-  const int64_t b = blockIdx.z;
-  const int64_t q0 = (int64_t)blockIdx.y * QT;
-  const int nq = (int)((n_q - q0) < QT ? (n_q - q0) : QT);
-  for (int o = threadIdx.x; o < QT * d; o += blockDim.x) {
-    int i = o / d;
-    bool ok = i < nq;
-    s_rot[o] = ok ? q_rot[(b * n_q + q0) * d + o] : 0.0f;
-    s_sk[o] = ok ? q_sk[(b * n_q + q0) * d + o] : 0.0f;
-  }
-  if (threadIdx.x < (1 << mb)) s_cent[threadIdx.x] = ly.centroids[threadIdx.x];
-  __syncthreads();
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n_k) return;
-  const int eff = eff_bits(mb), per = 8 / eff, row = idx_row_bytes(d, mb), srow = d >> 3;
-  const unsigned mask = (1u << eff) - 1u;
-  const uint8_t* ip = idx + (b * n_k + k) * row;
-  const uint8_t* sp = signs + (b * n_k + k) * srow;
-  float am[QT], aq[QT];
-#pragma unroll
-  for (int i = 0; i < QT; ++i) am[i] = aq[i] = 0.0f;
-  for (int c0 = 0; c0 < d; c0 += 8) {
-    unsigned sb = sp[c0 >> 3];
-    for (int s = 0; s < 8; ++s) {
-      int c = c0 + s;
-      unsigned byte = ip[c / per];
-      float cv = s_cent[(byte >> (eff * (c % per))) & mask];
-      float sg = ((sb >> s) & 1u) ? 1.0f : -1.0f;
-#pragma unroll
-      for (int i = 0; i < QT; ++i) {
-        am[i] = fmaf(s_rot[i * d + c], cv, am[i]);
-        aq[i] = fmaf(s_sk[i * d + c], sg, aq[i]);
-      }
-    }
-  }
-  const float nk = load_as_f32(norms, b * n_k + k, norm_dtype);
-  const float rk = __fmul_rn(ly.qjl_scale, rnorms[b * n_k + k]);
-  for (int i = 0; i < nq; ++i) scores[(b * n_q + q0 + i) * n_k + k] = __fadd_rn(__fmul_rn(am[i], nk), __fmul_rn(aq[i], rk));
 }
 
 // x_hat for a tile of TILE vectors: (c[idx] Pi) * norm + (sigma S) * (qjl_scale * rnorm)
@@ -795,17 +751,13 @@ extern "C" int tq_score(const void* q, int dtype, int64_t batch, int64_t n_q, co
   float* q_sk = work + batch * n_q * d;
   rc = tq_rotate_query(q, dtype, batch * n_q, layer, q_rot, q_sk, stream);
   if (rc) return rc;
-  if ((uintptr_t)idx % 4 == 0 && (uintptr_t)signs % 4 == 0) {
-    const int nt = score_query_tiles(batch, n_q, n_k);
-    const dim3 grid((unsigned)((n_k + SCORE_KEYS - 1) / SCORE_KEYS), (unsigned)((n_q + 16 * nt - 1) / (16 * nt)), (unsigned)batch);
-    auto kern = nt == 2 ? score_kernel<false, 2> : score_kernel<false, 1>;
-    kern<<<grid, dim3(256), 0, (hipStream_t)stream>>>(q_rot, q_sk, n_q, idx, signs, norms, norm_dtype, rnorms, n_k, *layer, scores,
-                                                      CacheTail{});
-  } else {
-    const dim3 grid((unsigned)((n_k + 255) / 256), (unsigned)((n_q + QT - 1) / QT), (unsigned)batch);
-    score_bytes_kernel<<<grid, dim3(256), (2 * QT * d + 16) * sizeof(float), (hipStream_t)stream>>>(
-        q_rot, q_sk, n_q, idx, signs, norms, norm_dtype, rnorms, n_k, *layer, scores);
-  }
+  const int nt = score_query_tiles(batch, n_q, n_k);
+  const dim3 grid((unsigned)((n_k + SCORE_KEYS - 1) / SCORE_KEYS), (unsigned)((n_q + 16 * nt - 1) / (16 * nt)), (unsigned)batch);
+  const bool words = (uintptr_t)idx % 4 == 0 && (uintptr_t)signs % 4 == 0;
+  auto kern = words ? (nt == 2 ? score_kernel<false, 2> : score_kernel<false, 1>)
+                    : (nt == 2 ? score_kernel<false, 2, true> : score_kernel<false, 1, true>);
+  kern<<<grid, dim3(256), 0, (hipStream_t)stream>>>(q_rot, q_sk, n_q, idx, signs, norms, norm_dtype, rnorms, n_k, *layer, scores,
+                                                    CacheTail{});
   TQ_CHECK_LAUNCH();
   return TQ_OK;
 }
