@@ -396,3 +396,28 @@ def test_bench_refuses_more_than_one_gpu_and_its_shape_table_is_well_formed():
     # 3-bit keys (2-bit indices), 2-bit values in groups of 32 at head_dim 256: 64 + 32 + 2 + 2 + 64 + 32 bytes
     assert bench.algorithmic_bytes_per_token_head(256, 2, 2, 32) == 196
     assert bench.algorithmic_bytes_per_token_head(128, 2, 4, 32) == 132
+
+
+def test_a_rearranged_block_table_leaves_the_lengths_alone(monkeypatch):
+    """A store's block_table is the caller's to rearrange (pages swapped, another page put in); the lengths and start positions
+    of later calls are numbers of their own."""
+    from turboquant_amd import store as ST
+    calls = []
+
+    class Pool:
+        def __init__(self, quantizer, heads, pages, *args, dtype, device):
+            self.num_pages, self.dtype, self.device = pages, dtype, torch.device("cpu")
+
+        def append(self, key, value, block_table, start_pos=None):
+            calls.append((block_table.tolist(), start_pos.tolist()))
+
+    monkeypatch.setattr(ST, "PagedKVPool", Pool)
+    st = ST.CompressedKVStore(64, 1, device=torch.device("cpu"))
+    x = torch.zeros(3, 1, 64)
+    st.append_chunk(x, x)
+    table = st.block_table
+    table.copy_(table.flip(1))
+    st.append_chunk(x, x)
+    pages = list(range(st.pool.num_pages))
+    assert calls == [([pages], [0]), ([pages[::-1]], [3])]
+    assert [st.lengths(n, 1).tolist() for n in (0, 3, 63)] == [[0], [3], [63]] and st.lengths(5, 3).tolist() == [5, 5, 5]

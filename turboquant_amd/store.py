@@ -73,9 +73,10 @@ class CompressedKVStore:
         elif need > self._pool.num_pages:
             self._pool.grow(max(need, 2 * self._pool.num_pages))
         if self._block_table is None or self._block_table.shape[1] != self._pool.num_pages:
-            # (0, 1, 2, ...: the pages in order, and every length the sequence can have, so that a step need not write its own)
+            self._block_table = torch.arange(self._pool.num_pages, dtype=torch.int32, device=self._pool.device)[None, :]
+            # (every length the sequence can have, so that a step need not write its own; memory apart from the table's, which a
+            # caller may rearrange)
             self._counts = torch.arange(self._pool.num_pages * PAGE_TOKENS + 1, dtype=torch.int32, device=self._pool.device)
-            self._block_table = self._counts[None, : self._pool.num_pages]
         return self._pool
 
     def lengths(self, n: int, rows: int) -> torch.Tensor:
