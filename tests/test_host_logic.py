@@ -421,3 +421,32 @@ def test_a_rearranged_block_table_leaves_the_lengths_alone(monkeypatch):
     pages = list(range(st.pool.num_pages))
     assert calls == [([pages], [0]), ([pages[::-1]], [3])]
     assert [st.lengths(n, 1).tolist() for n in (0, 3, 63)] == [[0], [3], [63]] and st.lengths(5, 3).tolist() == [5, 5, 5]
+
+
+def test_a_compressed_part_put_in_by_hand_is_taken_as_it_is():
+    """The cache object's entries for fp32 read codes of the cache's own bits and shape; any other state goes the general way."""
+    from turboquant_amd.kv_cache import TurboQuantKVCache
+    from turboquant_amd.quantizer import ProdQuantized
+    cache = TurboQuantKVCache(128, key_bits=4, value_bits=2, device=torch.device("cpu"), dtype=torch.float32)
+
+    def u8(w):
+        return torch.zeros(1, 2, 5, w, dtype=torch.uint8)
+
+    def f32(*w):
+        return torch.zeros(1, 2, 5, *w)
+
+    keys, values = ProdQuantized(u8(64), u8(16), f32(), f32(), 3), ValueQuantized(u8(32), f32(4), f32(4), 2)
+
+    def plain(k=keys, v=values):
+        cache.key_quantized, cache.value_quantized = k, v
+        return cache._compressed_plain()
+
+    assert plain()
+    assert not plain(v=ValueQuantized(u8(64), f32(4), f32(4), 4))                     # another number of bits
+    assert not plain(v=values._replace(bits=4)) and not plain(v=values._replace(data=u8(16)))
+    assert not plain(k=keys._replace(mse_indices=u8(32)))                             # codes of a narrower quantiser
+    assert not plain(k=keys._replace(residual_norms=f32().half())) and not plain(k=keys._replace(norms=f32().half()))
+    assert not plain(k=keys._replace(residual_norms=torch.zeros(1, 1, 5)))            # (the general path lets it broadcast)
+    assert not plain(k=keys._replace(qjl_signs=u8(16)[:, :1])) and not plain(v=values._replace(zeros=f32(4).half()))
+    assert not plain(v=values._replace(scales=f32(1))) and not plain(v=values._replace(scales=f32(4).mT.contiguous().mT))
+    assert not plain(k=None) and not plain(v=None)

@@ -15,7 +15,7 @@ from typing import NamedTuple, Optional
 import torch
 
 from . import _ffi
-from .quantizer import ProdQuantized, TurboQuantProd
+from .quantizer import ProdQuantized, TurboQuantProd, _packing
 
 
 class ValueQuantized(NamedTuple):
@@ -139,10 +139,20 @@ class TurboQuantKVCache:
     # host time, at 4096 tokens of 8 heads of 128.  The entries below are three launches for the token, two for the scores and
     # two for the values: 85 us.
     def _compressed_plain(self) -> bool:
+        """Whether the compressed part is what this cache writes itself in fp32.  One put in its place may have other bits, 16-bit norms
+        or pieces that broadcast: the entries would read those wrongly, or read past them."""
         kq, vq = self.key_quantized, self.value_quantized
-        return (kq is not None and vq is not None and self.head_dim in (64, 128, 256) and self.value_group_size % 16 == 0
-                and kq.norms.dtype == torch.float32 and vq.scales.dtype == torch.float32 and kq.norms.dim() == 3
-                and all(type(t) is torch.Tensor and t.is_contiguous() for t in (*kq[:4], *vq[:3])))
+        d, bits, gs = self.head_dim, self.value_bits, self.value_group_size
+        if kq is None or vq is None or vq.bits != bits or d not in (64, 128, 256) or gs % 16 or kq.norms.dim() != 3:
+            return False
+        idx, signs, rnorms, norms = kq[:4]
+        data, scales, zeros = vq[:3]
+        n, groups = norms.numel(), d // gs
+        return (idx.dtype is signs.dtype is data.dtype is torch.uint8
+                and rnorms.dtype is norms.dtype is scales.dtype is zeros.dtype is torch.float32
+                and idx.numel() == n * (d * _packing(self.key_bits - 1)[0] // 8) and signs.numel() == n * (d // 8) and rnorms.numel() == n
+                and data.numel() == n * (d * bits // 8) and scales.numel() == zeros.numel() == n * groups
+                and all([type(t) is torch.Tensor and t.is_contiguous() for t in (idx, signs, rnorms, norms, data, scales, zeros)]))
 
     def _append_spill(self, key: torch.Tensor, value: torch.Tensor) -> bool:
         """One token into a full buffer whose first row leaves for the compressed part, in one library call; False: the case is
