@@ -607,6 +607,40 @@ def test_cache_token_in_few_launches(gpu, monkeypatch, d, B, H, prompt, buffer, 
             assert r1.shape == r2.shape and float((r1 - r2).norm()) <= 2e-6 * float(r2.norm())
 
 
+def test_cache_codes_at_any_byte(gpu):
+    """Code sections that begin one byte into a buffer take the general paths: same codes, and scores and values as from aligned ones
+    (inner products of codes bit for bit, the rest within fp32 sums in another order)."""
+    from turboquant_amd.kv_cache import TurboQuantKVCache
+    g = torch.Generator().manual_seed(2)
+    k, v = (torch.randn(1, 3, 302, 128, generator=g).to(gpu) for _ in range(2))
+    q = torch.randn(1, 3, 2, 128, generator=g).to(gpu)
+
+    def moved(t):
+        return torch.cat([t.flatten()[:1], t.flatten()])[1:].view(t.shape)
+
+    results = []
+    for odd in (False, True):
+        cache = TurboQuantKVCache(128, buffer_size=128, device=gpu, dtype=torch.float32)
+        cache.prefill(k[..., :300, :], v[..., :300, :])
+        out = []
+        for t in (300, 301):
+            if odd:
+                kq, vq = cache.key_quantized, cache.value_quantized
+                cache.key_quantized = kq._replace(mse_indices=moved(kq.mse_indices), qjl_signs=moved(kq.qjl_signs))
+                cache.value_quantized = vq._replace(data=moved(vq.data))
+                assert cache.value_quantized.data.data_ptr() % 2 == 1
+            scores = cache.attention_scores(q)
+            out += [scores, cache.attend(torch.softmax(scores, dim=-1))]
+            cache.append(k[..., t:t + 1, :], v[..., t:t + 1, :])
+            assert cache.seq_len == t + 1
+        results.append((cache, out))
+    (a, oa), (b, ob) = results
+    for x, y in zip((*a.key_quantized[:4], *a.value_quantized[:3]), (*b.key_quantized[:4], *b.value_quantized[:3])):
+        assert torch.equal(x, y)
+    for x, y in zip(oa, ob):
+        assert x.shape == y.shape and float((x - y).norm()) <= 2e-6 * float(y.norm())
+
+
 def test_cache_token_that_has_to_be_differentiated(gpu):
     """Weights and queries with a gradient take the general paths, through which torch differentiates."""
     from turboquant_amd.kv_cache import TurboQuantKVCache

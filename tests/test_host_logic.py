@@ -450,3 +450,29 @@ def test_a_compressed_part_put_in_by_hand_is_taken_as_it_is():
     assert not plain(k=keys._replace(qjl_signs=u8(16)[:, :1])) and not plain(v=values._replace(zeros=f32(4).half()))
     assert not plain(v=values._replace(scales=f32(1))) and not plain(v=values._replace(scales=f32(4).mT.contiguous().mT))
     assert not plain(k=None) and not plain(v=None)
+
+
+def test_cache_entries_refuse_what_they_cannot_index_before_any_launch():
+    """With TQ_EUNSUPPORTED, on which the cache object takes its general path: code sections off a word boundary, blocks of queries and
+    buffers beyond the entries' limits.  (The addresses are never read.)"""
+    lib = _ffi.lib()
+    ly = _ffi.TqLayer()
+    ly.d, ly.mse_bits = 128, 2
+    ly.Pi = ly.PiT = ly.S = ly.ST = ly.centroids = ly.thresholds = 4096
+    A = 4096
+
+    def append(sections=(A,) * 7, n_buf=128):
+        return lib.tq_cache_append(A, A, 128, 128, A, A, 0, n_buf * 128, 128, 0, n_buf * 128, 128, 8, 8, n_buf, C.byref(ly), 2, 32, 100,
+                                   *sections, *(A,) * 7, A, A, A, None)
+
+    def scores(idx=A, signs=A, n_q=1):
+        return lib.tq_cache_scores(A, 8, 8, n_q, idx, signs, A, A, 100, C.byref(ly), A, 0, 128 * 128, 128, 128, 0.1, A, A, None)
+
+    def attend(data=A, n_q=1):
+        return lib.tq_cache_attend(A, 8, 8, n_q, data, A, A, 100, 128, 32, 2, A, 0, 128 * 128, 128, 128, A, A, None)
+
+    for i in range(7):
+        assert append(tuple(A + (j == i) for j in range(7))) == _ffi.TQ_EUNSUPPORTED
+    assert append(n_buf=(1 << 20) + 1) == _ffi.TQ_EUNSUPPORTED
+    assert scores(idx=A + 1) == scores(signs=A + 2) == scores(n_q=(1 << 18) + 1) == _ffi.TQ_EUNSUPPORTED
+    assert attend(data=A + 1) == attend(n_q=65536) == _ffi.TQ_EUNSUPPORTED

@@ -923,6 +923,9 @@ extern "C" int tq_cache_append(const float* key, const float* value, int64_t key
   if (ks_r != d || vs_r != d || ks_h < d || vs_h < d) return TQ_EUNSUPPORTED;      // a buffer's rows lie one behind another
   if (batch != H && (ks_b != H * ks_h || vs_b != H * vs_h)) return TQ_EUNSUPPORTED;
   if (n_c > 0 && (!idx || !signs || !norms || !rnorms || !data || !scales || !zeros)) return TQ_ENULL;
+  // (sections are copied in words; keys and values arrive as fp32)
+  if (n_c > 0 && (((uintptr_t)idx | (uintptr_t)signs | (uintptr_t)norms | (uintptr_t)rnorms | (uintptr_t)data | (uintptr_t)scales | (uintptr_t)zeros) & 3))
+    return TQ_EUNSUPPORTED;
   const int ng = d / group_size, ib = idx_row_bytes(d, layer->mse_bits), sb = d / 8, db = d * value_bits / 8;
   // the codes of the rows that leave the buffer
   uintptr_t at = ((uintptr_t)work + 15) & ~(uintptr_t)15;

@@ -137,7 +137,8 @@ class TurboQuantKVCache:
     # ---- a decode token in fp32 (the general paths below take everything else) -----------------------------------------
     # A step of the general paths is some thirty small launches and seven concatenations of the whole history: 270 us, nearly all of it
     # host time, at 4096 tokens of 8 heads of 128.  The entries below are three launches for the token, two for the scores and
-    # two for the values: 85 us.
+    # two for the values: 85 us.  What an entry does not take (sections that are not word-aligned, buffers or blocks of queries
+    # beyond its indexes) it refuses before it launches anything, and the general path goes on.
     def _compressed_plain(self) -> bool:
         """Whether the compressed part is what this cache writes itself in fp32.  One put in its place may have other bits, 16-bit norms
         or pieces that broadcast: the entries would read those wrongly, or read past them."""
@@ -178,13 +179,16 @@ class TurboQuantKVCache:
                            dtype=torch.uint8, device=dev)
         idx, signs, rnorms, norms = grown[:4]
         with _ffi.on_device(dev):
-            _ffi.check(lib.tq_cache_append(
+            rc = lib.tq_cache_append(
                 key.data_ptr(), value.data_ptr(), key.stride(1), value.stride(1), kb.data_ptr(), vb.data_ptr(), *kb.stride()[:3],
                 *vb.stride()[:3], B * H, H, n_buf, C.byref(ly), self.value_bits, self.value_group_size, n_c,
                 kq.mse_indices.data_ptr(), kq.qjl_signs.data_ptr(), kq.norms.data_ptr(), kq.residual_norms.data_ptr(),
                 vq.data.data_ptr(), vq.scales.data_ptr(), vq.zeros.data_ptr(), idx.data_ptr(), signs.data_ptr(),
                 norms.data_ptr(), rnorms.data_ptr(), *[t.data_ptr() for t in grown[4:]], nk.data_ptr(), nv.data_ptr(),
-                work.data_ptr(), _ffi.stream_ptr(dev)), "tq_cache_append")
+                work.data_ptr(), _ffi.stream_ptr(dev))
+        if rc == _ffi.TQ_EUNSUPPORTED:
+            return False
+        _ffi.check(rc, "tq_cache_append")
         self.key_quantized = ProdQuantized(idx, signs, rnorms, norms, kq.mse_bits)
         self.value_quantized = ValueQuantized(*grown[4:], bits=self.value_bits)
         self.key_buffer, self.value_buffer = nk, nv
@@ -193,9 +197,11 @@ class TurboQuantKVCache:
     def append(self, key: torch.Tensor, value: torch.Tensor):
         """One decode token (batch, heads, 1, head_dim); the oldest buffered
         tokens spill into the compressed part once the buffer overflows."""
+        if not self._append_spill(key, value):
+            self._append(key, value)
         self.seq_len += 1
-        if self._append_spill(key, value):
-            return
+
+    def _append(self, key: torch.Tensor, value: torch.Tensor):
         if self.key_buffer is None:
             self.key_buffer, self.value_buffer = key, value
         else:
@@ -222,11 +228,13 @@ class TurboQuantKVCache:
                 scores = torch.empty(B, H, n_q, n_c + n_buf, dtype=torch.float32, device=dev)
                 work = torch.empty(2 * B * H * n_q * d, dtype=torch.float32, device=dev)
                 with _ffi.on_device(dev):
-                    _ffi.check(_ffi.lib().tq_cache_scores(
+                    rc = _ffi.lib().tq_cache_scores(
                         q.data_ptr(), B * H, H, n_q, kq.mse_indices.data_ptr(), kq.qjl_signs.data_ptr(), kq.norms.data_ptr(),
                         kq.residual_norms.data_ptr(), n_c, C.byref(ly), kb.data_ptr(), *kb.stride()[:3], n_buf, float(scale),
-                        scores.data_ptr(), work.data_ptr(), _ffi.stream_ptr(dev)), "tq_cache_scores")
-                return scores
+                        scores.data_ptr(), work.data_ptr(), _ffi.stream_ptr(dev))
+                if rc != _ffi.TQ_EUNSUPPORTED:
+                    _ffi.check(rc, "tq_cache_scores")
+                    return scores
         pieces = []
         if self.key_quantized is not None:
             pieces.append(self.key_quantizer.attention_score(query, self.key_quantized) * scale)
@@ -247,11 +255,13 @@ class TurboQuantKVCache:
                 out = torch.empty(B, H, n_q, d, dtype=torch.float32, device=dev)
                 work = torch.empty(lib.tq_cache_attend_bytes(B * H, n_q, d, n_c, n_buf) // 4, dtype=torch.float32, device=dev)
                 with _ffi.on_device(dev):
-                    _ffi.check(lib.tq_cache_attend(
+                    rc = lib.tq_cache_attend(
                         w.data_ptr(), B * H, H, n_q, vq.data.data_ptr(), vq.scales.data_ptr(), vq.zeros.data_ptr(), n_c, d,
                         self.value_group_size, self.value_bits, vb.data_ptr(), *vb.stride()[:3], n_buf, out.data_ptr(),
-                        work.data_ptr(), _ffi.stream_ptr(dev)), "tq_cache_attend")
-                return out
+                        work.data_ptr(), _ffi.stream_ptr(dev))
+                if rc != _ffi.TQ_EUNSUPPORTED:
+                    _ffi.check(rc, "tq_cache_attend")
+                    return out
         result = None
         col = 0
         if self.value_quantized is not None:
