@@ -476,3 +476,35 @@ def test_cache_entries_refuse_what_they_cannot_index_before_any_launch():
     assert append(n_buf=(1 << 20) + 1) == _ffi.TQ_EUNSUPPORTED
     assert scores(idx=A + 1) == scores(signs=A + 2) == scores(n_q=(1 << 18) + 1) == _ffi.TQ_EUNSUPPORTED
     assert attend(data=A + 1) == attend(n_q=65536) == _ffi.TQ_EUNSUPPORTED
+
+
+def _paper_pool(d, heads, key_bits=4, value_bits=4):
+    """A pool without memory: what the split rules read of one."""
+    from types import SimpleNamespace
+    from turboquant_amd.paged import PagedKVPool
+    pool = object.__new__(PagedKVPool)
+    pool.head_dim, pool.num_kv_heads, pool.value_bits, pool.value_group_size = d, heads, value_bits, 32
+    pool.dtype, pool.quantizer = torch.bfloat16, SimpleNamespace(bits=key_bits)
+    pool.page_kernel = lambda: 2 if d > 256 else 1
+    return pool
+
+
+@pytest.mark.parametrize("d,heads,Hq,B", [(128, 8, 32, 16), (256, 2, 16, 4), (576, 1, 8, 3), (576, 1, 64, 1), (512, 2, 40, 5), (192, 1, 4, 7)])
+def test_a_step_never_leaves_the_workspace_it_is_given(d, heads, Hq, B):
+    """A split count of our own is cut to what the workspace holds, a caller's count that does not fit is refused."""
+    pool = _paper_pool(d, heads)
+    need = _ffi.lib().tq_decode_workspace_bytes
+    for held in (1, 2, 7, 64):
+        for spare in (0, 4, 400):
+            ws = torch.empty(need(B, Hq, d, held) // 4 + spare // 4, dtype=torch.float32, device="meta")
+            for n in (1, held, held + 1, 3 * held, 500):
+                got = pool._splits_within(ws, B, Hq, n, True)
+                assert 1 <= got <= n and need(B, Hq, d, got) <= 4 * ws.numel() and (got == n or need(B, Hq, d, got + 1) > 4 * ws.numel())
+                if need(B, Hq, d, n) <= 4 * ws.numel():
+                    assert pool._splits_within(ws, B, Hq, n, False) == n
+                else:
+                    with pytest.raises(ValueError, match="workspace"):
+                        pool._splits_within(ws, B, Hq, n, False)
+    small = torch.empty(need(B, Hq, d, 1) // 4 - 1, dtype=torch.float32, device="meta")
+    with pytest.raises(ValueError, match="workspace"):
+        pool._splits_within(small, B, Hq, 1, True)

@@ -242,6 +242,18 @@ class PagedKVPool:
         nbytes = _ffi.lib().tq_decode_workspace_bytes(B, Hq, self.head_dim, n_split)
         return torch.empty(nbytes // 4, dtype=torch.float32, device=self.device)
 
+    def _splits_within(self, workspace: torch.Tensor, B: int, Hq: int, n_split: int, ours: bool) -> int:
+        """The split count of a step in a caller's workspace.  A count of our own choice is cut to what the workspace holds (it may
+        be sized for fewer splits); one that the caller asks for has to fit."""
+        need = _ffi.lib().tq_decode_workspace_bytes
+        have, want = workspace.numel() * workspace.element_size(), need(B, Hq, self.head_dim, n_split)
+        if want <= have:
+            return n_split
+        least = need(B, Hq, self.head_dim, 1)
+        if ours and least <= have:
+            return 1 + (have - least) // (need(B, Hq, self.head_dim, 2) - least)
+        raise ValueError(f"the workspace holds {have} bytes, {B} x {Hq} query heads in {n_split} splits take {want}")
+
     def decode_attention(self, query: torch.Tensor, block_table: torch.Tensor, seq_lens: torch.Tensor,
                          scale: Optional[float] = None, recent_k: Optional[torch.Tensor] = None,
                          recent_v: Optional[torch.Tensor] = None, recent_len: Optional[torch.Tensor] = None,
@@ -253,7 +265,8 @@ class PagedKVPool:
         block_table (B, max_pages) or (max_pages,) shared; seq_lens (B,) int32;
         recent_k / recent_v (B, R, H, d) exact tokens, recent_len (B,) valid rows.
         `stages` (bit 0 query rotation, bit 1 page kernel, bit 2 merge) exists for
-        timing the stages apart; 7 runs the whole thing.  `static_scratch` runs the library's entry
+        timing the stages apart; 7 runs the whole thing.  A caller's `workspace` has to hold `n_split` splits
+        (`workspace()`); with the count left to us we take as many as it holds.  `static_scratch` runs the library's entry
         point that allocates nothing (tq_decode_attn_paged_noalloc): no workspace tensor, the partials live
         in a fixed device array inside the library (16 MiB; larger calls raise), shared by all calls on
         this GPU - pass `out` as well and the call touches no allocator at all."""
@@ -267,8 +280,8 @@ class PagedKVPool:
         bt = block_table.contiguous()
         bt_stride = -bt.shape[0] if bt.dim() == 1 else bt.shape[1]      # negative: one shared row of that length
         seq_lens = seq_lens.to(device=self.device, dtype=torch.int32).contiguous()
-        by_length = False
-        if n_split is None:
+        by_length, ours = False, n_split is None
+        if ours:
             if max_len is None:
                 max_len = (bt.shape[-1]) * PAGE_TOKENS
             n_split = self.default_splits(B, max_len, Hq, static_scratch)
@@ -278,6 +291,8 @@ class PagedKVPool:
                 raise ValueError("static_scratch takes no workspace and runs all stages")
         elif workspace is None:
             workspace = self.workspace(B, Hq, -n_split if by_length else n_split)
+        else:
+            n_split = self._splits_within(workspace, B, Hq, n_split, ours)
         if out is None:
             out = torch.empty_like(query)
         rk_ptr = rv_ptr = rl_ptr = None
@@ -351,14 +366,16 @@ class PagedKVPool:
         bt = block_table.contiguous()
         bt_stride = -bt.shape[0] if bt.dim() == 1 else bt.shape[1]      # negative: one shared row of that length
         seq_lens = seq_lens.to(device=self.device, dtype=torch.int32).contiguous()
-        by_length = False
-        if n_split is None:
+        by_length, ours = False, n_split is None
+        if ours:
             if max_len is None:
                 max_len = (bt.shape[-1]) * PAGE_TOKENS
             n_split = self.default_splits(B, max_len, Hq)
             by_length = workspace is None and self._shares_by_length(B, Hq)
         if workspace is None:
             workspace = self.workspace(B, Hq, -n_split if by_length else n_split)
+        else:
+            n_split = self._splits_within(workspace, B, Hq, n_split, ours)
         if out is None:
             out = torch.empty_like(query)
         ly = self.quantizer._layer()
