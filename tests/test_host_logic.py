@@ -508,3 +508,20 @@ def test_a_step_never_leaves_the_workspace_it_is_given(d, heads, Hq, B):
     small = torch.empty(need(B, Hq, d, 1) // 4 - 1, dtype=torch.float32, device="meta")
     with pytest.raises(ValueError, match="workspace"):
         pool._splits_within(small, B, Hq, 1, True)
+
+
+def test_short_contexts_of_many_heads_are_split_by_turns():
+    """The kernel of sixteen heads per wavefront: a workgroup per turn of its loop in short contexts, about four turns each in long ones,
+    never more workgroups than compute units (unless sequences alone are more), no split without tokens."""
+    pool = _paper_pool(576, 1)
+    for G, side in ((9, 3), (16, 3), (17, 2), (33, 1), (64, 1), (65, 1), (128, 1)):
+        groups = -(-G // 64)
+        for B in (2, 3, 16, 300):
+            most = max(1, 256 // (B * groups))
+            for N in (1, 31, 200, 500, 2000, 8192, 32768, 131072):
+                n, turns = pool.default_splits(B, N, G), -(-N // (32 * side))
+                each = -(-turns // n)
+                assert 1 <= n <= min(most, turns) and (n - 1) * each < turns <= n * each
+                assert each == 1 or (turns > most or turns > 40 * side) and (each <= 4 or -(-turns // most) == each)
+    assert [pool.default_splits(1, N, 16) for N in (1, 500, 8192, 65536)] == [1, 3, 64, 128]
+    assert pool.default_splits(1, 500, 8) == 1 and pool.default_splits(1, 8192, 64) == 64

@@ -193,10 +193,28 @@ class PagedKVPool:
         return max(1, Hq // self.num_kv_heads) <= 128       # (more than 8 heads per KV head: groups of at most 8)
 
     def _head_tiles_shape(self, Hq: int) -> bool:
-        """Whether a step runs the kernel of sixteen heads per wavefront (head_dim 512 / 576 with more than 8 query heads per
-        KV head); only the split heuristic depends on it."""
+        """Whether a step has more than 8 query heads on a KV head of 512 / 576; only the split heuristic depends on it."""
         return (self.head_dim in (512, 576) and self.quantizer.bits in (3, 4) and self.value_bits in (2, 4) and
                 8 < Hq // self.num_kv_heads <= 128 and self.page_kernel() == 2)
+
+    @staticmethod
+    def _head_tile_splits(pairs: int, max_len: int, heads: int) -> int:
+        """Split count of such a step: `pairs` sequences x KV heads, `heads` query heads on each."""
+        tiles = (heads + 15) // 16
+        if tiles == 1 and pairs == 1:
+            # the kernel of 8 heads per workgroup: two groups, four blocks of 32 tokens each (16 heads: 1 x 500 44 us with one split,
+            # 26 with 4; 1 x 8192 44 with 16, 33 with 64; 1 x 32768 51 with 64, 47 with 128, 64 with 192)
+            return max(1, min(128, max_len // 128))
+        # Up to four tiles of sixteen heads on the same pages (with two, two blocks of 32 tokens side by side, with one, three); one workgroup
+        # per compute unit.  A short context is a chain of turns (3.3 us each): up to 40 blocks side by side in the grid a workgroup takes one turn;
+        # beyond, four, as the merge reads every split (576, 4-bit: 64 heads 1 x 200 47 us with one split, 30 with 4; 128 heads
+        # 1 x 8192 80 with 16, 51 with 64; 16 heads 4 x 1024 53 with 2, 30 with 11; 4 x 8192 55 with 16, 42 with 64;
+        # 128 heads 16 x 8192 167 with 8, 176 with 16, 260 with 4)
+        groups, side = ((tiles + 3) // 4, 1) if tiles >= 3 else (1, 4 - tiles)
+        turns = max(1, (max_len + 32 * side - 1) // (32 * side))
+        n = min(max(1, 256 // (pairs * groups)), max(min(turns, 40 * side), (turns + 3) // 4), 512)
+        each = (turns + n - 1) // n                     # (whole turns: a split without tokens is written and merged too)
+        return (turns + each - 1) // each
 
     def default_splits(self, B: int, max_len: int, Hq: Optional[int] = None, static_scratch: bool = False) -> int:
         """Split count of the page-streaming kernel.  Matrix-core kernel: its workgroups (4 wavefronts,
@@ -206,13 +224,7 @@ class PagedKVPool:
         with at least one 256-token chunk."""
         pairs = max(1, B * self.num_kv_heads)
         if Hq is not None and self._head_tiles_shape(Hq) and not static_scratch:
-            # sixteen query heads per pair of wavefronts, up to four such tiles on the same pages (with two, two blocks of 32
-            # tokens side by side, with one, three): one workgroup per compute unit, at least four turns of its loop
-            # (128 heads of 576: 1 x 8192 56.9 us with 32 splits, 50.8 with 64; 16 x 8192 182 with 8, 192 with 16, 284 with 4)
-            tiles = (Hq // self.num_kv_heads + 15) // 16
-            groups, side = ((tiles + 3) // 4, 1) if tiles >= 3 else (1, 4 - tiles)
-            turns = max(1, (max_len + 32 * side - 1) // (32 * side))
-            return int(max(1, min(max(1, 256 // (pairs * groups)), max(1, turns // 4), 512)))
+            return self._head_tile_splits(pairs, max_len, Hq // self.num_kv_heads)
         if self.head_dim > 256 and self.page_kernel() == 2:
             # head sizes above 256: one workgroup per compute unit, a block of 32 tokens at a time; each workgroup
             # first packs its query operands, so it should have at least 16 blocks
