@@ -525,3 +525,14 @@ def test_short_contexts_of_many_heads_are_split_by_turns():
                 assert each == 1 or (turns > most or turns > 40 * side) and (each <= 4 or -(-turns // most) == each)
     assert [pool.default_splits(1, N, 16) for N in (1, 500, 8192, 65536)] == [1, 3, 64, 128]
     assert pool.default_splits(1, 500, 8) == 1 and pool.default_splits(1, 8192, 64) == 64
+
+
+@pytest.mark.parametrize("d", [64, 128, 256, 320, 512, 576])
+def test_a_split_count_without_query_heads_bounds_those_with_any(d):
+    """So that a workspace sized before the query heads are known holds a step at full speed."""
+    for heads in (1, 2, 8):
+        pool = _paper_pool(d, heads)
+        for B in (1, 2, 3, 17, 64, 300):
+            for N in (1, 90, 500, 3000, 8192, 20000, 32768, 131072):
+                most = pool.default_splits(B, N)
+                assert all(pool.default_splits(B, N, heads * per) <= most for per in (*range(1, 20), 24, 32, 33, 48, 64, 65, 80, 128))

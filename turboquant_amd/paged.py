@@ -192,10 +192,11 @@ class PagedKVPool:
             return True
         return max(1, Hq // self.num_kv_heads) <= 128       # (more than 8 heads per KV head: groups of at most 8)
 
-    def _head_tiles_shape(self, Hq: int) -> bool:
-        """Whether a step has more than 8 query heads on a KV head of 512 / 576; only the split heuristic depends on it."""
+    def _head_tiles_shape(self, Hq: Optional[int]) -> bool:
+        """Whether a step has more than 8 query heads on a KV head of 512 / 576 (Hq None: whether there are such steps); only the
+        split heuristic depends on it."""
         return (self.head_dim in (512, 576) and self.quantizer.bits in (3, 4) and self.value_bits in (2, 4) and
-                8 < Hq // self.num_kv_heads <= 128 and self.page_kernel() == 2)
+                (Hq is None or 8 < Hq // self.num_kv_heads <= 128) and self.page_kernel() == 2)
 
     @staticmethod
     def _head_tile_splits(pairs: int, max_len: int, heads: int) -> int:
@@ -221,8 +222,11 @@ class PagedKVPool:
         one per SIMD, each walking 64-token blocks) should number about two per CU (256 CUs) while every
         wavefront still gets several blocks, because each wavefront first builds its query operands.
         General kernel: it hides its memory latency by occupancy, so about eight workgroups per CU, each
-        with at least one 256-token chunk."""
+        with at least one 256-token chunk.  Without Hq: no fewer than with any."""
         pairs = max(1, B * self.num_kv_heads)
+        if Hq is None and not static_scratch and self._head_tiles_shape(None):
+            return max(self.default_splits(B, max_len, self.num_kv_heads),
+                       *(self._head_tile_splits(pairs, max_len, heads) for heads in (16, 32, 64)))
         if Hq is not None and self._head_tiles_shape(Hq) and not static_scratch:
             return self._head_tile_splits(pairs, max_len, Hq // self.num_kv_heads)
         if self.head_dim > 256 and self.page_kernel() == 2:
