@@ -656,6 +656,24 @@ def test_cache_token_that_has_to_be_differentiated(gpu):
     assert torch.allclose(out, cache.attend(torch.softmax(scores, dim=-1).detach()), rtol=1e-4, atol=1e-5)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_cache_products_under_autocast(gpu, dtype):
+    """Scores and values have the type, and the rounding, that autocast gives the products of the general paths."""
+    from turboquant_amd import kv_cache as KC
+    g = torch.Generator().manual_seed(4)
+    k, v = (torch.randn(1, 2, 300, 128, generator=g).to(gpu) for _ in range(2))
+    cache = KC.TurboQuantKVCache(128, buffer_size=128, device=gpu, dtype=torch.float32)
+    cache.prefill(k, v)
+    q = torch.randn(1, 2, 1, 128, generator=g).to(gpu)
+    w = torch.softmax(torch.randn(1, 2, 1, 300, generator=g), dim=-1).to(gpu)
+    with torch.autocast("cuda", dtype=dtype):
+        scores, out = cache.attention_scores(q), cache.attend(w)
+        tail = torch.matmul(q, cache.key_buffer.transpose(-2, -1).contiguous()) * (1 / 128 ** 0.5)
+        want = torch.matmul(w[..., :172], KC.dequantize_values(cache.value_quantized)) + torch.matmul(w[..., 172:], cache.value_buffer)
+    assert out.dtype == want.dtype == dtype and torch.equal(out, want)
+    assert torch.equal(scores[..., 172:], tail.to(scores.dtype))
+
+
 # ------------------------------------------------------------------ inner products and flat codes of small calls
 @pytest.mark.parametrize("d,bits,lead,n_k,n_q,dtype", [
     (64, 2, (), 1, 1, torch.float32), (128, 3, (2,), 63, 16, torch.bfloat16), (128, 5, (1, 3), 65, 17, torch.float32),

@@ -81,6 +81,11 @@ def _plain(*tensors) -> bool:
     return _ffi.ordinary(*tensors) and all(t.dtype == torch.float32 and t.dim() == 4 and t.stride(-1) == 1 for t in tensors)
 
 
+def _plain_product(*tensors) -> bool:
+    """... and a product of them in fp32 (under autocast it is one of 16-bit numbers)."""
+    return _plain(*tensors) and not torch.is_autocast_enabled("cuda")
+
+
 class TurboQuantKVCache:
     """Self-contained cache: the newest `buffer_size` tokens stay exact, older
     ones are TurboQuant keys + group-quantised values.  Tensors are
@@ -218,7 +223,7 @@ class TurboQuantKVCache:
         if scale is None:
             scale = 1.0 / math.sqrt(self.head_dim)
         kb = self.key_buffer
-        if kb is not None and isinstance(scale, (int, float)) and self._compressed_plain() and _plain(query, kb):
+        if kb is not None and isinstance(scale, (int, float)) and self._compressed_plain() and _plain_product(query, kb):
             kq = self.key_quantized
             B, H, n_buf, d = kb.shape
             n_c, n_q = kq.norms.shape[-1], query.shape[2]
@@ -239,13 +244,16 @@ class TurboQuantKVCache:
         if self.key_quantized is not None:
             pieces.append(self.key_quantizer.attention_score(query, self.key_quantized) * scale)
         if self.key_buffer is not None:
-            pieces.append(torch.matmul(query, self.key_buffer.transpose(-2, -1)) * scale)
+            kt = self.key_buffer.transpose(-2, -1)
+            if kt.dtype == torch.bfloat16 or torch.is_autocast_enabled("cuda"):
+                kt = kt.contiguous()         # (batched bf16 products with a transposed right operand have faulted in the library)
+            pieces.append(torch.matmul(query, kt) * scale)
         return torch.cat(pieces, dim=-1)
 
     def attend(self, attn_weights: torch.Tensor) -> torch.Tensor:
         """softmaxed weights (batch, heads, n_q, seq_len) -> (batch, heads, n_q, head_dim)."""
         vb = self.value_buffer
-        if vb is not None and self._compressed_plain() and _plain(attn_weights, vb):
+        if vb is not None and self._compressed_plain() and _plain_product(attn_weights, vb):
             vq = self.value_quantized
             B, H, n_buf, d = vb.shape
             n_c, n_q = vq.data.shape[-2], attn_weights.shape[2]
