@@ -656,6 +656,67 @@ def test_cache_token_that_has_to_be_differentiated(gpu):
     assert torch.allclose(out, cache.attend(torch.softmax(scores, dim=-1).detach()), rtol=1e-4, atol=1e-5)
 
 
+class _Counted:
+    """The library, counting the calls of each entry that it answered."""
+    def __init__(self, lib):
+        self._lib, self.answered = lib, {}
+
+    def __getattr__(self, name):
+        entry = getattr(self._lib, name)
+
+        def call(*args):
+            rc = entry(*args)
+            if rc == 0:
+                self.answered[name] = self.answered.get(name, 0) + 1
+            return rc
+        return call
+
+    def take(self, name):
+        return self.answered.pop(name, 0)
+
+
+@pytest.fixture
+def counted(monkeypatch):
+    from turboquant_amd import _ffi
+    lib = _Counted(_ffi.lib())
+    monkeypatch.setattr(_ffi, "lib", lambda: lib)
+    return lib
+
+
+@pytest.mark.parametrize("d,H,n_c,n_buf,vb", [(64, 8, 1000, 128, 2), (128, 8, 300, 128, 4), (256, 3, 2000, 33, 2)])
+def test_cache_blocks_of_queries_on_either_side_of_the_limit(gpu, counted, d, H, n_c, n_buf, vb):
+    """The largest block of queries that takes the entry, and the next one, which takes the general path: results as from products in fp64
+    of what the cache holds (fp32 sums, 2e-6 of the norm), and scratch that stays small."""
+    from turboquant_amd import kv_cache as KC
+    g = torch.Generator().manual_seed(d)
+    k, v = (torch.randn(1, H, n_c + n_buf, d, generator=g).to(gpu) for _ in range(2))
+    cache = KC.TurboQuantKVCache(d, value_bits=vb, buffer_size=n_buf, device=gpu, dtype=torch.float32)
+    cache.prefill(k, v)
+    keys = torch.cat([cache.key_quantizer.dequantize(cache.key_quantized), cache.key_buffer], dim=2).double()
+    values = torch.cat([KC.dequantize_values(cache.value_quantized), cache.value_buffer], dim=2).double()
+
+    def last(few):
+        lo, hi = 1, 1 << 16
+        while hi - lo > 1:
+            mid = (lo + hi) // 2
+            lo, hi = (mid, hi) if few(H * mid, n_c, n_buf, d) else (lo, mid)
+        return lo
+
+    most = last(KC.TurboQuantKVCache._few_score_queries)
+    for n_q in (most, most + 1):
+        q = torch.randn(1, H, n_q, d, generator=g).to(gpu)
+        got, want = cache.attention_scores(q), torch.matmul(q.double(), keys.transpose(-2, -1).contiguous()) / d ** 0.5
+        assert counted.take("tq_cache_scores") == (n_q == most)
+        assert float((got - want).norm()) <= 2e-6 * float(want.norm())
+    most = last(KC.TurboQuantKVCache._few_value_queries)
+    assert counted._lib.tq_cache_attend_bytes(H, most, d, n_c, n_buf) <= 32 << 20
+    for n_q in (most, most + 1):
+        w = torch.softmax(torch.randn(1, H, n_q, n_c + n_buf, generator=g), dim=-1).to(gpu)
+        got, want = cache.attend(w), torch.matmul(w.double(), values)
+        assert counted.take("tq_cache_attend") == (n_q == most)
+        assert float((got - want).norm()) <= 2e-6 * float(want.norm())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_cache_products_under_autocast(gpu, dtype):
     """Scores and values have the type, and the rounding, that autocast gives the products of the general paths."""

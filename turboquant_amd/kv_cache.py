@@ -199,6 +199,23 @@ class TurboQuantKVCache:
         self.key_buffer, self.value_buffer = nk, nv
         return True
 
+    # The entries are made for the few queries of a decode step; a block of queries is two matrix products in the general paths.
+    # us of a call, entry / general, buffers of 128 rows:
+    #   scores: a wavefront per exact row and query, which pays while the host time of the general path or its passes over the scores of
+    #   the compressed keys cost more. 8 heads of 128, 100 keys: 256 queries 35 / 63, 1024 202 / 61; 32 heads of 4096 keys: 32 queries 66 / 73,
+    #   128 206 / 199; 32 heads of 64, 1000 keys: 64 queries 43 / 68, 128 83 / 68; 2 heads of 256, 4096 keys: 256 queries 63 / 96,
+    #   1024 211 / 177; 8 heads of 128, 32768 keys: 128 queries 266 / 377, 2048 3953 / 5512.
+    @staticmethod
+    def _few_score_queries(rows: int, n_c: int, n_buf: int, d: int) -> bool:
+        return rows * (n_buf * max(48, d // 2) - n_c) <= 1 << 24
+
+    #   values: every query unpacks the history again and writes a partial per 128 tokens (within the limit 21 MB of them). 8 heads of 128, 4096 tokens:
+    #   48 queries 45 / 61, 128 99 / 61, 2048 1365 / 155; 32 heads: 16 queries 58 / 62, 24 84 / 62; 8 heads, 32768 tokens: 12 queries 80 / 96,
+    #   24 141 / 130; 8 heads of 64, 4096 tokens: 64 queries 42 / 64, 128 74 / 64; of 128, 100 tokens: 256 queries 31 / 64, 1024 96 / 60.
+    @staticmethod
+    def _few_value_queries(rows: int, n_c: int, n_buf: int, d: int) -> bool:
+        return rows * (d + 32) * (n_c + 4 * n_buf) * 32768 <= (5 << 26) * (32768 + n_c)
+
     def append(self, key: torch.Tensor, value: torch.Tensor):
         """One decode token (batch, heads, 1, head_dim); the oldest buffered
         tokens spill into the compressed part once the buffer overflows."""
@@ -228,7 +245,8 @@ class TurboQuantKVCache:
             B, H, n_buf, d = kb.shape
             n_c, n_q = kq.norms.shape[-1], query.shape[2]
             if (query.shape == (B, H, n_q, self.head_dim) and d == self.head_dim and tuple(kq.norms.shape) == (B, H, n_c)
-                    and n_c and n_buf and n_q and B * H <= 65535 and kq.norms.device == kb.device):
+                    and n_c and n_buf and n_q and B * H <= 65535 and kq.norms.device == kb.device
+                    and self._few_score_queries(B * H * n_q, n_c, n_buf, d)):
                 q, ly, dev = query.contiguous(), self.key_quantizer._layer(), kb.device
                 scores = torch.empty(B, H, n_q, n_c + n_buf, dtype=torch.float32, device=dev)
                 work = torch.empty(2 * B * H * n_q * d, dtype=torch.float32, device=dev)
@@ -258,7 +276,8 @@ class TurboQuantKVCache:
             B, H, n_buf, d = vb.shape
             n_c, n_q = vq.data.shape[-2], attn_weights.shape[2]
             if (attn_weights.shape == (B, H, n_q, n_c + n_buf) and d == self.head_dim and tuple(vq.scales.shape[:3]) == (B, H, n_c)
-                    and n_c and n_buf and 0 < n_q <= 65535 and B * H <= 65535 and vq.scales.device == vb.device):
+                    and n_c and n_buf and 0 < n_q <= 65535 and B * H <= 65535 and vq.scales.device == vb.device
+                    and self._few_value_queries(B * H * n_q, n_c, n_buf, d)):
                 w, dev, lib = attn_weights.contiguous(), vb.device, _ffi.lib()
                 out = torch.empty(B, H, n_q, d, dtype=torch.float32, device=dev)
                 work = torch.empty(lib.tq_cache_attend_bytes(B * H, n_q, d, n_c, n_buf) // 4, dtype=torch.float32, device=dev)
