@@ -735,6 +735,28 @@ def test_cache_products_under_autocast(gpu, dtype):
     assert torch.equal(scores[..., 172:], tail.to(scores.dtype))
 
 
+def test_cache_and_ring_of_tensors_that_are_negated_lazily(gpu):
+    """A tensor whose sign torch keeps beside its memory (the imaginary part of a conjugate) is read with that sign."""
+    from turboquant_amd.capture import RingBuffer
+    from turboquant_amd.kv_cache import TurboQuantKVCache
+    g = torch.Generator().manual_seed(6)
+    k, v = (torch.randn(1, 2, 302, 128, generator=g).to(gpu) for _ in range(2))
+    q = torch.randn(1, 2, 1, 128, generator=g).to(gpu)
+    results = []
+    for lazy in (False, True):
+        neg = torch._neg_view if lazy else torch.neg
+        cache = TurboQuantKVCache(128, buffer_size=128, device=gpu, dtype=torch.float32)
+        cache.prefill(k[..., :300, :], v[..., :300, :])
+        for t in (300, 301):
+            cache.append(neg(k[..., t:t + 1, :]), neg(v[..., t:t + 1, :]))
+        w = torch.softmax(cache.attention_scores(q), dim=-1)
+        ring = RingBuffer(4, 2, 128, device=gpu, dtype=torch.float32)
+        ring.write(neg(k[0, :, 0]).view(1, 2, 128), neg(v[0, :, 0]).view(1, 2, 128), 1)
+        results.append((cache.key_buffer, cache.value_buffer, cache.attention_scores(q), cache.attend(neg(w)), *ring.peek()))
+    for a, b in zip(*results):
+        assert a.shape == b.shape and float((a - b).norm()) <= 2e-6 * float(a.norm())
+
+
 # ------------------------------------------------------------------ inner products and flat codes of small calls
 @pytest.mark.parametrize("d,bits,lead,n_k,n_q,dtype", [
     (64, 2, (), 1, 1, torch.float32), (128, 3, (2,), 63, 16, torch.bfloat16), (128, 5, (1, 3), 65, 17, torch.float32),

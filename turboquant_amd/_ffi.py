@@ -170,6 +170,8 @@ def ordinary(*tensors) -> bool:
     for t in tensors:
         if type(t) is not torch.Tensor or not t.is_cuda or (grad and t.requires_grad) or t.device != tensors[0].device:
             return False
+        if t.is_neg() or t._is_zerotensor():             # (its memory does not hold its values)
+            return False
     return True
 
 
