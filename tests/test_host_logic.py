@@ -536,3 +536,20 @@ def test_a_split_count_without_query_heads_bounds_those_with_any(d):
             for N in (1, 90, 500, 3000, 8192, 20000, 32768, 131072):
                 most = pool.default_splits(B, N)
                 assert all(pool.default_splits(B, N, heads * per) <= most for per in (*range(1, 20), 24, 32, 33, 48, 64, 65, 80, 128))
+
+
+def test_splits_of_many_heads_in_the_static_area():
+    """Steps of more than 8 heads on a wide KV head take the split count of their kernel there too, cut to what the area holds."""
+    for d in (512, 576):
+        pool = _paper_pool(d, 1)
+        ly = _ffi.TqLayer()
+        ly.d, ly.mse_bits = d, 3
+        pool.quantizer._layer = lambda: ly
+        need = lambda B, Hq, n: _ffi.lib().tq_decode_noalloc_bytes(B, Hq, 1, n, C.byref(ly))
+        for Hq in (9, 16, 17, 64, 65, 128):
+            for B in (1, 2, 3, 8, 64):
+                for N in (1, 500, 8192, 131072):
+                    n, free = pool.default_splits(B, N, Hq, True), pool.default_splits(B, N, Hq)
+                    assert n == free or 1 <= n < free and need(B, Hq, n + 1) > _ffi.NOALLOC_SCRATCH_BYTES
+                    assert n == 1 or need(B, Hq, n) <= _ffi.NOALLOC_SCRATCH_BYTES
+        assert pool.default_splits(1, 8192, 128, True) >= 32

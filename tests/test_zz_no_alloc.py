@@ -72,6 +72,27 @@ def test_static_scratch_decode_equals_the_workspace_form_on_consecutive_calls(gp
     assert torch.equal(out, ref)
 
 
+@pytest.mark.parametrize("Hq,B,N", [(16, 1, 3000), (64, 1, 8192), (128, 1, 8192), (128, 2, 1000)])
+def test_static_scratch_decode_of_many_heads_chooses_its_splits(gpu, Hq, B, N):
+    """More than 8 heads on a KV head of 576, the split count left to the pool: as the workspace form with that count, bit for bit, at
+    two lengths behind one another."""
+    g = torch.Generator().manual_seed(Hq + N)
+    pages = (N + 15) // 16
+    pool, tq = _pool(gpu, 576, 4, 4, 1, B * pages)
+    table = torch.randperm(B * pages, generator=g).to(torch.int32).view(B, pages).to(gpu)
+    for b in range(B):
+        kv = torch.randn(1, N, 1, 576, generator=g).bfloat16().to(gpu)
+        pool.append(kv, kv.flip(1), table[b:b + 1])
+    q = torch.randn(B, Hq, 576, generator=g).bfloat16().to(gpu)
+    for n in (N, N // 2 + 1):
+        seq = torch.full((B,), n, dtype=torch.int32, device=gpu)
+        out = torch.full_like(q, float("nan"))
+        pool.decode_attention(q, table, seq, out=out, max_len=n, static_scratch=True)
+        ref = pool.decode_attention(q, table, seq, n_split=pool.default_splits(B, n, Hq, True))
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref) and not torch.isnan(out.float()).any()
+
+
 def test_static_scratch_decode_rejects_what_does_not_fit(gpu):
     """A call whose partials exceed the static area (16 MiB) is refused with TQ_ETOOBIG before anything is
     launched; bad arguments are refused as in the workspace form."""

@@ -18,6 +18,7 @@ TQ_PAGE_TOKENS = 16
 TQ_MAX_TERMS = 15
 ABI_VERSION = 2
 TQ_EUNSUPPORTED = -2
+NOALLOC_SCRATCH_BYTES = 16 << 20      # TQ_NOALLOC_SCRATCH_BYTES
 
 # TQ_HIP_LIBRARY overrides the in-tree library (e.g. to compare two builds)
 _LIB_PATH = os.environ.get("TQ_HIP_LIBRARY") or os.path.join(os.path.dirname(os.path.abspath(__file__)), "libtq_hip.so")

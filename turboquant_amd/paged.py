@@ -227,8 +227,9 @@ class PagedKVPool:
         if Hq is None and not static_scratch and self._head_tiles_shape(None):
             return max(self.default_splits(B, max_len, self.num_kv_heads),
                        *(self._head_tile_splits(pairs, max_len, heads) for heads in (16, 32, 64)))
-        if Hq is not None and self._head_tiles_shape(Hq) and not static_scratch:
-            return self._head_tile_splits(pairs, max_len, Hq // self.num_kv_heads)
+        if Hq is not None and self._head_tiles_shape(Hq):
+            n = self._head_tile_splits(pairs, max_len, Hq // self.num_kv_heads)
+            return self._splits_in_static_scratch(B, Hq, n) if static_scratch else n
         if self.head_dim > 256 and self.page_kernel() == 2:
             # head sizes above 256: one workgroup per compute unit, a block of 32 tokens at a time; each workgroup
             # first packs its query operands, so it should have at least 16 blocks
@@ -247,6 +248,12 @@ class PagedKVPool:
         want = max(1, 512 // pairs)
         longest = max(1, blocks // 16)          # keep >= 4 blocks per wavefront
         return int(max(1, min(want, longest, 512)))
+
+    def _splits_in_static_scratch(self, B: int, Hq: int, n_split: int) -> int:
+        """n_split, or as many as the library's static area holds (with one that does not fit the call itself is refused)."""
+        ly = self.quantizer._layer()
+        one, two = (_ffi.lib().tq_decode_noalloc_bytes(B, Hq, self.num_kv_heads, n, C.byref(ly)) for n in (1, 2))
+        return max(1, min(n_split, 1 + (_ffi.NOALLOC_SCRATCH_BYTES - one) // (two - one)))
 
     def _shares_by_length(self, B: int, Hq: int) -> bool:
         """Whether the library deals a step's workgroups out by length (matrix-core kernel, several sequences, at most 1024);
