@@ -198,11 +198,11 @@ int tq_rotate_query(const void *q, int dtype, int64_t rows, const tq_layer *laye
  * than one batch, s_b = H s_h; else TQ_EUNSUPPORTED, as for sections off a 4-byte boundary and for n_c or n_buf above 2^20.
  * n_c may be 0 (the sections are not read then).  work: tq_cache_append_bytes bytes.
  * tq_cache_scores (kv_cache.py:247-284): scores (batch, n_q, n_c + n_buf) = scale * <q, k> over the compressed keys, then the
- * exact ones; n_c, n_buf > 0.  TQ_EUNSUPPORTED: codes off a 4-byte boundary, n_q above 2^18, n_c above 2^28.  work: 2 * batch * n_q * d
- * floats.
+ * exact ones; n_c, n_buf > 0.  TQ_EUNSUPPORTED: codes off a 4-byte boundary, n_q above 2^18, n_c above 2^28, n_buf above 2^24.  work:
+ * 2 * batch * n_q * d floats.
  * tq_cache_attend (kv_cache.py:286-321): out (batch, n_q, d) = weights (batch, n_q, n_c + n_buf) times the values.
- * TQ_EUNSUPPORTED: codes off a 4-byte boundary, group sizes that are not a multiple of 16, n_q above 65535, n_c above 2^28.  work:
- * tq_cache_attend_bytes bytes.                                                                              */
+ * TQ_EUNSUPPORTED: codes off a 4-byte boundary, group sizes that are not a multiple of 16, n_q above 65535, n_c above 2^28, n_buf above 2^24.
+ * work: tq_cache_attend_bytes bytes.                                                                              */
 size_t tq_cache_append_bytes(int64_t batch, int d, int mse_bits, int value_bits, int group_size);
 int tq_cache_append(const float *key, const float *value, int64_t key_stride, int64_t value_stride, const float *key_buf,
                     const float *value_buf, int64_t ks_b, int64_t ks_h, int64_t ks_r, int64_t vs_b, int64_t vs_h,

@@ -787,6 +787,23 @@ def test_inner_products_on_the_matrix_cores(gpu, d, bits, lead, n_k, n_q, dtype)
     assert got.shape == want.shape and bool(((got - want).abs() <= bound + 4e-7 * want.abs()).all())
 
 
+def test_inner_products_with_more_keys_than_a_grid_counts(gpu):
+    """2^30 + 77 keys of 64 (29 GB): more threads along the keys than a launch may have.  The estimates at both ends and around the places where
+    a launch ends are those of the same codes alone, bit for bit."""
+    from turboquant_amd.quantizer import ProdQuantized, TurboQuantProd
+    n = (1 << 30) + 77
+    g = torch.Generator(device=gpu).manual_seed(3)
+    tq = TurboQuantProd(64, bits=2, device=gpu)
+    codes = torch.empty(2, n, 8, dtype=torch.uint8, device=gpu).random_(generator=g)
+    norms = torch.empty(2, n, device=gpu).uniform_(0.5, 2.0, generator=g)
+    q = torch.randn(1, 64, generator=g, device=gpu)
+    got = tq.attention_score(q, ProdQuantized(codes[0], codes[1], norms[0], norms[1], 1))
+    for at in (0, (1 << 28) - 40, (1 << 29) - 40, 3 * (1 << 28) - 40, (1 << 30) - 40, n - 100):
+        part = slice(at, at + 100)
+        want = tq.attention_score(q, ProdQuantized(codes[0, part].clone(), codes[1, part].clone(), norms[0, part].clone(), norms[1, part].clone(), 1))
+        assert torch.equal(got[:, part], want)
+
+
 @pytest.mark.parametrize("d,bits,dtype", [(128, 3, torch.float32), (128, 4, torch.bfloat16), (256, 3, torch.float16)])
 def test_flat_codes_of_few_vectors_are_those_of_many(gpu, d, bits, dtype):
     """A tile of 16 vectors per workgroup in small calls, groups of tiles in large ones: codes, norms and de-quantised rows bit for bit."""

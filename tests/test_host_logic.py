@@ -465,17 +465,18 @@ def test_cache_entries_refuse_what_they_cannot_index_before_any_launch():
         return lib.tq_cache_append(A, A, 128, 128, A, A, 0, n_buf * 128, 128, 0, n_buf * 128, 128, 8, 8, n_buf, C.byref(ly), 2, 32, 100,
                                    *sections, *(A,) * 7, A, A, A, None)
 
-    def scores(idx=A, signs=A, n_q=1):
-        return lib.tq_cache_scores(A, 8, 8, n_q, idx, signs, A, A, 100, C.byref(ly), A, 0, 128 * 128, 128, 128, 0.1, A, A, None)
+    def scores(idx=A, signs=A, n_q=1, n_buf=128):
+        return lib.tq_cache_scores(A, 8, 8, n_q, idx, signs, A, A, 100, C.byref(ly), A, 0, n_buf * 128, 128, n_buf, 0.1, A, A, None)
 
-    def attend(data=A, n_q=1):
-        return lib.tq_cache_attend(A, 8, 8, n_q, data, A, A, 100, 128, 32, 2, A, 0, 128 * 128, 128, 128, A, A, None)
+    def attend(data=A, n_q=1, n_buf=128):
+        return lib.tq_cache_attend(A, 8, 8, n_q, data, A, A, 100, 128, 32, 2, A, 0, n_buf * 128, 128, n_buf, A, A, None)
 
     for i in range(7):
         assert append(tuple(A + (j == i) for j in range(7))) == _ffi.TQ_EUNSUPPORTED
     assert append(n_buf=(1 << 20) + 1) == _ffi.TQ_EUNSUPPORTED
     assert scores(idx=A + 1) == scores(signs=A + 2) == scores(n_q=(1 << 18) + 1) == _ffi.TQ_EUNSUPPORTED
     assert attend(data=A + 1) == attend(n_q=65536) == _ffi.TQ_EUNSUPPORTED
+    assert scores(n_buf=(1 << 24) + 1) == attend(n_buf=(1 << 24) + 1) == _ffi.TQ_EUNSUPPORTED
 
 
 def _paper_pool(d, heads, key_bits=4, value_bits=4):

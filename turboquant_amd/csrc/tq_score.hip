@@ -258,7 +258,9 @@ struct CacheTail {
 // thread with the queries as LDS broadcasts, which this replaces, read 64 bytes of LDS per key and coordinate: 32 queries x 4096 keys of
 // 128 18.0 -> 5.1 us; the call with its rotation at 1000 keys of 576 and 33 queries 79 -> 27.
 // CACHE: the workgroups behind those of the compressed keys take the exact ones, a wavefront per row at a time
+// key0: first key of the launch (a grid dimension counts fewer than 2^32 threads: 2^28 keys at a time)
 constexpr int SCORE_KEYS = 64;     // keys per workgroup: sixteen for each of four wavefronts
+constexpr int64_t SCORE_LAUNCH_KEYS = 1 << 28;
 constexpr int SCORE_ROWS = 4;      // exact rows per workgroup: one per wavefront (eight behind one another, 4000 keys and 128 rows of 8 heads: 9.7 us, now 7.8)
 
 // Word w of a row of codes; BYTES: rows that are not 4-byte aligned
@@ -312,7 +314,8 @@ template <bool CACHE, int NT, bool BYTES = false>
 __global__ void __launch_bounds__(256)
 score_kernel(const float* __restrict__ q_rot, const float* __restrict__ q_sk, int64_t n_q,
              const uint8_t* __restrict__ idx, const uint8_t* __restrict__ signs, const void* __restrict__ norms,
-             int norm_dtype, const float* __restrict__ rnorms, int64_t n_k, tq_layer ly, float* __restrict__ scores, CacheTail tail) {
+             int norm_dtype, const float* __restrict__ rnorms, int64_t n_k, int64_t key0, tq_layer ly, float* __restrict__ scores,
+             CacheTail tail) {
   __shared__ float s_cent[16];
   const int d = ly.d, mb = ly.mse_bits;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -336,7 +339,7 @@ score_kernel(const float* __restrict__ q_rot, const float* __restrict__ q_sk, in
   }
   if (threadIdx.x < (1 << mb)) s_cent[threadIdx.x] = ly.centroids[threadIdx.x];
   __syncthreads();
-  const int64_t k0 = (int64_t)blockIdx.x * SCORE_KEYS + wave * 16;
+  const int64_t k0 = key0 + (int64_t)blockIdx.x * SCORE_KEYS + wave * 16;
   if (k0 >= n_k) return;
   const int n = lane & 15, kb = lane >> 4;
   const int64_t key = k0 + n < n_k ? k0 + n : n_k - 1;          // (keys and queries that do not exist: the last one, not stored)
@@ -752,13 +755,16 @@ extern "C" int tq_score(const void* q, int dtype, int64_t batch, int64_t n_q, co
   rc = tq_rotate_query(q, dtype, batch * n_q, layer, q_rot, q_sk, stream);
   if (rc) return rc;
   const int nt = score_query_tiles(batch, n_q, n_k);
-  const dim3 grid((unsigned)((n_k + SCORE_KEYS - 1) / SCORE_KEYS), (unsigned)((n_q + 16 * nt - 1) / (16 * nt)), (unsigned)batch);
   const bool words = (uintptr_t)idx % 4 == 0 && (uintptr_t)signs % 4 == 0;
   auto kern = words ? (nt == 2 ? score_kernel<false, 2> : score_kernel<false, 1>)
                     : (nt == 2 ? score_kernel<false, 2, true> : score_kernel<false, 1, true>);
-  kern<<<grid, dim3(256), 0, (hipStream_t)stream>>>(q_rot, q_sk, n_q, idx, signs, norms, norm_dtype, rnorms, n_k, *layer, scores,
-                                                    CacheTail{});
-  TQ_CHECK_LAUNCH();
+  for (int64_t key0 = 0; key0 < n_k; key0 += SCORE_LAUNCH_KEYS) {
+    const int64_t keys = std::min(n_k - key0, SCORE_LAUNCH_KEYS);
+    const dim3 grid((unsigned)((keys + SCORE_KEYS - 1) / SCORE_KEYS), (unsigned)((n_q + 16 * nt - 1) / (16 * nt)), (unsigned)batch);
+    kern<<<grid, dim3(256), 0, (hipStream_t)stream>>>(q_rot, q_sk, n_q, idx, signs, norms, norm_dtype, rnorms, n_k, key0, *layer, scores,
+                                                      CacheTail{});
+    TQ_CHECK_LAUNCH();
+  }
   return TQ_OK;
 }
 
@@ -971,7 +977,7 @@ extern "C" int tq_cache_scores(const float* q, int64_t batch, int H, int64_t n_q
   if (!q || !idx || !signs || !norms || !rnorms || !key_buf || !scores || !work) return TQ_ENULL;
   const int d = layer->d;
   if (!cache_dims(batch, H, d) || n_q <= 0 || n_c <= 0 || n_buf <= 0) return TQ_EINVAL;
-  if (((uintptr_t)idx | (uintptr_t)signs) & 3 || n_c > (1 << 28) || n_q > (1 << 18)) return TQ_EUNSUPPORTED;
+  if (((uintptr_t)idx | (uintptr_t)signs) & 3 || n_c > SCORE_LAUNCH_KEYS || n_q > (1 << 18) || n_buf > (1 << 24)) return TQ_EUNSUPPORTED;
   float* q_rot = work;
   float* q_sk = work + batch * n_q * d;
   rc = tq_rotate_query(q, TQ_F32, batch * n_q, layer, q_rot, q_sk, stream);
@@ -982,7 +988,7 @@ extern "C" int tq_cache_scores(const float* q, int64_t batch, int H, int64_t n_q
                   (unsigned)batch);
   auto kern = nt == 2 ? score_kernel<true, 2> : score_kernel<true, 1>;
   kern<<<grid, dim3(256), 0, (hipStream_t)stream>>>(
-      q_rot, q_sk, n_q, idx, signs, norms, TQ_F32, rnorms, n_c, *layer, scores, tail);
+      q_rot, q_sk, n_q, idx, signs, norms, TQ_F32, rnorms, n_c, 0, *layer, scores, tail);
   TQ_CHECK_LAUNCH();
   return TQ_OK;
 }
@@ -997,7 +1003,7 @@ extern "C" int tq_cache_attend(const float* weights, int64_t batch, int H, int64
                                int64_t s_b, int64_t s_h, int64_t s_r, int n_buf, float* out, float* work, void* stream) {
   if (!weights || !data || !scales || !zeros || !value_buf || !out || !work) return TQ_ENULL;
   if (!cache_dims(batch, H, d) || n_q <= 0 || n_c <= 0 || n_buf <= 0 || group_size < 16 || d % group_size) return TQ_EINVAL;
-  if (group_size % 16 || ((uintptr_t)data & 3) || n_c > (1 << 28) || n_q > 65535) return TQ_EUNSUPPORTED;
+  if (group_size % 16 || ((uintptr_t)data & 3) || n_c > (1 << 28) || n_q > 65535 || n_buf > (1 << 24)) return TQ_EUNSUPPORTED;
   const int shares = (int)((n_c + ATT_TOKENS - 1) / ATT_TOKENS), all = shares + (n_buf + ATT_ROWS - 1) / ATT_ROWS;
   const dim3 grid((unsigned)all, (unsigned)n_q, (unsigned)batch);
 #define TQ_ATTEND(VB)                                                                                                   \
