@@ -497,6 +497,35 @@ def test_rotation_of_hundreds_of_rows(gpu, d, Hq, B, dtype):
     assert float((outs[0] - outs[1]).abs().max()) <= 2.0 ** -7 * float(outs[1].abs().max())
 
 
+@pytest.mark.parametrize("dtype,unit,scale", [(torch.float16, 2.0 ** -15, 2.0 ** 11), (torch.bfloat16, 2.0 ** -69, 2.0 ** 65)])
+def test_rotation_of_rows_of_tiny_numbers(gpu, dtype, unit, scale):
+    """Rows of fp16 subnormals, of bf16 numbers whose squares are fp32 subnormals, and some of zeros and of single such numbers, with a scale
+    that makes their scores count: as the vector-ALU rotation."""
+    d, Hq, B = 576, 8, 40
+    pool, tq = _make_pool(gpu, d, 4, 4, 1, 6, dtype)
+    g = torch.Generator().manual_seed(9)
+    k, v = (torch.randn(1, 90, 1, d, generator=g).to(dtype).to(gpu) for _ in range(2))
+    table = torch.arange(6, dtype=torch.int32, device=gpu)
+    pool.append(k, v, table[None])
+    q = torch.rand(B, Hq, d, generator=g) * 2 - 1
+    q[::3, 1] = 0
+    q[1::3, 2, 5:] = 0
+    q[::4, 3] *= 1e3                                                 # (ordinary rows among them)
+    q = (q * unit).to(dtype).to(gpu)
+    assert int((q != 0).sum()) > q.numel() // 2
+    seq = torch.full((B,), 90, dtype=torch.int32, device=gpu)
+    outs = []
+    try:
+        for opt in (1, 0):
+            _set_option("prep_mfma", opt)
+            outs.append(pool.decode_attention(q, table, seq, n_split=1, max_len=90, scale=scale).float())
+    finally:
+        _set_option("prep_mfma", 1)
+    mean = pool.decode_attention(torch.zeros_like(q), table, seq, n_split=1, max_len=90).float()
+    assert float((outs[1] - mean).abs().max()) > 0.1 * float(mean.abs().max())                  # (the scores count)
+    assert float((outs[0] - outs[1]).abs().max()) <= 2.0 ** -7 * float(outs[1].abs().max())
+
+
 # ------------------------------------------------------------------ the exact tail on the matrix cores
 @pytest.mark.parametrize("d,Hq,Hkv,B,dtype,rows,n_split", [
     (128, 5, 1, 2, torch.bfloat16, [1, 16], 1), (128, 16, 1, 3, torch.float16, [15, 17, 0], 3), (128, 17, 1, 1, torch.bfloat16, [129], 2),
