@@ -161,18 +161,27 @@ def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+_transforms, _tracing, _compiling = torch._C._are_functorch_transforms_active, torch._C._is_tracing, torch.compiler.is_compiling
+_forward_ad, _grad_enabled = torch.autograd.forward_ad, torch.is_grad_enabled
+
+
 def ordinary(*tensors) -> bool:
     """Whether torch would run an operation on these GPU tensors as it stands: plain tensors of one GPU, nothing to differentiate,
     no transform, trace or dispatch mode that has to see the operation."""
-    if (torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack() or torch._C._are_functorch_transforms_active()
-            or torch.autograd.forward_ad._current_level >= 0 or torch.compiler.is_compiling() or torch.jit.is_tracing()):
+    if (_dispatch_modes() or _function_modes() or _transforms() or _forward_ad._current_level >= 0 or _compiling() or _tracing()):
         return False
-    grad = torch.is_grad_enabled()
+    grad, device = _grad_enabled(), -1
     for t in tensors:
-        if type(t) is not torch.Tensor or not t.is_cuda or (grad and t.requires_grad) or t.device != tensors[0].device:
+        if type(t) is not torch.Tensor or not t.is_cuda or (grad and t.requires_grad):
             return False
         if t.is_neg() or t._is_zerotensor():             # (its memory does not hold its values)
             return False
+        at = t.get_device()
+        if at != device:
+            if device >= 0:
+                return False
+            device = at
     return True
 
 

@@ -78,7 +78,12 @@ def dequantize_values(vq: ValueQuantized, group_size: int = 32) -> torch.Tensor:
 
 def _plain(*tensors) -> bool:
     """Ordinary fp32 tensors of four dimensions with contiguous channels, on which torch would run an operation as it stands."""
-    return _ffi.ordinary(*tensors) and all(t.dtype == torch.float32 and t.dim() == 4 and t.stride(-1) == 1 for t in tensors)
+    if not _ffi.ordinary(*tensors):
+        return False
+    for t in tensors:
+        if t.dtype is not torch.float32 or t.dim() != 4 or t.stride(3) != 1:
+            return False
+    return True
 
 
 def _plain_product(*tensors) -> bool:
@@ -153,12 +158,12 @@ class TurboQuantKVCache:
             return False
         idx, signs, rnorms, norms = kq[:4]
         data, scales, zeros = vq[:3]
-        n, groups = norms.numel(), d // gs
-        return (idx.dtype is signs.dtype is data.dtype is torch.uint8
-                and rnorms.dtype is norms.dtype is scales.dtype is zeros.dtype is torch.float32
-                and idx.numel() == n * (d * _packing(self.key_bits - 1)[0] // 8) and signs.numel() == n * (d // 8) and rnorms.numel() == n
-                and data.numel() == n * (d * bits // 8) and scales.numel() == zeros.numel() == n * groups
-                and all([type(t) is torch.Tensor and t.is_contiguous() for t in (idx, signs, rnorms, norms, data, scales, zeros)]))
+        n, groups, byte, f32, Tensor = norms.numel(), d // gs, torch.uint8, torch.float32, torch.Tensor
+        for t, dtype, count in ((idx, byte, d * _packing(self.key_bits - 1)[0] // 8), (signs, byte, d // 8), (rnorms, f32, 1), (norms, f32, 1),
+                                (data, byte, d * bits // 8), (scales, f32, groups), (zeros, f32, groups)):
+            if type(t) is not Tensor or t.dtype is not dtype or t.numel() != n * count or not t.is_contiguous():
+                return False
+        return True
 
     def _append_spill(self, key: torch.Tensor, value: torch.Tensor) -> bool:
         """One token into a full buffer whose first row leaves for the compressed part, in one library call; False: the case is
