@@ -591,14 +591,41 @@ def test_exact_tail_in_place_with_two_wavefronts_per_unit(gpu, dtype):
 
 
 # ------------------------------------------------------------------ a token of the cache object in fp32
+class _Counted:
+    """The library, counting the calls of each entry that it answered."""
+    def __init__(self, lib):
+        self._lib, self.answered = lib, {}
+
+    def __getattr__(self, name):
+        entry = getattr(self._lib, name)
+
+        def call(*args):
+            rc = entry(*args)
+            if rc == 0:
+                self.answered[name] = self.answered.get(name, 0) + 1
+            return rc
+        return call
+
+    def take(self, name):
+        return self.answered.pop(name, 0)
+
+
+@pytest.fixture
+def counted(monkeypatch):
+    from turboquant_amd import _ffi
+    lib = _Counted(_ffi.lib())
+    monkeypatch.setattr(_ffi, "lib", lambda: lib)
+    return lib
+
+
 @pytest.mark.parametrize("d,B,H,prompt,buffer,key_bits,vb,gs,n_q", [
     (128, 1, 8, 400, 128, 3, 2, 32, 1), (64, 2, 3, 150, 128, 4, 4, 32, 1), (256, 1, 2, 300, 1, 2, 8, 64, 3), (128, 2, 1, 129, 128, 3, 4, 16, 9),
     (64, 1, 5, 65, 64, 5, 2, 64, 2), (128, 3, 4, 384, 33, 3, 2, 128, 1)])
-def test_cache_token_in_few_launches(gpu, monkeypatch, d, B, H, prompt, buffer, key_bits, vb, gs, n_q):
+def test_cache_token_in_few_launches(gpu, counted, d, B, H, prompt, buffer, key_bits, vb, gs, n_q):
     """Tokens, scores and values of the cache object through the entries of their own, against the general paths: codes,
     norms and buffers bit for bit, inner products with the compressed keys bit for bit, everything else within fp32 sums in another
     order.  Prompts as views of a (batch, tokens, heads, d) tensor, the buffer's rows then not behind one another: the
-    first token takes the general path, the ones after it do not."""
+    first token takes the general path, the ones after it do not (all of them do where several batches' tokens lie apart as well)."""
     from turboquant_amd import kv_cache as KC
     g = torch.Generator().manual_seed(d + prompt)
     for view in (False, True):
@@ -609,8 +636,9 @@ def test_cache_token_in_few_launches(gpu, monkeypatch, d, B, H, prompt, buffer, 
         qs = torch.randn(4, B, H, n_q, d, generator=g).to(gpu)
         results = []
         for fast in (True, False):
+            patch = pytest.MonkeyPatch()
             if not fast:
-                monkeypatch.setattr(KC, "_plain", lambda *t: False)
+                patch.setattr(KC, "_plain", lambda *t: False)
             cache = KC.TurboQuantKVCache(d, key_bits=key_bits, value_bits=vb, value_group_size=gs, buffer_size=buffer, device=gpu,
                                          dtype=torch.float32)
             cache.prefill(k[..., :prompt, :], v[..., :prompt, :])
@@ -623,7 +651,9 @@ def test_cache_token_in_few_launches(gpu, monkeypatch, d, B, H, prompt, buffer, 
                 scores = cache.attention_scores(qs[i])
                 outs.append((scores, cache.attend(torch.softmax(scores, dim=-1))))
             results.append((cache, outs))
-            monkeypatch.undo()
+            patch.undo()
+            assert counted.take("tq_cache_append") == (0 if not fast else 4 if not view else 3 if B == 1 else 0)
+            assert counted.take("tq_cache_scores") == counted.take("tq_cache_attend") == (4 if fast else 0)
         (a, oa), (b, ob) = results
         assert a.get_seq_length() == b.get_seq_length() and a.memory_bytes() == b.memory_bytes()
         for x, y in zip((*a.key_quantized[:4], *a.value_quantized[:3], a.key_buffer, a.value_buffer),
@@ -683,33 +713,6 @@ def test_cache_token_that_has_to_be_differentiated(gpu):
     out.sum().backward()
     assert q.grad is not None and torch.isfinite(q.grad).all() and float(q.grad.abs().max()) > 0
     assert torch.allclose(out, cache.attend(torch.softmax(scores, dim=-1).detach()), rtol=1e-4, atol=1e-5)
-
-
-class _Counted:
-    """The library, counting the calls of each entry that it answered."""
-    def __init__(self, lib):
-        self._lib, self.answered = lib, {}
-
-    def __getattr__(self, name):
-        entry = getattr(self._lib, name)
-
-        def call(*args):
-            rc = entry(*args)
-            if rc == 0:
-                self.answered[name] = self.answered.get(name, 0) + 1
-            return rc
-        return call
-
-    def take(self, name):
-        return self.answered.pop(name, 0)
-
-
-@pytest.fixture
-def counted(monkeypatch):
-    from turboquant_amd import _ffi
-    lib = _Counted(_ffi.lib())
-    monkeypatch.setattr(_ffi, "lib", lambda: lib)
-    return lib
 
 
 @pytest.mark.parametrize("d,H,n_c,n_buf,vb", [(64, 8, 1000, 128, 2), (128, 8, 300, 128, 4), (256, 3, 2000, 33, 2)])
@@ -850,6 +853,17 @@ def test_flat_codes_of_few_vectors_are_those_of_many(gpu, d, bits, dtype):
 
 
 # ------------------------------------------------------------------ keys and values of a small append in one launch
+def _nodes(call):
+    """Nodes of a graph that `call` is captured into."""
+    import ctypes
+    from turboquant_amd import _ffi
+    graph, n = torch.cuda.CUDAGraph(keep_graph=True), ctypes.c_size_t()
+    with torch.cuda.graph(graph):
+        call()
+    assert _ffi.lib().hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    return n.value
+
+
 @pytest.mark.parametrize("d,B,H,T,kb,vb,gs,dtype,ragged", [
     (128, 1, 1, 1, 3, 2, 32, torch.bfloat16, False), (128, 33, 3, 1, 4, 4, 16, torch.float16, False),
     (256, 5, 2, 17, 3, 4, 128, torch.bfloat16, False), (256, 16, 8, 1, 2, 2, 64, torch.float16, False),
@@ -869,7 +883,8 @@ def test_small_append_in_one_launch(gpu, d, B, H, T, kb, vb, gs, dtype, ragged):
     rows = (sum(lens), H, d) if ragged else (B, T, H, d)
     k, v = (torch.randn(*rows, generator=g).to(gpu, dtype) for _ in range(2))
     fill = torch.randint(0, 256, (B * per_seq,), generator=g, dtype=torch.uint8).to(gpu)
-    got = []
+    table_gpu, starts_gpu = table.to(gpu), starts.to(gpu)
+    got, nodes = [], []
     for one in (True, False):
         pool = PagedKVPool(tq, H, B * per_seq, value_bits=vb, value_group_size=gs, dtype=dtype, device=gpu)
         pool.data += fill[:, None, None]
@@ -879,17 +894,19 @@ def test_small_append_in_one_launch(gpu, d, B, H, T, kb, vb, gs, dtype, ragged):
                 row0 = _i32([sum(lens[:b]) for b in range(B)], gpu)
                 pool.append_ragged(k, v, row0, _i32(lens, gpu), starts.to(gpu), table.to(gpu), max_run=T)
             else:
-                pool.append(k, v, table.to(gpu), start_pos=starts.to(gpu))
+                pool.append(k, v, table_gpu, start_pos=starts_gpu)
+                nodes.append(_nodes(lambda: pool.append(k, v, table_gpu, start_pos=starts_gpu)))
         finally:
             _set_option("append_small", -1)
         got.append(pool.data.clone())
+    assert ragged or nodes[0] == nodes[1] - 1
     assert torch.equal(*got) and not torch.equal(got[0], torch.zeros_like(got[0]) + fill[:, None, None])
 
 
 # ------------------------------------------------------------------ a ring's rows in one launch
 @pytest.mark.parametrize("H,d,dtype,n,capacity", [(8, 128, torch.bfloat16, 1, 4), (1, 64, torch.float16, 5, 3), (3, 64, torch.float32, 257, 300),
                                                   (5, 66, torch.bfloat16, 2, 4)])
-def test_ring_rows_from_any_layout(gpu, H, d, dtype, n, capacity):
+def test_ring_rows_from_any_layout(gpu, counted, H, d, dtype, n, capacity):
     """Rows of every layout a caller may hand over - side by side, in a wider tensor, heads transposed, one row repeated, misaligned, of
     another type, needing a gradient, the ring's own - end in the ring as torch's copies leave them, whoever copies them."""
     from turboquant_amd.capture import RingBuffer
@@ -898,8 +915,9 @@ def test_ring_rows_from_any_layout(gpu, H, d, dtype, n, capacity):
     flat = torch.randn(n * H * d + 1, generator=g).to(gpu, dtype)
     forms = [wide[:, 1].contiguous(), wide[:, 1], wide[:, 0].transpose(0, 1).contiguous().transpose(0, 1), wide[:1, 2].expand(n, H, d),
              flat[1:].view(n, H, d), wide[:, 2].double(), wide[:, 2].clone().requires_grad_()]
-    for x in forms:
-        for y in forms:
+    taken = set()
+    for ix, x in enumerate(forms):
+        for iy, y in enumerate(forms):
             ring, want = RingBuffer(capacity, H, d, gpu, dtype), RingBuffer(capacity, H, d, gpu, dtype)
             want._write_rows = lambda *a: False
             outs = []
@@ -908,6 +926,10 @@ def test_ring_rows_from_any_layout(gpu, H, d, dtype, n, capacity):
                 outs.append([t.detach() for o in out if o is not None for t in o] + [t.detach() for t in r.peek()])
             assert len(outs[0]) == len(outs[1]) and all(torch.equal(a, b) for a, b in zip(*outs))
             assert ring._rows.requires_grad == want._rows.requires_grad
+            if counted.take("tq_ring_write"):
+                taken.add((ix, iy))
+    plain = {(i, j) for i in (0, 1, 3) for j in (0, 1, 3)} if H * d * forms[0].element_size() % 16 == 0 else set()
+    assert plain <= taken and not any(i in (4, 5, 6) for pair in taken for i in pair)
     ring = RingBuffer(capacity, H, d, gpu, dtype)
     ring.write(forms[0], forms[0], 1)
     before = ring._rows._version
