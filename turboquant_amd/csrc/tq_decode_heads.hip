@@ -568,12 +568,8 @@ int launch_decode_heads(int B, int Hq, int Hkv, const uint8_t* pool, const int32
     else if (L.value_bits == 4) TQ_HEADS_T(D, 2, 4)                \
     else TQ_HEADS_T(D, 2, 2)                                       \
   }
-#ifdef HEADS_ONE
-  TQ_HEADS(576, 3, 4, false, HEADS_ONE)
-#else
   if (ly.d == 576) TQ_HEADS_V(576)
   else TQ_HEADS_V(512)
-#endif
 #undef TQ_HEADS_V
 #undef TQ_HEADS_T
 #undef TQ_HEADS_HW
