@@ -922,10 +922,12 @@ __device__ __forceinline__ void rotate_rows_body(const uint16_t* __restrict__ q,
         qn[kk][ti] = *(const prep_u32x4*)(qrow[ti] + min(ks + AHEAD, KS - 1) * 32);
         typedef float rot_f32x2 __attribute__((ext_vector_type(2)));
         typedef __bf16 rot_bf16x2 __attribute__((ext_vector_type(2)));
-        if constexpr (!F16Q) {                                       // (the sum of squares only bounds the row; fp16: below)
+        typedef _Float16 rot_f16x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            ss[ti] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(rot_bf16x2, qb[ti][e]), __builtin_bit_cast(rot_bf16x2, qb[ti][e]), ss[ti], false);
+        for (int e = 0; e < 4; ++e) {
+          // (the sum of squares only bounds the row)
+          if constexpr (F16Q) ss[ti] = __builtin_amdgcn_fdot2(__builtin_bit_cast(rot_f16x2, qb[ti][e]), __builtin_bit_cast(rot_f16x2, qb[ti][e]), ss[ti], false);
+          else ss[ti] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(rot_bf16x2, qb[ti][e]), __builtin_bit_cast(rot_bf16x2, qb[ti][e]), ss[ti], false);
         }
         if (word == 0 || F16Q) {
           float x[8];
@@ -942,8 +944,6 @@ __device__ __forceinline__ void rotate_rows_body(const uint16_t* __restrict__ q,
           if constexpr (F16Q) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-              // (not a dot product of fp16 pairs, which may take subnormal numbers for zero: a row of them would have no bound)
-              ss[ti] = fmaf(x[2 * e], x[2 * e], fmaf(x[2 * e + 1], x[2 * e + 1], ss[ti]));
               const rot_f32x2 xv = {x[2 * e], x[2 * e + 1]};
               const uint32_t hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(xv, rot_bf16x2));
               const rot_f32x2 rem = {xv[0] - __uint_as_float(hi << 16), xv[1] - __uint_as_float(hi & 0xffff0000u)};
@@ -964,29 +964,6 @@ __device__ __forceinline__ void rotate_rows_body(const uint16_t* __restrict__ q,
             acc[t][jt][ti] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ma, __builtin_bit_cast(prep_bf16x8, qb[ti]), acc[t][jt][ti], 0, 0, 0);
           }
         }
-    }
-    if constexpr (!F16Q) {
-      // Dot products of bf16 pairs take subnormal sums for zero: a row whose squares are that small is summed again in fp32
-#pragma unroll 1
-      for (int ti = 0; ti < NT; ++ti) {
-        float sum = ss[0];
-#pragma unroll
-        for (int j = 1; j < NT; ++j) sum = ti == j ? ss[j] : sum;
-        if (__builtin_amdgcn_ballot_w64(sum < 0x1p-100f) == 0) continue;
-        const uint16_t* row = q + (row0 + min(16 * ti + n, nr - 1)) * D + kb * 8;
-        sum = 0.0f;
-#pragma unroll 1
-        for (int ks = 0; ks < KS; ++ks) {
-          const prep_u32x4 x = *(const prep_u32x4*)(row + ks * 32);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float lo = __uint_as_float(x[e] << 16), hi = __uint_as_float(x[e] & 0xffff0000u);
-            sum = fmaf(lo, lo, fmaf(hi, hi, sum));
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < NT; ++j) ss[j] = ti == j ? sum : ss[j];
-      }
     }
     const float k = wp.sm_scale * 1.4426950408889634f;
 #pragma unroll
