@@ -1573,9 +1573,10 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
     if (prep_smem_bytes(prep_rows, d) > fsm) fsm = prep_smem_bytes(prep_rows, d);
     const int n_sched = plan.items ? SCHED_FRONT : 0;
     if (n_sched && fsm < SCHED_SMEM_INTS * sizeof(int)) fsm = SCHED_SMEM_INTS * sizeof(int);
-    // ... unless the tail's tiles leave room for one workgroup per compute unit only (head_dim 256 with 128 exact
-    // tokens: 139 KB) and the grid is larger than the card: the preparation workgroups would queue behind that
-    // LDS size too (128 x 2048, 16 q / 2 KV heads: 109.7 us per step fused, 88.1 as two launches)
+    // ... unless the tail's tiles leave room for one workgroup per compute unit only (fp32 rows, 139 KB at head_dim 128 with 128
+    // exact tokens; the matrix-core tail of 16-bit rows takes at most 66 KB) and the grid is larger than the card: the preparation
+    // workgroups would queue behind that LDS size too (measured when 16-bit rows of 256 took as much: 128 x 2048, 16 q / 2 KV heads
+    // 109.7 us per step in one launch, 88.1 in two)
     const bool one_per_unit = fsm > (size_t)80 * 1024;
     const bool tail_shares = tail && ta.wide && (tail_mfma || dtype == TQ_F32) && mfma_shape && stages == 7;
     // The preparation on the matrix cores shares the launch too (96 sequences of 61 .. 8190 tokens at 40 q / 8 KV heads of 128: a

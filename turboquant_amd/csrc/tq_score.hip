@@ -220,7 +220,7 @@ prep_query_kernel(const void* __restrict__ q, int G, int gpw, int64_t n_rows, in
     prefetch_pages_body<PREP_COLS * PREP_SLICES>(pf, id - n_prep);
 }
 
-// The preparation on the matrix cores (bf16 queries, head_dim 128 / 256): a workgroup per (tile of up to 16 query
+// The preparation on the matrix cores (bf16 queries, head_dim 128 / 256; fp16 queries, 128): a workgroup per (tile of up to 16 query
 // rows, plane word), then the page-prefetch workgroups.
 // WW: a workgroup per tile, its wavefronts each taking a plane word at a time.
 template <int D, bool WW, bool F16Q>
@@ -252,11 +252,12 @@ struct CacheTail {
 // scores[b, i, k] on the matrix cores: v_mfma_f32_16x16x4_f32 with sixteen rotated / sketched queries as rows, sixteen keys as columns
 // and fp32 operands on both sides (a centroid or a sign is an fp32 number), so nothing is split or rounded.  Of every sixteen
 // coordinates a lane holds four of its key and the same four of its query, which it reads straight from the rotation's rows: the four lanes
-// of a row take 64 consecutive bytes (a quarter of the coordinates in a row per lane touched 64 lines per load: 8 heads x 16384 keys x 128
-// queries 180 us; now 120).  NT tiles of sixteen queries share one expansion of the codes.
+// of a row take 64 consecutive bytes (a quarter of the coordinates in a row per lane touched 64 lines per load: 215 us where the kernel
+// that this replaces took 180).  NT tiles of sixteen queries share one expansion of the codes.
 // Bound by latency in small calls, else by the fp32 matrix rate (two MFMAs of 32 cycles per 4 coordinates of a 16 x 16 tile).  One key per
 // thread with the queries as LDS broadcasts, which this replaces, read 64 bytes of LDS per key and coordinate: 32 queries x 4096 keys of
-// 128 18.0 -> 5.1 us; the call with its rotation at 1000 keys of 576 and 33 queries 79 -> 27.
+// 128 18.0 -> 5.1 us; the call with its rotation, 8 heads x 16384 keys x 128 queries of 128 166 -> 130 us, of 256 308 -> 251, 1000 keys of 576
+// and 33 queries 78 -> 25.
 // CACHE: the workgroups behind those of the compressed keys take the exact ones, a wavefront per row at a time
 // key0: first key of the launch (a grid dimension counts fewer than 2^32 threads: 2^28 keys at a time)
 constexpr int SCORE_KEYS = 64;     // keys per workgroup: sixteen for each of four wavefronts
@@ -525,8 +526,8 @@ namespace tq {
 int launch_dequant_mfma(const uint8_t* idx, const uint8_t* signs, const void* norms, int norm_dtype, const float* rnorms,
                         int64_t n_vec, const tq_layer& ly, float* out, hipStream_t st);
 
-// Whether launch_rotate_query prepares these rows on the matrix cores (bf16 queries at head_dim 128 / 256 with the
-// split matrices at hand; whole groups of G heads; operands only).
+// Whether launch_rotate_query prepares these rows on the matrix cores (bf16 queries at head_dim 128 / 256, fp16 queries at 128, with
+// the split matrices at hand; whole groups of G heads; operands only).
 // (head_dim 256 with few rows keeps the vector-ALU kernel: 64 rows - 32 workgroups here, each pulling 96 KB of
 // matrix terms - measured 1 us slower per step; from 64 workgroups on the two are level or this one ahead:
 // 16 x 8192 at 32 q heads 35.0 -> 34.5 us per step, 64 x 2048 40.2 -> 36.4, 256 x 1024 107.6 -> 86.2)
@@ -553,14 +554,14 @@ static bool rotate_packs(int64_t rows, const tq_layer* layer, const WidePack* wi
   return wide != nullptr && wide->qa != nullptr && wide->q_stat != nullptr && layer->Pi_colsum && layer->S_colsum &&
          wide->ntp >= 2 && wide->ntp <= 9 && rows % wide->Hq == 0 && rows < (1 << 30) && layer->d <= 768;
 }
-// ... and whether it does so on the matrix cores (bf16 queries with the layer's split matrices)
 // Row tiles from which a rotation keeps a (plane word, product) pair's matrix terms in LDS and passes over the tiles
 // (rotate_rows_body) instead of running a workgroup per (tile, word, product): when the latter are more than the card holds
 // at once, two per compute unit.
 bool rotate_by_rows(int64_t rows, int d) {
   return ((rows + 15) / 16) * 8 * ((2 * (d / ROT_COLS) + 7) / 8) > 2 * (int64_t)device_compute_units();
 }
-// (bf16 queries; fp16 queries as two bf16 terms)
+// ... and whether the launch that packs does so on the matrix cores (with the layer's split matrices: bf16 queries, fp16 queries as
+// two bf16 terms)
 bool rotate_on_matrix_cores(const void* q, int dtype, int64_t rows, const tq_layer* layer, const WidePack* wide) {
   const int d = layer->d;
   return rotate_packs(rows, layer, wide) && layer->Pi_split && layer->S_split &&
@@ -662,7 +663,7 @@ int launch_rotate_query(const void* q, int dtype, int64_t rows, const tq_layer* 
   if (R < 1 || d % ROT_COLS || d % (8 * ROT_SLICES)) return TQ_EUNSUPPORTED;
   const bool pack = rotate_packs(rows, layer, wide);
   const WidePack wp = pack ? *wide : WidePack{};
-  // bf16 queries with the layer's split matrices: rotation and packing on the matrix cores
+  // bf16 and fp16 queries with the layer's split matrices: rotation and packing on the matrix cores
   if (rotate_on_matrix_cores(q, dtype, rows, layer, wide)) {
     const int n_tiles = (int)((rows + 15) / 16), pair_rounds = (2 * (d / ROT_COLS) + 7) / 8;
     if (rotate_by_rows(rows, d)) {
