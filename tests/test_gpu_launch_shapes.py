@@ -564,6 +564,16 @@ def test_exact_tail_on_the_matrix_cores(gpu, d, Hq, Hkv, B, dtype, rows, n_split
     assert float((outs[0] - outs[1]).abs().max()) <= 2.0 ** -7 * float(outs[1].abs().max())
 
 
+@pytest.mark.parametrize("Hq,Hkv,B,dtype,rows", [
+    (16, 2, 16, torch.float16, [16, 3, 0, 64]), (2, 2, 16, torch.bfloat16, [16, 1]),        # tail and preparation on the vector ALU in one launch
+    (16, 2, 16, torch.float16, [65, 128]), (32, 2, 16, torch.bfloat16, [16, 5]),            # the tail on the matrix cores, two rounds of workgroups
+    (32, 2, 1, torch.float16, [128]), (32, 2, 2, torch.bfloat16, [100, 128]),               # sixteen heads of few sequences
+    (8, 2, 128, torch.float16, [16, 9]), (8, 2, 128, torch.bfloat16, [128, 77])])           # three rounds: a launch each
+def test_exact_tail_at_head_dim_256_in_each_launch(gpu, Hq, Hkv, B, dtype, rows):
+    """The forms of the launch before the page kernel, as above."""
+    test_exact_tail_on_the_matrix_cores(gpu, 256, Hq, Hkv, B, dtype, rows, 1)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_exact_tail_in_place_with_two_wavefronts_per_unit(gpu, dtype):
     """The newest tokens read in place from a paged cache by 528 units, against the same rows gathered (same kernel, same bits up

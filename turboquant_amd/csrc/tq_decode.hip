@@ -1060,10 +1060,11 @@ exact_tail_mfma_kernel(TailArgs A, int B) {
 // (the first n_tail, so that the longer-running ones start first) and the query preparation of the
 // matrix-core kernel.  They are independent of each other, both have 512 lanes, and together they are
 // far fewer workgroups than the card has compute units, so the launch takes as long as the slower of
-// the two instead of their sum plus a dispatch gap.
+// the two instead of their sum plus a dispatch gap.  WORDS: the tail on the vector ALU (exact_tail_words_body), which leaves two workgroups
+// to a compute unit at head_dim 256.
 static_assert(TAIL_THREADS == PREP_COLS * PREP_SLICES, "the two roles share a workgroup size");
-template <int PER, int DT, bool PAGED, bool PACKED>
-__global__ void __launch_bounds__(TAIL_THREADS, DT != TQ_F32 && PER == 16 ? 2 : 4)
+template <int PER, int DT, bool PAGED, bool PACKED, bool WORDS>
+__global__ void __launch_bounds__(TAIL_THREADS, !WORDS && PER == 16 ? 2 : 4)
 prep_tail_kernel(TailArgs A, int n_tail, int B, int Gq, tq_layer ly, float* __restrict__ q_rot, float* __restrict__ q_sk,
                  float* __restrict__ q_stat, uint32_t* __restrict__ qa_pack, unsigned long long* __restrict__ arrivals,
                  int prep_gpw, int n_front, PagePrefetch pf, int g_tot, int head_rows, SplitPlan sp) {
@@ -1074,7 +1075,7 @@ prep_tail_kernel(TailArgs A, int n_tail, int B, int Gq, tq_layer ly, float* __re
   }
   const int id = blockIdx.x - (sp.items ? SCHED_FRONT : 0);
   if (id < n_tail) {
-    if constexpr (DT == TQ_F32) exact_tail_words_body<DT, 1, PAGED, true>(A, id % A.Hkv, (id / A.Hkv) % B, id / (A.Hkv * B), sm);
+    if constexpr (WORDS) exact_tail_words_body<DT, 1, PAGED, true>(A, id % A.Hkv, (id / A.Hkv) % B, id / (A.Hkv * B), sm);
     else if (A.wpu == 2) exact_tail_mfma_body<DT, PER * PREP_SLICES, PAGED, 2>(A, id, B, sm);
     else exact_tail_mfma_body<DT, PER * PREP_SLICES, PAGED, TAIL_WAVES>(A, id, B, sm);
   } else if (id >= n_front) {      // behind the tail and the preparation: the page kernel's first pages, read ahead of it
@@ -1569,9 +1570,27 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
     // per lane and the tail's LDS is sized by the rows it holds, so two workgroups fit a compute unit; with more
     // workgroups than that the rest follow as slots free up, which still measured faster than a launch each
     // (16 x 8192: 48.9 -> 45.2 us per step, 32 x 32768: 223.6 -> 221.5 us).
-    size_t fsm = tail_lds;
-    if (prep_smem_bytes(prep_rows, d) > fsm) fsm = prep_smem_bytes(prep_rows, d);
+    const int cus = device_compute_units();
     const int n_sched = plan.items ? SCHED_FRONT : 0;
+    const bool mfma_prep_fits = tail_mfma && prep_on_matrix_cores(q, dtype, (int64_t)B * Hq, layer, Gq, g_tot);
+    const int rows_tile = (16 / Gq) * Gq;                         // (whole groups of heads, see prep_mfma_body; Gq <= 8)
+    const int n_tiles = (int)(((int64_t)B * Hq + rows_tile - 1) / rows_tile);
+    const bool ww = prep_tile_per_workgroup(n_tiles, d);
+    const int n_mprep = ww ? n_tiles : n_tiles * (d / 32);
+    const int n_words = Hkv * B * ((G + TAIL_GC - 1) / TAIL_GC) * t_chunks;
+    const size_t words_lds = tail_words_smem(d, recent_rows, ta.tile_words);
+    // At head_dim 256 a compute unit holds one workgroup of the matrix-core tail and of what shares its launch, but two with tail and preparation on
+    // the vector ALU where few exact tokens leave the LDS for them.  Both stay there while that is so and the launch has more workgroups than the
+    // card has units - rows that the matrix cores do not prepare (fp16, few rows: 16 exact tokens, 16 x 150, 2 KV heads, 8 heads each 24.9 us, with
+    // the matrix-core tail 27.2, a launch each 28.5; with 128 tokens, where one fits, 30.3, 25.1, 30.5), and more tails than preparation
+    // (64 exact tokens, 24 x 150, 8 KV heads of a head each 22.9 us, on the matrix cores 26.4).  The tail alone stays there where a unit of sixteen
+    // heads is a long chain of few workgroups (1 x 150, 128 exact tokens: 24.1 us, 25.4).
+    const bool words_pair = tail_mfma && d == 256 && words_lds <= (size_t)80 * 1024;
+    const bool mfma_prep = mfma_prep_fits && !(words_pair && n_tail >= n_mprep && n_tail + n_mprep >= cus);
+    const bool words_tail = !tail_mfma || (d == 256 && !mfma_prep && (words_pair ? n_tail + n_prep >= cus : G > 8 && n_words + n_prep <= cus));
+    const int n_shared = words_tail ? n_words : n_tail;
+    size_t fsm = words_tail ? words_lds : tail_lds;
+    if (prep_smem_bytes(prep_rows, d) > fsm) fsm = prep_smem_bytes(prep_rows, d);
     if (n_sched && fsm < SCHED_SMEM_INTS * sizeof(int)) fsm = SCHED_SMEM_INTS * sizeof(int);
     // ... unless the tail's tiles leave room for one workgroup per compute unit only (fp32 rows, 139 KB at head_dim 128 with 128
     // exact tokens; the matrix-core tail of 16-bit rows takes at most 66 KB) and the grid is larger than the card: the preparation
@@ -1579,15 +1598,14 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
     // 109.7 us per step in one launch, 88.1 in two)
     const bool one_per_unit = fsm > (size_t)80 * 1024;
     const bool tail_shares = tail && ta.wide && (tail_mfma || dtype == TQ_F32) && mfma_shape && stages == 7;
-    // The preparation on the matrix cores shares the launch too (96 sequences of 61 .. 8190 tokens at 40 q / 8 KV heads of 128: a
-    // launch each 98 us, shared 89), but at head_dim 256 only while the card holds it beside the tail: its
-    // workgroups have the tail's registers and LDS there (128 x 2048 at 16 q / 2 KV heads: shared 73.6 us, a launch each 63.9)
-    const bool mfma_prep = tail_mfma && prep_on_matrix_cores(q, dtype, (int64_t)B * Hq, layer, Gq, g_tot);
-    const int rows_tile = (16 / Gq) * Gq;                         // (whole groups of heads, see prep_mfma_body; Gq <= 8)
-    const int n_tiles = (int)(((int64_t)B * Hq + rows_tile - 1) / rows_tile);
-    const bool ww = prep_tile_per_workgroup(n_tiles, d);
-    const int n_mprep = ww ? n_tiles : n_tiles * (d / 32);
-    if (tail_shares && mfma_prep && (d == 128 || n_mprep <= 2 * device_compute_units())) {
+    // 16-bit rows of 256 share while the launch is less than three rounds of the workgroups that a card holds at once.  fp16, 2 KV heads, 128 exact
+    // tokens: 64 x 150, 4 heads each (640 workgroups) 30.2 us, a launch each 31.9; 128 x 150 (1280) 46.7 and 40.2; 8 heads each (2304) 68.0
+    // and 50.5.  Both on the vector ALU, 64 exact tokens: 64 x 150, 8 KV heads of 2 heads (1152) 43.0 us, a launch each 47.1; with 16
+    // 128 x 150, 2 KV heads of 8 (2304) 52.1 and 46.8.  bf16, 128 tokens: 128 x 150, 4 heads each (768) 38.9 and 36.9.
+    // At 128 the preparation on the matrix cores shares the launch at any size (96 sequences of 61 .. 8190 tokens at 40 q / 8 KV heads, fp16: a
+    // launch each 98 us, shared 89).
+    const bool three_rounds = d == 256 && tail_mfma && n_tail + (mfma_prep ? n_mprep : n_prep) >= (words_tail ? 6 : 3) * cus;
+    if (tail_shares && mfma_prep && !three_rounds) {
       size_t fsm = tail_lds, psm = (size_t)prep_mfma_smem_floats() * sizeof(float) * (ww ? 4 : 1);
       if (psm > fsm) fsm = psm;
       if (n_sched && fsm < SCHED_SMEM_INTS * sizeof(int)) fsm = SCHED_SMEM_INTS * sizeof(int);
@@ -1612,25 +1630,30 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
 #undef TQ_LAUNCH_PMT
       TQ_CHECK_LAUNCH();
       tail_done = true;
-    } else if (tail_shares && !mfma_prep && !(one_per_unit && n_tail + n_prep > device_compute_units())) {
-#define TQ_LAUNCH_PT(PER, DT, PAGED)                                                                                 \
+    } else if (tail_shares && !mfma_prep && !three_rounds && !(one_per_unit && n_shared + n_prep > cus)) {
+#define TQ_LAUNCH_PT(PER, DT, PAGED, WORDS)                                                                          \
   {                                                                                                                  \
-    auto kern = prep_gpw > 1 ? prep_tail_kernel<PER, DT, PAGED, true> : prep_tail_kernel<PER, DT, PAGED, false>;     \
+    auto kern = prep_gpw > 1 ? prep_tail_kernel<PER, DT, PAGED, true, WORDS> : prep_tail_kernel<PER, DT, PAGED, false, WORDS>; \
     if (fsm > 48 * 1024) {                                                                                           \
       hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)fsm);   \
       if (e != hipSuccess) return (int)e;                                                                            \
     }                                                                                                                \
-    pf.front = n_tail + n_prep + n_sched;                                                                            \
-    if (pf.front > 2 * device_compute_units()) pf.blocks = 0;                                                        \
-    kern<<<dim3((unsigned)(n_sched + n_tail + n_prep + (pf.blocks > 0 ? pf.n_wg : 0))), dim3(TAIL_THREADS), fsm, st>>>( \
-        ta, n_tail, B, Gq, *layer, q_rot, q_sk, q_stat, qa_pack, fm.counters, prep_gpw, n_tail + n_prep, pf, g_tot, \
+    pf.front = n_shared + n_prep + n_sched;                                                                          \
+    if (pf.front > 2 * cus) pf.blocks = 0;                                                                           \
+    kern<<<dim3((unsigned)(n_sched + n_shared + n_prep + (pf.blocks > 0 ? pf.n_wg : 0))), dim3(TAIL_THREADS), fsm, st>>>( \
+        ta, n_shared, B, Gq, *layer, q_rot, q_sk, q_stat, qa_pack, fm.counters, prep_gpw, n_shared + n_prep, pf, g_tot, \
         decode_mfma_head_rows(d, Gq), plan);                                                                         \
   }
-#define TQ_LAUNCH_PT_DT(PER, PAGED)                                \
-  {                                                                \
-    if (dtype == TQ_BF16) TQ_LAUNCH_PT(PER, TQ_BF16, PAGED)        \
-    else if (dtype == TQ_F16) TQ_LAUNCH_PT(PER, TQ_F16, PAGED)     \
-    else TQ_LAUNCH_PT(PER, TQ_F32, PAGED)                          \
+#define TQ_LAUNCH_PT_DT(PER, PAGED)                                         \
+  {                                                                         \
+    if (dtype == TQ_F32) TQ_LAUNCH_PT(PER, TQ_F32, PAGED, true)             \
+    else if (dtype == TQ_BF16) TQ_LAUNCH_PT(PER, TQ_BF16, PAGED, false)     \
+    else TQ_LAUNCH_PT(PER, TQ_F16, PAGED, false)                            \
+  }
+#define TQ_LAUNCH_PT_WORDS(PAGED)                                           \
+  {                                                                         \
+    if (dtype == TQ_BF16) TQ_LAUNCH_PT(16, TQ_BF16, PAGED, true)            \
+    else TQ_LAUNCH_PT(16, TQ_F16, PAGED, true)                              \
   }
       if (d == 64) {
         if (ts.paged) TQ_LAUNCH_PT_DT(4, true)
@@ -1638,10 +1661,14 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
       } else if (d == 128) {
         if (ts.paged) TQ_LAUNCH_PT_DT(8, true)
         else TQ_LAUNCH_PT_DT(8, false)
+      } else if (words_tail && dtype != TQ_F32) {
+        if (ts.paged) TQ_LAUNCH_PT_WORDS(true)
+        else TQ_LAUNCH_PT_WORDS(false)
       } else {
         if (ts.paged) TQ_LAUNCH_PT_DT(16, true)
         else TQ_LAUNCH_PT_DT(16, false)
       }
+#undef TQ_LAUNCH_PT_WORDS
 #undef TQ_LAUNCH_PT_DT
 #undef TQ_LAUNCH_PT
       TQ_CHECK_LAUNCH();

@@ -327,7 +327,8 @@ __device__ __forceinline__ int64_t key_mfma_body(const void* __restrict__ x, con
   int64_t end = n_tiles;
   if constexpr (SPLIT) {
     const int64_t rounds = n_tiles / ((int64_t)ML * n_wg), whole = rounds * ML * n_wg;
-    if (n_tiles - whole <= (D == 128 ? n_wg : n_wg / 2)) end = whole;
+    const int64_t rest = n_tiles - whole;
+    if (D == 128 ? rest <= n_wg && (rounds <= 1 || rest <= n_wg / 8 || rest > n_wg / 8 * 7) : rest <= n_wg / 2) end = whole;
   }
   const int64_t n_groups = (end - first + ML - 1) / ML;         // a group = the TT vectors of one pass
   if (id >= n_groups) return end;
@@ -785,10 +786,13 @@ static int launch_dt_d(const void* x, const Source& src, const tq_layer& ly, con
   using Gm = KeyGeom<D>;
   using Sm = KeySmem<DT, D>;
   // Few tiles (the page write of a decode step: a token per sequence; a few thousand keys to codes): a workgroup per tile, which
-  // then computes that tile only, while they all fit the card at once.  4096 flat keys of 128 (fp32): 16.9 -> 11.7 us
+  // then computes that tile only: two tiles per compute unit of pages and of 16-bit flat keys of 128 (8192 keys: 15.2 -> 11.8 us), one of flat
+  // keys of 256 and of fp32 (LDS holds one workgroup; 4096 keys of 128 16.9 -> 10.7 us, of 256 26.7 -> 21.6, but 4097 26.4 -> 34.7;
+  // bf16 keys of 256 4096 21.7 -> 19.5, 4097 21.5 -> 24.7)
   if constexpr (ML == Gm::MT && !std::is_same<Source, RaggedSource>::value && !MSE_ONLY) {
     const int opt = opt_append_small.load(std::memory_order_relaxed);
-    if (opt != 0 && tiles <= (opt < 0 ? 2 * (int64_t)device_compute_units() : (int64_t)opt))
+    constexpr int per_cu = std::is_same<Sink, KeyPagedSink>::value || (D == 128 && DT != TQ_F32) ? 2 : 1;
+    if (opt != 0 && tiles <= (opt < 0 ? per_cu * (int64_t)device_compute_units() : (int64_t)opt))
       return launch_dt_d<DT, D, MSE_ONLY, FX, Source, Sink, 1>(x, src, ly, sink, tiles, st);
   }
   auto kern = key_mfma_kernel<DT, D, MSE_ONLY, FX, Source, Sink, ML>;
@@ -1062,9 +1066,10 @@ template <int D, bool QJL, int ML = KeyGeom<D>::MT>
 static int launch_deq_d(const uint8_t* idx, const uint8_t* signs, const void* norms, int norm_dtype, const float* rnorms,
                         int64_t n_vec, const tq_layer& ly, float* out, hipStream_t st) {
   using Sm = DeqSmem<D>;
-  // few vectors: a tile of sixteen per workgroup, by the quantiser's rule.  4096 of 128: 8.8 -> 7.6 us
+  // few vectors: a tile of sixteen per workgroup, up to three tiles on two compute units at 128 (4096 vectors 8.9 -> 7.5 us, 6144 9.4 -> 9.2,
+  // 8192 9.5 -> 10.3), one on each at 256 (3072 14.7 -> 13.5, 4096 level, 4097 14.7 -> 18.4)
   if constexpr (ML > 1)
-    if (n_vec <= 2 * TILE * (int64_t)device_compute_units())
+    if (2 * n_vec <= (D == 128 ? 3 : 2) * TILE * (int64_t)device_compute_units())
       return launch_deq_d<D, QJL, 1>(idx, signs, norms, norm_dtype, rnorms, n_vec, ly, out, st);
   auto kern = dequant_mfma_kernel<D, QJL, ML>;
   static std::atomic<unsigned long long> configured{0};
