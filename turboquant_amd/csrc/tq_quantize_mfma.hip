@@ -251,6 +251,14 @@ __device__ __forceinline__ void plane_bits(uint32_t (&bits)[2][4]) {
     }
 }
 
+// Tiles before the last round of an append, when that round is dealt out a tile each (key_mfma_kernel); else all of them
+template <int D>
+__host__ __device__ __forceinline__ int64_t whole_rounds(int64_t n_tiles, int n_wg) {
+  const int64_t round = (int64_t)KeyGeom<D>::MT * n_wg, rounds = n_tiles / round, rest = n_tiles - rounds * round;
+  const bool by_tile = D == 128 ? rest <= n_wg && (rounds <= 1 || rest <= n_wg / 8 || rest > n_wg / 8 * 7) : rest <= n_wg / 2;
+  return by_tile ? n_tiles - rest : n_tiles;
+}
+
 // MSE_ONLY (the stage-1 quantiser alone: no residual, no signs) is a template parameter: as a
 // run-time flag it adds control flow that costs the register allocator its footing.
 //
@@ -326,9 +334,7 @@ __device__ __forceinline__ int64_t key_mfma_body(const void* __restrict__ x, con
   }
   int64_t end = n_tiles;
   if constexpr (SPLIT) {
-    const int64_t rounds = n_tiles / ((int64_t)ML * n_wg), whole = rounds * ML * n_wg;
-    const int64_t rest = n_tiles - whole;
-    if (D == 128 ? rest <= n_wg && (rounds <= 1 || rest <= n_wg / 8 || rest > n_wg / 8 * 7) : rest <= n_wg / 2) end = whole;
+    end = whole_rounds<D>(n_tiles, n_wg);
   }
   const int64_t n_groups = (end - first + ML - 1) / ML;         // a group = the TT vectors of one pass
   if (id >= n_groups) return end;
@@ -727,15 +733,17 @@ __device__ __forceinline__ int64_t key_mfma_body(const void* __restrict__ x, con
   return end;
 }
 
-template <int DT, int D, bool MSE_ONLY, bool FX, class Source, class Sink, int ML = KeyGeom<D>::MT>
+template <int DT, int D, bool MSE_ONLY, bool FX, class Source, class Sink, int ML = KeyGeom<D>::MT, bool SPLIT = true>
 __global__ void __launch_bounds__(KQ_THREADS, 2)
 key_mfma_kernel(const void* __restrict__ x, Source src, tq_layer ly, Sink sink, int64_t n_tiles) {
   extern __shared__ __align__(16) unsigned char smem[];
-  if constexpr (ML == KeyGeom<D>::MT && std::is_same<Sink, KeyPagedSink>::value && !MSE_ONLY) {
+  if constexpr (SPLIT && ML == KeyGeom<D>::MT && std::is_same<Sink, KeyPagedSink>::value && !MSE_ONLY) {
     // A last round of fewer tiles than workgroups is dealt out a tile each instead of a group to a few of them: the round is as long as
     // a tile then, and not as a group: key kernel, head_dim 128, 8 heads of 4176 tokens (2088 tiles, 512 workgroups of four at a time)
-    // 28.7 -> 23.8 us, of 5120 28.0 -> 27.0, of 8384 39.9 -> 33.7.  At 256, where the matrices of a tile keep its compute unit busy, only up
-    // to a tile per compute unit: 2 heads of 8352 44.6 -> 42.1, of 10240 45.1 -> 43.5 (of 12288, two tiles per compute unit, 47.3 -> 56.2)
+    // 28.7 -> 23.8 us, of 5120 28.0 -> 27.0.  Behind more than one round only an eighth of a round or a nearly whole one: in between the values'
+    // kernel has filled the units that wait (69,632 tokens of a head, call: 51.0 us, by tiles 52.6; 71,680 52.4, 53.4; 73,728 54.3, 51.5).
+    // At 256, where the matrices of a tile keep its compute unit busy, only up to a tile per compute unit: 2 heads of 8352
+    // 44.6 -> 42.1, of 10240 45.1 -> 43.5 (of 12288, two tiles per compute unit, 47.3 -> 56.2)
     const int64_t rest = key_mfma_body<DT, D, MSE_ONLY, FX, Source, Sink, ML, true>(x, src, ly, sink, 0, n_tiles, blockIdx.x, gridDim.x, smem);
     if (rest + blockIdx.x < n_tiles)
       key_mfma_body<DT, D, MSE_ONLY, FX, Source, Sink, 1>(x, src, ly, sink, rest, n_tiles, blockIdx.x, gridDim.x, smem);
@@ -796,6 +804,10 @@ static int launch_dt_d(const void* x, const Source& src, const tq_layer& ly, con
       return launch_dt_d<DT, D, MSE_ONLY, FX, Source, Sink, 1>(x, src, ly, sink, tiles, st);
   }
   auto kern = key_mfma_kernel<DT, D, MSE_ONLY, FX, Source, Sink, ML>;
+  // (a kernel of its own for three and four index bits at 128 where no round is dealt out by tiles, which costs its registers: key kernel, 16,384
+  // vectors of a head 22.2 us alone, 23.5 with the other body in it)
+  constexpr bool ALONE = D == 128 && !FX && !MSE_ONLY && ML == Gm::MT && std::is_same<Sink, KeyPagedSink>::value && !std::is_same<Source, RaggedSource>::value;
+  auto alone = key_mfma_kernel<DT, D, MSE_ONLY, FX, Source, Sink, ML, !ALONE>;
   size_t smem = Sm::bytes;                               // + the index of the existing tiles (first pages, four partial sums)
   if constexpr (std::is_same<Source, RaggedSource>::value) smem += ((size_t)src.B + 1 + KQ_WAVES) * 4;
   constexpr size_t smem_max = Sm::bytes + (RaggedSource::MAX_COMPACT + 1 + KQ_WAVES) * 4;
@@ -803,8 +815,10 @@ static int launch_dt_d(const void* x, const Source& src, const tq_layer& ly, con
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return TQ_EINVAL;
   if (dev >= 64 || !(configured.load() >> dev & 1)) {
-    hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_max);
-    if (e != hipSuccess) return (int)e;
+    for (auto k : {kern, alone}) {
+      hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_max);
+      if (e != hipSuccess) return (int)e;
+    }
     if (dev < 64) configured.fetch_or(1ull << dev);
   }
   // persistent workgroups: as many as stay resident (LDS allows 160 KB / bytes per compute unit)
@@ -818,6 +832,7 @@ static int launch_dt_d(const void* x, const Source& src, const tq_layer& ly, con
   const int64_t groups = (tiles + ML - 1) / ML;
   const int64_t resident = (int64_t)cus * (per_cu > 0 ? per_cu : 1);
   const unsigned grid = (unsigned)(groups < resident ? groups : resident);
+  if (ALONE && whole_rounds<D>(tiles, (int)grid) == tiles) kern = alone;
   hipEvent_t ev_start = nullptr, ev_stop = nullptr;
   if (std::is_same<Sink, KeyPagedSink>::value && take_time_hook(1, ev_start, ev_stop)) {
     hipExtLaunchKernelGGL(kern, dim3(grid), dim3(KQ_THREADS), smem, st, ev_start, ev_stop, 0, x, src, ly, sink, tiles);
