@@ -1459,7 +1459,22 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
   const bool tail_wide = words && ((((uintptr_t)recent_k | (uintptr_t)recent_v) & 15) == 0) &&
                          !((tws_b | tws_r | tws_h | tws_blk) & 3) && (d / epw) / 4 <= TAIL_THREADS;
   // The exact tail on the matrix cores: a workgroup per sixteen heads
-  const bool tail_mfma = tail && tail_wide && epw == 2 && (((uintptr_t)q) & 15) == 0 && tail_mfma_size(d);
+  bool tail_mfma = tail && tail_wide && epw == 2 && (((uintptr_t)q) & 15) == 0 && tail_mfma_size(d);
+  // At head_dim 256 a compute unit holds one workgroup of that tail and of what shares its launch, but two with tail and preparation on the
+  // vector ALU where few exact tokens leave the LDS for them.  Both stay there for such rows, unless the matrix cores prepare them (16-bit rows,
+  // 16 exact tokens, 16 x 150, 2 KV heads of 8 heads, fp16: 24.9 us, with the matrix-core tail 27.2, a launch each 28.5; with 128 tokens, where one
+  // fits, 30.3, 25.1, 30.5; bf16 on the matrix cores, 32 x 150: 29.0 and 28.1) and there are fewer tails than workgroups of the
+  // preparation (64 exact tokens, 24 x 150, 8 KV heads of a head each, bf16: 22.9 us, on the matrix cores 26.4).
+  const int g_tot = kv_div > 1 && G % kv_div ? G : 0;             // groups of unequal size: query heads per KV head
+  const int rows_tile = (16 / Gq) * Gq;                           // (whole groups of heads, see prep_mfma_body; Gq <= 8)
+  const int n_prep_tiles = (int)(((int64_t)B * Hq + rows_tile - 1) / rows_tile);
+  const bool prep_ww = prep_tile_per_workgroup(n_prep_tiles, d);
+  const int n_mprep = prep_ww ? n_prep_tiles : n_prep_tiles * (d / 32);
+  const bool prep_mfma = mfma_shape && prep_on_matrix_cores(q, dtype, (int64_t)B * Hq, layer, Gq, g_tot);
+  if (tail_mfma && mfma_shape && d == 256 && tail_words_smem(d, recent_rows, tail_tile_words(d / epw, recent_rows, true)) <= (size_t)80 * 1024) {
+    const int64_t units = (int64_t)Hkv * B * ((G + 15) / 16);
+    tail_mfma = prep_mfma && (units < n_mprep || units + n_mprep < device_compute_units());
+  }
   // Workgroups per (sequence, KV head, group of TAIL_GC query heads) of the exact tail, each with a share of the
   // exact tokens and a partial of its own.  One such workgroup pulls 2 x recent_rows rows into one compute unit
   // and is the longest-running part of its launch; with few of them and a merge kernel behind (many splits - the
@@ -1560,7 +1575,6 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
     // (in the launch shared with the tail a compute unit holds two workgroups: beyond that the preparation
     // workgroups take several groups of heads each, see prep_query_body)
     // (groups of unequal size - the heads of a KV head do not divide into kv_div groups - take one workgroup each)
-    const int g_tot = kv_div > 1 && G % kv_div ? G : 0;
     const int prep_gpw = g_tot ? 1 : prep_groups_per_workgroup(Gq, n_tail + (int64_t)(B * Hq / Gq) * (d / PREP_COLS),
                                                                2 * (int64_t)device_compute_units());
     const int prep_rows = Gq * prep_gpw;                          // query rows of a preparation workgroup
@@ -1572,24 +1586,8 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
     // (16 x 8192: 48.9 -> 45.2 us per step, 32 x 32768: 223.6 -> 221.5 us).
     const int cus = device_compute_units();
     const int n_sched = plan.items ? SCHED_FRONT : 0;
-    const bool mfma_prep_fits = tail_mfma && prep_on_matrix_cores(q, dtype, (int64_t)B * Hq, layer, Gq, g_tot);
-    const int rows_tile = (16 / Gq) * Gq;                         // (whole groups of heads, see prep_mfma_body; Gq <= 8)
-    const int n_tiles = (int)(((int64_t)B * Hq + rows_tile - 1) / rows_tile);
-    const bool ww = prep_tile_per_workgroup(n_tiles, d);
-    const int n_mprep = ww ? n_tiles : n_tiles * (d / 32);
-    const int n_words = Hkv * B * ((G + TAIL_GC - 1) / TAIL_GC) * t_chunks;
-    const size_t words_lds = tail_words_smem(d, recent_rows, ta.tile_words);
-    // At head_dim 256 a compute unit holds one workgroup of the matrix-core tail and of what shares its launch, but two with tail and preparation on
-    // the vector ALU where few exact tokens leave the LDS for them.  Both stay there while that is so and the launch has more workgroups than the
-    // card has units - rows that the matrix cores do not prepare (fp16, few rows: 16 exact tokens, 16 x 150, 2 KV heads, 8 heads each 24.9 us, with
-    // the matrix-core tail 27.2, a launch each 28.5; with 128 tokens, where one fits, 30.3, 25.1, 30.5), and more tails than preparation
-    // (64 exact tokens, 24 x 150, 8 KV heads of a head each 22.9 us, on the matrix cores 26.4).  The tail alone stays there where a unit of sixteen
-    // heads is a long chain of few workgroups (1 x 150, 128 exact tokens: 24.1 us, 25.4).
-    const bool words_pair = tail_mfma && d == 256 && words_lds <= (size_t)80 * 1024;
-    const bool mfma_prep = mfma_prep_fits && !(words_pair && n_tail >= n_mprep && n_tail + n_mprep >= cus);
-    const bool words_tail = !tail_mfma || (d == 256 && !mfma_prep && (words_pair ? n_tail + n_prep >= cus : G > 8 && n_words + n_prep <= cus));
-    const int n_shared = words_tail ? n_words : n_tail;
-    size_t fsm = words_tail ? words_lds : tail_lds;
+    const bool mfma_prep = tail_mfma && prep_mfma;
+    size_t fsm = tail_lds;
     if (prep_smem_bytes(prep_rows, d) > fsm) fsm = prep_smem_bytes(prep_rows, d);
     if (n_sched && fsm < SCHED_SMEM_INTS * sizeof(int)) fsm = SCHED_SMEM_INTS * sizeof(int);
     // ... unless the tail's tiles leave room for one workgroup per compute unit only (fp32 rows, 139 KB at head_dim 128 with 128
@@ -1597,16 +1595,16 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
     // workgroups would queue behind that LDS size too (measured when 16-bit rows of 256 took as much: 128 x 2048, 16 q / 2 KV heads
     // 109.7 us per step in one launch, 88.1 in two)
     const bool one_per_unit = fsm > (size_t)80 * 1024;
-    const bool tail_shares = tail && ta.wide && (tail_mfma || dtype == TQ_F32) && mfma_shape && stages == 7;
+    const bool tail_shares = tail && ta.wide && (tail_mfma || dtype == TQ_F32 || d == 256) && mfma_shape && stages == 7;
     // 16-bit rows of 256 share while the launch is less than three rounds of the workgroups that a card holds at once.  fp16, 2 KV heads, 128 exact
     // tokens: 64 x 150, 4 heads each (640 workgroups) 30.2 us, a launch each 31.9; 128 x 150 (1280) 46.7 and 40.2; 8 heads each (2304) 68.0
     // and 50.5.  Both on the vector ALU, 64 exact tokens: 64 x 150, 8 KV heads of 2 heads (1152) 43.0 us, a launch each 47.1; with 16
     // 128 x 150, 2 KV heads of 8 (2304) 52.1 and 46.8.  bf16, 128 tokens: 128 x 150, 4 heads each (768) 38.9 and 36.9.
     // At 128 the preparation on the matrix cores shares the launch at any size (96 sequences of 61 .. 8190 tokens at 40 q / 8 KV heads, fp16: a
     // launch each 98 us, shared 89).
-    const bool three_rounds = d == 256 && tail_mfma && n_tail + (mfma_prep ? n_mprep : n_prep) >= (words_tail ? 6 : 3) * cus;
+    const bool three_rounds = d == 256 && epw == 2 && n_tail + (mfma_prep ? n_mprep : n_prep) >= (tail_mfma ? 3 : 6) * cus;
     if (tail_shares && mfma_prep && !three_rounds) {
-      size_t fsm = tail_lds, psm = (size_t)prep_mfma_smem_floats() * sizeof(float) * (ww ? 4 : 1);
+      size_t fsm = tail_lds, psm = (size_t)prep_mfma_smem_floats() * sizeof(float) * (prep_ww ? 4 : 1);
       if (psm > fsm) fsm = psm;
       if (n_sched && fsm < SCHED_SMEM_INTS * sizeof(int)) fsm = SCHED_SMEM_INTS * sizeof(int);
       pf.front = n_tail + n_mprep + n_sched;
@@ -1620,17 +1618,17 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
       hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)fsm);     \
       if (e != hipSuccess) return (int)e;                                                                              \
     }                                                                                                                  \
-    kern<<<pgrid, dim3(TAIL_THREADS), fsm, st>>>(ta, n_tail, B, Gq, *layer, q_stat, qa_pack, fm.counters, n_tiles,      \
+    kern<<<pgrid, dim3(TAIL_THREADS), fsm, st>>>(ta, n_tail, B, Gq, *layer, q_stat, qa_pack, fm.counters, n_prep_tiles, \
                                                  n_tail + n_mprep, pf, decode_mfma_head_rows(d, Gq), plan);            \
   }
-      if (d == 128 && ww) TQ_LAUNCH_PMT(128, true)
+      if (d == 128 && prep_ww) TQ_LAUNCH_PMT(128, true)
       else if (d == 128) TQ_LAUNCH_PMT(128, false)
-      else if (ww) TQ_LAUNCH_PMT(256, true)
+      else if (prep_ww) TQ_LAUNCH_PMT(256, true)
       else TQ_LAUNCH_PMT(256, false)
 #undef TQ_LAUNCH_PMT
       TQ_CHECK_LAUNCH();
       tail_done = true;
-    } else if (tail_shares && !mfma_prep && !three_rounds && !(one_per_unit && n_shared + n_prep > cus)) {
+    } else if (tail_shares && !mfma_prep && !three_rounds && !(one_per_unit && n_tail + n_prep > cus)) {
 #define TQ_LAUNCH_PT(PER, DT, PAGED, WORDS)                                                                          \
   {                                                                                                                  \
     auto kern = prep_gpw > 1 ? prep_tail_kernel<PER, DT, PAGED, true, WORDS> : prep_tail_kernel<PER, DT, PAGED, false, WORDS>; \
@@ -1638,10 +1636,10 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
       hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)fsm);   \
       if (e != hipSuccess) return (int)e;                                                                            \
     }                                                                                                                \
-    pf.front = n_shared + n_prep + n_sched;                                                                          \
+    pf.front = n_tail + n_prep + n_sched;                                                                            \
     if (pf.front > 2 * cus) pf.blocks = 0;                                                                           \
-    kern<<<dim3((unsigned)(n_sched + n_shared + n_prep + (pf.blocks > 0 ? pf.n_wg : 0))), dim3(TAIL_THREADS), fsm, st>>>( \
-        ta, n_shared, B, Gq, *layer, q_rot, q_sk, q_stat, qa_pack, fm.counters, prep_gpw, n_shared + n_prep, pf, g_tot, \
+    kern<<<dim3((unsigned)(n_sched + n_tail + n_prep + (pf.blocks > 0 ? pf.n_wg : 0))), dim3(TAIL_THREADS), fsm, st>>>( \
+        ta, n_tail, B, Gq, *layer, q_rot, q_sk, q_stat, qa_pack, fm.counters, prep_gpw, n_tail + n_prep, pf, g_tot, \
         decode_mfma_head_rows(d, Gq), plan);                                                                         \
   }
 #define TQ_LAUNCH_PT_DT(PER, PAGED)                                         \
@@ -1661,7 +1659,7 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
       } else if (d == 128) {
         if (ts.paged) TQ_LAUNCH_PT_DT(8, true)
         else TQ_LAUNCH_PT_DT(8, false)
-      } else if (words_tail && dtype != TQ_F32) {
+      } else if (!tail_mfma && dtype != TQ_F32) {
         if (ts.paged) TQ_LAUNCH_PT_WORDS(true)
         else TQ_LAUNCH_PT_WORDS(false)
       } else {
