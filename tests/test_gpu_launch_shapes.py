@@ -473,6 +473,33 @@ def test_sixteen_heads_per_wavefront_and_slots_without_tokens(gpu, case):
     assert torch.equal(pool.decode_attention(q, bad, seq, n_split=1, max_len=N), pool.decode_attention(q, table, short, n_split=1, max_len=N))
 
 
+@pytest.mark.parametrize("d", [512, 576])
+def test_sixteen_heads_per_wavefront_of_two_sequences_and_slots_without_tokens(gpu, d):
+    """The same with a second sequence beside it: one alone in few splits takes the kernel of 8 heads per workgroup, whose results it has to
+    within the rounding of the weighted scales (2^-9 each)."""
+    Hq, N = 32, 200
+    pool, tq = _make_pool(gpu, d, 4, 4, 1, 16, torch.bfloat16)
+    g = torch.Generator().manual_seed(5)
+    k, v = (torch.randn(1, N, 1, d, generator=g).bfloat16().to(gpu) for _ in range(2))
+    q = torch.randn(1, Hq, d, generator=g).bfloat16().to(gpu).expand(2, Hq, d).contiguous()
+    table = torch.arange(13, dtype=torch.int32, device=gpu)[None].repeat(2, 1)
+    pool.append(k, v, table[:1])
+    both = lambda t, lens, n=2: pool.decode_attention(q, t, _i32(lens, gpu), n_split=n, max_len=N)
+    want = both(table, [N, 31])
+    one = pool.decode_attention(q[:1], table[:1], _i32([N], gpu), n_split=2, max_len=N)
+    assert float((one[0].float() - want[0].float()).abs().max()) <= 2.0 ** -7 * float(one.float().abs().max())
+    L = pool.layout
+    page = pool.data[12, 0]                                       # tokens 192 .. 207, eight of them written
+    page[L.off_meta + 64:L.off_meta + 128] = 0xff
+    for off in (L.off_vscale, L.off_vzero):
+        page[off:off + 2 * (d // 32) * 16].view(torch.int16).view(d // 32, 16)[:, 8:] = 0x7f80
+    assert torch.equal(both(table, [N, 31]), want)
+    bad = table.clone()
+    bad[0, 12], bad[1] = -1, 99
+    assert torch.equal(both(bad, [N, 31], 1)[0], both(table, [192, 31], 1)[0])
+    assert torch.count_nonzero(both(bad, [N, 31])[1]) == 0
+
+
 @pytest.mark.parametrize("d,Hq,B,dtype", [(576, 8, 40, torch.bfloat16), (576, 5, 53, torch.float16), (704, 8, 33, torch.bfloat16),
                                           (320, 7, 80, torch.bfloat16), (576, 128, 3, torch.bfloat16), (576, 128, 17, torch.float16),
                                           (512, 100, 21, torch.bfloat16), (640, 3, 200, torch.float16)])

@@ -524,8 +524,22 @@ def test_short_contexts_of_many_heads_are_split_by_turns():
                 each = -(-turns // n)
                 assert 1 <= n <= min(most, turns) and (n - 1) * each < turns <= n * each
                 assert each == 1 or (turns > most or turns > 40 * side) and (each <= 4 or -(-turns // most) == each)
-    assert [pool.default_splits(1, N, 16) for N in (1, 500, 8192, 65536)] == [1, 3, 64, 128]
-    assert pool.default_splits(1, 500, 8) == 1 and pool.default_splits(1, 8192, 64) == 64
+
+
+@pytest.mark.parametrize("d,turns", [(576, 24), (512, 8)])
+def test_one_sequence_of_many_heads_takes_groups_of_eight_while_they_are_short(d, turns):
+    """Workgroups of 8 heads that the card holds at once, none without tokens, up to a number of turns; longer contexts of more than sixteen
+    heads take so many splits that the library runs the kernel of sixteen heads per wavefront pair."""
+    pool = _paper_pool(d, 1)
+    for G in (9, 16, 17, 24, 32, 33, 40, 48, 57, 64, 65, 72, 80, 100, 128):
+        groups = -(-G // 8)
+        for N in (1, 31, 33, 64, 300, 1000, 2000, 4000, 8192, 13000, 16384, 21800, 32768, 65536, 131072):
+            n, blocks = pool.default_splits(1, N, G), -(-N // 32)
+            if G <= 16 or -(-blocks * groups // 256) <= turns:
+                assert 1 <= n <= min(blocks, 128) and n * groups <= 256
+            else:
+                assert n * groups > 256
+    assert pool.default_splits(1, 500, 8) == 1
 
 
 @pytest.mark.parametrize("d", [64, 128, 256, 320, 512, 576])
@@ -553,4 +567,4 @@ def test_splits_of_many_heads_in_the_static_area():
                     n, free = pool.default_splits(B, N, Hq, True), pool.default_splits(B, N, Hq)
                     assert n == free or 1 <= n < free and need(B, Hq, n + 1) > _ffi.NOALLOC_SCRATCH_BYTES
                     assert n == 1 or need(B, Hq, n) <= _ffi.NOALLOC_SCRATCH_BYTES
-        assert pool.default_splits(1, 8192, 128, True) >= 32
+        assert pool.default_splits(1, 65536, 128, True) >= 32 and pool.default_splits(1, 8192, 128, True) >= 16

@@ -1515,7 +1515,7 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
     wide_pre.Hq = Hq; wide_pre.Hkv = Hkv; wide_pre.kv_div = kv_div; wide_pre.ntp = decode_wide_term_planes(*layer);
     wide_pre.sm_scale = sm_scale;
     // more than 8 heads per KV head at the sizes of latent attention: tiles of sixteen heads for a kernel of their own
-    if (decode_heads_has_kernel(*layer, *layout, G, (int64_t)B * Hkv) && (G + 15) / 16 * heads_qa_words(d) <= kv_div * wide_pre.ntp * 2 * wide_qa_stride(d)) {
+    if (decode_heads_has_kernel(*layer, *layout, G, (int64_t)B * Hkv, n_split) && (G + 15) / 16 * heads_qa_words(d) <= kv_div * wide_pre.ntp * 2 * wide_qa_stride(d)) {
       wide_pre.heads = true;
       wide_pre.kv_div = (G + 15) / 16;
       wide_pre.ntp = 2;

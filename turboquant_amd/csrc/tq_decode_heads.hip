@@ -509,12 +509,13 @@ decode_heads_kernel(const uint32_t* __restrict__ qa, const float* __restrict__ q
 }
 
 // Whether a step of this shape runs the kernel above: more than 8 query heads per KV head, head_dim 512 / 576, 3- or 4-bit
-// keys, 2- or 4-bit values, the page layout the library makes.  Not up to sixteen heads of one sequence on one KV head (pairs: their product),
-// where the two groups of 8 heads of the other kernel take a compute unit each and its turns are shorter
-// (16 heads of 576, 4-bit, best split counts of either: 500 tokens 23 us there, 30 here; 8192 33 / 40; 32768 47 / 53; four sequences
-// of 8192 37 / 42, of 32768 73 / 63).
-bool decode_heads_has_kernel(const tq_layer& ly, const tq_page_layout& L, int g_tot, int64_t pairs) {
-  if (opt_wide_heads.load(std::memory_order_relaxed) == 0 || g_tot <= 8 || g_tot > 128 || (g_tot <= 16 && pairs <= 1)) return false;
+// keys, 2- or 4-bit values, the page layout the library makes.  Not one sequence on one KV head (pairs: their product) whose splits of 8 heads each
+// the card holds at once: the other kernel's groups of 8 heads take a compute unit each then, and their turns are shorter
+// (576, 4-bit, best split counts of either, there / here: 16 heads x 8192 32 / 40 us, x 32768 47 / 53; 64 heads x 300 22.5 / 27.3, x 8192
+// 37 / 45, x 16384 49 / 55; two sequences fill the card here).
+bool decode_heads_has_kernel(const tq_layer& ly, const tq_page_layout& L, int g_tot, int64_t pairs, int n_split) {
+  if (opt_wide_heads.load(std::memory_order_relaxed) == 0 || g_tot <= 8 || g_tot > 128) return false;
+  if (pairs <= 1 && (g_tot <= 16 || n_split * ((g_tot + 7) / 8) <= device_compute_units())) return false;
   if ((ly.d != 512 && ly.d != 576) || L.d != ly.d || (ly.mse_bits != 2 && ly.mse_bits != 3) || L.mse_bits != ly.mse_bits) return false;
   if ((L.value_bits != 2 && L.value_bits != 4) || L.group_size != 32 || (L.dtype != TQ_BF16 && L.dtype != TQ_F16)) return false;
   int nx = 0;

@@ -173,7 +173,7 @@ constexpr int HQ_OP = 64 * 6;
 __host__ __device__ constexpr int heads_qa_words(int d) { return 4 * (d / 64) * HQ_OP; }     // dwords per tile of sixteen heads
 
 // The matrix-core kernel for more than 8 query heads per KV head at head_dim 512 / 576 (tq_decode_heads.hip)
-bool decode_heads_has_kernel(const tq_layer& ly, const tq_page_layout& L, int g_tot, int64_t pairs);
+bool decode_heads_has_kernel(const tq_layer& ly, const tq_page_layout& L, int g_tot, int64_t pairs, int n_split);
 int launch_decode_heads(int B, int Hq, int Hkv, const uint8_t* pool, const int32_t* block_table, int bt_stride,
                         const int32_t* seq_lens, const tq_layer& ly, const tq_page_layout& L, float* parts, int n_parts,
                         int n_split, int len_sub, int max_pages, int num_pages, const WidePack& pre, hipStream_t st);

@@ -199,13 +199,16 @@ class PagedKVPool:
                 (Hq is None or 8 < Hq // self.num_kv_heads <= 128) and self.page_kernel() == 2)
 
     @staticmethod
-    def _head_tile_splits(pairs: int, max_len: int, heads: int) -> int:
+    def _head_tile_splits(pairs: int, max_len: int, heads: int, d: int) -> int:
         """Split count of such a step: `pairs` sequences x KV heads, `heads` query heads on each."""
-        tiles = (heads + 15) // 16
-        if tiles == 1 and pairs == 1:
-            # the kernel of 8 heads per workgroup: two groups, four blocks of 32 tokens each (16 heads: 1 x 500 44 us with one split,
-            # 26 with 4; 1 x 8192 44 with 16, 33 with 64; 1 x 32768 51 with 64, 47 with 128, 64 with 192)
-            return max(1, min(128, max_len // 128))
+        tiles, blocks, groups8 = (heads + 15) // 16, max(1, (max_len + 31) // 32), (heads + 7) // 8
+        if pairs == 1 and (tiles == 1 or (blocks * groups8 + 255) // 256 <= (24 if d == 576 else 8)):
+            # One sequence: groups of 8 heads in workgroups of their own, all of which the card holds at once (256; by that the library knows
+            # which kernel is meant), up to 24 turns of 32 tokens (head_dim 512: 8); a few turns each, as the merge reads every split.
+            # 576, 4-bit, this way / sixteen heads per wavefront pair: 64 heads x 300 22.5 / 27.3 us, x 2000 27.5 / 33.2, x 8192 37 / 45, x 16384
+            # 49 / 55, x 32768 (32 turns) 72 / 69; 40 x 32768 59 / 66; 32 x 65536 (32) 75 / 71; 512: 64 x 8192 34.7 / 36.5, 24 x 32768 (12) 42 / 37
+            few, per = (16, 4) if d == 576 else (32, 2)
+            return min(128, max(1, 256 // groups8), blocks, max(few, (blocks + per - 1) // per))
         # Up to four tiles of sixteen heads on the same pages (with two, two blocks of 32 tokens side by side, with one, three); one workgroup
         # per compute unit.  A short context is a chain of turns (3.3 us each): up to 40 blocks side by side in the grid a workgroup takes one turn;
         # beyond, four, as the merge reads every split (576, 4-bit: 64 heads 1 x 200 47 us with one split, 30 with 4; 128 heads
@@ -226,9 +229,9 @@ class PagedKVPool:
         pairs = max(1, B * self.num_kv_heads)
         if Hq is None and not static_scratch and self._head_tiles_shape(None):
             return max(self.default_splits(B, max_len, self.num_kv_heads),
-                       *(self._head_tile_splits(pairs, max_len, heads) for heads in (16, 32, 64)))
+                       *(self._head_tile_splits(pairs, max_len, heads, self.head_dim) for heads in (*range(16, 65, 8), 128)))
         if Hq is not None and self._head_tiles_shape(Hq):
-            n = self._head_tile_splits(pairs, max_len, Hq // self.num_kv_heads)
+            n = self._head_tile_splits(pairs, max_len, Hq // self.num_kv_heads, self.head_dim)
             return self._splits_in_static_scratch(B, Hq, n) if static_scratch else n
         if self.head_dim > 256 and self.page_kernel() == 2:
             # head sizes above 256: one workgroup per compute unit, a block of 32 tokens at a time; each workgroup
