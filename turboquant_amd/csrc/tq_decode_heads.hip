@@ -25,8 +25,9 @@
 // Bound: instruction issue.  A block costs a SIMD 90 score and 38 value MFMAs (3,500 clocks of its matrix unit) and 1,040 vector
 // instructions; a 32 x 32 MFMA holds a wavefront's issue for 13 of its 32 clocks and a vector instruction for 4, so the two roles
 // together issue for about 6,000 clocks, and take 7,000 - 8,000.  A lone wavefront issues once in five clocks at best: with both roles
-// in one wavefront of 512 registers a block took 10,000.  16 x 8192 tokens, 128 heads of 576, 4-bit keys and values: page kernel
-// 411 -> 143 us with 8 splits, 64 heads 73 us, 32 heads 48, 16 heads 44 (kernel of 8 heads per workgroup: 16 heads 62).
+// in one wavefront of 512 registers a block took 10,000.  16 x 8192 tokens of 576, 4-bit keys and values, page kernel: 128 heads
+// 411 -> 154 us on average of twenty steps behind the filling of the pool (shortest 146; 125 in a run of hundreds), 64 heads 69, 32 heads 45,
+// 16 heads 42.  Steps: 451 -> 160, 236 -> 93, 128 -> 63, 75 -> 57.
 
 #include "tq_decode_mfma_impl.h"
 

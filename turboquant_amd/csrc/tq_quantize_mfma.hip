@@ -740,10 +740,10 @@ key_mfma_kernel(const void* __restrict__ x, Source src, tq_layer ly, Sink sink, 
   if constexpr (SPLIT && ML == KeyGeom<D>::MT && std::is_same<Sink, KeyPagedSink>::value && !MSE_ONLY) {
     // A last round of fewer tiles than workgroups is dealt out a tile each instead of a group to a few of them: the round is as long as
     // a tile then, and not as a group: key kernel, head_dim 128, 8 heads of 4176 tokens (2088 tiles, 512 workgroups of four at a time)
-    // 28.7 -> 23.8 us, of 5120 28.0 -> 27.0.  Behind more than one round only an eighth of a round or a nearly whole one: in between the values'
+    // 31.0 -> 26.1 us, of 5120 31.6 -> 30.2.  Behind more than one round only an eighth of a round or a nearly whole one: in between the values'
     // kernel has filled the units that wait (69,632 tokens of a head, call: 51.0 us, by tiles 52.6; 71,680 52.4, 53.4; 73,728 54.3, 51.5).
     // At 256, where the matrices of a tile keep its compute unit busy, only up to a tile per compute unit: 2 heads of 8352
-    // 44.6 -> 42.1, of 10240 45.1 -> 43.5 (of 12288, two tiles per compute unit, 47.3 -> 56.2)
+    // 48.8 -> 46.8, of 10240 (that many) level (of 12288, two tiles per compute unit, 47.3 -> 56.2)
     const int64_t rest = key_mfma_body<DT, D, MSE_ONLY, FX, Source, Sink, ML, true>(x, src, ly, sink, 0, n_tiles, blockIdx.x, gridDim.x, smem);
     if (rest + blockIdx.x < n_tiles)
       key_mfma_body<DT, D, MSE_ONLY, FX, Source, Sink, 1>(x, src, ly, sink, rest, n_tiles, blockIdx.x, gridDim.x, smem);

@@ -211,9 +211,8 @@ class PagedKVPool:
             return min(128, max(1, 256 // groups8), blocks, max(few, (blocks + per - 1) // per))
         # Up to four tiles of sixteen heads on the same pages (with two, two blocks of 32 tokens side by side, with one, three); one workgroup
         # per compute unit.  A short context is a chain of turns (3.3 us each): up to 40 blocks side by side in the grid a workgroup takes one turn;
-        # beyond, four, as the merge reads every split (576, 4-bit: 64 heads 1 x 200 47 us with one split, 30 with 4; 128 heads
-        # 1 x 8192 80 with 16, 51 with 64; 16 heads 4 x 1024 53 with 2, 30 with 11; 4 x 8192 55 with 16, 42 with 64;
-        # 128 heads 16 x 8192 167 with 8, 176 with 16, 260 with 4)
+        # beyond, four, as the merge reads every split (576, 4-bit: 16 heads 4 x 1024 53 us with 2 splits, 30 with 11; 4 x 8192 55 with
+        # 16, 42 with 64; 128 heads 16 x 8192 167 with 8, 176 with 16, 260 with 4)
         groups, side = ((tiles + 3) // 4, 1) if tiles >= 3 else (1, 4 - tiles)
         turns = max(1, (max_len + 32 * side - 1) // (32 * side))
         n = min(max(1, 256 // (pairs * groups)), max(min(turns, 40 * side), (turns + 3) // 4), 512)
