@@ -14,7 +14,8 @@
 //     as the value product wants them: the weights go to the same lane of the partner.
 //   * values: channels as rows, heads as columns; codes masked in place are bf16 denormals (row operand),
 //     weight x group scale is the column operand, one product for the two channel tiles of a group.  Zero points: one more
-//     product with the groups as rows.
+//     product with the groups as rows.  Where head tiles stand side by side a value wavefront sums two of them over half the channels:
+//     codes are unpacked and scales widened once for both, 400 vector instructions a block instead of 580.
 //   * softmax: a lane holds 8 scores of ONE head, every accumulator of a lane belongs to that head, so the running reference
 //     and its rare moves are per-lane scalars.
 // A workgroup of HW x TW pairs walks a range of tokens: HW head tiles side by side on the same pages (four: 64 heads
@@ -22,12 +23,16 @@
 // two of values, filled by LDS-direct loads that the value wavefronts spread over their turn (one occupies the
 // compute unit's address path for about 64 clocks, and a wavefront that issues several in a row waits for that).
 //
-// Bound: instruction issue.  A block costs a SIMD 90 score and 38 value MFMAs (3,500 clocks of its matrix unit) and 1,040 vector
-// instructions; a 32 x 32 MFMA holds a wavefront's issue for 13 of its 32 clocks and a vector instruction for 4, so the two roles
-// together issue for about 6,000 clocks, and take 7,000 - 8,000.  A lone wavefront issues once in five clocks at best: with both roles
-// in one wavefront of 512 registers a block took 10,000.  16 x 8192 tokens of 576, 4-bit keys and values, page kernel: 128 heads
-// 411 -> 154 us on average of twenty steps behind the filling of the pool (shortest 146; 125 in a run of hundreds), 64 heads 69, 32 heads 45,
-// 16 heads 42.  Steps: 451 -> 160, 236 -> 93, 128 -> 63, 75 -> 57.
+// Bound: instruction issue.  A block costs a SIMD 90 score and 38 value MFMAs (3,500 clocks of its matrix unit) and 860 vector
+// instructions; an MFMA holds a wavefront's issue for about 13 clocks and a vector instruction for 4, so the two roles
+// together issue for about 5,100 clocks, and take 6,700 - 7,700 (at 1.8 - 2.1 GHz, where the fp4 x fp6 products leave the card).  Without the
+// value wavefronts' work the kernel takes 113 us of its 137, without the scores' 87; the page requests and the masks of the bit
+// planes cost nothing.  A lone wavefront issues once in five clocks at best: with both roles
+// in one wavefront of 512 registers a block took 10,000.  16 x 8192 tokens of 576, 4-bit keys and values, page kernel of 128 heads, average of sixty
+// steps: 411 us with the kernel of 8 heads, 150 - 157 with a head tile per value wavefront and one sum per plane (its registers spilled), 138 now.
+// Steps: 128 heads 172 -> 165 (166 -> 157 on another card), 64 heads 105 -> 102, 32 heads 72 -> 66, 16 heads (one tile, as before) 60.
+// Measured and not kept: a plane's words read a pair of planes ahead 138, requests in the first half of a turn 137 - 141, the scores' wavefronts
+// first at issue 141 - 145.
 
 #include "tq_decode_mfma_impl.h"
 
@@ -57,6 +62,8 @@ __host__ __device__ constexpr HeadsGeom heads_geom(int d, int mb, int vb) {
 // pairs of wavefronts of a workgroup: head tiles side by side x blocks side by side
 constexpr int heads_hw(int tiles) { return tiles >= 3 ? 4 : tiles; }
 constexpr int heads_tw(int hw) { return hw == 4 ? 1 : 4 - hw; }
+// head tiles that a value wavefront sums (it takes as small a part of the channels)
+constexpr int heads_vt(int hw) { return hw >= 2 ? 2 : 1; }
 // LDS: sketched queries of the head tiles, two turns of key and of value parts, the weights a pair hands over
 constexpr int heads_qs_bytes(int d, int hw) { return hw * 2 * (d / 64) * HQ_OP * 4; }
 constexpr int HD_HAND = 9 * 64;            // floats of a pair's hand-over: 8 weights and the reference's move per lane
@@ -80,10 +87,10 @@ decode_heads_kernel(const uint32_t* __restrict__ qa, const float* __restrict__ q
                     const int32_t* __restrict__ seq_lens, tq_layer ly, float* __restrict__ parts, int n_parts, int n_split,
                     int len_sub, int max_pages, int num_pages) {
   constexpr int TW = heads_tw(HW), NP = HW * TW;                   // pairs of wavefronts
-  constexpr int NX = MB == 3 ? 1 : 0, NC = D / 64, W = D / 32, NG = D / 32, NZ = (NG + 15) / 16;
+  constexpr int NX = MB == 3 ? 1 : 0, NC = D / 64, W = D / 32, NG = D / 32;
   constexpr HeadsGeom GC = heads_geom(D, MB, VB);
   static_assert(VB == 2 || VB == 4, "2- and 4-bit values");
-  static_assert(MB == 2 || MB == 3, "3- and 4-bit keys");
+  static_assert(MB == 2 || MB == 3, "3- and 4-bit keys: an even number of index planes and multi-bit terms");
   static_assert(heads_smem(D, MB, VB, HW) <= 160 * 1024, "LDS");
   static_assert(heads_smem(D, MB, VB, HW) >= sizeof(float) * (NP * (NG * 16 + 128) + HW * (TW - 1) * 2 * NG * 256), "room for the sums handed over at the end");
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -263,42 +270,57 @@ decode_heads_kernel(const uint32_t* __restrict__ qa, const float* __restrict__ q
           }
           return *(const uint32_t*)(kp + ((p * W + 2 * c + half) * 16 + n) * 4);
         };
-        f32x16 s_sgn, s_idx, u;
+        f32x16 s_idx, u[2];
         uint32_t kx[NC];
+        auto mfma2 = [&](auto sel_c, uint32_t x, const i32x6& qv, f32x16 c) __attribute__((always_inline)) {
+          return mfma_keys<decltype(sel_c)::value>(x & 0x11111111u, x & 0x22222222u, x & 0x44444444u, (x >> 3) & 0x11111111u, qv, c, sq);
+        };
+        // Two sums at a time, their products in turn, so that a product need not wait for the one before it.
 #pragma unroll
-        for (int i = 0; i < 16; ++i) { s_sgn[i] = 0.0f; s_idx[i] = 0.0f; }
+        for (int p = 0; p < MB + NX; p += 2) {                     // the index planes and the multi-bit term, in pairs
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {                             // the sign plane
+          for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) u[k][i] = 0.0f;
+#pragma unroll
+          for (int c = 0; c < NC; ++c) {
+            uint32_t x[2];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+              if (p + k == MB) x[k] = kx[c];
+              else {
+                x[k] = word(p + k, c);
+                if (NX) kx[c] = p + k == 0 ? x[k] & xmask[0] : kx[c] ^ (x[k] & xmask[p + k]);
+              }
+            }
+            u[0] = mfma2(std::integral_constant<int, 0>{}, x[0], Q[0][c], u[0]);
+            u[1] = mfma2(std::integral_constant<int, 0>{}, x[1], Q[0][c], u[1]);
+            u[0] = mfma2(std::integral_constant<int, 1>{}, x[0], Q[1][c], u[0]);
+            u[1] = mfma2(std::integral_constant<int, 1>{}, x[1], Q[1][c], u[1]);
+          }
+#pragma unroll
+          for (int i = 0; i < 16; ++i) s_idx[i] = fmaf(coef[p + 1], u[1][i], p == 0 ? coef[0] * u[0][i] : fmaf(coef[p], u[0][i], s_idx[i]));
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) u[k][i] = 0.0f;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {                             // the sign plane, a sum per term pair
           const uint32_t x = word(MB, c);
-          const uint32_t b0 = x & 0x11111111u, b1 = x & 0x22222222u, b2 = x & 0x44444444u, b3 = (x >> 3) & 0x11111111u;
 #pragma unroll
           for (int tp = 0; tp < 2; ++tp) {
             const unsigned char* op = q_lds + (tp * NC + c) * (HQ_OP * 4);
             const u32x4 lo = *(const u32x4*)op;
             const uint2 hi = *(const uint2*)(op + 1024 - lane * 8);
             const i32x6 qv = {(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi.x, (int)hi.y};
-            s_sgn = tp ? mfma_keys<3>(b0, b1, b2, b3, qv, s_sgn, sq) : mfma_keys<2>(b0, b1, b2, b3, qv, s_sgn, sq);
+            if (tp) u[1] = mfma2(std::integral_constant<int, 3>{}, x, qv, u[1]);
+            else u[0] = mfma2(std::integral_constant<int, 2>{}, x, qv, u[0]);
           }
         }
+        f32x16 s_sgn;
 #pragma unroll
-        for (int p = 0; p < MB + NX; ++p) {                        // the index planes, then the multi-bit term
-#pragma unroll
-          for (int i = 0; i < 16; ++i) u[i] = 0.0f;
-#pragma unroll
-          for (int c = 0; c < NC; ++c) {
-            uint32_t x;
-            if (p == MB) x = kx[c];
-            else {
-              x = word(p, c);
-              if (NX) kx[c] = p == 0 ? x & xmask[0] : kx[c] ^ (x & xmask[p]);
-            }
-            const uint32_t b0 = x & 0x11111111u, b1 = x & 0x22222222u, b2 = x & 0x44444444u, b3 = (x >> 3) & 0x11111111u;
-            u = mfma_keys<0>(b0, b1, b2, b3, Q[0][c], u, sq);
-            u = mfma_keys<1>(b0, b1, b2, b3, Q[1][c], u, sq);
-          }
-#pragma unroll
-          for (int i = 0; i < 16; ++i) s_idx[i] = fmaf(coef[p], u[i], s_idx[i]);
-        }
+        for (int i = 0; i < 16; ++i) s_sgn[i] = u[0][i] + u[1][i];
         // register i of lane (column head + 16 t, half h) is token 8 (i / 4) + 4 h + i % 4; a head's two columns are
         // neighbouring rows of lanes.  The swap of registers i and i + 8 between them leaves lane row kb with tokens
         // 4 (kb / 2) + i % 4 + 8 (i / 4) of page kb % 2, i = 0..7, and both columns' sums of them.
@@ -358,13 +380,24 @@ decode_heads_kernel(const uint32_t* __restrict__ qa, const float* __restrict__ q
   }
 
   // ================================================================== values
+  // A value wavefront takes VT head tiles of its block and 1 / VT of the channels: codes are unpacked and scales widened once for both
+  // tiles, with as many accumulators as one tile of all channels.
+  constexpr int VT = heads_vt(HW), NGV = NG / VT, NZ = (NGV + 15) / 16;
+  static_assert(NG % VT == 0, "whole groups of channels");
+  const int part = hw % VT, vpair = pair - part;                   // channels; first pair whose weights are read
+  const int g0 = part * NGV, vtile = tile - part;
+  const bool vlive = vtile < n_tiles;                              // (the second tile may lack heads: its sums are dropped)
+  const float* vhand = hand - part * HD_HAND;
   // (the longer of the two roles, and the younger wavefronts, which a SIMD serves last)
   __builtin_amdgcn_s_setprio(2);
-  f32x4 acc[2 * NG], zacc[NZ];
+  f32x4 acc[VT][2 * NGV], zacc[VT][NZ];
 #pragma unroll
-  for (int c = 0; c < 2 * NG; ++c) acc[c] = f32x4{0, 0, 0, 0};
+  for (int v = 0; v < VT; ++v) {
 #pragma unroll
-  for (int c = 0; c < NZ; ++c) zacc[c] = f32x4{0, 0, 0, 0};
+    for (int c = 0; c < 2 * NGV; ++c) acc[v][c] = f32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int c = 0; c < NZ; ++c) zacc[v][c] = f32x4{0, 0, 0, 0};
+  }
   for (int k = 0; k < NR; ++k) request(k, -2);                     // the keys of turn 0
   const uint32_t sel = (kb & 2) ? 0x07060302u : 0x05040100u;       // 4-bit codes: this lane's sixteen bits of a channel's two words
   for (int t = -1; t < n_iter; ++t) {
@@ -377,17 +410,26 @@ decode_heads_kernel(const uint32_t* __restrict__ qa, const float* __restrict__ q
       asm volatile("" : "+v"(tbl_b));
     }
     const int blk = blk_begin + t * TW + tw;
-    if (live && t >= 0 && blk < blk_end) {
-      const f32x4 h0 = *(const f32x4*)(hand + lane * 4), h1 = *(const f32x4*)(hand + 256 + lane * 4);
-      const float alpha = hand[512 + lane];
-      float p[8] = {h0[0], h0[1], h0[2], h0[3], h1[0], h1[1], h1[2], h1[3]};
-      const unsigned char* vp = vring + ((t & 1) * TW * 2 + tw * 2 + (kb & 1)) * GC.vslot - GC.off_vdata;      // offsets are those of the page
-      if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+    if (vlive && t >= 0 && blk < blk_end) {
+      float p[VT][8];
 #pragma unroll
-        for (int c = 0; c < 2 * NG; ++c) acc[c] *= alpha;
+      for (int v = 0; v < VT; ++v) {
+        const float* hv = vhand + v * HD_HAND;
+        const f32x4 h0 = *(const f32x4*)(hv + lane * 4), h1 = *(const f32x4*)(hv + 256 + lane * 4);
+        const float alpha = vtile + v < n_tiles ? hv[512 + lane] : 1.0f;
 #pragma unroll
-        for (int c = 0; c < NZ; ++c) zacc[c] *= alpha;
+        for (int i = 0; i < 4; ++i) {
+          p[v][i] = h0[i];
+          p[v][4 + i] = h1[i];
+        }
+        if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+#pragma unroll
+          for (int c = 0; c < 2 * NGV; ++c) acc[v][c] *= alpha;
+#pragma unroll
+          for (int c = 0; c < NZ; ++c) zacc[v][c] *= alpha;
+        }
       }
+      const unsigned char* vp = vring + ((t & 1) * TW * 2 + tw * 2 + (kb & 1)) * GC.vslot - GC.off_vdata;      // offsets are those of the page
       if (partial(blk)) {
         // Tokens that do not exist: their slots may hold anything, and zero times anything has to be zero: their scales and
         // zero points become zero in LDS (the value wavefronts of a block all write the same).
@@ -400,38 +442,40 @@ decode_heads_kernel(const uint32_t* __restrict__ qa, const float* __restrict__ q
         }
         stage_release();
       }
-      {
-        // zero points: groups as rows, tokens in natural order
-        u32x4 pz;
+      // zero points: groups as rows, tokens in natural order
 #pragma unroll
-        for (int r = 0; r < 4; ++r) pz[r] = F16P ? pack_f16(p[2 * r], p[2 * r + 1]) : pack_bf16(p[2 * r], p[2 * r + 1]);
+      for (int zt = 0; zt < NZ; ++zt) {
+        const unsigned char* zr = vp + GC.off_vzero + ((g0 + min(16 * zt + n, NGV - 1)) * 16 + 4 * (kb >> 1)) * 2;
+        const uint2 z0 = *(const uint2*)zr, z1 = *(const uint2*)(zr + 16);
+        const u32x4 az = {z0.x, z0.y, z1.x, z1.y};
 #pragma unroll
-        for (int zt = 0; zt < NZ; ++zt) {
-          const unsigned char* zr = vp + GC.off_vzero + (min(16 * zt + n, NG - 1) * 16 + 4 * (kb >> 1)) * 2;
-          const uint2 z0 = *(const uint2*)zr, z1 = *(const uint2*)(zr + 16);
-          const u32x4 az = {z0.x, z0.y, z1.x, z1.y};
-          zacc[zt] = F16P ? mfma_f16(az, pz, zacc[zt]) : mfma(az, pz, zacc[zt]);
+        for (int v = 0; v < VT; ++v) {
+          u32x4 pz;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) pz[r] = F16P ? pack_f16(p[v][2 * r], p[v][2 * r + 1]) : pack_bf16(p[v][2 * r], p[v][2 * r + 1]);
+          zacc[v][zt] = F16P ? mfma_f16(az, pz, zacc[v][zt]) : mfma(az, pz, zacc[v][zt]);
         }
       }
       // the code of register r's tokens sits at bit s of its 16-bit half, where it is the bf16 number code x 2^(s - 133): the
       // weight carries 2^(80 - s)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int r = i & 3;
-        p[i] *= VB == 4 ? ((r & 1) ? 0x1p76f : 0x1p80f) : (r == 0 ? 0x1p80f : (r == 1 ? 0x1p78f : (r == 2 ? 0x1p76f : 0x1p74f)));
-      }
-      const unsigned char* srow = vp + GC.off_vscale + 8 * (kb >> 1);
-      const unsigned char* vrow = vp + GC.off_vdata + n * (D / 16) * (VB * 2);
+      for (int v = 0; v < VT; ++v)
 #pragma unroll
-      for (int g = 0; g < NG; ++g) {
+        for (int i = 0; i < 8; ++i) {
+          const int r = i & 3;
+          p[v][i] *= VB == 4 ? ((r & 1) ? 0x1p76f : 0x1p80f) : (r == 0 ? 0x1p80f : (r == 1 ? 0x1p78f : (r == 2 ? 0x1p76f : 0x1p74f)));
+        }
+      const unsigned char* srow = vp + GC.off_vscale + 8 * (kb >> 1) + g0 * 32;
+      const unsigned char* vrow = vp + GC.off_vdata + n * (D / 16) * (VB * 2) + g0 * (VB * 4);
+#pragma unroll
+      for (int g = 0; g < NGV; ++g) {
 #pragma unroll
         for (int k = 0; k < NR; ++k)
-          if (k * NG / NR == g) request(k, t);
+          if (k * NGV / NR == g) request(k, t);
         const uint2 f0 = *(const uint2*)(srow + g * 32), f1 = *(const uint2*)(srow + g * 32 + 16);      // scales of tokens 4 u .., 8 + 4 u ..
         auto lo = [&](uint32_t w) { return F16P ? f16_lo(w) : __uint_as_float(w << 16); };
         auto hi = [&](uint32_t w) { return F16P ? f16_hi(w) : __uint_as_float(w & 0xffff0000u); };
-        const u32x4 wv = {pack_bf16(p[0] * lo(f0.x), p[4] * lo(f1.x)), pack_bf16(p[1] * hi(f0.x), p[5] * hi(f1.x)),
-                          pack_bf16(p[2] * lo(f0.y), p[6] * lo(f1.y)), pack_bf16(p[3] * hi(f0.y), p[7] * hi(f1.y))};
+        const float sv[8] = {lo(f0.x), hi(f0.x), lo(f0.y), hi(f0.y), lo(f1.x), hi(f1.x), lo(f1.y), hi(f1.y)};
         u32x4 a0, a1;
         if (VB == 4) {
           const uint32_t m0 = 0x000F000Fu, m1 = 0x00F000F0u;
@@ -446,8 +490,14 @@ decode_heads_kernel(const uint32_t* __restrict__ qa, const float* __restrict__ q
           a0 = u32x4{x & m0, x & m1, x & m2, x & m3};
           a1 = u32x4{y & m0, y & m1, y & m2, y & m3};
         }
-        acc[2 * g] = mfma(a0, wv, acc[2 * g]);
-        acc[2 * g + 1] = mfma(a1, wv, acc[2 * g + 1]);
+#pragma unroll
+        for (int v = 0; v < VT; ++v) {
+          u32x4 wv;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) wv[r] = pack_bf16(p[v][r] * sv[r], p[v][4 + r] * sv[4 + r]);
+          acc[v][2 * g] = mfma(a0, wv, acc[v][2 * g]);
+          acc[v][2 * g + 1] = mfma(a1, wv, acc[v][2 * g + 1]);
+        }
       }
     } else {
       for (int k = 0; k < NR; ++k) request(k, t);
@@ -458,53 +508,65 @@ decode_heads_kernel(const uint32_t* __restrict__ qa, const float* __restrict__ q
   // ---------------------------------------------------------------- the partial (m, l, acc[d]) of every head
   __syncthreads();                                                 // LDS is free
   float* s_ep = (float*)smem_raw;
-  const float* xm = s_ep + pair * 128;                             // the scorer's (m, l)
-  float* mine = s_ep + NP * 128 + pair * (NG * 16);                // zero-point sums [group][head]: lane (head n, groups 4 kb ..) of tile zt
+  float* mine = s_ep + NP * 128 + pair * (NG * 16);                // zero-point sums [tile][group][head]: lane (head n, groups 4 kb ..) of tile zt
 #pragma unroll
-  for (int zt = 0; zt < NZ; ++zt)
+  for (int v = 0; v < VT; ++v)
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (16 * zt + 4 * kb + i < NG) mine[(16 * zt + 4 * kb + i) * 16 + n] = zacc[zt][i];
+    for (int zt = 0; zt < NZ; ++zt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (16 * zt + 4 * kb + i < NGV) mine[(v * NGV + 16 * zt + 4 * kb + i) * 16 + n] = zacc[v][zt][i];
   stage_release();                                                 // (read back by the same wavefront only)
 #pragma unroll
-  for (int g = 0; g < NG; ++g) {
-    const float z = mine[g * 16 + n];
+  for (int v = 0; v < VT; ++v)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      acc[2 * g][i] = fmaf(acc[2 * g][i], 0x1p53f, z);
-      acc[2 * g + 1][i] = fmaf(acc[2 * g + 1][i], 0x1p53f, z);
+    for (int g = 0; g < NGV; ++g) {
+      const float z = mine[(v * NGV + g) * 16 + n];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        acc[v][2 * g][i] = fmaf(acc[v][2 * g][i], 0x1p53f, z);
+        acc[v][2 * g + 1][i] = fmaf(acc[v][2 * g + 1][i], 0x1p53f, z);
+      }
     }
-  }
   float* xa = s_ep + NP * (128 + NG * 16) + (hw * (TW - 1)) * (2 * NG * 256);      // [TW - 1][2 NG][64][4]
   if (TW > 1 && tw > 0) {
 #pragma unroll
-    for (int c = 0; c < 2 * NG; ++c) *(f32x4*)(xa + (((tw - 1) * 2 * NG + c) * 64 + lane) * 4) = acc[c];
+    for (int v = 0; v < VT; ++v)
+#pragma unroll
+      for (int c = 0; c < 2 * NGV; ++c) *(f32x4*)(xa + (((tw - 1) * 2 * NG + v * 2 * NGV + c) * 64 + lane) * 4) = acc[v][c];
   }
   __syncthreads();
   if (TW > 1) __syncthreads();
-  if (tw > 0 || !live) return;
-  float m_run = xm[lane], l_run = xm[64 + lane];
-  // the blocks side by side: the first pair of a head tile adds the others' sums
+  if (tw > 0) return;
+#pragma unroll
+  for (int v = 0; v < VT; ++v) {
+    if (vtile + v >= n_tiles) return;
+    const float* xm = s_ep + (vpair + v) * 128;                    // the scorer's (m, l)
+    float m_run = xm[lane], l_run = xm[64 + lane];
+    // the blocks side by side: the first wavefront of a head tile and channel part adds the others' sums
 #pragma unroll 1
-  for (int o = 1; o < TW; ++o) {
-    const float m1 = xm[o * HW * 128 + lane], l1 = xm[o * HW * 128 + 64 + lane], m_new = fmaxf(m_run, m1);
-    const float f0 = __builtin_amdgcn_exp2f(m_run - m_new), f1 = __builtin_amdgcn_exp2f(m1 - m_new);
-    l_run = fmaf(l_run, f0, l1 * f1);
-    m_run = m_new;
+    for (int o = 1; o < TW; ++o) {
+      const float m1 = xm[o * HW * 128 + lane], l1 = xm[o * HW * 128 + 64 + lane], m_new = fmaxf(m_run, m1);
+      const float f0 = __builtin_amdgcn_exp2f(m_run - m_new), f1 = __builtin_amdgcn_exp2f(m1 - m_new);
+      l_run = fmaf(l_run, f0, l1 * f1);
+      m_run = m_new;
 #pragma unroll
-    for (int c = 0; c < 2 * NG; ++c) {
-      const f32x4 x = *(const f32x4*)(xa + (((o - 1) * 2 * NG + c) * 64 + lane) * 4);
+      for (int c = 0; c < 2 * NGV; ++c) {
+        const f32x4 x = *(const f32x4*)(xa + (((o - 1) * 2 * NG + v * 2 * NGV + c) * 64 + lane) * 4);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[c][i] = fmaf(acc[c][i], f0, x[i] * f1);
+        for (int i = 0; i < 4; ++i) acc[v][c][i] = fmaf(acc[v][c][i], f0, x[i] * f1);
+      }
     }
-  }
-  if (n < G) {
-    float* row = parts + (((int64_t)b * Hq + qbase + n) * n_parts + split) * (D + 2);
-    if (kb == 0) *(f32x2*)row = f32x2{m_run * 0.6931471805599453f, l_run};      // natural-log domain
+    const int vbase = qbase + (v - part) * 16;                     // query head of column 0
+    if (n < min(16, g_tot - (vtile + v) * 16)) {
+      float* row = parts + (((int64_t)b * Hq + vbase + n) * n_parts + split) * (D + 2);
+      if (part == 0 && kb == 0) *(f32x2*)row = f32x2{m_run * 0.6931471805599453f, l_run};      // natural-log domain
+      row += 2 + 32 * g0 + 4 * kb;
 #pragma unroll
-    for (int c = 0; c < 2 * NG; ++c) {
-      *(f32x2*)(row + 2 + 16 * c + 4 * kb) = f32x2{acc[c][0], acc[c][1]};
-      *(f32x2*)(row + 4 + 16 * c + 4 * kb) = f32x2{acc[c][2], acc[c][3]};
+      for (int c = 0; c < 2 * NGV; ++c) {
+        *(f32x2*)(row + 16 * c) = f32x2{acc[v][c][0], acc[v][c][1]};
+        *(f32x2*)(row + 16 * c + 2) = f32x2{acc[v][c][2], acc[v][c][3]};
+      }
     }
   }
 }
