@@ -377,6 +377,22 @@ def test_quotient_of_bf16_numbers_rounds_like_its_product_with_a_reciprocal():
         assert np.array_equal(got, np.broadcast_to(ref, got.shape)), step
 
 
+def test_quotient_of_fp16_numbers_is_its_product_with_a_reciprocal_and_one_correction():
+    """The value quantiser replaces a / s of fp16 numbers by q + (a - q s) r with q = a r, r an fp32 reciprocal of s good to one ulp:
+    the same fp32 number, for all pairs of significands and the three reciprocals nearest to 1 / s (powers of two change nothing
+    within the range that the kernel takes it for).  Both multiply-adds round once: their products have 35 and 48 bits."""
+    def fma(a, b, c):
+        return (np.float64(a) * np.float64(b) + np.float64(c)).astype(np.float32)
+    s = np.arange(1024, 2048, dtype=np.float32)[:, None]
+    a = np.arange(1024, 2048, dtype=np.float32)[None, :]
+    ref = (a / s).astype(np.float32)
+    r0 = (np.float32(1.0) / s).astype(np.float32)
+    for step in (-1, 0, 1):
+        r = (r0.view(np.int32) + step).view(np.float32)
+        q = (a * r).astype(np.float32)
+        assert np.array_equal(fma(fma(-q, s, a), r, q), ref), step
+
+
 def test_bench_refuses_more_than_one_gpu_and_its_shape_table_is_well_formed():
     """bench.py measures one GPU: --gpus 2 exits with a message instead of running; the shapes of its table mode
     are ones the entry points accept (query heads a multiple of KV heads, head sizes a multiple of 64 up to 768,

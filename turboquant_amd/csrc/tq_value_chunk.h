@@ -23,7 +23,7 @@ struct ValPagedSink {
 };
 
 __host__ inline size_t value_chunk_smem(int slab, int bits) {
-  return (size_t)(slab / 8) * (TILE * (bits == 2 ? 2 : 4) + 16) + TILE * sizeof(int);
+  return (size_t)(slab / 8) * (TILE * (bits == 2 ? 2 : 4) + 16);
 }
 // inputs that the body takes: group sizes that are a power of two of 16 .. 128 and do not cross a slab
 __host__ inline bool value_chunk_takes(int dtype, int bits, int gs, int slab) {
@@ -76,17 +76,26 @@ __device__ __forceinline__ void round_pairs(const float (&in)[8], float sub, flo
   }
 }
 
+// bits of a number that a rounding to the input dtype has left (or one of the input's): nothing is left to round
+template <int DT>
+__device__ __forceinline__ uint16_t stored_bits(float v) {
+  return DT == TQ_BF16 ? (uint16_t)(__float_as_uint(v) >> 16) : f32_to_f16_bits(v);
+}
+
 // Value quantiser for 16-bit inputs and 2/4-bit codes: a thread owns 8 consecutive channels of one token (one
 // 16-byte load), a group's minimum / maximum meet through cross-lane exchanges, and the codes pass through LDS only to
 // be transposed into the page's per-channel fields.  Arithmetic and rounding are those of value_tile_kernel.
 // A workgroup takes one tile's `slab` channels (64, 128 or 256: whole tokens in a row of 16 lanes); head sizes that are
 // not one of these are slabs side by side in the grid's second dimension (a group never crosses a slab).
-// Bound by memory: 8192 vectors of 576, 4-bit codes, 9.4 MB in: value_tile_kernel 17.5 us, nine slabs of 64 7.8 us.
+// Bound by vector instructions: about 185 per wavefront of 512 values, and the kernel takes the time that a SIMD needs to issue them (262,144
+// vectors of 128 in bf16, 67 MB in: 25.5 us; reading them takes 10).  What exists of a tile follows from two numbers and not from flags in
+// LDS counted over the workgroup, the minimum and maximum are the bare instructions, a NaN is looked for by wavefront, groups are shifts,
+// fp16 quotients are products: bf16 31.2 -> 25.5 us, 120,000 vectors in fp16 21.1 -> 15.5, 262,144 of 256 33 -> 27.
+// 8192 vectors of 576, 4-bit codes, 9.4 MB in: value_tile_kernel 17.5 us, nine slabs of 64 7.8 us.
 // A workgroup of 2 * slab threads; c0: its first channel; smem: value_chunk_smem(slab, VB) bytes.
 template <int DT, int VB, class Source, class Sink>
 __device__ __forceinline__ void value_chunk_body(const void* __restrict__ v, const Source& src, int d, int slab, int gs, const Sink& sink,
                                                  int tile, int c0, unsigned char* smem) {
-  using E = Elem<DT>;
   static_assert(DT != TQ_F32, "16-bit inputs");
   const int tid = threadIdx.x;
   const int cpt = slab >> 3;                       // chunks (threads) per token
@@ -98,37 +107,38 @@ __device__ __forceinline__ void value_chunk_body(const void* __restrict__ v, con
   using CodeWord = typename std::conditional<VB == 2, uint16_t, uint32_t>::type;
   constexpr int CROW = TILE * (int)sizeof(CodeWord) + 16;      // bytes per chunk row
   unsigned char* scode = smem;                     // [slab / 8] rows of CROW bytes
-  int* svalid = (int*)(smem + (size_t)cpt * CROW); // [TILE]
 
   // where the tile's rows are and which of its slots exist: uniform, looked up through the scalar cache
   TileAddr ta;
-  // page lookup issued together with the input load (clamped into the table: a tile without a
-  // single existing slot may lie beyond it, and then nothing is stored anyway)
-  int64_t page = 0;
-  int head = 0;
+  int head = 0, b = 0, lpage = 0;
   if constexpr (std::is_base_of<PagedSource, Source>::value) {
     PagedSource::Coord c[1] = {src.coord(tile)};
     TileAddr ta1[1];
-    int lpage[1];
-    src.template tile_addrs<1>(c, ta1, lpage);
+    int lp[1];
+    src.template tile_addrs<1>(c, ta1, lp);
     ta = ta1[0];
     head = c[0].h;
-    if constexpr (!std::is_same<Sink, ValFlatSink>::value)
-      page = checked_page(sink.block_table, sink.max_pages, sink.num_pages, c[0].b, lpage[0]);
+    b = c[0].b;
+    lpage = lp[0];
   } else {
     ta = src.tile_addr(tile);
   }
-  if (ta.hi <= 0) return;                          // (uniform) a page behind the end of a ragged run
-  const bool ok = t >= ta.lo && t < ta.hi;
-  const int64_t off = ta.base + (int64_t)t * src.slot_stride();
+  // (a tile none of whose slots exists may lie beyond the block table, or behind the end of a ragged run: leave before looking it up)
+  const int first = max(ta.lo, 0), last = min(ta.hi, TILE);      // its existing slots
+  if (last <= first) return;
+  const bool full_tile = last - first == TILE, ok = t >= first && t < last;
+  // the page is looked up while the input is on its way
+  int64_t page = 0;
+  if constexpr (!std::is_same<Sink, ValFlatSink>::value) page = checked_page(sink.block_table, sink.max_pages, sink.num_pages, b, lpage);
   const bool page_ok = page >= 0;                    // uniform over the workgroup; false: nothing is stored
-  // unconditional load (slots that do not exist read the first vector)
-  const uint4 raw = *(const uint4*)((const uint16_t*)v + (ok ? off : 0) + c0 + ck * 8);
-  if (ck == 0) svalid[t] = ok;
-  // a tile none of whose slots exists may lie beyond the block table: leave before looking it up
-  const int n_ok = __syncthreads_count(ok);
-  if (n_ok == 0) return;
-  const bool full_tile = n_ok == 2 * slab;
+  // unconditional load (slots that do not exist read the nearest one that does); a lane's part of the address in 24-bit numbers where
+  // the strides are, which they are but for exotic views
+  const int tr = min(max(t, first), last - 1);
+  const uint16_t* rows = (const uint16_t*)v + ta.base + c0;
+  const int64_t stride = src.slot_stride();
+  uint4 raw;
+  if ((uint64_t)stride < (1u << 24)) raw = *(const uint4*)(rows + (__umul24(tr, (uint32_t)stride) + (uint32_t)(ck * 8)));
+  else raw = *(const uint4*)(rows + tr * stride + ck * 8);
   float x[8];
   {
     const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
@@ -138,56 +148,57 @@ __device__ __forceinline__ void value_chunk_body(const void* __restrict__ v, con
       x[2 * i + 1] = DT == TQ_BF16 ? __uint_as_float(w[i] & 0xffff0000u) : f16_bits_to_f32((uint16_t)(w[i] >> 16));
     }
   }
-  float lo = x[0], hi = x[0];
-#pragma unroll
-  for (int i = 1; i < 8; ++i) {
-    lo = fminf(lo, x[i]);
-    hi = fmaxf(hi, x[i]);
-  }
-  // a NaN among the 8 inputs, on the packed 16-bit patterns: magnitude bits above those of infinity
-  int has_nan;
-  {
-    typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
-    u16x2_t m = __builtin_bit_cast(u16x2_t, raw.x & 0x7fff7fffu);
-    m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2_t, raw.y & 0x7fff7fffu));
-    m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2_t, raw.z & 0x7fff7fffu));
-    m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2_t, raw.w & 0x7fff7fffu));
-    constexpr uint16_t inf_bits = DT == TQ_BF16 ? 0x7f80 : 0x7c00;
-    has_nan = (m[0] > inf_bits) | (m[1] > inf_bits);
-  }
+  // (the instructions themselves: fminf / fmaxf first make every operand canonical, an instruction each; the comparisons below see a NaN)
+  auto min2 = [](float p, float q) { float r; asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(p), "v"(q)); return r; };
+  auto max2 = [](float p, float q) { float r; asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(p), "v"(q)); return r; };
+  auto min3 = [](float p, float q, float s) { float r; asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(p), "v"(q), "v"(s)); return r; };
+  auto max3 = [](float p, float q, float s) { float r; asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(p), "v"(q), "v"(s)); return r; };
+  float lo = min2(min3(min3(min3(x[0], x[1], x[2]), x[3], x[4]), x[5], x[6]), x[7]);
+  float hi = max2(max3(max3(max3(x[0], x[1], x[2]), x[3], x[4]), x[5], x[6]), x[7]);
   // the threads of a group are neighbouring lanes inside a row of 16: DPP moves (quad swaps, then half-row and
   // row mirrors, which pair quads that already agree) instead of shuffles through the LDS
-  auto reduce_step = [&](auto ctrl_c) {
-    constexpr int CTRL = decltype(ctrl_c)::value;
-    lo = fminf(lo, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, lo), CTRL, 0xF, 0xF, true)));
-    hi = fmaxf(hi, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, hi), CTRL, 0xF, 0xF, true)));
-    has_nan |= __builtin_amdgcn_update_dpp(0, has_nan, CTRL, 0xF, 0xF, true);
+  auto over_group = [&](auto step) {
+    step(std::integral_constant<int, 0xB1>{});                   // (a group has at least 16 channels)
+    if (tpg >= 4) step(std::integral_constant<int, 0x4E>{});
+    if (tpg >= 8) step(std::integral_constant<int, 0x141>{});
+    if (tpg >= 16) step(std::integral_constant<int, 0x140>{});
   };
-  if (tpg >= 2) reduce_step(std::integral_constant<int, 0xB1>{});
-  if (tpg >= 4) reduce_step(std::integral_constant<int, 0x4E>{});
-  if (tpg >= 8) reduce_step(std::integral_constant<int, 0x141>{});
-  if (tpg >= 16) reduce_step(std::integral_constant<int, 0x140>{});
-  if (has_nan) lo = hi = __uint_as_float(0x7fc00000u);       // torch min/max propagate NaN
+  over_group([&](auto ctrl_c) {
+    constexpr int CTRL = decltype(ctrl_c)::value;
+    lo = min2(lo, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, lo), CTRL, 0xF, 0xF, true)));
+    hi = max2(hi, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, hi), CTRL, 0xF, 0xF, true)));
+  });
+  // torch min / max propagate NaN, the instructions do not: a wavefront that holds one looks for its group
+  const bool nan = __builtin_isunordered(x[0], x[1]) || __builtin_isunordered(x[2], x[3]) || __builtin_isunordered(x[4], x[5]) || __builtin_isunordered(x[6], x[7]);
+  if (__builtin_amdgcn_ballot_w64(nan) != 0) {
+    int has_nan = nan;
+    over_group([&](auto ctrl_c) { has_nan |= __builtin_amdgcn_update_dpp(0, has_nan, decltype(ctrl_c)::value, 0xF, 0xF, true); });
+    if (has_nan) lo = hi = __uint_as_float(0x7fc00000u);
+  }
   const float levels = (float)((1 << VB) - 1);
   // (hi - lo) / levels as a product: both are numbers of at most 8 significant bits, so is the divisor of every
   // quotient below, and such a quotient is never a rounding tie of the 16-bit format and at least 2^-17
   // (relative) away from one: a product with a reciprocal good to an ulp rounds like the division (checked
-  // over all pairs of significands and the three nearest reciprocals).  fp16 keeps the division.
+  // over all pairs of significands and the three nearest reciprocals).  fp16 keeps the division here.
   const float range = round_hw<DT>(hi - lo);
   float sc = round_hw<DT>(DT == TQ_BF16 ? range * (1.0f / levels) : range / levels);
   const float floor_v = round_hw<DT>(1e-10f);
   sc = (sc != sc) ? sc : fmaxf(sc, floor_v);
   const float z = lo;
-  // Quotients of bf16 numbers, rounded to bf16: a * (1/s) with any reciprocal good to an ulp (see above).
-  // Used when the scale is an ordinary number; everything else takes the division.
-  const bool fast_div = DT == TQ_BF16 && sc > 0x1p-60f && sc < 0x1p60f;
+  // Quotients of bf16 numbers, rounded to bf16: a * (1/s) with any reciprocal good to an ulp (see above).  Quotients of fp16 numbers: the
+  // product and one correction by its remainder are the fp32 quotient itself, to the bit (11 significant bits on either side, the three
+  // nearest reciprocals, all pairs).  Used when the scale is an ordinary number; everything else takes the division.
+  const bool fast_div = DT == TQ_BF16 ? sc > 0x1p-60f && sc < 0x1p60f : sc >= 0x1p-24f && sc < 0x1p16f;
   const float rsc = __builtin_amdgcn_rcpf(sc);
   float quo[8];
   if (fast_div) {                // every a of the group is finite and at most (levels + 1) * sc < 2^64 then
     float a[8];
     round_pairs<DT>(x, z, a);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) quo[i] = a[i] * rsc;
+    for (int i = 0; i < 8; ++i) {
+      quo[i] = a[i] * rsc;
+      if constexpr (DT == TQ_F16) quo[i] = fmaf(fmaf(-quo[i], sc, a[i]), rsc, quo[i]);
+    }
   } else {
 #pragma unroll
     for (int i = 0; i < 8; ++i) quo[i] = round_hw<DT>(x[i] - z) / sc;
@@ -200,18 +211,18 @@ __device__ __forceinline__ void value_chunk_body(const void* __restrict__ v, con
 #pragma unroll
   for (int hw = 0; hw < (VB == 2 ? 1 : 2); ++hw) {
     constexpr int PER = 16 / VB;                   // codes per 16 bits
-    float acc = 0.0f;
+    float acc;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       // clamp to [0, levels]; a NaN becomes code 0 (the median-of-three instruction returns the minimum of
       // its operands when one of them is a NaN)
       const float q = __builtin_amdgcn_fmed3f(rintf(qr[hw * PER + i]), 0.0f, levels);
-      acc = fmaf(q, (float)(1 << (VB * i)), acc);
+      acc = i == 0 ? q : fmaf(q, (float)(1 << (VB * i)), acc);
     }
     codes |= (uint32_t)acc << (16 * hw);
   }
   if constexpr (!std::is_same<Sink, ValFlatSink>::value) *(CodeWord*)(scode + ck * CROW + t * sizeof(CodeWord)) = (CodeWord)codes;
-  const int ng = d / gs, g = (c0 + ck * 8) / gs;
+  const int g_bits = __builtin_ctz((unsigned)gs), ng = d >> g_bits, g = (c0 + ck * 8) >> g_bits;      // (groups are powers of two)
   const bool leader = (ck & (tpg - 1)) == 0;
 
   if constexpr (std::is_same<Sink, ValFlatSink>::value) {
@@ -221,16 +232,16 @@ __device__ __forceinline__ void value_chunk_body(const void* __restrict__ v, con
       if (VB == 2) *(uint16_t*)dst = (uint16_t)codes;
       else *(uint32_t*)dst = codes;
       if (leader) {
-        E::store(sink.scale, vec * ng + g, sc);
-        E::store(sink.zero, vec * ng + g, z);
+        ((uint16_t*)sink.scale)[vec * ng + g] = stored_bits<DT>(sc);
+        ((uint16_t*)sink.zero)[vec * ng + g] = stored_bits<DT>(z);
       }
     }
   } else {
     const tq_page_layout& L = sink.L;
     uint8_t* pg = sink.pool + (page * src.H + head) * (int64_t)L.page_bytes;
     if (ok && leader && page_ok) {
-      E::store(pg + L.off_vscale, g * TILE + t, sc);
-      E::store(pg + L.off_vzero, g * TILE + t, z);
+      *(uint16_t*)(pg + (uint32_t)(L.off_vscale + (g * TILE + t) * 2)) = stored_bits<DT>(sc);
+      *(uint16_t*)(pg + (uint32_t)(L.off_vzero + (g * TILE + t) * 2)) = stored_bits<DT>(z);
     }
     __syncthreads();
     // channel c: a field of 16*VB bits, token n at bit VB*n; read-modify-write keeps the codes of
@@ -238,7 +249,8 @@ __device__ __forceinline__ void value_chunk_body(const void* __restrict__ v, con
     // every thread assembles half a field: 8 tokens of one channel (16 bits of 2-bit codes, 32 of 4-bit)
     {
       const int c = tid >> 1, half = tid & 1;
-      uint8_t* fbytes = pg + vfield_off(L, c0 + c) + half * VB;
+      const int cc = c0 + c;                         // (vfield_off, with 24-bit products)
+      uint8_t* fbytes = pg + (uint32_t)(L.off_vdata + (__umul24(cc & 15, d >> 4) + (cc >> 4)) * (VB * 2) + half * VB);
       const unsigned char* row = scode + (c >> 3) * CROW + half * 8 * sizeof(CodeWord);
       const int sh = (c & 7) * VB;                   // the channel's code inside a word
       uint32_t neu = 0, mask = VB == 2 ? 0xffffu : 0xffffffffu;
@@ -257,9 +269,10 @@ __device__ __forceinline__ void value_chunk_body(const void* __restrict__ v, con
         for (int k = 0; k < 8; ++k) neu |= ((ww[k] >> sh) & 0xfu) << (4 * k);
       }
       if (!full_tile) {                              // uniform over the workgroup
-        mask = 0;
-#pragma unroll
-        for (int s2 = 0; s2 < 8; ++s2) mask |= (svalid[half * 8 + s2] ? (1u << VB) - 1u : 0u) << (VB * s2);
+        // the bits of tokens first .. last - 1, those of this half
+        const int f = min(max(first - half * 8, 0), 8), l = min(max(last - half * 8, 0), 8);
+        const uint64_t below = ((uint64_t)1 << (VB * l)) - 1, before = ((uint64_t)1 << (VB * f)) - 1;
+        mask = (uint32_t)(below & ~before);
         neu &= mask;
       }
       if (mask != 0 && page_ok) {
