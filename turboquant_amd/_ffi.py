@@ -23,6 +23,7 @@ NOALLOC_SCRATCH_BYTES = 16 << 20      # TQ_NOALLOC_SCRATCH_BYTES
 # TQ_HIP_LIBRARY overrides the in-tree library (e.g. to compare two builds)
 _LIB_PATH = os.environ.get("TQ_HIP_LIBRARY") or os.path.join(os.path.dirname(os.path.abspath(__file__)), "libtq_hip.so")
 _lib: Optional[C.CDLL] = None
+_host = None                          # the native host side of small calls (csrc/tq_host.cpp), where it is built for this torch
 
 _ERR = {-1: "TQ_EINVAL (a size, stride or enum is out of range)",
         -2: "TQ_EUNSUPPORTED (no kernel for this shape / bit-width)",
@@ -129,7 +130,36 @@ def lib() -> C.CDLL:
         if got != ABI_VERSION:
             raise RuntimeError(f"libtq_hip.so has ABI version {got}, the bindings expect {ABI_VERSION}")
         _lib = handle
+        _bind_host(handle)
     return _lib
+
+
+_HOST_CALLS = ("tq_quantize_keys", "tq_dequant_keys", "tq_score", "tq_ring_write", "tq_append_kv_paged", "tq_decode_workspace_bytes",
+               "tq_decode_attn_paged", "tq_decode_attn_paged_by_length", "tq_decode_attn_paged_ring", "tq_decode_attn_paged_ring_by_length",
+               "tq_cache_append_bytes", "tq_cache_append", "tq_cache_scores", "tq_cache_attend_bytes", "tq_cache_attend")
+
+
+def _bind_host(handle):
+    """Hand the library's functions to the native host side.  It launches nothing that the Python methods do not: without it (not
+    built, or built for another torch) a small call takes longer on the host and is otherwise the same."""
+    global _host
+    try:
+        from . import _tq_host
+    except ImportError:
+        return
+    _tq_host.bind({name: C.cast(getattr(handle, name), C.c_void_p).value for name in _HOST_CALLS})
+    _host = _tq_host
+
+
+def native():
+    """The native host side for a call that runs now (not one that a compiler is tracing); None: the Python method does it all.  Its
+    functions return None for every case that is not the plain one, and have done nothing then."""
+    if _host is None or lib is not _lib_entry or _compiling():        # (a `lib` put in place of ours is there to see the calls)
+        return None
+    return _host
+
+
+_lib_entry = lib
 
 
 def check(rc: int, what: str):

@@ -13,6 +13,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libtq_hip.so")
+HOST = os.path.join(HERE, "_tq_host.so")           # (imported by _ffi.py, where it fits the torch that runs)
 # (the matrix-core page kernel is instantiated by one file per head size, so that they compile side by side)
 SOURCES = ["tq_decode_mfma_d128.hip", "tq_decode_mfma_d128_f16.hip", "tq_decode_mfma_d64.hip", "tq_decode_mfma_d64_f16.hip",
            "tq_decode_mfma_d256.hip", "tq_quantize_mfma.hip", "tq_quantize_wide.hip", "tq_decode_wide.hip", "tq_decode_heads.hip",
@@ -42,6 +43,20 @@ def _run(cmd):
     return res.returncode, err
 
 
+def _host_command():
+    """The native host side of small calls: a Python module against torch's headers, no device code."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    headers = [*include_paths(), sysconfig.get_paths()["include"], "/opt/rocm/include"]
+    return ([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"] + [x for h in headers for x in ("-isystem", h)] +
+            [os.path.join(CSRC, "tq_host.cpp"), "-L" + lib] + [f"-l{n}" for n in ("c10", "c10_hip", "torch_cpu", "torch", "torch_python")] +
+            ["-o", HOST])
+
+
 def build_library(verbose: bool = False) -> str:
     """Compile every source to an object file (in parallel: the files are independent translation units)
     and link them into libtq_hip.so."""
@@ -55,6 +70,7 @@ def build_library(verbose: bool = False) -> str:
     for src in SOURCES:
         obj = os.path.join(objdir, src.replace(".hip", ".o"))
         jobs.append((obj, [hipcc] + compile_flags + ["-c", os.path.join(CSRC, src), "-o", obj]))
+    jobs.append((HOST, _host_command()))
     if verbose:
         for _, cmd in jobs:
             print(" ".join(cmd))
@@ -62,10 +78,10 @@ def build_library(verbose: bool = False) -> str:
         results = list(pool.map(lambda j: _run(j[1]), jobs))
     for (obj, _), (rc, err) in zip(jobs, results):
         if rc != 0:
-            raise RuntimeError(f"hipcc failed ({rc}) for {obj}:\n{err}")
+            raise RuntimeError(f"compiling {obj} failed ({rc}):\n{err}")
         if verbose and err.strip():
             print(err, file=sys.stderr)
-    link = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-fno-gpu-rdc"] + [obj for obj, _ in jobs] + ["-o", LIB]
+    link = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-fno-gpu-rdc"] + [obj for obj, _ in jobs if obj != HOST] + ["-o", LIB]
     if verbose:
         print(" ".join(link))
     rc, err = _run(link)

@@ -165,11 +165,31 @@ class TurboQuantKVCache:
                 return False
         return True
 
+    def _sections(self) -> Optional[tuple]:
+        """The seven tensors of the compressed part, for the native host side, which looks at each; None: not for it."""
+        kq, vq = self.key_quantized, self.value_quantized
+        if (_ffi.native() is None or kq is None or vq is None or vq.bits != self.value_bits or self.head_dim not in (64, 128, 256)
+                or self.value_group_size % 16 or kq.norms.dim() != 3):
+            return None
+        return (*kq[:4], *vq[:3])
+
     def _append_spill(self, key: torch.Tensor, value: torch.Tensor) -> bool:
         """One token into a full buffer whose first row leaves for the compressed part, in one library call; False: the case is
         not that one, nothing was done."""
         kb, vb = self.key_buffer, self.value_buffer
-        if kb is None or vb is None or not self._compressed_plain() or not _plain(key, value, kb, vb):
+        if kb is None or vb is None:
+            return False
+        part = self._sections()
+        if part is not None and kb.shape[-2] == self.buffer_size:
+            q = self.key_quantizer
+            new = _ffi.native().cache_append(*part, key, value, kb, vb, C.addressof(q._layer()), self.head_dim, self.key_bits - 1,
+                                             self.value_bits, self.value_group_size)
+            if new is not None:
+                self.key_quantized = ProdQuantized(*new[:4], self.key_quantized.mse_bits)
+                self.value_quantized = ValueQuantized(*new[4:7], bits=self.value_bits)
+                self.key_buffer, self.value_buffer = new[7:]
+                return True
+        if not self._compressed_plain() or not _plain(key, value, kb, vb):
             return False
         B, H, n_buf, d = kb.shape
         kq, vq = self.key_quantized, self.value_quantized
@@ -245,6 +265,14 @@ class TurboQuantKVCache:
         if scale is None:
             scale = 1.0 / math.sqrt(self.head_dim)
         kb = self.key_buffer
+        part = self._sections() if kb is not None and isinstance(scale, (int, float)) else None
+        if part is not None and query.dim() == 4 and kb.dim() == 4:
+            B, H, n_buf, d = kb.shape
+            if self._few_score_queries(B * H * query.shape[2], part[3].shape[-1], n_buf, d):
+                scores = _ffi.native().cache_scores(*part, query, kb, C.addressof(self.key_quantizer._layer()), self.head_dim, self.key_bits - 1,
+                                                    self.value_bits, self.value_group_size, scale)
+                if scores is not None:
+                    return scores
         if kb is not None and isinstance(scale, (int, float)) and self._compressed_plain() and _plain_product(query, kb):
             kq = self.key_quantized
             B, H, n_buf, d = kb.shape
@@ -276,6 +304,14 @@ class TurboQuantKVCache:
     def attend(self, attn_weights: torch.Tensor) -> torch.Tensor:
         """softmaxed weights (batch, heads, n_q, seq_len) -> (batch, heads, n_q, head_dim)."""
         vb = self.value_buffer
+        part = self._sections() if vb is not None else None
+        if part is not None and attn_weights.dim() == 4 and vb.dim() == 4:
+            B, H, n_buf, d = vb.shape
+            if self._few_value_queries(B * H * attn_weights.shape[2], part[3].shape[-1], n_buf, d):
+                out = _ffi.native().cache_attend(*part, attn_weights, vb, self.head_dim, self.key_bits - 1, self.value_bits,
+                                                 self.value_group_size)
+                if out is not None:
+                    return out
         if vb is not None and self._compressed_plain() and _plain_product(attn_weights, vb):
             vq = self.value_quantized
             B, H, n_buf, d = vb.shape

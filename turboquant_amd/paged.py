@@ -59,6 +59,10 @@ class PagedKVPool:
         """Quantise key/value (B, T, H, d) and store token t of sequence b at
         logical position start_pos[b] + t through block_table (B, max_pages) int32."""
         _ffi.require_gpu(key, "key")
+        fast = _ffi.native()
+        if fast is not None and fast.append(key, value, block_table, start_pos, self.data, self.num_pages, self.num_kv_heads, self.head_dim,
+                                            _ffi.dtype_tag(self.dtype), C.addressof(self.quantizer._layer()), C.addressof(self.layout)):
+            return
         if key.dim() != 4 or key.shape != value.shape:
             raise ValueError("key and value must both be (B, T, H, d)")
         B, T, H, d = key.shape
@@ -279,6 +283,14 @@ class PagedKVPool:
             return 1 + (have - least) // (need(B, Hq, self.head_dim, 2) - least)
         raise ValueError(f"the workspace holds {have} bytes, {B} x {Hq} query heads in {n_split} splits take {want}")
 
+    def _decode_native(self, query, block_table, seq_lens, first, scale, recent_k, recent_v, n_split, by_length) -> Optional[torch.Tensor]:
+        """A whole step (lengths from element `first` on) by the native host side; None: not a case for it, nothing was done."""
+        fast = _ffi.native()
+        if fast is None:
+            return None
+        return fast.decode(query, block_table, seq_lens, first, self.data, self.num_pages, self.num_kv_heads, self.head_dim, scale, recent_k,
+                           recent_v, C.addressof(self.quantizer._layer()), C.addressof(self.layout), n_split, by_length)
+
     def decode_attention(self, query: torch.Tensor, block_table: torch.Tensor, seq_lens: torch.Tensor,
                          scale: Optional[float] = None, recent_k: Optional[torch.Tensor] = None,
                          recent_v: Optional[torch.Tensor] = None, recent_len: Optional[torch.Tensor] = None,
@@ -299,18 +311,22 @@ class PagedKVPool:
         B, Hq, d = query.shape
         if d != self.head_dim or Hq % self.num_kv_heads:
             raise ValueError(f"Incompatible GQA shapes: Q={Hq}, H_kv={self.num_kv_heads}, d={d}")
-        query = query.contiguous()
         if scale is None:
             scale = 1.0 / math.sqrt(d)
-        bt = block_table.contiguous()
-        bt_stride = -bt.shape[0] if bt.dim() == 1 else bt.shape[1]      # negative: one shared row of that length
-        seq_lens = seq_lens.to(device=self.device, dtype=torch.int32).contiguous()
         by_length, ours = False, n_split is None
         if ours:
             if max_len is None:
-                max_len = (bt.shape[-1]) * PAGE_TOKENS
+                max_len = block_table.shape[-1] * PAGE_TOKENS
             n_split = self.default_splits(B, max_len, Hq, static_scratch)
             by_length = workspace is None and not static_scratch and stages == 7 and self._shares_by_length(B, Hq)
+        if workspace is None and out is None and recent_len is None and stages == 7 and not static_scratch:
+            done = self._decode_native(query, block_table, seq_lens, 0, scale, recent_k, recent_v, n_split, by_length)
+            if done is not None:
+                return done
+        query = query.contiguous()
+        bt = block_table.contiguous()
+        bt_stride = -bt.shape[0] if bt.dim() == 1 else bt.shape[1]      # negative: one shared row of that length
+        seq_lens = seq_lens.to(device=self.device, dtype=torch.int32).contiguous()
         if static_scratch:
             if workspace is not None or stages != 7:
                 raise ValueError("static_scratch takes no workspace and runs all stages")
@@ -385,18 +401,25 @@ class PagedKVPool:
         if tuple(key_cache.shape[2:]) != (self.num_kv_heads, d) or not self.ring_cache_ok(key_cache, value_cache):
             raise ValueError("decode_attention_ring needs a (blocks, 16, H_kv, d) cache with contiguous channels, "
                              "equal key / value strides and word-aligned rows")
-        query = query.contiguous()
         if scale is None:
             scale = 1.0 / math.sqrt(d)
-        bt = block_table.contiguous()
-        bt_stride = -bt.shape[0] if bt.dim() == 1 else bt.shape[1]      # negative: one shared row of that length
-        seq_lens = seq_lens.to(device=self.device, dtype=torch.int32).contiguous()
         by_length, ours = False, n_split is None
         if ours:
             if max_len is None:
-                max_len = (bt.shape[-1]) * PAGE_TOKENS
+                max_len = block_table.shape[-1] * PAGE_TOKENS
             n_split = self.default_splits(B, max_len, Hq)
             by_length = workspace is None and self._shares_by_length(B, Hq)
+        fast = _ffi.native()
+        if fast is not None and workspace is None and out is None:
+            done = fast.decode_ring(query, block_table, seq_lens, self.data, self.num_pages, self.num_kv_heads, self.head_dim, scale,
+                                    key_cache, value_cache, ring_rows, C.addressof(self.quantizer._layer()), C.addressof(self.layout),
+                                    n_split, by_length)
+            if done is not None:
+                return done
+        query = query.contiguous()
+        bt = block_table.contiguous()
+        bt_stride = -bt.shape[0] if bt.dim() == 1 else bt.shape[1]      # negative: one shared row of that length
+        seq_lens = seq_lens.to(device=self.device, dtype=torch.int32).contiguous()
         if workspace is None:
             workspace = self.workspace(B, Hq, -n_split if by_length else n_split)
         else:

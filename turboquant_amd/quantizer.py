@@ -223,9 +223,14 @@ class TurboQuantProd(torch.nn.Module):
 
     def quantize(self, x: torch.Tensor) -> ProdQuantized:
         _ffi.require_gpu(x, "x")
+        mb = self.bits - 1
+        fast = _ffi.native()
+        if fast is not None:
+            code = fast.quantize(x, C.addressof(self._layer()), self.dim, mb)
+            if code is not None:
+                return ProdQuantized(*code, mb)
         rows, stride = _rows(x)
         n, d = rows.shape[0], self.dim
-        mb = self.bits - 1
         width, per_byte = _packing(mb)
         packed, signs = _codes(x, n, (d + per_byte - 1) // per_byte), _codes(x, n, (d + 7) // 8)
         norms, rnorms = _codes(x, n, dtype=x.dtype), _codes(x, n, dtype=torch.float32)
@@ -263,7 +268,13 @@ class TurboQuantProd(torch.nn.Module):
         return code, y.reshape(*lead, d), p.reshape(*lead, d)
 
     def dequantize(self, q: ProdQuantized) -> torch.Tensor:
-        idx = _ffi.require_gpu(q.mse_indices, "mse_indices").contiguous()
+        _ffi.require_gpu(q.mse_indices, "mse_indices")
+        fast = _ffi.native()
+        if fast is not None:
+            out = fast.dequantize(q.mse_indices, q.qjl_signs, q.residual_norms, q.norms, C.addressof(self._layer()), self.dim, self.bits - 1)
+            if out is not None:
+                return out
+        idx = q.mse_indices.contiguous()
         signs = q.qjl_signs.contiguous()
         norms = q.norms.contiguous()
         rnorms = q.residual_norms.contiguous().float()
@@ -282,6 +293,12 @@ class TurboQuantProd(torch.nn.Module):
         without the 1/sqrt(d) factor."""
         _ffi.require_gpu(query, "query")
         d = self.dim
+        fast = _ffi.native()
+        if fast is not None:
+            k = quantized_key
+            scores = fast.score(query, k.mse_indices, k.qjl_signs, k.residual_norms, k.norms, C.addressof(self._layer()), d, self.bits - 1)
+            if scores is not None:
+                return scores
         lead = query.shape[:-2]
         if lead != quantized_key.norms.shape[:-1]:
             lead = torch.broadcast_shapes(lead, quantized_key.norms.shape[:-1])

@@ -46,6 +46,14 @@ def compute_hybrid_attention(query: torch.Tensor, store: CompressedKVStore, rece
     if Q != num_kv_heads * gqa_ratio:
         raise ValueError(f"Incompatible GQA shapes: Q={Q}, H_kv={num_kv_heads}, gqa_ratio={gqa_ratio}")
 
+    # one query token over a store that holds its pages already, everything plain: the tensors as they are, without a view of any
+    if T == 1 and has_history and isinstance(store, CompressedKVStore) and store.has_pages(n_hist):
+        pool = store.pool
+        out = pool._decode_native(query, store.block_table, store.counts, n_hist, scale, recent_k if has_recent else None, recent_v,
+                                  pool.default_splits(1, n_hist, Q), False)
+        if out is not None:
+            return out
+
     # the kernel reads q and the recent tokens in one dtype; mixed inputs are widened to fp32 (lossless)
     work_dtype = query.dtype
     if has_recent and (recent_k.dtype != work_dtype or recent_v.dtype != work_dtype):

@@ -65,6 +65,16 @@ class CompressedKVStore:
         """(1, num_pages) int32: this sequence's pages, in order."""
         return self._block_table
 
+    @property
+    def counts(self) -> Optional[torch.Tensor]:
+        """0, 1, 2 ... on the device: every length the sequence can have (see lengths)."""
+        return self._counts
+
+    def has_pages(self, n: int) -> bool:
+        """Whether the pool and the table exist as ensure_pool leaves them, and `n` is a length they can hold."""
+        return (self._pool is not None and self._block_table is not None and self._block_table.shape[1] == self._pool.num_pages and
+                n < self._counts.shape[0])
+
     def ensure_pool(self, dtype: torch.dtype, min_tokens: int = 0) -> PagedKVPool:
         need = max(self._INITIAL_PAGES, (min_tokens + PAGE_TOKENS - 1) // PAGE_TOKENS)
         if self._pool is None:
