@@ -196,7 +196,8 @@ int tq_rotate_query(const void *q, int dtype, int64_t rows, const tq_layer *laye
  * the buffer's first row leaves it and is quantised: every section is written anew with one more token, and the
  * buffers with their rows one further (contiguous).  The buffers' rows have to lie one behind another (s_r = d) and, with more
  * than one batch, s_b = H s_h; else TQ_EUNSUPPORTED, as for sections off a 4-byte boundary and for n_c or n_buf above 2^20.
- * n_c may be 0 (the sections are not read then).  work: tq_cache_append_bytes bytes.
+ * n_c may be 0 (the sections are not read then).  work: tq_cache_append_bytes bytes.  One launch at d = 128 / 256 and copies of
+ * up to 16 MB, else two.
  * tq_cache_scores (kv_cache.py:247-284): scores (batch, n_q, n_c + n_buf) = scale * <q, k> over the compressed keys, then the
  * exact ones; n_c, n_buf > 0.  TQ_EUNSUPPORTED: codes off a 4-byte boundary, n_q above 2^18, n_c above 2^28, n_buf above 2^24.  work:
  * 2 * batch * n_q * d floats.
@@ -215,6 +216,11 @@ int tq_cache_scores(const float *q, int64_t batch, int H, int64_t n_q, const uin
                     const float *norms, const float *rnorms, int64_t n_c, const tq_layer *layer, const float *key_buf,
                     int64_t s_b, int64_t s_h, int64_t s_r, int n_buf, float scale, float *scores, float *work,
                     void *stream);
+/* ... with queries q_row >= d elements apart (a token's slice of a longer tensor needs no copy). */
+int tq_cache_scores_rows(const float *q, int64_t q_row, int64_t batch, int H, int64_t n_q, const uint8_t *idx,
+                         const uint8_t *signs, const float *norms, const float *rnorms, int64_t n_c, const tq_layer *layer,
+                         const float *key_buf, int64_t s_b, int64_t s_h, int64_t s_r, int n_buf, float scale, float *scores,
+                         float *work, void *stream);
 size_t tq_cache_attend_bytes(int64_t batch, int64_t n_q, int d, int64_t n_c, int n_buf);
 int tq_cache_attend(const float *weights, int64_t batch, int H, int64_t n_q, const uint8_t *data, const float *scales,
                     const float *zeros, int64_t n_c, int d, int group_size, int value_bits, const float *value_buf,

@@ -752,6 +752,55 @@ def test_cache_token_that_has_to_be_differentiated(gpu):
     assert torch.allclose(out, cache.attend(torch.softmax(scores, dim=-1).detach()), rtol=1e-4, atol=1e-5)
 
 
+@pytest.mark.parametrize("d,B,H,n_c,n_buf,key_bits,vb,gs", [
+    (128, 1, 8, 300, 64, 3, 2, 32), (128, 1, 1, 1, 1, 2, 8, 16), (128, 2, 8, 77, 5, 4, 4, 128), (128, 1, 17, 40, 3, 5, 2, 64),
+    (256, 3, 11, 129, 2, 3, 4, 32), (256, 1, 2, 1000, 130, 4, 2, 256), (64, 1, 5, 33, 7, 3, 2, 32), (128, 1, 4, 9001, 128, 3, 4, 32)])
+def test_cache_token_in_one_launch(gpu, d, B, H, n_c, n_buf, key_bits, vb, gs):
+    """A token into the cache object by the launch that quantises and copies at once, by the two behind one another, and by the quantisers
+    and concatenations: the same bytes in every section and buffer.  Rows around a tile of sixteen, a section of one token, pieces of 16
+    and of 4 bytes, copies of several rounds; channels that are one group, equal, infinite or no numbers."""
+    from turboquant_amd import _ffi
+    from turboquant_amd.kv_cache import TurboQuantKVCache
+    g = torch.Generator().manual_seed(n_c + d)
+    k, v = (torch.randn(B, H, n_c + n_buf + 1, d, generator=g).to(gpu) for _ in range(2))
+    v[0, 0, n_c, : d // 2] = 2.5
+    v[-1, -1, n_c, 3] = float("inf")
+    v[0, -1, n_c, 5] = float("nan")
+    states = []
+    try:
+        for how in (-1, 0, None):                              # one launch, two, the general path
+            cache = TurboQuantKVCache(d, key_bits=key_bits, value_bits=vb, value_group_size=gs, buffer_size=n_buf, device=gpu, dtype=torch.float32)
+            cache.prefill(k[..., :n_c + n_buf, :].contiguous(), v[..., :n_c + n_buf, :].contiguous())
+            assert _ffi.lib().tq_set_option(b"append_small", how if how is not None else -1) == 0
+            cache.key_buffer, cache.value_buffer = cache.key_buffer.contiguous(), cache.value_buffer.contiguous()
+            new = [t[..., n_c + n_buf:, :].contiguous() for t in (k, v)]
+            if how is None:
+                cache._append(*new)
+            else:
+                assert cache._append_spill(*new)
+            states.append([*cache.key_quantized[:4], *cache.value_quantized[:3], cache.key_buffer, cache.value_buffer])
+    finally:
+        _ffi.lib().tq_set_option(b"append_small", -1)
+    for other in states[1:]:
+        for a, b in zip(states[0], other):
+            assert a.shape == b.shape and torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
+
+
+@pytest.mark.parametrize("d,B,H,n_c,n_q,step", [(128, 1, 8, 300, 1, 3), (64, 2, 3, 65, 1, 2), (256, 1, 2, 40, 5, 2), (128, 2, 2, 17, 3, 1)])
+def test_cache_scores_of_queries_that_lie_apart(gpu, d, B, H, n_c, n_q, step):
+    """A token's slice of a tensor of all queries gives the scores of its copy, bit for bit."""
+    from turboquant_amd.kv_cache import TurboQuantKVCache
+    g = torch.Generator().manual_seed(d + n_c)
+    k, v = (torch.randn(B, H, n_c + 9, d, generator=g).to(gpu) for _ in range(2))
+    q = torch.randn(B, H, n_q * step, d, generator=g).to(gpu)
+    cache = TurboQuantKVCache(d, key_bits=3, value_bits=2, buffer_size=9, device=gpu, dtype=torch.float32)
+    cache.prefill(k, v)
+    part = q[..., 1 % step::step, :] if n_q > 1 else q[..., step - 1:, :]
+    assert torch.equal(cache.attention_scores(part), cache.attention_scores(part.clone(memory_format=torch.contiguous_format)))
+    wide = torch.randn(B, H, n_q, 2 * d, generator=g).to(gpu)[..., d:]
+    assert torch.equal(cache.attention_scores(wide), cache.attention_scores(wide.contiguous()))
+
+
 @pytest.mark.parametrize("d,H,n_c,n_buf,vb", [(64, 8, 1000, 128, 2), (128, 8, 300, 128, 4), (256, 3, 2000, 33, 2)])
 def test_cache_blocks_of_queries_on_either_side_of_the_limit(gpu, counted, d, H, n_c, n_buf, vb):
     """The largest block of queries that takes the entry, and the next one, which takes the general path: results as from products in fp64

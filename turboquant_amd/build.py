@@ -53,7 +53,7 @@ def _host_command():
     headers = [*include_paths(), sysconfig.get_paths()["include"], "/opt/rocm/include"]
     return ([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
              f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"] + [x for h in headers for x in ("-isystem", h)] +
-            [os.path.join(CSRC, "tq_host.cpp"), "-L" + lib] + [f"-l{n}" for n in ("c10", "c10_hip", "torch_cpu", "torch", "torch_python")] +
+            [os.path.join(CSRC, "tq_host.cpp"), "-L" + lib] + [f"-l{n}" for n in ("c10", "c10_hip", "torch_cpu", "torch_hip", "torch", "torch_python")] +
             ["-o", HOST])
 
 

@@ -1256,7 +1256,7 @@ namespace tq {
 int launch_rotate_query(const void* q, int dtype, int64_t rows, const tq_layer* layer, float* q_rot, float* q_sk,
                         float* q_stat, uint32_t* qa_pack, int G, float sm_scale, hipStream_t st, bool q_rot_unused,
                         unsigned long long* arrivals, const PagePrefetch* prefetch, int g_tot, const WidePack* wide,
-                        const SplitPlan& plan);
+                        const SplitPlan& plan, int64_t q_row);
 bool prep_on_matrix_cores(const void* q, int dtype, int64_t rows, const tq_layer* layer, int G, int g_tot);
 bool rotate_on_matrix_cores(const void* q, int dtype, int64_t rows, const tq_layer* layer, const WidePack* wide);
 bool rotate_by_rows(int64_t rows, int d);
@@ -1701,7 +1701,7 @@ static int decode_stages(const void* q, int dtype, int B, int Hq, int Hkv, const
     } else {
       int rc = launch_rotate_query(q, dtype, (int64_t)B * Hq, layer, q_rot, q_sk, q_stat,
                                    mfma_shape ? qa_pack : nullptr, mfma_shape ? Gq : G, sm_scale, st, mfma_shape,
-                                   fm.counters, &pf, mfma_shape ? g_tot : 0, wide_pre.qa ? &wide_pre : nullptr, plan);
+                                   fm.counters, &pf, mfma_shape ? g_tot : 0, wide_pre.qa ? &wide_pre : nullptr, plan, layer->d);
       if (rc) return rc;
     }
   }

@@ -2,7 +2,7 @@
 //
 // A decode token of one sequence, a token of the cache object or a few thousand keys to codes are two to eight launches of a few
 // microseconds each; the tensor attributes, allocations and foreign-function conversions around them took longer than the launches (a chat
-// token 41 us of host time against 21 us of the card, a token of the cache object 95 against 53).  Every function here takes the case that
+// token 41 us of host time against 21 us of the card, a token of the cache object 95 against 53; here 27 and 48).  Every function here takes the case that
 // the Python method in front of it meets in a decode loop - plain dense tensors of the current device, contiguous where the library
 // wants it - and returns None (ring_write: False) for everything else, before it allocates or launches anything: the Python method then goes on as if
 // it had not been called.  What the library refuses comes back as None too, and the Python method meets the refusal itself.
@@ -11,6 +11,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/InferenceMode.h>
@@ -41,14 +42,14 @@ struct Library {
   decltype(&tq_decode_attn_paged_ring_by_length) decode_attn_paged_ring_by_length;
   decltype(&tq_cache_append_bytes) cache_append_bytes;
   decltype(&tq_cache_append) cache_append;
-  decltype(&tq_cache_scores) cache_scores;
+  decltype(&tq_cache_scores_rows) cache_scores_rows;
   decltype(&tq_cache_attend_bytes) cache_attend_bytes;
   decltype(&tq_cache_attend) cache_attend;
 } g_lib{};
 constexpr const char* kNames[] = {"tq_quantize_keys", "tq_dequant_keys", "tq_score", "tq_ring_write", "tq_append_kv_paged",
                                   "tq_decode_workspace_bytes", "tq_decode_attn_paged", "tq_decode_attn_paged_by_length",
                                   "tq_decode_attn_paged_ring", "tq_decode_attn_paged_ring_by_length", "tq_cache_append_bytes",
-                                  "tq_cache_append", "tq_cache_scores", "tq_cache_attend_bytes", "tq_cache_attend"};
+                                  "tq_cache_append", "tq_cache_scores_rows", "tq_cache_attend_bytes", "tq_cache_attend"};
 static_assert(sizeof(Library) == sizeof(kNames) / sizeof(kNames[0]) * sizeof(void*), "a pointer per name, in order");
 bool g_bound = false;
 
@@ -62,7 +63,7 @@ bool nothing_watches() {
     exc = exc | c10::autograd_dispatch_keyset;
   }
   return tls.included_ == inc && tls.excluded_ == exc && c10::impl::TorchDispatchModeTLS::stack_len() == 0 &&
-         at::impl::PythonTorchFunctionTLS::stack_len() == 0;
+         at::impl::PythonTorchFunctionTLS::stack_len() == 0 && !at::globalContext().deterministicAlgorithms();      // (which fills new tensors)
 }
 
 // The arguments' tensors: plain ones (torch.Tensor itself; dense, its memory holding its values: no lazy conjugation or negation,
@@ -95,7 +96,10 @@ struct Plain {
     return t;
   }
   void* stream() const { return (void*)c10::hip::getCurrentHIPStream(device).stream(); }
-  at::TensorOptions options(at::ScalarType dt) const { return at::TensorOptions().dtype(dt).device(at::kCUDA, device); }
+  // (nothing watches: the dispatcher, half of an allocation's time, has nothing to do)
+  at::Tensor fresh(at::IntArrayRef size, at::ScalarType dt) const {
+    return at::Tensor(at::detail::empty_cuda(size, dt, c10::Device(at::kCUDA, device), std::nullopt));
+  }
 };
 
 int dtype_tag(at::ScalarType t) {
@@ -155,9 +159,9 @@ PyObject* quantize(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     const int tag = dtype_tag(x.scalar_type()), per = 8 / code_bits(mb);
     if (tag < 0) return nullptr;
     const auto lead = x.sizes().slice(0, x.dim() - 1);
-    const auto bytes = p.options(at::kByte);
-    at::Tensor idx = at::empty(shape(lead, {(d + per - 1) / per}), bytes), sgn = at::empty(shape(lead, {(d + 7) / 8}), bytes);
-    at::Tensor nrm = at::empty(lead, p.options(x.scalar_type())), rn = at::empty(lead, p.options(at::kFloat));
+    constexpr auto bytes = at::kByte;
+    at::Tensor idx = p.fresh(shape(lead, {(d + per - 1) / per}), bytes), sgn = p.fresh(shape(lead, {(d + 7) / 8}), bytes);
+    at::Tensor nrm = p.fresh(lead, x.scalar_type()), rn = p.fresh(lead, at::kFloat);
     if (unlocked(g_lib.quantize_keys, x.data_ptr(), tag, x.numel() / d, d, address<tq_layer>(a[1]), (uint8_t*)idx.data_ptr(), (uint8_t*)sgn.data_ptr(),
                             nrm.data_ptr(), (float*)rn.data_ptr(), nullptr, nullptr, 0, p.stream()) != TQ_OK)
       return nullptr;
@@ -190,7 +194,7 @@ PyObject* dequantize(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     const int64_t d = int_arg(a[5]);
     const int mb = (int)int_arg(a[6]);
     if (PyErr_Occurred() || !c.take(p, a, d, mb)) return nullptr;
-    at::Tensor out = at::empty(shape(c.nrm.sizes(), {d}), p.options(at::kFloat));
+    at::Tensor out = p.fresh(shape(c.nrm.sizes(), {d}), at::kFloat);
     if (unlocked(g_lib.dequant_keys, (const uint8_t*)c.idx.data_ptr(), (const uint8_t*)c.sgn.data_ptr(), c.nrm.data_ptr(), dtype_tag(c.nrm.scalar_type()),
                            (const float*)c.rn.data_ptr(), c.n, address<tq_layer>(a[4]), (float*)out.data_ptr(), p.stream()) != TQ_OK)
       return nullptr;
@@ -212,7 +216,7 @@ PyObject* score(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     const auto lead = c.nrm.sizes().slice(0, c.nrm.dim() - 1);
     if (q.sizes().slice(0, q.dim() - 2) != lead) return nullptr;
     const int64_t n_q = q.size(-2), n_k = c.nrm.size(-1), batch = c.n / n_k;
-    at::Tensor out = at::empty(shape(lead, {n_q, n_k}), p.options(at::kFloat)), work = at::empty({2 * batch * n_q * d}, p.options(at::kFloat));
+    at::Tensor out = p.fresh(shape(lead, {n_q, n_k}), at::kFloat), work = p.fresh({2 * batch * n_q * d}, at::kFloat);
     if (unlocked(g_lib.score, q.data_ptr(), tag, batch, n_q, (const uint8_t*)c.idx.data_ptr(), (const uint8_t*)c.sgn.data_ptr(), c.nrm.data_ptr(),
                     dtype_tag(c.nrm.scalar_type()), (const float*)c.rn.data_ptr(), n_k, address<tq_layer>(a[5]), (float*)out.data_ptr(),
                     (float*)work.data_ptr(), p.stream()) != TQ_OK)
@@ -295,7 +299,7 @@ struct Step {
     return true;
   }
   at::Tensor workspace(const Plain& p, int64_t d, int n_split) const {
-    return at::empty({(int64_t)(g_lib.decode_workspace_bytes((int)B, (int)Hq, (int)d, n_split) / 4)}, p.options(at::kFloat));
+    return p.fresh({(int64_t)(g_lib.decode_workspace_bytes((int)B, (int)Hq, (int)d, n_split) / 4)}, at::kFloat);
   }
 };
 
@@ -324,7 +328,7 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
         rs[1] = k.stride(i); rs[2] = k.stride(i + 1);
       }
     }
-    const at::Tensor ws = s.workspace(p, d, by_length ? -n_split : n_split), out = at::empty(s.q.sizes(), s.q.options());
+    const at::Tensor ws = s.workspace(p, d, by_length ? -n_split : n_split), out = p.fresh(s.q.sizes(), s.q.scalar_type());
     const auto call = by_length ? g_lib.decode_attn_paged_by_length : g_lib.decode_attn_paged;
     if (unlocked(call, s.q.data_ptr(), s.tag, (int)s.B, (int)s.Hq, (int)H, (const uint8_t*)s.pool.data_ptr(), pages, (const int32_t*)s.table.data_ptr(),
              (int)s.bt_stride, s.len_ptr, (float)scale, address<tq_layer>(a[11]), address<tq_page_layout>(a[12]), rk, rv, (int)R, rs[0], rs[1],
@@ -350,7 +354,7 @@ PyObject* decode_ring(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
       return nullptr;
     if (k.element_size() == 2 && ((k.stride(0) | k.stride(1) | k.stride(2)) % 2 || (((uintptr_t)k.data_ptr() | (uintptr_t)v.data_ptr()) & 3)))
       return nullptr;
-    const at::Tensor ws = s.workspace(p, d, by_length ? -n_split : n_split), out = at::empty(s.q.sizes(), s.q.options());
+    const at::Tensor ws = s.workspace(p, d, by_length ? -n_split : n_split), out = p.fresh(s.q.sizes(), s.q.scalar_type());
     const auto call = by_length ? g_lib.decode_attn_paged_ring_by_length : g_lib.decode_attn_paged_ring;
     if (unlocked(call, s.q.data_ptr(), s.tag, (int)s.B, (int)s.Hq, (int)H, (const uint8_t*)s.pool.data_ptr(), pages, (const int32_t*)s.table.data_ptr(),
              (int)s.bt_stride, s.len_ptr, (float)scale, address<tq_layer>(a[11]), address<tq_page_layout>(a[12]), k.data_ptr(), v.data_ptr(),
@@ -402,11 +406,11 @@ PyObject* cache_append(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     auto grown = [&](const at::Tensor& t) {
       auto s = t.sizes().vec();
       s[2] = c.n + 1;
-      return at::empty(s, t.options());
+      return p.fresh(s, t.scalar_type());
     };
     const at::Tensor idx = grown(c.idx), sgn = grown(c.sgn), rn = grown(c.rn), nrm = grown(c.nrm), data = grown(c.data), scales = grown(c.scales),
-                     zeros = grown(c.zeros), nk = at::empty(kb.sizes(), kb.options()), nv = at::empty(kb.sizes(), kb.options());
-    const at::Tensor work = at::empty({(int64_t)g_lib.cache_append_bytes(B * H, (int)d, mb, bits, (int)gs)}, p.options(at::kByte));
+                     zeros = grown(c.zeros), nk = p.fresh(kb.sizes(), at::kFloat), nv = p.fresh(kb.sizes(), at::kFloat);
+    const at::Tensor work = p.fresh({(int64_t)g_lib.cache_append_bytes(B * H, (int)d, mb, bits, (int)gs)}, at::kByte);
     if (unlocked(g_lib.cache_append, (const float*)key.data_ptr(), (const float*)value.data_ptr(), key.stride(1), value.stride(1), (const float*)kb.data_ptr(),
                            (const float*)vb.data_ptr(), kb.stride(0), kb.stride(1), kb.stride(2), vb.stride(0), vb.stride(1), vb.stride(2), B * H, (int)H,
                            (int)n_buf, address<tq_layer>(a[11]), bits, (int)gs, c.n, (const uint8_t*)c.idx.data_ptr(), (const uint8_t*)c.sgn.data_ptr(),
@@ -432,9 +436,13 @@ PyObject* cache_scores(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     if (!p.ok || !rows4(query) || !rows4(kb) || kb.size(0) != c.B || kb.size(1) != c.H || kb.size(3) != d || kb.size(2) < 1 || kb.size(2) > INT_MAX) return nullptr;
     const int64_t n_q = query.size(2), n_buf = kb.size(2), batch = c.B * c.H;
     if (query.size(0) != c.B || query.size(1) != c.H || query.size(3) != d || n_q < 1 || batch > 65535) return nullptr;
-    const at::Tensor q = query.contiguous(), out = at::empty({c.B, c.H, n_q, c.n + n_buf}, p.options(at::kFloat));
-    const at::Tensor work = at::empty({2 * batch * n_q * d}, p.options(at::kFloat));
-    if (unlocked(g_lib.cache_scores, (const float*)q.data_ptr(), batch, (int)c.H, n_q, (const uint8_t*)c.idx.data_ptr(), (const uint8_t*)c.sgn.data_ptr(),
+    // rows that lie evenly apart are read where they are (a token's slice of all queries)
+    const bool even = (n_q == 1 || query.stride(1) == n_q * query.stride(2)) && (c.B == 1 || query.stride(0) == c.H * query.stride(1));
+    const int64_t apart = n_q == 1 ? query.stride(1) : query.stride(2);
+    const bool in_place = even && apart >= d;
+    const at::Tensor q = in_place ? query : query.contiguous(), out = p.fresh({c.B, c.H, n_q, c.n + n_buf}, at::kFloat);
+    const at::Tensor work = p.fresh({2 * batch * n_q * d}, at::kFloat);
+    if (unlocked(g_lib.cache_scores_rows, (const float*)q.data_ptr(), in_place ? apart : d, batch, (int)c.H, n_q, (const uint8_t*)c.idx.data_ptr(), (const uint8_t*)c.sgn.data_ptr(),
                            (const float*)c.nrm.data_ptr(), (const float*)c.rn.data_ptr(), c.n, address<tq_layer>(a[9]), (const float*)kb.data_ptr(),
                            kb.stride(0), kb.stride(1), kb.stride(2), (int)n_buf, (float)scale, (float*)out.data_ptr(), (float*)work.data_ptr(),
                            p.stream()) != TQ_OK)
@@ -455,8 +463,8 @@ PyObject* cache_attend(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     if (!p.ok || !rows4(weights) || !rows4(vb) || vb.size(0) != c.B || vb.size(1) != c.H || vb.size(3) != d || vb.size(2) < 1 || vb.size(2) > INT_MAX) return nullptr;
     const int64_t n_q = weights.size(2), n_buf = vb.size(2), batch = c.B * c.H;
     if (weights.size(0) != c.B || weights.size(1) != c.H || weights.size(3) != c.n + n_buf || n_q < 1 || n_q > 65535 || batch > 65535) return nullptr;
-    const at::Tensor w = weights.contiguous(), out = at::empty({c.B, c.H, n_q, d}, p.options(at::kFloat));
-    const at::Tensor work = at::empty({(int64_t)(g_lib.cache_attend_bytes(batch, n_q, (int)d, c.n, (int)n_buf) / 4)}, p.options(at::kFloat));
+    const at::Tensor w = weights.contiguous(), out = p.fresh({c.B, c.H, n_q, d}, at::kFloat);
+    const at::Tensor work = p.fresh({(int64_t)(g_lib.cache_attend_bytes(batch, n_q, (int)d, c.n, (int)n_buf) / 4)}, at::kFloat);
     if (unlocked(g_lib.cache_attend, (const float*)w.data_ptr(), batch, (int)c.H, n_q, (const uint8_t*)c.data.data_ptr(), (const float*)c.scales.data_ptr(),
                            (const float*)c.zeros.data_ptr(), c.n, (int)d, (int)gs, bits, (const float*)vb.data_ptr(), vb.stride(0), vb.stride(1),
                            vb.stride(2), (int)n_buf, (float*)out.data_ptr(), (float*)work.data_ptr(), p.stream()) != TQ_OK)

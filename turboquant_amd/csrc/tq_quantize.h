@@ -228,6 +228,7 @@ struct KeyFlatSink {
   float* rnorm;
   float* y_dbg;
   float* p_dbg;
+  int64_t step = 1;        // rows from one vector to the next (matrix-core kernels of 128 / 256)
 };
 
 struct KeyPagedSink {

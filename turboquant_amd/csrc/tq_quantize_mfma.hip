@@ -27,6 +27,7 @@
 
 #include <atomic>
 
+#include "tq_cache_append.h"
 #include "tq_key_mfma.h"
 #include "tq_value_chunk.h"
 #include "tq_decode_mfma.h"
@@ -686,16 +687,16 @@ __device__ __forceinline__ int64_t key_mfma_body(const void* __restrict__ x, con
         }                                                         // eff == 1: the plane word is the dword
         dw |= x << (mb - 1 - p);
       }
-      ((uint32_t*)sink.idx)[(tile0 * TILE + t) * row_dw + k] = dw;
+      ((uint32_t*)sink.idx)[(tile0 * TILE + t) * sink.step * row_dw + k] = dw;
     }
     if (!mse_only) {
       for (int o = tid; o < TT * W; o += KQ_THREADS) {
         const int t = o / W, w = o - t * W;
-        if (svalid[t]) ((uint32_t*)sink.sign)[(tile0 * TILE + t) * W + w] = spl[(mb * TT + t) * W + w];
+        if (svalid[t]) ((uint32_t*)sink.sign)[(tile0 * TILE + t) * sink.step * W + w] = spl[(mb * TT + t) * W + w];
       }
     }
     if (tid < TT && svalid[tid]) {
-      const int64_t v = tile0 * TILE + tid;
+      const int64_t v = (tile0 * TILE + tid) * sink.step;
       E::store(sink.norm, v, snorm[tid]);
       if (!mse_only) sink.rnorm[v] = srn[tid];
     }
@@ -771,6 +772,21 @@ append_small_kernel(const void* __restrict__ k, const void* __restrict__ v, Page
   const int id = blockIdx.x - n_tiles, tile = id / (D / SLAB), c0 = id % (D / SLAB) * SLAB;
   if (vs.L.value_bits == 2) value_chunk_body<DT, 2>(v, src, D, SLAB, gs, vs, tile, c0, smem);
   else value_chunk_body<DT, 4>(v, src, D, SLAB, gs, vs, tile, c0, smem);
+}
+
+// A token of the cache object in one launch (kv_cache.py:203-245): the workgroups of the keys that leave the buffer, a tile each, whose codes go
+// straight to the last row of the new sections, and behind them those of the values and of the copies, which depend on nothing that
+// the keys' write.  Bound by the serial chain of a key tile; three launches took 9.7, 6.7 and 4.9 us behind one another.
+template <int D, bool FX>
+__global__ void __launch_bounds__(KQ_THREADS, 2)
+cache_append_kernel(const float* __restrict__ keys, FlatSource src, tq_layer ly, KeyFlatSink ks, int n_tiles, CacheRest rest) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  if ((int)blockIdx.x >= n_tiles) {
+    cache_rest_body(rest, (int)blockIdx.x - n_tiles);
+    return;
+  }
+  int64_t end = n_tiles;
+  key_mfma_body<TQ_F32, D, false, FX, FlatSource, KeyFlatSink, 1>(keys, src, ly, ks, 0, end, blockIdx.x, n_tiles, smem);
 }
 
 __host__ static bool aligned_for_chunks(const void* x, int dtype, const FlatSource& s) {
@@ -872,6 +888,42 @@ static int launch_append_small_d(const void* k, const void* v, const PagedSource
     kern<<<grid, dim3(KQ_THREADS), smem, st>>>(k, v, src, ly, ks, vs, tiles, ks.L.group_size);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? TQ_OK : (int)e;
+}
+
+template <int D, bool FX>
+static int launch_cache_append_d(const float* keys, const FlatSource& src, const tq_layer& ly, const KeyFlatSink& ks, int tiles,
+                                 const CacheRest& rest, hipStream_t st) {
+  constexpr size_t smem = KeySmem<TQ_F32, D>::bytes;
+  auto kern = cache_append_kernel<D, FX>;
+  static std::atomic<uint64_t> configured{0};           // one bit per device; the attribute is sticky
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return TQ_EINVAL;
+  if (dev >= 64 || !(configured.load() >> dev & 1)) {
+    hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    if (e != hipSuccess) return (int)e;
+    if (dev < 64) configured.fetch_or(1ull << dev);
+  }
+  kern<<<dim3((unsigned)(tiles + rest.rows + rest.copies)), dim3(KQ_THREADS), smem, st>>>(keys, src, ly, ks, tiles, rest);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? TQ_OK : (int)e;
+}
+
+// The whole token in one launch, at head_dim 128 / 256.  Every workgroup of it reserves a key tile's LDS, so a compute unit holds one: up to
+// four rounds of copies (16 MB); beyond, and where the matrix-core kernel does not take the keys, TQ_EUNSUPPORTED: the caller launches two or three.
+int launch_cache_append(const float* keys, int64_t stride, int64_t rows, const tq_layer& ly, const KeyFlatSink& ks, const CacheRest& rest,
+                        hipStream_t st) {
+  const FlatSource src{rows, stride};
+  const int64_t tiles = (rows + TILE - 1) / TILE;
+  if (opt_append_small.load(std::memory_order_relaxed) == 0 || tiles > device_compute_units() / 2 ||
+      (int64_t)rest.rows + rest.copies > 4 * (int64_t)device_compute_units())
+    return TQ_EUNSUPPORTED;
+  if (!ly.Pi_split || !ly.PiT_split || !ly.S_split || ly.mse_bits < 1 || ly.mse_bits > 4) return TQ_EUNSUPPORTED;
+  if (!aligned_for_chunks(keys, TQ_F32, src) || !sink_ok(ks, 0)) return TQ_EUNSUPPORTED;
+  if (ly.d == 128)
+    return fp6_centroids(ly) ? launch_cache_append_d<128, true>(keys, src, ly, ks, (int)tiles, rest, st)
+                             : launch_cache_append_d<128, false>(keys, src, ly, ks, (int)tiles, rest, st);
+  if (ly.d == 256) return launch_cache_append_d<256, false>(keys, src, ly, ks, (int)tiles, rest, st);
+  return TQ_EUNSUPPORTED;
 }
 
 // Keys and values of a small append in one launch: where the keys take a workgroup per tile and the values are 16-bit chunks.

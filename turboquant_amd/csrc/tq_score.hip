@@ -3,6 +3,7 @@
 
 #include <algorithm>
 #include "tq_common.h"
+#include "tq_cache_append.h"
 #include "tq_prep.h"
 #include "tq_options.h"
 #include "tq_decode_mfma.h"
@@ -19,10 +20,13 @@ bool prep_tile_per_workgroup(int n_tiles, int d);
 constexpr int ROT_SLICES = 8;      // (ROT_COLS = 32 output columns per workgroup: tq_prep.h)
 
 // sq[0 .. tot) = elements off .. off + have of q as fp32, zeros behind them (off, have and tot multiples of 8):
-// 16-byte loads, all of a thread's in flight together, when q allows them
+// 16-byte loads, all of a thread's in flight together, when q allows them.  fp32 rows of d may lie q_row > d elements apart.
 __device__ __forceinline__ void rows_to_lds(const void* __restrict__ q, int dtype, int64_t off, int have, int tot,
-                                            float* __restrict__ sq, int tid, int n_threads) {
-  if ((((uintptr_t)q) & 15) == 0 && dtype != TQ_F32) {
+                                            float* __restrict__ sq, int tid, int n_threads, int d, int64_t q_row) {
+  if (q_row != d) {
+    const float* src = (const float*)q + off / d * q_row;
+    for (int o = tid; o < tot; o += n_threads) sq[o] = o < have ? src[o / d * q_row + o % d] : 0.0f;
+  } else if ((((uintptr_t)q) & 15) == 0 && dtype != TQ_F32) {
     const uint4* src = (const uint4*)((const uint16_t*)q + off);
     const bool bf = dtype == TQ_BF16;
 #pragma unroll 4
@@ -63,7 +67,7 @@ __device__ __forceinline__ void rows_to_lds(const void* __restrict__ q, int dtyp
 template <int BATCH, int HALVES, bool PACK>
 __global__ void __launch_bounds__(ROT_COLS * ROT_SLICES * HALVES)
 rotate_query_kernel(const void* __restrict__ q, int dtype, int64_t rows, int R, tq_layer ly, float* __restrict__ q_rot,
-                    float* __restrict__ q_sk, WidePack wp) {
+                    float* __restrict__ q_sk, WidePack wp, int64_t q_row) {
   extern __shared__ __align__(16) float sm[];
   constexpr int T1 = ROT_COLS * ROT_SLICES;
   const int d = ly.d, tid = threadIdx.x, half = tid / T1, t1 = tid - half * T1, jl = t1 % ROT_COLS, sl = t1 / ROT_COLS;
@@ -91,7 +95,7 @@ rotate_query_kernel(const void* __restrict__ q, int dtype, int64_t rows, int R, 
       cs2[k] = ly.S_colsum[c];
     }
   }
-  rows_to_lds(q, dtype, row0 * d, nr * d, R * d, sq, tid, (int)blockDim.x);
+  rows_to_lds(q, dtype, row0 * d, nr * d, R * d, sq, tid, (int)blockDim.x, d, q_row);
   __syncthreads();
   float* s_rot = pb + ROT_SLICES * R * ROT_COLS;   // PACK: [R][ROT_COLS] this word's rotated values, then the sketched ones
   float* s_sk = s_rot + R * ROT_COLS;
@@ -243,6 +247,7 @@ prep_mfma_kernel(const uint16_t* __restrict__ q, int G, int64_t n_rows, tq_layer
 // The exact tokens of a cache object: fp32 rows (batch, H, n, d) with element strides, and the queries they meet.
 struct CacheTail {
   const float* q;
+  int64_t q_row;             // elements from a query to the next
   const float* k;
   int64_t s_b, s_h, s_r;
   int H, n;
@@ -328,7 +333,7 @@ score_kernel(const float* __restrict__ q_rot, const float* __restrict__ q_sk, in
       for (int r = ((int)blockIdx.x - (int)nkb) * SCORE_ROWS + wave, e = min(r - wave + SCORE_ROWS, tail.n); r < e; r += 4) {
         const float* row = tail.k + b / tail.H * tail.s_b + b % tail.H * tail.s_h + r * tail.s_r;
         for (int i = 0; i < ni; ++i) {
-          const float* qr = tail.q + (b * n_q + q0 + i) * d;
+          const float* qr = tail.q + (b * n_q + q0 + i) * tail.q_row;
           float a = 0.0f;
           for (int c = lane; c < d; c += 64) a = fmaf(qr[c], row[c], a);
           a = wave_sum_fast(a);
@@ -575,7 +580,7 @@ bool rotate_on_matrix_cores(const void* q, int dtype, int64_t rows, const tq_lay
 int launch_rotate_query(const void* q, int dtype, int64_t rows, const tq_layer* layer, float* q_rot, float* q_sk,
                         float* q_stat, uint32_t* qa_pack, int G, float sm_scale, hipStream_t st, bool q_rot_unused,
                         unsigned long long* arrivals, const PagePrefetch* prefetch, int g_tot, const WidePack* wide,
-                        const SplitPlan& plan) {
+                        const SplitPlan& plan, int64_t q_row) {
   const int d = layer->d;
   if (qa_pack) {       // operands of the matrix-core decode kernel wanted
     // g_tot: query heads per KV head when its groups of G are unequal (0: the rows are whole groups of G)
@@ -713,7 +718,7 @@ int launch_rotate_query(const void* q, int dtype, int64_t rows, const tq_layer* 
       hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);    \
       if (e != hipSuccess) return (int)e;                                                                              \
     }                                                                                                                  \
-    kern<<<rgrid, rblock, smem, st>>>(q, dtype, rows, R, *layer, q_rot, q_sk, wp);                                     \
+    kern<<<rgrid, rblock, smem, st>>>(q, dtype, rows, R, *layer, q_rot, q_sk, wp, q_row);                              \
   }
 #define TQ_ROTATE_R(BATCH)                 \
   {                                        \
@@ -738,7 +743,7 @@ extern "C" int tq_rotate_query(const void* q, int dtype, int64_t rows, const tq_
   if (!q || !q_rot || !q_sk) return TQ_ENULL;
   if (rows < 0 || dtype < TQ_F32 || dtype > TQ_BF16) return TQ_EINVAL;
   if (rows == 0) return TQ_OK;
-  return launch_rotate_query(q, dtype, rows, layer, q_rot, q_sk, nullptr, nullptr, 1, 0.0f, (hipStream_t)stream, false, nullptr, nullptr, 0, nullptr, SplitPlan{});
+  return launch_rotate_query(q, dtype, rows, layer, q_rot, q_sk, nullptr, nullptr, 1, 0.0f, (hipStream_t)stream, false, nullptr, nullptr, 0, nullptr, SplitPlan{}, layer->d);
 }
 
 extern "C" int tq_score(const void* q, int dtype, int64_t batch, int64_t n_q, const uint8_t* idx, const uint8_t* signs,
@@ -818,28 +823,10 @@ extern "C" int tq_dequant_values(const uint8_t* data, const void* scales, const 
 // ---- a step of the self-contained cache object (kv_cache.py:119-349): fp32 rows, one flat tensor per section --------
 namespace tq {
 
-// Rows of several sections at once: row r of section s becomes its `a` bytes followed by its `b` bytes.  One launch where a
-// concatenation per section (and its host time) stood; bound by the latency of a small copy.
-constexpr int CAT_MAX = 9;
-struct CatSection { const uint8_t *a, *b; uint8_t* dst; int64_t a_stride, b_stride; int a_bytes, b_bytes; };
-struct CatArgs { CatSection s[CAT_MAX]; };
+// (values and copies of a token, behind the key quantiser's launch: one launch where a concatenation per section, and its host time, stood)
+__global__ void __launch_bounds__(256) cache_rest_kernel(CacheRest A) { cache_rest_body(A, (int)blockIdx.x); }
 
-__global__ void __launch_bounds__(256)
-cat_rows_kernel(CatArgs A) {
-  const CatSection c = A.s[blockIdx.z];
-  const int64_t r = blockIdx.y;
-  const uint8_t *a = c.a + r * c.a_stride, *b = c.b + r * c.b_stride;
-  uint8_t* dst = c.dst + r * ((int64_t)c.a_bytes + c.b_bytes);
-  const int total = c.a_bytes + c.b_bytes;
-  // (16-byte pieces where a row of the section and both its parts allow them, else words)
-  if (((((uintptr_t)a | (uintptr_t)b | (uintptr_t)dst) & 15) | ((c.a_bytes | c.b_bytes) & 15)) == 0) {
-    for (int o = (blockIdx.x * 256 + threadIdx.x) * 16; o < total; o += gridDim.x * 256 * 16)
-      *(uint4*)(dst + o) = *(const uint4*)(o < c.a_bytes ? a + o : b + (o - c.a_bytes));
-  } else {
-    for (int o = (blockIdx.x * 256 + threadIdx.x) * 4; o < total; o += gridDim.x * 256 * 4)
-      *(uint32_t*)(dst + o) = *(const uint32_t*)(o < c.a_bytes ? a + o : b + (o - c.a_bytes));
-  }
-}
+int launch_cache_append(const float* keys, int64_t stride, int64_t rows, const tq_layer& ly, const KeyFlatSink& ks, const CacheRest& rest, hipStream_t st);
 
 // Weighted sum of the values: a share of the compressed tokens, or 32 exact rows, per workgroup.  A thread owns one word of
 // codes (32 / VB channels of one group) of every 256 / words-th token of the share; code * scale + zero rounds twice, as
@@ -925,6 +912,7 @@ extern "C" int tq_cache_append(const float* key, const float* value, int64_t key
     return TQ_ENULL;
   const int d = layer->d;
   if (!cache_dims(batch, H, d) || n_buf < 1 || n_c < 0 || group_size < 16 || d % group_size || key_stride < d || value_stride < d) return TQ_EINVAL;
+  if (value_bits != 2 && value_bits != 4 && value_bits != 8) return TQ_EUNSUPPORTED;
   // (lengths in bytes of a section's row are ints)
   if (n_c > (1 << 20) || n_buf > (1 << 20)) return TQ_EUNSUPPORTED;
   if (ks_r != d || vs_r != d || ks_h < d || vs_h < d) return TQ_EUNSUPPORTED;      // a buffer's rows lie one behind another
@@ -941,35 +929,51 @@ extern "C" int tq_cache_append(const float* key, const float* value, int64_t key
   uint8_t* n_sgn = (uint8_t*)take(batch * sb);
   float* n_nrm = (float*)take(batch * 4);
   float* n_rn = (float*)take(batch * 4);
-  uint8_t* n_dat = (uint8_t*)take(batch * db);
-  float* n_sc = (float*)take(batch * ng * 4);
-  float* n_z = (float*)take(batch * ng * 4);
-  int rc = tq_quantize_keys(key_buf, TQ_F32, batch, ks_h, layer, n_idx, n_sgn, n_nrm, n_rn, nullptr, nullptr, 0, stream);
-  if (rc) return rc;
-  rc = tq_quantize_values(value_buf, TQ_F32, batch, vs_h, d, group_size, value_bits, n_dat, n_sc, n_z, stream);
-  if (rc) return rc;
-  CatArgs A;
-  auto section = [&](int i, const void* a, int64_t a_stride, int a_bytes, const void* b, int64_t b_stride, int b_bytes, void* dst) {
-    A.s[i] = CatSection{(const uint8_t*)a, (const uint8_t*)b, (uint8_t*)dst, a_stride, b_stride, a_bytes, b_bytes};
-  };
   const int n = (int)n_c;
-  section(0, idx, (int64_t)n * ib, n * ib, n_idx, ib, ib, idx_out);
-  section(1, signs, (int64_t)n * sb, n * sb, n_sgn, sb, sb, signs_out);
-  section(2, norms, (int64_t)n * 4, n * 4, n_nrm, 4, 4, norms_out);
-  section(3, rnorms, (int64_t)n * 4, n * 4, n_rn, 4, 4, rnorms_out);
-  section(4, data, (int64_t)n * db, n * db, n_dat, db, db, data_out);
-  section(5, scales, (int64_t)n * ng * 4, n * ng * 4, n_sc, ng * 4, ng * 4, scales_out);
-  section(6, zeros, (int64_t)n * ng * 4, n * ng * 4, n_z, ng * 4, ng * 4, zeros_out);
-  section(7, key_buf + d, ks_h * 4, (n_buf - 1) * d * 4, key, key_stride * 4, d * 4, key_buf_out);
-  section(8, value_buf + d, vs_h * 4, (n_buf - 1) * d * 4, value, value_stride * 4, d * 4, value_buf_out);
-  const int longest = std::max(n * std::max(std::max(ib, db), std::max(sb, ng * 4)), n_buf * d * 4);
-  const int blocks = std::max(1, std::min(32, longest / (256 * 16 * 2)));
-  cat_rows_kernel<<<dim3(blocks, (unsigned)batch, CAT_MAX), dim3(256), 0, (hipStream_t)stream>>>(A);
+  CacheRest A;
+  A.rows = (int)batch;
+  A.v = value_buf; A.v_stride = vs_h;
+  A.data = data_out + (size_t)n * db; A.scales = scales_out + (size_t)n * ng; A.zeros = zeros_out + (size_t)n * ng;
+  A.step = n + 1;
+  A.d = d; A.gs = group_size; A.bits = value_bits;
+  auto section = [&](int i, const void* a, int64_t a_stride, int a_bytes, const void* b, int64_t b_stride, int b_bytes, void* dst, int64_t dst_stride) {
+    A.s[i] = CopySection{(const uint8_t*)a, (const uint8_t*)b, (uint8_t*)dst, a_stride, b_stride, dst_stride, a_bytes, b_bytes, 0};
+  };
+  section(0, data, (int64_t)n * db, n * db, nullptr, 0, 0, data_out, (int64_t)(n + 1) * db);
+  section(1, scales, (int64_t)n * ng * 4, n * ng * 4, nullptr, 0, 0, scales_out, (int64_t)(n + 1) * ng * 4);
+  section(2, zeros, (int64_t)n * ng * 4, n * ng * 4, nullptr, 0, 0, zeros_out, (int64_t)(n + 1) * ng * 4);
+  section(3, key_buf + d, ks_h * 4, (n_buf - 1) * d * 4, key, key_stride * 4, d * 4, key_buf_out, (int64_t)n_buf * d * 4);
+  section(4, value_buf + d, vs_h * 4, (n_buf - 1) * d * 4, value, value_stride * 4, d * 4, value_buf_out, (int64_t)n_buf * d * 4);
+  // the key's sections, with the codes from `work` behind them or (alone) without
+  auto key_sections = [&](bool with_codes) {
+    section(5, idx, (int64_t)n * ib, n * ib, with_codes ? n_idx : nullptr, ib, with_codes ? ib : 0, idx_out, (int64_t)(n + 1) * ib);
+    section(6, signs, (int64_t)n * sb, n * sb, with_codes ? n_sgn : nullptr, sb, with_codes ? sb : 0, signs_out, (int64_t)(n + 1) * sb);
+    section(7, norms, (int64_t)n * 4, n * 4, with_codes ? n_nrm : nullptr, 4, with_codes ? 4 : 0, norms_out, (int64_t)(n + 1) * 4);
+    section(8, rnorms, (int64_t)n * 4, n * 4, with_codes ? n_rn : nullptr, 4, with_codes ? 4 : 0, rnorms_out, (int64_t)(n + 1) * 4);
+    A.copies = 0;
+    for (auto& c : A.s) {
+      c.first = A.copies;
+      A.copies += copy_workgroups(c, batch);
+    }
+    return A.copies <= 1 << 23;                  // (a grid counts fewer than 2^32 threads)
+  };
+  int rc = check_layer_rd(layer, true);
+  if (rc) return rc;
+  if (!layer->thresholds) return TQ_ENULL;
+  if (!key_sections(false)) return TQ_EUNSUPPORTED;
+  KeyFlatSink ks{idx_out + (size_t)n * ib, signs_out + (size_t)n * sb, norms_out + n, rnorms_out + n, nullptr, nullptr};
+  ks.step = n + 1;
+  rc = launch_cache_append(key_buf, ks_h, batch, *layer, ks, A, (hipStream_t)stream);
+  if (rc != TQ_EUNSUPPORTED) return rc;
+  if (!key_sections(true)) return TQ_EUNSUPPORTED;
+  rc = tq_quantize_keys(key_buf, TQ_F32, batch, ks_h, layer, n_idx, n_sgn, n_nrm, n_rn, nullptr, nullptr, 0, stream);
+  if (rc) return rc;
+  cache_rest_kernel<<<dim3((unsigned)(A.rows + A.copies)), dim3(256), 0, (hipStream_t)stream>>>(A);
   TQ_CHECK_LAUNCH();
   return TQ_OK;
 }
 
-extern "C" int tq_cache_scores(const float* q, int64_t batch, int H, int64_t n_q, const uint8_t* idx, const uint8_t* signs,
+extern "C" int tq_cache_scores_rows(const float* q, int64_t q_row, int64_t batch, int H, int64_t n_q, const uint8_t* idx, const uint8_t* signs,
                                const float* norms, const float* rnorms, int64_t n_c, const tq_layer* layer, const float* key_buf,
                                int64_t s_b, int64_t s_h, int64_t s_r, int n_buf, float scale, float* scores, float* work,
                                void* stream) {
@@ -979,11 +983,13 @@ extern "C" int tq_cache_scores(const float* q, int64_t batch, int H, int64_t n_q
   const int d = layer->d;
   if (!cache_dims(batch, H, d) || n_q <= 0 || n_c <= 0 || n_buf <= 0) return TQ_EINVAL;
   if (((uintptr_t)idx | (uintptr_t)signs) & 3 || n_c > SCORE_LAUNCH_KEYS || n_q > (1 << 18) || n_buf > (1 << 24)) return TQ_EUNSUPPORTED;
+  if (q_row < d) return TQ_EINVAL;
   float* q_rot = work;
   float* q_sk = work + batch * n_q * d;
-  rc = tq_rotate_query(q, TQ_F32, batch * n_q, layer, q_rot, q_sk, stream);
+  rc = launch_rotate_query(q, TQ_F32, batch * n_q, layer, q_rot, q_sk, nullptr, nullptr, 1, 0.0f, (hipStream_t)stream, false, nullptr, nullptr, 0,
+                           nullptr, SplitPlan{}, q_row);
   if (rc) return rc;
-  const CacheTail tail{q, key_buf, s_b, s_h, s_r, H, n_buf, scale};
+  const CacheTail tail{q, q_row, key_buf, s_b, s_h, s_r, H, n_buf, scale};
   const int nt = score_query_tiles(batch, n_q, n_c);
   const dim3 grid((unsigned)((n_c + SCORE_KEYS - 1) / SCORE_KEYS + (n_buf + SCORE_ROWS - 1) / SCORE_ROWS), (unsigned)((n_q + 16 * nt - 1) / (16 * nt)),
                   (unsigned)batch);
@@ -992,6 +998,14 @@ extern "C" int tq_cache_scores(const float* q, int64_t batch, int H, int64_t n_q
       q_rot, q_sk, n_q, idx, signs, norms, TQ_F32, rnorms, n_c, 0, *layer, scores, tail);
   TQ_CHECK_LAUNCH();
   return TQ_OK;
+}
+
+extern "C" int tq_cache_scores(const float* q, int64_t batch, int H, int64_t n_q, const uint8_t* idx, const uint8_t* signs,
+                               const float* norms, const float* rnorms, int64_t n_c, const tq_layer* layer, const float* key_buf,
+                               int64_t s_b, int64_t s_h, int64_t s_r, int n_buf, float scale, float* scores, float* work,
+                               void* stream) {
+  return tq_cache_scores_rows(q, layer ? layer->d : 0, batch, H, n_q, idx, signs, norms, rnorms, n_c, layer, key_buf, s_b, s_h, s_r, n_buf, scale,
+                              scores, work, stream);
 }
 
 extern "C" size_t tq_cache_attend_bytes(int64_t batch, int64_t n_q, int d, int64_t n_c, int n_buf) {
