@@ -197,7 +197,7 @@ int tq_rotate_query(const void *q, int dtype, int64_t rows, const tq_layer *laye
  * buffers with their rows one further (contiguous).  The buffers' rows have to lie one behind another (s_r = d) and, with more
  * than one batch, s_b = H s_h; else TQ_EUNSUPPORTED, as for sections off a 4-byte boundary and for n_c or n_buf above 2^20.
  * n_c may be 0 (the sections are not read then).  work: tq_cache_append_bytes bytes.  One launch at d = 128 / 256 and copies of
- * up to 16 MB, else two.
+ * up to 48 MB, else two.
  * tq_cache_scores (kv_cache.py:247-284): scores (batch, n_q, n_c + n_buf) = scale * <q, k> over the compressed keys, then the
  * exact ones; n_c, n_buf > 0.  TQ_EUNSUPPORTED: codes off a 4-byte boundary, n_q above 2^18, n_c above 2^28, n_buf above 2^24.  work:
  * 2 * batch * n_q * d floats.

@@ -38,23 +38,33 @@ __host__ inline int copy_workgroups(const CopySection& c, int64_t rows) {
   return (int)((pieces + 256 * CACHE_CHUNKS - 1) / (256 * CACHE_CHUNKS));
 }
 
+typedef uint32_t U4 __attribute__((ext_vector_type(4)));
+
 template <class Piece>
 __device__ __forceinline__ void copy_rows(const CopySection& c, int64_t rows, int64_t wg) {
   const uint32_t per = (uint32_t)(c.a_bytes + c.b_bytes) / sizeof(Piece), a_per = (uint32_t)c.a_bytes / sizeof(Piece);
   const int64_t o0 = wg * (CACHE_CHUNKS * 256), r0 = o0 / per;      // (uniform; the lanes go on in 32 bits)
   const uint32_t e0 = (uint32_t)(o0 - r0 * per);
+  // (every load unconditional, all in flight together: one under a branch is waited for at once; pieces behind the last row read its last)
   Piece x[CACHE_CHUNKS];
   Piece* to[CACHE_CHUNKS];
+  bool in[CACHE_CHUNKS];
 #pragma unroll
   for (int k = 0; k < CACHE_CHUNKS; ++k) {
-    const uint32_t o = e0 + k * 256 + threadIdx.x, rr = o / per, e = o - rr * per;
-    const int64_t r = r0 + rr;
-    to[k] = r < rows ? (Piece*)(c.dst + r * c.dst_stride) + e : nullptr;
-    if (to[k]) x[k] = e < a_per ? ((const Piece*)(c.a + r * c.a_stride))[e] : ((const Piece*)(c.b + r * c.b_stride))[e - a_per];
+    const uint32_t o = e0 + k * 256 + threadIdx.x, rr = o / per;
+    in[k] = r0 + rr < rows;
+    const int64_t r = in[k] ? r0 + rr : rows - 1;
+    const uint32_t e = in[k] ? o - rr * per : per - 1;
+    const Piece* a = (const Piece*)(c.a + r * c.a_stride) + e;
+    const Piece* b = (const Piece*)(c.b + r * c.b_stride) + (e - a_per);
+    x[k] = *(e < a_per ? a : b);
+    to[k] = (Piece*)(c.dst + r * c.dst_stride) + e;
   }
+  // (written past the L2, whose dirty lines a launch's end waits for: 15 MB of copies behind a key's own launch 18.9 -> 6.4 us, though the
+  // scores that read them next take 15.6 us for 13.9)
 #pragma unroll
   for (int k = 0; k < CACHE_CHUNKS; ++k)
-    if (to[k]) *to[k] = x[k];
+    if (in[k]) __builtin_nontemporal_store(x[k], to[k]);
 }
 
 // Workgroup `id` of rows + copies, 256 threads; d <= 256.  The values' arithmetic and rounding are those of value_tile_kernel.
@@ -67,7 +77,7 @@ __device__ __forceinline__ void cache_rest_body(const CacheRest& A, int id) {
 #pragma unroll
     for (int i = 1; i < CACHE_SECTIONS; ++i) k += id >= A.s[i].first;
     const CopySection c = A.s[k];
-    if (copy_piece(c) == 16) copy_rows<uint4>(c, A.rows, id - c.first);
+    if (copy_piece(c) == 16) copy_rows<U4>(c, A.rows, id - c.first);
     else copy_rows<uint32_t>(c, A.rows, id - c.first);
     return;
   }

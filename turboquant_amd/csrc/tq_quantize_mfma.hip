@@ -776,7 +776,8 @@ append_small_kernel(const void* __restrict__ k, const void* __restrict__ v, Page
 
 // A token of the cache object in one launch (kv_cache.py:203-245): the workgroups of the keys that leave the buffer, a tile each, whose codes go
 // straight to the last row of the new sections, and behind them those of the values and of the copies, which depend on nothing that
-// the keys' write.  Bound by the serial chain of a key tile; three launches took 9.7, 6.7 and 4.9 us behind one another.
+// the keys' write.  Bound by the serial chain of a key tile (15 MB of copies beside it: 11.0 us); three launches took 9.7, 6.7 and 4.9 us
+// behind one another.
 template <int D, bool FX>
 __global__ void __launch_bounds__(KQ_THREADS, 2)
 cache_append_kernel(const float* __restrict__ keys, FlatSource src, tq_layer ly, KeyFlatSink ks, int n_tiles, CacheRest rest) {
@@ -909,13 +910,14 @@ static int launch_cache_append_d(const float* keys, const FlatSource& src, const
 }
 
 // The whole token in one launch, at head_dim 128 / 256.  Every workgroup of it reserves a key tile's LDS, so a compute unit holds one: up to
-// four rounds of copies (16 MB); beyond, and where the matrix-core kernel does not take the keys, TQ_EUNSUPPORTED: the caller launches two or three.
+// twelve rounds of copies (48 MB; four tokens and their attention, one launch and two: of 15 MB 361 and 383 us, of 31 MB 733 and 766, of
+// 62 MB 1172 and 1164); beyond, and where the matrix-core kernel does not take the keys, TQ_EUNSUPPORTED: the caller launches two.
 int launch_cache_append(const float* keys, int64_t stride, int64_t rows, const tq_layer& ly, const KeyFlatSink& ks, const CacheRest& rest,
                         hipStream_t st) {
   const FlatSource src{rows, stride};
   const int64_t tiles = (rows + TILE - 1) / TILE;
   if (opt_append_small.load(std::memory_order_relaxed) == 0 || tiles > device_compute_units() / 2 ||
-      (int64_t)rest.rows + rest.copies > 4 * (int64_t)device_compute_units())
+      (int64_t)rest.rows + rest.copies > 12 * (int64_t)device_compute_units())
     return TQ_EUNSUPPORTED;
   if (!ly.Pi_split || !ly.PiT_split || !ly.S_split || ly.mse_bits < 1 || ly.mse_bits > 4) return TQ_EUNSUPPORTED;
   if (!aligned_for_chunks(keys, TQ_F32, src) || !sink_ok(ks, 0)) return TQ_EUNSUPPORTED;

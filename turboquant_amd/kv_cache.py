@@ -146,7 +146,7 @@ class TurboQuantKVCache:
 
     # ---- a decode token in fp32 (the general paths below take everything else) -----------------------------------------
     # A step of the general paths is some thirty small launches and seven concatenations of the whole history: 270 us, nearly all of it
-    # host time, at 4096 tokens of 8 heads of 128.  The entries below are one launch for the token (head_dim 64, and copies beyond 16 MB:
+    # host time, at 4096 tokens of 8 heads of 128.  The entries below are one launch for the token (head_dim 64, and copies beyond 48 MB:
     # two), two for the scores and two for the values: 85 us through the Python methods, 48 us through the native host side, 35 us of the
     # card.  What an entry does not take (sections that are not word-aligned, buffers or blocks of queries
     # beyond its indexes) it refuses before it launches anything, and the general path goes on.
