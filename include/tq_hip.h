@@ -245,6 +245,13 @@ int tq_append_kv_paged(const void *k, const void *v, int dtype, int B, int T, in
                        int max_pages, const tq_layer *layer, const tq_page_layout *layout, uint8_t *pool,
                        int64_t num_pages, void *stream);
 
+/* The same for the newest T tokens of sequences that hold seq_lens[b] tokens with them: token t goes to position
+ * seq_lens[b] - T + t, what an engine's step metadata says without a subtraction of its own on the device. */
+int tq_append_kv_newest(const void *k, const void *v, int dtype, int B, int T, int H, int64_t stride_b,
+                        int64_t stride_t, int64_t stride_h, const int32_t *seq_lens, const int32_t *block_table,
+                        int max_pages, const tq_layer *layer, const tq_page_layout *layout, uint8_t *pool,
+                        int64_t num_pages, void *stream);
+
 /* Ragged batch of runs (the batch counterpart of CompressedKVStore.append_chunk, store.py:73-90, for an
  * engine step that carries several sequences): k / v are (rows, H, d) `dtype` with element strides
  * stride_t / stride_h, the run of sequence b is rows row0[b] .. row0[b] + run_len[b] - 1 (run_len[b] <=

@@ -228,6 +228,26 @@ def test_steps_of_equal_length_are_those_of_equal_shares(gpu, d, kb, G, H, B, N,
         assert torch.equal(*outs) and bool(outs[0].any())
 
 
+@pytest.mark.parametrize("d,B,H,T,dtype", [(128, 32, 8, 1, torch.bfloat16), (128, 300, 2, 1, torch.float16), (128, 3, 2, 70, torch.bfloat16),
+                                           (256, 5, 1, 17, torch.float16), (64, 7, 3, 1, torch.bfloat16), (128, 4, 1, 3, torch.float32),
+                                           (576, 9, 1, 1, torch.bfloat16), (128, 2, 4, 1500, torch.bfloat16)])
+def test_append_of_the_newest_tokens_takes_the_lengths(gpu, d, B, H, T, dtype):
+    """Lengths with the new tokens, or the positions they begin at: every kernel of an append, the rows that begin or end on a page
+    boundary and a sequence whose length leaves no room for its tokens among them.  Byte for byte."""
+    g = torch.Generator(device=gpu).manual_seed(d + B + T)
+    tq = TurboQuantProd(d, bits=3, device=gpu)
+    per_seq = -(-(T + 40) // 16)
+    table = torch.randperm(B * per_seq, generator=g, device=gpu).view(B, per_seq).to(torch.int32)
+    lens = _i32([T + (0, 15, 16, 17, 33, -1)[b % 6] for b in range(B)], gpu)
+    k, v = torch.randn(2, B, T, H, d, generator=g, device=gpu).to(dtype)
+    _say(f"newest d={d} B={B} H={H} T={T} {dtype}")
+    pools = [PagedKVPool(tq, H, B * per_seq, value_bits=4, value_group_size=32, dtype=dtype, device=gpu) for _ in range(2)]
+    pools[0].append(k, v, table, start_pos=lens - T)
+    pools[1]._append_newest(k, v, table, lens)
+    torch.cuda.synchronize()
+    assert torch.equal(pools[0].data, pools[1].data) and bool(pools[0].data.any())
+
+
 # every count of column tiles per wavefront, 1 .. 4 bits, groups of one tile (up to a tile per compute unit) and of several, and
 # one tile more and less than that
 @pytest.mark.parametrize("d,key_bits,vb,dtype", [(64, 3, 2, torch.bfloat16), (192, 2, 4, torch.float16), (320, 5, 2, torch.bfloat16),

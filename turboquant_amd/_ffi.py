@@ -77,6 +77,8 @@ _SIGNATURES = {
     "tq_cache_attend": (C.c_int, [_vp, _i64, _i, _i64, _vp, _vp, _vp, _i64, _i, _i, _i, _vp, _i64, _i64, _i64, _i, _vp, _vp, _vp]),
     "tq_append_kv_paged": (C.c_int, [_vp, _vp, _i, _i, _i, _i, _i64, _i64, _i64, _vp, _vp, _i,
                                      C.POINTER(TqLayer), C.POINTER(TqPageLayout), _vp, _i64, _vp]),
+    "tq_append_kv_newest": (C.c_int, [_vp, _vp, _i, _i, _i, _i, _i64, _i64, _i64, _vp, _vp, _i,
+                                     C.POINTER(TqLayer), C.POINTER(TqPageLayout), _vp, _i64, _vp]),
     "tq_append_kv_ragged": (C.c_int, [_vp, _vp, _i, _i, _i, _i, _i64, _i64, _vp, _vp, _vp, _vp, _i,
                                       C.POINTER(TqLayer), C.POINTER(TqPageLayout), _vp, _i64, _vp]),
     "tq_append_kv_from_blocks": (C.c_int, [_vp, _vp, _i, _i, _i, _i, _i64, _i64, _i64, _vp, _i, _vp, _vp, _vp, _i,
@@ -136,7 +138,7 @@ def lib() -> C.CDLL:
     return _lib
 
 
-_HOST_CALLS = ("tq_quantize_keys", "tq_dequant_keys", "tq_score", "tq_ring_write", "tq_append_kv_paged", "tq_decode_workspace_bytes",
+_HOST_CALLS = ("tq_quantize_keys", "tq_dequant_keys", "tq_score", "tq_ring_write", "tq_append_kv_paged", "tq_append_kv_newest", "tq_decode_workspace_bytes",
                "tq_decode_attn_paged", "tq_decode_attn_paged_by_length", "tq_decode_attn_paged_ring", "tq_decode_attn_paged_ring_by_length",
                "tq_cache_append_bytes", "tq_cache_append", "tq_cache_scores_rows", "tq_cache_attend_bytes", "tq_cache_attend")
 

@@ -35,6 +35,7 @@ struct Library {
   decltype(&tq_score) score;
   decltype(&tq_ring_write) ring_write;
   decltype(&tq_append_kv_paged) append_kv_paged;
+  decltype(&tq_append_kv_newest) append_kv_newest;
   decltype(&tq_decode_workspace_bytes) decode_workspace_bytes;
   decltype(&tq_decode_attn_paged) decode_attn_paged;
   decltype(&tq_decode_attn_paged_by_length) decode_attn_paged_by_length;
@@ -47,7 +48,7 @@ struct Library {
   decltype(&tq_cache_attend) cache_attend;
 } g_lib{};
 constexpr const char* kNames[] = {"tq_quantize_keys", "tq_dequant_keys", "tq_score", "tq_ring_write", "tq_append_kv_paged",
-                                  "tq_decode_workspace_bytes", "tq_decode_attn_paged", "tq_decode_attn_paged_by_length",
+                                  "tq_append_kv_newest", "tq_decode_workspace_bytes", "tq_decode_attn_paged", "tq_decode_attn_paged_by_length",
                                   "tq_decode_attn_paged_ring", "tq_decode_attn_paged_ring_by_length", "tq_cache_append_bytes",
                                   "tq_cache_append", "tq_cache_scores_rows", "tq_cache_attend_bytes", "tq_cache_attend"};
 static_assert(sizeof(Library) == sizeof(kNames) / sizeof(kNames[0]) * sizeof(void*), "a pointer per name, in order");
@@ -257,12 +258,13 @@ PyObject* ring_write(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   return r;
 }
 
-// append(key, value (B, T, H, d), block table, start positions or None, pool, pages, H, d, dtype tag, layer, layout) -> True
+// append(key, value (B, T, H, d), block table, start positions or None, pool, pages, H, d, dtype tag, layer, layout, newest) -> True; newest: the
+// positions are the lengths with the new tokens
 PyObject* append(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
-  return entry<11>(args, n_args, [](PyObject* const* a) -> PyObject* {
+  return entry<12>(args, n_args, [](PyObject* const* a) -> PyObject* {
     Plain p;
     const at::Tensor key = p.take(a[0]), value = p.take(a[1]), table = p.take(a[2]), pool = p.take(a[4]);
-    const bool from_zero = a[3] == Py_None;
+    const bool from_zero = a[3] == Py_None, newest = a[11] == Py_True;
     at::Tensor start;
     if (!from_zero) start = p.take(a[3]);
     const int64_t pages = int_arg(a[5]), H = int_arg(a[6]), d = int_arg(a[7]), tag = int_arg(a[8]);
@@ -272,7 +274,7 @@ PyObject* append(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     const int64_t B = key.size(0), T = key.size(1);
     if (B > INT_MAX || T > INT_MAX || table.dim() != 2 || table.size(0) != B || table.size(1) > INT_MAX || !dense_as(table, at::kInt)) return nullptr;
     if (!from_zero && (start.dim() != 1 || start.size(0) != B || !dense_as(start, at::kInt))) return nullptr;
-    if (unlocked(g_lib.append_kv_paged, key.data_ptr(), value.data_ptr(), (int)tag, (int)B, (int)T, (int)H, key.stride(0), key.stride(1), key.stride(2),
+    if (unlocked(newest ? g_lib.append_kv_newest : g_lib.append_kv_paged, key.data_ptr(), value.data_ptr(), (int)tag, (int)B, (int)T, (int)H, key.stride(0), key.stride(1), key.stride(2),
                               from_zero ? nullptr : (const int32_t*)start.data_ptr(), (const int32_t*)table.data_ptr(), (int)table.size(1),
                               address<tq_layer>(a[9]), address<tq_page_layout>(a[10]), (uint8_t*)pool.data_ptr(), pages, p.stream()) != TQ_OK)
       return nullptr;

@@ -83,6 +83,7 @@ struct PagedSource {         // (b, t, h, :) strided, tokens mapped onto 16-toke
   // run of sequence b begins at row row0[b] (stride_b is unused, run_len gives its length).
   const int32_t* row0 = nullptr;
   int compact = 0;                       // (host) the kernels with a RaggedSource take this call
+  int start_add = 0;                     // added to start_pos[b]: -T where start_pos holds the runs' ends
   // (sequence, page slot window, head) of a tile, and of the tile after it (a walk that leaves the last
   // sequence stays on its last tile): the divisions by run-time sizes are done once per group of tiles
   struct Coord { int b, pg, h; };
@@ -113,6 +114,7 @@ struct PagedSource {         // (b, t, h, :) strided, tokens mapped onto 16-toke
     if (row0) sload<N>(row0, at, r0);
 #pragma unroll
     for (int m = 0; m < N; ++m) {
+      s0[m] += start_add;
       lpage[m] = s0[m] / TILE + c[m].pg;
       at[m] = c[m].b * src_stride + min(lpage[m], src_stride - 1);
     }
@@ -132,7 +134,7 @@ struct PagedSource {         // (b, t, h, :) strided, tokens mapped onto 16-toke
     int r = tile / H;
     int pg = r % tiles_per_seq;
     b = r / tiles_per_seq;
-    int s0 = start_pos ? start_pos[b] : 0;
+    int s0 = start_pos ? start_pos[b] + start_add : 0;
     lpage = s0 / TILE + pg;
   }
   // the part of locate() that is the same for the 16 slots of a tile
@@ -144,7 +146,7 @@ struct PagedSource {         // (b, t, h, :) strided, tokens mapped onto 16-toke
     int b = r / tiles_per_seq;
     // unconditional loads (no branch on the null pointers): a load under a branch makes the
     // compiler wait for every outstanding load at the join
-    int s0 = *(start_pos ? start_pos + b : &k_zero_i32);
+    int s0 = *(start_pos ? start_pos + b : &k_zero_i32) + start_add;
     const int lpage = s0 / TILE + pg, t0 = lpage * TILE - s0;
     const int lim = min(*(run_len ? run_len + b : &k_max_i32), T);
     const int64_t blk = *(src_table ? src_table + (int64_t)b * src_stride + min(lpage, src_stride - 1) : &k_zero_i32);
@@ -169,7 +171,7 @@ struct PagedSource {         // (b, t, h, :) strided, tokens mapped onto 16-toke
 struct RaggedSource : PagedSource {
   static constexpr int MAX_COMPACT = 1024;     // sequences
   __device__ int run_pages(int b) const {
-    const int s0 = start_pos ? start_pos[b] : 0, n = min(run_len[b], T);
+    const int s0 = start_pos ? start_pos[b] + start_add : 0, n = min(run_len[b], T);
     return n > 0 ? (s0 % TILE + n + TILE - 1) / TILE : 0;
   }
   // cum[b] = pages of the sequences before b, b = 0 .. B; called by all NT threads of the workgroup (with a barrier)

@@ -701,10 +701,9 @@ static int append_runs(const void* k, const void* v, int dtype, const PagedSourc
   return launch_value(v, dtype, src, layer->d, layout->group_size, layout->value_bits, vs, tiles, (hipStream_t)stream);
 }
 
-extern "C" int tq_append_kv_paged(const void* k, const void* v, int dtype, int B, int T, int H, int64_t stride_b,
-                                  int64_t stride_t, int64_t stride_h, const int32_t* start_pos,
-                                  const int32_t* block_table, int max_pages, const tq_layer* layer,
-                                  const tq_page_layout* layout, uint8_t* pool, int64_t num_pages, void* stream) {
+static int append_paged(const void* k, const void* v, int dtype, int B, int T, int H, int64_t stride_b, int64_t stride_t, int64_t stride_h,
+                        const int32_t* start_pos, int start_add, const int32_t* block_table, int max_pages, const tq_layer* layer,
+                        const tq_page_layout* layout, uint8_t* pool, int64_t num_pages, void* stream) {
   int rc = check_layer(layer, true);
   if (rc) return rc;
   if (!k || !v || !block_table || !layout || !pool) return TQ_ENULL;
@@ -718,7 +717,25 @@ extern "C" int tq_append_kv_paged(const void* k, const void* v, int dtype, int B
   // (the run may begin at any of the 16 slots of its first page when start_pos is given)
   const int tiles_per_seq = start_pos ? (T + TILE - 2) / TILE + 1 : (T + TILE - 1) / TILE;
   PagedSource src{B, T, H, tiles_per_seq, stride_b, stride_t, stride_h, start_pos};
+  src.start_add = start_add;
   return append_runs(k, v, dtype, src, block_table, max_pages, layer, layout, pool, num_pages, stream);
+}
+
+extern "C" int tq_append_kv_paged(const void* k, const void* v, int dtype, int B, int T, int H, int64_t stride_b,
+                                  int64_t stride_t, int64_t stride_h, const int32_t* start_pos,
+                                  const int32_t* block_table, int max_pages, const tq_layer* layer,
+                                  const tq_page_layout* layout, uint8_t* pool, int64_t num_pages, void* stream) {
+  return append_paged(k, v, dtype, B, T, H, stride_b, stride_t, stride_h, start_pos, 0, block_table, max_pages, layer, layout, pool, num_pages,
+                      stream);
+}
+
+extern "C" int tq_append_kv_newest(const void* k, const void* v, int dtype, int B, int T, int H, int64_t stride_b,
+                                   int64_t stride_t, int64_t stride_h, const int32_t* seq_lens,
+                                   const int32_t* block_table, int max_pages, const tq_layer* layer,
+                                   const tq_page_layout* layout, uint8_t* pool, int64_t num_pages, void* stream) {
+  if (!seq_lens) return TQ_ENULL;
+  return append_paged(k, v, dtype, B, T, H, stride_b, stride_t, stride_h, seq_lens, -T, block_table, max_pages, layer, layout, pool, num_pages,
+                      stream);
 }
 
 extern "C" int tq_append_kv_ragged(const void* k, const void* v, int dtype, int B, int T_max, int H, int64_t stride_t,

@@ -76,8 +76,7 @@ class BatchedLayerState:
         v = value[:n].reshape(n, cfg.num_kv_heads, cfg.head_dim)
         table = meta.block_table
         if int(meta.max_query_len) == 1:                       # one token per sequence: a single batched append
-            start = meta.seq_lens.to(torch.int32) - 1
-            self.pool.append(k[:, None], v[:, None], table, start_pos=start)
+            self.pool._append_newest(k[:, None], v[:, None], table, meta.seq_lens)
         else:                                                  # ragged rows: still one call, nothing read back
             qsl = meta.query_start_loc.to(device=k.device, dtype=torch.int32)
             run = qsl[1:] - qsl[:-1]
