@@ -817,8 +817,9 @@ def test_cache_scores_of_queries_that_lie_apart(gpu, d, B, H, n_c, n_q, step):
     cache.prefill(k, v)
     part = q[..., 1 % step::step, :] if n_q > 1 else q[..., step - 1:, :]
     assert torch.equal(cache.attention_scores(part), cache.attention_scores(part.clone(memory_format=torch.contiguous_format)))
-    wide = torch.randn(B, H, n_q, 2 * d, generator=g).to(gpu)[..., d:]
-    assert torch.equal(cache.attention_scores(wide), cache.attention_scores(wide.contiguous()))
+    for pad in (0, 1):                                  # rows on 16-byte boundaries, and a word off them
+        wide = torch.randn(B, H, n_q, 2 * d + pad, generator=g).to(gpu)[..., d + pad:]
+        assert torch.equal(cache.attention_scores(wide), cache.attention_scores(wide.contiguous()))
 
 
 @pytest.mark.parametrize("d,H,n_c,n_buf,vb", [(64, 8, 1000, 128, 2), (128, 8, 300, 128, 4), (256, 3, 2000, 33, 2)])
