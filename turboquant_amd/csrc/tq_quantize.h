@@ -76,17 +76,18 @@ struct PagedSource {         // (b, t, h, :) strided, tokens mapped onto 16-toke
   // are stride_blk elements apart and stride_b is unused.  run_len (optional) bounds the run of each
   // sequence separately (<= T).
   const int32_t* src_table = nullptr;
-  int src_stride = 0;
+  int src_stride = 0;                    // without src_table: what is added to start_pos[b], -T where that holds the runs' ends
   int64_t stride_blk = 0;
   const int32_t* run_len = nullptr;
   // Optional ragged mode: the rows of all sequences lie one after another in one (rows, H, :) tensor; the
   // run of sequence b begins at row row0[b] (stride_b is unused, run_len gives its length).
   const int32_t* row0 = nullptr;
   int compact = 0;                       // (host) the kernels with a RaggedSource take this call
-  int start_add = 0;                     // added to start_pos[b]: -T where start_pos holds the runs' ends
   // (sequence, page slot window, head) of a tile, and of the tile after it (a walk that leaves the last
   // sequence stays on its last tile): the divisions by run-time sizes are done once per group of tiles
   struct Coord { int b, pg, h; };
+  // (a member of its own is another wait for arguments in front of every tile: a token of 17 sequences of a head of 256 15.86 -> 16.04 us, now 15.90)
+  __device__ int start_add() const { return src_table ? 0 : src_stride; }
   __device__ Coord coord(int64_t tile) const {
     Coord c;
     c.h = (int)tile % H;
@@ -114,7 +115,7 @@ struct PagedSource {         // (b, t, h, :) strided, tokens mapped onto 16-toke
     if (row0) sload<N>(row0, at, r0);
 #pragma unroll
     for (int m = 0; m < N; ++m) {
-      s0[m] += start_add;
+      s0[m] += start_add();
       lpage[m] = s0[m] / TILE + c[m].pg;
       at[m] = c[m].b * src_stride + min(lpage[m], src_stride - 1);
     }
@@ -134,7 +135,7 @@ struct PagedSource {         // (b, t, h, :) strided, tokens mapped onto 16-toke
     int r = tile / H;
     int pg = r % tiles_per_seq;
     b = r / tiles_per_seq;
-    int s0 = start_pos ? start_pos[b] + start_add : 0;
+    int s0 = start_pos ? start_pos[b] + start_add() : 0;
     lpage = s0 / TILE + pg;
   }
   // the part of locate() that is the same for the 16 slots of a tile
@@ -146,7 +147,7 @@ struct PagedSource {         // (b, t, h, :) strided, tokens mapped onto 16-toke
     int b = r / tiles_per_seq;
     // unconditional loads (no branch on the null pointers): a load under a branch makes the
     // compiler wait for every outstanding load at the join
-    int s0 = *(start_pos ? start_pos + b : &k_zero_i32) + start_add;
+    int s0 = *(start_pos ? start_pos + b : &k_zero_i32) + start_add();
     const int lpage = s0 / TILE + pg, t0 = lpage * TILE - s0;
     const int lim = min(*(run_len ? run_len + b : &k_max_i32), T);
     const int64_t blk = *(src_table ? src_table + (int64_t)b * src_stride + min(lpage, src_stride - 1) : &k_zero_i32);
@@ -171,7 +172,7 @@ struct PagedSource {         // (b, t, h, :) strided, tokens mapped onto 16-toke
 struct RaggedSource : PagedSource {
   static constexpr int MAX_COMPACT = 1024;     // sequences
   __device__ int run_pages(int b) const {
-    const int s0 = start_pos ? start_pos[b] + start_add : 0, n = min(run_len[b], T);
+    const int s0 = start_pos ? start_pos[b] + start_add() : 0, n = min(run_len[b], T);
     return n > 0 ? (s0 % TILE + n + TILE - 1) / TILE : 0;
   }
   // cum[b] = pages of the sequences before b, b = 0 .. B; called by all NT threads of the workgroup (with a barrier)
@@ -230,7 +231,11 @@ struct KeyFlatSink {
   float* rnorm;
   float* y_dbg;
   float* p_dbg;
-  int64_t step = 1;        // rows from one vector to the next (matrix-core kernels of 128 / 256)
+  static constexpr int64_t step = 1;
+};
+
+struct KeyRowsSink : KeyFlatSink {         // `step` rows from one vector to the next (a type of its own: the others' stores carry no product)
+  int64_t step;
 };
 
 struct KeyPagedSink {

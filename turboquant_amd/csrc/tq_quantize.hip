@@ -717,7 +717,7 @@ static int append_paged(const void* k, const void* v, int dtype, int B, int T, i
   // (the run may begin at any of the 16 slots of its first page when start_pos is given)
   const int tiles_per_seq = start_pos ? (T + TILE - 2) / TILE + 1 : (T + TILE - 1) / TILE;
   PagedSource src{B, T, H, tiles_per_seq, stride_b, stride_t, stride_h, start_pos};
-  src.start_add = start_add;
+  src.src_stride = start_add;
   return append_runs(k, v, dtype, src, block_table, max_pages, layer, layout, pool, num_pages, stream);
 }
 

@@ -359,7 +359,7 @@ __device__ __forceinline__ int64_t key_mfma_body(const void* __restrict__ x, con
   // page of that tile, read now so that the write phase does not wait for it (a page outside the table or
   // the pool comes back as -1 and is not written)
   int64_t wpage = 0;
-  if constexpr (!std::is_same<Sink, KeyFlatSink>::value) {
+  if constexpr (!std::is_base_of<KeyFlatSink, Sink>::value) {
     if (tile0 + wave % ML < end) wpage = checked_page(sink.block_table, sink.max_pages, sink.num_pages, wr_b, wr_lpage);
   }
   stg.template store<XRS>(sx, svalid, tid);
@@ -472,7 +472,7 @@ __device__ __forceinline__ int64_t key_mfma_body(const void* __restrict__ x, con
             if constexpr (TWO) spl[(1 * TT + t) * W + (wave * NPW) / 2 + wl] = lo;
           }
         }
-        if constexpr (std::is_same<Sink, KeyFlatSink>::value) {
+        if constexpr (std::is_base_of<KeyFlatSink, Sink>::value) {
 #pragma unroll
           for (int c = 0; c < NPW; ++c) {
             const int col0 = 16 * (wave * NPW + c) + 4 * kb;
@@ -531,7 +531,7 @@ __device__ __forceinline__ int64_t key_mfma_body(const void* __restrict__ x, con
           *(u32x2*)(terms + ((size_t)1 * TT + t) * RS + col0) = t1;
           *(u32x2*)(terms + ((size_t)2 * TT + t) * RS + col0) = t2;
         }
-        if constexpr (std::is_same<Sink, KeyFlatSink>::value) {
+        if constexpr (std::is_base_of<KeyFlatSink, Sink>::value) {
           if (sink.y_dbg && svalid[t]) *(f32x4*)(sink.y_dbg + (tile0 * TILE + t) * D + col0) = acc[m][c];
         }
       }
@@ -650,7 +650,7 @@ __device__ __forceinline__ int64_t key_mfma_body(const void* __restrict__ x, con
         v = or_over_kb(v << (4 * kb));
         if (kb == 0) spl[(mb * TT + t) * W + (wave * NPW) / 2 + wl] = v;
       }
-      if constexpr (std::is_same<Sink, KeyFlatSink>::value) {
+      if constexpr (std::is_base_of<KeyFlatSink, Sink>::value) {
         if (sink.p_dbg && svalid[t]) {
 #pragma unroll
           for (int c = 0; c < NPW; ++c)
@@ -661,7 +661,7 @@ __device__ __forceinline__ int64_t key_mfma_body(const void* __restrict__ x, con
   }
   __syncthreads();
   // (6) write
-  if constexpr (std::is_same<Sink, KeyFlatSink>::value) {
+  if constexpr (std::is_base_of<KeyFlatSink, Sink>::value) {
     // flat format of the reference (quantizer.py:38-69): indices packed eff_bits apiece, signs 8 per byte
     // A thread builds one dword of a row: n = 32 / eff codes, code s at bit eff * s, plane 0 the top bit of a
     // code.  The n bits a plane contributes are spread to a stride of eff bits with shift-and-mask steps.
@@ -780,14 +780,14 @@ append_small_kernel(const void* __restrict__ k, const void* __restrict__ v, Page
 // behind one another.
 template <int D, bool FX>
 __global__ void __launch_bounds__(KQ_THREADS, 2)
-cache_append_kernel(const float* __restrict__ keys, FlatSource src, tq_layer ly, KeyFlatSink ks, int n_tiles, CacheRest rest) {
+cache_append_kernel(const float* __restrict__ keys, FlatSource src, tq_layer ly, KeyRowsSink ks, int n_tiles, CacheRest rest) {
   extern __shared__ __align__(16) unsigned char smem[];
   if ((int)blockIdx.x >= n_tiles) {
     cache_rest_body(rest, (int)blockIdx.x - n_tiles);
     return;
   }
   int64_t end = n_tiles;
-  key_mfma_body<TQ_F32, D, false, FX, FlatSource, KeyFlatSink, 1>(keys, src, ly, ks, 0, end, blockIdx.x, n_tiles, smem);
+  key_mfma_body<TQ_F32, D, false, FX, FlatSource, KeyRowsSink, 1>(keys, src, ly, ks, 0, end, blockIdx.x, n_tiles, smem);
 }
 
 __host__ static bool aligned_for_chunks(const void* x, int dtype, const FlatSource& s) {
@@ -892,7 +892,7 @@ static int launch_append_small_d(const void* k, const void* v, const PagedSource
 }
 
 template <int D, bool FX>
-static int launch_cache_append_d(const float* keys, const FlatSource& src, const tq_layer& ly, const KeyFlatSink& ks, int tiles,
+static int launch_cache_append_d(const float* keys, const FlatSource& src, const tq_layer& ly, const KeyRowsSink& ks, int tiles,
                                  const CacheRest& rest, hipStream_t st) {
   constexpr size_t smem = KeySmem<TQ_F32, D>::bytes;
   auto kern = cache_append_kernel<D, FX>;
@@ -912,7 +912,7 @@ static int launch_cache_append_d(const float* keys, const FlatSource& src, const
 // The whole token in one launch, at head_dim 128 / 256.  Every workgroup of it reserves a key tile's LDS, so a compute unit holds one: up to
 // twelve rounds of copies (48 MB; four tokens and their attention, one launch and two: of 15 MB 361 and 383 us, of 31 MB 733 and 766, of
 // 62 MB 1172 and 1164); beyond, and where the matrix-core kernel does not take the keys, TQ_EUNSUPPORTED: the caller launches two.
-int launch_cache_append(const float* keys, int64_t stride, int64_t rows, const tq_layer& ly, const KeyFlatSink& ks, const CacheRest& rest,
+int launch_cache_append(const float* keys, int64_t stride, int64_t rows, const tq_layer& ly, const KeyRowsSink& ks, const CacheRest& rest,
                         hipStream_t st) {
   const FlatSource src{rows, stride};
   const int64_t tiles = (rows + TILE - 1) / TILE;

@@ -834,7 +834,7 @@ namespace tq {
 // (values and copies of a token, behind the key quantiser's launch: one launch where a concatenation per section, and its host time, stood)
 __global__ void __launch_bounds__(256) cache_rest_kernel(CacheRest A) { cache_rest_body(A, (int)blockIdx.x); }
 
-int launch_cache_append(const float* keys, int64_t stride, int64_t rows, const tq_layer& ly, const KeyFlatSink& ks, const CacheRest& rest, hipStream_t st);
+int launch_cache_append(const float* keys, int64_t stride, int64_t rows, const tq_layer& ly, const KeyRowsSink& ks, const CacheRest& rest, hipStream_t st);
 
 // Weighted sum of the values: a share of the compressed tokens, or 32 exact rows, per workgroup.  A thread owns one word of
 // codes (32 / VB channels of one group) of every 256 / words-th token of the share; code * scale + zero rounds twice, as
@@ -976,8 +976,7 @@ extern "C" int tq_cache_append(const float* key, const float* value, int64_t key
   if (rc) return rc;
   if (!layer->thresholds) return TQ_ENULL;
   if (!key_sections(false)) return TQ_EUNSUPPORTED;
-  KeyFlatSink ks{idx_out + (size_t)n * ib, signs_out + (size_t)n * sb, norms_out + n, rnorms_out + n, nullptr, nullptr};
-  ks.step = n + 1;
+  const KeyRowsSink ks{{idx_out + (size_t)n * ib, signs_out + (size_t)n * sb, norms_out + n, rnorms_out + n, nullptr, nullptr}, (int64_t)n + 1};
   rc = launch_cache_append(key_buf, ks_h, batch, *layer, ks, A, (hipStream_t)stream);
   if (rc != TQ_EUNSUPPORTED) return rc;
   if (!key_sections(true)) return TQ_EUNSUPPORTED;
