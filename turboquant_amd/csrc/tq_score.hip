@@ -22,16 +22,17 @@ constexpr int ROT_SLICES = 8;      // (ROT_COLS = 32 output columns per workgrou
 // sq[0 .. tot) = the first `have` elements of row row0 of q and those behind it as fp32, zeros behind them (have and tot multiples of 8):
 // 16-byte loads, all of a thread's in flight together, when q allows them.  fp32 rows of d may lie q_row > d elements apart (a word at a time,
 // 8 rows of 128 took four loads behind one another: the rotation 6.5 us, now 5.5).
+template <bool APART>
 __device__ __forceinline__ void rows_to_lds(const void* __restrict__ q, int dtype, int64_t row0, int have, int tot,
                                             float* __restrict__ sq, int tid, int n_threads, int d, int64_t q_row) {
   const int64_t off = row0 * d;
-  if (q_row != d && ((uintptr_t)q & 15) == 0 && q_row % 4 == 0) {
+  if (APART && ((uintptr_t)q & 15) == 0 && q_row % 4 == 0) {
     const float* src = (const float*)q + row0 * q_row;
     const unsigned per = (unsigned)d / 4;
 #pragma unroll 2
     for (int c = tid; c < tot / 4; c += n_threads)
       *(float4*)(sq + 4 * c) = 4 * c < have ? *(const float4*)(src + (unsigned)c / per * q_row + (unsigned)c % per * 4) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  } else if (q_row != d) {
+  } else if (APART) {
     const float* src = (const float*)q + row0 * q_row;
     for (int o = tid; o < tot; o += n_threads) sq[o] = o < have ? src[o / d * q_row + o % d] : 0.0f;
   } else if ((((uintptr_t)q) & 15) == 0 && dtype != TQ_F32) {
@@ -72,7 +73,8 @@ __device__ __forceinline__ void rows_to_lds(const void* __restrict__ q, int dtyp
 // and the workgroups of the first word write the rows' statistics.  The operands are normalised by bounds every
 // workgroup can compute from the raw query: |q_rot_j| <= ||q|| (Pi is orthogonal) and |q_sk_j| <= ||q|| max_j ||S_j||;
 // the sums over all coordinates the scores need are q . colsum(Pi), q . colsum(S).
-template <int BATCH, int HALVES, bool PACK>
+// APART: rows of q that are not one behind another (an instance of its own: 45 rows of 64 took 4.6 us without the branch and 5.0 with it)
+template <int BATCH, int HALVES, bool PACK, bool APART>
 __global__ void __launch_bounds__(ROT_COLS * ROT_SLICES * HALVES)
 rotate_query_kernel(const void* __restrict__ q, int dtype, int64_t rows, int R, tq_layer ly, float* __restrict__ q_rot,
                     float* __restrict__ q_sk, WidePack wp, int64_t q_row) {
@@ -103,7 +105,7 @@ rotate_query_kernel(const void* __restrict__ q, int dtype, int64_t rows, int R, 
       cs2[k] = ly.S_colsum[c];
     }
   }
-  rows_to_lds(q, dtype, row0, nr * d, R * d, sq, tid, (int)blockDim.x, d, q_row);
+  rows_to_lds<APART>(q, dtype, row0, nr * d, R * d, sq, tid, (int)blockDim.x, d, q_row);
   __syncthreads();
   float* s_rot = pb + ROT_SLICES * R * ROT_COLS;   // PACK: [R][ROT_COLS] this word's rotated values, then the sketched ones
   float* s_sk = s_rot + R * ROT_COLS;
@@ -721,7 +723,8 @@ int launch_rotate_query(const void* q, int dtype, int64_t rows, const tq_layer* 
   const int per = d / ROT_SLICES;
 #define TQ_ROTATE(BATCH, MAXR)                                                                                         \
   {                                                                                                                    \
-    auto kern = pack ? rotate_query_kernel<BATCH, MAXR, true> : rotate_query_kernel<BATCH, MAXR, false>;             \
+    auto kern = pack ? rotate_query_kernel<BATCH, MAXR, true, false> : rotate_query_kernel<BATCH, MAXR, false, false>; \
+    if (q_row != layer->d) kern = rotate_query_kernel<BATCH, MAXR, false, true>;                                       \
     if (smem > 48 * 1024) {                                                                                            \
       hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);    \
       if (e != hipSuccess) return (int)e;                                                                              \
