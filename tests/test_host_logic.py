@@ -4,9 +4,11 @@ geometry, codebook files, ring / capture policy against the reference's trace,
 and the loud failure on CPU tensors."""
 
 import ctypes as C
+import gc
 import json
 import os
 import re
+import weakref
 
 import numpy as np
 import pytest
@@ -584,3 +586,77 @@ def test_splits_of_many_heads_in_the_static_area():
                     assert n == free or 1 <= n < free and need(B, Hq, n + 1) > _ffi.NOALLOC_SCRATCH_BYTES
                     assert n == 1 or need(B, Hq, n) <= _ffi.NOALLOC_SCRATCH_BYTES
         assert pool.default_splits(1, 65536, 128, True) >= 32 and pool.default_splits(1, 8192, 128, True) >= 16
+
+
+class _Evicting:
+    """A native host side that has another descriptor built before it reads the one of the call (as another thread may while the call has
+    given up the interpreter's lock), and says whether that one and its matrices are still there."""
+
+    def __init__(self, rebuild, built):
+        self.rebuild, self.built, self.calls = rebuild, built, []
+
+    def __getattr__(self, name):
+        def call(*args):
+            self.rebuild()
+            gc.collect()
+            self.calls.append(name)
+            assert self.built[-1]() is not None, f"{name}: the descriptor was freed under the call"
+            assert all(t() is not None for t in self.built[-1].terms), f"{name}: the matrices it points to were freed under the call"
+            raise _Seen
+        return call
+
+
+class _Seen(Exception):
+    pass
+
+
+def test_a_descriptor_outlives_the_native_call_that_reads_it(monkeypatch):
+    """Every call of the native host side, with the quantiser's kept descriptor replaced in the middle of it."""
+    from turboquant_amd.kv_cache import TurboQuantKVCache
+    from turboquant_amd.paged import PagedKVPool
+    from turboquant_amd.quantizer import ProdQuantized
+    monkeypatch.setattr(_ffi, "require_gpu", lambda t, name: t)
+    tq = TurboQuantProd(128, bits=3, device="cpu")
+    built, build = [], tq._layer
+
+    class Ref(weakref.ref):
+        terms = ()
+
+    def layer():
+        ly = build()
+        ref = Ref(ly)
+        ref.terms = [weakref.ref(t) for t in (*tq.mse_quantizer._splits[1][:4], *tq.mse_quantizer._splits[1][4])]
+        built.append(ref)
+        return ly
+    tq._layer = layer
+
+    def rebuild():
+        tq.S.add_(0)                                           # (a buffer that is written)
+        build()
+    _ffi.lib()
+    host = _Evicting(rebuild, built)
+    monkeypatch.setattr(_ffi, "_host", host)
+    pool = PagedKVPool.__new__(PagedKVPool)
+    pool.quantizer, pool.head_dim, pool.num_kv_heads, pool.value_bits, pool.value_group_size = tq, 128, 2, 4, 32
+    pool.dtype, pool.device, pool.num_pages = torch.bfloat16, torch.device("cpu"), 4
+    pool.layout = _ffi.make_page_layout(128, 2, 4, 32, torch.bfloat16)
+    pool.data = torch.zeros(4, 2, pool.layout.page_bytes, dtype=torch.uint8)
+    cache = TurboQuantKVCache(128, buffer_size=3, device="cpu", dtype=torch.float32)
+    cache.key_quantizer = tq
+    rows = torch.zeros(1, 2, 3, 128)
+    code = ProdQuantized(torch.zeros(1, 2, 5, 32, dtype=torch.uint8), torch.zeros(1, 2, 5, 16, dtype=torch.uint8), torch.zeros(1, 2, 5), torch.zeros(1, 2, 5), 2)
+    cache.key_quantized, cache.key_buffer, cache.value_buffer = code, rows, rows
+    cache.value_quantized = ValueQuantized(torch.zeros(1, 2, 5, 32, dtype=torch.uint8), torch.zeros(1, 2, 5, 4), torch.zeros(1, 2, 5, 4), 2)
+    kv = torch.zeros(1, 1, 2, 128, dtype=torch.bfloat16)
+    q = torch.zeros(1, 4, 128, dtype=torch.bfloat16)
+    table, one = torch.zeros(1, 4, dtype=torch.int32), torch.ones(1, dtype=torch.int32)
+    exact = torch.zeros(4, 16, 2, 128, dtype=torch.bfloat16)
+    calls = [("quantize", lambda: tq.quantize(rows)), ("dequantize", lambda: tq.dequantize(code)), ("score", lambda: tq.attention_score(rows, code)),
+             ("append", lambda: pool.append(kv, kv, table)), ("append", lambda: pool._append_newest(kv, kv, table, one)),
+             ("decode", lambda: pool.decode_attention(q, table, one)),
+             ("decode_ring", lambda: pool.decode_attention_ring(q, table, one, exact, exact, 16)),
+             ("cache_append", lambda: cache.append(rows[..., :1, :], rows[..., :1, :])), ("cache_scores", lambda: cache.attention_scores(rows))]
+    for name, call in calls:
+        with pytest.raises(_Seen):
+            call()
+        assert host.calls[-1] == name

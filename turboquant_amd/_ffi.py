@@ -257,8 +257,7 @@ def walsh_terms(centroids_host: torch.Tensor, mse_bits: int, layer: TqLayer):
 def make_layer(d: int, mse_bits: int, Pi: torch.Tensor, PiT: torch.Tensor, centroids: torch.Tensor,
                thresholds: torch.Tensor, S: Optional[torch.Tensor] = None, ST: Optional[torch.Tensor] = None,
                centroids_host: Optional[torch.Tensor] = None, splits=None, query_consts=None) -> TqLayer:
-    """Describe a layer's constants to the library.  The tensors must stay alive
-    while the struct is in use; they must be fp32, contiguous and on one GPU."""
+    """Describe a layer's constants to the library.  The tensors must be fp32, contiguous and on one GPU; the struct keeps them."""
     for name, t in (("Pi", Pi), ("PiT", PiT), ("centroids", centroids), ("thresholds", thresholds), ("S", S), ("ST", ST)):
         if t is None:
             continue
@@ -283,6 +282,8 @@ def make_layer(d: int, mse_bits: int, Pi: torch.Tensor, PiT: torch.Tensor, centr
     if query_consts is not None:
         pi_cs, s_cs, s_max = query_consts
         ly.Pi_colsum, ly.S_colsum, ly.S_rownorm_max = pi_cs.data_ptr(), s_cs.data_ptr(), float(s_max)
+    # (a caller that holds the struct holds what it points to, whatever its quantiser builds or moves meanwhile)
+    ly.tensors = (Pi, PiT, S, ST, centroids, thresholds, splits, query_consts)
     walsh_terms(centroids_host if centroids_host is not None else centroids.detach().cpu(), mse_bits, ly)
     return ly
 

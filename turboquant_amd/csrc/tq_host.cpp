@@ -108,7 +108,20 @@ int dtype_tag(at::ScalarType t) {
 }
 int code_bits(int mse_bits) { return mse_bits == 1 ? 1 : mse_bits == 2 ? 2 : mse_bits <= 4 ? 4 : 8; }
 int64_t int_arg(PyObject* o) { return PyLong_AsLongLong(o); }
-template <class T> const T* address(PyObject* o) { return (const T*)PyLong_AsVoidPtr(o); }
+// The memory of a descriptor (a ctypes structure), and a reference to it: the library reads it while the interpreter's lock is given up, and
+// another thread may make its owner build a new one meanwhile.
+template <class T> class Held {
+  Py_buffer view_{};
+
+ public:
+  explicit Held(PyObject* o) {
+    if (PyObject_GetBuffer(o, &view_, PyBUF_SIMPLE) == 0 && view_.len != (Py_ssize_t)sizeof(T)) PyErr_SetString(PyExc_TypeError, "not that descriptor");
+  }
+  ~Held() { PyBuffer_Release(&view_); }
+  Held(const Held&) = delete;
+  Held& operator=(const Held&) = delete;
+  const T* get() const { return (const T*)view_.buf; }
+};
 bool dense_as(const at::Tensor& t, at::ScalarType dt) { return t.scalar_type() == dt && t.is_contiguous(); }
 std::vector<int64_t> shape(at::IntArrayRef lead, std::initializer_list<int64_t> tail = {}) {
   std::vector<int64_t> s(lead.begin(), lead.end());
@@ -156,6 +169,7 @@ PyObject* quantize(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     const at::Tensor x = p.take(a[0]);
     const int64_t d = int_arg(a[2]);
     const int mb = (int)int_arg(a[3]);
+    const Held<tq_layer> layer(a[1]);
     if (!p.ok || PyErr_Occurred() || d <= 0 || x.dim() < 1 || x.size(-1) != d || x.numel() == 0 || !x.is_contiguous()) return nullptr;
     const int tag = dtype_tag(x.scalar_type()), per = 8 / code_bits(mb);
     if (tag < 0) return nullptr;
@@ -163,7 +177,7 @@ PyObject* quantize(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     constexpr auto bytes = at::kByte;
     at::Tensor idx = p.fresh(shape(lead, {(d + per - 1) / per}), bytes), sgn = p.fresh(shape(lead, {(d + 7) / 8}), bytes);
     at::Tensor nrm = p.fresh(lead, x.scalar_type()), rn = p.fresh(lead, at::kFloat);
-    if (unlocked(g_lib.quantize_keys, x.data_ptr(), tag, x.numel() / d, d, address<tq_layer>(a[1]), (uint8_t*)idx.data_ptr(), (uint8_t*)sgn.data_ptr(),
+    if (unlocked(g_lib.quantize_keys, x.data_ptr(), tag, x.numel() / d, d, layer.get(), (uint8_t*)idx.data_ptr(), (uint8_t*)sgn.data_ptr(),
                             nrm.data_ptr(), (float*)rn.data_ptr(), nullptr, nullptr, 0, p.stream()) != TQ_OK)
       return nullptr;
     return tuple({idx, sgn, rn, nrm});
@@ -194,10 +208,11 @@ PyObject* dequantize(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     Codes c;
     const int64_t d = int_arg(a[5]);
     const int mb = (int)int_arg(a[6]);
+    const Held<tq_layer> layer(a[4]);
     if (PyErr_Occurred() || !c.take(p, a, d, mb)) return nullptr;
     at::Tensor out = p.fresh(shape(c.nrm.sizes(), {d}), at::kFloat);
     if (unlocked(g_lib.dequant_keys, (const uint8_t*)c.idx.data_ptr(), (const uint8_t*)c.sgn.data_ptr(), c.nrm.data_ptr(), dtype_tag(c.nrm.scalar_type()),
-                           (const float*)c.rn.data_ptr(), c.n, address<tq_layer>(a[4]), (float*)out.data_ptr(), p.stream()) != TQ_OK)
+                           (const float*)c.rn.data_ptr(), c.n, layer.get(), (float*)out.data_ptr(), p.stream()) != TQ_OK)
       return nullptr;
     return THPVariable_Wrap(out);
   });
@@ -211,6 +226,7 @@ PyObject* score(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     Codes c;
     const int64_t d = int_arg(a[6]);
     const int mb = (int)int_arg(a[7]);
+    const Held<tq_layer> layer(a[5]);
     if (PyErr_Occurred() || !c.take(p, a + 1, d, mb)) return nullptr;
     const int tag = dtype_tag(q.scalar_type());
     if (tag < 0 || !q.is_contiguous() || q.dim() != c.nrm.dim() + 1 || q.size(-1) != d || q.numel() == 0) return nullptr;
@@ -219,7 +235,7 @@ PyObject* score(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     const int64_t n_q = q.size(-2), n_k = c.nrm.size(-1), batch = c.n / n_k;
     at::Tensor out = p.fresh(shape(lead, {n_q, n_k}), at::kFloat), work = p.fresh({2 * batch * n_q * d}, at::kFloat);
     if (unlocked(g_lib.score, q.data_ptr(), tag, batch, n_q, (const uint8_t*)c.idx.data_ptr(), (const uint8_t*)c.sgn.data_ptr(), c.nrm.data_ptr(),
-                    dtype_tag(c.nrm.scalar_type()), (const float*)c.rn.data_ptr(), n_k, address<tq_layer>(a[5]), (float*)out.data_ptr(),
+                    dtype_tag(c.nrm.scalar_type()), (const float*)c.rn.data_ptr(), n_k, layer.get(), (float*)out.data_ptr(),
                     (float*)work.data_ptr(), p.stream()) != TQ_OK)
       return nullptr;
     return THPVariable_Wrap(out);
@@ -268,6 +284,8 @@ PyObject* append(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     at::Tensor start;
     if (!from_zero) start = p.take(a[3]);
     const int64_t pages = int_arg(a[5]), H = int_arg(a[6]), d = int_arg(a[7]), tag = int_arg(a[8]);
+    const Held<tq_layer> layer(a[9]);
+    const Held<tq_page_layout> layout(a[10]);
     if (!p.ok || PyErr_Occurred() || key.dim() != 4 || key.sizes() != value.sizes() || key.strides() != value.strides()) return nullptr;
     if (key.size(2) != H || key.size(3) != d || key.stride(3) != 1 || key.numel() == 0) return nullptr;
     if (dtype_tag(key.scalar_type()) != tag || value.scalar_type() != key.scalar_type()) return nullptr;
@@ -276,7 +294,7 @@ PyObject* append(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     if (!from_zero && (start.dim() != 1 || start.size(0) != B || !dense_as(start, at::kInt))) return nullptr;
     if (unlocked(newest ? g_lib.append_kv_newest : g_lib.append_kv_paged, key.data_ptr(), value.data_ptr(), (int)tag, (int)B, (int)T, (int)H, key.stride(0), key.stride(1), key.stride(2),
                               from_zero ? nullptr : (const int32_t*)start.data_ptr(), (const int32_t*)table.data_ptr(), (int)table.size(1),
-                              address<tq_layer>(a[9]), address<tq_page_layout>(a[10]), (uint8_t*)pool.data_ptr(), pages, p.stream()) != TQ_OK)
+                              layer.get(), layout.get(), (uint8_t*)pool.data_ptr(), pages, p.stream()) != TQ_OK)
       return nullptr;
     Py_RETURN_TRUE;
   });
@@ -314,6 +332,8 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     const int64_t at = int_arg(a[3]), pages = int_arg(a[5]), H = int_arg(a[6]), d = int_arg(a[7]);
     const double scale = PyFloat_AsDouble(a[8]);
     const int n_split = (int)int_arg(a[13]), by_length = PyObject_IsTrue(a[14]);
+    const Held<tq_layer> layer(a[11]);
+    const Held<tq_page_layout> layout(a[12]);
     if (PyErr_Occurred() || !s.take(p, a[0], a[1], a[2], at, a[4], H, d)) return nullptr;
     const void *rk = nullptr, *rv = nullptr;
     int64_t R = 0, rs[3] = {0, 0, 0};
@@ -333,7 +353,7 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     const at::Tensor ws = s.workspace(p, d, by_length ? -n_split : n_split), out = p.fresh(s.q.sizes(), s.q.scalar_type());
     const auto call = by_length ? g_lib.decode_attn_paged_by_length : g_lib.decode_attn_paged;
     if (unlocked(call, s.q.data_ptr(), s.tag, (int)s.B, (int)s.Hq, (int)H, (const uint8_t*)s.pool.data_ptr(), pages, (const int32_t*)s.table.data_ptr(),
-             (int)s.bt_stride, s.len_ptr, (float)scale, address<tq_layer>(a[11]), address<tq_page_layout>(a[12]), rk, rv, (int)R, rs[0], rs[1],
+             (int)s.bt_stride, s.len_ptr, (float)scale, layer.get(), layout.get(), rk, rv, (int)R, rs[0], rs[1],
              rs[2], nullptr, out.data_ptr(), (float*)ws.data_ptr(), n_split, p.stream()) != TQ_OK)
       return nullptr;
     return THPVariable_Wrap(out);
@@ -349,6 +369,8 @@ PyObject* decode_ring(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     const int64_t pages = int_arg(a[4]), H = int_arg(a[5]), d = int_arg(a[6]), ring = int_arg(a[10]);
     const double scale = PyFloat_AsDouble(a[7]);
     const int n_split = (int)int_arg(a[13]), by_length = PyObject_IsTrue(a[14]);
+    const Held<tq_layer> layer(a[11]);
+    const Held<tq_page_layout> layout(a[12]);
     if (PyErr_Occurred() || ring > INT_MAX || ring < INT_MIN || !s.take(p, a[0], a[1], a[2], 0, a[3], H, d)) return nullptr;
     const at::Tensor k = p.take(a[8]), v = p.take(a[9]);
     if (!p.ok || k.dim() != 4 || k.sizes() != v.sizes() || k.strides() != v.strides() || k.size(1) != TQ_PAGE_TOKENS || k.size(2) != H ||
@@ -359,7 +381,7 @@ PyObject* decode_ring(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     const at::Tensor ws = s.workspace(p, d, by_length ? -n_split : n_split), out = p.fresh(s.q.sizes(), s.q.scalar_type());
     const auto call = by_length ? g_lib.decode_attn_paged_ring_by_length : g_lib.decode_attn_paged_ring;
     if (unlocked(call, s.q.data_ptr(), s.tag, (int)s.B, (int)s.Hq, (int)H, (const uint8_t*)s.pool.data_ptr(), pages, (const int32_t*)s.table.data_ptr(),
-             (int)s.bt_stride, s.len_ptr, (float)scale, address<tq_layer>(a[11]), address<tq_page_layout>(a[12]), k.data_ptr(), v.data_ptr(),
+             (int)s.bt_stride, s.len_ptr, (float)scale, layer.get(), layout.get(), k.data_ptr(), v.data_ptr(),
              k.stride(0), k.stride(1), k.stride(2), (int)ring, out.data_ptr(), (float*)ws.data_ptr(), n_split, p.stream()) != TQ_OK)
       return nullptr;
     return THPVariable_Wrap(out);
@@ -394,6 +416,7 @@ PyObject* cache_append(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     Part c;
     const int64_t d = int_arg(a[12]), gs = int_arg(a[15]);
     const int mb = (int)int_arg(a[13]), bits = (int)int_arg(a[14]);
+    const Held<tq_layer> layer(a[11]);
     if (PyErr_Occurred() || !c.take(p, a, d, mb, bits, gs)) return nullptr;
     const at::Tensor key = p.take(a[7]), value = p.take(a[8]), kb = p.take(a[9]), vb = p.take(a[10]);
     if (!p.ok || !rows4(key) || !rows4(value) || !rows4(kb) || !rows4(vb)) return nullptr;
@@ -415,7 +438,7 @@ PyObject* cache_append(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     const at::Tensor work = p.fresh({(int64_t)g_lib.cache_append_bytes(B * H, (int)d, mb, bits, (int)gs)}, at::kByte);
     if (unlocked(g_lib.cache_append, (const float*)key.data_ptr(), (const float*)value.data_ptr(), key.stride(1), value.stride(1), (const float*)kb.data_ptr(),
                            (const float*)vb.data_ptr(), kb.stride(0), kb.stride(1), kb.stride(2), vb.stride(0), vb.stride(1), vb.stride(2), B * H, (int)H,
-                           (int)n_buf, address<tq_layer>(a[11]), bits, (int)gs, c.n, (const uint8_t*)c.idx.data_ptr(), (const uint8_t*)c.sgn.data_ptr(),
+                           (int)n_buf, layer.get(), bits, (int)gs, c.n, (const uint8_t*)c.idx.data_ptr(), (const uint8_t*)c.sgn.data_ptr(),
                            (const float*)c.nrm.data_ptr(), (const float*)c.rn.data_ptr(), (const uint8_t*)c.data.data_ptr(),
                            (const float*)c.scales.data_ptr(), (const float*)c.zeros.data_ptr(), (uint8_t*)idx.data_ptr(), (uint8_t*)sgn.data_ptr(),
                            (float*)nrm.data_ptr(), (float*)rn.data_ptr(), (uint8_t*)data.data_ptr(), (float*)scales.data_ptr(), (float*)zeros.data_ptr(),
@@ -433,6 +456,7 @@ PyObject* cache_scores(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     const int64_t d = int_arg(a[10]), gs = int_arg(a[13]);
     const int mb = (int)int_arg(a[11]), bits = (int)int_arg(a[12]);
     const double scale = PyFloat_AsDouble(a[14]);
+    const Held<tq_layer> layer(a[9]);
     if (PyErr_Occurred() || !c.take(p, a, d, mb, bits, gs)) return nullptr;
     const at::Tensor query = p.take(a[7]), kb = p.take(a[8]);
     if (!p.ok || !rows4(query) || !rows4(kb) || kb.size(0) != c.B || kb.size(1) != c.H || kb.size(3) != d || kb.size(2) < 1 || kb.size(2) > INT_MAX) return nullptr;
@@ -445,7 +469,7 @@ PyObject* cache_scores(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     const at::Tensor q = in_place ? query : query.contiguous(), out = p.fresh({c.B, c.H, n_q, c.n + n_buf}, at::kFloat);
     const at::Tensor work = p.fresh({2 * batch * n_q * d}, at::kFloat);
     if (unlocked(g_lib.cache_scores_rows, (const float*)q.data_ptr(), in_place ? apart : d, batch, (int)c.H, n_q, (const uint8_t*)c.idx.data_ptr(), (const uint8_t*)c.sgn.data_ptr(),
-                           (const float*)c.nrm.data_ptr(), (const float*)c.rn.data_ptr(), c.n, address<tq_layer>(a[9]), (const float*)kb.data_ptr(),
+                           (const float*)c.nrm.data_ptr(), (const float*)c.rn.data_ptr(), c.n, layer.get(), (const float*)kb.data_ptr(),
                            kb.stride(0), kb.stride(1), kb.stride(2), (int)n_buf, (float)scale, (float*)out.data_ptr(), (float*)work.data_ptr(),
                            p.stream()) != TQ_OK)
       return nullptr;

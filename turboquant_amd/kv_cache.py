@@ -183,7 +183,7 @@ class TurboQuantKVCache:
         part = self._sections()
         if part is not None and kb.shape[-2] == self.buffer_size:
             q = self.key_quantizer
-            new = _ffi.native().cache_append(*part, key, value, kb, vb, C.addressof(q._layer()), self.head_dim, self.key_bits - 1,
+            new = _ffi.native().cache_append(*part, key, value, kb, vb, q._layer(), self.head_dim, self.key_bits - 1,
                                              self.value_bits, self.value_group_size)
             if new is not None:
                 self.key_quantized = ProdQuantized(*new[:4], self.key_quantized.mse_bits)
@@ -270,7 +270,7 @@ class TurboQuantKVCache:
         if part is not None and query.dim() == 4 and kb.dim() == 4:
             B, H, n_buf, d = kb.shape
             if self._few_score_queries(B * H * query.shape[2], part[3].shape[-1], n_buf, d):
-                scores = _ffi.native().cache_scores(*part, query, kb, C.addressof(self.key_quantizer._layer()), self.head_dim, self.key_bits - 1,
+                scores = _ffi.native().cache_scores(*part, query, kb, self.key_quantizer._layer(), self.head_dim, self.key_bits - 1,
                                                     self.value_bits, self.value_group_size, scale)
                 if scores is not None:
                     return scores

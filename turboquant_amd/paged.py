@@ -61,7 +61,7 @@ class PagedKVPool:
         _ffi.require_gpu(key, "key")
         fast = _ffi.native()
         if fast is not None and fast.append(key, value, block_table, start_pos, self.data, self.num_pages, self.num_kv_heads, self.head_dim,
-                                            _ffi.dtype_tag(self.dtype), C.addressof(self.quantizer._layer()), C.addressof(self.layout), False):
+                                            _ffi.dtype_tag(self.dtype), self.quantizer._layer(), self.layout, False):
             return
         if key.dim() != 4 or key.shape != value.shape:
             raise ValueError("key and value must both be (B, T, H, d)")
@@ -90,7 +90,7 @@ class PagedKVPool:
         fast = _ffi.native()
         # (the kernels take the lengths as they are: a subtraction is a launch of 5 us, half of what the page write of a token takes)
         if fast is not None and fast.append(key, value, block_table, seq_lens, self.data, self.num_pages, self.num_kv_heads, self.head_dim,
-                                            _ffi.dtype_tag(self.dtype), C.addressof(self.quantizer._layer()), C.addressof(self.layout), True):
+                                            _ffi.dtype_tag(self.dtype), self.quantizer._layer(), self.layout, True):
             return
         self.append(key, value, block_table, start_pos=seq_lens.to(torch.int32) - key.shape[1])
 
@@ -298,7 +298,7 @@ class PagedKVPool:
         if fast is None:
             return None
         return fast.decode(query, block_table, seq_lens, first, self.data, self.num_pages, self.num_kv_heads, self.head_dim, scale, recent_k,
-                           recent_v, C.addressof(self.quantizer._layer()), C.addressof(self.layout), n_split, by_length)
+                           recent_v, self.quantizer._layer(), self.layout, n_split, by_length)
 
     def decode_attention(self, query: torch.Tensor, block_table: torch.Tensor, seq_lens: torch.Tensor,
                          scale: Optional[float] = None, recent_k: Optional[torch.Tensor] = None,
@@ -421,7 +421,7 @@ class PagedKVPool:
         fast = _ffi.native()
         if fast is not None and workspace is None and out is None:
             done = fast.decode_ring(query, block_table, seq_lens, self.data, self.num_pages, self.num_kv_heads, self.head_dim, scale,
-                                    key_cache, value_cache, ring_rows, C.addressof(self.quantizer._layer()), C.addressof(self.layout),
+                                    key_cache, value_cache, ring_rows, self.quantizer._layer(), self.layout,
                                     n_split, by_length)
             if done is not None:
                 return done

@@ -226,7 +226,7 @@ class TurboQuantProd(torch.nn.Module):
         mb = self.bits - 1
         fast = _ffi.native()
         if fast is not None:
-            code = fast.quantize(x, C.addressof(self._layer()), self.dim, mb)
+            code = fast.quantize(x, self._layer(), self.dim, mb)
             if code is not None:
                 return ProdQuantized(*code, mb)
         rows, stride = _rows(x)
@@ -271,7 +271,7 @@ class TurboQuantProd(torch.nn.Module):
         _ffi.require_gpu(q.mse_indices, "mse_indices")
         fast = _ffi.native()
         if fast is not None:
-            out = fast.dequantize(q.mse_indices, q.qjl_signs, q.residual_norms, q.norms, C.addressof(self._layer()), self.dim, self.bits - 1)
+            out = fast.dequantize(q.mse_indices, q.qjl_signs, q.residual_norms, q.norms, self._layer(), self.dim, self.bits - 1)
             if out is not None:
                 return out
         idx = q.mse_indices.contiguous()
@@ -296,7 +296,7 @@ class TurboQuantProd(torch.nn.Module):
         fast = _ffi.native()
         if fast is not None:
             k = quantized_key
-            scores = fast.score(query, k.mse_indices, k.qjl_signs, k.residual_norms, k.norms, C.addressof(self._layer()), d, self.bits - 1)
+            scores = fast.score(query, k.mse_indices, k.qjl_signs, k.residual_norms, k.norms, self._layer(), d, self.bits - 1)
             if scores is not None:
                 return scores
         lead = query.shape[:-2]
