@@ -625,7 +625,7 @@ def test_a_descriptor_outlives_the_native_call_that_reads_it(monkeypatch):
     def layer():
         ly = build()
         ref = Ref(ly)
-        ref.terms = [weakref.ref(t) for t in (*tq.mse_quantizer._splits[1][:4], *tq.mse_quantizer._splits[1][4])]
+        ref.terms = [weakref.ref(t) for t in (*tq.mse_quantizer._splits[True][1][:4], *tq.mse_quantizer._splits[True][1][4])]
         built.append(ref)
         return ly
     tq._layer = layer
@@ -660,3 +660,23 @@ def test_a_descriptor_outlives_the_native_call_that_reads_it(monkeypatch):
         with pytest.raises(_Seen):
             call()
         assert host.calls[-1] == name
+
+
+def test_the_stages_of_a_quantiser_keep_a_descriptor_each(monkeypatch):
+    """The first stage used alone, in turn with the whole and in the middle of the other's build (where it waits for the card, another
+    thread may run): each has its own matrices, and neither is built again."""
+    monkeypatch.setattr(_ffi, "require_gpu", lambda t, name: t)
+    for other_first in (False, True):
+        tq = TurboQuantProd(128, bits=3, device="cpu")
+        mse, norm, inside = tq.mse_quantizer, torch.Tensor.norm, []
+        if other_first:
+            mse._layer()
+        with monkeypatch.context() as m:
+            m.setattr(torch.Tensor, "norm", lambda t, *a, **k: (inside.append(mse._layer()), norm(t, *a, **k))[1])
+            ly = tq._layer()
+        alone = mse._layer()
+        assert inside and all(x is alone for x in inside) and tq._layer() is ly and mse._layer() is alone
+        assert alone.S is None and not alone.S_split and not alone.PiT_fp6
+        pi, pit, s, st, fp6 = mse._splits[True][1]
+        assert (ly.Pi_split, ly.PiT_split, ly.S_split, ly.ST_split, ly.PiT_fp6) == tuple(t.data_ptr() for t in (pi, pit, s, st, fp6[0]))
+        assert ly.Pi == alone.Pi and ly.S_rownorm_max > 0

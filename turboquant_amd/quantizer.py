@@ -118,8 +118,9 @@ class TurboQuantMSE(torch.nn.Module):
         # kernel-side companions (not part of the reference's state dict)
         self.register_buffer("_PiT", self.Pi.T.contiguous(), persistent=False)
         self._centroids_host = centroids.detach().float().cpu()
-        self._splits = None           # (Pi, Pi^T[, S, S^T]) as bf16 term triples, built on first GPU use
-        self._layer_cache = None      # (key, TqLayer): the descriptor of the buffers as they are now
+        # with S or without (this stage alone, or the second one behind it): kept side by side, neither frees what a call of the other reads
+        self._splits = {}             # -> (key, (Pi, Pi^T[, S, S^T]) as bf16 term triples, query constants), built on first GPU use
+        self._layers = {}             # -> (state, TqLayer): the descriptor of the buffers as they are now
 
     # -- library plumbing ---------------------------------------------------------
     def _layer(self, S: Optional[torch.Tensor] = None, ST: Optional[torch.Tensor] = None) -> _ffi.TqLayer:
@@ -128,11 +129,11 @@ class TurboQuantMSE(torch.nn.Module):
         Pi, cen, thr = _buffer(self, "Pi"), _buffer(self, "centroids"), _buffer(self, "decision_boundaries")
         state = (Pi.data_ptr(), Pi._version, cen.data_ptr(), cen._version, thr.data_ptr(), thr._version,
                  None if S is None else (S.data_ptr(), S._version, None if ST is None else ST.data_ptr()))
-        cached = self._layer_cache
+        cached = self._layers.get(S is not None)
         if cached is not None and cached[0] == state:
             return cached[1]
         ly = self._build_layer(S, ST)
-        self._layer_cache = (state, ly)
+        self._layers[S is not None] = (state, ly)
         return ly
 
     def _build_layer(self, S: Optional[torch.Tensor] = None, ST: Optional[torch.Tensor] = None) -> _ffi.TqLayer:
@@ -140,29 +141,29 @@ class TurboQuantMSE(torch.nn.Module):
             raise TypeError("the kernels need float32 rotation / codebook buffers")
         if self._PiT.device != self.Pi.device or self._PiT.data_ptr() == 0:
             self._PiT = self.Pi.T.contiguous()
-            self._splits = None
+            self._splits.clear()
         key = (self.Pi.data_ptr(), self.Pi._version, None if S is None else (S.data_ptr(), S._version))
-        if self._splits is None or self._splits[0] != key:
-            self._PiT = self.Pi.T.contiguous()
+        kept = self._splits.get(S is not None)
+        if kept is None or kept[0] != key:
+            self._PiT = PiT = self.Pi.T.contiguous()
             # every head size has a matrix-core key quantiser (Pi, Pi^T, S); the de-quantiser of head_dim
             # 128 / 256 takes S^T too.  Split side by side: a quantiser's first call waits for it (head_dim 64: 470 -> 310 us)
-            mats = [self.Pi, self._PiT] + ([] if S is None else [S])
+            mats = [self.Pi, PiT] + ([] if S is None else [S])
             if ST is not None and self.dim in (128, 256):
                 mats.append(ST)
             splits = [None] * 4
             if self.dim % 64 == 0 and self.dim <= 768:
                 splits[:len(mats)] = _ffi.split_bf16x3(torch.stack(mats))
             # head_dim 128: Pi^T also as fp6 terms, for the centroid contraction on the block-scaled MFMA
-            fp6 = _ffi.split_fp6x5(self._PiT) if (self.dim == 128 and S is not None) else None
-            self._splits = (key, (*splits, fp6))
-        qc = None
-        if S is not None:
-            if getattr(self, "_query_consts", None) is None or self._query_consts[0] != key:
-                self._query_consts = (key, (self.Pi.sum(dim=0).contiguous(), S.sum(dim=0).contiguous(),
-                                            float(S.norm(dim=1).max())))
-            qc = self._query_consts[1]
+            fp6 = _ffi.split_fp6x5(PiT) if (self.dim == 128 and S is not None) else None
+            qc = None
+            if S is not None:
+                qc = (self.Pi.sum(dim=0).contiguous(), S.sum(dim=0).contiguous(), float(S.norm(dim=1).max()))
+            kept = (key, (*splits, fp6), qc)
+            self._splits[S is not None] = kept
+        # (what this call built or found: another thread may be building as well)
         return _ffi.make_layer(self.dim, self.bits, self.Pi, self._PiT, self.centroids, self.decision_boundaries,
-                               S, ST, centroids_host=self._centroids_host, splits=self._splits[1], query_consts=qc)
+                               S, ST, centroids_host=self._centroids_host, splits=kept[1], query_consts=kept[2])
 
     def quantize(self, x: torch.Tensor) -> MSEQuantized:
         """x (..., d) -> packed indices (..., d*eff/8) and norms (...) in x's dtype."""
