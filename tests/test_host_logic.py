@@ -3,10 +3,12 @@ loads and exports what include/tq_hip.h declares, argument checking, page
 geometry, codebook files, ring / capture policy against the reference's trace,
 and the loud failure on CPU tensors."""
 
+import copy
 import ctypes as C
 import gc
 import json
 import os
+import pickle
 import re
 import weakref
 
@@ -680,3 +682,17 @@ def test_the_stages_of_a_quantiser_keep_a_descriptor_each(monkeypatch):
         pi, pit, s, st, fp6 = mse._splits[True][1]
         assert (ly.Pi_split, ly.PiT_split, ly.S_split, ly.ST_split, ly.PiT_fp6) == tuple(t.data_ptr() for t in (pi, pit, s, st, fp6[0]))
         assert ly.Pi == alone.Pi and ly.S_rownorm_max > 0
+
+
+def test_a_quantiser_in_use_can_be_copied_and_pickled(monkeypatch):
+    """Its descriptors hold addresses of its own tensors: a copy builds its own, also of a sketch matrix that was written since."""
+    monkeypatch.setattr(_ffi, "require_gpu", lambda t, name: t)
+    for d in (64, 128):
+        tq = TurboQuantProd(d, bits=3, device="cpu")
+        tq._layer(), tq.mse_quantizer._layer()
+        tq.S.neg_()
+        for other in (copy.deepcopy(tq), pickle.loads(pickle.dumps(tq))):
+            ly = other._layer()
+            assert ly.Pi == other.mse_quantizer.Pi.data_ptr() != tq.mse_quantizer.Pi.data_ptr()
+            assert torch.equal(other._ST, other.S.T) and torch.equal(other.S, tq.S) and ly.ST == other._ST.data_ptr()
+            assert set(other.state_dict()) == set(tq.state_dict())

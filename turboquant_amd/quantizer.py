@@ -122,6 +122,10 @@ class TurboQuantMSE(torch.nn.Module):
         self._splits = {}             # -> (key, (Pi, Pi^T[, S, S^T]) as bf16 term triples, query constants), built on first GPU use
         self._layers = {}             # -> (state, TqLayer): the descriptor of the buffers as they are now
 
+    def __getstate__(self):
+        # (descriptors hold addresses of this object's tensors: a copy builds its own)
+        return {**super().__getstate__(), "_splits": {}, "_layers": {}}
+
     # -- library plumbing ---------------------------------------------------------
     def _layer(self, S: Optional[torch.Tensor] = None, ST: Optional[torch.Tensor] = None) -> _ffi.TqLayer:
         # One descriptor per state of the buffers: building it costs more host time than a decode call has to
@@ -214,6 +218,9 @@ class TurboQuantProd(torch.nn.Module):
         self.register_buffer("S", generate_qjl_matrix(dim, self.device, dtype, seed=seed + 1000))
         self.register_buffer("_ST", self.S.T.contiguous(), persistent=False)
         self.qjl_scale = math.sqrt(math.pi / 2.0) / dim
+
+    def __getstate__(self):
+        return {**super().__getstate__(), "_ST_version": None}
 
     def _layer(self) -> _ffi.TqLayer:
         S, ST = _buffer(self, "S"), _buffer(self, "_ST")
