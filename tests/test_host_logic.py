@@ -10,6 +10,8 @@ import json
 import os
 import pickle
 import re
+import sys
+import types
 import weakref
 
 import numpy as np
@@ -696,3 +698,34 @@ def test_a_quantiser_in_use_can_be_copied_and_pickled(monkeypatch):
             assert ly.Pi == other.mse_quantizer.Pi.data_ptr() != tq.mse_quantizer.Pi.data_ptr()
             assert torch.equal(other._ST, other.S.T) and torch.equal(other.S, tq.S) and ly.ST == other._ST.data_ptr()
             assert set(other.state_dict()) == set(tq.state_dict())
+
+
+@pytest.mark.parametrize("built_for,bound", [("this", True), ("Python 3.10, torch 2.9.0 abc, library 2, interface 1", False), (None, False)])
+def test_a_native_host_side_built_for_something_else_is_left_alone(monkeypatch, built_for, bound):
+    """One for another torch or Python, or from before it said what it is for (whose calls may take other arguments): never called."""
+    calls = []
+
+    class Module(types.ModuleType):
+        def bind(self, addresses):
+            calls.append(addresses)
+            if not bound:
+                raise KeyError("a call that this library lacks")
+    module = Module("_tq_host")
+    if built_for is not None:
+        module.built_for = _ffi.host_stamp() if built_for == "this" else built_for
+    library = _ffi.lib()
+    monkeypatch.setitem(sys.modules, "turboquant_amd._tq_host", module)
+    monkeypatch.setattr(turboquant_amd, "_tq_host", module, raising=False)
+    monkeypatch.setattr(_ffi, "_host", None)
+    _ffi._bind_host(library)
+    assert (_ffi._host is module) == bound and len(calls) == bound
+    if bound:
+        assert set(calls[0]) == set(_ffi._HOST_CALLS) and all(calls[0].values())
+
+
+def test_the_native_host_side_is_for_this_torch():
+    from turboquant_amd.build import HOST
+    if not os.path.exists(HOST):
+        pytest.skip("not built here")
+    _ffi.lib()
+    assert _ffi._host is not None and _ffi._host.built_for == _ffi.host_stamp()

@@ -7,11 +7,15 @@ is missing or a tensor is not on a GPU the call raises.
 from __future__ import annotations
 
 import ctypes as C
+import logging
 import math
 import os
+import sys
 from typing import Optional
 
 import torch
+
+logger = logging.getLogger("turboquant.ffi")
 
 TQ_F32, TQ_F16, TQ_BF16 = 0, 1, 2
 TQ_PAGE_TOKENS = 16
@@ -143,13 +147,27 @@ _HOST_CALLS = ("tq_quantize_keys", "tq_dequant_keys", "tq_score", "tq_ring_write
                "tq_cache_append_bytes", "tq_cache_append", "tq_cache_scores_rows", "tq_cache_attend_bytes", "tq_cache_attend")
 
 
+HOST_INTERFACE = 1                    # of csrc/tq_host.cpp: goes up with every change of a call's arguments or results
+
+
+def host_stamp() -> str:
+    """What the native host side has to be compiled for to run here."""
+    return (f"Python {sys.version_info.major}.{sys.version_info.minor}, torch {torch.__version__} {torch.version.git_version}, "
+            f"library {ABI_VERSION}, interface {HOST_INTERFACE}")
+
+
 def _bind_host(handle):
     """Hand the library's functions to the native host side.  It launches nothing that the Python methods do not: without it (not
-    built, or built for another torch) a small call takes longer on the host and is otherwise the same."""
+    built, or built for another torch, Python or state of this package) a small call takes longer on the host and is otherwise the same."""
     global _host
     try:
         from . import _tq_host
     except ImportError:
+        return
+    built_for = getattr(_tq_host, "built_for", "something else")
+    if built_for != host_stamp():
+        logger.warning("the native host side is built for %s, this is %s: it is left alone and small calls take longer (python -m turboquant_amd.build)",
+                       built_for, host_stamp())
         return
     _tq_host.bind({name: C.cast(getattr(handle, name), C.c_void_p).value for name in _HOST_CALLS})
     _host = _tq_host

@@ -49,11 +49,14 @@ def _host_command():
 
     import torch
     from torch.utils.cpp_extension import include_paths
+
+    from ._ffi import host_stamp
     lib = os.path.join(os.path.dirname(torch.__file__), "lib")
     # NDEBUG: without it pybind11 keeps a thread-local count of references, and a module with thread-local data that is loaded behind
     # libtq_hip.so slows the lookup of that library's own, about 1 us per launch (a ragged write of 3 short prompts 10.0 -> 11.4 us)
     headers = [*include_paths(), sysconfig.get_paths()["include"], "/opt/rocm/include"]
     return ([os.environ.get("CXX", "g++"), "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+             f'-DTQ_HOST_STAMP="{host_stamp()}"',
              f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"] + [x for h in headers for x in ("-isystem", h)] +
             [os.path.join(CSRC, "tq_host.cpp"), "-L" + lib] + [f"-l{n}" for n in ("c10", "c10_hip", "torch_cpu", "torch_hip", "torch", "torch_python")] +
             ["-o", HOST])

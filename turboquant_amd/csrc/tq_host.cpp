@@ -27,6 +27,12 @@
 
 #include "../../include/tq_hip.h"
 
+// The Python, the torch and the interface that this file is compiled for (_ffi.host_stamp): it reads their structures through their headers, and
+// its calls take their arguments by position.
+#ifndef TQ_HOST_STAMP
+#error "TQ_HOST_STAMP is not defined"
+#endif
+
 namespace {
 
 struct Library {
@@ -525,4 +531,8 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_tq_host", "host side of small ca
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__tq_host(void) { return PyModule_Create(&kModule); }
+PyMODINIT_FUNC PyInit__tq_host(void) {
+  PyObject* m = PyModule_Create(&kModule);
+  if (m && PyModule_AddStringConstant(m, "built_for", TQ_HOST_STAMP) < 0) { Py_DECREF(m); m = nullptr; }
+  return m;
+}
