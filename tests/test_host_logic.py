@@ -729,3 +729,34 @@ def test_the_native_host_side_is_for_this_torch():
         pytest.skip("not built here")
     _ffi.lib()
     assert _ffi._host is not None and _ffi._host.built_for == _ffi.host_stamp()
+
+
+@pytest.mark.parametrize("fails", [None, "host", "headers", "hipcc", "link"])
+def test_a_library_is_built_with_the_native_host_side_or_without(monkeypatch, tmp_path, capsys, fails):
+    """What the module alone needs (a host compiler, torch's headers) may be missing: the library stands, and a module of before is gone.
+    Where the library does not build, the module of before stays beside it."""
+    from turboquant_amd import build
+    monkeypatch.setattr(build, "HERE", str(tmp_path))
+    monkeypatch.setattr(build, "LIB", str(tmp_path / "libtq_hip.so"))
+    monkeypatch.setattr(build, "HOST", str(tmp_path / "_tq_host.so"))
+    (tmp_path / "_tq_host.so").write_text("before")
+
+    def run(cmd, **_):
+        out = cmd[cmd.index("-o") + 1]
+        kind = "host" if out.endswith("_tq_host.so") else "link" if out.endswith("libtq_hip.so") else "hipcc"
+        if kind == "host" and fails == "host":
+            raise FileNotFoundError("g++")
+        if kind != fails:
+            open(out, "w").write("now")
+        return types.SimpleNamespace(returncode=int(kind == fails), stderr="")
+    monkeypatch.setattr(build.subprocess, "run", run)
+    if fails == "headers":
+        monkeypatch.setitem(sys.modules, "torch.utils.cpp_extension", None)
+    if fails in ("hipcc", "link"):
+        with pytest.raises(RuntimeError, match="hipcc"):
+            build.build_library()
+        assert (tmp_path / "_tq_host.so").read_text() == "before"
+        return
+    assert build.build_library() == str(tmp_path / "libtq_hip.so") and (tmp_path / "libtq_hip.so").read_text() == "now"
+    assert os.path.exists(build.HOST) == (fails is None) == ("not built" not in capsys.readouterr().err)
+    assert fails or (tmp_path / "_tq_host.so").read_text() == "now"

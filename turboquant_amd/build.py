@@ -37,13 +37,16 @@ FLAGS = [
 
 
 def _run(cmd):
-    res = subprocess.run(cmd, capture_output=True, text=True)
+    try:
+        res = subprocess.run(cmd, capture_output=True, text=True)
+    except OSError as e:                       # (no such compiler)
+        return 127, str(e)
     # the host pass warns that it does not know the packed-fp32 feature; that is harmless
     err = "\n".join(l for l in res.stderr.splitlines() if "packed-fp32-ops" not in l)
     return res.returncode, err
 
 
-def _host_command():
+def _host_command(out):
     """The native host side of small calls: a Python module against torch's headers, no device code."""
     import sysconfig
 
@@ -59,12 +62,21 @@ def _host_command():
              f'-DTQ_HOST_STAMP="{host_stamp()}"',
              f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"] + [x for h in headers for x in ("-isystem", h)] +
             [os.path.join(CSRC, "tq_host.cpp"), "-L" + lib] + [f"-l{n}" for n in ("c10", "c10_hip", "torch_cpu", "torch_hip", "torch", "torch_python")] +
-            ["-o", HOST])
+            ["-o", out])
+
+
+def _build_host(out):
+    """(status, messages) of the native host side, compiled to `out`: it needs more than hipcc (g++, torch's and Python's headers)."""
+    try:
+        return _run(_host_command(out))
+    except Exception as e:
+        return 1, f"{type(e).__name__}: {e}"
 
 
 def build_library(verbose: bool = False) -> str:
     """Compile every source to an object file (in parallel: the files are independent translation units)
-    and link them into libtq_hip.so."""
+    and link them into libtq_hip.so; with it the native host side of small calls, which the package does without where it does not
+    compile (it takes the place of the former one once the library stands, and the former one does not stay behind)."""
     from concurrent.futures import ThreadPoolExecutor
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     objdir = os.path.join(HERE, "build")
@@ -75,23 +87,31 @@ def build_library(verbose: bool = False) -> str:
     for src in SOURCES:
         obj = os.path.join(objdir, src.replace(".hip", ".o"))
         jobs.append((obj, [hipcc] + compile_flags + ["-c", os.path.join(CSRC, src), "-o", obj]))
-    jobs.append((HOST, _host_command()))
+    host_built = os.path.join(objdir, os.path.basename(HOST))
     if verbose:
         for _, cmd in jobs:
             print(" ".join(cmd))
-    with ThreadPoolExecutor(max_workers=min(len(jobs), os.cpu_count() or 1)) as pool:
+    with ThreadPoolExecutor(max_workers=min(len(jobs) + 1, os.cpu_count() or 1)) as pool:
+        host = pool.submit(_build_host, host_built)
         results = list(pool.map(lambda j: _run(j[1]), jobs))
+        host_rc, host_err = host.result()
     for (obj, _), (rc, err) in zip(jobs, results):
         if rc != 0:
-            raise RuntimeError(f"compiling {obj} failed ({rc}):\n{err}")
+            raise RuntimeError(f"hipcc failed ({rc}) for {obj}:\n{err}")
         if verbose and err.strip():
             print(err, file=sys.stderr)
-    link = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-fno-gpu-rdc"] + [obj for obj, _ in jobs if obj != HOST] + ["-o", LIB]
+    link = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-fno-gpu-rdc"] + [obj for obj, _ in jobs] + ["-o", LIB]
     if verbose:
         print(" ".join(link))
     rc, err = _run(link)
     if rc != 0:
         raise RuntimeError(f"hipcc link failed ({rc}):\n{err}")
+    if host_rc == 0:
+        os.replace(host_built, HOST)
+    else:
+        print(f"warning: the native host side is not built ({host_rc}), small calls take longer on the host:\n{host_err}", file=sys.stderr)
+        if os.path.exists(HOST):
+            os.remove(HOST)
     return LIB
 
 
