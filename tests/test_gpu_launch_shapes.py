@@ -243,7 +243,7 @@ def test_append_of_the_newest_tokens_takes_the_lengths(gpu, d, B, H, T, dtype):
     _say(f"newest d={d} B={B} H={H} T={T} {dtype}")
     pools = [PagedKVPool(tq, H, B * per_seq, value_bits=4, value_group_size=32, dtype=dtype, device=gpu) for _ in range(2)]
     pools[0].append(k, v, table, start_pos=lens - T)
-    pools[1]._append_newest(k, v, table, lens)
+    assert pools[1]._append_newest(k, v, table, lens)
     torch.cuda.synchronize()
     assert torch.equal(pools[0].data, pools[1].data) and bool(pools[0].data.any())
 

@@ -760,3 +760,90 @@ def test_a_library_is_built_with_the_native_host_side_or_without(monkeypatch, tm
     assert build.build_library() == str(tmp_path / "libtq_hip.so") and (tmp_path / "libtq_hip.so").read_text() == "now"
     assert os.path.exists(build.HOST) == (fails is None) == ("not built" not in capsys.readouterr().err)
     assert fails or (tmp_path / "_tq_host.so").read_text() == "now"
+
+
+@pytest.mark.parametrize("how", ["as it is", "subclass", "object", "class", "stand-in"])
+def test_a_method_in_the_place_of_one_that_native_calls_go_past_sees_every_call(monkeypatch, how):
+    """Writes and decode steps of the engine's hooks and of a store, which reach the native host side without the pool's `append`,
+    `decode_attention` and `workspace` where those are the package's own."""
+    from turboquant_amd import score, store as S
+    from turboquant_amd.integration import batched
+    from turboquant_amd.paged import PagedKVPool
+    seen, native = [], []
+
+    class Host:
+        def append(self, *a):
+            native.append("append")
+            return True
+
+        def decode(self, *a):
+            native.append("decode_attention")
+            return torch.zeros(1)
+
+        def decode_ring(self, *a):
+            native.append("decode_attention_ring")
+            return torch.zeros(1)
+
+    def spy(name, result=None):
+        return lambda *a, **k: (seen.append(name), result)[1]
+
+    class Own(PagedKVPool):
+        append, decode_attention, workspace = spy("append"), spy("decode_attention", torch.zeros(1)), spy("workspace")
+
+    class StandIn:
+        __slots__ = ("dtype", "num_pages", "device")
+        append, decode_attention, default_splits = spy("append"), spy("decode_attention", torch.zeros(1)), lambda *a: 1
+    monkeypatch.setattr(_ffi, "require_gpu", lambda t, name: t)
+    _ffi.lib()
+    monkeypatch.setattr(_ffi, "_host", Host())
+    tq = TurboQuantProd(128, bits=3, device="cpu")
+    monkeypatch.setattr(TurboQuantProd, "_layer", lambda self: None)
+    pool = {"subclass": Own, "stand-in": StandIn}.get(how, PagedKVPool)
+    pool = pool.__new__(pool)
+    pool.dtype, pool.device, pool.num_pages = torch.bfloat16, torch.device("cpu"), 64
+    if how != "stand-in":
+        pool.quantizer, pool.head_dim, pool.num_kv_heads, pool.data, pool.layout = tq, 128, 2, torch.zeros(1), None
+        pool.value_bits, pool.value_group_size = 4, 32
+    if how in ("object", "class"):
+        for name in ("append", "decode_attention"):
+            monkeypatch.setattr(pool if how == "object" else PagedKVPool, name, spy(name, torch.zeros(1)))
+    meta = types.SimpleNamespace(num_actual_tokens=3, max_query_len=1, block_table=torch.zeros(3, 2, dtype=torch.int32), seq_lens=torch.ones(3, dtype=torch.int32))
+    config = types.SimpleNamespace(num_kv_heads=2, head_dim=128)
+    kv = torch.zeros(3, 2, 128, dtype=torch.bfloat16)
+    batched.BatchedLayerState(config=config, quantizer=tq, pool=pool).write(kv, kv, meta)
+    store = S.CompressedKVStore(128, 2, value_bits=4, device="cpu")
+    store._pool, store._block_table, store._counts = pool, torch.arange(64, dtype=torch.int32)[None], torch.arange(1025, dtype=torch.int32)
+    store._chunk_lengths = [100]
+    query = torch.zeros(1, 4, 128, dtype=torch.bfloat16)
+    score.compute_hybrid_attention(query, store, None, None, 4)
+    assert (seen, native) == (([], ["append", "decode_attention"]) if how == "as it is" else (["append", "decode_attention"], []))
+    # a store whose lengths or pages come from elsewhere takes its step through them
+    for cls in (type("Lengths", (S.CompressedKVStore,), {"lengths": lambda self, n, rows: seen.append("lengths")}),
+                type("Pages", (S.CompressedKVStore,), {"ensure_pool": lambda self, dtype, n=0: (seen.append("ensure_pool"), pool)[1]})):
+        store.__class__, before = cls, len(seen)
+        score.compute_hybrid_attention(query, store, None, None, 4)
+        assert len(seen) > before and seen[before] in ("lengths", "ensure_pool")
+
+
+def test_a_workspace_of_its_own_is_taken_by_every_decode_step(monkeypatch):
+    from turboquant_amd.paged import PagedKVPool
+
+    class Asked(Exception):
+        pass
+
+    class Pool(PagedKVPool):
+        def workspace(self, B, Hq, n_split):
+            raise Asked
+    monkeypatch.setattr(_ffi, "require_gpu", lambda t, name: t)
+    _ffi.lib()
+    monkeypatch.setattr(_ffi, "_host", types.SimpleNamespace(decode=lambda *a: torch.zeros(1), decode_ring=lambda *a: torch.zeros(1)))
+    pool = Pool.__new__(Pool)
+    pool.quantizer, pool.head_dim, pool.num_kv_heads = TurboQuantProd(128, bits=3, device="cpu"), 128, 2
+    pool.value_bits, pool.value_group_size = 4, 32
+    pool.dtype, pool.device, pool.num_pages, pool.data, pool.layout = torch.bfloat16, torch.device("cpu"), 4, torch.zeros(1), None
+    monkeypatch.setattr(TurboQuantProd, "_layer", lambda self: None)
+    q, table, one = torch.zeros(1, 4, 128, dtype=torch.bfloat16), torch.zeros(1, 4, dtype=torch.int32), torch.ones(1, dtype=torch.int32)
+    exact = torch.zeros(4, 16, 2, 128, dtype=torch.bfloat16)
+    for step in (lambda: pool.decode_attention(q, table, one), lambda: pool.decode_attention_ring(q, table, one, exact, exact, 16)):
+        with pytest.raises(Asked):
+            step()

@@ -184,6 +184,16 @@ def native():
 _lib_entry = lib
 
 
+def as_defined(obj, methods) -> bool:
+    """Whether `methods` ((name, function), ...) are still what obj calls by those names, so that a caller may go past them to what
+    they call: a subclass's, a stand-in's, or one put on the class or the object sees every call."""
+    cls, own = type(obj), getattr(obj, "__dict__", ())
+    for name, function in methods:
+        if getattr(cls, name, None) is not function or name in own:
+            return False
+    return True
+
+
 def check(rc: int, what: str):
     if rc == 0:
         return

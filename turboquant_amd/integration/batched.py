@@ -39,7 +39,8 @@ from typing import Dict, Optional
 import torch
 import torch.nn.functional as F
 
-from ..paged import PAGE_TOKENS, PagedKVPool
+from .. import _ffi
+from ..paged import APPEND, PAGE_TOKENS, PagedKVPool
 from ..quantizer import TurboQuantProd
 from . import vllm as _single
 from .vllm import (MODE_CAPTURE_ONLY, MODE_HYBRID, MODE_OFF, LayerConfig, _bind, _is_mla_impl, _query_heads_of,
@@ -76,7 +77,9 @@ class BatchedLayerState:
         v = value[:n].reshape(n, cfg.num_kv_heads, cfg.head_dim)
         table = meta.block_table
         if int(meta.max_query_len) == 1:                       # one token per sequence: a single batched append
-            self.pool._append_newest(k[:, None], v[:, None], table, meta.seq_lens)
+            k, v, lens = k[:, None], v[:, None], meta.seq_lens
+            if not (_ffi.as_defined(self.pool, APPEND) and self.pool._append_newest(k, v, table, lens)):
+                self.pool.append(k, v, table, start_pos=lens.to(torch.int32) - 1)
         else:                                                  # ragged rows: still one call, nothing read back
             qsl = meta.query_start_loc.to(device=k.device, dtype=torch.int32)
             run = qsl[1:] - qsl[:-1]

@@ -85,14 +85,13 @@ class PagedKVPool:
                 C.byref(self.layout), self.data.data_ptr(), self.num_pages, _ffi.stream_ptr(self.device)),
                 "tq_append_kv_paged")
 
-    def _append_newest(self, key: torch.Tensor, value: torch.Tensor, block_table: torch.Tensor, seq_lens: torch.Tensor):
-        """`append` of the newest T tokens of sequences that hold seq_lens (B,) tokens with them."""
+    def _append_newest(self, key: torch.Tensor, value: torch.Tensor, block_table: torch.Tensor, seq_lens: torch.Tensor) -> bool:
+        """`append` of the newest T tokens of sequences that hold seq_lens (B,) tokens with them; False: not a case for it, nothing was done."""
         fast = _ffi.native()
         # (the kernels take the lengths as they are: a subtraction is a launch of 5 us, half of what the page write of a token takes)
-        if fast is not None and fast.append(key, value, block_table, seq_lens, self.data, self.num_pages, self.num_kv_heads, self.head_dim,
-                                            _ffi.dtype_tag(self.dtype), self.quantizer._layer(), self.layout, True):
-            return
-        self.append(key, value, block_table, start_pos=seq_lens.to(torch.int32) - key.shape[1])
+        return fast is not None and bool(fast.append(
+            key, value, block_table, seq_lens, self.data, self.num_pages, self.num_kv_heads, self.head_dim, _ffi.dtype_tag(self.dtype),
+            self.quantizer._layer(), self.layout, True))
 
     def append_from_blocks(self, key_cache: torch.Tensor, value_cache: torch.Tensor, src_table: torch.Tensor,
                            block_table: torch.Tensor, run_len: torch.Tensor, start_pos: Optional[torch.Tensor] = None,
@@ -328,7 +327,8 @@ class PagedKVPool:
                 max_len = block_table.shape[-1] * PAGE_TOKENS
             n_split = self.default_splits(B, max_len, Hq, static_scratch)
             by_length = workspace is None and not static_scratch and stages == 7 and self._shares_by_length(B, Hq)
-        if workspace is None and out is None and recent_len is None and stages == 7 and not static_scratch:
+        if (workspace is None and out is None and recent_len is None and stages == 7 and not static_scratch
+                and _ffi.as_defined(self, WORKSPACE)):
             done = self._decode_native(query, block_table, seq_lens, 0, scale, recent_k, recent_v, n_split, by_length)
             if done is not None:
                 return done
@@ -419,7 +419,7 @@ class PagedKVPool:
             n_split = self.default_splits(B, max_len, Hq)
             by_length = workspace is None and self._shares_by_length(B, Hq)
         fast = _ffi.native()
-        if fast is not None and workspace is None and out is None:
+        if fast is not None and workspace is None and out is None and _ffi.as_defined(self, WORKSPACE):
             done = fast.decode_ring(query, block_table, seq_lens, self.data, self.num_pages, self.num_kv_heads, self.head_dim, scale,
                                     key_cache, value_cache, ring_rows, self.quantizer._layer(), self.layout,
                                     n_split, by_length)
@@ -445,3 +445,9 @@ class PagedKVPool:
                 key_cache.stride(1), key_cache.stride(2), int(ring_rows), out.data_ptr(), workspace.data_ptr(),
                 n_split, _ffi.stream_ptr(self.device)), "tq_decode_attn_paged_ring")
         return out
+
+
+# what a native call goes past, as it is defined here (_ffi.as_defined)
+APPEND = (("append", PagedKVPool.append),)
+WORKSPACE = (("workspace", PagedKVPool.workspace),)
+DECODE = (("decode_attention", PagedKVPool.decode_attention), *WORKSPACE)

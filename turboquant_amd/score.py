@@ -16,7 +16,9 @@ from typing import Optional
 
 import torch
 
-from .store import CompressedKVStore
+from . import _ffi
+from .paged import DECODE
+from .store import STEP, CompressedKVStore
 
 logger = logging.getLogger("turboquant.score")
 
@@ -47,7 +49,8 @@ def compute_hybrid_attention(query: torch.Tensor, store: CompressedKVStore, rece
         raise ValueError(f"Incompatible GQA shapes: Q={Q}, H_kv={num_kv_heads}, gqa_ratio={gqa_ratio}")
 
     # one query token over a store that holds its pages already, everything plain: the tensors as they are, without a view of any
-    if T == 1 and has_history and isinstance(store, CompressedKVStore) and store.has_pages(n_hist):
+    if (T == 1 and has_history and _ffi.as_defined(store, STEP) and store.has_pages(n_hist) and
+            _ffi.as_defined(store.pool, DECODE)):
         pool = store.pool
         out = pool._decode_native(query, store.block_table, store.counts, n_hist, scale, recent_k if has_recent else None, recent_v,
                                   pool.default_splits(1, n_hist, Q), False)

@@ -157,3 +157,7 @@ class CompressedKVStore:
     def reset(self):
         self._chunk_lengths.clear()
         self._flat = None
+
+
+# what a decode step goes past where the pages exist, as it is defined here (_ffi.as_defined)
+STEP = (("ensure_pool", CompressedKVStore.ensure_pool), ("lengths", CompressedKVStore.lengths))
