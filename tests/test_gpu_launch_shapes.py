@@ -1,5 +1,7 @@
 """Launch shapes that depend on the sizes of a call: each rule of a dispatch at the sizes where it can go wrong."""
 
+import copy
+
 import pytest
 import torch
 
@@ -663,16 +665,24 @@ class _Counted:
             return rc
         return call
 
-    def take(self, name):
-        return self.answered.pop(name, 0)
+    def take(self, *names):
+        return sum(self.answered.pop(name, 0) for name in names)
 
 
 @pytest.fixture
 def counted(monkeypatch):
+    """The library as the Python methods and the native host side in front of them call it."""
+    import ctypes
     from turboquant_amd import _ffi
-    lib = _Counted(_ffi.lib())
+    real = _ffi.lib()
+    assert _ffi.native() is not None, "the native host side is not built"
+    host, lib = _ffi._host, _Counted(real)
+    seen = {name: ctypes.CFUNCTYPE(*[t for ts in _ffi._SIGNATURES[name] for t in (ts if isinstance(ts, list) else [ts])])(getattr(lib, name))
+            for name in _ffi._HOST_CALLS}
     monkeypatch.setattr(_ffi, "lib", lambda: lib)
-    return lib
+    host.bind({name: _ffi.address(f) for name, f in seen.items()})
+    yield lib
+    host.bind({name: _ffi.address(getattr(real, name)) for name in _ffi._HOST_CALLS})
 
 
 @pytest.mark.parametrize("d,B,H,prompt,buffer,key_bits,vb,gs,n_q", [
@@ -683,7 +693,7 @@ def test_cache_token_in_few_launches(gpu, counted, d, B, H, prompt, buffer, key_
     norms and buffers bit for bit, inner products with the compressed keys bit for bit, everything else within fp32 sums in another
     order.  Prompts as views of a (batch, tokens, heads, d) tensor, the buffer's rows then not behind one another: the
     first token takes the general path, the ones after it do not (all of them do where several batches' tokens lie apart as well)."""
-    from turboquant_amd import kv_cache as KC
+    from turboquant_amd import _ffi, kv_cache as KC
     g = torch.Generator().manual_seed(d + prompt)
     for view in (False, True):
         shape = (B, prompt + 4, H, d) if view else (B, H, prompt + 4, d)
@@ -692,10 +702,13 @@ def test_cache_token_in_few_launches(gpu, counted, d, B, H, prompt, buffer, key_
             k, v = k.transpose(1, 2), v.transpose(1, 2)
         qs = torch.randn(4, B, H, n_q, d, generator=g).to(gpu)
         results = []
-        for fast in (True, False):
+        for how in ("native", "python", "general"):
+            fast = how != "general"
             patch = pytest.MonkeyPatch()
             if not fast:
                 patch.setattr(KC, "_plain", lambda *t: False)
+            if how != "native":
+                patch.setattr(_ffi, "_host", None)
             cache = KC.TurboQuantKVCache(d, key_bits=key_bits, value_bits=vb, value_group_size=gs, buffer_size=buffer, device=gpu,
                                          dtype=torch.float32)
             cache.prefill(k[..., :prompt, :], v[..., :prompt, :])
@@ -710,8 +723,9 @@ def test_cache_token_in_few_launches(gpu, counted, d, B, H, prompt, buffer, key_
             results.append((cache, outs))
             patch.undo()
             assert counted.take("tq_cache_append") == (0 if not fast else 4 if not view else 3 if B == 1 else 0)
-            assert counted.take("tq_cache_scores") == counted.take("tq_cache_attend") == (4 if fast else 0)
-        (a, oa), (b, ob) = results
+            assert counted.take("tq_cache_scores", "tq_cache_scores_rows") == counted.take("tq_cache_attend") == (4 if fast else 0)
+        assert all(torch.equal(x, y) for s, t in zip(results[0][1], results[1][1]) for x, y in zip(s, t))
+        (a, oa), _, (b, ob) = results
         assert a.get_seq_length() == b.get_seq_length() and a.memory_bytes() == b.memory_bytes()
         for x, y in zip((*a.key_quantized[:4], *a.value_quantized[:3], a.key_buffer, a.value_buffer),
                         (*b.key_quantized[:4], *b.value_quantized[:3], b.key_buffer, b.value_buffer)):
@@ -797,6 +811,9 @@ def test_cache_token_in_one_launch(gpu, d, B, H, n_c, n_buf, key_bits, vb, gs):
             if how is None:
                 cache._append(*new)
             else:
+                spare = copy.copy(cache)
+                launches = _nodes(lambda: spare._append_spill(*new))
+                assert launches == (1 if how == -1 and d != 64 else 2)
                 assert cache._append_spill(*new)
             states.append([*cache.key_quantized[:4], *cache.value_quantized[:3], cache.key_buffer, cache.value_buffer])
     finally:
@@ -804,6 +821,38 @@ def test_cache_token_in_one_launch(gpu, d, B, H, n_c, n_buf, key_bits, vb, gs):
     for other in states[1:]:
         for a, b in zip(states[0], other):
             assert a.shape == b.shape and torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
+
+
+@pytest.mark.parametrize("d,rows,n_buf,how", [(128, 3, 4, -1), (128, 17, 1, 0), (256, 2, 2, -1), (64, 5, 3, -1)])
+def test_cache_token_into_an_empty_part(gpu, d, rows, n_buf, how):
+    """The library's entry with no compressed tokens yet, whose old sections are not there: the first ones are the quantisers' codes of the row that
+    leaves, byte for byte."""
+    import ctypes as C
+    from turboquant_amd import _ffi
+    from turboquant_amd.kv_cache import quantize_values
+    lib, tq = _ffi.lib(), TurboQuantProd(d, bits=3, device=gpu)
+    g = torch.Generator().manual_seed(d)
+    kb, vb = (torch.randn(rows, n_buf, d, generator=g).to(gpu) for _ in range(2))
+    key, value = (torch.randn(rows, d, generator=g).to(gpu) for _ in range(2))
+    byte = dict(dtype=torch.uint8, device=gpu)
+    idx, signs, data = torch.empty(rows, d // 4, **byte), torch.empty(rows, d // 8, **byte), torch.empty(rows, d // 2, **byte)
+    norms, rnorms, scales, zeros = (torch.empty(rows, n, device=gpu) for n in (1, 1, d // 32, d // 32))
+    nk, nv = torch.empty_like(kb), torch.empty_like(vb)
+    work = torch.empty(lib.tq_cache_append_bytes(rows, d, 2, 4, 32), **byte)
+    ly = tq._layer()
+    _set_option("append_small", how)
+    try:
+        _ffi.check(lib.tq_cache_append(
+            key.data_ptr(), value.data_ptr(), d, d, kb.data_ptr(), vb.data_ptr(), rows * n_buf * d, n_buf * d, d, rows * n_buf * d, n_buf * d, d, rows, rows,
+            n_buf, C.byref(ly), 4, 32, 0, *[None] * 7, idx.data_ptr(), signs.data_ptr(), norms.data_ptr(), rnorms.data_ptr(), data.data_ptr(),
+            scales.data_ptr(), zeros.data_ptr(), nk.data_ptr(), nv.data_ptr(), work.data_ptr(), _ffi.stream_ptr(gpu)), "tq_cache_append")
+        torch.cuda.synchronize()
+    finally:
+        _set_option("append_small", -1)
+    kq, vq = tq.quantize(kb[:, 0]), quantize_values(vb[:, :1], bits=4, group_size=32)
+    for got, want in zip((idx, signs, rnorms, norms, data, scales, zeros), (*kq[:4], *vq[:3])):
+        assert torch.equal(got.flatten(), want.flatten())
+    assert torch.equal(nk, torch.cat([kb[:, 1:], key[:, None]], dim=1)) and torch.equal(nv, torch.cat([vb[:, 1:], value[:, None]], dim=1))
 
 
 @pytest.mark.parametrize("d,B,H,n_c,n_q,step", [(128, 1, 8, 300, 1, 3), (64, 2, 3, 65, 1, 2), (256, 1, 2, 40, 5, 2), (128, 2, 2, 17, 3, 1)])
@@ -845,7 +894,7 @@ def test_cache_blocks_of_queries_on_either_side_of_the_limit(gpu, counted, d, H,
     for n_q in (most, most + 1):
         q = torch.randn(1, H, n_q, d, generator=g).to(gpu)
         got, want = cache.attention_scores(q), torch.matmul(q.double(), keys.transpose(-2, -1).contiguous()) / d ** 0.5
-        assert counted.take("tq_cache_scores") == (n_q == most)
+        assert counted.take("tq_cache_scores", "tq_cache_scores_rows") == (n_q == most)
         assert float((got - want).norm()) <= 2e-6 * float(want.norm())
     most = last(KC.TurboQuantKVCache._few_value_queries)
     assert counted._lib.tq_cache_attend_bytes(H, most, d, n_c, n_buf) <= 32 << 20

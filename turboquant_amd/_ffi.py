@@ -156,6 +156,10 @@ def host_stamp() -> str:
             f"library {ABI_VERSION}, interface {HOST_INTERFACE}")
 
 
+def address(function) -> int:
+    return C.cast(function, C.c_void_p).value
+
+
 def _bind_host(handle):
     """Hand the library's functions to the native host side.  It launches nothing that the Python methods do not: without it (not
     built, or built for another torch, Python or state of this package) a small call takes longer on the host and is otherwise the same."""
@@ -169,19 +173,14 @@ def _bind_host(handle):
         logger.warning("the native host side is built for %s, this is %s: it is left alone and small calls take longer (python -m turboquant_amd.build)",
                        built_for, host_stamp())
         return
-    _tq_host.bind({name: C.cast(getattr(handle, name), C.c_void_p).value for name in _HOST_CALLS})
+    _tq_host.bind({name: address(getattr(handle, name)) for name in _HOST_CALLS})
     _host = _tq_host
 
 
 def native():
     """The native host side for a call that runs now (not one that a compiler is tracing); None: the Python method does it all.  Its
     functions return None for every case that is not the plain one, and have done nothing then."""
-    if _host is None or lib is not _lib_entry or _compiling():        # (a `lib` put in place of ours is there to see the calls)
-        return None
-    return _host
-
-
-_lib_entry = lib
+    return None if _host is None or _compiling() else _host
 
 
 def as_defined(obj, methods) -> bool:
