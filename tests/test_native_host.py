@@ -1,8 +1,12 @@
 """The native host side of small calls (csrc/tq_host.cpp) against the Python methods it stands in front of: the same results bit for
 bit where it takes a call, and nothing done where it does not."""
 
+import threading
+
 import pytest
 import torch
+from torch.overrides import TorchFunctionMode
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from turboquant_amd import _ffi
 from turboquant_amd.capture import RingBuffer
@@ -52,7 +56,7 @@ def both(gpu, monkeypatch):
 
 def _same(a, b):
     if torch.is_tensor(a):
-        return a.dtype == b.dtype and a.shape == b.shape and torch.equal(a.flatten().view(torch.uint8), b.flatten().view(torch.uint8))
+        return a.dtype == b.dtype and a.is_inference() == b.is_inference() and a.shape == b.shape and torch.equal(a.flatten().view(torch.uint8), b.flatten().view(torch.uint8))
     if isinstance(a, (tuple, list)):
         return len(a) == len(b) and all(_same(x, y) for x, y in zip(a, b))
     return a == b
@@ -158,7 +162,16 @@ def test_ring_rows(gpu, both, form):
     assert (taken > 0) == (form not in ("narrow", "autocast")) and (left > 0) == (form in ("narrow", "autocast", "own rows"))
 
 
-@pytest.mark.parametrize("form", ["plain", "batches apart", "no value groups", "autocast", "bits put in", "gradient"])
+def _move_codes(cache):
+    """The codes of a cache, one byte into buffers of their own."""
+    def moved(t):
+        return torch.cat([t.flatten()[:1], t.flatten()])[1:].view(t.shape)
+    kq, vq = cache.key_quantized, cache.value_quantized
+    cache.key_quantized = kq._replace(mse_indices=moved(kq.mse_indices), qjl_signs=moved(kq.qjl_signs))
+    cache.value_quantized = vq._replace(data=moved(vq.data))
+
+
+@pytest.mark.parametrize("form", ["plain", "batches apart", "no value groups", "autocast", "bits put in", "gradient", "codes at odd bytes"])
 def test_cache_tokens(gpu, both, form):
     g = torch.Generator().manual_seed(9)
     B, H, n, d = 2, 3, 150, 128
@@ -176,8 +189,12 @@ def test_cache_tokens(gpu, both, form):
         outs = []
         with torch.autocast("cuda", torch.bfloat16, enabled=form == "autocast"):
             for i in range(3):
+                if form == "codes at odd bytes":                   # (the library refuses what the checks before it let pass)
+                    _move_codes(cache)
                 if form != "bits put in":
                     cache.append(k[..., n + i:n + i + 1, :], v[..., n + i:n + i + 1, :])
+                    if form == "codes at odd bytes":
+                        _move_codes(cache)
                 x = w[i].clone().requires_grad_() if form == "gradient" else w[i]
                 scores = cache.attention_scores(x)
                 outs += [scores.detach(), cache.attend(torch.softmax(scores.float(), dim=-1)).detach()]
@@ -186,7 +203,112 @@ def test_cache_tokens(gpu, both, form):
     assert _same(a, b)
     # (a prompt's keys are a slice of the tensor: one call left to Python; where batches lie apart their tokens are too)
     assert (taken, left) == {"plain": (9, 1), "no value groups": (9, 1), "batches apart": (6, 7), "autocast": (0, 13), "bits put in": (3, 7),
-                             "gradient": (3, 10)}[form]
+                             "gradient": (3, 10), "codes at odd bytes": (3, 13)}[form]
+
+
+@pytest.mark.parametrize("watch", ["vmap", "forward mode", "dispatch mode", "function mode", "trace", "deterministic"])
+def test_what_has_to_see_an_operation_sees_it(gpu, both, watch):
+    """Transforms, modes and traces, and fills of new memory: the calls are the Python methods', with their results, derivatives and errors."""
+    g = torch.Generator().manual_seed(2)
+    quant = TurboQuantProd(128, bits=3, device=gpu)
+    k, v = (torch.randn(1, 2, 150, 128, generator=g).to(gpu) for _ in range(2))
+    cache = TurboQuantKVCache(128, value_bits=2, buffer_size=64, device=gpu, dtype=torch.float32)
+    cache.prefill(k, v)
+    code = quant.quantize(k)
+    query = torch.randn(1, 2, 3, 128, generator=g).to(gpu)
+    weights = torch.softmax(torch.randn(1, 2, 3, 150, generator=g), dim=-1).to(gpu)
+    calls = {"codes": (lambda x: list(quant.quantize(x)[:4]), k), "products": (lambda x: quant.attention_score(x, code), query),
+             "scores": (cache.attention_scores, query), "values": (cache.attend, weights)}
+    if watch == "trace":                                           # (a trace of torch's own operations)
+        calls = {"values": calls["values"]}
+
+    class Dispatch(TorchDispatchMode):
+        seen = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            Dispatch.seen += 1
+            return func(*args, **(kwargs or {}))
+
+    class Function(TorchFunctionMode):
+        seen = 0
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            Function.seen += 1
+            return func(*args, **(kwargs or {}))
+
+    def watched(call, x):
+        if watch == "vmap":
+            return torch.vmap(call)(torch.stack([x, x]))
+        if watch == "forward mode":
+            with torch.autograd.forward_ad.dual_level():
+                out = call(torch.autograd.forward_ad.make_dual(x, torch.ones_like(x)))
+                return [y for t in (out if isinstance(out, list) else [out]) for y in torch.autograd.forward_ad.unpack_dual(t) if y is not None]
+        if watch == "trace":
+            return torch.jit.trace(call, (x,), check_trace=False)(x)
+        with {"dispatch mode": Dispatch, "function mode": Function}[watch]():
+            return call(x)
+
+    def run():
+        outs = []
+        Dispatch.seen = Function.seen = 0
+        for call, x in calls.values():
+            if watch == "deterministic":
+                torch.use_deterministic_algorithms(True, warn_only=True)
+                try:
+                    outs.append(call(x))
+                finally:
+                    torch.use_deterministic_algorithms(False)
+                continue
+            try:
+                outs.append(watched(call, x))
+            except RuntimeError as e:                              # (what the Python methods cannot do they refuse)
+                outs.append(type(e).__name__)
+        return outs + [Dispatch.seen, Function.seen]
+    a, b, taken, left = both(run)
+    assert _same(a, b) and taken == 0 and left >= 1
+    if watch == "forward mode":
+        assert len(a[3]) == 2 and float(a[3][1].abs().max()) > 0           # (the values' sum has a derivative)
+    if watch in ("dispatch mode", "function mode"):
+        assert a[-2] + a[-1] > 0
+
+
+def test_threads_share_a_quantiser(gpu, both):
+    """Calls of several threads, one of which has the quantiser's descriptors built again and again: the results of one thread alone."""
+    quant = TurboQuantProd(128, bits=3, device=gpu)
+    g = torch.Generator().manual_seed(8)
+    xs = [torch.randn(40 + i, 128, generator=g).to(gpu) for i in range(3)]
+    want = [list(quant.quantize(x)[:4]) + [quant.attention_score(x[:5], quant.quantize(x))] for x in xs]
+    first = quant.mse_quantizer.quantize(xs[0]).indices
+
+    def run():
+        torch.cuda.synchronize()
+        wrong = []
+
+        def use(x, result):
+            try:
+                for _ in range(20):
+                    code = quant.quantize(x)
+                    if not _same(list(code[:4]) + [quant.attention_score(x[:5], code)], result):
+                        wrong.append(x.shape)
+            except Exception as e:
+                wrong.append(repr(e))
+
+        def rebuild():
+            try:
+                for _ in range(10):
+                    quant.S.add_(0)
+                    if not torch.equal(quant.mse_quantizer.quantize(xs[0]).indices, first):
+                        wrong.append("first stage")
+            except Exception as e:
+                wrong.append(repr(e))
+        threads = [threading.Thread(target=use, args=a) for a in zip(xs, want)] + [threading.Thread(target=rebuild)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        return wrong
+    a, b, taken, left = both(run)
+    assert a == b == [] and taken > 0 and left == 0
 
 
 def test_a_captured_step_and_a_side_stream(gpu, both):
