@@ -813,7 +813,7 @@ def test_a_method_in_the_place_of_one_that_native_calls_go_past_sees_every_call(
     batched.BatchedLayerState(config=config, quantizer=tq, pool=pool).write(kv, kv, meta)
     store = S.CompressedKVStore(128, 2, value_bits=4, device="cpu")
     store._pool, store._block_table, store._counts = pool, torch.arange(64, dtype=torch.int32)[None], torch.arange(1025, dtype=torch.int32)
-    store._chunk_lengths = [100]
+    store._chunk_lengths, store._table_pages = [100], 64
     query = torch.zeros(1, 4, 128, dtype=torch.bfloat16)
     score.compute_hybrid_attention(query, store, None, None, 4)
     assert (seen, native) == (([], ["append", "decode_attention"]) if how == "as it is" else (["append", "decode_attention"], []))

@@ -9,6 +9,7 @@ from __future__ import annotations
 import ctypes as C
 import logging
 import math
+import operator
 import os
 import sys
 from typing import Optional
@@ -183,14 +184,20 @@ def native():
     return None if _host is None or _compiling() else _host
 
 
+def own_methods(cls, *names: str):
+    """What `as_defined` compares an object's methods `names` with: the functions that cls defines."""
+    functions = tuple(getattr(cls, n) for n in names)
+    return operator.attrgetter(*(n + ".__func__" for n in names)), functions if len(names) > 1 else functions[0]
+
+
 def as_defined(obj, methods) -> bool:
-    """Whether `methods` ((name, function), ...) are still what obj calls by those names, so that a caller may go past them to what
-    they call: a subclass's, a stand-in's, or one put on the class or the object sees every call."""
-    cls, own = type(obj), getattr(obj, "__dict__", ())
-    for name, function in methods:
-        if getattr(cls, name, None) is not function or name in own:
-            return False
-    return True
+    """Whether `methods` (own_methods) are still what obj calls by those names, so that a caller may go past them to what they call: a
+    subclass's, a stand-in's, or a function put on the class or the object sees every call.  (0.1 us: it stands in front of every small call.)"""
+    find, functions = methods
+    try:
+        return find(obj) == functions
+    except AttributeError:
+        return False
 
 
 def check(rc: int, what: str):

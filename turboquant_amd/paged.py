@@ -447,7 +447,7 @@ class PagedKVPool:
         return out
 
 
-# what a native call goes past, as it is defined here (_ffi.as_defined)
-APPEND = (("append", PagedKVPool.append),)
-WORKSPACE = (("workspace", PagedKVPool.workspace),)
-DECODE = (("decode_attention", PagedKVPool.decode_attention), *WORKSPACE)
+# what a native call goes past
+APPEND = _ffi.own_methods(PagedKVPool, "append")
+WORKSPACE = _ffi.own_methods(PagedKVPool, "workspace")
+DECODE = _ffi.own_methods(PagedKVPool, "decode_attention", "workspace")

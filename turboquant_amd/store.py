@@ -15,6 +15,7 @@ from typing import NamedTuple, Optional
 
 import torch
 
+from . import _ffi
 from .kv_cache import ValueQuantized
 from .paged import PAGE_TOKENS, PagedKVPool
 from .quantizer import ProdQuantized, TurboQuantProd
@@ -44,6 +45,7 @@ class CompressedKVStore:
         self._chunk_lengths: list[int] = []
         self._pool: Optional[PagedKVPool] = None
         self._block_table: Optional[torch.Tensor] = None
+        self._table_pages = 0
         self._counts: Optional[torch.Tensor] = None
         self._flat: Optional[FlatCache] = None
 
@@ -72,8 +74,7 @@ class CompressedKVStore:
 
     def has_pages(self, n: int) -> bool:
         """Whether the pool and the table exist as ensure_pool leaves them, and `n` is a length they can hold."""
-        return (self._pool is not None and self._block_table is not None and self._block_table.shape[1] == self._pool.num_pages and
-                n < self._counts.shape[0])
+        return self._pool is not None and self._table_pages == self._pool.num_pages and n <= self._table_pages * PAGE_TOKENS
 
     def ensure_pool(self, dtype: torch.dtype, min_tokens: int = 0) -> PagedKVPool:
         need = max(self._INITIAL_PAGES, (min_tokens + PAGE_TOKENS - 1) // PAGE_TOKENS)
@@ -83,6 +84,7 @@ class CompressedKVStore:
         elif need > self._pool.num_pages:
             self._pool.grow(max(need, 2 * self._pool.num_pages))
         if self._block_table is None or self._block_table.shape[1] != self._pool.num_pages:
+            self._table_pages = self._pool.num_pages
             self._block_table = torch.arange(self._pool.num_pages, dtype=torch.int32, device=self._pool.device)[None, :]
             # (every length the sequence can have, so that a step need not write its own; memory apart from the table's, which a
             # caller may rearrange)
@@ -159,5 +161,5 @@ class CompressedKVStore:
         self._flat = None
 
 
-# what a decode step goes past where the pages exist, as it is defined here (_ffi.as_defined)
-STEP = (("ensure_pool", CompressedKVStore.ensure_pool), ("lengths", CompressedKVStore.lengths))
+# what a decode step goes past where the pages exist
+STEP = _ffi.own_methods(CompressedKVStore, "ensure_pool", "lengths")
