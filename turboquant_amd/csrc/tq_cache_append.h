@@ -67,7 +67,7 @@ __device__ __forceinline__ void copy_rows(const CopySection& c, int64_t rows, in
     if (in[k]) __builtin_nontemporal_store(x[k], to[k]);
 }
 
-// Workgroup `id` of rows + copies, 256 threads; d <= 256.  The values' arithmetic and rounding are those of value_tile_kernel.
+// Workgroup `id` of rows + copies, 256 threads; d <= 256.
 __device__ __forceinline__ void cache_rest_body(const CacheRest& A, int id) {
   __shared__ float sx[256], s_sc[16], s_z[16];
   __shared__ uint8_t s_code[256];
@@ -86,18 +86,8 @@ __device__ __forceinline__ void cache_rest_body(const CacheRest& A, int id) {
   if (tid < d) sx[tid] = A.v[id * A.v_stride + tid];
   __syncthreads();
   if (tid < ng) {
-    const float* row = sx + tid * gs;
-    float lo = row[0], hi = row[0];
-    bool has_nan = false;
-    for (int i = 0; i < gs; ++i) {
-      const float a = row[(i + tid) % gs];         // (another bank per group)
-      has_nan |= (a != a);
-      lo = fminf(lo, a);
-      hi = fmaxf(hi, a);
-    }
-    if (has_nan) lo = hi = __uint_as_float(0x7fc00000u);      // torch min / max propagate NaN
-    float sc = (hi - lo) / levels;
-    sc = (sc != sc) ? sc : fmaxf(sc, 1e-10f);
+    float sc, lo;
+    value_group<TQ_F32>(sx + tid * gs, gs, tid, levels, sc, lo);
     s_sc[tid] = sc;
     s_z[tid] = lo;
     const int64_t at = id * A.step * ng + tid;
@@ -105,10 +95,7 @@ __device__ __forceinline__ void cache_rest_body(const CacheRest& A, int id) {
     A.zeros[at] = lo;
   }
   __syncthreads();
-  if (tid < d) {
-    const float q = fminf(fmaxf(rintf((sx[tid] - s_z[tid / gs]) / s_sc[tid / gs]), 0.0f), levels);
-    s_code[tid] = (q != q) ? (uint8_t)0 : (uint8_t)q;
-  }
+  if (tid < d) s_code[tid] = value_code<TQ_F32>(sx[tid], s_z[tid / gs], s_sc[tid / gs], levels);
   __syncthreads();
   const int per = 32 / A.bits, words = d / per;
   if (tid < words) {

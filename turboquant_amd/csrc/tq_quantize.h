@@ -221,6 +221,37 @@ struct RaggedSource : PagedSource {
 };
 
 // ------------------------------------------------------------------------------------
+// values: a group's scale and zero, and an element's code (value_chunk_body has the same numbers by other instructions)
+// ------------------------------------------------------------------------------------
+
+// `turn`: where the reading begins (another bank per thread)
+template <int DT>
+__device__ __forceinline__ void value_group(const float* row, int gs, int turn, float levels, float& sc, float& zero) {
+  using E = Elem<DT>;
+  float lo = row[0], hi = row[0];
+  bool has_nan = false;
+  for (int i = 0; i < gs; ++i) {
+    const float a = row[(i + turn) % gs];
+    has_nan |= (a != a);
+    lo = fminf(lo, a);
+    hi = fmaxf(hi, a);
+  }
+  if (has_nan) lo = hi = __uint_as_float(0x7fc00000u);       // torch min / max propagate NaN
+  sc = E::round(E::round(hi - lo) / levels);
+  const float floor_v = E::round(1e-10f);
+  sc = (sc != sc) ? sc : fmaxf(sc, floor_v);
+  zero = lo;
+}
+template <int DT>
+__device__ __forceinline__ uint8_t value_code(float x, float zero, float sc, float levels) {
+  using E = Elem<DT>;
+  float q = E::round(E::round(x - zero) / sc);
+  q = rintf(q);
+  q = fminf(fmaxf(q, 0.0f), levels);
+  return (q != q) ? (uint8_t)0 : (uint8_t)q;
+}
+
+// ------------------------------------------------------------------------------------
 // key tile
 // ------------------------------------------------------------------------------------
 

@@ -229,30 +229,12 @@ value_tile_kernel(const void* __restrict__ v, Source src, int d, int gs, int bit
   const float levels = (float)((1 << bits) - 1);
   for (int o = j; o < TILE * ng; o += d) {
     int t = o / ng, g = o - t * ng;
-    const float* row = sv + t * d + g * gs;
-    float lo = row[0], hi = row[0];
-    bool has_nan = false;
-    for (int i = 0; i < gs; ++i) {
-      float a = row[(i + j) % gs];           // rotate the start to spread LDS banks
-      has_nan |= (a != a);
-      lo = fminf(lo, a);
-      hi = fmaxf(hi, a);
-    }
-    if (has_nan) lo = hi = __uint_as_float(0x7fc00000u);   // torch min/max propagate NaN
-    float sc = E::round(E::round(hi - lo) / levels);
-    float floor_v = E::round(1e-10f);
-    sc = (sc != sc) ? sc : fmaxf(sc, floor_v);
-    sscale[o] = sc;
-    szero[o] = lo;
+    value_group<DT>(sv + t * d + g * gs, gs, j, levels, sscale[o], szero[o]);
   }
   __syncthreads();
   for (int t = 0; t < TILE; ++t) {
     int g = j / gs;
-    float sc = sscale[t * ng + g], z = szero[t * ng + g];
-    float q = E::round(E::round(sv[t * d + j] - z) / sc);
-    q = rintf(q);
-    q = fminf(fmaxf(q, 0.0f), levels);
-    scode[t * d + j] = (q != q) ? (uint8_t)0 : (uint8_t)q;
+    scode[t * d + j] = value_code<DT>(sv[t * d + j], szero[t * ng + g], sscale[t * ng + g], levels);
   }
   __syncthreads();
 
