@@ -847,3 +847,18 @@ def test_a_workspace_of_its_own_is_taken_by_every_decode_step(monkeypatch):
     for step in (lambda: pool.decode_attention(q, table, one), lambda: pool.decode_attention_ring(q, table, one, exact, exact, 16)):
         with pytest.raises(Asked):
             step()
+
+
+@pytest.mark.parametrize("d,mse_bits", [(64, 1), (128, 2), (128, 3), (256, 4)])
+def test_the_workspace_of_a_cache_token_holds_the_keys_codes_and_no_more(d, mse_bits):
+    """Four sections (indices, signs, norms, residual norms), each begun on a 16-byte boundary, from any address: a value's codes are not among
+    them."""
+    for batch in (1, 3, 17, 4096):
+        sections = [batch * d * (1, 1, 2, 4, 4)[mse_bits] // 8, batch * d // 8, batch * 4, batch * 4]
+        at = 15
+        for n in sections:
+            at += (n + 15) // 16 * 16
+        for value_bits, group_size in ((2, 16), (4, 32), (8, 64)):
+            have = _ffi.lib().tq_cache_append_bytes(batch, d, mse_bits, value_bits, group_size)
+            assert at <= have <= sum(sections) + 5 * 16
+    assert _ffi.lib().tq_cache_append_bytes(1, 128, 5, 2, 32) == 0 == _ffi.lib().tq_cache_append_bytes(0, 128, 2, 2, 32)

@@ -914,8 +914,8 @@ static bool cache_dims(int64_t batch, int H, int d) { return batch > 0 && batch 
 
 extern "C" size_t tq_cache_append_bytes(int64_t batch, int d, int mse_bits, int value_bits, int group_size) {
   if (batch <= 0 || d <= 0 || mse_bits < 1 || mse_bits > 4 || value_bits <= 0 || group_size <= 0) return 0;
-  const size_t per = (size_t)idx_row_bytes(d, mse_bits) + d / 8 + 8 + (size_t)d * value_bits / 8 + 8 * (size_t)(d / group_size);
-  return batch * per + 7 * 16;
+  // (the key's codes and norms, where two launches hand them on; a value's go straight to their place)
+  return batch * ((size_t)idx_row_bytes(d, mse_bits) + d / 8 + 8) + 5 * 16;
 }
 
 extern "C" int tq_cache_append(const float* key, const float* value, int64_t key_stride, int64_t value_stride, const float* key_buf,
