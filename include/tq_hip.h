@@ -196,8 +196,9 @@ int tq_rotate_query(const void *q, int dtype, int64_t rows, const tq_layer *laye
  * the buffer's first row leaves it and is quantised: every section is written anew with one more token, and the
  * buffers with their rows one further (contiguous).  The buffers' rows have to lie one behind another (s_r = d) and, with more
  * than one batch, s_b = H s_h; else TQ_EUNSUPPORTED, as for sections off a 4-byte boundary and for n_c or n_buf above 2^20.
- * n_c may be 0 (the sections are not read then).  work: tq_cache_append_bytes bytes.  One launch at d = 128 / 256 and copies of
- * up to 48 MB, else two.
+ * n_c may be 0 (the sections are not read then).  work: tq_cache_append_bytes bytes.  One launch at d = 128 / 256 where the
+ * matrix cores take the keys, up to twelve workgroups of values and copies per compute unit (48 MB in 16-byte pieces, a
+ * quarter of that in words); else two.
  * tq_cache_scores (kv_cache.py:247-284): scores (batch, n_q, n_c + n_buf) = scale * <q, k> over the compressed keys, then the
  * exact ones; n_c, n_buf > 0.  TQ_EUNSUPPORTED: codes off a 4-byte boundary, n_q above 2^18, n_c above 2^28, n_buf above 2^24.  work:
  * 2 * batch * n_q * d floats.

@@ -910,8 +910,10 @@ static int launch_cache_append_d(const float* keys, const FlatSource& src, const
 }
 
 // The whole token in one launch, at head_dim 128 / 256.  Every workgroup of it reserves a key tile's LDS, so a compute unit holds one: up to
-// twelve rounds of copies (48 MB; four tokens and their attention, one launch and two: of 15 MB 361 and 383 us, of 31 MB 733 and 766, of
-// 62 MB 1172 and 1164); beyond, and where the matrix-core kernel does not take the keys, TQ_EUNSUPPORTED: the caller launches two.
+// twelve rounds of values and copies.  A round copies 4 MB in 16-byte pieces, 1 MB in words (norms of most lengths, 7 % of the bytes at
+// 128; a value buffer off a 16-byte boundary, all of its): 48 MB where sections and buffers begin on such boundaries, as those that the cache
+// writes do.  Four tokens and their attention, one launch and two: of 15 MB 361 and 383 us, of 31 MB 733 and 766, of 62 MB 1172 and 1164.
+// Beyond, and where the matrix-core kernel does not take the keys (rows off 16 bytes), TQ_EUNSUPPORTED: the caller launches two.
 int launch_cache_append(const float* keys, int64_t stride, int64_t rows, const tq_layer& ly, const KeyRowsSink& ks, const CacheRest& rest,
                         hipStream_t st) {
   const FlatSource src{rows, stride};
