@@ -862,3 +862,31 @@ def test_the_workspace_of_a_cache_token_holds_the_keys_codes_and_no_more(d, mse_
             have = _ffi.lib().tq_cache_append_bytes(batch, d, mse_bits, value_bits, group_size)
             assert at <= have <= sum(sections) + 5 * 16
     assert _ffi.lib().tq_cache_append_bytes(1, 128, 5, 2, 32) == 0 == _ffi.lib().tq_cache_append_bytes(0, 128, 2, 2, 32)
+
+
+@pytest.mark.parametrize("query", [torch.zeros(1, 4, 128), torch.zeros(1, 4, 128, dtype=torch.bfloat16), torch.zeros(2, 4, 128, dtype=torch.bfloat16),
+                                   torch.zeros(1, 4, 64, dtype=torch.bfloat16)])
+def test_a_step_that_the_native_host_side_leaves_is_looked_at_once_and_checked(monkeypatch, query):
+    """A query on the CPU (or of another head size) raises before the library is called, and one token is offered to the native host side
+    once where nothing about it changes on the way."""
+    from turboquant_amd import score, store as S
+    from turboquant_amd.paged import PagedKVPool
+    offered = []
+    library = _ffi.lib()
+
+    class Library:
+        def __getattr__(self, name):
+            assert "attn" not in name, f"{name} was called"
+            return getattr(library, name)
+    monkeypatch.setattr(_ffi, "lib", lambda: Library())
+    monkeypatch.setattr(_ffi, "_host", types.SimpleNamespace(decode=lambda *a: offered.append(a)))
+    monkeypatch.setattr(TurboQuantProd, "_layer", lambda self: None)
+    pool = PagedKVPool.__new__(PagedKVPool)
+    pool.quantizer, pool.head_dim, pool.num_kv_heads, pool.data, pool.layout = TurboQuantProd(128, bits=3, device="cpu"), 128, 2, torch.zeros(1), None
+    pool.dtype, pool.device, pool.num_pages, pool.value_bits, pool.value_group_size = torch.bfloat16, torch.device("cpu"), 64, 4, 32
+    store = S.CompressedKVStore(128, 2, value_bits=4, device="cpu")
+    store._pool, store._block_table, store._counts = pool, torch.arange(64, dtype=torch.int32)[None], torch.arange(1025, dtype=torch.int32)
+    store._chunk_lengths, store._table_pages = [100], 64
+    with pytest.raises((RuntimeError, ValueError), match="lives on cpu|Incompatible"):
+        score.compute_hybrid_attention(query, store, None, None, 4)
+    assert len(offered) <= 1

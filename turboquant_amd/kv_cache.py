@@ -170,7 +170,7 @@ class TurboQuantKVCache:
         """The seven tensors of the compressed part, for the native host side, which looks at each; None: not for it."""
         kq, vq = self.key_quantized, self.value_quantized
         if (_ffi.native() is None or kq is None or vq is None or vq.bits != self.value_bits or self.head_dim not in (64, 128, 256)
-                or self.value_group_size % 16 or kq.norms.dim() != 3):
+                or self.value_group_size % 16 or kq.norms.dim() != 3 or kq.norms.dtype is not torch.float32):
             return None
         return (*kq[:4], *vq[:3])
 

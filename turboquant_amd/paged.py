@@ -59,9 +59,9 @@ class PagedKVPool:
         """Quantise key/value (B, T, H, d) and store token t of sequence b at
         logical position start_pos[b] + t through block_table (B, max_pages) int32."""
         _ffi.require_gpu(key, "key")
-        fast = _ffi.native()
+        ly, fast = self.quantizer._layer(), _ffi.native()
         if fast is not None and fast.append(key, value, block_table, start_pos, self.data, self.num_pages, self.num_kv_heads, self.head_dim,
-                                            _ffi.dtype_tag(self.dtype), self.quantizer._layer(), self.layout, False):
+                                            _ffi.dtype_tag(self.dtype), ly, self.layout, False):
             return
         if key.dim() != 4 or key.shape != value.shape:
             raise ValueError("key and value must both be (B, T, H, d)")
@@ -77,7 +77,6 @@ class PagedKVPool:
         block_table = block_table.contiguous()
         if start_pos is not None:
             start_pos = start_pos.to(device=self.device, dtype=torch.int32).contiguous()
-        ly = self.quantizer._layer()
         with _ffi.on_device(self.device):
             _ffi.check(_ffi.lib().tq_append_kv_paged(
                 key.data_ptr(), value.data_ptr(), _ffi.dtype_tag(self.dtype), B, T, H, key.stride(0), key.stride(1),
@@ -291,13 +290,13 @@ class PagedKVPool:
             return 1 + (have - least) // (need(B, Hq, self.head_dim, 2) - least)
         raise ValueError(f"the workspace holds {have} bytes, {B} x {Hq} query heads in {n_split} splits take {want}")
 
-    def _decode_native(self, query, block_table, seq_lens, first, scale, recent_k, recent_v, n_split, by_length) -> Optional[torch.Tensor]:
+    def _decode_native(self, ly, query, block_table, seq_lens, first, scale, recent_k, recent_v, n_split, by_length) -> Optional[torch.Tensor]:
         """A whole step (lengths from element `first` on) by the native host side; None: not a case for it, nothing was done."""
         fast = _ffi.native()
         if fast is None:
             return None
         return fast.decode(query, block_table, seq_lens, first, self.data, self.num_pages, self.num_kv_heads, self.head_dim, scale, recent_k,
-                           recent_v, self.quantizer._layer(), self.layout, n_split, by_length)
+                           recent_v, ly, self.layout, n_split, by_length)
 
     def decode_attention(self, query: torch.Tensor, block_table: torch.Tensor, seq_lens: torch.Tensor,
                          scale: Optional[float] = None, recent_k: Optional[torch.Tensor] = None,
@@ -321,7 +320,7 @@ class PagedKVPool:
             raise ValueError(f"Incompatible GQA shapes: Q={Hq}, H_kv={self.num_kv_heads}, d={d}")
         if scale is None:
             scale = 1.0 / math.sqrt(d)
-        by_length, ours = False, n_split is None
+        by_length, ours, ly = False, n_split is None, self.quantizer._layer()
         if ours:
             if max_len is None:
                 max_len = block_table.shape[-1] * PAGE_TOKENS
@@ -329,9 +328,17 @@ class PagedKVPool:
             by_length = workspace is None and not static_scratch and stages == 7 and self._shares_by_length(B, Hq)
         if (workspace is None and out is None and recent_len is None and stages == 7 and not static_scratch
                 and _ffi.as_defined(self, WORKSPACE)):
-            done = self._decode_native(query, block_table, seq_lens, 0, scale, recent_k, recent_v, n_split, by_length)
+            done = self._decode_native(ly, query, block_table, seq_lens, 0, scale, recent_k, recent_v, n_split, by_length)
             if done is not None:
                 return done
+        return self._decode(ly, query, block_table, seq_lens, scale, recent_k, recent_v, recent_len, n_split, by_length, ours, workspace, out,
+                            stages, static_scratch)
+
+    def _decode(self, ly, query, block_table, seq_lens, scale, recent_k, recent_v, recent_len, n_split, by_length=False, ours=True, workspace=None,
+                out=None, stages=7, static_scratch=False) -> torch.Tensor:
+        """decode_attention behind its checks of shapes and its choice of splits, for whatever the native host side leaves."""
+        _ffi.require_gpu(query, "query")
+        B, Hq, _ = query.shape
         query = query.contiguous()
         bt = block_table.contiguous()
         bt_stride = -bt.shape[0] if bt.dim() == 1 else bt.shape[1]      # negative: one shared row of that length
@@ -359,7 +366,6 @@ class PagedKVPool:
             if recent_len is not None:
                 recent_len = recent_len.to(device=self.device, dtype=torch.int32).contiguous()
                 rl_ptr = recent_len.data_ptr()
-        ly = self.quantizer._layer()
         if static_scratch:
             with _ffi.on_device(self.device):
                 _ffi.check(_ffi.lib().tq_decode_attn_paged_noalloc(
@@ -418,10 +424,10 @@ class PagedKVPool:
                 max_len = block_table.shape[-1] * PAGE_TOKENS
             n_split = self.default_splits(B, max_len, Hq)
             by_length = workspace is None and self._shares_by_length(B, Hq)
-        fast = _ffi.native()
+        ly, fast = self.quantizer._layer(), _ffi.native()
         if fast is not None and workspace is None and out is None and _ffi.as_defined(self, WORKSPACE):
             done = fast.decode_ring(query, block_table, seq_lens, self.data, self.num_pages, self.num_kv_heads, self.head_dim, scale,
-                                    key_cache, value_cache, ring_rows, self.quantizer._layer(), self.layout,
+                                    key_cache, value_cache, ring_rows, ly, self.layout,
                                     n_split, by_length)
             if done is not None:
                 return done
@@ -435,7 +441,6 @@ class PagedKVPool:
             n_split = self._splits_within(workspace, B, Hq, n_split, ours)
         if out is None:
             out = torch.empty_like(query)
-        ly = self.quantizer._layer()
         with _ffi.on_device(self.device):
             entry = _ffi.lib().tq_decode_attn_paged_ring_by_length if by_length else _ffi.lib().tq_decode_attn_paged_ring
             _ffi.check(entry(

@@ -224,17 +224,17 @@ class TurboQuantProd(torch.nn.Module):
 
     def _layer(self) -> _ffi.TqLayer:
         S, ST = _buffer(self, "S"), _buffer(self, "_ST")
-        if ST.device != S.device or getattr(self, "_ST_version", None) != S._version:
+        if ST.get_device() != S.get_device() or getattr(self, "_ST_version", None) != S._version:
             self._ST = ST = S.T.contiguous()
             self._ST_version = S._version
-        return self.mse_quantizer._layer(S, ST)
+        mse = self._modules.get("mse_quantizer")               # (past nn.Module's look-up, as _buffer)
+        return (self.mse_quantizer if mse is None else mse)._layer(S, ST)
 
     def quantize(self, x: torch.Tensor) -> ProdQuantized:
         _ffi.require_gpu(x, "x")
-        mb = self.bits - 1
-        fast = _ffi.native()
+        mb, ly, fast = self.bits - 1, self._layer(), _ffi.native()
         if fast is not None:
-            code = fast.quantize(x, self._layer(), self.dim, mb)
+            code = fast.quantize(x, ly, self.dim, mb)
             if code is not None:
                 return ProdQuantized(*code, mb)
         rows, stride = _rows(x)
@@ -242,7 +242,6 @@ class TurboQuantProd(torch.nn.Module):
         width, per_byte = _packing(mb)
         packed, signs = _codes(x, n, (d + per_byte - 1) // per_byte), _codes(x, n, (d + 7) // 8)
         norms, rnorms = _codes(x, n, dtype=x.dtype), _codes(x, n, dtype=torch.float32)
-        ly = self._layer()
         with _ffi.on_device(x.device):
             _ffi.check(_ffi.lib().tq_quantize_keys(
                 rows.data_ptr(), _ffi.dtype_tag(x.dtype), n, stride, C.byref(ly), packed.data_ptr(), signs.data_ptr(),
@@ -277,9 +276,9 @@ class TurboQuantProd(torch.nn.Module):
 
     def dequantize(self, q: ProdQuantized) -> torch.Tensor:
         _ffi.require_gpu(q.mse_indices, "mse_indices")
-        fast = _ffi.native()
+        ly, fast = self._layer(), _ffi.native()
         if fast is not None:
-            out = fast.dequantize(q.mse_indices, q.qjl_signs, q.residual_norms, q.norms, self._layer(), self.dim, self.bits - 1)
+            out = fast.dequantize(q.mse_indices, q.qjl_signs, q.residual_norms, q.norms, ly, self.dim, self.bits - 1)
             if out is not None:
                 return out
         idx = q.mse_indices.contiguous()
@@ -289,7 +288,6 @@ class TurboQuantProd(torch.nn.Module):
         lead = norms.shape
         n = norms.numel()
         out = torch.empty(n, self.dim, dtype=torch.float32, device=idx.device)
-        ly = self._layer()
         with _ffi.on_device(idx.device):
             _ffi.check(_ffi.lib().tq_dequant_keys(
                 idx.data_ptr(), signs.data_ptr(), norms.data_ptr(), _ffi.dtype_tag(norms.dtype), rnorms.data_ptr(), n,
@@ -300,11 +298,10 @@ class TurboQuantProd(torch.nn.Module):
         """query (..., n_q, d), keys (..., n_k, ...) -> raw logits (..., n_q, n_k), fp32,
         without the 1/sqrt(d) factor."""
         _ffi.require_gpu(query, "query")
-        d = self.dim
-        fast = _ffi.native()
+        d, ly, fast = self.dim, self._layer(), _ffi.native()
         if fast is not None:
             k = quantized_key
-            scores = fast.score(query, k.mse_indices, k.qjl_signs, k.residual_norms, k.norms, self._layer(), d, self.bits - 1)
+            scores = fast.score(query, k.mse_indices, k.qjl_signs, k.residual_norms, k.norms, ly, d, self.bits - 1)
             if scores is not None:
                 return scores
         lead = query.shape[:-2]
@@ -323,7 +320,6 @@ class TurboQuantProd(torch.nn.Module):
         batch = int(math.prod(lead)) if len(lead) else 1
         scores = torch.empty(*lead, n_q, n_k, dtype=torch.float32, device=q.device)
         work = torch.empty(2 * batch * n_q * d, dtype=torch.float32, device=q.device)
-        ly = self._layer()
         with _ffi.on_device(q.device):
             _ffi.check(_ffi.lib().tq_score(
                 q.data_ptr(), _ffi.dtype_tag(q.dtype), batch, n_q, idx.data_ptr(), signs.data_ptr(), norms.data_ptr(),

@@ -49,11 +49,13 @@ def compute_hybrid_attention(query: torch.Tensor, store: CompressedKVStore, rece
         raise ValueError(f"Incompatible GQA shapes: Q={Q}, H_kv={num_kv_heads}, gqa_ratio={gqa_ratio}")
 
     # one query token over a store that holds its pages already, everything plain: the tensors as they are, without a view of any
+    ly = None
     if (T == 1 and has_history and _ffi.as_defined(store, STEP) and store.has_pages(n_hist) and
-            _ffi.as_defined(store.pool, DECODE)):
+            _ffi.as_defined(store.pool, DECODE) and (not has_recent or recent_k.dtype is query.dtype)):
         pool = store.pool
-        out = pool._decode_native(query, store.block_table, store.counts, n_hist, scale, recent_k if has_recent else None, recent_v,
-                                  pool.default_splits(1, n_hist, Q), False)
+        ly, n_split = pool.quantizer._layer(), pool.default_splits(1, n_hist, Q)
+        out = pool._decode_native(ly, query, store.block_table, store.counts, n_hist, scale, recent_k if has_recent else None, recent_v,
+                                  n_split, False)
         if out is not None:
             return out
 
@@ -70,6 +72,9 @@ def compute_hybrid_attention(query: torch.Tensor, store: CompressedKVStore, rece
         rk, rv = recent_k.to(work_dtype).unsqueeze(0), recent_v.to(work_dtype).unsqueeze(0)
         if T != 1:
             rk, rv = rk.expand(T, *recent_k.shape), rv.expand(T, *recent_v.shape)
-    out = pool.decode_attention(q, store.block_table[0], seq_lens, scale=scale, recent_k=rk, recent_v=rv,
-                                max_len=max(n_hist, 1))
+    if ly is not None and q is query and D == head_dim:        # (the native host side would leave it again)
+        out = pool._decode(ly, q, store.block_table[0], seq_lens, scale, rk, rv, None, n_split)
+    else:
+        out = pool.decode_attention(q, store.block_table[0], seq_lens, scale=scale, recent_k=rk, recent_v=rv,
+                                    max_len=max(n_hist, 1))
     return out.to(query.dtype)
