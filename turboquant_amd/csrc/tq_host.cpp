@@ -2,8 +2,8 @@
 //
 // A decode token of one sequence, a token of the cache object or a few thousand keys to codes are two to eight launches of a few
 // microseconds each; the tensor attributes, allocations and foreign-function conversions around them took longer than the launches.  Host time
-// through the Python methods, through here, and the kernels' time, us: a chat token (ring, decode step) 53, 29, 22; a token of the cache object
-// (append, scores, softmax, weighted values; 8 heads of 128, 4096 tokens) 111, 60, 38; 4096 keys of 128 to codes, scores with 32 queries and back 45, 24, 31.
+// through the Python methods, through here, and the kernels' time, us: a chat token (ring, decode step) 47, 25, 22; a token of the cache object
+// (append, scores, softmax, weighted values; 8 heads of 128, 4096 tokens) 101, 53, 38; 4096 keys of 128 to codes, scores with 32 queries and back 43, 23, 31.
 // Every function here takes the case that the Python method in front of it meets in a decode loop - plain dense tensors of the current
 // device, contiguous where the library wants it - and returns None (ring_write: False) for everything else, before it allocates or launches
 // anything: the Python method then goes on as if it had not been called.  What the library refuses comes back as None too, with the outputs and

@@ -147,8 +147,8 @@ class TurboQuantKVCache:
     # ---- a decode token in fp32 (the general paths below take everything else) -----------------------------------------
     # A step of the general paths is some thirty small launches and seven concatenations of the whole history: 270 us, nearly all of it
     # host time, at 4096 tokens of 8 heads of 128.  The entries below are one launch for the token (two at head_dim 64, beyond 48 MB of copies
-    # and for rows off a 16-byte boundary), two for the scores and two for the values: with the softmax between them 38 us of the card, 60 of the
-    # host through its native side and 111 through the Python methods.  What an entry does not take (sections that are not word-aligned,
+    # and for rows off a 16-byte boundary), two for the scores and two for the values: with the softmax between them 38 us of the card, 53 of the
+    # host through its native side and 101 through the Python methods.  What an entry does not take (sections that are not word-aligned,
     # buffers or blocks of queries beyond its indexes) it refuses before it launches anything, and the general path goes on.
     def _compressed_plain(self) -> bool:
         """Whether the compressed part is what this cache writes itself in fp32.  One put in its place may have other bits, 16-bit norms
